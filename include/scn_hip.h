@@ -19,7 +19,10 @@
  *   - feature matrices are row-major fp32 [rows x channels]; rule books are
  *     row-major int32 [output rows x rule width]; rows are batch-global;
  *   - numeric kernels never allocate: every buffer is the caller's
- *     (SpatiallySparseBatchSubInterface, SpatiallySparseBatchInterface.h:8-17).
+ *     (SpatiallySparseBatchSubInterface, SpatiallySparseBatchInterface.h:8-17);
+ *     the one exception is the context's own copy of a layer's weights, which a
+ *     long contraction makes and the context keeps (never while its stream is
+ *     being captured: the weights are then converted on the way).
  *     scn_grids objects own their tables and only ever grow them.
  */
 #ifndef SCN_HIP_H
@@ -51,9 +54,15 @@ enum {
 };
 
 /* Operand precision of the NiN contraction (accumulation is always fp32):
- * fp32 MFMA; bf16 operands; or bf16 hi + lo pairs with three MFMAs per tile,
- * which keeps fp32-grade results at bf16-matrix-core speed. */
-enum { SCN_FP32 = 0, SCN_BF16 = 1, SCN_BF16X3 = 2 };
+ * fp32; bf16 operands; or bf16 hi + lo pairs with three MFMAs per tile, close
+ * to fp32 results at bf16-matrix-core speed.  SCN_FP32 and SCN_FP32_PLANES are
+ * the same precision: fp32 operands whole, fp32 sums.  SCN_FP32_PLANES splits
+ * every operand into three bf16 planes, x = hi + mid + lo exactly, and keeps the
+ * six largest of the nine products (the rest is below 2^-25 of the product), on
+ * the bf16 matrix cores; its sums have a third of the rounding error of the fp32
+ * MFMA's.  SCN_FP32 runs on the fp32 MFMA except for long contractions and few
+ * rows, which it computes as SCN_FP32_PLANES does. */
+enum { SCN_FP32 = 0, SCN_BF16 = 1, SCN_BF16X3 = 2, SCN_FP32_PLANES = 3 };
 
 typedef struct scn_ctx scn_ctx;
 typedef struct scn_grids scn_grids;

@@ -18,7 +18,7 @@ HEADER = os.path.join(ROOT, "include", "scn_hip.h")
 
 # ActivationFunction (reference types.h:11-20)
 NOSIGMOID, RELU, VLEAKYRELU, LEAKYRELU, TANH, SOFTMAX, PRELU, SIGMOID = range(8)
-FP32, BF16, BF16X3 = 0, 1, 2
+FP32, BF16, BF16X3, FP32_PLANES = 0, 1, 2, 3
 OK, ERR_ARG, ERR_HIP, ERR_CAPACITY, ERR_STATE = range(5)
 K_GRID_BUILD, K_RULES, K_GATHER, K_NIN, K_MAXPOOL, K_TERMINAL, K_SOFTMAX, K_CONV_NIN, K_PROBE, K_BACKWARD = range(10)
 KERNEL_FAMILIES = ["grid_build", "rules", "gather", "nin", "maxpool", "terminal", "softmax", "conv_nin", "probe",

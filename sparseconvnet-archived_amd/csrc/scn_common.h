@@ -40,6 +40,7 @@ struct ProfSpan {
 };
 
 #define SCN_ZERO_FLOATS 4096
+#define SCN_IMAGE_BYTES (16u << 20)
 #define SCN_MAX_PENDING 62 // plans per settle; 16 + 4 * 62 = 264 pinned words
 #define SCN_PINNED_WORDS (16 + 4 * SCN_MAX_PENDING)
 struct scn_ctx {
@@ -51,11 +52,11 @@ struct scn_ctx {
   int64_t *d_pinned; // the same memory as the device sees it
   int64_t *d_scalars; // 16 int64
   float *d_zeros;     // SCN_ZERO_FLOATS zeros: the row a negative rule stands for
+  unsigned char *d_image; // SCN_IMAGE_BYTES or null: a layer's weights as a long contraction streams them
   long long ticket;   // number of the last count readback (h_pinned[14] echoes it)
   // deferred counts (scn_ctx_defer_counts): plans whose counts are still on
   // their way; slot i of them reports into h_pinned[16 + 4 i ..]
   bool deferCounts;
-  bool wstream; // NiN: W-streaming kernel allowed (SCN_NIN_WSTREAM=0 turns it off)
   std::vector<struct scn_grids *> pendingGrids;
   struct ChainState *chain; // recorded rule-book plans (scn_chain.hip)
   // profiling
@@ -112,6 +113,9 @@ static inline int scn_ceil_div(int64_t a, int64_t b) {
 // address of the static scratch of scn_sgemm_ABt_static on `device` (scn_train.hip)
 int scn_abt_static_setup(int device);
 void scn_abt_static_forget(const scn_ctx *ctx);
+
+// counts contexts, and takes back ctx's image when one goes (scn_planes.hip)
+void scn_image_context(scn_ctx *ctx, bool alive);
 
 // runs the recorded rule-book plans of the context, if any (scn_chain.hip)
 int scn_chain_flush(scn_ctx *ctx);

@@ -33,10 +33,7 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   c->ticket = 0;
   c->deferCounts = false;
   c->chain = nullptr;
-  {
-    const char *e = getenv("SCN_NIN_WSTREAM");
-    c->wstream = !(e && e[0] == '0');
-  }
+  c->d_image = nullptr;
   memset(c->profMs, 0, sizeof(c->profMs));
   memset(c->profCalls, 0, sizeof(c->profCalls));
   hipDeviceProp_t prop;
@@ -58,6 +55,7 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   // than in front of the first batch that happens to use the stream)
   SCN_HIP_CHECK(hipMemsetAsync(c->d_zeros, 0, SCN_ZERO_FLOATS * sizeof(float), c->stream));
   SCN_HIP_CHECK(hipStreamSynchronize(c->stream));
+  scn_image_context(c, true);
   *out = c;
   return SCN_OK;
 }
@@ -69,6 +67,7 @@ extern "C" int scn_ctx_destroy(scn_ctx *c) {
   (void)hipStreamSynchronize(c->stream);
   scn_abt_static_forget(c);
   scn_chain_release(c);
+  scn_image_context(c, false);
   for (auto &s : c->spans) {
     (void)hipEventDestroy(s.a);
     (void)hipEventDestroy(s.b);

@@ -1,0 +1,82 @@
+// What the NetworkInNetwork kernels of several files share: the epilogue's
+// constants, the source of a gathered matrix, bf16 conversions.
+#pragma once
+#include "scn_common.h"
+#include <mutex>
+
+// Kernel attributes (the dynamic LDS limit) are set per device: fn runs once for
+// every device a context of this process lives on, and again if it failed.
+struct OncePerDevice {
+  std::mutex m;
+  unsigned long long done = 0;
+  template <class F> int run(int device, F fn) {
+    std::lock_guard<std::mutex> lock(m);
+    if (device >= 0 && device < 64 && ((done >> device) & 1ull))
+      return SCN_OK;
+    const int rc = fn();
+    if (rc == SCN_OK && device >= 0 && device < 64)
+      done |= 1ull << device;
+    return rc;
+  }
+};
+
+struct Epilogue {
+  const float *bias;
+  const float *prelu;
+  float p;
+  float slope;
+  int act;
+};
+
+// Bias, p and activation of one column, branch-free: every supported activation is v > 0 ? v : v * slope with slope
+// 1 (none), 0 (ReLU), a constant (leaky) or PReLU's learnt per-column value.
+struct ColEpilogue {
+  float pb;    // p * bias[n]
+  float p;
+  float slope;
+};
+__device__ __forceinline__ ColEpilogue load_col(const Epilogue &e, int n) {
+  ColEpilogue c;
+  c.p = e.p;
+  c.pb = e.p * e.bias[n];
+  c.slope = e.act == SCN_PRELU
+                ? e.prelu[n]
+                : (e.act == SCN_RELU ? 0.f
+                                     : (e.act == SCN_LEAKYRELU || e.act == SCN_VLEAKYRELU ? e.slope : 1.f));
+  return c;
+}
+__device__ __forceinline__ float finish(float acc, const ColEpilogue &c) {
+  const float v = c.p * acc + c.pb;
+  const float neg = c.slope == 0.f ? 0.f : v * c.slope;
+  return v > 0.f ? v : neg;
+}
+
+//
+// GATHER: A is never materialised.  Row m of A is the receptive field of
+// output site m, column q * nIn + c = channel c of input row
+// rules[m * fs + q] (what scn_gather_rows would have written).
+#define GF_MAX_FS 27
+struct GatherSource {
+  const int *rules;   // [M x fs]
+  int fs;             // rule-row width
+  int nIn;            // channels of the gathered matrix, nIn % 4 == 0
+  unsigned magic;     // floor(2^32 / nIn) + 1: k / nIn == mulhi(k, magic) for k nIn < 2^32
+  const float *zeros; // at least nIn zeros: the row a negative rule stands for
+};
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned pack_bf16x2(float a, float b) {
+  floatx2 f = {a, b};
+  bf16x2 h = __builtin_convertvector(f, bf16x2);
+  return __builtin_bit_cast(unsigned, h);
+}
+
+// scn_planes.hip: the contraction with fp32 operands as `planes` bf16 planes
+bool scn_planes_shape(int K);
+// ... takes the split contraction: few rows
+bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N);
+int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
+                       float *out, long long M, int K, int N,
+                       const Epilogue &ep, const GatherSource *gs, bool a16);

@@ -1,0 +1,718 @@
+// NetworkInNetwork contraction on the bf16 matrix cores, in one, two or three
+// bf16 planes per fp32 operand.
+//
+// A float has 24 significant bits and a bf16 8, so x = hi + mid + lo with
+// hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid is exact (both
+// subtractions are; |mid| <= 2^-9 |x|, |lo| <= 2^-17 |x|).  With three planes
+// of both operands the six products hi hi, hi mid, mid hi, mid mid, hi lo and
+// lo hi, each exact in the MFMA's fp32 accumulator, are the product a b up to
+// the 2^-25 |a b| of the three that are left out: less than the rounding of
+// one fp32 multiplication, and than that of the accumulation either way.
+// v_mfma_f32_32x32x16_bf16 does 32768 flops in the 32 cycles in which
+// v_mfma_f32_32x32x2_f32 does 2048 * 2, so six of them are 2.7 times as fast.
+//   PL 3: SCN_FP32; PL 2: SCN_BF16X3 (hi hi, hi lo, lo hi); PL 1: SCN_BF16.
+#include "scn_nin_dev.h"
+#include <math.h>
+#include <utility>
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// The PL planes of eight floats, each as an MFMA operand.
+template <int PL>
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[PL]) {
+  unsigned w[PL][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int l = 0; l < PL; ++l) {
+      const unsigned h = pack_bf16x2(a, b);
+      w[l][i] = h;
+      if (l + 1 < PL) {
+        a -= __uint_as_float(h << 16);
+        b -= __uint_as_float(h & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < PL; ++l)
+    p[l] = __builtin_bit_cast(bf16x8, uint4{w[l][0], w[l][1], w[l][2], w[l][3]});
+}
+
+// Four channels (A16: eight) of a gathered row: columns k .. of the row that
+// `rules` (in LDS, fs of them) stand for.
+template <bool A16>
+__device__ __forceinline__ floatx4 gathered_piece(const unsigned char *A, const GatherSource &gs,
+                                                  const int *rules, int k) {
+  const int f = (int)__umulhi((unsigned)k, gs.magic);
+  const int rule = rules[f];
+  const unsigned char *const row = rule >= 0 ? A + (long long)rule * gs.nIn * (A16 ? 2 : 4)
+                                             : reinterpret_cast<const unsigned char *>(gs.zeros);
+  return *reinterpret_cast<const floatx4 *>(row + (k - f * gs.nIn) * (A16 ? 2 : 4));
+}
+
+// A workgroup of four wavefronts owns 128 MT rows x 32 NT columns, a wavefront
+// 32 MT rows of them, and walks k in blocks of 32, two MFMA steps.
+// W passes through two LDS buffers, a block each, split into planes on the way
+// in and laid out as the MFMA reads it, [plane][16 k][tile][lane]: every
+// operand read is a contiguous kilobyte.  A goes from global memory (GATHER:
+// through the rules of the workgroup's rows, staged in LDS) straight into
+// registers, PD blocks ahead as W does, and is split there.
+// Lane (c, q) supplies k = 8 q .. 8 q + 7 of a step's sixteen for row c of A
+// and for its columns of W; it owns the NT adjacent columns NT c .. NT c + NT -
+// 1 (tile j of the MFMA = columns {NT c + j}).
+// The products beyond hi hi are a 2^-8 of it and go to accumulators of their
+// own: added to the large ones each of them would be rounded at their scale.
+//
+// The matrix pipe is kept busy by what is issued between its instructions: a
+// unit is one row tile's step, its 6 NT MFMAs (32 cycles each, 4 to issue) have
+// the splitting of the next unit's operand (44 vector instructions) dealt out
+// among them, the request for the operand a block on, and the reads of the W
+// tiles of the next step, each as soon as its registers have had their last
+// use.  The barrier of a block stands before its last tile's MFMAs.
+//
+// K is a multiple of 32.  GATHER 1: so are a gathered row's channels, and a
+// block lies within one filter position; GATHER 2: they are a multiple of 4 and
+// every four of them are looked up.  A16: the rows are bf16 already.
+template <int PL, int MT, int NT, int PD, int GATHER, bool A16, bool IMG>
+__global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 : 4)
+    k_nin_planes(const float *__restrict__ A, const float *__restrict__ W,
+                 float *__restrict__ out, long long M, int K, int N,
+                 Epilogue ep, GatherSource gs, int nSplits) {
+  constexpr int ES = A16 ? 2 : 4;
+  constexpr int WAVES = 4, THREADS = 64 * WAVES;
+  constexpr int ROWS = 32 * MT * WAVES, NW = 32 * NT;
+  constexpr int STEP_BYTES = NT * 1024;       // one plane of 16 k
+  constexpr int PLANE_BYTES = 2 * STEP_BYTES; // ... of a block
+  constexpr int BUF_BYTES = PL * PLANE_BYTES;
+  constexpr int UNITS = 2 * MT; // of a block: (step, row tile)
+  extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [2][BUF_BYTES], then the rules
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 31, q = lane >> 5;
+  const int split = blockIdx.x % nSplits; // workgroups that share rows are neighbours
+  const long long wgRow0 = (long long)(blockIdx.x / nSplits) * ROWS;
+  const long long row0 = wgRow0 + wave * 32 * MT;
+  const int n0 = split * NW;
+  const int T = K / 32;
+
+  // ---- W.  One item = 8 consecutive k of one column; IMG: 16 bytes of the image
+  constexpr int ITEMS = IMG ? BUF_BYTES / 16 : 4 * NW;
+  constexpr int WPER = (ITEMS + THREADS - 1) / THREADS;
+  constexpr int WREGS = IMG ? 4 : 8;
+  float wv[PD][WPER][WREGS];
+  int wDst[WPER];
+  const float *wSrc[WPER];
+#pragma unroll
+  for (int u = 0; u < WPER; ++u) {
+    int x = tid + THREADS * u;
+    x = x < ITEMS ? x : ITEMS - 1; // past the end: the last item again (same value, same place)
+    if (IMG) {
+      wDst[u] = x * 16;
+      wSrc[u] = W + (long long)split * T * (BUF_BYTES / 4) + x * 4;
+    } else {
+      const int kg = x / NW, tile = (x % NW) / 32, cc = x % 32;
+      int n = n0 + NT * cc + tile;
+      n = n < N ? n : N - 1; // (a column past the end is not stored)
+      wDst[u] = (kg / 2) * STEP_BYTES + tile * 1024 + (kg & 1) * 512 + cc * 16;
+      wSrc[u] = W + (long long)(8 * kg) * N + n;
+    }
+  }
+  auto w_load = [&](int slot, int t) {
+    t = t < T ? t : T - 1;
+#pragma unroll
+    for (int u = 0; u < WPER; ++u) {
+      if (IMG) {
+        const floatx4 v = *reinterpret_cast<const floatx4 *>(wSrc[u] + (long long)t * (BUF_BYTES / 4));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          wv[slot][u][i] = v[i];
+      } else {
+        const float *p = wSrc[u] + (long long)t * 32 * N;
+#pragma unroll
+        for (int i = 0; i < WREGS; ++i)
+          wv[slot][u][i] = p[(long long)i * N];
+      }
+    }
+  };
+  auto w_store = [&](int slot, int buf) {
+#pragma unroll
+    for (int u = 0; u < WPER; ++u) {
+      if constexpr (IMG) {
+        *reinterpret_cast<floatx4 *>(sW + buf * BUF_BYTES + wDst[u]) =
+            floatx4{wv[slot][u][0], wv[slot][u][1], wv[slot][u][2], wv[slot][u][3]};
+      } else {
+        bf16x8 p[PL];
+        split8<PL>(wv[slot][u], p);
+#pragma unroll
+        for (int l = 0; l < PL; ++l)
+          *reinterpret_cast<bf16x8 *>(sW + buf * BUF_BYTES + l * PLANE_BYTES + wDst[u]) = p[l];
+      }
+    }
+  };
+
+  // ---- A
+  const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
+  int *const sRules = reinterpret_cast<int *>(sW + 2 * BUF_BYTES);
+  const unsigned char *rowPtr[MT]; // this lane's rows at the filter position of the block to fetch
+  int fetchT = 0, f = 0, ch = 0;   // the block to fetch
+  auto aim = [&]() {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int rule = sRules[(wave * 32 * MT + 32 * i + c) * gs.fs + f];
+      rowPtr[i] = (rule >= 0 ? Ab + (long long)rule * gs.nIn * ES
+                             : reinterpret_cast<const unsigned char *>(gs.zeros)) + 8 * q * ES;
+    }
+  };
+  auto next_block = [&]() { // (past the last block: the last one again)
+    if (fetchT + 1 < T) {
+      ++fetchT;
+      ch += 32;
+      if (GATHER == 1 && ch == gs.nIn) {
+        ch = 0, ++f;
+        aim();
+      }
+    }
+  };
+  floatx4 raw[PD][UNITS][A16 ? 1 : 2];
+  auto a_load = [&](int slot, int u) {
+    if (GATHER == 2) {
+#pragma unroll
+      for (int h = 0; h < (A16 ? 1 : 2); ++h)
+        raw[slot][u][h] = gathered_piece<A16>(Ab, gs, sRules + (wave * 32 * MT + 32 * (u % MT) + c) * gs.fs,
+                                        ch + 16 * (u / MT) + 8 * q + 4 * h);
+      return;
+    }
+    const floatx4 *const p = reinterpret_cast<const floatx4 *>(rowPtr[u % MT] + (ch + 16 * (u / MT)) * ES);
+    raw[slot][u][0] = p[0];
+    if (!A16)
+      raw[slot][u][A16 ? 0 : 1] = p[1];
+  };
+  bf16x8 ap[2][PL]; // the unit in hand and the next one
+  auto a_split = [&](int slot, int u, int dst) {
+    if (A16) {
+      ap[dst][0] = __builtin_bit_cast(bf16x8, raw[slot][u][0]);
+    } else {
+      const floatx4 x = raw[slot][u][0], y = raw[slot][u][A16 ? 0 : 1];
+      const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+      split8<PL>(v, ap[dst]);
+    }
+  };
+
+  // ---- prologue
+#pragma unroll
+  for (int p = 0; p < PD; ++p)
+    w_load(p, p);
+  if (GATHER) {
+    const long long first = wgRow0 * gs.fs, last = M * gs.fs - 1;
+    for (int i = tid; i < ROWS * gs.fs; i += THREADS) {
+      const long long r = first + i;
+      sRules[i] = gs.rules[r < last ? r : last];
+    }
+    __syncthreads();
+    if (GATHER == 1)
+      aim();
+  } else {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      long long m = row0 + 32 * i + c;
+      m = m < M ? m : M - 1; // rows past the end: read a valid row, store nothing
+      rowPtr[i] = Ab + (m * K + 8 * q) * ES;
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PD; ++p) {
+    if (p)
+      next_block();
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u)
+      a_load(p, u);
+  }
+  w_store(0, 0);
+  __syncthreads();
+
+  constexpr int NACC = PL > 1 ? 2 : 1;
+  floatx16 acc[NACC][MT][NT];
+#pragma unroll
+  for (int h = 0; h < NACC; ++h)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[h][i][j][v] = 0.f;
+
+  const unsigned char *const wLane = sW + lane * 16;
+  constexpr int BB = NT == 1 ? 2 : 1; // a single tile has no other's MFMAs to be read under
+  bf16x8 b[BB][NT][PL];
+  int cur = 0;
+  auto read_b = [&](int buf, int s, int j) {
+#pragma unroll
+    for (int l = 0; l < PL; ++l)
+      b[s % BB][j][l] = *reinterpret_cast<const bf16x8 *>(wLane + buf * BUF_BYTES + l * PLANE_BYTES +
+                                                          s * STEP_BYTES + j * 1024);
+  };
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    read_b(0, 0, j);
+  a_split(0, 0, 0);
+
+  auto tile = [&](int s, int i, int j, int src) {
+    // products x y with x + y < PL: the largest terms of the product of the sums
+#pragma unroll
+    for (int x = 0; x < PL; ++x)
+#pragma unroll
+      for (int y = 0; x + y < PL; ++y) {
+        floatx16 &d = acc[x + y == 0 ? 0 : NACC - 1][i][j];
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[src][x], b[s % BB][j][y], d, 0, 0, 0);
+      }
+  };
+  auto deal = [&](int mfmas) {
+#pragma unroll
+    for (int i = 0; i < mfmas; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x320, 1, 0); // a load, an LDS read or write
+      __builtin_amdgcn_sched_group_barrier(0x002, 5, 0); // vector arithmetic
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int PRODUCTS = PL * (PL + 1) / 2;
+  auto block = [&](int p, bool firstOfAll) {
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int s = u / MT, i = u % MT, src = u & 1; // (UNITS is even)
+      // the next unit's operand; its registers then take a later block's
+      if (u + 1 < UNITS)
+        a_split(p, u + 1, src ^ 1);
+      else
+        a_split((p + 1) % PD, 0, src ^ 1);
+      if (u == 0) {
+        next_block();
+        a_load(p, 0); // (unit 0 was split a unit ago)
+      }
+      if (u + 1 < UNITS)
+        a_load(p, u + 1);
+      else
+        w_store((p + 1) % PD, cur ^ 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (u == UNITS - 1 && j == (NT > 1)) { // before the first read of the next block's W
+          if (NT > 1)
+            deal(PRODUCTS);
+          __syncthreads();
+          cur ^= 1;
+        }
+        // a tile's W is read as soon as its registers are free
+        if (NT == 1) {
+          if (i == MT - 1)
+            read_b(cur, s ^ 1, 0);
+        } else if (i == MT - 1 && j > 0) {
+          read_b(cur, s ^ 1, j - 1);
+        } else if (i == 0 && j == 0 && !(s == 0 && firstOfAll)) {
+          read_b(cur, s, NT - 1);
+        }
+        tile(s, i, j, src);
+      }
+      deal(u == UNITS - 1 && NT > 1 ? PRODUCTS * (NT - 1) : PRODUCTS * NT);
+    }
+  };
+  for (int t = 0; t < T; t += PD) {
+#pragma unroll
+    for (int p = 0; p < PD; ++p)
+      if (t + p < T) { // uniform
+        w_load(p, t + p + PD);
+        block(p, t + p == 0);
+      }
+  }
+
+  // ---- epilogue: register v of a tile is row 8 (v / 4) + 4 q + v % 4
+  const int n = n0 + NT * c;
+  ColEpilogue col[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    col[j] = load_col(ep, n + j < N ? n + j : N - 1);
+  const bool whole = n0 + NW <= N && N % NT == 0;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const long long r0 = row0 + 32 * i + 4 * q;
+    float *const o = out + r0 * N + n;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int dr = 8 * (v / 4) + v % 4;
+      if (r0 + dr >= M)
+        continue;
+      float r[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        r[j] = finish(NACC == 2 ? acc[0][i][j][v] + acc[NACC - 1][i][j][v] : acc[0][i][j][v], col[j]);
+      float *const orow = o + (long long)dr * N;
+      if (whole && NT == 4) {
+        *reinterpret_cast<float4 *>(orow) = make_float4(r[0], r[1 % NT], r[2 % NT], r[3 % NT]);
+      } else if (whole && NT == 2) {
+        *reinterpret_cast<float2 *>(orow) = make_float2(r[0], r[1 % NT]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (whole || n + j < N)
+            orow[j] = r[j];
+      }
+    }
+  }
+}
+
+// Few rows: a workgroup owns 32 rows x 32 columns and its eight wavefronts take
+// the blocks of 32 k in turn, so that a contraction of a few hundred k is one
+// or two trips to memory long, whatever it is wide: W comes straight from
+// global memory (no two wavefronts want the same piece of it), and the eight
+// partial tiles meet in LDS.
+template <int PL, bool GATHER, bool A16>
+__global__ void __launch_bounds__(512, 2)
+    k_nin_planes_splitk(const float *__restrict__ A, const float *__restrict__ W,
+                        float *__restrict__ out, long long M, int K, int N,
+                        Epilogue ep, GatherSource gs, int nSplits) {
+  constexpr int ES = A16 ? 2 : 4;
+  __shared__ __attribute__((aligned(16))) float sPart[8 * 16 * 64];
+  __shared__ int sRules[GATHER ? 32 * GF_MAX_FS : 1];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 31, q = lane >> 5;
+  const int split = blockIdx.x % nSplits;
+  const long long row0 = (long long)(blockIdx.x / nSplits) * 32;
+  const int n0 = split * 32;
+  const int T = K / 32;
+  const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
+  const int n = n0 + c < N ? n0 + c : N - 1; // (a column past the end is not stored)
+  const float *const wCol = W + (long long)(8 * q) * N + n;
+  struct Block {
+    floatx4 a[2][A16 ? 1 : 2];
+    float w[2][8];
+  };
+  long long m = row0 + c;
+  m = m < M ? m : M - 1; // rows past the end: read a valid row, store nothing
+  auto load_w = [&](Block &b, int t) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        b.w[s][i] = wCol[(long long)(32 * t + 16 * s + i) * N];
+  };
+  auto load_a = [&](Block &b, int t) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int h = 0; h < (A16 ? 1 : 2); ++h) {
+        const int k = 32 * t + 16 * s + 8 * q + 4 * h;
+        b.a[s][h] = GATHER ? gathered_piece<A16>(Ab, gs, sRules + c * gs.fs, k)
+                           : *reinterpret_cast<const floatx4 *>(Ab + (m * K + k) * ES);
+      }
+  };
+  constexpr int NACC = PL > 1 ? 2 : 1;
+  floatx16 acc[NACC];
+#pragma unroll
+  for (int h = 0; h < NACC; ++h)
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      acc[h][v] = 0.f;
+  auto compute = [&](const Block &b) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 ap[PL], bp[PL];
+      if constexpr (A16) {
+        ap[0] = __builtin_bit_cast(bf16x8, b.a[s][0]);
+      } else {
+        const floatx4 x = b.a[s][0], y = b.a[s][1];
+        const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+        split8<PL>(v, ap);
+      }
+      split8<PL>(b.w[s], bp);
+#pragma unroll
+      for (int x = 0; x < PL; ++x)
+#pragma unroll
+        for (int y = 0; x + y < PL; ++y) {
+          floatx16 &d = acc[x + y == 0 ? 0 : NACC - 1];
+          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[x], bp[y], d, 0, 0, 0);
+        }
+    }
+  };
+
+  Block b0, b1;
+  const int t0 = wave < T ? wave : T - 1;
+  load_w(b0, t0);
+  if (GATHER) {
+    const long long first = row0 * gs.fs, last = M * gs.fs - 1;
+    for (int i = tid; i < 32 * gs.fs; i += 512) {
+      const long long r = first + i;
+      sRules[i] = gs.rules[r < last ? r : last];
+    }
+    __syncthreads();
+  }
+  load_a(b0, t0);
+  for (int t = wave; t < T; t += 16) {
+    const int t1 = t + 8 < T ? t + 8 : T - 1;
+    load_w(b1, t1);
+    load_a(b1, t1);
+    compute(b0);
+    if (t + 8 >= T)
+      break;
+    const int t2 = t + 16 < T ? t + 16 : T - 1;
+    load_w(b0, t2);
+    load_a(b0, t2);
+    compute(b1);
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    sPart[(wave * 16 + v) * 64 + lane] = NACC == 2 ? acc[0][v] + acc[NACC - 1][v] : acc[0][v];
+  __syncthreads();
+  // register v of lane (c, q) is row 8 (v / 4) + 4 q + v % 4
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int v = 8 * h + wave;
+    const int dr = 8 * (v / 4) + 4 * q + v % 4;
+    if (row0 + dr >= M || n0 + c >= N)
+      continue;
+    float sum = sPart[v * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 8; ++w)
+      sum += sPart[(w * 16 + v) * 64 + lane];
+    out[(row0 + dr) * N + n0 + c] = finish(sum, load_col(ep, n0 + c));
+  }
+}
+
+// The image of W that the long contractions stream: for every slice of 32 NT
+// columns and every block of 32 k what w_store leaves in LDS, in that order.
+template <int PL, int NT>
+__global__ void __launch_bounds__(256)
+    k_planes_image(const float *__restrict__ W, unsigned char *__restrict__ image,
+                   int K, int N, int nSplits) {
+  constexpr int NW = 32 * NT, BUF_BYTES = PL * 2 * NT * 1024;
+  const int T = K / 32;
+  const long long item = (long long)blockIdx.x * 256 + threadIdx.x; // (slice, block, 8 k, column)
+  if (item >= (long long)nSplits * T * 4 * NW)
+    return;
+  const int x = (int)(item % (4 * NW));
+  const long long st = item / (4 * NW); // slice * T + block
+  const int t = (int)(st % T), split = (int)(st / T);
+  const int kg = x / NW, tile = (x % NW) / 32, cc = x % 32;
+  int n = split * NW + NT * cc + tile;
+  n = n < N ? n : N - 1;
+  const float *const src = W + (long long)(32 * t + 8 * kg) * N + n;
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    v[i] = src[(long long)i * N];
+  bf16x8 p[PL];
+  split8<PL>(v, p);
+#pragma unroll
+  for (int l = 0; l < PL; ++l)
+    *reinterpret_cast<bf16x8 *>(image + st * BUF_BYTES + l * 2 * NT * 1024 + (kg / 2) * NT * 1024 + tile * 1024 +
+                                (kg & 1) * 512 + cc * 16) = p[l];
+}
+
+// Room for an image: the context's from its first long contraction on.  Up to
+// four rooms of closed contexts are kept for the next ones (a new 16 MB costs
+// the first batch of a net half a millisecond) until the last context is gone.
+static struct {
+  std::mutex m;
+  int contexts = 0;
+  std::vector<std::pair<int, unsigned char *>> spare; // (device, room)
+} g_images;
+void scn_image_context(scn_ctx *ctx, bool alive) {
+  std::lock_guard<std::mutex> lock(g_images.m);
+  g_images.contexts += alive ? 1 : -1;
+  if (!alive && ctx->d_image) { // (its stream has been waited for)
+    if (g_images.spare.size() < 4)
+      g_images.spare.push_back({ctx->device, ctx->d_image});
+    else
+      (void)hipFree(ctx->d_image);
+    ctx->d_image = nullptr;
+  }
+  if (g_images.contexts == 0) {
+    for (auto &s : g_images.spare)
+      (void)hipFree(s.second);
+    g_images.spare.clear();
+  }
+}
+// False: convert on the way instead -- no memory, or the stream is being
+// captured and may not allocate.
+static bool planes_image(scn_ctx *ctx) {
+  if (ctx->d_image)
+    return true;
+  {
+    std::lock_guard<std::mutex> lock(g_images.m);
+    for (auto &s : g_images.spare)
+      if (s.first == ctx->device) {
+        ctx->d_image = s.second;
+        std::swap(s, g_images.spare.back());
+        g_images.spare.pop_back();
+        return true;
+      }
+  }
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess ||
+      capturing != hipStreamCaptureStatusNone ||
+      hipMalloc((void **)&ctx->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->d_image = nullptr;
+    return false;
+  }
+  return true;
+}
+
+// Blocks ahead: two where the registers allow it (a wavefront alone on its SIMD
+// waits for the trip to L2 in every block otherwise: one tile, three planes at
+// one workgroup a compute unit 0.79 -> 0.64 us a block; with three planes of
+// wider tiles it spills and loses).
+constexpr int planes_depth(int PL, int MT, int NT) {
+  return PL * MT * NT <= 4 || (PL < 3 && MT == 1) ? 2 : 1;
+}
+template <int PL, int MT, int NT, bool IMG, bool FINE = false>
+static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
+                         float *out, long long M, int K, int N,
+                         const Epilogue &ep, const GatherSource *gs, bool a16) {
+  const int nSplits = scn_ceil_div(N, 32 * NT);
+  const size_t lds = (size_t)2 * PL * 2 * NT * 1024 + (gs ? (size_t)128 * MT * gs->fs * 4 : 0);
+  constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
+  static OncePerDevice configured;
+  const int rc = configured.run(ctx->device, [&]() {
+    int rc = SCN_OK;
+#define SCN_PLANES_LDS(G, H)                                                   \
+  if (hipFuncSetAttribute(                                                     \
+          reinterpret_cast<const void *>(k_nin_planes<PL, MT, NT, PD, G, H, IMG>), \
+          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) \
+    rc = SCN_ERR_HIP;
+    SCN_PLANES_LDS(0, false) SCN_PLANES_LDS(G, false)
+    if (PL == 1)
+      SCN_PLANES_LDS(G, PL == 1)
+#undef SCN_PLANES_LDS
+    return rc;
+  });
+  SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  if (IMG) {
+    const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;
+    hipLaunchKernelGGL((k_planes_image<PL, NT>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream, W,
+                       ctx->d_image, K, N, nSplits);
+    W = reinterpret_cast<const float *>(ctx->d_image);
+  }
+  const dim3 grid((unsigned)(scn_ceil_div(M, 128 * MT) * (long long)nSplits));
+#define SCN_PLANES_GO(G, H, src)                                               \
+  hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, IMG>), grid,       \
+                     dim3(256), lds, ctx->stream, A, W, out, M, K, N,   \
+                     ep, src, nSplits)
+  if (!gs)
+    SCN_PLANES_GO(0, false, GatherSource());
+  else if (PL == 1 && a16)
+    SCN_PLANES_GO(G, PL == 1, *gs);
+  else
+    SCN_PLANES_GO(G, false, *gs);
+#undef SCN_PLANES_GO
+  return SCN_OK;
+}
+template <int PL>
+static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
+                         float *out, long long M, int K, int N,
+                         const Epilogue &ep, const GatherSource *gs, bool a16) {
+  const int nSplits = scn_ceil_div(N, 32);
+  const dim3 grid((unsigned)(scn_ceil_div(M, 32) * (long long)nSplits));
+#define SCN_SPLITK_GO(G, H, src)                                               \
+  hipLaunchKernelGGL((k_nin_planes_splitk<PL, G, H>), grid, dim3(512), 0,      \
+                     ctx->stream, A, W, out, M, K, N, ep, src, nSplits)
+  if (!gs)
+    SCN_SPLITK_GO(false, false, GatherSource());
+  else if (PL == 1 && a16)
+    SCN_SPLITK_GO(true, PL == 1, *gs);
+  else
+    SCN_SPLITK_GO(true, false, *gs);
+#undef SCN_SPLITK_GO
+  return SCN_OK;
+}
+
+bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
+
+// Which tile.  With n workgroups on every compute unit a block of 32 k takes tn
+// n microseconds, and no less than t1 (its chain: request, split, barrier); both
+// were measured on contractions of 256 and 1152 k at 256 to 2048 workgroups,
+// with W converted on the way and from its image.  A wavefront of two row tiles
+// and two column tiles (2, 2) is the fastest per flop (three planes: 232
+// TFLOP/s from the image, (1, 1) 173) and the first to leave the chip idle, so
+// the row count decides; every choice gives the same bits.  The start and the
+// stores of a workgroup cost by its tiles, the image 5 us.
+struct PlanesCost {
+  float t1, tn;
+};
+static const int planesTiles[4][2] = {{1, 1}, {1, 2}, {1, 3}, {2, 2}}; // row tiles, column tiles of a wavefront
+static const PlanesCost planesCost[2][4][2] = {
+    // one plane: converted, image
+    {{{.45f, .28f}, {.39f, .25f}}, {{.55f, .44f}, {.41f, .25f}}, {{.71f, .58f}, {.43f, .27f}}, {{.8f, .65f}, {.56f, .47f}}},
+    // three planes
+    {{{.64f, .46f}, {.54f, .39f}}, {{.96f, .72f}, {.95f, .64f}}, {{1.6f, 1.16f}, {1.23f, .99f}}, {{1.36f, 1.29f}, {1.22f, 1.16f}}}};
+
+struct PlanesChoice {
+  int tile; // index into planesTiles, -1: split contraction
+  bool image;
+};
+static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N) {
+  const int T = K / 32;
+  PlanesChoice best = {0, false};
+  float least = 1e30f;
+  for (int i = 0; i < 4; ++i) {
+    const int mt = planesTiles[i][0], nt = planesTiles[i][1];
+    const long long nSplits = scn_ceil_div(N, 32 * nt);
+    const float wgs = (float)(scn_ceil_div(M, 128 * mt) * nSplits) / ctx->numCU;
+    const float n = wgs <= 4.f ? ceilf(wgs) : wgs + .5f;
+    const int units = 4 * mt * nt;
+    for (int img = 0; img < 2; ++img) {
+      if (img && (size_t)nSplits * T * planes * 2 * nt * 1024 > SCN_IMAGE_BYTES)
+        continue;
+      const PlanesCost &c = planesCost[planes == 1 ? 0 : 1][i][img];
+      const float cost = T * fmaxf(c.t1, c.tn * n) + 3.f + units * (.2f + .17f * n) + (img ? 5.f : 0.f);
+      if (cost < least)
+        least = cost, best = {i, img != 0};
+    }
+  }
+  // The split contraction: one or two trips to memory while its workgroups are
+  // few; every 32 rows read the whole of W, out of L2 up to about 512 k.
+  const float wgs = (float)(scn_ceil_div(M, 32) * (long long)scn_ceil_div(N, 32)) / ctx->numCU;
+  const float splitk = fmaxf(3.f + .005f * K, 2.5f + wgs * ((planes == 1 ? 1.5f + .001f * K : 2.4f + .0027f * K) +
+                                                            (K > 512 ? .004f * (K - 512) : 0.f)));
+  if (splitk < least)
+    best = {-1, false};
+  return best;
+}
+bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
+  return planes_choose(ctx, planes, M, K, N).tile < 0;
+}
+
+template <int PL>
+static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
+                          float *out, long long M, int K, int N,
+                          const Epilogue &ep, const GatherSource *gs, bool a16) {
+  PlanesChoice choice = planes_choose(ctx, PL, M, K, N);
+  choice.image = choice.image && planes_image(ctx);
+  if (choice.tile < 0)
+    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16);
+  // (channels in other than 32s, seldom met: one tile)
+  if (gs && gs->nIn % 32 != 0)
+    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16);
+#define SCN_PLANES_CASE(I, MT, NT)                                             \
+  case I:                                                                      \
+    return choice.image ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16) \
+                        : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16);
+  switch (choice.tile) {
+    SCN_PLANES_CASE(0, 1, 1)
+    SCN_PLANES_CASE(1, 1, 2)
+    SCN_PLANES_CASE(2, 1, 3)
+    SCN_PLANES_CASE(3, 2, 2)
+  }
+#undef SCN_PLANES_CASE
+  return SCN_ERR_ARG;
+}
+
+int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
+                       float *out, long long M, int K, int N,
+                       const Epilogue &ep, const GatherSource *gs, bool a16) {
+  return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16)
+         : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16)
+                       : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16);
+}

@@ -269,6 +269,11 @@ static bool nin_shrunk(SpatiallySparseBatch &batch, int nFeaturesIn,
 }
 // the training branch of forwards() (NetworkInNetworkLayer.cu:165-184): no
 // scaling by the kept fraction, weights and bias of the features present
+// A layer at fp32 computes on three bf16 planes per operand: fp32 operands and
+// sums, at the rate of the bf16 matrix cores.
+static int abi_precision(int precision) {
+  return precision == SCN_FP32 ? SCN_FP32_PLANES : precision;
+}
 static void nin_forwards_shrunk(cudaMemStream &ms,
                                 SpatiallySparseBatchInterface &input,
                                 SpatiallySparseBatchInterface &output,
@@ -291,7 +296,7 @@ static void nin_forwards_shrunk(cudaMemStream &ms,
   SCN_CHECKED(scn_nin_forward(ms.ctx, input.sub->features.dPtr(), w.dPtr(),
                               b.dPtr(), PReLU ? PReLU->dPtr() : nullptr,
                               output.sub->features.dPtr(), output.nSpatialSites,
-                              Kp, Np, 1.0f, act, precision));
+                              Kp, Np, 1.0f, act, abi_precision(precision)));
   addMultiplyAdds((__int128_t)output.nSpatialSites * Kp * Np);
 }
 // When the preceding convolutional layer deferred its gather: run the fused
@@ -328,7 +333,7 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
   SCN_CHECKED(scn_conv_nin_forward_p(
       ms.ctx, src->sub->features.dPtr(), input.rules.dPtr(), fs, nIn, W.dPtr(),
       B.dPtr(), prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(),
-      output.nSpatialSites, nFeaturesOut, p, act, precision));
+      output.nSpatialSites, nFeaturesOut, p, act, abi_precision(precision)));
   return true;
 }
 
@@ -461,7 +466,7 @@ void NetworkInNetworkLayer::forwards(SpatiallySparseBatch &batch,
                                 W.dPtr(), B.dPtr(), nullptr,
                                 output.sub->features.dPtr(),
                                 output.nSpatialSites, nFeaturesIn, nFeaturesOut,
-                                p, (int)fn, precision));
+                                p, (int)fn, abi_precision(precision)));
   addMultiplyAdds((__int128_t)output.nSpatialSites * nFeaturesIn * nFeaturesOut);
 }
 void NetworkInNetworkLayer::backwards(SpatiallySparseBatch &batch,
@@ -592,7 +597,7 @@ void NetworkInNetworkPReLULayer::forwards(
                                 W.dPtr(), B.dPtr(), PReLU.dPtr(),
                                 output.sub->features.dPtr(),
                                 output.nSpatialSites, nFeaturesIn, nFeaturesOut,
-                                p, (int)PRELU, precision));
+                                p, (int)PRELU, abi_precision(precision)));
   addMultiplyAdds((__int128_t)output.nSpatialSites * nFeaturesIn * nFeaturesOut);
 }
 void NetworkInNetworkPReLULayer::backwards(

@@ -1,0 +1,56 @@
+"""The contraction on bf16 planes (SCN_FP32_PLANES, and SCN_FP32 where it goes there): every tile, the split
+contraction, the image of W, ragged rows and columns, fused with the gather and not."""
+import numpy as np
+import pytest
+
+import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows, fs, nIn, N): split contraction from one row on, N no multiple of a tile; every tile converted on the way,
+# a block more or less than a full group of rows; an odd number of blocks; channels looked up in fours; images
+@pytest.mark.parametrize("rows,fs,nIn,N", [(1, 4, 32, 32), (33, 3, 32, 100), (257, 9, 96, 36), (300, 4, 24, 64),
+                                           (20000, 4, 32, 64), (40001, 4, 32, 32), (66049, 3, 32, 96), (30000, 8, 12, 64),
+                                           (70001, 4, 64, 128), (65537, 27, 64, 64), (33005, 9, 96, 96)])
+@pytest.mark.parametrize("act", ["RELU", "PRELU"])
+def test_planes_against_float64(scn, ctx, rows, fs, nIn, N, act):
+    a = getattr(scn, act)
+    rng = np.random.default_rng(rows + fs + nIn + N)
+    nInRows, K = 500, fs * nIn
+    inp = (rng.standard_normal((nInRows, nIn)) * 10.0 ** rng.uniform(-3, 3, (nInRows, 1))).astype(np.float32)
+    rules = rng.integers(0, nInRows, (rows, fs)).astype(np.int32)
+    rules[rng.random((rows, fs)) < 0.1] = -1
+    W = (rng.standard_normal((K, N)) * np.sqrt(2.0 / K)).astype(np.float32)
+    B = rng.uniform(-0.5, 0.5, N).astype(np.float32)
+    pr = rng.uniform(0.1, 0.4, N).astype(np.float32)
+    d_in, d_rules, d_W, d_B, d_pr = (ctx.array(x) for x in (inp, rules, W, B, pr))
+    fused, two = ctx.array(np.full((rows, N), 7, np.float32)), ctx.array(np.full((rows, N), 7, np.float32))
+    print("planes", rows, fs, nIn, N, flush=True)
+    ctx.conv_nin_forward(d_in, d_rules, fs, nIn, d_W, d_B, d_pr, fused, rows, N, 1.0, a, scn.FP32_PLANES)
+    g = ctx.empty((rows, K), np.float32)
+    ctx.gather_rows(d_in, g, d_rules, rows * fs, nIn)
+    ctx.nin_forward(g, d_W, d_B, d_pr, two, rows, K, N, 1.0, a, scn.FP32_PLANES)
+    got = fused.download()
+    assert np.array_equal(got, two.download())
+    some = np.unique(np.concatenate([np.arange(min(rows, 300)), np.arange(max(0, rows - 300), rows)]))
+    A = np.where(rules[some, :, None] >= 0, inp[np.maximum(rules[some], 0)], 0).reshape(len(some), K).astype(np.float32)
+    want = orc.nin_forward(A, W, B, pr, 1.0, a, f64=True)
+    scale = np.abs(A).astype(np.float64) @ np.abs(W).astype(np.float64) + np.abs(B)
+    err = np.abs(got[some] - want) / scale
+    # products to 2^-25, one rounding of the sum every few k: within the plain fp32 accumulation's own error
+    plain = np.abs(orc.nin_forward(A, W, B, pr, 1.0, a) - want) / scale
+    assert err.max() <= 2e-6 and np.sqrt((err ** 2).mean()) <= np.sqrt((plain ** 2).mean()) + 1e-8
+
+
+def test_fp32_takes_the_planes_where_they_pay(scn, ctx):
+    """few rows and long contractions: the same bits as SCN_FP32_PLANES"""
+    rng = np.random.default_rng(5)
+    for M, K, N in ((100, 256, 64), (200000, 1728, 64)):
+        A = ctx.array(rng.standard_normal((M, K), dtype=np.float32))
+        W = ctx.array(rng.standard_normal((K, N), dtype=np.float32))
+        B = ctx.array(np.zeros(N, np.float32))
+        out = [ctx.empty((M, N), np.float32) for _ in range(2)]
+        for o, precision in zip(out, (scn.FP32, scn.FP32_PLANES)):
+            ctx.nin_forward(A, W, B, None, o, M, K, N, 1.0, scn.NOSIGMOID, precision)
+        assert np.array_equal(out[0].download(), out[1].download())
