@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
 // or two trips to memory long, whatever it is wide: W comes straight from
 // global memory (no two wavefronts want the same piece of it), and the eight
 // partial tiles meet in LDS.
-template <int PL, bool GATHER, bool A16>
+template <int PL, bool GATHER, bool A16, bool WT>
 __global__ void __launch_bounds__(512, 2)
     k_nin_planes_splitk(const float *__restrict__ A, const float *__restrict__ W,
                         float *__restrict__ out, long long M, int K, int N,
@@ -384,7 +384,7 @@ __global__ void __launch_bounds__(512, 2)
   const int T = K / 32;
   const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
   const int n = n0 + c < N ? n0 + c : N - 1; // (a column past the end is not stored)
-  const float *const wCol = W + (long long)(8 * q) * N + n;
+  const float *const wCol = WT ? W + (long long)n * K + 8 * q : W + (long long)(8 * q) * N + n;
   struct Block {
     floatx4 a[2][A16 ? 1 : 2];
     float w[2][8];
@@ -396,7 +396,7 @@ __global__ void __launch_bounds__(512, 2)
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        b.w[s][i] = wCol[(long long)(32 * t + 16 * s + i) * N];
+        b.w[s][i] = wCol[(long long)(32 * t + 16 * s + i) * (WT ? 1 : N)];
   };
   auto load_a = [&](Block &b, int t) {
 #pragma unroll
@@ -482,7 +482,8 @@ __global__ void __launch_bounds__(512, 2)
 
 // The image of W that the long contractions stream: for every slice of 32 NT
 // columns and every block of 32 k what w_store leaves in LDS, in that order.
-template <int PL, int NT>
+// WT: W is given as its transpose, [N x K].
+template <int PL, int NT, bool WT>
 __global__ void __launch_bounds__(256)
     k_planes_image(const float *__restrict__ W, unsigned char *__restrict__ image,
                    int K, int N, int nSplits) {
@@ -497,11 +498,11 @@ __global__ void __launch_bounds__(256)
   const int kg = x / NW, tile = (x % NW) / 32, cc = x % 32;
   int n = split * NW + NT * cc + tile;
   n = n < N ? n : N - 1;
-  const float *const src = W + (long long)(32 * t + 8 * kg) * N + n;
+  const float *const src = WT ? W + (long long)n * K + 32 * t + 8 * kg : W + (long long)(32 * t + 8 * kg) * N + n;
   float v[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    v[i] = src[(long long)i * N];
+    v[i] = src[WT ? i : (long long)i * N];
   bf16x8 p[PL];
   split8<PL>(v, p);
 #pragma unroll
@@ -570,7 +571,7 @@ constexpr int planes_depth(int PL, int MT, int NT) {
 template <int PL, int MT, int NT, bool IMG, bool FINE = false>
 static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
-                         const Epilogue &ep, const GatherSource *gs, bool a16) {
+                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT) {
   const int nSplits = scn_ceil_div(N, 32 * NT);
   const size_t lds = (size_t)2 * PL * 2 * NT * 1024 + (gs ? (size_t)128 * MT * gs->fs * 4 : 0);
   constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
@@ -591,8 +592,12 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
   SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
   if (IMG) {
     const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;
-    hipLaunchKernelGGL((k_planes_image<PL, NT>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream, W,
-                       ctx->d_image, K, N, nSplits);
+    if (PL == 3 && wT)
+      hipLaunchKernelGGL((k_planes_image<PL, NT, PL == 3>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream,
+                         W, ctx->d_image, K, N, nSplits);
+    else
+      hipLaunchKernelGGL((k_planes_image<PL, NT, false>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream, W,
+                         ctx->d_image, K, N, nSplits);
     W = reinterpret_cast<const float *>(ctx->d_image);
   }
   const dim3 grid((unsigned)(scn_ceil_div(M, 128 * MT) * (long long)nSplits));
@@ -612,18 +617,20 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
 template <int PL>
 static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
-                         const Epilogue &ep, const GatherSource *gs, bool a16) {
+                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT) {
   const int nSplits = scn_ceil_div(N, 32);
   const dim3 grid((unsigned)(scn_ceil_div(M, 32) * (long long)nSplits));
-#define SCN_SPLITK_GO(G, H, src)                                               \
-  hipLaunchKernelGGL((k_nin_planes_splitk<PL, G, H>), grid, dim3(512), 0,      \
+#define SCN_SPLITK_GO(G, H, T, src)                                            \
+  hipLaunchKernelGGL((k_nin_planes_splitk<PL, G, H, T>), grid, dim3(512), 0,   \
                      ctx->stream, A, W, out, M, K, N, ep, src, nSplits)
-  if (!gs)
-    SCN_SPLITK_GO(false, false, GatherSource());
+  if (PL == 3 && wT)
+    SCN_SPLITK_GO(false, false, PL == 3, GatherSource());
+  else if (!gs)
+    SCN_SPLITK_GO(false, false, false, GatherSource());
   else if (PL == 1 && a16)
-    SCN_SPLITK_GO(true, PL == 1, *gs);
+    SCN_SPLITK_GO(true, PL == 1, false, *gs);
   else
-    SCN_SPLITK_GO(true, false, *gs);
+    SCN_SPLITK_GO(true, false, false, *gs);
 #undef SCN_SPLITK_GO
   return SCN_OK;
 }
@@ -652,7 +659,8 @@ struct PlanesChoice {
   int tile; // index into planesTiles, -1: split contraction
   bool image;
 };
-static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N) {
+// needImage: of the tiles, only from the image
+static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool needImage = false) {
   const int T = K / 32;
   PlanesChoice best = {0, false};
   float least = 1e30f;
@@ -662,7 +670,7 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
     const float wgs = (float)(scn_ceil_div(M, 128 * mt) * nSplits) / ctx->numCU;
     const float n = wgs <= 4.f ? ceilf(wgs) : wgs + .5f;
     const int units = 4 * mt * nt;
-    for (int img = 0; img < 2; ++img) {
+    for (int img = needImage; img < 2; ++img) {
       if (img && (size_t)nSplits * T * planes * 2 * nt * 1024 > SCN_IMAGE_BYTES)
         continue;
       const PlanesCost &c = planesCost[planes == 1 ? 0 : 1][i][img];
@@ -687,18 +695,18 @@ bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
 template <int PL>
 static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
                           float *out, long long M, int K, int N,
-                          const Epilogue &ep, const GatherSource *gs, bool a16) {
-  PlanesChoice choice = planes_choose(ctx, PL, M, K, N);
-  choice.image = choice.image && planes_image(ctx);
+                          const Epilogue &ep, const GatherSource *gs, bool a16,
+                          const PlanesChoice &choice, bool wT = false) {
   if (choice.tile < 0)
-    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16);
+    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT);
   // (channels in other than 32s, seldom met: one tile)
   if (gs && gs->nIn % 32 != 0)
-    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16);
+    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false);
 #define SCN_PLANES_CASE(I, MT, NT)                                             \
   case I:                                                                      \
-    return choice.image ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16) \
-                        : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16);
+    return choice.image                                                        \
+               ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16, wT) \
+               : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16, false);
   switch (choice.tile) {
     SCN_PLANES_CASE(0, 1, 1)
     SCN_PLANES_CASE(1, 1, 2)
@@ -712,7 +720,244 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
                        const Epilogue &ep, const GatherSource *gs, bool a16) {
-  return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16)
-         : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16)
-                       : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16);
+  PlanesChoice choice = planes_choose(ctx, planes, M, K, N);
+  choice.image = choice.image && planes_image(ctx);
+  return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
+         : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
+                       : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16, choice);
+}
+
+// out = A Wt^T for Wt [N x K].  False: not a shape for it, or no room for the
+// image (nothing has been launched).
+bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
+                    long long M, int K, int N, const float *zeros, int *rc) {
+  if (!scn_planes_shape(K) || ((uintptr_t)A & 15) || ((uintptr_t)out & 15) || N % 4 != 0)
+    return false;
+  const PlanesChoice choice = planes_choose(ctx, 3, M, K, N, true);
+  if (choice.tile >= 0 && (!choice.image || !planes_image(ctx)))
+    return false;
+  Epilogue ep = Epilogue();
+  ep.bias = zeros;
+  ep.p = 1.f;
+  ep.act = SCN_NOSIGMOID;
+  *rc = planes_forward<3>(ctx, A, Wt, out, M, K, N, ep, nullptr, false, choice, true);
+  return true;
+}
+
+// ------------------------------------------------------- dW = A^T D in planes
+// The contraction runs over the rows of both matrices, so an MFMA operand is
+// eight consecutive rows of one column: dword loads (pairs of columns for two
+// tiles) that 32 lanes make of 32 neighbouring columns, whole lines, and no
+// turning in LDS.  A workgroup owns 32 MT x 32 NT of dW and a range of rows; its
+// eight wavefronts take sixteen rows each in turn and their sums meet in LDS.
+// The workgroups of one tile add to dW with float atomics, some 200 of which
+// retire in a nanosecond: few workgroups (one a compute unit), each with as many
+// rows as that leaves it.  29827 x 256 x 96 in 22 us (32 on the fp32 MFMA with
+// a thousand workgroups), 200000 x 1728 x 64 in 350 (470): the rate at which A
+// comes from HBM.
+#define ATB_STEP 16
+template <int MT, int NT>
+__global__ void __launch_bounds__(512, 2)
+    k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
+                 float *__restrict__ dW, long long M, int K, int N, int nTiles,
+                 long long rowsPerSplit) {
+  constexpr int PL = 3, GM = 8;
+  constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
+  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int c = lane & 31, q = lane >> 5;
+  const int k0 = (blockIdx.x / nTiles) * 32 * MT;
+  const int n0 = (blockIdx.x % nTiles) * 32 * NT;
+  const long long m0 = (long long)blockIdx.y * rowsPerSplit;
+  const long long m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
+  // this lane's columns (past the end: the last ones, not stored)
+  int ka = k0 + MT * c, na = n0 + NT * c;
+  ka = ka + MT <= K ? ka : K - MT;
+  na = na + NT <= N ? na : N - NT;
+  const unsigned offA = (unsigned)(8 * q) * K + ka, offD = (unsigned)(8 * q) * N + na;
+
+  struct Step {
+    float a[8][MT], d[8][NT];
+  };
+  auto load = [&](Step &s, long long m, bool guard) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float *pa, *pd;
+      if (guard) {
+        long long r = m + 8 * q + i;
+        r = r < m1 ? r : m1 - 1;
+        pa = A + r * K + ka;
+        pd = D + r * N + na;
+      } else {
+        pa = A + (m + i) * K + offA;
+        pd = D + (m + i) * N + offD;
+      }
+      if constexpr (MT == 2) {
+        const floatx2 v = *reinterpret_cast<const floatx2 *>(pa);
+        s.a[i][0] = v[0], s.a[i][1] = v[1];
+      } else {
+        s.a[i][0] = *pa;
+      }
+      if constexpr (NT == 2) {
+        const floatx2 v = *reinterpret_cast<const floatx2 *>(pd);
+        s.d[i][0] = v[0], s.d[i][1] = v[1];
+      } else {
+        s.d[i][0] = *pd;
+      }
+      if (guard && m + 8 * q + i >= m1) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          s.a[i][j] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          s.d[i][j] = 0.f;
+      }
+    }
+  };
+  floatx16 acc[2][MT][NT];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[h][i][j][v] = 0.f;
+  auto compute = [&](const Step &s) {
+    bf16x8 ap[MT][PL], dp[NT][PL];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const float v[8] = {s.a[0][i], s.a[1][i], s.a[2][i], s.a[3][i], s.a[4][i], s.a[5][i], s.a[6][i], s.a[7][i]};
+      split8<PL>(v, ap[i]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const float v[8] = {s.d[0][j], s.d[1][j], s.d[2][j], s.d[3][j], s.d[4][j], s.d[5][j], s.d[6][j], s.d[7][j]};
+      split8<PL>(v, dp[j]);
+    }
+#pragma unroll
+    for (int x = 0; x < PL; ++x)
+#pragma unroll
+      for (int y = 0; x + y < PL; ++y)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            floatx16 &d = acc[x + y == 0 ? 0 : 1][i][j];
+            d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[i][x], dp[j][y], d, 0, 0, 0);
+          }
+  };
+  const long long whole = m1 - ATB_STEP; // last start of a step without a guard
+  Step s0, s1;
+  long long m = m0 + ATB_STEP * wave; // a step in eight is this wavefront's
+  auto fetch = [&](Step &s, long long at) {
+    if (at <= whole)
+      load(s, at, false);
+    else
+      load(s, at < m1 ? at : m1 - 1, true);
+  };
+  if (m < m1) {
+    fetch(s0, m);
+    for (;;) {
+      const long long ma = m + ATB_STEP * GM;
+      if (ma < m1)
+        fetch(s1, ma);
+      compute(s0);
+      if (ma >= m1)
+        break;
+      const long long mb = ma + ATB_STEP * GM;
+      if (mb < m1)
+        fetch(s0, mb);
+      compute(s1);
+      if (mb >= m1)
+        break;
+      m = mb;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        sTile[wave * TILE + ((i * NT + j) * 16 + v) * 64 + lane] = acc[0][i][j][v] + acc[1][i][j][v];
+  __syncthreads();
+  // element e of the tile: register v of lane l of sub-tile (i, j): row (of dW)
+  // MT (8 (v / 4) + 4 (l / 32) + v % 4) + i, column NT (l % 32) + j
+  for (int e = tid; e < TILE; e += 512) {
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+      sum += sTile[g * TILE + e];
+    const int l = e & 63, v = (e >> 6) & 15, ij = e >> 10;
+    const int kk = k0 + MT * (8 * (v / 4) + 4 * (l >> 5) + v % 4) + ij / NT;
+    const int nn = n0 + NT * (l & 31) + ij % NT;
+    if (kk < K && nn < N)
+      unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
+  }
+}
+
+template <int MT, int NT>
+static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
+                      long long M, int K, int N, long long splits) {
+  const size_t lds = (size_t)8 * 32 * MT * 32 * NT * sizeof(float);
+  static OncePerDevice configured;
+  const int rc = configured.run(ctx->device, [&]() {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess
+               ? SCN_OK
+               : SCN_ERR_HIP;
+  });
+  SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  const int nTiles = scn_ceil_div(N, 32 * NT);
+  const long long tiles = (long long)scn_ceil_div(K, 32 * MT) * nTiles;
+  long long rows = (M + splits - 1) / splits;
+  rows = (rows + 8 * ATB_STEP - 1) / (8 * ATB_STEP) * (8 * ATB_STEP);
+  hipLaunchKernelGGL((k_atb_planes<MT, NT>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)), dim3(512),
+                     lds, ctx->stream, A, D, dW, M, K, N, nTiles, rows);
+  return SCN_OK;
+}
+
+// The tile and the number of row ranges that cost least: rounds of one workgroup
+// a compute unit, each `ti` microseconds for every 128 rows (two thirds of it
+// waiting for memory) and `f` to start, to sum and to store, and the atomics.
+// Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
+int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
+                   long long M, int K, int N) {
+  static const struct {
+    int mt, nt;
+    double ti, f;
+  } tile[] = {{1, 1, .8, 4.}, {2, 1, 1.13, 4.}, {1, 2, 1.13, 4.}, {2, 2, 1.95, 6.}};
+  int best = 0;
+  long long splits = 1;
+  double least = 1e300;
+  for (int i = 0; i < 4; ++i) {
+    if ((tile[i].mt == 2 && (K % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
+      continue;
+    const long long tiles = (long long)scn_ceil_div(K, 32 * tile[i].mt) * scn_ceil_div(N, 32 * tile[i].nt);
+    if (tiles > 0x7fffffffll)
+      continue;
+    const long long most = scn_ceil_div(M, 8 * ATB_STEP);
+    for (long long s = 1; s <= most && s <= 4096; s += s < 64 ? 1 : s / 32) {
+      const long long rounds = (tiles * s + ctx->numCU - 1) / ctx->numCU;
+      const long long steps = (M + s * 8 * ATB_STEP - 1) / (s * 8 * ATB_STEP);
+      const double cost = rounds * (steps * tile[i].ti + tile[i].f) +
+                          (double)tiles * s * tile[i].mt * tile[i].nt * 1024 / 2e5;
+      if (cost < least)
+        least = cost, best = i, splits = s;
+      if (rounds > 8)
+        break;
+    }
+  }
+  SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
+  switch (best) {
+  case 1:
+    return launch_atb<2, 1>(ctx, A, D, dW, M, K, N, splits);
+  case 2:
+    return launch_atb<1, 2>(ctx, A, D, dW, M, K, N, splits);
+  case 3:
+    return launch_atb<2, 2>(ctx, A, D, dW, M, K, N, splits);
+  }
+  return launch_atb<1, 1>(ctx, A, D, dW, M, K, N, splits);
 }

@@ -10,7 +10,7 @@
 //   max-pooling                dMaxPoolBackProp, MaxPoolingLayer.cu:74-82
 //   terminal pooling           dTerminalPoolBackProp, TerminalPoolingLayer.cu:48-62
 #include <mutex>
-#include "scn_common.h"
+#include "scn_nin_dev.h"
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -50,10 +50,10 @@ extern "C" int scn_softmax_grad(scn_ctx *ctx, const float *d_probs,
 // One pass over the [M x N] gradient: multiplies it in place by the
 // derivative of the activation (expressed through the layer's output, as the
 // reference does), and leaves the column sums of the result in db (the bias
-// gradient) and, for PReLU, the slope gradient in dprelu.  A workgroup covers
-// P columns (the power of two that covers min(N, 64)) with 256 / P lanes per
-// column, which interleave rows and take four of them per trip so that eight
-// loads are in flight per lane.
+// gradient) and, for PReLU, the slope gradient in dprelu.  A lane owns V
+// neighbouring columns (four where the rows are 16-byte aligned) and takes four
+// rows per trip, so that eight 16-byte loads are in flight; the lanes of a row
+// lie side by side, as many rows to a workgroup as fit.
 __device__ __forceinline__ float act_derivative(int act, float b, float d,
                                                 float alpha, float &t) {
   switch (act) {
@@ -73,52 +73,76 @@ __device__ __forceinline__ float act_derivative(int act, float b, float d,
     return d;
   }
 }
-__global__ __launch_bounds__(256) void k_act_backward(
+#define ACTB_THREADS 512
+template <int V>
+__global__ __launch_bounds__(ACTB_THREADS) void k_act_backward(
     const float *__restrict__ out, float *__restrict__ delta, long long M,
     int N, int act, const float *__restrict__ prelu, float *__restrict__ db,
     float *__restrict__ dprelu, int P) {
-  __shared__ float sS[256], sT[256];
-  const int tx = threadIdx.x % P, ty = threadIdx.x / P, lanesPerCol = 256 / P;
-  const int c = blockIdx.x * P + tx;
-  float s = 0.f, t = 0.f;
-  if (c < N) {
-    const float alpha = act == SCN_PRELU      ? prelu[c]
-                        : act == SCN_LEAKYRELU ? 0.01f
-                                               : 0.333f;
-    const long long step = (long long)lanesPerCol * gridDim.y;
-    long long r = (long long)blockIdx.y * lanesPerCol + ty;
+  typedef float vec __attribute__((ext_vector_type(V)));
+  __shared__ float sS[ACTB_THREADS * V], sT[ACTB_THREADS * V];
+  // P lanes a row, rows of lanes; lanes beyond the last whole row idle
+  const int rows = ACTB_THREADS / P;
+  const int tx = threadIdx.x % P, ty = threadIdx.x / P;
+  const int c = (blockIdx.x * P + tx) * V;
+  float s[V], t[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i)
+    s[i] = t[i] = 0.f;
+  if (c < N && ty < rows) {
+    float alpha[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      alpha[i] = act == SCN_PRELU ? prelu[c + i] : act == SCN_LEAKYRELU ? 0.01f : 0.333f;
+    const long long step = (long long)rows * gridDim.y;
+    long long r = (long long)blockIdx.y * rows + ty;
     for (; r + 3 * step < M; r += 4 * step) {
-      float b[4], d[4];
+      vec b[4], d[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        b[u] = out[(r + u * step) * N + c];
-        d[u] = delta[(r + u * step) * N + c];
+        b[u] = *reinterpret_cast<const vec *>(out + (r + u * step) * N + c);
+        d[u] = *reinterpret_cast<const vec *>(delta + (r + u * step) * N + c);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        d[u] = act_derivative(act, b[u], d[u], alpha, t);
-        delta[(r + u * step) * N + c] = d[u];
-        s += d[u];
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          d[u][i] = act_derivative(act, b[u][i], d[u][i], alpha[i], t[i]);
+          s[i] += d[u][i];
+        }
+        *reinterpret_cast<vec *>(delta + (r + u * step) * N + c) = d[u];
       }
     }
     for (; r < M; r += step) {
-      const float d = act_derivative(act, out[r * N + c], delta[r * N + c], alpha, t);
-      delta[r * N + c] = d;
-      s += d;
+      vec d = *reinterpret_cast<const vec *>(delta + r * N + c);
+      const vec b = *reinterpret_cast<const vec *>(out + r * N + c);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        d[i] = act_derivative(act, b[i], d[i], alpha[i], t[i]);
+        s[i] += d[i];
+      }
+      *reinterpret_cast<vec *>(delta + r * N + c) = d;
     }
   }
-  sS[threadIdx.x] = s;
-  sT[threadIdx.x] = t;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    sS[threadIdx.x * V + i] = s[i];
+    sT[threadIdx.x * V + i] = t[i];
+  }
   __syncthreads();
-  if (ty == 0 && c < N) {
-    s = 0.f, t = 0.f;
-    for (int k = 0; k < lanesPerCol; ++k) {
-      s += sS[k * P + tx];
-      t += sT[k * P + tx];
+  // column x of the workgroup's P V: the sum over its rows of lanes
+  for (int x = threadIdx.x; x < P * V; x += ACTB_THREADS) {
+    const int col = blockIdx.x * P * V + x;
+    if (col >= N)
+      continue;
+    float sum = 0.f, sumT = 0.f;
+    for (int k = 0; k < rows; ++k) {
+      sum += sS[k * P * V + x];
+      sumT += sT[k * P * V + x];
     }
-    unsafeAtomicAdd(db + c, s);
+    unsafeAtomicAdd(db + col, sum);
     if (act == SCN_PRELU)
-      unsafeAtomicAdd(dprelu + c, t);
+      unsafeAtomicAdd(dprelu + col, sumT);
   }
 }
 
@@ -144,22 +168,20 @@ static int activation_backward(scn_ctx *ctx, const float *d_out,
     return SCN_OK;
   SCN_REQUIRE(d_out && d_delta, SCN_ERR_ARG,
               "scn_activation_backward: null buffer");
-  int P = 1;
-  while (P < N && P < 64)
-    P <<= 1;
-  const int lanesPerCol = 256 / P;
-  int colBlocks = scn_ceil_div(N, P);
-  // every workgroup ends with one atomic per column onto the same N
-  // addresses, and those serialise (about 25 ns each): few, long-lived
-  // workgroups, two per compute unit
-  int rowBlocks = scn_ceil_div(M, 8 * lanesPerCol); // at least eight rows per lane
-  int cap = (ctx->numCU * 2 + colBlocks - 1) / colBlocks;
+  const int V = N % 4 == 0 && (((uintptr_t)d_out | (uintptr_t)d_delta) & 15) == 0 ? 4 : 1;
+  // (a row of up to 64 lanes: with fewer rows of lanes the sums below are short)
+  const int colBlocks = scn_ceil_div(N, V * 64);
+  const int P = scn_ceil_div(N / V, colBlocks);
+  // every workgroup ends with one atomic per column onto the same N addresses,
+  // and those serialise (about 25 ns each): few, long-lived workgroups, one per
+  // compute unit (60478 x 64: 11.4 -> 8.2 us)
+  const int rows = ACTB_THREADS / P;
+  int rowBlocks = scn_ceil_div(M, 4 * rows); // at least four rows per lane
+  const int cap = scn_ceil_div(ctx->numCU, colBlocks);
   if (rowBlocks > cap)
     rowBlocks = cap;
-  if (rowBlocks < 1)
-    rowBlocks = 1;
-  hipLaunchKernelGGL(k_act_backward, dim3(colBlocks, rowBlocks), dim3(256), 0,
-                     ctx->stream, d_out, d_delta, (long long)M, N, act,
+  hipLaunchKernelGGL((V == 4 ? k_act_backward<4> : k_act_backward<1>), dim3(colBlocks, rowBlocks),
+                     dim3(ACTB_THREADS), 0, ctx->stream, d_out, d_delta, (long long)M, N, act,
                      d_prelu, d_db, d_dprelu, P);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
@@ -181,218 +203,7 @@ extern "C" int scn_activation_backward_acc(scn_ctx *ctx, const float *d_out,
                              d_dprelu, false);
 }
 
-// ------------------------------------------------------- dW = A^T D (MFMA)
-// Output tile 64 (rows of dW = columns of A) x 64 (columns of D) per
-// workgroup, reduction over a range of the M rows; the row ranges of one tile
-// add their partial tiles into dW with float atomics.  A chunk of 32 rows of
-// both operands is staged in LDS (row pitch 80 words: the four row groups
-// that one v_mfma_f32_16x16x4_f32 operand read touches fall on disjoint
-// banks); wavefront w owns columns 16 w .. 16 w + 15 of the tile and all 64 of
-// its rows (four accumulator tiles).
-#define ATB_ROWS 32
-#define ATB_PITCH 80
-__global__ __launch_bounds__(256) void k_gemm_atb(
-    const float *__restrict__ A, const float *__restrict__ D,
-    float *__restrict__ dW, long long M, int K, int N, int nTiles,
-    long long rowsPerSplit) {
-  __shared__ float sA[ATB_ROWS * ATB_PITCH], sD[ATB_ROWS * ATB_PITCH];
-  const int k0 = (blockIdx.x / nTiles) * 64, n0 = (blockIdx.x % nTiles) * 64;
-  const long long m0 = (long long)blockIdx.y * rowsPerSplit;
-  const long long m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
-  const int t = threadIdx.x, col = t & 63, rg = t >> 6;
-  const int lane = t & 63, w = t >> 6, c = lane & 15, q = lane >> 4;
-  const bool aIn = k0 + col < K, dIn = n0 + col < N;
-  floatx4 acc[4];
-  for (int i = 0; i < 4; ++i)
-    acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // the next chunk's loads are in flight under this chunk's MFMAs
-  float ra[ATB_ROWS / 4], rd[ATB_ROWS / 4];
-  auto fetch = [&](long long m) {
-#pragma unroll
-    for (int i = 0; i < ATB_ROWS / 4; ++i) {
-      const long long row = m + rg + 4 * i;
-      const bool live = row < m1;
-      ra[i] = live && aIn ? A[row * K + k0 + col] : 0.f;
-      rd[i] = live && dIn ? D[row * N + n0 + col] : 0.f;
-    }
-  };
-  fetch(m0);
-  for (long long m = m0; m < m1; m += ATB_ROWS) {
-#pragma unroll
-    for (int i = 0; i < ATB_ROWS / 4; ++i) {
-      const int r = rg + 4 * i;
-      sA[r * ATB_PITCH + col] = ra[i];
-      sD[r * ATB_PITCH + col] = rd[i];
-    }
-    __syncthreads();
-    if (m + ATB_ROWS < m1)
-      fetch(m + ATB_ROWS);
-#pragma unroll
-    for (int s = 0; s < ATB_ROWS / 4; ++s) {
-      const float *pa = sA + (4 * s + q) * ATB_PITCH + c;
-      const float b = sD[(4 * s + q) * ATB_PITCH + 16 * w + c];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[16 * i], b, acc[i], 0,
-                                                      0, 0);
-    }
-    __syncthreads();
-  }
-  const int n = n0 + 16 * w + c;
-  if (n < N)
-    for (int i = 0; i < 4; ++i)
-      for (int v = 0; v < 4; ++v) {
-        const int k = k0 + 16 * i + 4 * q + v;
-        if (k < K)
-          unsafeAtomicAdd(dW + (long long)k * N + n, acc[i][v]);
-      }
-}
-
-// The same product for shapes that fill wider tiles (K and N multiples of 4,
-// 16-byte aligned operands).  WK x WN wavefronts per workgroup, 64 x 64 of
-// the output each: 16 accumulator tiles per wavefront fed by ONE 128-bit LDS
-// read per operand and k-step (lane (c, q) reads columns 4c..4c+3 of row
-// 4s + q, so MFMA tile i covers the output rows 4 * (its A-operand index) + i
-// and tile j the output columns 4c + j: 0.125 LDS reads per MFMA instead of
-// 1.25).  Chunks of 16 rows, double-buffered: the global loads of the next
-// chunk are in flight under the MFMAs of this one, one barrier per chunk.
-#define ATBW_ROWS 16
-template <int WK, int WN>
-__global__ __launch_bounds__(64 * WK * WN) void k_gemm_atb_wide(
-    const float *__restrict__ A, const float *__restrict__ D,
-    float *__restrict__ dW, long long M, int K, int N, int nTiles,
-    long long rowsPerSplit) {
-  constexpr int TK = 64 * WK, TN = 64 * WN, PA = TK + 16, PD = TN + 16;
-  constexpr int NT = 64 * WK * WN;
-  constexpr int LA = ATBW_ROWS * TK / 4 / NT; // float4 loads per lane, A
-  constexpr int LD = ATBW_ROWS * TN / 4 / NT; // ... and D
-  static_assert(LA * NT * 4 == ATBW_ROWS * TK && LD * NT * 4 == ATBW_ROWS * TN &&
-                    LD >= 1,
-                "chunk loads divide evenly");
-  __shared__ __align__(16) float sA[2][ATBW_ROWS * PA];
-  __shared__ __align__(16) float sD[2][ATBW_ROWS * PD];
-  const int k0 = (blockIdx.x / nTiles) * TK, n0 = (blockIdx.x % nTiles) * TN;
-  const long long m0 = (long long)blockIdx.y * rowsPerSplit;
-  const long long m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wk = wave / WN, wn = wave % WN, c = lane & 15, q = lane >> 4;
-  floatx4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float4 ra[LA], rd[LD];
-  auto fetch = [&](long long m) {
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      const int f = t + u * NT, r = f / (TK / 4), col = (f % (TK / 4)) * 4;
-      const long long row = m + r;
-      ra[u] = row < m1 && k0 + col < K
-                  ? *(const float4 *)(A + row * K + k0 + col)
-                  : float4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int u = 0; u < LD; ++u) {
-      const int f = t + u * NT, r = f / (TN / 4), col = (f % (TN / 4)) * 4;
-      const long long row = m + r;
-      rd[u] = row < m1 && n0 + col < N
-                  ? *(const float4 *)(D + row * N + n0 + col)
-                  : float4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      const int f = t + u * NT, r = f / (TK / 4), col = (f % (TK / 4)) * 4;
-      *(float4 *)(&sA[buf][r * PA + col]) = ra[u];
-    }
-#pragma unroll
-    for (int u = 0; u < LD; ++u) {
-      const int f = t + u * NT, r = f / (TN / 4), col = (f % (TN / 4)) * 4;
-      *(float4 *)(&sD[buf][r * PD + col]) = rd[u];
-    }
-  };
-  fetch(m0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (long long m = m0; m < m1; m += ATBW_ROWS, buf ^= 1) {
-    const bool more = m + ATBW_ROWS < m1;
-    if (more)
-      fetch(m + ATBW_ROWS);
-    const float *pa = &sA[buf][q * PA + wk * 64 + 4 * c];
-    const float *pd = &sD[buf][q * PD + wn * 64 + 4 * c];
-#pragma unroll
-    for (int s4 = 0; s4 < ATBW_ROWS / 4; ++s4) {
-      const float4 a = *(const float4 *)(pa + 4 * s4 * PA);
-      const float4 d = *(const float4 *)(pd + 4 * s4 * PD);
-      const float av[4] = {a.x, a.y, a.z, a.w}, dv[4] = {d.x, d.y, d.z, d.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], dv[j],
-                                                           acc[i][j], 0, 0, 0);
-    }
-    if (more)
-      stage(buf ^ 1);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int k = k0 + wk * 64 + 4 * (4 * q + v) + i;
-      if (k >= K)
-        continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = n0 + wn * 64 + 4 * c + j;
-        if (n < N)
-          unsafeAtomicAdd(dW + (long long)k * N + n, acc[i][j][v]);
-      }
-    }
-}
-
-template <int WK, int WN>
-static int launch_atb_wide(scn_ctx *ctx, const float *d_A, const float *d_D,
-                           float *d_dW, int64_t M, int K, int N) {
-  constexpr int TK = 64 * WK, TN = 64 * WN;
-  const int kTiles = scn_ceil_div(K, TK), nTiles = scn_ceil_div(N, TN);
-  const long long tiles = (long long)kTiles * nTiles;
-  // Row ranges: more of them shorten every workgroup's walk, but each adds
-  // one more tile of float atomics onto the same K x N addresses, and those
-  // serialise.  Measured on MI355X: a workgroup walks a row in about 60 ns
-  // (it waits for memory more than for the matrix cores; four of them share a
-  // compute unit), the part retires about 45 contended atomics per ns.  Take
-  // the count that minimises the sum.
-  const long long maxSplits = (M + 8 * ATBW_ROWS - 1) / (8 * ATBW_ROWS);
-  const double flushNs = (double)K * N / (double)tiles / 45.0;
-  long long splits = 1;
-  double best = 1e300;
-  for (long long cand = 1; cand <= maxSplits && cand <= 4096;
-       cand += cand < 16 ? 1 : cand / 8) {
-    const long long wgs = tiles * cand;
-    const long long rounds = (wgs + 4 * ctx->numCU - 1) / (4 * ctx->numCU);
-    const double cost = (double)rounds * ((double)M / cand) * 60.0 +
-                        (double)wgs * flushNs;
-    if (cost < best) {
-      best = cost;
-      splits = cand;
-    }
-  }
-  long long rowsPerSplit = (M + splits - 1) / splits;
-  rowsPerSplit = (rowsPerSplit + ATBW_ROWS - 1) / ATBW_ROWS * ATBW_ROWS;
-  splits = (M + rowsPerSplit - 1) / rowsPerSplit;
-  hipLaunchKernelGGL((k_gemm_atb_wide<WK, WN>),
-                     dim3((unsigned)tiles, (unsigned)splits),
-                     dim3(64 * WK * WN), 0, ctx->stream, d_A, d_D, d_dW,
-                     (long long)M, K, N, nTiles, rowsPerSplit);
-  SCN_HIP_CHECK(hipGetLastError());
-  return SCN_OK;
-}
-
+// ---------------------------------------------- dW = A^T D (scn_planes.hip)
 static int sgemm_AtB(scn_ctx *ctx, const float *d_A, const float *d_D,
                      float *d_dW, int64_t M, int K, int N, bool clear) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_sgemm_AtB: null context");
@@ -405,38 +216,7 @@ static int sgemm_AtB(scn_ctx *ctx, const float *d_A, const float *d_D,
   if (M == 0)
     return SCN_OK;
   SCN_REQUIRE(d_A && d_D, SCN_ERR_ARG, "scn_sgemm_AtB: null buffer");
-  // The wide tiles pay on long walks over the rows (measured: 200000 x 1728 x
-  // 64 and 100000 x 800 x 800 gain 20 %); up to some ten thousand rows, or with
-  // an output of a few tiles only, the narrow kernel's many short walks win.
-  if (K % 4 == 0 && N % 4 == 0 && N >= 48 && M >= 65536 &&
-      ((long long)K * N >= 160 * 1024 || (K >= 1024 && N >= 64)) &&
-      ((uintptr_t)d_A & 15) == 0 && ((uintptr_t)d_D & 15) == 0) {
-    // 256 x 64 or 128 x 128 tiles: whichever pads the output less
-    const long long pad41 = (long long)scn_ceil_div(K, 256) * 256 *
-                            scn_ceil_div(N, 64) * 64;
-    const long long pad22 = (long long)scn_ceil_div(K, 128) * 128 *
-                            scn_ceil_div(N, 128) * 128;
-    return pad41 < pad22 ? launch_atb_wide<4, 1>(ctx, d_A, d_D, d_dW, M, K, N)
-                         : launch_atb_wide<2, 2>(ctx, d_A, d_D, d_dW, M, K, N);
-  }
-  const int kTiles = scn_ceil_div(K, 64), nTiles = scn_ceil_div(N, 64);
-  const long long tiles = (long long)kTiles * nTiles;
-  SCN_REQUIRE(tiles <= 0x7fffffffll, SCN_ERR_CAPACITY,
-              "scn_sgemm_AtB: %lld tiles", tiles);
-  long long splits = (ctx->numCU * 4 + tiles - 1) / tiles;
-  const long long maxSplits = (M + 8 * ATB_ROWS - 1) / (8 * ATB_ROWS);
-  if (splits > maxSplits)
-    splits = maxSplits;
-  if (splits > 65535)
-    splits = 65535;
-  if (splits < 1)
-    splits = 1;
-  long long rowsPerSplit = (M + splits - 1) / splits;
-  rowsPerSplit = (rowsPerSplit + ATB_ROWS - 1) / ATB_ROWS * ATB_ROWS;
-  splits = (M + rowsPerSplit - 1) / rowsPerSplit;
-  hipLaunchKernelGGL(k_gemm_atb, dim3((unsigned)tiles, (unsigned)splits),
-                     dim3(256), 0, ctx->stream, d_A, d_D, d_dW, (long long)M, K,
-                     N, nTiles, rowsPerSplit);
+  SCN_TRY(scn_atb_planes(ctx, d_A, d_D, d_dW, (long long)M, K, N));
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
 }
@@ -485,6 +265,15 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
     return SCN_OK;
   SCN_REQUIRE(d_D && d_W && d_dA && d_workspace, SCN_ERR_ARG,
               "scn_sgemm_ABt: null buffer");
+  if (K <= SCN_ZERO_FLOATS) { // the planes read W [K x N] as it stands
+    int rc = SCN_OK;
+    ProfScope prof(ctx, SCN_K_BACKWARD);
+    if (scn_planes_abt(ctx, d_D, d_W, d_dA, (long long)M, N, K, ctx->d_zeros, &rc)) {
+      SCN_TRY(rc);
+      SCN_HIP_CHECK(hipGetLastError());
+      return SCN_OK;
+    }
+  }
   // the zero bias: the context's own zeros when they are enough of them
   float *Wt = d_workspace, *zeros = d_workspace + (size_t)N * K;
   {

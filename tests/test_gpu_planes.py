@@ -54,3 +54,38 @@ def test_fp32_takes_the_planes_where_they_pay(scn, ctx):
         for o, precision in zip(out, (scn.FP32, scn.FP32_PLANES)):
             ctx.nin_forward(A, W, B, None, o, M, K, N, 1.0, scn.NOSIGMOID, precision)
         assert np.array_equal(out[0].download(), out[1].download())
+
+
+# one row; fewer rows than a step; odd K or N (no pairs of columns); every tile; ragged row ranges
+@pytest.mark.parametrize("M,K,N", [(1, 32, 32), (15, 12, 32), (129, 27, 33), (130, 34, 31), (1000, 66, 100),
+                                   (40001, 12, 32), (30011, 256, 96), (5000, 128, 62), (70003, 432, 128)])
+def test_weight_gradient_and_input_gradient(scn, ctx, M, K, N):
+    rng = np.random.default_rng(M + K + N)
+    A, D = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((M, N), dtype=np.float32)
+    W, start = rng.standard_normal((K, N), dtype=np.float32), rng.standard_normal((K, N), dtype=np.float32)
+    dW = ctx.array(start)
+    print("products", M, K, N, flush=True)
+    ctx.sgemm_AtB(ctx.array(A), ctx.array(D), dW, M, K, N, accumulate=True)
+    scale = np.abs(A).astype(np.float64).T @ np.abs(D).astype(np.float64) + np.abs(start)
+    assert np.all(np.abs(dW.download() - start - A.astype(np.float64).T @ D) <= 2e-6 * scale)
+    dA = ctx.array(np.full((M, K), 7, np.float32))
+    ctx.sgemm_ABt(ctx.array(D), ctx.array(W), dA, M, N, K, ctx.empty(N * K + K, np.float32))
+    some = np.unique(np.concatenate([np.arange(min(M, 300)), np.arange(max(0, M - 300), M)]))
+    scale = np.abs(D[some]).astype(np.float64) @ np.abs(W).astype(np.float64).T
+    assert np.all(np.abs(dA.download()[some] - D[some].astype(np.float64) @ W.astype(np.float64).T) <= 2e-6 * scale)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (3, 4), (700, 260), (5001, 64), (9000, 37), (40000, 96)])
+@pytest.mark.parametrize("act", ["RELU", "PRELU"])
+def test_activation_backward_column_sums(scn, ctx, M, N, act):
+    rng = np.random.default_rng(M + N)
+    out, delta = (rng.standard_normal((M, N)).astype(np.float32) for _ in range(2))
+    pr = rng.uniform(0.1, 0.4, N).astype(np.float32)
+    d, db, dp = ctx.array(delta), ctx.array(np.zeros(N, np.float32)), ctx.array(np.zeros(N, np.float32))
+    ctx.activation_backward(ctx.array(out), d, M, N, getattr(scn, act), ctx.array(pr), db, dp)
+    want = np.where(out > 0, delta, delta * pr if act == "PRELU" else np.float32(0)).astype(np.float32)
+    assert np.array_equal(d.download(), want)
+    assert np.allclose(db.download(), want.astype(np.float64).sum(0), atol=2e-6 * M ** 0.5 * 4 + 1e-6, rtol=1e-5)
+    if act == "PRELU":
+        slope = np.where(out > 0, 0, delta * (out / pr)).astype(np.float64).sum(0)
+        assert np.allclose(dp.download(), slope, atol=1e-5 * M ** 0.5 * 4 + 1e-5, rtol=1e-4)
