@@ -203,6 +203,22 @@ int scn_rules_terminal_plan(scn_ctx *ctx, const scn_grids *in, scn_grids *out,
  * plans the batch again with deferral off (that also raises the bounds). */
 int scn_ctx_defer_counts(scn_ctx *ctx, int on);
 int scn_rules_settle(scn_ctx *ctx);
+/* The layers' kernels ahead of the counts.  Until it is called with null, the
+ * feature calls that follow on the context (scn_gather_rows, scn_nin_forward,
+ * scn_conv_nin_forward*, scn_maxpool*, scn_terminal_pool) take the number of
+ * their output rows, where it is still deferred, from `grids` on the device;
+ * their row argument (count, ruleWidth) is the bound that the plan returned.  So
+ * a forward pass can be queued behind its recorded plans without a wait between
+ * them; scn_rules_settle then waits for both, and where it returns
+ * SCN_ERR_CAPACITY the pass has computed nothing and is queued again.  A plan
+ * whose counts have to be settled first returns SCN_ERR_STATE (it was not part
+ * of recorded plans that overflow together); one that is settled is no matter. */
+int scn_ctx_rows_from(scn_ctx *ctx, const scn_grids *grids);
+/* After scn_rules_settle: whether the real counts would have chosen the kernels
+ * that a pass so queued was given.  0: another kernel would have rounded
+ * differently, and a caller that wants the bits of a pass with known counts
+ * queues it again. */
+int scn_ctx_rows_held(scn_ctx *ctx, int *held);
 /* Recorded plans.  gridRules runs per sample (ConvolutionalLayer.cu:114-118,
  * MaxPoolingLayer.cu:116-118) and the layers' preprocess() calls follow one
  * another without anything else in between (BatchProducer.cu:79-81).  With

@@ -95,6 +95,8 @@ def lib():
         "scn_ctx_chain_rules": (C.c_int, [vp, C.c_int]),
         "scn_ctx_chain_count": (C.c_int, [vp, P(i64), P(i64)]),
         "scn_rules_settle": (C.c_int, [vp]),
+        "scn_ctx_rows_from": (C.c_int, [vp, vp]),
+        "scn_ctx_rows_held": (C.c_int, [vp, P(C.c_int)]),
         "scn_grids_destroy": (C.c_int, [vp, vp]),
         "scn_grids_build": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_int, vp, vp, vp, i64, vp, i32]),
         "scn_grids_info": (C.c_int, [vp, P(C.c_int), P(C.c_int), P(C.c_int), P(i64), P(i32)]),

@@ -1208,6 +1208,7 @@ static void chain_mark_output(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   out->tableValid = false;
   out->indexValid = false;
   out->chained = true;
+  out->atOnce = false;
   out->planIn = in;
   mark_pending(ctx, out, slot);
 }
@@ -1432,6 +1433,8 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   cs->pyrAtMax = ldsB >= PYR_LDS_MAX;
   *done = true;
   cs->nPyramids += 1;
+  for (const ChainRec &r : recs)
+    r.out->atOnce = true;
   SCN_TRY(scn_grids_ensure_table(ctx, src)); // pass B reads the source's rows through it
   a.table = src->table.p;
   a.dense = (long long)src->batch * src->vol <= SCN_DENSE_MAX_SITES ? src->dense.p : nullptr;

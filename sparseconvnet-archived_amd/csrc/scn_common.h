@@ -33,6 +33,9 @@ void scn_set_error(const char *fmt, ...);
       return rc_;                                                              \
   } while (0)
 
+// words of a plan's counts on the device (scn_grids::meta)
+enum { META_SITES = 0, META_ACTIVE = 1, META_OVERFLOW = 2, META_WIDTH = 3 };
+
 struct ProfSpan {
   int family;
   int tag;
@@ -58,6 +61,19 @@ struct scn_ctx {
   // their way; slot i of them reports into h_pinned[16 + 4 i ..]
   bool deferCounts;
   std::vector<struct scn_grids *> pendingGrids;
+  // scn_ctx_rows_from: where the feature kernels read their number of rows
+  // (META_* words of the grids), the bound they were launched with, and the
+  // pinned slot that holds the same once the stream is through
+  const long long *d_meta;
+  long long rowsBound, rowsHint; // (hint: what they are likely to be)
+  int rowsSlot;
+  // the kernels chosen meanwhile are those for above < rows <= upTo
+  struct RowsChosen {
+    int slot;
+    long long above, upTo;
+  };
+  std::vector<RowsChosen> rowsChosen;
+  bool rowsHeld;
   struct ChainState *chain; // recorded rule-book plans (scn_chain.hip)
   // profiling
   bool prof;
@@ -116,6 +132,28 @@ void scn_abt_static_forget(const scn_ctx *ctx);
 
 // counts contexts, and takes back ctx's image when one goes (scn_planes.hip)
 void scn_image_context(scn_ctx *ctx, bool alive);
+
+// For a feature call that can not read its rows on the device: waits for the
+// stream and replaces the bound M by the rows there are (per: rows of the call
+// for each of the grids' rows).
+int scn_rows_exact(scn_ctx *ctx, int64_t *M);
+// The number of rows by which a call chooses its kernel ...
+static inline long long scn_rows_hint(const scn_ctx *ctx, long long M) {
+  return ctx->d_meta && ctx->rowsHint < M ? ctx->rowsHint : M;
+}
+// ... and the numbers for which another choice would have given other roundings:
+// kept until the counts are settled.
+static inline void scn_rows_chosen(scn_ctx *ctx, long long above, long long upTo) {
+  if (ctx->d_meta)
+    ctx->rowsChosen.push_back({ctx->rowsSlot, above, upTo});
+}
+// what a kernel does with the bound it was launched with
+__device__ __forceinline__ long long live_rows(long long bound, const long long *d_rows) {
+  if (!d_rows)
+    return bound;
+  const long long n = *d_rows;
+  return n < bound ? n : bound;
+}
 
 // runs the recorded rule-book plans of the context, if any (scn_chain.hip)
 int scn_chain_flush(scn_ctx *ctx);

@@ -33,6 +33,8 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   c->ticket = 0;
   c->deferCounts = false;
   c->chain = nullptr;
+  c->d_meta = nullptr;
+  c->rowsHeld = true;
   c->d_image = nullptr;
   memset(c->profMs, 0, sizeof(c->profMs));
   memset(c->profCalls, 0, sizeof(c->profCalls));

@@ -15,7 +15,9 @@ template <typename VecT, int VEC>
 __global__ void __launch_bounds__(GATHER_THREADS)
     k_gather(const float *__restrict__ in, float *__restrict__ out,
              const int *__restrict__ rules, long long count, int nIn,
-             int chunks) {
+             int chunks, const long long *dRows, int perRow) {
+  if (dRows)
+    count = live_rows(count / perRow, dRows) * perRow;
   __shared__ long long roff[GATHER_TILE];
   const int tid = threadIdx.x;
   const int q0 = tid / chunks, ch0 = tid - q0 * chunks;
@@ -81,17 +83,20 @@ extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
   SCN_REQUIRE(d_in && d_out && d_rules, SCN_ERR_ARG,
               "scn_gather_rows: null buffer");
   ProfScope ps(ctx, SCN_K_GATHER);
+  // (rows not known on the host yet: count is their bound times the rule width)
+  const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
+  const int perRow = dRows && ctx->rowsBound > 0 ? (int)(count / ctx->rowsBound) : 1;
   long long tiles = (count + GATHER_TILE - 1) / GATHER_TILE;
   long long maxBlocks = (long long)ctx->numCU * 16;
   int blocks = (int)(tiles < maxBlocks ? tiles : maxBlocks);
   if (nIn % 4 == 0 && aligned16(d_in) && aligned16(d_out)) {
     hipLaunchKernelGGL((k_gather<float4, 4>), dim3(blocks),
                        dim3(GATHER_THREADS), 0, ctx->stream, d_in, d_out,
-                       d_rules, (long long)count, nIn, nIn / 4);
+                       d_rules, (long long)count, nIn, nIn / 4, dRows, perRow);
   } else {
     hipLaunchKernelGGL((k_gather<float, 1>), dim3(blocks),
                        dim3(GATHER_THREADS), 0, ctx->stream, d_in, d_out,
-                       d_rules, (long long)count, nIn, nIn);
+                       d_rules, (long long)count, nIn, nIn, dRows, perRow);
   }
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
@@ -104,8 +109,9 @@ __global__ void __launch_bounds__(256)
     k_maxpool(const float *__restrict__ in, float *__restrict__ out,
               const int *__restrict__ rules, long long nOutSites, int ps,
               int C, int chunks, int *__restrict__ choice,
-              const float *__restrict__ spare) {
+              const float *__restrict__ spare, const long long *dRows) {
   long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  nOutSites = live_rows(nOutSites, dRows);
   if (idx >= nOutSites * chunks)
     return;
   long long r = idx / chunks;
@@ -186,18 +192,19 @@ extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
   SCN_REQUIRE(d_out && d_rules && d_choice, SCN_ERR_ARG,
               "scn_maxpool: null buffer");
   ProfScope prof(ctx, SCN_K_MAXPOOL);
+  const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   if (C % 4 == 0 && aligned16(d_in) && aligned16(d_out) && aligned16(d_choice)) {
     long long total = nOutSites * (C / 4);
     hipLaunchKernelGGL(k_maxpool<4>, dim3(scn_ceil_div(total, 256)), dim3(256),
                        0, ctx->stream, d_in, d_out, d_rules,
                        (long long)nOutSites, ps, C, C / 4, d_choice,
-                       (const float *)ctx->d_zeros);
+                       (const float *)ctx->d_zeros, dRows);
   } else {
     long long total = nOutSites * C;
     hipLaunchKernelGGL(k_maxpool<1>, dim3(scn_ceil_div(total, 256)), dim3(256),
                        0, ctx->stream, d_in, d_out, d_rules,
                        (long long)nOutSites, ps, C, C, d_choice,
-                       (const float *)ctx->d_zeros);
+                       (const float *)ctx->d_zeros, dRows);
   }
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
@@ -221,7 +228,10 @@ extern "C" int scn_maxpool_checked(scn_ctx *ctx, const float *d_in,
 __global__ void k_terminal_pool(const float *__restrict__ in,
                                 float *__restrict__ out,
                                 const int *__restrict__ rules, long long count,
-                                int S, int C, const float *__restrict__ spare) {
+                                int S, int C, const float *__restrict__ spare,
+                                const long long *meta) {
+  if (meta) // (the width is a bound, the rows lie at the true one)
+    S = meta[META_OVERFLOW] ? 0 : (int)(meta[META_WIDTH] < S ? meta[META_WIDTH] : S);
   long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= count * C)
     return;
@@ -270,7 +280,8 @@ extern "C" int scn_terminal_pool(scn_ctx *ctx, const float *d_in, float *d_out,
   ProfScope prof(ctx, SCN_K_TERMINAL);
   hipLaunchKernelGGL(k_terminal_pool, dim3(scn_ceil_div(count * C, 256)),
                      dim3(256), 0, ctx->stream, d_in, d_out, d_rules,
-                     (long long)count, S, C, (const float *)ctx->d_zeros);
+                     (long long)count, S, C, (const float *)ctx->d_zeros,
+                     ctx->d_meta);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
 }

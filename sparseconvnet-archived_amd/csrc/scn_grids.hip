@@ -1236,6 +1236,7 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
   g->tableValid = withTable;
   g->indexValid = true;
   g->chained = false;
+  g->atOnce = false;
   g->planKind = PLAN_NONE;
   g->planIn = nullptr;
   g->pending = false;
@@ -1528,6 +1529,12 @@ extern "C" int scn_rules_settle(scn_ctx *ctx) {
   SCN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   std::atomic_thread_fence(std::memory_order_acquire);
   bool overflowed = false;
+  ctx->rowsHeld = true;
+  for (const auto &c : ctx->rowsChosen) {
+    const volatile int64_t *slot = ctx->h_pinned + 16 + 4 * c.slot;
+    ctx->rowsHeld = ctx->rowsHeld && slot[0] > c.above && slot[0] <= c.upTo;
+  }
+  ctx->rowsChosen.clear();
   for (scn_grids *g : ctx->pendingGrids) {
     const volatile int64_t *slot = ctx->h_pinned + 16 + 4 * g->pinnedSlot;
     if (g->chained)
@@ -1541,6 +1548,8 @@ extern "C" int scn_rules_settle(scn_ctx *ctx) {
       g->nSites = (int)slot[0];
       g->nActive = slot[1];
       g->seenRows = slot[0] > g->seenRows ? slot[0] : g->seenRows;
+      g->lastRows = slot[0];
+      g->lastBatch = g->batch;
       g->seenActive = slot[1] > g->seenActive ? slot[1] : g->seenActive;
       if (g->planKind == PLAN_TERMINAL) {
         g->termS = slot[3];
@@ -1561,6 +1570,33 @@ extern "C" int scn_rules_settle(scn_ctx *ctx) {
   SCN_REQUIRE(!overflowed, SCN_ERR_CAPACITY,
               "scn_rules_settle: a batch outgrew the bounds of its deferred "
               "plans; plan it again with deferral off");
+  return SCN_OK;
+}
+extern "C" int scn_ctx_rows_from(scn_ctx *ctx, const scn_grids *g) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_ctx_rows_from: null context");
+  ctx->d_meta = nullptr;
+  if (!g || !g->pending)
+    return SCN_OK;
+  SCN_TRY(scn_chain_flush(ctx));
+  SCN_REQUIRE(g->atOnce, SCN_ERR_STATE, "scn_ctx_rows_from: the counts of this plan have to be settled first");
+  ctx->d_meta = g->meta.p;
+  ctx->rowsBound = g->nSites;
+  ctx->rowsHint = g->lastBatch > 0 ? g->lastRows * g->batch / g->lastBatch : g->nSites;
+  ctx->rowsSlot = g->pinnedSlot;
+  return SCN_OK;
+}
+extern "C" int scn_ctx_rows_held(scn_ctx *ctx, int *held) {
+  SCN_REQUIRE(ctx && held, SCN_ERR_ARG, "scn_ctx_rows_held: null argument");
+  *held = ctx->rowsHeld;
+  return SCN_OK;
+}
+int scn_rows_exact(scn_ctx *ctx, int64_t *M) {
+  SCN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+  std::atomic_thread_fence(std::memory_order_acquire);
+  const volatile int64_t *slot = ctx->h_pinned + 16 + 4 * ctx->rowsSlot;
+  const int64_t rows = slot[2] ? 0 : slot[0];
+  ctx->rowsHint = rows;
+  *M = rows < *M ? rows : *M;
   return SCN_OK;
 }
 void mark_pending(scn_ctx *ctx, scn_grids *g, int slot) {

@@ -84,7 +84,6 @@ static inline unsigned xcd_grid(long long blocks) {
   return (unsigned)((blocks + 7) / 8 * 8);
 }
 // per-grids device record
-enum { META_SITES = 0, META_ACTIVE = 1, META_OVERFLOW = 2, META_WIDTH = 3 };
 
 struct scn_grids {
   int batch = 0, d = 0, n = 0;
@@ -106,6 +105,7 @@ struct scn_grids {
   bool rankRowValid = false;
   bool tableValid = false;
   bool indexValid = true;
+  bool atOnce = false; // ... and all of its plans overflow together or not at all
   bool chained = false; // plan and rules came from a chain of recorded plans
   long long seenSample = 0; // most active sites one sample has had (chained plans)
   // how much of table / bits is known to be empty right now (scn_grids_clear_many)
@@ -117,6 +117,8 @@ struct scn_grids {
   bool pending = false;
   int pinnedSlot = -1;
   long long seenRows = 0, seenActive = 0, seenWidth = 0;
+  // the last settled plan, to guess the next one by
+  long long lastRows = 0, lastBatch = 0;
   DevBuf<long long> meta; // META_* words
   DevBuf<Slot> table;
   DevBuf<int> dense;

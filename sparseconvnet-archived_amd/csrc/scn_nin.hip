@@ -132,7 +132,10 @@ template <int NB, bool SOFTMAX>
 __global__ void __launch_bounds__(FR_THREADS)
     k_nin_fewrows(const float *__restrict__ A, const float *__restrict__ W,
                   float *__restrict__ out, long long M, int K, int N,
-                  Epilogue ep, GatherSource gs, bool gather) {
+                  Epilogue ep, GatherSource gs, bool gather, const long long *dRows) {
+  M = live_rows(M, dRows);
+  if ((long long)blockIdx.x * FR_ROWS >= M)
+    return;
   __shared__ float sA[FR_ROWS * FR_MAX_K];
   __shared__ float part[FR_WAVES][FR_ROWS][64 * NB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -275,8 +278,12 @@ __global__ void __launch_bounds__(FR_THREADS)
 #define TK_MAX_K 32
 __global__ void __launch_bounds__(256)
     k_nin_thin(const float *__restrict__ A, const float *__restrict__ W,
-               float *__restrict__ out, long long M, int K, int N, Epilogue ep) {
+               float *__restrict__ out, long long M, int K, int N, Epilogue ep,
+               const long long *dRows) {
   __shared__ __attribute__((aligned(16))) float sW[TK_MAX_K * 32];
+  M = live_rows(M, dRows);
+  if ((long long)blockIdx.x * 32 >= M)
+    return;
   const int tid = threadIdx.x;
   const int n0 = blockIdx.y * 32;
   for (int x = tid; x < K * 32; x += 256) {
@@ -325,7 +332,10 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(256)
     k_conv_thin(const float *__restrict__ A, const float *__restrict__ W,
                 float *__restrict__ out, long long M, int K, int N, Epilogue ep,
-                GatherSource gs) {
+                GatherSource gs, const long long *dRows) {
+  M = live_rows(M, dRows);
+  if ((long long)blockIdx.x * (32 * CT_GROUPS) >= M)
+    return;
   // LDS: the gathered rows, then this workgroup's columns of W at pitch wp
   extern __shared__ __attribute__((aligned(16))) float ctLds[];
   float *const sA = ctLds;
@@ -1624,13 +1634,32 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   bool softmaxDone = false;
   const bool vec = K % 4 == 0 && N % 4 == 0 && ((uintptr_t)d_A & 15) == 0 &&
                    ((uintptr_t)d_W & 15) == 0 && ((uintptr_t)d_out & 15) == 0;
+  // the kernels of ordinary layers read their number of rows on the device
+  // where the host does not know it yet; the others are told here
+  const long long *const dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
+  const bool rounded = precision == SCN_BF16 || precision == SCN_BF16X3; // operands
+  const bool shape = vec && scn_planes_shape(K);
+  const bool few = K <= FR_MAX_K && !(shape && N % 16 == 0);
+  bool fewRows = few && scn_rows_hint(ctx, M) <= FR_MAX_M;
+  const bool planes = shape && ((rounded && act != SCN_SOFTMAX) || precision == SCN_FP32_PLANES ||
+                                2e0 * M * K * N >= PLANES_MIN_FLOPS || scn_planes_splitk(ctx, 3, M, K, N));
+  const bool tiledBf16 = vec && K >= 64 && act != SCN_SOFTMAX && rounded && !planes;
+  if (dRows && (precision == SCN_FP32 || act == SCN_TANH || act == SCN_SIGMOID ||
+                (act == SCN_SOFTMAX && !(fewRows && N <= 128)) || tiledBf16 || !(planes || fewRows || (vec && (gs ? gs->nIn % 4 != 0 : K <= TK_MAX_K))))) {
+    SCN_TRY(scn_rows_exact(ctx, &M));
+    if (M == 0)
+      return SCN_OK;
+    fewRows = few && M <= FR_MAX_M;
+  }
+  if (few && !(planes && rounded))
+    scn_rows_chosen(ctx, fewRows ? -1 : FR_MAX_M, fewRows ? FR_MAX_M : 1ll << 62);
   // bf16 operands only where the contraction is big enough to matter; the
   // classifier head and the thin first layers stay fp32
-  if (vec && act != SCN_SOFTMAX && (precision == SCN_BF16 || precision == SCN_BF16X3) && scn_planes_shape(K)) {
+  if (planes && rounded && act != SCN_SOFTMAX) {
     const bool a16 = precision == SCN_BF16 && rows16 && gs && gs->nIn % 8 == 0 && ((uintptr_t)rows16 & 15) == 0;
     SCN_TRY(scn_planes_forward(ctx, precision == SCN_BF16 ? 1 : 2, a16 ? (const float *)rows16 : d_A, d_W, d_out, M,
                                K, N, ep, gs, a16));
-  } else if (vec && K >= 64 && act != SCN_SOFTMAX && (precision == SCN_BF16 || precision == SCN_BF16X3)) {
+  } else if (tiledBf16) {
     SCN_REQUIRE(!gs, SCN_ERR_ARG,
                 "fused convolution: shape outside the bf16 kernel's range");
     const bool split = precision == SCN_BF16X3;
@@ -1641,7 +1670,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
       launch_mfma_bf16<4, 1, 2>(ctx, d_A, d_W, d_out, M, K, N, ep, split);
     else
       launch_mfma_bf16<1, 4, 1>(ctx, d_A, d_W, d_out, M, K, N, ep, split);
-  } else if (M <= FR_MAX_M && K <= FR_MAX_K && !(vec && scn_planes_shape(K) && N % 16 == 0)) {
+  } else if (fewRows) {
     // (the classifier's head, whose soft-max rides along, and what the planes do not take)
     GatherSource none = GatherSource();
     if (act == SCN_SOFTMAX && N <= 128) {
@@ -1649,25 +1678,24 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
       softmaxDone = true;
       hipLaunchKernelGGL((k_nin_fewrows<2, true>), dim3(scn_ceil_div(M, FR_ROWS), 1),
                          dim3(FR_THREADS), 0, ctx->stream, d_A, d_W, d_out,
-                         (long long)M, K, N, ep, gs ? *gs : none, gs != nullptr);
+                         (long long)M, K, N, ep, gs ? *gs : none, gs != nullptr, dRows);
     } else {
       hipLaunchKernelGGL((k_nin_fewrows<1, false>),
                          dim3(scn_ceil_div(M, FR_ROWS), scn_ceil_div(N, 64)),
                          dim3(FR_THREADS), 0, ctx->stream, d_A, d_W, d_out,
-                         (long long)M, K, N, ep, gs ? *gs : none, gs != nullptr);
+                         (long long)M, K, N, ep, gs ? *gs : none, gs != nullptr, dRows);
     }
   } else if (vec && gs && gs->nIn % 4 != 0) {
     // channels in other than fours: K <= TK_MAX_K (scn_conv_nin_supported)
     const size_t lds = (size_t)(CT_GROUPS * 32 * TK_MAX_K + K * (N < CT_COLS ? N : CT_COLS)) * sizeof(float);
     hipLaunchKernelGGL(k_conv_thin, dim3(scn_ceil_div(M, 32 * CT_GROUPS), scn_ceil_div(N, CT_COLS)),
                        dim3(256), lds, ctx->stream, d_A, d_W, d_out, (long long)M,
-                       K, N, ep, *gs);
+                       K, N, ep, *gs, dRows);
   } else if (vec && !gs && K <= TK_MAX_K) {
     hipLaunchKernelGGL(k_nin_thin, dim3(scn_ceil_div(M, 32), scn_ceil_div(N, 32)),
                        dim3(256), 0, ctx->stream, d_A, d_W, d_out, (long long)M,
-                       K, N, ep);
-  } else if (vec && scn_planes_shape(K) &&
-             (precision == SCN_FP32_PLANES || 2e0 * M * K * N >= PLANES_MIN_FLOPS || scn_planes_splitk(ctx, 3, M, K, N))) {
+                       K, N, ep, dRows);
+  } else if (planes) {
     SCN_TRY(scn_planes_forward(ctx, 3, d_A, d_W, d_out, M, K, N, ep, gs, false));
   } else if (vec && wres_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
     // W-resident kernel took it

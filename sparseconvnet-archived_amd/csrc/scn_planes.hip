@@ -40,6 +40,20 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[PL]) {
     p[l] = __builtin_bit_cast(bf16x8, uint4{w[l][0], w[l][1], w[l][2], w[l][3]});
 }
 
+// Rows that are known on the device only.  Which kernel takes a layer depends
+// on their number; where either may be right both are launched, and one of them
+// finds that it is not its.
+struct RowRange {
+  const long long *d_rows; // null: as many as the host says
+  long long above, upTo;   // this kernel's: above < rows <= upTo
+  __device__ __forceinline__ long long live(long long bound) const {
+    if (!d_rows)
+      return bound;
+    const long long n = *d_rows;
+    return n <= above || n > upTo ? 0 : n < bound ? n : bound;
+  }
+};
+
 // Four channels (A16: eight) of a gathered row: columns k .. of the row that
 // `rules` (in LDS, fs of them) stand for.
 template <bool A16>
@@ -79,7 +93,10 @@ template <int PL, int MT, int NT, int PD, int GATHER, bool A16, bool IMG>
 __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 : 4)
     k_nin_planes(const float *__restrict__ A, const float *__restrict__ W,
                  float *__restrict__ out, long long M, int K, int N,
-                 Epilogue ep, GatherSource gs, int nSplits) {
+                 Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
+  M = rows.live(M);
+  if ((long long)(blockIdx.x / nSplits) * (128 * MT) >= M)
+    return;
   constexpr int ES = A16 ? 2 : 4;
   constexpr int WAVES = 4, THREADS = 64 * WAVES;
   constexpr int ROWS = 32 * MT * WAVES, NW = 32 * NT;
@@ -371,7 +388,10 @@ template <int PL, bool GATHER, bool A16, bool WT>
 __global__ void __launch_bounds__(512, 2)
     k_nin_planes_splitk(const float *__restrict__ A, const float *__restrict__ W,
                         float *__restrict__ out, long long M, int K, int N,
-                        Epilogue ep, GatherSource gs, int nSplits) {
+                        Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
+  M = rows.live(M);
+  if ((long long)(blockIdx.x / nSplits) * 32 >= M)
+    return;
   constexpr int ES = A16 ? 2 : 4;
   __shared__ __attribute__((aligned(16))) float sPart[8 * 16 * 64];
   __shared__ int sRules[GATHER ? 32 * GF_MAX_FS : 1];
@@ -571,7 +591,8 @@ constexpr int planes_depth(int PL, int MT, int NT) {
 template <int PL, int MT, int NT, bool IMG, bool FINE = false>
 static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
-                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT) {
+                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT,
+                         const RowRange &rows) {
   const int nSplits = scn_ceil_div(N, 32 * NT);
   const size_t lds = (size_t)2 * PL * 2 * NT * 1024 + (gs ? (size_t)128 * MT * gs->fs * 4 : 0);
   constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
@@ -604,7 +625,7 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
 #define SCN_PLANES_GO(G, H, src)                                               \
   hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, IMG>), grid,       \
                      dim3(256), lds, ctx->stream, A, W, out, M, K, N,   \
-                     ep, src, nSplits)
+                     ep, src, nSplits, rows)
   if (!gs)
     SCN_PLANES_GO(0, false, GatherSource());
   else if (PL == 1 && a16)
@@ -617,12 +638,13 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
 template <int PL>
 static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
-                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT) {
+                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT,
+                         const RowRange &rows) {
   const int nSplits = scn_ceil_div(N, 32);
   const dim3 grid((unsigned)(scn_ceil_div(M, 32) * (long long)nSplits));
 #define SCN_SPLITK_GO(G, H, T, src)                                            \
   hipLaunchKernelGGL((k_nin_planes_splitk<PL, G, H, T>), grid, dim3(512), 0,   \
-                     ctx->stream, A, W, out, M, K, N, ep, src, nSplits)
+                     ctx->stream, A, W, out, M, K, N, ep, src, nSplits, rows)
   if (PL == 3 && wT)
     SCN_SPLITK_GO(false, false, PL == 3, GatherSource());
   else if (!gs)
@@ -655,12 +677,24 @@ static const PlanesCost planesCost[2][4][2] = {
     // three planes
     {{{.64f, .46f}, {.54f, .39f}}, {{.96f, .72f}, {.95f, .64f}}, {{1.6f, 1.16f}, {1.23f, .99f}}, {{1.36f, 1.29f}, {1.22f, 1.16f}}}};
 
+// The split contraction takes up to this many rows: one or two trips to memory
+// while its workgroups are up to so many a compute unit (measured: three planes,
+// 390 workgroups of 512 k 10.2 us against 14.2 for the tile, 1460 of 384 k 23.9
+// against 16); every 32 rows read the whole of W, out of L2 up to about 512 k.
+static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
+  const float perCU = planes == 1 ? (K <= 512 ? 1.4f + K / 160.f : 3.3f) : fminf(1.f + K / 230.f, 3.1f);
+  const long long rows = (long long)(perCU * ctx->numCU / scn_ceil_div(N, 32));
+  return 32 * (rows < 1 ? 1 : rows);
+}
+
 struct PlanesChoice {
   int tile; // index into planesTiles, -1: split contraction
   bool image;
 };
 // needImage: of the tiles, only from the image
 static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool needImage = false) {
+  if (M <= split_rows(ctx, planes, K, N))
+    return {-1, false};
   const int T = K / 32;
   PlanesChoice best = {0, false};
   float least = 1e30f;
@@ -679,17 +713,10 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
         least = cost, best = {i, img != 0};
     }
   }
-  // The split contraction: one or two trips to memory while its workgroups are
-  // few; every 32 rows read the whole of W, out of L2 up to about 512 k.
-  const float wgs = (float)(scn_ceil_div(M, 32) * (long long)scn_ceil_div(N, 32)) / ctx->numCU;
-  const float splitk = fmaxf(3.f + .005f * K, 2.5f + wgs * ((planes == 1 ? 1.5f + .001f * K : 2.4f + .0027f * K) +
-                                                            (K > 512 ? .004f * (K - 512) : 0.f)));
-  if (splitk < least)
-    best = {-1, false};
   return best;
 }
 bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
-  return planes_choose(ctx, planes, M, K, N).tile < 0;
+  return M <= split_rows(ctx, planes, K, N);
 }
 
 template <int PL>
@@ -697,16 +724,34 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
                           float *out, long long M, int K, int N,
                           const Epilogue &ep, const GatherSource *gs, bool a16,
                           const PlanesChoice &choice, bool wT = false) {
-  if (choice.tile < 0)
-    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT);
+  RowRange rows = {ctx->d_meta ? ctx->d_meta + META_SITES : nullptr, -1, 1ll << 62};
+  if (rows.d_rows) {
+    // Near the line both are launched, each for its numbers of rows; away from
+    // it the guess decides, and is held against the counts when they are known.
+    const long long split = split_rows(ctx, PL, K, N), hint = scn_rows_hint(ctx, M);
+    const long long few = M < split ? M : split;
+    if (M > split && 6 * hint > 5 * split && 5 * hint < 6 * split) {
+      RowRange upper = rows;
+      rows.upTo = upper.above = split;
+      SCN_TRY(launch_splitk<PL>(ctx, A, W, out, few, K, N, ep, gs, a16, wT, rows));
+      rows = upper;
+    } else if (hint <= split) {
+      scn_rows_chosen(ctx, -1, split);
+      return launch_splitk<PL>(ctx, A, W, out, few, K, N, ep, gs, a16, wT, rows);
+    } else {
+      scn_rows_chosen(ctx, split, 1ll << 62);
+    }
+  } else if (choice.tile < 0) {
+    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
+  }
   // (channels in other than 32s, seldom met: one tile)
   if (gs && gs->nIn % 32 != 0)
-    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false);
+    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
 #define SCN_PLANES_CASE(I, MT, NT)                                             \
   case I:                                                                      \
     return choice.image                                                        \
-               ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16, wT) \
-               : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16, false);
+               ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows) \
+               : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
   switch (choice.tile) {
     SCN_PLANES_CASE(0, 1, 1)
     SCN_PLANES_CASE(1, 1, 2)
@@ -720,7 +765,9 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
                        const Epilogue &ep, const GatherSource *gs, bool a16) {
-  PlanesChoice choice = planes_choose(ctx, planes, M, K, N);
+  // (rows guessed: a tile in any case, they may be more)
+  const long long split = split_rows(ctx, planes, K, N), hint = scn_rows_hint(ctx, M);
+  PlanesChoice choice = planes_choose(ctx, planes, M > split && hint <= split ? split + 1 : hint, K, N);
   choice.image = choice.image && planes_image(ctx);
   return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
          : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)

@@ -175,5 +175,14 @@ public:
   void ensureInterfaces();
   // Fills slot cc's input interface from a batch that already sits in HBM
   // (see ResidentBatch) and builds every rule book, on the slot's stream.
-  void preprocessResident(int cc, const struct ResidentBatch &input);
+  // mayRunAhead: the counts may stay on the device (batch.countsPending), for a
+  // caller that queues the forward pass on the same stream and then calls
+  // settleRuleBooks
+  void preprocessResident(int cc, const struct ResidentBatch &input,
+                          bool mayRunAhead = false);
+  // Waits for the batch's counts and puts the real sizes in place.  False: a
+  // forward pass queued before is queued again, since the batch outgrew the
+  // bounds (it has been planned again, the pass has computed nothing) or the
+  // real sizes would have chosen kernels that round differently.
+  bool settleRuleBooks(SpatiallySparseBatch &batch);
 };

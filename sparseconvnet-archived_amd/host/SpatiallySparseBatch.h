@@ -69,6 +69,9 @@ public:
   std::vector<std::vector<float>> probabilities;
   float negativeLogLikelihood;
   int mistakes;
+  // the rule books' counts are still on the device: the interfaces hold bounds
+  // until SparseConvNetCUDA::settleRuleBooks
+  bool countsPending;
   // device staging of the input sites (sample, key as two ints, row,
   // backgroundCol), reused from batch to batch
   vectorCUDA<int> stagingSample, stagingKey, stagingRow, stagingBackground;

@@ -398,6 +398,7 @@ SpatiallySparseBatch::SpatiallySparseBatch(
   reset();
 }
 void SpatiallySparseBatch::reset() {
+  countsPending = false;
   batchSize = 0;
   sampleNumbers.resize(0);
   for (auto &i : interfaces)

@@ -286,26 +286,47 @@ static void clearDeviceGrids(scn_ctx *ctx, SpatiallySparseBatch &b) {
 // one scn_rules_settle at the end, after which the real sizes are put in
 // place.  A batch that outgrows the bounds (or the first batch of a slot, which
 // has no bounds yet: its plans simply wait) is planned again the exact way.
+static void planAllLayers(SparseConvNetCUDA &cnn, scn_ctx *ctx,
+                          SpatiallySparseBatch &b) {
+  for (size_t i = 0; i < cnn.layers.size(); i++) {
+    scn_prof_tag(ctx, (int)i);
+    cnn.layers[i]->preprocess(b, b.interfaces[i], b.interfaces[i + 1]);
+  }
+}
 static void buildRuleBooks(SparseConvNetCUDA &cnn, scn_ctx *ctx,
-                           SpatiallySparseBatch &b) {
-  auto all = [&]() {
-    for (size_t i = 0; i < cnn.layers.size(); i++) {
-      scn_prof_tag(ctx, (int)i);
-      cnn.layers[i]->preprocess(b, b.interfaces[i], b.interfaces[i + 1]);
-    }
-  };
+                           SpatiallySparseBatch &b, bool mayRunAhead = false) {
   // (plans that continue from one another are recorded and run together)
   SCN_CHECKED(scn_ctx_defer_counts(ctx, 1));
   SCN_CHECKED(scn_ctx_chain_rules(ctx, cnn.chainRuleBooks ? 1 : 0));
-  all();
+  planAllLayers(cnn, ctx, b);
   SCN_CHECKED(scn_ctx_chain_rules(ctx, 0));
   SCN_CHECKED(scn_ctx_defer_counts(ctx, 0));
+  // Running ahead: every layer's rows can be read on the device, and the result
+  // has a row per sample whatever the counts turn out to be.
+  bool ahead = mayRunAhead && b.interfaces.back().nSpatialSites == b.batchSize;
+  for (size_t i = 1; ahead && i < b.interfaces.size(); ++i)
+    ahead = !b.interfaces[i].ownsDeviceGrids ||
+            scn_ctx_rows_from(ctx, b.interfaces[i].deviceGrids) == SCN_OK;
+  SCN_CHECKED(scn_ctx_rows_from(ctx, nullptr));
+  if (ahead)
+    b.countsPending = true;
+  else
+    cnn.settleRuleBooks(b);
+}
+bool SparseConvNetCUDA::settleRuleBooks(SpatiallySparseBatch &b) {
+  SparseConvNetCUDA &cnn = *this;
+  scn_ctx *ctx = b.preprocessStream ? b.preprocessStream->ctx : memStream.ctx;
+  const bool ahead = b.countsPending;
+  b.countsPending = false;
   const int rc = scn_rules_settle(ctx);
   if (rc == SCN_ERR_CAPACITY) {
-    all(); // every plan empties its own output tables again
-    return;
+    planAllLayers(cnn, ctx, b); // every plan empties its own output tables again
+    return false;
   }
   SCN_CHECKED(rc);
+  int held = 1;
+  if (ahead)
+    SCN_CHECKED(scn_ctx_rows_held(ctx, &held));
   // real sizes: a layer that owns its grids asks them, the others inherit
   for (size_t i = 0; i < cnn.layers.size(); i++) {
     SpatiallySparseBatchInterface &in = b.interfaces[i], &out = b.interfaces[i + 1];
@@ -320,12 +341,29 @@ static void buildRuleBooks(SparseConvNetCUDA &cnn, scn_ctx *ctx,
     } else {
       out.nSpatialSites = in.nSpatialSites;
     }
+    if (!ahead)
+      continue;
+    // what the forward pass sized and counted by the bounds
+    const size_t n = (size_t)out.nSpatialSites;
+    if (out.sub->features.size64() > 0)
+      out.sub->features.resize64(n * out.featuresPresent.size());
+    if (out.sub->poolingChoices.size64() > 0)
+      out.sub->poolingChoices.resize64(n * out.featuresPresent.size());
+    int nIn = 0, nOut = 0;
+    if (auto *l = dynamic_cast<NetworkInNetworkLayer *>(layers[i]))
+      nIn = l->nFeaturesIn, nOut = l->nFeaturesOut;
+    else if (auto *l = dynamic_cast<NetworkInNetworkPReLULayer *>(layers[i]))
+      nIn = l->nFeaturesIn, nOut = l->nFeaturesOut;
+    if (held)
+      addMultiplyAdds((__int128_t)n * nIn * nOut);
   }
+  return held != 0;
 }
 // Host-resident input of at least this many bytes is uploaded by the copy
 // engine rather than read over the bus by the kernels that use it.
 static const size_t kCopyEngineBytes = 4u << 20;
-void SparseConvNetCUDA::preprocessResident(int cc, const ResidentBatch &input) {
+void SparseConvNetCUDA::preprocessResident(int cc, const ResidentBatch &input,
+                                           bool mayRunAhead) {
   SpatiallySparseBatch &b = batchPool[cc];
   scn_ctx *ctx = b.preprocessStream ? b.preprocessStream->ctx : memStream.ctx;
   b.reset();
@@ -380,8 +418,9 @@ void SparseConvNetCUDA::preprocessResident(int cc, const ResidentBatch &input) {
   else
     SCN_CHECKED(scn_copy(ctx, in.sub->features.dPtr(), input.d_features,
                          nElems * sizeof(float)));
-  buildRuleBooks(*this, ctx, b);
-  SCN_CHECKED(scn_sync(ctx));
+  buildRuleBooks(*this, ctx, b, mayRunAhead);
+  if (!b.countsPending)
+    SCN_CHECKED(scn_sync(ctx));
 }
 void SparseConvNetCUDA::setPrecision(int precision) {
   for (auto *l : layers) {
@@ -438,6 +477,8 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   for (size_t i = 0; i < layers.size(); i++) {
     batch.interfaces[i + 1].sub->reset();
     scn_prof_tag(ms.ctx, (int)i);
+    if (batch.countsPending)
+      SCN_CHECKED(scn_ctx_rows_from(ms.ctx, batch.interfaces[i + 1].deviceGrids));
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);
     if (batch.type == RESCALEBATCH) {
       std::cout << i << ":"
@@ -448,6 +489,8 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
                               scalingUnderneath, i == layers.size() - 1);
     }
   }
+  if (batch.countsPending)
+    SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
   SoftmaxClassifierLaunch(batch.interfaces.back(), batch, ms);
 }
 void SparseConvNetCUDA::finishBatch(SpatiallySparseBatch &batch,

@@ -541,14 +541,25 @@ int scnh_forward_resident(scnh_net *net, int batch, const int32_t *d_sample,
   cnn->batchPool[0].preprocessStream = nullptr;
   cnn->preprocessResident(0, resident_of(batch, d_sample, d_key, d_row,
                                          d_background, nActive, nSpatialSites,
-                                         d_features));
-  cnn->batchPool[0].preprocessStream = keep;
+                                         d_features),
+                          net->hasClassifier);
   SpatiallySparseBatch &b = cnn->batchPool[0];
   net->batch = &b;
-  forward_layers(net, b);
+  if (b.countsPending) {
+    // rule books and layers are queued in one go; the one wait of the batch
+    cnn->forwardBatch(b);
+    if (!cnn->settleRuleBooks(b))
+      cnn->forwardBatch(b);
+    std::ofstream f, g;
+    cnn->finishBatch(b, f, g);
+  } else {
+    forward_layers(net, b);
+  }
+  cnn->batchPool[0].preprocessStream = keep;
   if (net->hasClassifier && h_probs)
     scnh_batch_probabilities(net, h_probs);
-  cnn->memStream.synchronize();
+  if (!net->hasClassifier) // (a classifier's probabilities are the last thing on the stream)
+    cnn->memStream.synchronize();
   return b.interfaces.back().nSpatialSites;
 }
 
