@@ -486,58 +486,166 @@ extern "C" int scn_nag_update_many(scn_ctx *ctx, const scn_nag_item *items,
 }
 
 // ------------------------------------------------- scatter-add through rules
-// A group of P lanes (P = the power of two that covers min(nIn, 64)) walks a
-// run of consecutive rule entries; lane j of it owns channel j (+ P, + 2P ..).
-// Consecutive entries that name the same input row (a sample's background row
-// fills most of a sparse rule book) are summed in a register and reach memory
-// as one atomic add.  Runs of 8: measured on the 2-D benchmark net, one atomic
-// per entry and runs of 32 both cost 10 % more of a training step.
-#define SCATTER_RUN 8
-__global__ __launch_bounds__(256) void k_gather_backward(
+// A float atomic costs by the 64-byte pieces it touches, some 20 of which retire
+// in a nanosecond however many of their lanes are live, and pieces of one line
+// follow one another at 2 ns: a matrix of two and a half inputs a row, a fifth of
+// them background, was added at a quarter of the rate it can be read at.  So a
+// workgroup takes EN consecutive entries, whose neighbouring windows share most
+// of their input rows, sorts them by row in LDS (a hash table, then a scan over
+// its slots) and adds every row to memory once.  An item is up to eight entries
+// of a row, summed in registers by a lane per channel, two items in flight; a
+// row of more items (the background row of a sample, named by a fifth to a half
+// of the entries) is put together in LDS first.
+// 94264 x 4 x 96: 39 us (97 with runs of eight entries and no sorting; it takes
+// 36 to read), 249376 x 8 x 32 74 (540), 60448 x 8 x 64 32 (211), 121924 x 27 x
+// 64 255 (3078), 34485 x 4 x 64 15.5 (36), 1858 x 4 x 128 6.1 (9).
+#define GB_RUN 8  // entries of one item
+#define GB_FLIGHT 2 // items of a lane in flight
+#define GB_LONG 4 // rows of more than one item that are summed in LDS
+#define GB_LONG_WIDTH 512
+struct GbItem {
+  int row; // -1 - l: the l-th long row
+  unsigned short start, len;
+};
+template <int T, int EN>
+__global__ __launch_bounds__(T) void k_gather_backward(
     float *__restrict__ din, const float *__restrict__ dconv,
-    const int *__restrict__ rules, long long count, int nIn, int P) {
-  const long long lane = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long group = lane / P;
-  const int li = (int)(lane - group * P);
-  const long long e0 = group * SCATTER_RUN;
-  if (e0 >= count)
-    return;
-  const long long e1 = e0 + SCATTER_RUN < count ? e0 + SCATTER_RUN : count;
-  // the run's rules and values are all requested before the first is used
-  int rl[SCATTER_RUN];
-#pragma unroll
-  for (int u = 0; u < SCATTER_RUN; ++u)
-    rl[u] = e0 + u < e1 ? rules[e0 + u] : -1;
-  for (int j = li; j < nIn; j += P) {
-    float dv[SCATTER_RUN];
-#pragma unroll
-    for (int u = 0; u < SCATTER_RUN; ++u)
-      dv[u] = e0 + u < e1 ? dconv[(e0 + u) * nIn + j] : 0.f;
-    int cur = -1;
-    float acc = 0.f;
-#pragma unroll
-    for (int u = 0; u < SCATTER_RUN; ++u) {
-      const int r = rl[u];
-      if (r < 0)
-        continue;
-      if (r != cur) {
-        if (cur >= 0)
-          unsafeAtomicAdd(din + (long long)cur * nIn + j, acc);
-        cur = r;
-        acc = 0.f;
-      }
-      acc += dv[u];
+    const int *__restrict__ rules, long long count, int nIn, int channels,
+    int splits) {
+  constexpr int SLOTS = 2 * EN;
+  __shared__ int sRow[SLOTS];   // hash table of the tile's rows
+  __shared__ int sCount[SLOTS]; // entries of each; then where they begin
+  __shared__ unsigned short sEntry[EN]; // entries, row by row
+  __shared__ GbItem sItem[EN];
+  __shared__ int sWave[3][T / 64];
+  __shared__ int sLongRow[GB_LONG];
+  __shared__ float sLong[GB_LONG * GB_LONG_WIDTH];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long long e0 = (long long)(blockIdx.x / splits) * EN;
+  const int c0 = (int)(blockIdx.x % splits) * channels;
+  const int width = nIn - c0 < channels ? nIn - c0 : channels;
+  const int longRows = width <= GB_LONG_WIDTH ? GB_LONG : 0;
+  for (int i = tid; i < SLOTS; i += T)
+    sRow[i] = -1, sCount[i] = 0;
+  for (int i = tid; i < longRows * width; i += T)
+    sLong[i] = 0.f;
+  const int r = tid < EN && e0 + tid < count ? rules[e0 + tid] : -1;
+  __syncthreads();
+  int slot = 0, place = 0;
+  if (r >= 0) {
+    unsigned h = ((unsigned)r * 2654435761u) >> 7 & (SLOTS - 1);
+    while (true) { // (twice as many slots as entries: ends)
+      const int was = atomicCAS(&sRow[h], -1, r);
+      if (was == -1 || was == r)
+        break;
+      h = (h + 1) & (SLOTS - 1);
     }
-    if (cur >= 0)
-      unsafeAtomicAdd(din + (long long)cur * nIn + j, acc);
+    slot = (int)h;
+    place = atomicAdd(&sCount[h], 1);
   }
-}
-
-static int group_width(int n) {
-  int P = 1;
-  while (P < n && P < 64)
-    P <<= 1;
-  return P;
+  __syncthreads();
+  // entries, items and long rows before every slot (a thread has one or two)
+  constexpr int SPT = SLOTS > T ? SLOTS / T : 1;
+  int n[SPT], entries = 0, items = 0, longs = 0;
+#pragma unroll
+  for (int u = 0; u < SPT; ++u) {
+    n[u] = tid * SPT + u < SLOTS ? sCount[tid * SPT + u] : 0;
+    entries += n[u];
+    items += (n[u] + GB_RUN - 1) / GB_RUN;
+    longs += n[u] > GB_RUN;
+  }
+  int pe = entries, pi = items, pl = longs;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int ve = __shfl_up(pe, d), vi = __shfl_up(pi, d), vl = __shfl_up(pl, d);
+    if (lane >= d)
+      pe += ve, pi += vi, pl += vl;
+  }
+  if (lane == 63)
+    sWave[0][wave] = pe, sWave[1][wave] = pi, sWave[2][wave] = pl;
+  __syncthreads();
+  int total = 0, nLong = 0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    if (w < wave)
+      pe += sWave[0][w], pi += sWave[1][w], pl += sWave[2][w];
+    total += sWave[1][w];
+    nLong += sWave[2][w];
+  }
+  nLong = nLong < longRows ? nLong : longRows;
+  pe -= entries;
+  pi -= items;
+  pl -= longs;
+#pragma unroll
+  for (int u = 0; u < SPT; ++u) {
+    if (n[u] == 0)
+      continue;
+    GbItem it;
+    it.row = sRow[tid * SPT + u];
+    sCount[tid * SPT + u] = pe;
+    if (n[u] > GB_RUN) {
+      if (pl < longRows) {
+        sLongRow[pl] = it.row;
+        it.row = -1 - pl;
+      }
+      ++pl;
+    }
+    for (int k = 0; k < n[u]; k += GB_RUN) {
+      it.start = (unsigned short)(pe + k);
+      it.len = (unsigned short)(n[u] - k < GB_RUN ? n[u] - k : GB_RUN);
+      sItem[pi++] = it;
+    }
+    pe += n[u];
+  }
+  __syncthreads();
+  if (r >= 0)
+    sEntry[sCount[slot] + place] = (unsigned short)tid;
+  __syncthreads();
+  const float *const src = dconv + e0 * nIn + c0;
+  float *const dst = din + c0;
+  const unsigned work = (unsigned)total * width;
+  const unsigned magic = 0xffffffffu / width + 1; // (x / width, exact for 2^32 / width of them)
+  auto of = [&](unsigned x) {
+    return width > 1024 ? x / (unsigned)width : width == 1 ? x : __umulhi(x, magic);
+  };
+  for (unsigned x = tid; x < work; x += GB_FLIGHT * T) {
+    float v[GB_FLIGHT][GB_RUN];
+    GbItem it[GB_FLIGHT];
+    unsigned j[GB_FLIGHT];
+#pragma unroll
+    for (int h = 0; h < GB_FLIGHT; ++h) {
+      const unsigned xh = x + h * T;
+      const unsigned i = of(xh);
+      j[h] = xh - i * width;
+      it[h].len = 0;
+      if (xh < work)
+        it[h] = sItem[i];
+#pragma unroll
+      for (int u = 0; u < GB_RUN; ++u) {
+        v[h][u] = 0.f;
+        if (u < it[h].len)
+          v[h][u] = src[(long long)sEntry[it[h].start + u] * nIn + j[h]];
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < GB_FLIGHT; ++h) {
+      if (it[h].len == 0)
+        continue;
+      float acc = v[h][0];
+#pragma unroll
+      for (int u = 1; u < GB_RUN; ++u)
+        acc += v[h][u];
+      if (it[h].row >= 0)
+        unsafeAtomicAdd(dst + (long long)it[h].row * nIn + j[h], acc);
+      else
+        unsafeAtomicAdd(&sLong[(-1 - it[h].row) * width + j[h]], acc);
+    }
+  }
+  if (nLong == 0)
+    return;
+  __syncthreads();
+  for (int i = tid; i < nLong * width; i += T)
+    unsafeAtomicAdd(dst + (long long)sLongRow[i / width] * nIn + i % width, sLong[i]);
 }
 
 extern "C" int scn_gather_rows_backward(scn_ctx *ctx, float *d_din,
@@ -553,20 +661,48 @@ extern "C" int scn_gather_rows_backward(scn_ctx *ctx, float *d_din,
   SCN_REQUIRE(d_din && d_dconv && d_rules, SCN_ERR_ARG,
               "scn_gather_rows_backward: null buffer");
   ProfScope prof(ctx, SCN_K_BACKWARD);
-  const int P = group_width(nIn);
-  const long long groups = (count + SCATTER_RUN - 1) / SCATTER_RUN;
-  const long long blocks = (groups * P + 255) / 256;
-  SCN_REQUIRE(blocks <= 0x7fffffffll, SCN_ERR_CAPACITY,
-              "scn_gather_rows_backward: %lld workgroups", blocks);
-  hipLaunchKernelGGL(k_gather_backward, dim3((unsigned)blocks), dim3(256), 0,
-                     ctx->stream, d_din, d_dconv, d_rules, (long long)count,
-                     nIn, P);
+  // Tiles of 512 entries while there are two and a half for every compute unit
+  // (60448 x 8 x 64: 32 us, 36 with 256), of 64 while there is no more than one
+  // of 128 (6041 x 4 x 96: 7.7 us, 9.1 with 256), and where tiles are few, each
+  // is given to several workgroups by its channels.
+  const int most = scn_ceil_div(nIn, 32);
+  const int EN = count >= 1280ll * ctx->numCU ? 512 : count > 128ll * ctx->numCU ? 256 : 64;
+  const long long tiles = scn_ceil_div(count, EN);
+  int splits = scn_ceil_div(EN == 64 ? 4 * ctx->numCU : 3 * ctx->numCU / 2, tiles);
+  const int channels = 32 * scn_ceil_div(most, splits < most ? splits : most);
+  splits = scn_ceil_div(nIn, channels);
+  SCN_REQUIRE(tiles * splits <= 0x7fffffffll, SCN_ERR_CAPACITY,
+              "scn_gather_rows_backward: %lld workgroups", tiles * splits);
+#define SCN_GB_GO(T, EN)                                                       \
+  hipLaunchKernelGGL((k_gather_backward<T, EN>),                               \
+                     dim3((unsigned)(tiles * splits)), dim3(T), 0,             \
+                     ctx->stream, d_din, d_dconv, d_rules, (long long)count,   \
+                     nIn, channels, splits)
+  if (EN == 512)
+    SCN_GB_GO(512, 512);
+  else if (EN == 256)
+    SCN_GB_GO(512, 256);
+  else
+    SCN_GB_GO(256, 64);
+#undef SCN_GB_GO
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
 }
 
-// dMaxPoolBackProp: the same walk over output rows, every lane following the
-// choices of its own channel.
+static int group_width(int n) {
+  int P = 1;
+  while (P < n && P < 64)
+    P <<= 1;
+  return P;
+}
+
+// dMaxPoolBackProp.  A group of P lanes (P = the power of two that covers
+// min(C, 64)) walks a run of output rows, every lane following the choices of
+// its own channel; consecutive rows that chose the same input are summed in a
+// register and reach memory as one atomic add.  (Sorted by input row in LDS the
+// runs touch as many 64-byte pieces: a row is chosen by some of its channels in
+// most of the windows that it is in.)
+#define SCATTER_RUN 8
 __global__ __launch_bounds__(256) void k_maxpool_backward(
     float *__restrict__ din, const float *__restrict__ dout, long long count,
     int C, const int *__restrict__ choice, int P) {
