@@ -54,6 +54,35 @@ struct RowRange {
   }
 };
 
+// An infinite operand, or one that rounds to an infinite bf16, leaves NaN in its
+// other planes (x - hi), where fp32 arithmetic has an infinity or a finite sum.
+// So with three planes a sum that is not finite is taken again from the
+// operands themselves; the test costs an instruction a result.
+template <int PL> __device__ __forceinline__ bool doubtful(float sum) {
+  return PL == 3 && !(fabsf(sum) <= 3.4028235e38f);
+}
+struct PlainW { // W as the caller gave it
+  const float *W;
+  int wT; // [N x K] and not [K x N]
+};
+// Row m of A (GATHER: through rules, fs of them, in LDS) times column n of W.
+template <bool GATHER>
+__device__ __forceinline__ float plain_sum(const float *A, const GatherSource &gs, const int *rules,
+                                           const PlainW &w, long long m, int n, int K, int N) {
+  const float *const wp = w.W + (w.wT ? (long long)n * K : n);
+  const int stride = w.wT ? 1 : N, run = GATHER ? gs.nIn : K;
+  float sum = 0.f;
+  for (int k0 = 0, f = 0; k0 < K; k0 += run, ++f) {
+    const float *a = A + m * K;
+    if (GATHER)
+      a = rules[f] >= 0 ? A + (long long)rules[f] * run : gs.zeros;
+#pragma unroll 1
+    for (int i = 0; i < run; ++i)
+      sum = fmaf(a[i], wp[(long long)(k0 + i) * stride], sum);
+  }
+  return sum;
+}
+
 // Four channels (A16: eight) of a gathered row: columns k .. of the row that
 // `rules` (in LDS, fs of them) stand for.
 template <bool A16>
@@ -93,7 +122,7 @@ template <int PL, int MT, int NT, int PD, int GATHER, bool A16, bool IMG>
 __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 : 4)
     k_nin_planes(const float *__restrict__ A, const float *__restrict__ W,
                  float *__restrict__ out, long long M, int K, int N,
-                 Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
+                 Epilogue ep, GatherSource gs, int nSplits, RowRange rows, PlainW plain) {
   M = rows.live(M);
   if ((long long)(blockIdx.x / nSplits) * (128 * MT) >= M)
     return;
@@ -351,6 +380,27 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
   for (int j = 0; j < NT; ++j)
     col[j] = load_col(ep, n + j < N ? n + j : N - 1);
   const bool whole = n0 + NW <= N && N % NT == 0;
+  unsigned long long again = 0; // results to be taken from the operands themselves
+  if constexpr (PL == 3) {
+    float none = 0.f; // 0 sum: NaN for a sum that is not finite
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          none = fmaf(acc[0][i][j][v] + acc[NACC - 1][i][j][v], 0.f, none);
+    if (none != 0.f) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (doubtful<PL>(acc[0][i][j][v] + acc[NACC - 1][i][j][v]))
+              again |= 1ull << ((i * NT + j) * 16 + v);
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const long long r0 = row0 + 32 * i + 4 * q;
@@ -376,6 +426,14 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
             orow[j] = r[j];
       }
     }
+  }
+  for (; again; again &= again - 1) {
+    const int e = __ffsll(again) - 1, v = e & 15, j = (e >> 4) % NT;
+    const int dr = 32 * ((e >> 4) / NT) + 8 * (v / 4) + 4 * q + v % 4;
+    if (row0 + dr < M && n + j < N)
+      out[(row0 + dr) * N + n + j] =
+          finish(plain_sum<GATHER != 0>(A, gs, sRules + (wave * 32 * MT + dr) * gs.fs, plain, row0 + dr, n + j, K, N),
+                 load_col(ep, n + j));
   }
 }
 
@@ -496,6 +554,8 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
     for (int w = 1; w < 8; ++w)
       sum += sPart[(w * 16 + v) * 64 + lane];
+    if (doubtful<PL>(sum))
+      sum = plain_sum<GATHER>(A, gs, sRules + dr * gs.fs, PlainW{W, WT}, row0 + dr, n0 + c, K, N);
     out[(row0 + dr) * N + n0 + c] = finish(sum, load_col(ep, n0 + c));
   }
 }
@@ -611,6 +671,7 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
     return rc;
   });
   SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  const PlainW plain = {W, wT};
   if (IMG) {
     const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;
     if (PL == 3 && wT)
@@ -625,7 +686,7 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
 #define SCN_PLANES_GO(G, H, src)                                               \
   hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, IMG>), grid,       \
                      dim3(256), lds, ctx->stream, A, W, out, M, K, N,   \
-                     ep, src, nSplits, rows)
+                     ep, src, nSplits, rows, plain)
   if (!gs)
     SCN_PLANES_GO(0, false, GatherSource());
   else if (PL == 1 && a16)
@@ -940,8 +1001,15 @@ __global__ void __launch_bounds__(512, 2)
     const int l = e & 63, v = (e >> 6) & 15, ij = e >> 10;
     const int kk = k0 + MT * (8 * (v / 4) + 4 * (l >> 5) + v % 4) + ij / NT;
     const int nn = n0 + NT * (l & 31) + ij % NT;
-    if (kk < K && nn < N)
-      unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
+    if (kk >= K || nn >= N)
+      continue;
+    if (doubtful<PL>(sum)) {
+      sum = 0.f;
+#pragma unroll 1
+      for (long long r = m0; r < m1; ++r)
+        sum = fmaf(A[r * K + kk], D[r * N + nn], sum);
+    }
+    unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
   }
 }
 

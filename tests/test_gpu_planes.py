@@ -56,6 +56,46 @@ def test_fp32_takes_the_planes_where_they_pay(scn, ctx):
         assert np.array_equal(out[0].download(), out[1].download())
 
 
+# split contraction; tiles converted on the way, in fours, from the image
+@pytest.mark.parametrize("rows,fs,nIn,N", [(40, 4, 32, 36), (20000, 4, 32, 64), (30000, 8, 12, 64), (70001, 4, 64, 128),
+                                           (65537, 9, 64, 64)])
+def test_infinite_operands_are_what_fp32_makes_of_them(scn, ctx, rows, fs, nIn, N):
+    """infinities, NaN and values past the largest bf16 in few rows of A: no NaN where the sum has none"""
+    rng = np.random.default_rng(rows + N)
+    K, special = fs * nIn, np.array([np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 0], np.float32)
+    inp = rng.standard_normal((600, nIn)).astype(np.float32)
+    inp[rng.choice(600, 12, False), rng.integers(0, nIn, 12)] = np.tile(special, 2)
+    rules = rng.integers(0, 600, (rows, fs)).astype(np.int32)
+    W = (0.5 * rng.standard_normal((K, N)) / K).astype(np.float32)
+    A = inp[rules].reshape(rows, K)
+    some = np.unique(np.concatenate([np.arange(min(rows, 300)), np.arange(max(0, rows - 300), rows)]))
+    with np.errstate(invalid="ignore"):
+        want = np.einsum("mk,kn->mn", A[some].astype(np.float64), W.astype(np.float64))
+        scale = np.einsum("mk,kn->mn", np.abs(A[some]).astype(np.float64), np.abs(W).astype(np.float64))
+    d_rules, d_in, d_W, d_B = ctx.array(rules), ctx.array(inp), ctx.array(W), ctx.array(np.zeros(N, np.float32))
+    d_A, fused, two, dA = ctx.array(A), *(ctx.array(np.full((rows, N), 7, np.float32)) for _ in range(3))
+    ctx.conv_nin_forward(d_in, d_rules, fs, nIn, d_W, d_B, None, fused, rows, N, 1.0, scn.NOSIGMOID, scn.FP32_PLANES)
+    ctx.nin_forward(d_A, d_W, d_B, None, two, rows, K, N, 1.0, scn.NOSIGMOID, scn.FP32_PLANES)
+    ctx.sgemm_ABt(d_A, ctx.array(np.ascontiguousarray(W.T)), dA, rows, K, N, ctx.empty(N * K + K, np.float32))
+    for name, out in (("fused", fused), ("two", two), ("ABt", dA)):
+        got, sure = out.download()[some], np.isfinite(want)
+        assert np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True), name
+        assert np.all(np.abs(got[sure] - want[sure]) <= 2e-6 * scale[sure]), name
+    # dW = A^T D over the first rows, an infinity in a row of its own and in D
+    M = min(rows, 2000)
+    A = rng.standard_normal((M, K), dtype=np.float32)
+    D = (0.1 * rng.standard_normal((M, N)) / M).astype(np.float32)
+    A[3, 5], A[M - 1, 7], A[4, 9], D[M // 2, 11] = np.inf, -np.inf, 3.4e38, np.inf
+    dW = ctx.array(np.zeros((K, N), np.float32))
+    ctx.sgemm_AtB(ctx.array(A), ctx.array(D), dW, M, K, N)
+    with np.errstate(invalid="ignore"):
+        want, got = np.einsum("mk,mn->kn", A.astype(np.float64), D.astype(np.float64)), dW.download()
+    scale = np.einsum("mk,mn->kn", np.abs(A).astype(np.float64), np.abs(D).astype(np.float64))
+    sure = np.isfinite(want)
+    assert np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True)
+    assert np.all(np.abs(got[sure] - want[sure]) <= 2e-6 * scale[sure])
+
+
 # one row; fewer rows than a step; odd K or N (no pairs of columns); every tile; ragged row ranges
 @pytest.mark.parametrize("M,K,N", [(1, 32, 32), (15, 12, 32), (129, 27, 33), (130, 34, 31), (1000, 66, 100),
                                    (40001, 12, 32), (30011, 256, 96), (5000, 128, 62), (70003, 432, 128)])
