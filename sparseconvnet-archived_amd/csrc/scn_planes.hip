@@ -721,20 +721,31 @@ static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
 bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
 
 // Which tile.  With n workgroups on every compute unit a block of 32 k takes tn
-// n microseconds, and no less than t1 (its chain: request, split, barrier); both
-// were measured on contractions of 256 and 1152 k at 256 to 2048 workgroups,
-// with W converted on the way and from its image.  A wavefront of two row tiles
-// and two column tiles (2, 2) is the fastest per flop (three planes: 232
+// n microseconds, and no less than t1 (its chain: request, split, barrier).
+// Three planes: measured on contractions of 256 and 1152 k at 256 to 2048
+// workgroups, with W converted on the way and from its image.  A wavefront of
+// two row tiles and two column tiles (2, 2) is the fastest per flop (232
 // TFLOP/s from the image, (1, 1) 173) and the first to leave the chip idle, so
-// the row count decides; every choice gives the same bits.  The start and the
-// stores of a workgroup cost by its tiles, the image 5 us.
+// the row count decides.
+// One plane: fitted to 148 shapes (2800 to 200000 rows, 256 to 2592 k, 64 to 640
+// columns), fp32 and bf16 rows, which it gives within 1 % of the best tile on
+// average.  What bounds it is the fetching of A, once for every slice of
+// columns, so the tile is one row tile by up to four column tiles: from the
+// image, with bf16 rows, 570000 x 2592 x 128 511 -> 430 us (875 TFLOP/s) against
+// (2, 2), which goes twice through A; 5900 x 1920 x 640 with fp32 rows 57 -> 38
+// against (1, 2).  Five and eight column tiles, or two by four, gain no more.
+// Every choice gives the same bits.  The start and the stores of a workgroup
+// cost by its tiles, the image 5 us.
 struct PlanesCost {
   float t1, tn;
 };
-static const int planesTiles[4][2] = {{1, 1}, {1, 2}, {1, 3}, {2, 2}}; // row tiles, column tiles of a wavefront
-static const PlanesCost planesCost[2][4][2] = {
+static const int planesTiles[2][4][2] = {{{1, 1}, {1, 2}, {1, 3}, {1, 4}},  // row tiles, column tiles of a wavefront:
+                                         {{1, 1}, {1, 2}, {1, 3}, {2, 2}}}; // one plane, more
+static const PlanesCost planesCost[3][4][2] = {
     // one plane: converted, image
-    {{{.45f, .28f}, {.39f, .25f}}, {{.55f, .44f}, {.41f, .25f}}, {{.71f, .58f}, {.43f, .27f}}, {{.8f, .65f}, {.56f, .47f}}},
+    {{{.5f, .5f}, {.44f, .44f}}, {{.67f, .66f}, {.43f, .43f}}, {{.81f, .81f}, {.48f, .48f}}, {{1.21f, 1.21f}, {.46f, .46f}}},
+    // ... of bf16 rows
+    {{{.36f, .26f}, {.22f, .22f}}, {{.44f, .44f}, {.24f, .24f}}, {{.6f, .6f}, {.28f, .28f}}, {{.95f, .95f}, {.3f, .3f}}},
     // three planes
     {{{.64f, .46f}, {.54f, .39f}}, {{.96f, .72f}, {.95f, .64f}}, {{1.6f, 1.16f}, {1.23f, .99f}}, {{1.36f, 1.29f}, {1.22f, 1.16f}}}};
 
@@ -753,14 +764,15 @@ struct PlanesChoice {
   bool image;
 };
 // needImage: of the tiles, only from the image
-static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool needImage = false) {
+static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16,
+                                   bool needImage = false) {
   if (M <= split_rows(ctx, planes, K, N))
     return {-1, false};
   const int T = K / 32;
   PlanesChoice best = {0, false};
   float least = 1e30f;
   for (int i = 0; i < 4; ++i) {
-    const int mt = planesTiles[i][0], nt = planesTiles[i][1];
+    const int mt = planesTiles[planes > 1][i][0], nt = planesTiles[planes > 1][i][1];
     const long long nSplits = scn_ceil_div(N, 32 * nt);
     const float wgs = (float)(scn_ceil_div(M, 128 * mt) * nSplits) / ctx->numCU;
     const float n = wgs <= 4.f ? ceilf(wgs) : wgs + .5f;
@@ -768,7 +780,7 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
     for (int img = needImage; img < 2; ++img) {
       if (img && (size_t)nSplits * T * planes * 2 * nt * 1024 > SCN_IMAGE_BYTES)
         continue;
-      const PlanesCost &c = planesCost[planes == 1 ? 0 : 1][i][img];
+      const PlanesCost &c = planesCost[planes > 1 ? 2 : a16][i][img];
       const float cost = T * fmaxf(c.t1, c.tn * n) + 3.f + units * (.2f + .17f * n) + (img ? 5.f : 0.f);
       if (cost < least)
         least = cost, best = {i, img != 0};
@@ -817,7 +829,7 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
     SCN_PLANES_CASE(0, 1, 1)
     SCN_PLANES_CASE(1, 1, 2)
     SCN_PLANES_CASE(2, 1, 3)
-    SCN_PLANES_CASE(3, 2, 2)
+    SCN_PLANES_CASE(3, (PL > 1 ? 2 : 1), (PL > 1 ? 2 : 4))
   }
 #undef SCN_PLANES_CASE
   return SCN_ERR_ARG;
@@ -828,7 +840,7 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        const Epilogue &ep, const GatherSource *gs, bool a16) {
   // (rows guessed: a tile in any case, they may be more)
   const long long split = split_rows(ctx, planes, K, N), hint = scn_rows_hint(ctx, M);
-  PlanesChoice choice = planes_choose(ctx, planes, M > split && hint <= split ? split + 1 : hint, K, N);
+  PlanesChoice choice = planes_choose(ctx, planes, M > split && hint <= split ? split + 1 : hint, K, N, a16);
   choice.image = choice.image && planes_image(ctx);
   return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
          : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
@@ -841,7 +853,7 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
                     long long M, int K, int N, const float *zeros, int *rc) {
   if (!scn_planes_shape(K) || ((uintptr_t)A & 15) || ((uintptr_t)out & 15) || N % 4 != 0)
     return false;
-  const PlanesChoice choice = planes_choose(ctx, 3, M, K, N, true);
+  const PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
   if (choice.tile >= 0 && (!choice.image || !planes_image(ctx)))
     return false;
   Epilogue ep = Epilogue();

@@ -129,3 +129,38 @@ def test_activation_backward_column_sums(scn, ctx, M, N, act):
     if act == "PRELU":
         slope = np.where(out > 0, 0, delta * (out / pr)).astype(np.float64).sum(0)
         assert np.allclose(dp.download(), slope, atol=1e-5 * M ** 0.5 * 4 + 1e-5, rtol=1e-4)
+
+
+# one plane, up to four column tiles a wavefront: N a multiple of them or not, ragged rows, few and many blocks; bf16
+# rows and fp32 rows; a window of channels in other than 32s
+@pytest.mark.parametrize("rows,fs,nIn,N", [(12801, 4, 64, 128), (33005, 9, 96, 160), (20001, 27, 32, 96), (9001, 4, 160, 320),
+                                           (6001, 4, 480, 640), (60001, 8, 24, 224)])
+def test_one_plane_against_float64(scn, ctx, rows, fs, nIn, N):
+    rng = np.random.default_rng(rows + N)
+    K = fs * nIn
+    inp = rng.standard_normal((700, nIn), dtype=np.float32)
+    rules = rng.integers(-1, 700, (rows, fs)).astype(np.int32)
+    W = (rng.standard_normal((K, N)) * np.sqrt(2.0 / K)).astype(np.float32)
+    B = rng.uniform(-0.5, 0.5, N).astype(np.float32)
+    d_in, d_rules, d_W, d_B = (ctx.array(x) for x in (inp, rules, W, B))
+    one, two, three = (ctx.array(np.full((rows, N), 7, np.float32)) for _ in range(3))
+    print("one plane", rows, fs, nIn, N, flush=True)
+    ctx.conv_nin_forward(d_in, d_rules, fs, nIn, d_W, d_B, None, one, rows, N, 1.0, scn.RELU, scn.BF16)
+    ctx.conv_nin_forward_a16(d_in, 700, ctx.empty((700, nIn), np.float32), d_rules, fs, nIn, d_W, d_B, None, two, rows, N,
+                             1.0, scn.RELU)
+    g = ctx.empty((rows, K), np.float32)
+    ctx.gather_rows(d_in, g, d_rules, rows * fs, nIn)
+    ctx.nin_forward(g, d_W, d_B, None, three, rows, K, N, 1.0, scn.RELU, scn.BF16)
+    got = one.download()
+    assert np.array_equal(got, two.download()) and np.array_equal(got, three.download())
+
+    def bf16(x):
+        u = x.view(np.uint32)
+        return ((u + 0x7fff + (u >> 16 & 1)) & 0xffff0000).astype(np.uint32).view(np.float32)
+
+    some = np.unique(np.concatenate([np.arange(300), np.arange(rows - 300, rows)]))
+    A = np.where(rules[some, :, None] >= 0, inp[np.maximum(rules[some], 0)], 0).reshape(len(some), K).astype(np.float32)
+    want = orc.nin_forward(bf16(A), bf16(W), B, None, 1.0, scn.RELU, f64=True)
+    scale = np.abs(A).astype(np.float64) @ np.abs(W).astype(np.float64) + np.abs(B)
+    # products exact, their sum in fp32: a rounding every eight or sixteen of the K
+    assert np.all(np.abs(got[some] - want) <= 2e-6 * scale)
