@@ -162,8 +162,20 @@ void scn_chain_release(scn_ctx *ctx);
 // exclusive prefix sum of n uint32 values; out has n + 1 elements (out[n] =
 // total).  `tmp` must hold scn_scan_tmp_elems(n) uint32.
 size_t scn_scan_tmp_elems(size_t n);
+// What a scan of n elements wants zero in `tmp`.  The kernel that writes its
+// input, with as many lanes at least, may clear it (`cleared`): a launch of its
+// own takes 4 us.
+struct ScanState {
+  unsigned long long *state;
+  size_t words;
+  __device__ __forceinline__ void clear(size_t lane) const {
+    if (lane < words)
+      state[lane] = 0ull;
+  }
+};
+ScanState scn_scan_state(size_t n, uint32_t *tmp);
 int scn_scan_exclusive_u32(hipStream_t s, const uint32_t *in, uint32_t *out,
-                           size_t n, uint32_t *tmp);
+                           size_t n, uint32_t *tmp, bool cleared = false);
 // same, over popcounts of 64-bit words
 int scn_scan_exclusive_popc64(hipStream_t s, const uint64_t *words,
-                              uint32_t *out, size_t n, uint32_t *tmp);
+                              uint32_t *out, size_t n, uint32_t *tmp, bool cleared = false);

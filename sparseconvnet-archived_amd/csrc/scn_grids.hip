@@ -68,7 +68,8 @@ template <int D>
 __global__ void k_plan_count(GridView in, Geom g, const long long *ekey,
                              Count nEntries, const long long *inMeta,
                              unsigned *cntByRank, unsigned long long *ownMask,
-                             unsigned *rankOf) {
+                             unsigned *rankOf, ScanState scan) {
+  scan.clear((size_t)blockIdx.x * blockDim.x + threadIdx.x);
   long long e = xcd_contiguous_block((count_now(nEntries) + 255) / 256) * blockDim.x + threadIdx.x;
   if (e >= nEntries.bound)
     return;
@@ -683,7 +684,8 @@ template <int D>
 __global__ void __launch_bounds__(256)
     k_tile2_owners(GridView in, Geom g, const long long *inMeta,
                    unsigned long long *ownBits, long long nWords,
-                   long long totalBits) {
+                   long long totalBits, ScanState scan) {
+  scan.clear((size_t)blockIdx.x * blockDim.x + threadIdx.x);
   const long long w = xcd_contiguous_block((nWords + 255) / 256) * blockDim.x + threadIdx.x;
   if (w >= nWords)
     return;
@@ -1211,10 +1213,10 @@ static long long ipow_ll(long long b, int e) {
 }
 
 // (re)shape a grids object for `batch` samples of an n^d field holding up to
-// nActive sites; clears the mask, and the hash table when the caller is about
-// to fill it (withTable)
+// nActive sites; clears the mask, unless the caller writes every word of it
+// (wholeMask), and the hash table when the caller is about to fill it (withTable)
 static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
-                         long long nActive, bool withTable = false) {
+                         long long nActive, bool withTable = false, bool wholeMask = false) {
   SCN_REQUIRE(batch >= 0 && d >= 1 && d <= 3 && n >= 1, SCN_ERR_ARG,
               "grids: batch %d dimension %d spatialSize %d (dimension must be 1..3)",
               batch, d, n);
@@ -1264,7 +1266,7 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
   SCN_TRY(g->bg.reserve((size_t)batch + 1));
   // (a dense row table needs no clearing: it is read where the mask is set)
   const size_t clearSlots = withTable && !dense && cap > g->cleanSlots ? cap : 0;
-  const size_t clearWords = g->nWords + 2 > g->cleanWords ? g->nWords + 2 : 0;
+  const size_t clearWords = !wholeMask && g->nWords + 2 > g->cleanWords ? g->nWords + 2 : 0;
   if (withTable && !dense)
     g->cleanSlots = 0; // about to be written
   g->cleanWords = 0;
@@ -1807,7 +1809,8 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
     SCN_TRY(out->scanTmp.reserve(scn_scan_tmp_elems((size_t)ownWords)));
     hipLaunchKernelGGL(k_tile2_owners<D>, dim3(xcd_grid(scn_ceil_div(ownWords, 256))),
                        dim3(256), 0, ctx->stream, vin, g, inMeta, out->ownMask.p,
-                       ownWords, (long long)in->batch * g.volIn);
+                       ownWords, (long long)in->batch * g.volIn,
+                       scn_scan_state((size_t)ownWords, out->scanTmp.p));
     SCN_HIP_CHECK(hipGetLastError());
   } else if (masked) {
     SCN_TRY(out->ownMask.reserve((size_t)nE + 2));
@@ -1816,14 +1819,15 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   if (nE > 0 && !tiled) {
     hipLaunchKernelGGL(k_plan_count<D>, dim3(xcd_grid(scn_ceil_div(nE, 256))), dim3(256),
                        0, ctx->stream, vin, g, in->ekey.p, nEc, inMeta, out->cnt.p,
-                       masked ? out->ownMask.p : nullptr, out->rankOf.p);
+                       masked ? out->ownMask.p : nullptr, out->rankOf.p,
+                       scn_scan_state((size_t)nE, out->scanTmp.p));
     SCN_HIP_CHECK(hipGetLastError());
   }
   const long long *bad = (const long long *)(ctx->d_scalars + 15);
   const long long ticket = ++ctx->ticket;
   if (tiled) {
     SCN_TRY(scn_scan_exclusive_popc64(ctx->stream, (const uint64_t *)out->ownMask.p,
-                                      out->base.p, (size_t)ownWords, out->scanTmp.p));
+                                      out->base.p, (size_t)ownWords, out->scanTmp.p, true));
     GridView owners = vin;
     owners.bits = out->ownMask.p;
     owners.prefix = out->base.p;
@@ -1839,7 +1843,7 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
                        inMeta, boundRows, boundActive, slot);
   } else {
     SCN_TRY(scn_scan_exclusive_u32(ctx->stream, out->cnt.p, out->base.p,
-                                   (size_t)nE, out->scanTmp.p));
+                                   (size_t)nE, out->scanTmp.p, true));
     hipLaunchKernelGGL(k_plan_samples<false>, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream, vin,
                        out->base.p, nE, fullSize, out->bg.p, out->bgBefore.p,
                        out->sampleStart.p, (long long *)ctx->d_pinned, bad, ticket, out->meta.p,
@@ -1858,7 +1862,8 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
               "rules: %lld output rows do not fit 32-bit row numbers", nSites);
   // out->bg already holds what k_plan_samples wrote: grids_prepare only
   // reserves it (no reallocation at the same size) and clears table and mask
-  SCN_TRY(grids_prepare(ctx, out, in->batch, g.d, g.nOut, nOutActive));
+  const bool dilated = g.mode == MODE_SQ_NOMIN && g.size <= 64;
+  SCN_TRY(grids_prepare(ctx, out, in->batch, g.d, g.nOut, nOutActive, false, dilated));
   out->nSites = (int)nSites;
   if (deferred)
     mark_pending(ctx, out, slot);
@@ -1867,8 +1872,8 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   // the output mask: word by word from the input mask where the mode allows
   // it, else bit by bit as the emit pass finds the sites
   GridView vout = view_of(out);
-  if (g.mode == MODE_SQ_NOMIN && g.size <= 64) {
-    const long long words = (long long)out->nWords + 2;
+  if (dilated) {
+    const long long words = (long long)out->nWords + 2; // all that grids_prepare would clear
     const long long blocks = (scn_ceil_div(words, 256) + 7) / 8 * 8; // whole rounds of the 8 XCDs
     auto dilate = g.size == 2 ? k_mask_dilate<D, 2>
                               : (g.size == 3 ? k_mask_dilate<D, 3> : k_mask_dilate<D, 0>);

@@ -142,9 +142,16 @@ size_t scn_scan_tmp_elems(size_t n) {
   return 2 * (nb + 1) + 8; // a 64-bit word a tile, one for the tickets, room to align them
 }
 
+ScanState scn_scan_state(size_t n, uint32_t *tmp) {
+  if (n <= SCAN1_MAX_ELEMS)
+    return ScanState{nullptr, 0};
+  return ScanState{reinterpret_cast<unsigned long long *>(((uintptr_t)tmp + 7) & ~(uintptr_t)7),
+                   (n + LB_TILE - 1) / LB_TILE + 1};
+}
+
 template <bool POPC>
 static int scan_impl(hipStream_t s, const void *in, uint32_t *out, size_t n,
-                     uint32_t *tmp) {
+                     uint32_t *tmp, bool cleared) {
   if (n <= SCAN1_MAX_ELEMS) { // one launch; n == 0 still writes out[0] = 0
     hipLaunchKernelGGL(k_scan_single<POPC>, dim3(1), dim3(SCAN1_THREADS), 0, s,
                        in, out, n);
@@ -155,11 +162,13 @@ static int scan_impl(hipStream_t s, const void *in, uint32_t *out, size_t n,
   SCN_REQUIRE(nb < 0x7FFFFFFFull, SCN_ERR_CAPACITY, "scan: %zu elements", n);
   SCN_REQUIRE(((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0, SCN_ERR_ARG,
               "scan: buffers must be 16-byte aligned");
-  unsigned long long *state =
-      reinterpret_cast<unsigned long long *>(((uintptr_t)tmp + 7) & ~(uintptr_t)7);
-  hipLaunchKernelGGL(k_scan_clear, dim3((unsigned)((nb + 1 + 255) / 256)), dim3(256), 0, s,
-                     state, nb + 1);
-  SCN_HIP_CHECK(hipGetLastError());
+  const ScanState scan = scn_scan_state(n, tmp);
+  unsigned long long *const state = scan.state;
+  if (!cleared) {
+    hipLaunchKernelGGL(k_scan_clear, dim3((unsigned)((nb + 1 + 255) / 256)), dim3(256), 0, s,
+                       state, nb + 1);
+    SCN_HIP_CHECK(hipGetLastError());
+  }
   hipLaunchKernelGGL(k_scan_lookback<POPC>, dim3((unsigned)nb), dim3(SCAN_THREADS), 0, s, in,
                      out, n, state, (unsigned)nb);
   SCN_HIP_CHECK(hipGetLastError());
@@ -167,11 +176,11 @@ static int scan_impl(hipStream_t s, const void *in, uint32_t *out, size_t n,
 }
 
 int scn_scan_exclusive_u32(hipStream_t s, const uint32_t *in, uint32_t *out,
-                           size_t n, uint32_t *tmp) {
-  return scan_impl<false>(s, in, out, n, tmp);
+                           size_t n, uint32_t *tmp, bool cleared) {
+  return scan_impl<false>(s, in, out, n, tmp, cleared);
 }
 
 int scn_scan_exclusive_popc64(hipStream_t s, const uint64_t *words,
-                              uint32_t *out, size_t n, uint32_t *tmp) {
-  return scan_impl<true>(s, words, out, n, tmp);
+                              uint32_t *out, size_t n, uint32_t *tmp, bool cleared) {
+  return scan_impl<true>(s, words, out, n, tmp, cleared);
 }

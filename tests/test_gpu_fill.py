@@ -1,4 +1,5 @@
-"""Fills at any alignment."""
+"""Memory that is written whole without being cleared first: fills at any alignment, the masks and scan states of rule
+books whose objects were used for other sites before."""
 import numpy as np
 import pytest
 
@@ -14,3 +15,36 @@ def test_fill_touches_its_words_only(scn, ctx, n, off):
     want = np.arange(n + 8, dtype=np.int32)
     want[off:off + n] = 0x12345678
     assert np.array_equal(d.download(), want)
+
+
+# more entries than one workgroup scans, with and without tiled windows, and few; a denser set of sites before
+@pytest.mark.parametrize("d,field,samples,size,stride", [(3, 40, 9, 3, 1), (3, 40, 9, 2, 2), (2, 121, 33, 3, 2), (2, 20, 3, 2, 1)])
+def test_rule_books_on_used_objects(scn, ctx, d, field, samples, size, stride):
+    out = (field - size) // stride + 1
+    field = (out - 1) * stride + size
+    rng = np.random.default_rng(field + size)
+    used, results = [scn.Grids(ctx), scn.Grids(ctx)], []
+    for share in (0.4, 0.15):
+        active = rng.random((samples, field ** d)) < share
+        sample, key = (a.astype(t) for a, t in zip(np.nonzero(active), (np.int32, np.int64)))
+        per = active.sum(1)
+        row = (np.arange(len(key)) + sample + 1).astype(np.int32)
+        bg = (np.concatenate([[0], np.cumsum(per)[:-1]]) + np.arange(samples)).astype(np.int32)
+        n = len(key) + samples
+        results = []
+        for gin, gout in (used, (scn.Grids(ctx), scn.Grids(ctx))):
+            gin.build_device(samples, d, field, *(ctx.array(a) for a in (sample, key, row, bg)), len(key), n)
+            rows = gin.plan_square(gout, field, out, size, stride)
+            rules = ctx.empty((rows * size ** d,), np.int32)
+            gin.fill(gout, rules, rows * size ** d)
+            gnext = scn.Grids(ctx)  # what stands on the mask of the output
+            rows2 = gout.plan_square(gnext, out, out - 1, 2, 1)
+            rules2 = ctx.empty((rows2 * 2 ** d,), np.int32)
+            gout.fill(gnext, rules2, rows2 * 2 ** d)
+            results.append((rows, rules.download(), rows2, rules2.download()))
+        mask = active.reshape((samples,) + (field,) * d)
+        for axis in range(1, d + 1):
+            mask = np.logical_or.reduce([np.take(mask, np.arange(out) * stride + o, axis) for o in range(size)])
+        full = (mask.reshape(samples, -1).sum(1) == out ** d).sum()
+        assert results[0][0] == mask.sum() + samples - full or results[0][0] == mask.sum() + samples
+        assert all(np.array_equal(a, b) for a, b in zip(*results))
