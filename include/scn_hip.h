@@ -112,6 +112,10 @@ int scn_d2d(scn_ctx *ctx, void *d_dst, const void *d_src, size_t bytes);
  * upload or download that costs the host one kernel launch. */
 int scn_copy(scn_ctx *ctx, void *dst, const void *src, size_t bytes);
 int scn_fill32(scn_ctx *ctx, void *d_dst, uint32_t word, size_t nWords);
+/* up to SCN_FILL_MAX buffers in one launch */
+#define SCN_FILL_MAX 32
+int scn_fill32_many(scn_ctx *ctx, void *const *d_dst, const size_t *nWords,
+                    int n, uint32_t word);
 
 /* ---- sparse grids ----------------------------------------------------- */
 /* A scn_grids holds, for one depth of the net, the SparseGrid of every sample

@@ -89,6 +89,7 @@ def lib():
         "scn_event_wait": (C.c_int, [vp]),
         "scn_d2d": (C.c_int, [vp, vp, vp, sz]),
         "scn_fill32": (C.c_int, [vp, vp, C.c_uint32, sz]),
+        "scn_fill32_many": (C.c_int, [vp, C.POINTER(vp), C.POINTER(sz), C.c_int, C.c_uint32]),
         "scn_grids_create": (C.c_int, [vp, P(vp)]),
         "scn_grids_clear_many": (C.c_int, [vp, C.POINTER(vp), C.c_int]),
         "scn_ctx_defer_counts": (C.c_int, [vp, C.c_int]),

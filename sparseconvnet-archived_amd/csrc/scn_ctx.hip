@@ -245,10 +245,9 @@ extern "C" int scn_d2d(scn_ctx *c, void *d_dst, const void *d_src,
 
 // Four words a store between the ends that are not on 16 bytes: the fills of the
 // backward kernels of a middle layer (77 MB and less) 9.2 -> 7.0 us on average.
-__global__ __launch_bounds__(256) void k_fill32(uint32_t *dst, uint32_t w, size_t n) {
+__device__ __forceinline__ void fill32(uint32_t *dst, uint32_t w, size_t n, size_t i, size_t step) {
   const size_t off = (16 - ((uintptr_t)dst & 15) & 15) / 4;
   const size_t head = off < n ? off : n, quads = (n - head) / 4, tail = head + 4 * quads;
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
   uint4 *const body = reinterpret_cast<uint4 *>(dst + head);
   for (size_t q = i; q < quads; q += step)
     body[q] = make_uint4(w, w, w, w);
@@ -256,6 +255,50 @@ __global__ __launch_bounds__(256) void k_fill32(uint32_t *dst, uint32_t w, size_
     dst[i] = w;
   if (i < n - tail)
     dst[tail + i] = w;
+}
+__global__ __launch_bounds__(256) void k_fill32(uint32_t *dst, uint32_t w, size_t n) {
+  fill32(dst, w, n, (size_t)blockIdx.x * 256 + threadIdx.x, (size_t)gridDim.x * 256);
+}
+
+// Several buffers in one launch (a launch of its own is 2 us and the gap before
+// it): a workgroup finds its buffer from the running workgroup counts.
+struct FillList {
+  uint32_t *dst[SCN_FILL_MAX];
+  size_t n[SCN_FILL_MAX];
+  unsigned firstBlock[SCN_FILL_MAX + 1];
+  int count;
+};
+__global__ __launch_bounds__(256) void k_fill32_many(FillList l, uint32_t w) {
+  int t = 0;
+  while (t + 1 < l.count && blockIdx.x >= l.firstBlock[t + 1])
+    ++t;
+  const unsigned blocks = l.firstBlock[t + 1] - l.firstBlock[t];
+  fill32(l.dst[t], w, l.n[t], (size_t)(blockIdx.x - l.firstBlock[t]) * 256 + threadIdx.x, (size_t)blocks * 256);
+}
+
+extern "C" int scn_fill32_many(scn_ctx *c, void *const *d_dst,
+                               const size_t *nWords, int n, uint32_t word) {
+  SCN_REQUIRE(c && n >= 0 && n <= SCN_FILL_MAX && ((d_dst && nWords) || n == 0), SCN_ERR_ARG,
+              "scn_fill32_many: %d buffers (at most %d)", n, SCN_FILL_MAX);
+  FillList l;
+  l.count = 0;
+  unsigned total = 0;
+  for (int k = 0; k < n; ++k) {
+    if (nWords[k] == 0)
+      continue;
+    SCN_REQUIRE(d_dst[k], SCN_ERR_ARG, "scn_fill32_many: null buffer");
+    const size_t blocks = (nWords[k] + 1023) / 1024;
+    l.dst[l.count] = (uint32_t *)d_dst[k];
+    l.n[l.count] = nWords[k];
+    l.firstBlock[l.count++] = total;
+    total += (unsigned)(blocks < 65536 ? blocks : 65536);
+  }
+  if (l.count == 0)
+    return SCN_OK;
+  l.firstBlock[l.count] = total;
+  hipLaunchKernelGGL(k_fill32_many, dim3(total), dim3(256), 0, c->stream, l, word);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
 }
 
 extern "C" int scn_fill32(scn_ctx *c, void *d_dst, uint32_t word,

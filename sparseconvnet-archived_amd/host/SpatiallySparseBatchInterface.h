@@ -27,6 +27,9 @@ public:
   int nSpatialSites; // active rows of the whole batch, background rows included
   int spatialSize;
   bool backpropErrors;
+  // sub->dfeatures has been cleared for the layer that adds to it next
+  // (SparseConvNetCUDA::backwardBatch clears those of a whole pass at once)
+  bool gradientCleared = false;
   // Host view of the sparse grids.  Filled by the Pictures for the input
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().

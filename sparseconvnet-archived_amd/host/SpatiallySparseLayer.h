@@ -37,6 +37,8 @@ public:
   virtual void loadWeightsFromStream(std::ifstream &f, bool momentum);
   virtual void putWeightsToStream(std::ofstream &f, bool momentum);
   virtual int calculateInputSpatialSize(int outputSpatialSize) = 0;
+  // backwards() adds to the input's gradient (and does not assign it)
+  virtual bool addsInputGradient() const { return false; }
 };
 
 // ConvolutionalLayer.h:3-33 -- gathers each output site's receptive field
@@ -66,6 +68,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -97,6 +100,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -203,6 +207,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -227,6 +232,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -268,6 +274,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -306,6 +313,7 @@ public:
   void forwards(SpatiallySparseBatch &batch,
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
+  bool addsInputGradient() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,

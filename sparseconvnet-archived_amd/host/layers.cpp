@@ -78,6 +78,18 @@ static void gather_now(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
   output.deferredGatherFrom = nullptr;
 }
 
+// the input's gradient at nf features a site, zero
+static void clear_gradient(cudaMemStream &ms,
+                           SpatiallySparseBatchInterface &input, size_t nf) {
+  const size_t n = (size_t)input.nSpatialSites * nf;
+  const bool cleared = input.gradientCleared && input.sub->dfeatures.size64() == n;
+  input.gradientCleared = false;
+  if (cleared)
+    return;
+  input.sub->dfeatures.resize64(n);
+  input.sub->dfeatures.setZero(ms);
+}
+
 // ConvolutionalLayer::backwards (ConvolutionalLayer.cu:134-147): scatter-add of
 // the gathered matrix's gradient through the rules
 static void conv_backwards(SpatiallySparseBatchInterface &input,
@@ -87,8 +99,7 @@ static void conv_backwards(SpatiallySparseBatchInterface &input,
     return;
   const size_t nIn = input.featuresPresent.size();
   const size_t width = output.featuresPresent.size();
-  input.sub->dfeatures.resize64((size_t)input.nSpatialSites * nIn);
-  input.sub->dfeatures.setZero(ms);
+  clear_gradient(ms, input, nIn);
   SCN_CHECKED(scn_gather_rows_backward(
       ms.ctx, input.sub->dfeatures.dPtr(), output.sub->dfeatures.dPtr(),
       output.rules.dPtr(), (int64_t)output.nSpatialSites * (width / nIn),
@@ -688,8 +699,7 @@ static void pool_backwards(cudaMemStream &ms,
   if (!input.backpropErrors)
     return;
   const size_t nf = output.featuresPresent.size();
-  input.sub->dfeatures.resize64((size_t)input.nSpatialSites * nf);
-  input.sub->dfeatures.setZero(ms);
+  clear_gradient(ms, input, nf);
   SCN_CHECKED(scn_maxpool_backward(
       ms.ctx, input.sub->dfeatures.dPtr(), output.sub->dfeatures.dPtr(),
       output.nSpatialSites, (int)nf, output.sub->poolingChoices.dPtr()));
@@ -947,8 +957,7 @@ void TerminalPoolingLayer::backwards(SpatiallySparseBatch &batch,
   if (!input.backpropErrors)
     return;
   const size_t nf = output.featuresPresent.size();
-  input.sub->dfeatures.resize64((size_t)input.nSpatialSites * nf);
-  input.sub->dfeatures.setZero(memStream);
+  clear_gradient(memStream, input, nf);
   SCN_CHECKED(scn_terminal_pool_backward(
       memStream.ctx, input.sub->dfeatures.dPtr(), output.sub->dfeatures.dPtr(),
       output.rules.dPtr(), output.nSpatialSites, (int)nf,

@@ -17,6 +17,19 @@ def test_fill_touches_its_words_only(scn, ctx, n, off):
     assert np.array_equal(d.download(), want)
 
 
+@pytest.mark.parametrize("sizes", [(1,), (0, 5, 0), (1023, 1, 70001, 0, 4096, 3) * 5])
+def test_fill_of_several_buffers(scn, ctx, sizes):
+    import ctypes
+    bufs = [ctx.array(np.arange(n + 5, dtype=np.int32)) for n in sizes]
+    print("fills", sizes, flush=True)
+    ptrs = (ctypes.c_void_p * len(sizes))(*[b.ptr + 4 * (i % 4) for i, b in enumerate(bufs)])
+    assert scn.lib().scn_fill32_many(ctx.h, ptrs, (ctypes.c_size_t * len(sizes))(*sizes), len(sizes), 7) == 0
+    for i, (b, n) in enumerate(zip(bufs, sizes)):
+        want = np.arange(n + 5, dtype=np.int32)
+        want[i % 4:i % 4 + n] = 7
+        assert np.array_equal(b.download(), want), i
+
+
 # more entries than one workgroup scans, with and without tiled windows, and few; a denser set of sites before
 @pytest.mark.parametrize("d,field,samples,size,stride", [(3, 40, 9, 3, 1), (3, 40, 9, 2, 2), (2, 121, 33, 3, 2), (2, 20, 3, 2, 1)])
 def test_rule_books_on_used_objects(scn, ctx, d, field, samples, size, stride):
