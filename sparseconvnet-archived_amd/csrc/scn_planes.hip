@@ -801,16 +801,17 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   if (rows.d_rows) {
     // Near the line both are launched, each for its numbers of rows; away from
     // it the guess decides, and is held against the counts when they are known.
+    // A kernel launched by itself is launched for every row there may be: where
+    // the guess was wrong its rows are rounded otherwise, not left out.
     const long long split = split_rows(ctx, PL, K, N), hint = scn_rows_hint(ctx, M);
-    const long long few = M < split ? M : split;
     if (M > split && 6 * hint > 5 * split && 5 * hint < 6 * split) {
       RowRange upper = rows;
       rows.upTo = upper.above = split;
-      SCN_TRY(launch_splitk<PL>(ctx, A, W, out, few, K, N, ep, gs, a16, wT, rows));
+      SCN_TRY(launch_splitk<PL>(ctx, A, W, out, split, K, N, ep, gs, a16, wT, rows));
       rows = upper;
     } else if (hint <= split) {
       scn_rows_chosen(ctx, -1, split);
-      return launch_splitk<PL>(ctx, A, W, out, few, K, N, ep, gs, a16, wT, rows);
+      return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
     } else {
       scn_rows_chosen(ctx, split, 1ll << 62);
     }

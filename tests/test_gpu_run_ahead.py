@@ -1,8 +1,13 @@
 """A resident batch's layers queued behind its rule books, their numbers of rows read on the device: whatever batches
 came before, the probabilities and the multiply-adds are those of a net that has seen no other batch (which waits for
 its counts), bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
+
+import brute
+from gpu_util import flatten_samples
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +54,55 @@ def test_layers_ahead_of_the_counts(scn, config, sizes, fused, bf16):
         for x, y in zip(a[2:], w[2:]):
             assert x["nSpatialSites"] == y["nSpatialSites"] and np.array_equal(x["features"], y["features"]), (i, b)
     net.close()
+
+
+def _one_plan(scn, ctx, src, out, samples, nSites, record):
+    """the rule book of a side-2 window over a 41^2 field, deferred or not -> (rules, rows or their bound)"""
+    scn.clear_many(ctx, [src, out])
+    src.build(len(samples), 2, 41, *flatten_samples(samples), nSites)
+    if record:
+        scn.defer_counts(ctx, True)
+        scn.chain_rules(ctx, True)
+    _, rules, n, w = scn.rules_square(ctx, src, 41, 40, 2, 1, 1, out=out)
+    if record:
+        scn.chain_rules(ctx, False)
+        scn.defer_counts(ctx, False)
+    return rules, n
+
+
+# split contraction up to 1248 rows (three planes) and 1792 (one), tiles above: dense batches lie above, sparse ones below
+@pytest.mark.parametrize("precision", ["FP32_PLANES", "BF16"])
+def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
+    """Batches on both sides of the line between two kernels, each queued by the rows of the one before: every row is
+    computed, and where scn_ctx_rows_held says so it is the row that known counts give, bit for bit."""
+    p = getattr(scn, precision)
+    rng = np.random.default_rng(11)
+    nIn, N, fs = 32, 320, 4
+    src, out = scn.Grids(ctx), scn.Grids(ctx)
+    W = (rng.standard_normal((fs * nIn, N)) * 0.1).astype(np.float32)
+    d_W, d_B = ctx.array(W), ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+    seen = []
+    for i, density in enumerate((0.08, 0.08, 0.02, 0.02, 0.08, 0.08, 0.02)):
+        samples, nSites = brute.random_samples(rng, 6, 2, 41, density)
+        inp = rng.standard_normal((nSites, nIn)).astype(np.float32)
+        d_in = ctx.array(inp)
+        rules, bound = _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+        got = ctx.array(np.full((bound, N), 7, np.float32))
+        print("rows ahead", precision, density, bound, flush=True)
+        assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+        ctx.conv_nin_forward(d_in, rules, fs, nIn, d_W, d_B, None, got, bound, N, 1.0, scn.RELU, p)
+        scn.lib().scn_ctx_rows_from(ctx.h, None)
+        assert scn.settle(ctx)
+        held = C.c_int()
+        assert scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK
+        n = out.info()["nSpatialSites"]
+        known = ctx.array(np.full((n, N), 7, np.float32))
+        ctx.conv_nin_forward(d_in, rules, fs, nIn, d_W, d_B, None, known, n, N, 1.0, scn.RELU, p)
+        a, b = got.download(), known.download()
+        # two orders of summation of the same products: a rounding of each of the K partial sums at most
+        assert np.abs(a[:n] - b).max() <= 2 * fs * nIn * 2.0 ** -24 * (np.abs(inp).max() * np.abs(W).sum(0).max() + 0.5)
+        assert (a[n:] == 7).all()
+        assert not held.value or np.array_equal(a[:n], b), (i, n)
+        seen += [held.value] if i else []  # (the first batch's counts are known)
+    # wrong where the density changed and right where it did not
+    assert seen == [1, 0, 1, 0, 1, 0]
