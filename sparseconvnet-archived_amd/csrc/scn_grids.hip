@@ -1526,12 +1526,12 @@ extern "C" int scn_ctx_defer_counts(scn_ctx *ctx, int on) {
 extern "C" int scn_rules_settle(scn_ctx *ctx) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_rules_settle: null context");
   SCN_TRY(scn_chain_flush(ctx));
+  ctx->rowsHeld = true; // (of the passes settled here: none, when nothing is pending)
   if (ctx->pendingGrids.empty())
     return SCN_OK;
   SCN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   std::atomic_thread_fence(std::memory_order_acquire);
   bool overflowed = false;
-  ctx->rowsHeld = true;
   for (const auto &c : ctx->rowsChosen) {
     const volatile int64_t *slot = ctx->h_pinned + 16 + 4 * c.slot;
     ctx->rowsHeld = ctx->rowsHeld && slot[0] > c.above && slot[0] <= c.upTo;

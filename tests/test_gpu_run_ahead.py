@@ -103,6 +103,8 @@ def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
         assert np.abs(a[:n] - b).max() <= 2 * fs * nIn * 2.0 ** -24 * (np.abs(inp).max() * np.abs(W).sum(0).max() + 0.5)
         assert (a[n:] == 7).all()
         assert not held.value or np.array_equal(a[:n], b), (i, n)
-        seen += [held.value] if i else []  # (the first batch's counts are known)
+        seen.append(held.value)
     # wrong where the density changed and right where it did not
-    assert seen == [1, 0, 1, 0, 1, 0]
+    assert seen == [1, 1, 0, 1, 0, 1, 0]
+    # a settling that settles nothing speaks of no earlier pass
+    assert scn.settle(ctx) and scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK and held.value == 1
