@@ -1641,15 +1641,20 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   const bool shape = vec && scn_planes_shape(K);
   const bool few = K <= FR_MAX_K && !(shape && N % 16 == 0);
   bool fewRows = few && scn_rows_hint(ctx, M) <= FR_MAX_M;
-  const bool planes = shape && ((rounded && act != SCN_SOFTMAX) || precision == SCN_FP32_PLANES ||
-                                2e0 * M * K * N >= PLANES_MIN_FLOPS || scn_planes_splitk(ctx, 3, M, K, N));
+  auto takes_planes = [&]() {
+    return shape && ((rounded && act != SCN_SOFTMAX) || precision == SCN_FP32_PLANES ||
+                     2e0 * M * K * N >= PLANES_MIN_FLOPS || scn_planes_splitk(ctx, 3, M, K, N));
+  };
+  bool planes = takes_planes();
   const bool tiledBf16 = vec && K >= 64 && act != SCN_SOFTMAX && rounded && !planes;
   if (dRows && (precision == SCN_FP32 || act == SCN_TANH || act == SCN_SIGMOID ||
                 (act == SCN_SOFTMAX && !(fewRows && N <= 128)) || tiledBf16 || !(planes || fewRows || (vec && (gs ? gs->nIn % 4 != 0 : K <= TK_MAX_K))))) {
     SCN_TRY(scn_rows_exact(ctx, &M));
     if (M == 0)
       return SCN_OK;
+    // (whatever the bound said; tiledBf16 does not depend on the rows)
     fewRows = few && M <= FR_MAX_M;
+    planes = takes_planes();
   }
   if (few && !(planes && rounded))
     scn_rows_chosen(ctx, fewRows ? -1 : FR_MAX_M, fewRows ? FR_MAX_M : 1ll << 62);

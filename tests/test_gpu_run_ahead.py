@@ -70,6 +70,33 @@ def _one_plan(scn, ctx, src, out, samples, nSites, record):
     return rules, n
 
 
+def test_fp32_waits_for_its_rows_and_chooses_by_them(scn, ctx):
+    """SCN_FP32 takes the planes for few rows and for long contractions: queued behind a plan whose bound says otherwise,
+    it gives the bits of the rows that there are."""
+    rng = np.random.default_rng(12)
+    # (few rows under a wide bound; a bound of some 11000 rows makes a long contraction, 3900 of them do not)
+    for nIn, N, densities in ((32, 320, (0.08, 0.08, 0.02)), (1024, 1024, (0.5, 0.5, 0.12))):
+        fs, src, out = 4, scn.Grids(ctx), scn.Grids(ctx)
+        d_W = ctx.array((rng.standard_normal((fs * nIn, N)) * 0.1).astype(np.float32))
+        d_B = ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+        for i, density in enumerate(densities):
+            samples, nSites = brute.random_samples(rng, 6, 2, 41, density)
+            d_in = ctx.array(rng.standard_normal((nSites, nIn)).astype(np.float32))
+            rules, bound = _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+            got = ctx.array(np.full((bound, N), 7, np.float32))
+            print("fp32 ahead", density, nIn, bound, flush=True)
+            assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+            ctx.conv_nin_forward(d_in, rules, fs, nIn, d_W, d_B, None, got, bound, N, 1.0, scn.RELU, scn.FP32)
+            scn.lib().scn_ctx_rows_from(ctx.h, None)
+            assert scn.settle(ctx)
+            held = C.c_int()
+            assert scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK and held.value == 1
+            n = out.info()["nSpatialSites"]
+            known = ctx.array(np.full((n, N), 7, np.float32))
+            ctx.conv_nin_forward(d_in, rules, fs, nIn, d_W, d_B, None, known, n, N, 1.0, scn.RELU, scn.FP32)
+            assert np.array_equal(got.download()[:n], known.download()), (density, n, bound)
+
+
 # split contraction up to 1248 rows (three planes) and 1792 (one), tiles above: dense batches lie above, sparse ones below
 @pytest.mark.parametrize("precision", ["FP32_PLANES", "BF16"])
 def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
