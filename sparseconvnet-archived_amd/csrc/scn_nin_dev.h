@@ -83,6 +83,7 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
 // dW += A^T D
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
                    long long M, int K, int N);
-// out = A Wt^T; false: the caller's other way
+// out = A Wt^T; false: the caller's other way, or (transpose) scn_planes_forward
+// on the transpose
 bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
-                    long long M, int K, int N, const float *zeros, int *rc);
+                    long long M, int K, int N, const Epilogue &ep, int *rc, bool *transpose);

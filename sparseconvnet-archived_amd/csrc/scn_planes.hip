@@ -615,9 +615,15 @@ void scn_image_context(scn_ctx *ctx, bool alive) {
     g_images.spare.clear();
   }
 }
-// False: convert on the way instead -- no memory, or the stream is being
-// captured and may not allocate.
+// False: convert on the way instead -- the stream is being captured (a graph may
+// be replayed beside the context's own calls, whose weights the room holds, and
+// after the context; nor may a capture allocate), or there is no memory.
 static bool planes_image(scn_ctx *ctx) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
   if (ctx->d_image)
     return true;
   {
@@ -630,10 +636,7 @@ static bool planes_image(scn_ctx *ctx) {
         return true;
       }
   }
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess ||
-      capturing != hipStreamCaptureStatusNone ||
-      hipMalloc((void **)&ctx->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
+  if (hipMalloc((void **)&ctx->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
     (void)hipGetLastError();
     ctx->d_image = nullptr;
     return false;
@@ -848,19 +851,19 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16, choice);
 }
 
-// out = A Wt^T for Wt [N x K].  False: not a shape for it, or no room for the
-// image (nothing has been launched).
+// out = A Wt^T for Wt [N x K].  False: nothing has been launched; not a shape for
+// it, or (transpose) one that scn_planes_forward takes to the same bits from the
+// transpose, because the image may not be used now.
 bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
-                    long long M, int K, int N, const float *zeros, int *rc) {
+                    long long M, int K, int N, const Epilogue &ep, int *rc, bool *transpose) {
+  *transpose = false;
   if (!scn_planes_shape(K) || ((uintptr_t)A & 15) || ((uintptr_t)out & 15) || N % 4 != 0)
     return false;
   const PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
-  if (choice.tile >= 0 && (!choice.image || !planes_image(ctx)))
+  if (choice.tile >= 0 && !(choice.image && planes_image(ctx))) {
+    *transpose = choice.image;
     return false;
-  Epilogue ep = Epilogue();
-  ep.bias = zeros;
-  ep.p = 1.f;
-  ep.act = SCN_NOSIGMOID;
+  }
   *rc = planes_forward<3>(ctx, A, Wt, out, M, K, N, ep, nullptr, false, choice, true);
   return true;
 }

@@ -265,10 +265,15 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
     return SCN_OK;
   SCN_REQUIRE(d_D && d_W && d_dA && d_workspace, SCN_ERR_ARG,
               "scn_sgemm_ABt: null buffer");
+  bool transpose = false;
+  Epilogue ep = Epilogue();
+  ep.bias = ctx->d_zeros;
+  ep.p = 1.f;
+  ep.act = SCN_NOSIGMOID;
   if (K <= SCN_ZERO_FLOATS) { // the planes read W [K x N] as it stands
     int rc = SCN_OK;
     ProfScope prof(ctx, SCN_K_BACKWARD);
-    if (scn_planes_abt(ctx, d_D, d_W, d_dA, (long long)M, N, K, ctx->d_zeros, &rc)) {
+    if (scn_planes_abt(ctx, d_D, d_W, d_dA, (long long)M, N, K, ep, &rc, &transpose)) {
       SCN_TRY(rc);
       SCN_HIP_CHECK(hipGetLastError());
       return SCN_OK;
@@ -285,6 +290,12 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
       zeros = ctx->d_zeros;
     else
       SCN_TRY(scn_fill32(ctx, zeros, 0, (size_t)K));
+  }
+  if (transpose) {
+    ProfScope prof(ctx, SCN_K_BACKWARD);
+    SCN_TRY(scn_planes_forward(ctx, 3, d_D, Wt, d_dA, (long long)M, N, K, ep, nullptr, false));
+    SCN_HIP_CHECK(hipGetLastError());
+    return SCN_OK;
   }
   return scn_nin_forward(ctx, d_D, Wt, zeros, nullptr, d_dA, M, N, K, 1.0f,
                          SCN_NOSIGMOID, SCN_FP32);
