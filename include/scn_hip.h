@@ -19,10 +19,11 @@
  *   - feature matrices are row-major fp32 [rows x channels]; rule books are
  *     row-major int32 [output rows x rule width]; rows are batch-global;
  *   - numeric kernels never allocate: every buffer is the caller's
- *     (SpatiallySparseBatchSubInterface, SpatiallySparseBatchInterface.h:8-17);
- *     the one exception is the context's own copy of a layer's weights, which a
- *     long contraction makes and the context keeps (never while its stream is
- *     being captured: the weights are then converted on the way).
+ *     (SpatiallySparseBatchSubInterface, SpatiallySparseBatchInterface.h:8-17).
+ *     A long contraction puts its layer's weights, laid out for the matrix
+ *     cores, into room that scn_ctx_create has made for the context (16 MB;
+ *     never while its stream is being captured, or where there was no memory
+ *     for it: the weights are then converted on the way, to the same bits).
  *     scn_grids objects own their tables and only ever grow them.
  */
 #ifndef SCN_HIP_H

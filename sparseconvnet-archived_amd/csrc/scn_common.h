@@ -130,9 +130,6 @@ static inline int scn_ceil_div(int64_t a, int64_t b) {
 int scn_abt_static_setup(int device);
 void scn_abt_static_forget(const scn_ctx *ctx);
 
-// counts contexts, and takes back ctx's image when one goes (scn_planes.hip)
-void scn_image_context(scn_ctx *ctx, bool alive);
-
 // For a feature call that can not read its rows on the device: waits for the
 // stream and replaces the bound M by the rows there are (per: rows of the call
 // for each of the grids' rows).

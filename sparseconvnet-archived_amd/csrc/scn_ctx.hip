@@ -52,12 +52,16 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   SCN_HIP_CHECK(hipMalloc((void **)&c->d_scalars, 16 * sizeof(int64_t)));
   SCN_HIP_CHECK(hipMemset(c->d_scalars, 0, 16 * sizeof(int64_t)));
   SCN_HIP_CHECK(hipMalloc((void **)&c->d_zeros, SCN_ZERO_FLOATS * sizeof(float)));
+  // (here and not with the first long contraction: numeric calls never allocate)
+  if (hipMalloc((void **)&c->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
+    (void)hipGetLastError();
+    c->d_image = nullptr;
+  }
   // (on the context's own stream: HIP gives a stream its hardware queue with
   // the first work it gets, which takes about a millisecond -- here rather
   // than in front of the first batch that happens to use the stream)
   SCN_HIP_CHECK(hipMemsetAsync(c->d_zeros, 0, SCN_ZERO_FLOATS * sizeof(float), c->stream));
   SCN_HIP_CHECK(hipStreamSynchronize(c->stream));
-  scn_image_context(c, true);
   *out = c;
   return SCN_OK;
 }
@@ -69,7 +73,6 @@ extern "C" int scn_ctx_destroy(scn_ctx *c) {
   (void)hipStreamSynchronize(c->stream);
   scn_abt_static_forget(c);
   scn_chain_release(c);
-  scn_image_context(c, false);
   for (auto &s : c->spans) {
     (void)hipEventDestroy(s.a);
     (void)hipEventDestroy(s.b);
@@ -78,6 +81,7 @@ extern "C" int scn_ctx_destroy(scn_ctx *c) {
     (void)hipEventDestroy(e);
   (void)hipFree(c->d_scalars);
   (void)hipFree(c->d_zeros);
+  (void)hipFree(c->d_image);
   (void)hipHostFree(c->h_pinned);
   (void)hipStreamDestroy(c->stream);
   delete c;

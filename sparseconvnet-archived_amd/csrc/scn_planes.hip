@@ -591,57 +591,16 @@ __global__ void __launch_bounds__(256)
                                 (kg & 1) * 512 + cc * 16) = p[l];
 }
 
-// Room for an image: the context's from its first long contraction on.  Up to
-// four rooms of closed contexts are kept for the next ones (a new 16 MB costs
-// the first batch of a net half a millisecond) until the last context is gone.
-static struct {
-  std::mutex m;
-  int contexts = 0;
-  std::vector<std::pair<int, unsigned char *>> spare; // (device, room)
-} g_images;
-void scn_image_context(scn_ctx *ctx, bool alive) {
-  std::lock_guard<std::mutex> lock(g_images.m);
-  g_images.contexts += alive ? 1 : -1;
-  if (!alive && ctx->d_image) { // (its stream has been waited for)
-    if (g_images.spare.size() < 4)
-      g_images.spare.push_back({ctx->device, ctx->d_image});
-    else
-      (void)hipFree(ctx->d_image);
-    ctx->d_image = nullptr;
-  }
-  if (g_images.contexts == 0) {
-    for (auto &s : g_images.spare)
-      (void)hipFree(s.second);
-    g_images.spare.clear();
-  }
-}
 // False: convert on the way instead -- the stream is being captured (a graph may
 // be replayed beside the context's own calls, whose weights the room holds, and
-// after the context; nor may a capture allocate), or there is no memory.
+// after the context), or the context found no memory for the room.
 static bool planes_image(scn_ctx *ctx) {
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  if (ctx->d_image)
-    return true;
-  {
-    std::lock_guard<std::mutex> lock(g_images.m);
-    for (auto &s : g_images.spare)
-      if (s.first == ctx->device) {
-        ctx->d_image = s.second;
-        std::swap(s, g_images.spare.back());
-        g_images.spare.pop_back();
-        return true;
-      }
-  }
-  if (hipMalloc((void **)&ctx->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
-    (void)hipGetLastError();
-    ctx->d_image = nullptr;
-    return false;
-  }
-  return true;
+  return ctx->d_image && capturing == hipStreamCaptureStatusNone;
 }
 
 // Blocks ahead: two where the registers allow it (a wavefront alone on its SIMD

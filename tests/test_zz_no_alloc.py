@@ -92,6 +92,39 @@ def test_the_static_call_allocates_nothing(scn, ctx):
         fresh.close()
 
 
+# the static product by the split contraction and by the tiles that stream a copy of the weights; the other long ones
+@pytest.mark.parametrize("what,M", [("static", 60000), ("conv", 66000), ("conv bf16", 66000), ("ABt", 60000), ("AtB", 9000)])
+def test_numeric_calls_of_a_new_context_allocate_nothing(scn, ctx, what, M):
+    rng = np.random.default_rng(8)
+    N, K, fs = 256, 512, 27
+    c = scn.Context()
+    try:
+        if what.startswith("conv"):
+            x, rules = c.array(rng.standard_normal((300, 64), dtype=np.float32)), c.array(
+                rng.integers(0, 300, (M, fs)).astype(np.int32))
+            W, B, out = c.array(rng.standard_normal((fs * 64, 64), dtype=np.float32)), c.array(np.zeros(64, np.float32)), c.empty(
+                (M, 64), np.float32)
+        else:
+            D, W = c.array(rng.standard_normal((M, N), dtype=np.float32)), c.array(rng.standard_normal((K, N), dtype=np.float32))
+            A, out = c.empty((M, K), np.float32), c.empty((K, N), np.float32)
+            ws = c.empty(scn.lib().scn_sgemm_ABt_workspace(N, K), np.float32)
+        c.sync()
+        before = free_device_memory()
+        if what == "static":
+            c.sgemm_ABt_static(D, W, A, M, N, K)
+        elif what == "ABt":
+            c.sgemm_ABt(D, W, A, M, N, K, ws)
+        elif what == "AtB":
+            c.sgemm_AtB(A, D, out, M, K, N)
+        else:
+            c.conv_nin_forward(x, rules, fs, 64, W, B, None, out, M, 64, 1.0, scn.RELU,
+                               scn.BF16 if "bf16" in what else scn.FP32_PLANES)
+        c.sync()
+        assert free_device_memory() == before
+    finally:
+        c.close()
+
+
 def test_a_second_context_waits_its_turn(scn, ctx):
     """The array is one per device: a call from another context is refused while the last call that used the array
     has not finished, and accepted once it has."""
