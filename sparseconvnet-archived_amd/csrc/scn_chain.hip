@@ -1223,8 +1223,8 @@ int scn_chain_record_regions(scn_ctx *ctx, scn_grids *in, scn_grids *out,
     return SCN_OK;
   ChainState *cs = ctx->chain;
   const long long volOutAll = (long long)in->batch * g.volOut;
-  const long long boundActive = grow_bound(out->seenActive, 64, volOutAll);
-  const long long boundRows = grow_bound(out->seenRows, 64, boundActive + in->batch);
+  const long long boundActive = grow_bound(out->nextActive, out->seenActive, 64, volOutAll);
+  const long long boundRows = grow_bound(out->nextRows, out->seenRows, 64, boundActive + in->batch);
   if (boundRows >= 2147483647ll)
     return SCN_OK;
   SCN_TRY(out->meta.reserve(8));
@@ -1274,7 +1274,7 @@ int scn_chain_record_terminal(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   if (out->seenWidth <= 0 || !chain_accepts(ctx, in, out, 1))
     return SCN_OK;
   ChainState *cs = ctx->chain;
-  const long long boundWidth = grow_bound(out->seenWidth, 8, in->vol);
+  const long long boundWidth = grow_bound(out->nextWidth, out->seenWidth, 8, in->vol);
   SCN_TRY(out->meta.reserve(8));
   SCN_TRY(out->ekey.reserve((size_t)in->batch + 1));
   SCN_TRY(out->erow.reserve((size_t)in->batch + 1));

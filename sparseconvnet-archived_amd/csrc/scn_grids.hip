@@ -1508,9 +1508,12 @@ static Count count_width(const scn_grids *g) {
   c.live = g->pending ? g->meta.p + META_WIDTH : nullptr;
   return c;
 }
-long long grow_bound(long long seen, long long slack, long long cap) {
-  long long b = seen + seen / 4 + slack;
-  return b < cap ? b : cap;
+// A quarter more than has been seen; it stands while a sixteenth of that is left,
+// so that the buffers sized by it are not outgrown with every new maximum.
+long long grow_bound(long long &bound, long long seen, long long slack, long long cap) {
+  if (bound < seen + seen / 16)
+    bound = seen + seen / 4 + slack;
+  return bound < cap ? bound : cap;
 }
 
 // Deferred counts.  With deferral on, a plan whose output object has held a
@@ -1778,9 +1781,9 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   const long long *inMeta = in->pending ? in->meta.p : nullptr;
   const long long volOutAll = (long long)in->batch * g.volOut;
   const long long boundActive =
-      deferred ? grow_bound(out->seenActive, 64, volOutAll) : 0x7FFFFFFFFFFFll;
+      deferred ? grow_bound(out->nextActive, out->seenActive, 64, volOutAll) : 0x7FFFFFFFFFFFll;
   const long long boundRows =
-      deferred ? grow_bound(out->seenRows, 64, boundActive + in->batch)
+      deferred ? grow_bound(out->nextRows, out->seenRows, 64, boundActive + in->batch)
                : 0x7FFFFFFFFFFFll;
   const int slot = deferred ? (int)ctx->pendingGrids.size() : -1;
   SCN_TRY(out->meta.reserve(8));
@@ -2146,7 +2149,7 @@ extern "C" int scn_rules_terminal_plan(scn_ctx *ctx, const scn_grids *cin,
   SCN_TRY(out->sampleStart.reserve((size_t)in->batch + 2));
   SCN_TRY(out->meta.reserve(8));
   const long long boundWidth =
-      deferred ? grow_bound(out->seenWidth, 8, in->vol) : 0x7FFFFFFFFFFFll;
+      deferred ? grow_bound(out->nextWidth, out->seenWidth, 8, in->vol) : 0x7FFFFFFFFFFFll;
   const int slot = deferred ? (int)ctx->pendingGrids.size() : -1;
   const long long ticket = ++ctx->ticket;
   hipLaunchKernelGGL(k_terminal_plan, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream,

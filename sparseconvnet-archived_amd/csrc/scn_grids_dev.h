@@ -113,10 +113,11 @@ struct scn_grids {
   // Deferred counts: while pending, nActive / nSites / termS hold upper bounds
   // and the real values are in meta (device) and on their way to the pinned
   // slot; seen* are the largest values this object has ever held, from which
-  // the next bounds are derived.
+  // the next bounds, next*, are derived.
   bool pending = false;
   int pinnedSlot = -1;
   long long seenRows = 0, seenActive = 0, seenWidth = 0;
+  long long nextRows = 0, nextActive = 0, nextWidth = 0;
   // the last settled plan, to guess the next one by
   long long lastRows = 0, lastBatch = 0;
   DevBuf<long long> meta; // META_* words
@@ -695,7 +696,7 @@ __device__ __forceinline__ int split_site(long long p, long long vol, int n,
 
 // ---- host helpers shared by scn_grids.hip and scn_chain.hip
 GridView view_of(const scn_grids *g);
-long long grow_bound(long long seen, long long slack, long long cap);
+long long grow_bound(long long &bound, long long seen, long long slack, long long cap);
 void mark_pending(scn_ctx *ctx, scn_grids *g, int slot);
 // fills the hash table of grids that do not have it yet (scn_grids.hip)
 int scn_grids_ensure_table(scn_ctx *ctx, scn_grids *g);

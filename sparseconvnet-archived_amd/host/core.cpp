@@ -277,7 +277,7 @@ template <typename t> void vectorCUDA<t>::setUniform(float a, float b) {
 template <typename t> void vectorCUDA<t>::resize(int n) {
   resize64((size_t)(n < 0 ? 0 : n));
 }
-template <typename t> void vectorCUDA<t>::resize64(size_t n) {
+template <typename t> void vectorCUDA<t>::resize64(size_t n, size_t head) {
   if (!onGPU) {
     vec.resize(n);
     return;
@@ -285,7 +285,7 @@ template <typename t> void vectorCUDA<t>::resize64(size_t n) {
   if (n > dAllocated) {
     if (d_vec)
       SCN_CHECKED(scn_free(nullptr, d_vec));
-    size_t want = n + n / 4;
+    size_t want = n + n / 4 + head;
     void *p = nullptr;
     SCN_CHECKED(scn_malloc(scnDefaultContext(), want * sizeof(t), &p));
     d_vec = (t *)p;

@@ -57,7 +57,8 @@ public:
   void setUniform(float a = 0, float b = 1);
   void resize(int n);
   // 64-bit clean variants: the reference's int sizes overflow on feature
-  // matrices beyond 2^31 elements (large 3-D batches)
-  void resize64(size_t n);
+  // matrices beyond 2^31 elements (large 3-D batches).  An allocation leaves
+  // room for a quarter more and `head` elements.
+  void resize64(size_t n, size_t head = 0);
   size_t size64();
 };

@@ -135,3 +135,32 @@ def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
     assert seen == [1, 1, 0, 1, 0, 1, 0]
     # a settling that settles nothing speaks of no earlier pass
     assert scn.settle(ctx) and scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK and held.value == 1
+
+
+def test_the_second_batch_finds_room_in_the_firsts_buffers(scn):
+    """The bounds that a pass ahead of its counts is queued with fit the buffers that the first batch has left: none is
+    allocated anew for a batch of the same kind (each a wait for the device)."""
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    cfg = synthetic.config(2, batch=100)
+    net = _net(cfg, None, False)
+    weights = synthetic.he_normal_weights(net.layers(), 5)
+    net.close()
+    net = _net(cfg, weights, False)
+    ctx = scn.Context(handle=net.context_handle())
+    hip, free = C.CDLL("libamdhip64.so"), []
+    batches = []
+    for i in range(3):
+        S, K, R, bg, feats, n = synthetic.codify(synthetic.make_samples(cfg, 400 + i), cfg.dimension, cfg.lattice,
+                                                 net.inputSpatialSize, cfg.nInputFeatures)
+        batches.append(([ctx.array(S, np.int32), ctx.array(K, np.int64), ctx.array(R, np.int32), ctx.array(bg, np.int32)],
+                        len(K), n, ctx.array(feats, np.float32)))
+    for d, k, n, f in batches:
+        p = np.zeros((100, cfg.nClasses), np.float32)
+        net.forward_resident(100, d[0].ptr, d[1].ptr, d[2].ptr, d[3].ptr, k, n, f.ptr, p)
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        free.append(a.value)
+    net.close()
+    print("free memory taken", free[0] - free[1], free[1] - free[2], flush=True)
+    # (the layers' buffers anew were 48 MB; the second batch's recorded plans need some masks and tables of their own)
+    assert free[0] - free[1] <= 8 << 20 and free[1] == free[2]
