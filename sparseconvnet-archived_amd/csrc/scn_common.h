@@ -60,6 +60,7 @@ struct scn_ctx {
   // deferred counts (scn_ctx_defer_counts): plans whose counts are still on
   // their way; slot i of them reports into h_pinned[16 + 4 i ..]
   bool deferCounts;
+  bool wstream; // NiN: W-streaming kernel allowed (SCN_NIN_WSTREAM=0 turns it off)
   std::vector<struct scn_grids *> pendingGrids;
   // scn_ctx_rows_from: where the feature kernels read their number of rows
   // (META_* words of the grids), the bound they were launched with, and the

@@ -32,6 +32,10 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   c->profTag = 0;
   c->ticket = 0;
   c->deferCounts = false;
+  {
+    const char *e = getenv("SCN_NIN_WSTREAM");
+    c->wstream = !(e && e[0] == '0');
+  }
   c->chain = nullptr;
   c->d_meta = nullptr;
   c->rowsHeld = true;

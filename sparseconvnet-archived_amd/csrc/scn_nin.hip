@@ -1704,7 +1704,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
     SCN_TRY(scn_planes_forward(ctx, 3, d_A, d_W, d_out, M, K, N, ep, gs, false));
   } else if (vec && wres_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
     // W-resident kernel took it
-  } else if (vec && wstream_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
+  } else if (vec && ctx->wstream && wstream_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
     // W-streaming kernel took it
   } else if ((vec && K >= 8) || gs) {
     // Tall tiles (128 rows), 64 columns wide, or 96 where that divides N

@@ -168,6 +168,28 @@ def test_nin_fp32_squashing_activations(scn, ctx, M, K, N, act):
     assert np.allclose(orc.nin_forward(A, W, B, None, 0.9, a), closed, rtol=1e-4, atol=1e-5)
 
 
+def test_nin_fp32_wstream_switch(scn, ctx, monkeypatch):
+    """SCN_NIN_WSTREAM=0, read when a context is created: the W-streaming kernel's shapes on the tiled one, another order
+    of summation."""
+    rng = np.random.default_rng(17)
+    M, K, N = 14000, 1728, 64  # (no few rows, no long contraction)
+    A, W = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((K, N), dtype=np.float32)
+    d_A, d_W, d_B = ctx.array(A), ctx.array(W), ctx.array(np.zeros(N, np.float32))
+    got = []
+    for value in (None, "0", "1"):
+        monkeypatch.setenv("SCN_NIN_WSTREAM", value) if value else monkeypatch.delenv("SCN_NIN_WSTREAM", raising=False)
+        c = scn.Context()
+        out = ctx.array(np.full((M, N), 7, np.float32))
+        c.nin_forward(d_A, d_W, d_B, None, out, M, K, N, 1.0, scn.NOSIGMOID, scn.FP32)
+        c.sync()
+        got.append(out.download())
+        c.close()
+    assert np.array_equal(got[0], got[2]) and not np.array_equal(got[0], got[1])
+    # a rounding of each of the K partial sums at most, in either order
+    scale = np.abs(A[:500]).astype(np.float64) @ np.abs(W).astype(np.float64)
+    assert np.all(np.abs(got[0][:500] - got[1][:500].astype(np.float64)) <= 2 * K * 2.0 ** -24 * scale)
+
+
 def test_nin_special_cases(scn, ctx):
     rng = np.random.default_rng(3)
     M, K = 70, 64
