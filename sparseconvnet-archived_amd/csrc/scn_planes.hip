@@ -56,8 +56,11 @@ struct RowRange {
 
 // An infinite operand, or one that rounds to an infinite bf16, leaves NaN in its
 // other planes (x - hi), where fp32 arithmetic has an infinity or a finite sum.
-// So with three planes a sum that is not finite is taken again from the
-// operands themselves; the test costs an instruction a result.
+// So with three planes a sum that is not finite is taken again from the operands
+// themselves; the test costs an instruction a result.  The tiles that hold such
+// sums are taken again whole, on the fp32 MFMA: a net whose weights have all gone
+// to infinities costs a few times what a sound one does, not a serial chain of K
+// a result.
 template <int PL> __device__ __forceinline__ bool doubtful(float sum) {
   return PL == 3 && !(fabsf(sum) <= 3.4028235e38f);
 }
@@ -65,22 +68,12 @@ struct PlainW { // W as the caller gave it
   const float *W;
   int wT; // [N x K] and not [K x N]
 };
-// Row m of A (GATHER: through rules, fs of them, in LDS) times column n of W.
-template <bool GATHER>
-__device__ __forceinline__ float plain_sum(const float *A, const GatherSource &gs, const int *rules,
-                                           const PlainW &w, long long m, int n, int K, int N) {
-  const float *const wp = w.W + (w.wT ? (long long)n * K : n);
-  const int stride = w.wT ? 1 : N, run = GATHER ? gs.nIn : K;
-  float sum = 0.f;
-  for (int k0 = 0, f = 0; k0 < K; k0 += run, ++f) {
-    const float *a = A + m * K;
-    if (GATHER)
-      a = rules[f] >= 0 ? A + (long long)rules[f] * run : gs.zeros;
-#pragma unroll 1
-    for (int i = 0; i < run; ++i)
-      sum = fmaf(a[i], wp[(long long)(k0 + i) * stride], sum);
-  }
-  return sum;
+// Eight k of a 32 x 32 tile on v_mfma_f32_32x32x2_f32: lane (c, q) holds a[i] and
+// b[i] of the same k for its row of A and column of W.
+__device__ __forceinline__ void mfma8_f32(const float (&a)[8], const float (&b)[8], floatx16 &acc) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[i], acc, 0, 0, 0);
 }
 
 // Four channels (A16: eight) of a gathered row: columns k .. of the row that
@@ -93,6 +86,45 @@ __device__ __forceinline__ floatx4 gathered_piece(const unsigned char *A, const 
   const unsigned char *const row = rule >= 0 ? A + (long long)rule * gs.nIn * (A16 ? 2 : 4)
                                              : reinterpret_cast<const unsigned char *>(gs.zeros);
   return *reinterpret_cast<const floatx4 *>(row + (k - f * gs.nIn) * (A16 ? 2 : 4));
+}
+
+// A 32 x 32 tile on the fp32 MFMA by one wavefront: row m of A (GATHER: through
+// its rules, in LDS) and column n of W are this lane's, as in mfma8_f32; `mine`
+// are the registers of the result it has a use for.
+template <bool GATHER>
+__device__ __forceinline__ floatx16 tile_f32(const float *A, const GatherSource &gs, const int *rules,
+                                             const PlainW &w, long long m, int n, int K, int N, unsigned mine) {
+  const int q = (threadIdx.x & 63) >> 5;
+  floatx16 sum;
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    sum[v] = 0.f;
+#pragma unroll 1
+  for (int t = 0; t < K; t += 16) { // (K is a multiple of 32)
+    const int k = t + 8 * q;
+    float a[8], b[8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const floatx4 x = GATHER ? gathered_piece<false>(reinterpret_cast<const unsigned char *>(A), gs, rules, k + 4 * h)
+                               : *reinterpret_cast<const floatx4 *>(A + m * K + k + 4 * h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a[4 * h + i] = x[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      b[i] = w.W[w.wT ? (long long)n * K + k + i : (long long)(k + i) * N + n];
+    mfma8_f32(a, b, sum);
+    if (t % 128 == 112) { // a NaN stays one: through when there is nothing else
+      bool open = false;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        open |= (mine >> v & 1) && sum[v] == sum[v];
+      if (!__any(open))
+        break;
+    }
+  }
+  return sum;
 }
 
 // A workgroup of four wavefronts owns 128 MT rows x 32 NT columns, a wavefront
@@ -427,13 +459,27 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
       }
     }
   }
-  for (; again; again &= again - 1) {
-    const int e = __ffsll(again) - 1, v = e & 15, j = (e >> 4) % NT;
-    const int dr = 32 * ((e >> 4) / NT) + 8 * (v / 4) + 4 * q + v % 4;
-    if (row0 + dr < M && n + j < N)
-      out[(row0 + dr) * N + n + j] =
-          finish(plain_sum<GATHER != 0>(A, gs, sRules + (wave * 32 * MT + dr) * gs.fs, plain, row0 + dr, n + j, K, N),
-                 load_col(ep, n + j));
+  if constexpr (PL == 3) {
+    if (!__any(again != 0))
+      return;
+#pragma unroll 1
+    for (int e = 0; e < MT * NT; ++e) { // tile (i, j); uniform
+      const unsigned mine = (unsigned)(again >> (16 * e)) & 0xffffu;
+      if (!__any(mine != 0))
+        continue;
+      const int i = e / NT, j = e % NT;
+      long long m = row0 + 32 * i + c;
+      m = m < M ? m : M - 1;
+      const int nn = n + j < N ? n + j : N - 1;
+      const floatx16 sum = tile_f32<GATHER != 0>(A, gs, sRules + (m - wgRow0) * gs.fs, plain, m, nn, K, N, mine);
+      const ColEpilogue last = load_col(ep, nn);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long long r = row0 + 32 * i + 8 * (v / 4) + 4 * q + v % 4;
+        if ((mine >> v & 1) && r < M && n + j < N)
+          out[r * N + n + j] = finish(sum[v], last);
+      }
+    }
   }
 }
 
@@ -543,20 +589,36 @@ __global__ void __launch_bounds__(512, 2)
   for (int v = 0; v < 16; ++v)
     sPart[(wave * 16 + v) * 64 + lane] = NACC == 2 ? acc[0][v] + acc[NACC - 1][v] : acc[0][v];
   __syncthreads();
-  // register v of lane (c, q) is row 8 (v / 4) + 4 q + v % 4
+  // register v of lane (c, q) is row 8 (v / 4) + 4 q + v % 4; this wavefront's
+  // are v = wave and wave + 8
+  float sum[2];
+  unsigned again = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int v = 8 * h + wave;
+    sum[h] = sPart[v * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 8; ++w)
+      sum[h] += sPart[(w * 16 + v) * 64 + lane];
+    if (doubtful<PL>(sum[h]))
+      again |= 1u << v;
+  }
+  if constexpr (PL == 3) {
+    if (__any(again != 0)) {
+      const floatx16 plain =
+          tile_f32<GATHER>(A, gs, sRules + (GATHER ? (int)(m - row0) * gs.fs : 0), PlainW{W, WT}, m, n, K, N, again);
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (again >> v & 1)
+          sum[v / 8] = plain[v];
+    }
+  }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int v = 8 * h + wave;
     const int dr = 8 * (v / 4) + 4 * q + v % 4;
-    if (row0 + dr >= M || n0 + c >= N)
-      continue;
-    float sum = sPart[v * 64 + lane];
-#pragma unroll
-    for (int w = 1; w < 8; ++w)
-      sum += sPart[(w * 16 + v) * 64 + lane];
-    if (doubtful<PL>(sum))
-      sum = plain_sum<GATHER>(A, gs, sRules + dr * gs.fs, PlainW{W, WT}, row0 + dr, n0 + c, K, N);
-    out[(row0 + dr) * N + n0 + c] = finish(sum, load_col(ep, n0 + c));
+    if (row0 + dr < M && n0 + c < N)
+      out[(row0 + dr) * N + n0 + c] = finish(sum[h], load_col(ep, n0 + c));
   }
 }
 
@@ -846,7 +908,8 @@ __global__ void __launch_bounds__(512, 2)
                  long long rowsPerSplit) {
   constexpr int PL = 3, GM = 8;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
-  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE]
+  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], then a flag
+  int *const sAgain = reinterpret_cast<int *>(sTile + 8 * TILE);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
   const int k0 = (blockIdx.x / nTiles) * 32 * MT;
@@ -965,37 +1028,87 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         sTile[wave * TILE + ((i * NT + j) * 16 + v) * 64 + lane] = acc[0][i][j][v] + acc[1][i][j][v];
+  if (tid == 0)
+    *sAgain = 0;
   __syncthreads();
   // element e of the tile: register v of lane l of sub-tile (i, j): row (of dW)
   // MT (8 (v / 4) + 4 (l / 32) + v % 4) + i, column NT (l % 32) + j
-  for (int e = tid; e < TILE; e += 512) {
+  auto add = [&](int e) {
     float sum = 0.f;
 #pragma unroll
     for (int g = 0; g < GM; ++g)
       sum += sTile[g * TILE + e];
+    return sum;
+  };
+  auto put = [&](int e, float sum) {
     const int l = e & 63, v = (e >> 6) & 15, ij = e >> 10;
     const int kk = k0 + MT * (8 * (v / 4) + 4 * (l >> 5) + v % 4) + ij / NT;
     const int nn = n0 + NT * (l & 31) + ij % NT;
-    if (kk >= K || nn >= N)
-      continue;
-    if (doubtful<PL>(sum)) {
-      sum = 0.f;
-#pragma unroll 1
-      for (long long r = m0; r < m1; ++r)
-        sum = fmaf(A[r * K + kk], D[r * N + nn], sum);
+    if (kk < K && nn < N)
+      unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
+  };
+  unsigned again = 0; // this lane's elements that are to be taken again
+  for (int e = tid; e < TILE; e += 512) {
+    const float sum = add(e);
+    if (doubtful<PL>(sum))
+      again |= 1u << (e / 512);
+    else
+      put(e, sum);
+  }
+  if (again)
+    *sAgain = 1;
+  __syncthreads();
+  if (*sAgain) { // the workgroup's rows on the fp32 MFMA, two a step
+    floatx16 plain[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          plain[i][j][v] = 0.f;
+#pragma unroll 4
+    for (long long r0 = m0 + 2 * wave; r0 < m1; r0 += 2 * GM) {
+      const int l = __lane_id(); // (anew: its columns need no registers until here)
+      const long long r = r0 + (l >> 5);
+      int ka = k0 + MT * (l & 31), na = n0 + NT * (l & 31);
+      ka = ka + MT <= K ? ka : K - MT;
+      na = na + NT <= N ? na : N - NT;
+      float a[MT], d[NT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        a[i] = r < m1 ? A[r * K + ka + i] : 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        d[j] = r < m1 ? D[r * N + na + j] : 0.f;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          plain[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], d[j], plain[i][j], 0, 0, 0);
     }
-    unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          sTile[wave * TILE + ((i * NT + j) * 16 + v) * 64 + lane] = plain[i][j][v];
+    __syncthreads();
+    for (int e = tid; e < TILE; e += 512)
+      if (again >> (e / 512) & 1)
+        put(e, add(e));
   }
 }
 
 template <int MT, int NT>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
                       long long M, int K, int N, long long splits) {
-  const size_t lds = (size_t)8 * 32 * MT * 32 * NT * sizeof(float);
+  const size_t lds = ((size_t)8 * 32 * MT * 32 * NT + 1) * sizeof(float);
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
                ? SCN_OK
                : SCN_ERR_HIP;
   });

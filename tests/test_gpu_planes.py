@@ -164,3 +164,40 @@ def test_one_plane_against_float64(scn, ctx, rows, fs, nIn, N):
     scale = np.abs(A).astype(np.float64) @ np.abs(W).astype(np.float64) + np.abs(B)
     # products exact, their sum in fp32: a rounding every eight or sixteen of the K
     assert np.all(np.abs(got[some] - want) <= 2e-6 * scale)
+
+
+# a contraction of the tiles, the split contraction, the input gradient, the weight gradient
+@pytest.mark.parametrize("what,M,K,N", [("forward", 40000, 1728, 64), ("forward", 4000, 1728, 64), ("ABt", 40000, 256, 512),
+                                        ("AtB", 40000, 256, 96)])
+def test_a_net_that_diverged_costs_a_few_times_what_a_sound_one_does(scn, ctx, what, M, K, N):
+    """weights that have all gone to NaN, or to infinities (which leave no early way out): sums that are not finite are
+    taken again a tile at a time"""
+    import time
+    rng = np.random.default_rng(M + K)
+    A = ctx.array(rng.standard_normal((M, K), dtype=np.float32))
+    D = ctx.array(rng.standard_normal((M, N), dtype=np.float32))
+    B, out, ws = ctx.array(np.zeros(N, np.float32)), ctx.empty((M, N), np.float32), ctx.empty(N * K + N, np.float32)
+    dW, best = ctx.array(np.zeros((K, N), np.float32)), {}
+    W = rng.standard_normal((K, N), dtype=np.float32)
+    for name, value in (("sound", None), ("nan", np.nan), ("inf", np.inf)):
+        w = W if value is None else np.where(W > 0, np.float32(value), -np.float32(value))
+        d_W = ctx.array(w.T if what == "ABt" else w)
+        if what == "AtB":
+            D.upload(rng.standard_normal((M, N), dtype=np.float32) if value is None else np.full((M, N), value, np.float32))
+        print("diverged", what, M, K, N, name, flush=True)
+        for _ in range(4):
+            ctx.sync()
+            t = time.perf_counter()
+            if what == "forward":
+                ctx.nin_forward(A, d_W, B, None, out, M, K, N, 1.0, scn.NOSIGMOID, scn.FP32_PLANES)
+            elif what == "ABt":  # [M x 256] times the transpose of [512 x 256]
+                ctx.sgemm_ABt(A, d_W, out, M, K, N, ws)
+            else:
+                ctx.sgemm_AtB(A, D, dW, M, K, N)
+            ctx.sync()
+            best[name] = min(best.get(name, 1e9), 1e6 * (time.perf_counter() - t))
+        got = (dW if what == "AtB" else out).download()
+        assert np.isfinite(got).all() if value is None else not np.isfinite(got).any()
+    print("us", {k: round(v) for k, v in best.items()}, flush=True)
+    # (launches and waits are some 50 us of each)
+    assert best["nan"] <= 5 * best["sound"] + 50 and best["inf"] <= 15 * best["sound"] + 50
