@@ -201,3 +201,41 @@ def test_a_net_that_diverged_costs_a_few_times_what_a_sound_one_does(scn, ctx, w
     print("us", {k: round(v) for k, v in best.items()}, flush=True)
     # (launches and waits are some 50 us of each)
     assert best["nan"] <= 5 * best["sound"] + 50 and best["inf"] <= 15 * best["sound"] + 50
+
+
+@pytest.mark.parametrize("M,K,N", [(14000, 1728, 64), (30000, 256, 96), (20000, 512, 160)])
+def test_planes_round_less_than_the_fp32_mfma(scn, ctx, M, K, N):
+    """root mean square error against float64: 0.31 to 0.38 of the fp32 MFMA kernels' on these shapes, none of them
+    a long contraction or few rows"""
+    rng = np.random.default_rng(M)
+    A, W = np.maximum(rng.standard_normal((M, K), dtype=np.float32), 0), rng.standard_normal((K, N), dtype=np.float32)
+    want, err = A.astype(np.float64) @ W.astype(np.float64), []
+    d_A, d_W, d_B, out = ctx.array(A), ctx.array(W), ctx.array(np.zeros(N, np.float32)), ctx.empty((M, N), np.float32)
+    for p in (scn.FP32, scn.FP32_PLANES):
+        ctx.nin_forward(d_A, d_W, d_B, None, out, M, K, N, 1.0, scn.NOSIGMOID, p)
+        err.append(np.sqrt(((out.download() - want) ** 2).mean()))
+    assert 0 < err[1] <= 0.5 * err[0]
+
+
+# tiles, split contraction, weight gradient
+@pytest.mark.parametrize("what,M", [("forward", 30000), ("forward", 200), ("AtB", 30000)])
+@pytest.mark.parametrize("exponent", [-105, -112, -120, -130])
+def test_operands_below_the_range_of_the_lower_planes(scn, ctx, what, M, exponent):
+    """bf16 resolves 2^-133: of an operand so small that its lowest plane lies below that, 2^-134 is left out at most"""
+    rng = np.random.default_rng(M - exponent)
+    K, N = 256, 96
+    tiny = (rng.standard_normal((M, K)) * 2.0 ** exponent).astype(np.float32)
+    other = rng.standard_normal((K, N) if what == "forward" else (M, N)).astype(np.float32)
+    if what == "forward":
+        out = ctx.empty((M, N), np.float32)
+        ctx.nin_forward(ctx.array(tiny), ctx.array(other), ctx.array(np.zeros(N, np.float32)), None, out, M, K, N, 1.0,
+                        scn.NOSIGMOID, scn.FP32_PLANES)
+        a, length = tiny, K
+    else:
+        out = ctx.array(np.zeros((K, N), np.float32))
+        ctx.sgemm_AtB(ctx.array(tiny), ctx.array(other), out, M, K, N)
+        a, length = tiny.T, M
+    a, b = a.astype(np.float64), other.astype(np.float64)
+    # what is left out of each operand, the rounding of the sums as for ordinary operands, and fp32's own grid
+    allowed = 2.0 ** -134 * np.abs(b).sum(0) + 2e-6 * (np.abs(a) @ np.abs(b)) + length * 2.0 ** -149
+    assert np.all(np.abs(out.download() - a @ b) <= allowed)
