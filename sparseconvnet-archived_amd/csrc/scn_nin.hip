@@ -2,7 +2,6 @@
 // fused into the contraction's epilogue (the reference runs replicateArray,
 // cublasSgemm and applySigmoid / PreLU as three passes over the output).
 #include "scn_nin_dev.h"
-#include <stdlib.h>
 #include <type_traits>
 
 int scn_squash_launch(scn_ctx *ctx, float *d_x, long long n, int logistic);
