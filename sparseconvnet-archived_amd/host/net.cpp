@@ -301,12 +301,15 @@ static void buildRuleBooks(SparseConvNetCUDA &cnn, scn_ctx *ctx,
   planAllLayers(cnn, ctx, b);
   SCN_CHECKED(scn_ctx_chain_rules(ctx, 0));
   SCN_CHECKED(scn_ctx_defer_counts(ctx, 0));
-  // Running ahead: every layer's rows can be read on the device, and the result
-  // has a row per sample whatever the counts turn out to be.
+  // Running ahead: every layer's rows can be read on the device, the result has
+  // a row per sample whatever the counts turn out to be, and no bound is refused
+  // where the rows there are might not be (32-bit pooling choices).
   bool ahead = mayRunAhead && b.interfaces.back().nSpatialSites == b.batchSize;
-  for (size_t i = 1; ahead && i < b.interfaces.size(); ++i)
-    ahead = !b.interfaces[i].ownsDeviceGrids ||
-            scn_ctx_rows_from(ctx, b.interfaces[i].deviceGrids) == SCN_OK;
+  for (size_t i = 1; ahead && i < b.interfaces.size(); ++i) {
+    SpatiallySparseBatchInterface &f = b.interfaces[i];
+    ahead = (int64_t)f.nSpatialSites * (int64_t)f.featuresPresent.size() <= 2147483647ll &&
+            (!f.ownsDeviceGrids || scn_ctx_rows_from(ctx, f.deviceGrids) == SCN_OK);
+  }
   SCN_CHECKED(scn_ctx_rows_from(ctx, nullptr));
   if (ahead)
     b.countsPending = true;

@@ -199,3 +199,34 @@ def test_wrong_guesses_over_a_net(scn):
     net.close()
     # (the first drawing's counts are known, the next is guessed by it)
     assert held[:2] == [1, 1] and held.count(0) >= 3 and held.count(1) >= 4, held
+
+
+def test_a_bound_beyond_32_bit_choices_is_no_batch_beyond_them(scn):
+    """A layer in front of a pooling with 1.8 of the 2.1 billion elements that 32-bit choices index: a quarter more, its
+    bound in the next batch, passes them.  That batch waits for its counts and is taken as the first one was."""
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    rng = np.random.default_rng(6)
+    batch, field = 200, 41
+    net = hostapi.Net(2, 1, 2, threads=1)
+    net.addLeNetLayerMP(8192, 2, 1, 2, 2, scn.RELU)
+    net.addTerminalPoolingLayer(20)
+    net.addSoftmaxLayer()
+    net.setFusedConvolutions(True)
+    assert net.inputSpatialSize == field
+    for i, (W, B, pr) in synthetic.he_normal_weights(net.layers(), 5).items():
+        net.set_weights(i, W, B, pr)
+    ctx = scn.Context(handle=net.context_handle())
+    samples, n = brute.random_samples(rng, batch, 2, field, 0.26)
+    S, K, R, bg = flatten_samples(samples)
+    feats = rng.standard_normal((n, 1)).astype(np.float32)
+    d = [ctx.array(S, np.int32), ctx.array(K, np.int64), ctx.array(R, np.int32), ctx.array(bg, np.int32), ctx.array(feats)]
+    got = []
+    for _ in range(3):
+        p = np.zeros((batch, 2), np.float32)
+        print("a batch of 1.8e9 elements", flush=True)
+        net.forward_resident(batch, d[0].ptr, d[1].ptr, d[2].ptr, d[3].ptr, len(K), n, d[4].ptr, p)
+        got.append(p)
+    rows = net.interface(2, want_features=False)["nSpatialSites"]
+    net.close()
+    assert 1.75e9 < rows * 8192 < 2 ** 31 < 1.25 * rows * 8192
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
