@@ -78,6 +78,10 @@ const char *scn_version(void);
 /* initializeGPU (utilities.cu:105-130) + cudaMemStream ctor (:171-174).
  * device < 0 selects device 0. */
 int scn_ctx_create(int device, scn_ctx **ctx);
+/* The same without the room for a layer's weights, for a stream that rule books
+ * are built on (the producers' of a net).  Every call works on it; long
+ * contractions convert their weights on the way, to the same bits. */
+int scn_ctx_create_for_plans(int device, scn_ctx **ctx);
 int scn_ctx_destroy(scn_ctx *ctx);
 /* the hipStream_t all work is issued on */
 void *scn_ctx_stream(scn_ctx *ctx);

@@ -71,6 +71,7 @@ def lib():
         "scn_last_error": (C.c_char_p, []),
         "scn_version": (C.c_char_p, []),
         "scn_ctx_create": (C.c_int, [C.c_int, P(vp)]),
+        "scn_ctx_create_for_plans": (C.c_int, [C.c_int, P(vp)]),
         "scn_ctx_destroy": (C.c_int, [vp]),
         "scn_ctx_stream": (vp, [vp]),
         "scn_sync": (C.c_int, [vp]),

@@ -16,7 +16,7 @@ void scn_set_error(const char *fmt, ...) {
 extern "C" const char *scn_last_error(void) { return g_err; }
 extern "C" const char *scn_version(void) { return "scn_hip 0.1 (gfx950)"; }
 
-extern "C" int scn_ctx_create(int device, scn_ctx **out) {
+static int ctx_create(int device, bool room, scn_ctx **out) {
   SCN_REQUIRE(out != nullptr, SCN_ERR_ARG, "scn_ctx_create: null out pointer");
   int n = 0;
   SCN_HIP_CHECK(hipGetDeviceCount(&n));
@@ -57,7 +57,7 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   SCN_HIP_CHECK(hipMemset(c->d_scalars, 0, 16 * sizeof(int64_t)));
   SCN_HIP_CHECK(hipMalloc((void **)&c->d_zeros, SCN_ZERO_FLOATS * sizeof(float)));
   // (here and not with the first long contraction: numeric calls never allocate)
-  if (hipMalloc((void **)&c->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
+  if (room && hipMalloc((void **)&c->d_image, SCN_IMAGE_BYTES) != hipSuccess) {
     (void)hipGetLastError();
     c->d_image = nullptr;
   }
@@ -68,6 +68,13 @@ extern "C" int scn_ctx_create(int device, scn_ctx **out) {
   SCN_HIP_CHECK(hipStreamSynchronize(c->stream));
   *out = c;
   return SCN_OK;
+}
+
+extern "C" int scn_ctx_create(int device, scn_ctx **out) {
+  return ctx_create(device, true, out);
+}
+extern "C" int scn_ctx_create_for_plans(int device, scn_ctx **out) {
+  return ctx_create(device, false, out);
 }
 
 extern "C" int scn_ctx_destroy(scn_ctx *c) {

@@ -140,9 +140,9 @@ scn_ctx *scnDefaultContext() {
   }
   return g_defaultCtx;
 }
-cudaMemStream::cudaMemStream() : ctx(nullptr) {
+cudaMemStream::cudaMemStream(bool layers) : ctx(nullptr) {
   std::lock_guard<std::mutex> lock(g_ctxMutex);
-  SCN_CHECKED(scn_ctx_create(-1, &ctx));
+  SCN_CHECKED(layers ? scn_ctx_create(-1, &ctx) : scn_ctx_create_for_plans(-1, &ctx));
   g_liveCtx.push_back(ctx);
   g_defaultCtx = g_liveCtx.front();
 }

@@ -37,7 +37,7 @@ SparseConvNetCUDA::SparseConvNetCUDA(int dimension, int nInputFeatures,
   batchPool.reserve(nBatchProducerThreads);
   const int nStreams = std::min(nBatchProducerThreads, N_PRODUCER_STREAMS);
   for (int c = 0; c < nStreams; c++) {
-    batchMemStreams.emplace_back(new cudaMemStream());
+    batchMemStreams.emplace_back(new cudaMemStream(false));
     freeProducerStreams.push_back(batchMemStreams.back().get());
   }
   for (int c = 0; c < nBatchProducerThreads; c++) {

@@ -13,7 +13,10 @@
 class cudaMemStream {
 public:
   scn_ctx *ctx;
-  cudaMemStream();
+  // layers: the stream runs layers, and not only the producers' rule books
+  // (16 MB for each of those would be memory that nothing uses, and 1 ms of a
+  // new net's first batch)
+  explicit cudaMemStream(bool layers = true);
   ~cudaMemStream();
   cudaMemStream(const cudaMemStream &) = delete;
   cudaMemStream &operator=(const cudaMemStream &) = delete;

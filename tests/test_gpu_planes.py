@@ -239,3 +239,24 @@ def test_operands_below_the_range_of_the_lower_planes(scn, ctx, what, M, exponen
     # what is left out of each operand, the rounding of the sums as for ordinary operands, and fp32's own grid
     allowed = 2.0 ** -134 * np.abs(b).sum(0) + 2e-6 * (np.abs(a) @ np.abs(b)) + length * 2.0 ** -149
     assert np.all(np.abs(out.download() - a @ b) <= allowed)
+
+
+def test_a_context_without_room_for_weights_gives_the_same_bits(scn, ctx):
+    import ctypes as C
+    h = C.c_void_p()
+    assert scn.lib().scn_ctx_create_for_plans(0, C.byref(h)) == scn.OK
+    plain = scn.Context(handle=h.value)
+    rng = np.random.default_rng(4)
+    M, N = 60000, 256
+    for K in (512, 1728):
+        A, W = ctx.array(rng.standard_normal((M, K), dtype=np.float32)), ctx.array(rng.standard_normal((K, N), dtype=np.float32))
+        D, B, ws = ctx.array(rng.standard_normal((M, N), dtype=np.float32)), ctx.array(np.zeros(N, np.float32)), ctx.empty(
+            scn.lib().scn_sgemm_ABt_workspace(N, K), np.float32)
+        outs = [(ctx.empty((M, N), np.float32), ctx.empty((M, N), np.float32), ctx.empty((M, K), np.float32)) for _ in range(2)]
+        for c, (a, b, d) in zip((ctx, plain), outs):
+            c.nin_forward(A, W, B, None, a, M, K, N, 1.0, scn.RELU, scn.FP32_PLANES)
+            c.nin_forward(A, W, B, None, b, M, K, N, 1.0, scn.RELU, scn.BF16)
+            c.sgemm_ABt(D, W, d, M, N, K, ws)
+            c.sync()
+        assert all(np.array_equal(x.download(), y.download()) for x, y in zip(*outs))
+    scn.lib().scn_ctx_destroy(h)
