@@ -1597,10 +1597,13 @@ static void launch_mfma(scn_ctx *ctx, const float *A, const float *W,
 }
 
 // SCN_FP32 goes to the bf16 matrix cores where the contraction is long (40
-// GFLOP, a third of a millisecond on the fp32 ones: 2.24 -> 1.39 ms for 1.36 M x
-// 1728 x 64) or its rows are few (the split contraction: 600 x 384 x 128 in 5.0
-// us for 9.5).  In between it keeps to fp32 MFMA and so to the bits it has
-// always given; SCN_FP32_PLANES asks for the planes at every size.
+// GFLOP: 1.36 M x 1728 x 64 and its pooling 2.24 -> 1.41 ms) or its rows are few
+// (the split contraction: 600 x 384 x 128 in 5.0 us for 9.5).  In between it
+// keeps to fp32 MFMA, and so to the bits it has always given, whichever is the
+// faster (fp32 MFMA, planes, in us: 30000 x 256 x 96 19.8, 24.6; 66000 x 1728 x
+// 64 169, 209; 150000 x 1728 x 64 306, 277; 41600 x 640 x 320 151, 128; 9000 x
+// 1920 x 640 186, 140).  SCN_FP32_PLANES, which the host classes ask for, takes
+// the planes at every size.
 #define PLANES_MIN_FLOPS 4e10
 // rows16: a bf16 copy of the matrix the rules point into, or null
 static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,

@@ -754,13 +754,14 @@ bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
 // Three planes: measured on contractions of 256 and 1152 k at 256 to 2048
 // workgroups, with W converted on the way and from its image.  A wavefront of
 // two row tiles and two column tiles (2, 2) is the fastest per flop (232
-// TFLOP/s from the image, (1, 1) 173) and the first to leave the chip idle, so
+// TFLOP/s from the image with the chip full, (1, 1) 173; 1.36 M x 1728 x 64
+// through its rules 222) and the first to leave the chip idle, so
 // the row count decides.
 // One plane: fitted to 148 shapes (2800 to 200000 rows, 256 to 2592 k, 64 to 640
 // columns), fp32 and bf16 rows, which it gives within 1 % of the best tile on
 // average.  What bounds it is the fetching of A, once for every slice of
 // columns, so the tile is one row tile by up to four column tiles: from the
-// image, with bf16 rows, 570000 x 2592 x 128 511 -> 430 us (875 TFLOP/s) against
+// image, with bf16 rows, 596000 x 2592 x 128 511 -> 433 us (913 TFLOP/s) against
 // (2, 2), which goes twice through A; 5900 x 1920 x 640 with fp32 rows 57 -> 38
 // against (1, 2).  Five and eight column tiles, or two by four, gain no more.
 // Every choice gives the same bits.  The start and the stores of a workgroup
@@ -902,9 +903,9 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // eight wavefronts take sixteen rows each in turn and their sums meet in LDS.
 // The workgroups of one tile add to dW with float atomics, some 200 of which
 // retire in a nanosecond: few workgroups (one a compute unit), each with as many
-// rows as that leaves it.  29827 x 256 x 96 in 22 us (32 on the fp32 MFMA with
-// a thousand workgroups), 200000 x 1728 x 64 in 350 (470): the rate at which A
-// comes from HBM.
+// rows as that leaves it.  29827 x 256 x 96 in 23 us (32 on the fp32 MFMA with
+// a thousand workgroups), 200000 x 1728 x 64 in 350 (470): A from HBM at 3.9
+// TB/s.
 #define ATB_STEP 16
 template <int MT, int NT>
 __global__ void __launch_bounds__(512, 2)
@@ -1131,6 +1132,7 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
 // a compute unit, each `ti` microseconds for every 128 rows (two thirds of it
 // waiting for memory) and `f` to start, to sum and to store, and the atomics.
 // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
+// (The search is 0.1 to 2 us of the host's time, a launch some 5.)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
                    long long M, int K, int N) {
   static const struct {
