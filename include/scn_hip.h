@@ -291,8 +291,8 @@ int scn_conv_nin_forward(scn_ctx *ctx, const float *d_in,
                          const float *d_prelu, float *d_out, int64_t M, int N,
                          float p, int act);
 /* The same with the operand precision of scn_nin_forward: SCN_FP32, or SCN_BF16
- * for shapes with nIn a multiple of 8, fs * nIn of 64 and N of 32 (operands
- * rounded to bf16 on their way to the MFMA, fp32 accumulation); bit-identical to
+ * for shapes with nIn a multiple of 8, fs * nIn of 64 (of 32 from 256 on) and N
+ * of 32 (operands rounded to bf16 on their way to the MFMA, fp32 accumulation); bit-identical to
  * scn_gather_rows followed by scn_nin_forward with that precision.  (Contractions
  * of up to 32 stay fp32 in every precision, fused or not.) */
 int scn_conv_nin_supported_p(int fs, int nIn, int N, int precision);
@@ -307,8 +307,7 @@ int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
  * contraction reads its rows from there, half the bytes for a matrix whose
  * rows the rules visit many times over.  The operands that reach the MFMA are
  * the ones scn_conv_nin_forward_p(SCN_BF16) rounds in registers, so the result
- * is the same bit for bit; shapes the bf16 W-streaming kernel does not take
- * run as scn_conv_nin_forward_p(SCN_BF16) does.  Same reference operator
+ * is the same bit for bit.  Same reference operator
  * (NetworkInNetworkLayer.cu:187-200 after ConvolutionalLayer.cu:125-133). */
 int scn_conv_nin_forward_a16(scn_ctx *ctx, const float *d_in, int64_t nInRows,
                              void *d_in16, const int32_t *d_rules, int fs,
@@ -357,13 +356,15 @@ int scn_activation_backward(scn_ctx *ctx, const float *d_out, float *d_delta,
                             float *d_db, float *d_dprelu);
 /* d_rowMajorSGEMM_alphaAtB_betaC with alpha 1, beta 0 (utilities.cu:144-152;
  * call site NetworkInNetworkLayer.cu:225-228): dW[K x N] = A^T D, A [M x K],
- * D [M x N], all row-major.  fp32 MFMA, fp32 atomics across row ranges. */
+ * D [M x N], all row-major.  In three bf16 planes (as SCN_FP32_PLANES), fp32
+ * atomics across row ranges. */
 int scn_sgemm_AtB(scn_ctx *ctx, const float *d_A, const float *d_D,
                   float *d_dW, int64_t M, int K, int N);
 /* d_rowMajorSGEMM_alphaABt_betaC with alpha 1, beta 0 (utilities.cu:153-161;
  * call site NetworkInNetworkLayer.cu:269-272): dA[M x K] = D[M x N] W^T,
- * W [K x N].  d_workspace holds scn_sgemm_ABt_workspace(N, K) floats (the
- * transposed weights, which the forward contraction kernels then stream). */
+ * W [K x N].  d_workspace holds scn_sgemm_ABt_workspace(N, K) floats: the
+ * transposed weights, for shapes and streams (under capture) whose weights the
+ * context's own room does not take. */
 int64_t scn_sgemm_ABt_workspace(int N, int K);
 int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
                   float *d_dA, int64_t M, int N, int K, float *d_workspace);

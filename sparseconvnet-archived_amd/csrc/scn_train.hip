@@ -235,8 +235,10 @@ extern "C" int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A,
 }
 
 // ------------------------------------------------------------ dA = D W^T
-// The forward contraction with W transposed: the transposed copy (and the
-// zero bias the forward kernels add) live in the caller's workspace.
+// The forward contraction with W transposed.  The planes make their image from W
+// as it stands, or read it so; other shapes, and calls that may not use the
+// context's room (under capture), take a transposed copy in the caller's
+// workspace, where the zero bias of a wide result is too.
 __global__ void k_transpose(const float *__restrict__ W, float *__restrict__ Wt,
                             int K, int N) {
   __shared__ float tile[32][33];

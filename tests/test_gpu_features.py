@@ -226,8 +226,8 @@ def test_nin_bf16(scn, ctx, M, K, N, act):
     check_nin_bf16(scn, ctx, M, K, N, act)
 
 
-# the bf16 W-streaming kernel with wide slices (64 and 96 columns), every depth of its prefetch ring
-# (K / 32 a multiple of 4, of 6, of neither), ragged last groups
+# bf16 operands over slices of every width
+# (K / 32 a multiple of 4, of 6, of neither; ragged last groups)
 # ... and the wide contractions of the GEMM-bound 2-D net (K up to 2560, N up to 800)
 @pytest.mark.parametrize("M,K,N", [(66001, 1728, 64), (33005, 192, 96), (40003, 256, 96), (70001, 320, 128),
                                    (1, 64, 32), (15, 128, 32), (255, 512, 160), (1025, 3200, 320), (2600, 2560, 800)])
