@@ -37,8 +37,9 @@ sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "oracle"))
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
-# dense MFMA peaks; bf16x3 issues three bf16 MFMAs per useful one
-MFMA_PEAK_TFLOPS = {"fp32": 157.3, "bf16": 2500.0, "bf16x3": 2500.0 / 3}
+# dense MFMA peaks in useful operations; fp32 operands go as three bf16 planes, six bf16 MFMAs per useful one, bf16x3 as
+# two planes, three
+MFMA_PEAK_TFLOPS = {"fp32": 2500.0 / 6, "bf16": 2500.0, "bf16x3": 2500.0 / 3}
 BALANCE_FLOP_PER_BYTE = {k: v * 1e12 / 8e12 for k, v in MFMA_PEAK_TFLOPS.items()}
 
 
