@@ -1529,6 +1529,7 @@ extern "C" int scn_ctx_defer_counts(scn_ctx *ctx, int on) {
 extern "C" int scn_rules_settle(scn_ctx *ctx) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_rules_settle: null context");
   SCN_TRY(scn_chain_flush(ctx));
+  ctx->d_meta = nullptr; // (the counts that scn_ctx_rows_from spoke of are the host's from here on)
   ctx->rowsHeld = true; // (of the passes settled here: none, when nothing is pending)
   if (ctx->pendingGrids.empty())
     return SCN_OK;
@@ -1622,6 +1623,8 @@ extern "C" int scn_grids_destroy(scn_ctx *ctx, scn_grids *g) {
   if (ctx) {
     (void)scn_chain_flush(ctx);
     (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->d_meta && ctx->d_meta == g->meta.p)
+      ctx->d_meta = nullptr;
     auto &pl = ctx->pendingGrids;
     for (size_t i = 0; i < pl.size(); ++i)
       if (pl[i] == g) {

@@ -659,8 +659,8 @@ __global__ void __launch_bounds__(256)
 }
 
 // False: convert on the way instead -- the stream is being captured (a graph may
-// be replayed beside the context's own calls, whose weights the room holds, and
-// after the context), or the context found no memory for the room.
+// be replayed beside the context's own calls, whose weights the room holds), or
+// the context has no such room.
 static bool planes_image(scn_ctx *ctx) {
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) {

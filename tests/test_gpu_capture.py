@@ -1,6 +1,5 @@
 """Long contractions captured into a HIP graph.  The context's copy of a layer's weights belongs to the context's own
-calls: a graph, which may be replayed beside them and outlive the context, converts the weights on the way and gives the
-same bits."""
+calls: a graph, which may be replayed beside them, converts the weights on the way and gives the same bits."""
 import ctypes as C
 
 import numpy as np

@@ -97,6 +97,29 @@ def test_fp32_waits_for_its_rows_and_chooses_by_them(scn, ctx):
             assert np.array_equal(got.download()[:n], known.download()), (density, n, bound)
 
 
+def test_settled_counts_are_no_longer_read_on_the_device(scn, ctx):
+    """scn_ctx_rows_from ends with the settling (and with its grids): a call of more rows takes its own number."""
+    rng = np.random.default_rng(13)
+    nIn, N, fs, M = 32, 320, 4, 5000
+    src, out = scn.Grids(ctx), scn.Grids(ctx)
+    A, W, B = (ctx.array(rng.standard_normal(s, dtype=np.float32)) for s in ((M, fs * nIn), (fs * nIn, N), (N,)))
+    known = ctx.empty((M, N), np.float32)
+    ctx.nin_forward(A, W, B, None, known, M, fs * nIn, N, 1.0, scn.RELU, scn.FP32_PLANES)
+    for end in ("settle", "destroy"):
+        for i in range(2):
+            samples, nSites = brute.random_samples(rng, 6, 2, 41, 0.02)
+            _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+        assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+        if end == "settle":
+            assert scn.settle(ctx)
+        else:
+            out.close()
+        got = ctx.array(np.full((M, N), 7, np.float32))
+        ctx.nin_forward(A, W, B, None, got, M, fs * nIn, N, 1.0, scn.RELU, scn.FP32_PLANES)
+        assert np.array_equal(got.download(), known.download()), end
+    assert scn.lib().scn_rules_settle(ctx.h) == scn.OK
+
+
 # split contraction up to 1248 rows (three planes) and 1792 (one), tiles above: dense batches lie above, sparse ones below
 @pytest.mark.parametrize("precision", ["FP32_PLANES", "BF16"])
 def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
