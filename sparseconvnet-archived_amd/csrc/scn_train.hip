@@ -267,6 +267,14 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
     return SCN_OK;
   SCN_REQUIRE(d_D && d_W && d_dA && d_workspace, SCN_ERR_ARG,
               "scn_sgemm_ABt: null buffer");
+  // (M is the caller's number of rows, whatever scn_ctx_rows_from says to the
+  // forward calls, whose kernels run here)
+  struct OwnRows {
+    scn_ctx *ctx;
+    const long long *meta;
+    explicit OwnRows(scn_ctx *c) : ctx(c), meta(c->d_meta) { c->d_meta = nullptr; }
+    ~OwnRows() { ctx->d_meta = meta; }
+  } ownRows(ctx);
   bool transpose = false;
   Epilogue ep = Epilogue();
   ep.bias = ctx->d_zeros;

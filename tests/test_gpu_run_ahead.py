@@ -120,6 +120,24 @@ def test_settled_counts_are_no_longer_read_on_the_device(scn, ctx):
     assert scn.lib().scn_rules_settle(ctx.h) == scn.OK
 
 
+@pytest.mark.parametrize("M", [200, 20000])  # split contraction, tiles
+def test_backward_products_keep_their_own_rows(scn, ctx, M):
+    """scn_ctx_rows_from speaks to the forward calls: a product with W^T meanwhile computes the rows it is given."""
+    rng = np.random.default_rng(14)
+    N, K = 256, 128
+    src, out = scn.Grids(ctx), scn.Grids(ctx)
+    D, W = ctx.array(rng.standard_normal((M, N), dtype=np.float32)), ctx.array(rng.standard_normal((K, N), dtype=np.float32))
+    ws, outs = ctx.empty(N * K + K, np.float32), [ctx.array(np.full((M, K), 7, np.float32)) for _ in range(2)]
+    ctx.sgemm_ABt(D, W, outs[0], M, N, K, ws)
+    for i in range(2):
+        _one_plan(scn, ctx, src, out, *brute.random_samples(rng, 2, 2, 41, 0.003), i > 0)
+    assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+    ctx.sgemm_ABt(D, W, outs[1], M, N, K, ws)
+    scn.lib().scn_ctx_rows_from(ctx.h, None)
+    assert scn.settle(ctx) and out.info()["nSpatialSites"] < M
+    assert np.array_equal(outs[0].download(), outs[1].download())
+
+
 # split contraction up to 1248 rows (three planes) and 1792 (one), tiles above: dense batches lie above, sparse ones below
 @pytest.mark.parametrize("precision", ["FP32_PLANES", "BF16"])
 def test_a_wrong_guess_of_rows_leaves_none_out(scn, ctx, precision):
