@@ -13,13 +13,16 @@
 // layer may end them) are built from the output side (second half of this
 // file, per-lane bodies in scn_pyr_dev.h):
 //
-//   k_pyr_masks     one wavefront per sample: the occupancy masks of all
-//                   layers, each the dilation of the one before, their rank
-//                   prefixes and the sample's site counts;
-//   k_pyr_rules     one workgroup per sample: the counts of the samples before
-//                   it, then per output site in sweeps over all layers at once
-//                   -- sites by rank, owners, rows, entry lists, rule rows --
-//                   written at their batch-global places.
+//   k_pyr_levels    one wavefront per sample, layer and slab of it: the layer's
+//                   occupancy mask, straight from the source's, and its sites
+//                   (k_pyr_masks where that does not go: one wavefront per
+//                   sample, layer after layer);
+//   k_pyr_rules     as many workgroups per sample as the batch leaves room for,
+//                   each with some of the layers or a slab of one: rank
+//                   prefixes, the counts of the samples before, then per output
+//                   site in sweeps over its layers -- sites by rank, owners,
+//                   rows, entry lists, rule rows -- written at their
+//                   batch-global places.
 //
 // Every other chain (a minimum of active inputs, triangular lattices, windows
 // of more than 16 sites) goes the older way, from the input side:
@@ -53,6 +56,7 @@
 #define CHAIN_LDS_MAX (152 * 1024)
 // most LDS a workgroup of k_pyr_rules asks for
 #define PYR_LDS_MAX CHAIN_LDS_MAX
+#define PYR_CUS 256 // compute units: one workgroup of k_pyr_rules each
 #define CHAIN_HEADER_BYTES 512
 #define CHAIN_MIN_ARENA (16 * 1024)
 // bytes of arena per entry of the input grid (key, row, ownership mask, base)
@@ -156,6 +160,17 @@ __device__ __forceinline__ unsigned wave_scan_incl_dpp(unsigned v) {
   v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false); // row_shr:8
   v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false); // row_bcast:15
   v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false); // row_bcast:31
+  return v;
+}
+// the largest of all lanes' values (0 and more), in lane 63
+__device__ __forceinline__ int wave_max_dpp(int v) {
+  auto step = [&](int o) { v = o > v ? o : v; };
+  step(__builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
   return v;
 }
 __device__ __forceinline__ unsigned wave_last(unsigned v) {
@@ -790,15 +805,21 @@ __global__ void __launch_bounds__(PLACE_THREADS) k_chain_place(ChainArgs a) {
 // ------------------------------------------------ chains built from the output side
 //
 // scn_pyr_dev.h has the per-lane bodies; here are the two kernels around them.
-// k_pyr_masks, one workgroup per sample: the occupancy masks of all layers
-// (each the dilation of the one before), their rank prefixes and the sample's
-// site counts, left in global memory.  k_pyr_rules, one workgroup per sample:
-// everything per site, in sweeps over all layers at once -- the sums over the
-// samples before (which k_pyr_masks has finished writing), sites by rank,
-// owners, rows, entry lists and rule rows at their batch-global places.  Nothing
-// is staged and nothing is copied afterwards.
-// k_pyr_masks runs ONE wavefront per sample.  With four wavefronts per
-// workgroup the kernel was measured to give wrong mask words now and then --
+// Pass A: the occupancy masks of all layers and the sample's site counts, left
+// in global memory.  k_pyr_levels makes each layer's mask from the source's rows
+// (the windows of all layers before it taken together), so that its wavefronts do
+// not wait for each other: 14 us -> 6.5 for a batch of 100 fields of 126 x 126 and
+// ten layers, 44 -> 12 for 33 of 47^3 and eight, against k_pyr_masks, where one
+// wavefront makes a sample's layers one after the other.  What is left is the
+// fetch of the rows and a launch.  k_pyr_masks stays for one dimension, for rows
+// longer than 256 sites (64 in three dimensions) and for windows that leave gaps.
+// k_pyr_rules, one workgroup per part of a sample: everything per site, in sweeps
+// over all of the part's layers at once -- rank prefixes, the sums over the samples
+// before (which pass A has finished writing), sites by rank, owners, rows, entry
+// lists and rule rows at their batch-global places.  Nothing is staged and nothing
+// is copied afterwards.
+// Both kernels of pass A run ONE wavefront per workgroup.  With four wavefronts
+// per workgroup k_pyr_masks was measured to give wrong mask words now and then --
 // only while workgroups of other streams' chains shared the compute units, with
 // either kind of barrier, its arguments, its input and its own first level
 // intact, and never with one chain at a time; the instruction stream shows
@@ -819,30 +840,14 @@ struct PyrGeoA {
   int pad;
 };
 static_assert(sizeof(PyrGeoA) == 48, "three 16-byte reads");
-#define PYR_A_EXTRA (128 + (PYR_MAX_LEVELS + 1) * (int)sizeof(PyrGeoA)) // counts, geometry: after the pyramid
-
-// Rank prefixes of `words` mask words (the two spare words included) by one
-// wavefront; the number of set bits comes back
-__device__ __forceinline__ unsigned pyr_prefixes(const pyr_u64 *m, unsigned short *p, int words, int lane) {
-  unsigned carry = 0;
-  for (int w0 = 0; w0 < words + 2; w0 += 64) {
-    const int w = w0 + lane;
-    const unsigned pc = w < words ? (unsigned)pyr_popc64(m[w]) : 0u;
-    const unsigned incl = wave_scan_incl_dpp(pc);
-    if (w < words + 2)
-      p[w] = (unsigned short)(carry + incl - pc);
-    carry += wave_last(incl);
-  }
-  return carry;
-}
+#define PYR_A_GEO ((PYR_MAX_LEVELS + 1) * (int)sizeof(PyrGeoA)) // geometry: after the masks
 
 template <int D>
 __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   pyr_u64 *masks = reinterpret_cast<pyr_u64 *>(lds);
-  unsigned short *pref = reinterpret_cast<unsigned short *>(lds + 8ll * a.maskWords);
-  int *cnt = reinterpret_cast<int *>(lds + 8ll * a.pyrStride);
-  PyrGeoA *geo = reinterpret_cast<PyrGeoA *>(lds + 8ll * a.pyrStride + 128);
+  PyrGeoA *geo = reinterpret_cast<PyrGeoA *>(lds + (8ll * a.maskWords + 15) / 16 * 16);
+  int *const counts = a.counts + (long long)blockIdx.x * a.slabs; // (slabs: 1)
   const int b = blockIdx.x, t = threadIdx.x;
   static_assert(PYR_A_THREADS == 64, "one wavefront: the levels below pass no barrier");
   if (t >= 1 && t < a.nMasks) {
@@ -866,7 +871,7 @@ __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
     const PyrLevel &L = a.lv[0];
     const int words = L.words;
     const long long vol = L.volOut;
-    unsigned carry = 0;
+    unsigned n = 0;
     for (int w0 = 0; w0 < words + 2; w0 += 256) {
       pyr_u64 v[4];
 #pragma unroll
@@ -877,17 +882,14 @@ __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int w = w0 + 64 * u + t;
-        const unsigned pc = (unsigned)pyr_popc64(v[u]);
-        const unsigned incl = wave_scan_incl_dpp(pc);
-        if (w < words + 2) {
+        n += (unsigned)pyr_popc64(v[u]);
+        if (w < words + 2)
           masks[w] = v[u];
-          pref[w] = (unsigned short)(carry + incl - pc);
-        }
-        carry += wave_last(incl);
       }
     }
+    n = wave_last(wave_scan_incl_dpp(n));
     if (t == 0)
-      cnt[0] = (int)carry;
+      counts[0] = (int)n;
     // the other levels start empty: their pieces are OR-ed in
     for (int w = words + 2 + t; w < a.maskWords; w += PYR_A_THREADS)
       masks[w] = 0ull;
@@ -911,38 +913,72 @@ __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
     pyr_sweep_dilate<D>(masks + g.offIn, masks + g.offOut, g.nIn, g.nOut, g.size, g.stride, g.magicN, g.seg, g.segs,
                         g.magicSegs, t, PYR_A_THREADS);
     PYR_A_BARRIER();
-    const unsigned n = pyr_prefixes(masks + g.offOut, pref + g.offOut, g.words, t);
+    unsigned n = 0;
+    for (int w = t; w < g.words; w += 64)
+      n += (unsigned)pyr_popc64(masks[g.offOut + w]);
+    n = wave_last(wave_scan_incl_dpp(n));
     if (t == 0)
-      cnt[x] = (int)n;
+      counts[(long long)x * a.batch * a.slabs] = (int)n;
+  }
+  pyr_u64 *dst = a.pyramid + (long long)b * a.maskWords;
+  for (int i = t; i < a.maskWords; i += PYR_A_THREADS)
+    dst[i] = masks[i];
+}
+
+// Pass A with a wavefront per (sample, level, slab): blockIdx.x the sample, .y the
+// level and slab.
+template <int D, int RW>
+__global__ void __launch_bounds__(64) k_pyr_levels(PyrArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int b = blockIdx.x, x = a.slabLevel[blockIdx.y], slab = a.slabOf[blockIdx.y], t = threadIdx.x;
+  const PyrLevel &L = a.lv[x];
+  const int nOut = L.nOut, n0 = a.lv[0].nOut;
+  const long long vol0 = a.lv[0].volOut;
+  int *const count = a.counts + ((long long)x * a.batch + b) * a.slabs + slab;
+  const PyrSlab z = pyr_slab(D, L, L.magicN, slab, pyr_slabs(D, n0, L, a.slabs));
+  const int words = z.w1 - z.w0;
+  pyr_u64 *const out = a.pyramid + (long long)b * a.maskWords + L.maskOff + z.w0;
+  pyr_u64 *const rows = reinterpret_cast<pyr_u64 *>(lds);
+  const int plane = D == 3 ? n0 : 1;
+  const bool deep = D == 3 && L.foldW > PYR_FOLD_DIRECT;
+  pyr_u64 *const mid = rows + RW * plane * (z.p1 - z.p0);
+  pyr_u64 *const mask = mid + (deep ? RW * (z.p1 - z.p0) * nOut : 0);
+  if (x > 0) {
+    for (int w = t; w < words; w += 64)
+      mask[w] = 0ull;
+    pyr_sweep_stage<RW>(a.bits, (long long)b * vol0 + (long long)z.p0 * plane * n0, n0, plane * (z.p1 - z.p0), rows, t,
+                        64);
+    PYR_A_BARRIER();
+    if (deep) {
+      pyr_sweep_mid<RW>(rows, mid, z.p1 - z.p0, n0, nOut, L.magicN, L.foldW, L.foldS, t, 64);
+      PYR_A_BARRIER();
+    }
+    pyr_sweep_fold<D, RW>(rows, mid, mask, z, n0, nOut, L.magicN, L.foldW, L.foldS, t, 64);
     PYR_A_BARRIER();
   }
-  {
-    uint4 *dst = reinterpret_cast<uint4 *>(a.pyramid + (long long)b * a.pyrStride);
-    const uint4 *src = reinterpret_cast<const uint4 *>(lds);
-    for (int i = t; i < a.pyrStride / 2; i += PYR_A_THREADS)
-      dst[i] = src[i];
+  unsigned n = 0;
+#pragma unroll 4
+  for (int w = t; w < words; w += 64) {
+    const pyr_u64 v = x > 0 ? mask[w] : pyr_source_word(a.bits, vol0, b, (unsigned)(z.w0 + w));
+    n += (unsigned)pyr_popc64(v);
+    out[w] = v;
   }
-  if (t < a.nMasks) {
-    int *c = a.counts + ((long long)t * a.batch + b) * 2;
-    c[0] = cnt[t];
-    c[1] = (long long)cnt[t] < a.lv[t].fullSize;
-  }
-  if (t == 0) {
-    bool fits = pyr_fits(a, cnt);
-    for (int x = 0; x < a.nMasks; ++x)
-      fits = fits && cnt[x] <= PYR_ROWS_MAX;
-    if (!fits)
-      atomicMax(a.flag, a.ticket);
-  }
+  if (z.w1 == L.words && t < 2) // (two spare words)
+    out[words + t] = 0ull;
+  n = wave_last(wave_scan_incl_dpp(n));
+  if (t == 0)
+    *count = (int)n;
 }
 
 template <int D>
 __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   PyrHdr *h = reinterpret_cast<PyrHdr *>(lds);
-  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  // (the last workgroup has no sample: it reports the counts to the host)
+  const bool reports = blockIdx.x == (unsigned)(a.batch * a.nParts);
+  const int b = reports ? 0 : blockIdx.x % a.batch, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const PyrPart part = a.parts[reports ? 0 : blockIdx.x / a.batch];
   constexpr int T = PYR_B_THREADS;
-  const bool gaveUp = *reinterpret_cast<volatile unsigned long long *>(a.flag) == a.ticket;
   // lane t keeps layer t's arguments from here on: fetched while the masks
   // come in, not when the level table wants them
   PyrLevel mine;
@@ -952,27 +988,47 @@ __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
     mine = a.lv[t];
     inMaskOff = a.lv[t > 0 ? t - 1 : 0].maskOff;
   }
-  if (t == 0)
+  if (t == 0) {
     h->over = 0;
-  { // the sample's masks and prefixes
-    const uint4 *src = reinterpret_cast<const uint4 *>(a.pyramid + (long long)b * a.pyrStride);
-    uint4 *dst = reinterpret_cast<uint4 *>(lds + PYR_HDR_BYTES);
-    for (int i = t; i < a.pyrStride / 2; i += T)
-      dst[i] = src[i];
+    h->cut = part.F > 1;
+    h->emitFrom = part.la;
+    h->slab = part.f;
+    h->plane[0] = part.f ? a.lv[part.la].nOut : 0;
+    h->plane[1] = a.lv[part.la].nOut;
+  }
+  if (t < a.nMasks) {
+    h->before[t] = 0;
+    h->words[t] = mine.words + 2;
+    h->maskOff[t] = mine.maskOff;
+  }
+  // the masks of the part's levels and of the two before it
+  const int xFirst = part.la >= 3 ? part.la - 2 : 0, xLast = part.lb;
+  pyr_u64 *const masks = reinterpret_cast<pyr_u64 *>(lds + PYR_HDR_BYTES);
+  unsigned short *const pref = reinterpret_cast<unsigned short *>(masks + a.maskWords);
+  {
+    const pyr_u64 *src = a.pyramid + (long long)b * a.maskWords;
+    const int end = xLast + 1 < a.nMasks ? a.lv[xLast + 1].maskOff : a.maskWords;
+    for (int i = a.lv[xFirst].maskOff + t; i < end; i += T)
+      masks[i] = src[i];
   }
   // sums over the samples, a wavefront per level
   for (int x = wave; x < a.nMasks; x += T / 64) {
-    const int *cnt = a.counts + (long long)x * a.batch * 2;
+    const int *cnt = a.counts + (long long)x * a.batch * a.slabs;
+    const long long full = a.lv[x].fullSize;
+    const int slabs = a.slabs == 1 ? 1 : pyr_slabs(a.d, a.lv[0].nOut, a.lv[x], a.slabs);
     // (a batch's rows are numbered in 32 bits, so these sums fit)
-    unsigned v0 = 0, v1 = 0, v2 = 0, v3 = 0;
+    unsigned v0 = 0, v1 = 0, v2 = 0, v3 = 0, own = 0;
     int mx = 0;
     for (int s = lane; s < a.batch; s += 64) {
-      const int2 c = reinterpret_cast<const int2 *>(cnt)[s];
-      const int n = c.x, hb = c.y;
+      int n = 0;
+      for (int z = 0; z < slabs; ++z)
+        n += cnt[s * a.slabs + z];
+      const int hb = n < full;
       if (s < b) {
         v0 += n;
         v1 += hb;
       }
+      own = s == b ? n : own;
       v2 += n;
       v3 += hb;
       mx = n > mx ? n : mx;
@@ -981,14 +1037,11 @@ __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
     v1 = wave_last(wave_scan_incl_dpp(v1));
     v2 = wave_last(wave_scan_incl_dpp(v2));
     v3 = wave_last(wave_scan_incl_dpp(v3));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const int o = __shfl_xor(mx, off, 64);
-      mx = o > mx ? o : mx;
-    }
+    own = wave_last(wave_scan_incl_dpp(own));
+    mx = (int)wave_last((unsigned)wave_max_dpp(mx));
     if (lane == 0) {
-      h->n[x] = cnt[2 * b];
-      h->hasBg[x] = cnt[2 * b + 1];
+      h->n[x] = (int)own;
+      h->hasBg[x] = (int)own < full;
       h->actBefore[x] = v0;
       h->bgBefore[x] = v1;
       h->actAll[x] = v2;
@@ -999,11 +1052,70 @@ __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
   lds_barrier();
   if (t >= 1 && t <= a.nLevels && pyr_report(a, mine, h, t).over)
     atomicOr(&h->over, 1);
-  if (t == 0 && !pyr_fits(a, h->n))
-    atomicOr(&h->over, 2);
+  // (a sample that does not fit: the whole batch is planned another way.  The
+  // largest counts of two levels need not be one sample's: they only say whether
+  // the samples have to be asked)
+  if (t < a.nMasks && (h->maxAct[t] > PYR_ROWS_MAX ||
+                       !pyr_pair_fits(a, h->maxAct[t], t + 1 < a.nMasks ? h->maxAct[t + 1] : 0)))
+    atomicOr(&h->over, 4);
+  // rank prefixes, a wavefront per chunk of 256 words of a level: within the
+  // chunk now, what lies before it once the chunks' sums are there
+  unsigned *const sums = reinterpret_cast<unsigned *>(lds + PYR_HDR_BYTES + 8ll * a.pyrStride);
+  for (int i = wave; i < a.nChunks; i += T / 64) {
+    const int x = a.chunkLevel[i];
+    if (x < xFirst || x > xLast)
+      continue;
+    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * a.chunkOf[i] + 4 * lane;
+    unsigned pc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      pc[u] = w0 + u < words ? (unsigned)pyr_popc64(masks[at + w0 + u]) : 0u;
+    const unsigned four = pc[0] + pc[1] + pc[2] + pc[3];
+    const unsigned incl = wave_scan_incl_dpp(four);
+    unsigned run = incl - four;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (w0 + u < words)
+        pref[at + w0 + u] = (unsigned short)run;
+      run += pc[u];
+    }
+    if (lane == 63)
+      sums[i] = incl;
+  }
   lds_barrier();
-  const bool over = h->over != 0 || gaveUp;
-  if (b == 0 && t >= 1 && t <= a.nLevels) {
+  for (int i = wave; i < a.nChunks; i += T / 64) {
+    const int x = a.chunkLevel[i], c = a.chunkOf[i];
+    if (c == 0 || x < xFirst || x > xLast)
+      continue;
+    unsigned before = 0;
+    for (int k = lane; k < c; k += 64)
+      before += sums[i - c + k];
+    before = wave_last(wave_scan_incl_dpp(before));
+    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * c + 4 * lane;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (w0 + u < words)
+        pref[at + w0 + u] = (unsigned short)(pref[at + w0 + u] + before);
+  }
+  if (h->over & 4) {
+    for (int sample = t; sample < a.batch; sample += T) {
+      const int *c = a.counts + (long long)sample * a.slabs;
+      auto sites = [&](int x) {
+        int n = 0;
+        for (int z = 0; z < pyr_slabs(a.d, a.lv[0].nOut, a.lv[x], a.slabs); ++z)
+          n += c[(long long)x * a.batch * a.slabs + z];
+        return n;
+      };
+      bool fits = pyr_fits_of(a, sites);
+      for (int x = 0; x < a.nMasks; ++x)
+        fits = fits && sites(x) <= PYR_ROWS_MAX;
+      if (!fits)
+        atomicOr(&h->over, 2);
+    }
+  }
+  lds_barrier();
+  const bool over = (h->over & 3) != 0;
+  if (reports && t >= 1 && t <= a.nLevels) {
     const PyrLevel &L = mine;
     const PyrReport r = pyr_report(a, mine, h, t);
     L.meta[META_SITES] = over ? 0 : r.nSites;
@@ -1016,34 +1128,57 @@ __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
     slot[2] = over;
     slot[3] = r.extra;
   }
-  if (b == 0 && t == 0) {
+  if (reports && t == 0) {
     a.scalars[15] = *a.badSites;
     a.scalars[13] = h->maxAct[0];
   }
-  if (over)
+  if (over || reports)
     return;
-  // the layers a window of levels at a time: as many as the LDS holds (all of
-  // them, for all but the largest samples)
-  for (int xa = 0;;) {
-    const int xb = pyr_window_end(a, h->n, xa);
+  if (part.F > 1) {
+    const PyrLds all = pyr_lds_view(a, lds, 0, 0);
+    pyr_sweep_planes(a, all, part, t, T);
+    lds_barrier();
+    pyr_fill_cut(a, all, part, t);
+    lds_barrier();
+    if (t == 0)
+      pyr_fix_cut(h, part);
+    lds_barrier();
+  }
+  // the part's layers a window of levels at a time: as many as the LDS holds (all
+  // of them, for all but the largest samples); the rows of the layer before the
+  // first of them are worked out here once more
+  for (int xa = part.la >= 3 ? part.la - 2 : 0;;) {
+    // (pyr_window_end and pyr_fill_offsets, a lane a level: every wavefront by itself)
+    const int levelSites = lane >= xa && lane <= part.lb ? pyr_held(h, lane) : 0;
+    const int sitesTo = (int)wave_scan_incl_dpp((unsigned)levelSites);
+    const int firstSites = __builtin_amdgcn_readlane(levelSites, xa);
+    const long long room = a.ldsBytesB - (PYR_HDR_BYTES + 8ll * a.pyrStride + 4ll * firstSites + 6 * 16);
+    const int fit = __popcll(__ballot(lane > xa + 1 && lane <= part.lb && 11ll * sitesTo <= room));
+    const int xb = xa < part.lb ? xa + 1 + fit : xa;
     const int la = xa + 1, lb = xb;
-    const bool last = xb == a.nMasks - 1;
-    pyr_fill_offsets(h, xa, xb, t);
+    const bool last = xb == part.lb;
+    if (t >= xa && t <= xb + 1) {
+      const int sum = sitesTo - levelSites;
+      h->siteOff[t] = sum;
+      h->itemOff[t] = t > xa ? sum - firstSites : 0;
+      if (t == xb + 1)
+        h->total = sum;
+    }
     lds_barrier();
     if (t < a.nMasks)
       pyr_fill_en(mine, lds, t, h->siteOff[t]);
-    const PyrLds s = pyr_lds_view(a, lds, h->total, h->n[xa]);
-    if ((t >= la && t <= lb) || (last && t == a.nLevels && t > lb))
+    const PyrLds s = pyr_lds_view(a, lds, h->total, pyr_held(h, xa));
+    if ((t >= la && t <= lb) || (last && lb == a.nMasks - 1 && t == a.nLevels && t > lb))
       pyr_fill_level(mine, inMaskOff, bgSource, s, t, xa);
     pyr_sweep_clear(s, t, T);
     lds_barrier();
     pyr_sweep_enumerate<D>(a, s, xa, xb, t, T);
     lds_barrier();
-    if (xa == 0) { // the batch's rows of the source's sites: their loads go out first
+    if (xa == 0 && part.la == 1) { // the batch's rows of the source's sites: their loads go out first
       const PyrLevel &L = a.lv[0];
       const long long p0 = (long long)b * L.volOut;
       const Slot *table = reinterpret_cast<const Slot *>(a.table);
-      for (int r = t; r < h->n[0]; r += T) {
+      for (int r = t; r < pyr_held(h, 0); r += T) {
         int c[D];
         pyr_unpack<D>(s.key[r], c);
         long long p = p0 + pyr_key<D>(c, L.nOut);
@@ -1055,15 +1190,25 @@ __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
     lds_barrier();
     // rows owned by the sites before, a wavefront per level
     for (int x = xa + wave; x < xb; x += T / 64) {
-      const int n = h->n[x];
-      const unsigned off = (unsigned)h->siteOff[x];
-      unsigned carry = 0;
-      for (int r0 = 0; r0 < n; r0 += 64) {
-        const int r = r0 + lane;
-        const unsigned v = r < n ? (unsigned)pyr_popc32(pyr_own_mask(s, off + r)) : 0u;
-        const unsigned incl = wave_scan_incl_dpp(v);
-        if (r < n)
-          s.base[off + r] = (unsigned short)(carry + incl - v);
+      const int from = h->cut ? h->own[x] : 0;
+      const int n = (h->cut ? h->ownEnd[x] : h->n[x]) - from;
+      const unsigned off = (unsigned)(h->siteOff[x] + from - pyr_lo(h, x));
+      unsigned carry = (unsigned)pyr_base_start(h, x);
+      for (int r0 = 0; r0 < n; r0 += 256) { // (four sites a lane: the chain of sums is what this takes)
+        const int r = r0 + 4 * lane;
+        unsigned v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[u] = r + u < n ? (unsigned)pyr_popc32(pyr_own_mask(s, off + r + u)) : 0u;
+        const unsigned four = v[0] + v[1] + v[2] + v[3];
+        const unsigned incl = wave_scan_incl_dpp(four);
+        unsigned run = carry + incl - four;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (r + u < n)
+            s.base[off + r + u] = (unsigned short)run;
+          run += v[u];
+        }
         carry += wave_last(incl);
       }
     }
@@ -1408,25 +1553,52 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   long long pyrStride = maskWords + (maskWords + 3) / 4;
   pyrStride = (pyrStride + 1) / 2 * 2;
   const long long fixedB = PYR_HDR_BYTES + 8 * pyrStride + 6 * 16;
-  if (fixedB + CHAIN_MIN_ARENA > PYR_LDS_MAX)
+  if (fixedB + CHAIN_MIN_ARENA > PYR_LDS_MAX || !pyr_set_chunks(a))
     return SCN_OK;
   a.maskWords = (int)maskWords;
   a.pyrStride = (int)pyrStride;
-  // pass B's LDS: from the largest samples seen at every level, or all there is
+  {
+    // A workgroup of pass B has a compute unit to itself (sixteen wavefronts of 82
+    // registers) and issues what there is to issue: a batch of few samples leaves
+    // units idle.  One drawing 26.5 us with a workgroup a sample, 14 with as many
+    // as it is worth; 61 images 24 and 16.5 with four; 33 samples of a 47^3 field 73
+    // and 28 with seven.  Two (100 drawings) are 31.5 and 28, and what they work out
+    // twice costs a pass with forward lanes beside them 1 %: one, then.
+    long long n[PYR_MAX_LEVELS + 1];
+    n[0] = src->nActive / a.batch + 1;
+    for (int l = 1; l < a.nMasks; ++l)
+      n[l] = recs[l - 1].out->seenActive / a.batch + 1;
+    const int want = PYR_CUS / a.batch;
+    pyr_plan_parts(a, n, want < 3 ? 1 : want);
+  }
+  // pass B's LDS: from the largest samples seen at every level, or all there is.
+  // What a part needs is what lets several workgroups share a compute unit; every
+  // layer of a sample has to fit with its input, however it is cut (a sample of
+  // which one does not is planned another way)
   long long ldsB = PYR_LDS_MAX;
   {
     bool known = !cs->wide && src->seenSample > 0;
-    long long sites = src->seenSample + src->seenSample / 2 + 64;
-    long long need = 15 * sites;
-    for (int l = 1; l < a.nMasks; ++l) {
-      const long long seen = recs[l - 1].out->seenSample;
+    long long n[PYR_MAX_LEVELS + 1];
+    for (int x = 0; x < a.nMasks; ++x) {
+      const long long seen = x ? recs[x - 1].out->seenSample : src->seenSample;
       known = known && seen > 0;
-      need += 11 * (seen + seen / 2 + 64);
+      n[x] = seen + seen / 2 + 64;
     }
-    if (known) {
-      need += fixedB;
-      ldsB = need < ldsB ? need : ldsB;
+    long long need = 4 * a.nChunks; // (the sums of the prefixes' chunks)
+    for (int x = 0; x < a.nMasks; ++x) {
+      const long long pair = 15 * n[x] + (x + 1 < a.nMasks ? 11 * n[x + 1] : 0);
+      need = pair > need ? pair : need;
     }
+    for (int p = 0; p < a.nParts; ++p) {
+      const PyrPart &part = a.parts[p];
+      const int xa = part.la >= 3 ? part.la - 2 : 0;
+      long long sites = 4 * n[xa];
+      for (int x = xa; x <= part.lb; ++x)
+        sites += 11 * (part.F > 1 ? n[x] / part.F + n[x] / (2 * part.F) + 64 : n[x]);
+      need = sites > need ? sites : need;
+    }
+    need += fixedB;
+    ldsB = known && need < ldsB ? need : ldsB;
   }
   ldsB = (ldsB + 15) / 16 * 16;
   a.ldsBytesB = (int)ldsB;
@@ -1442,16 +1614,37 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   a.mask = (1u << src->log2cap) - 1u;
   a.bits = src->bits.p;
   a.bg = src->bg.p;
-  SCN_TRY(cs->pyramid.reserve((size_t)a.batch * (size_t)pyrStride + 2));
-  SCN_TRY(cs->counts.reserve((size_t)a.nMasks * a.batch * 2 + 2));
-  if (!cs->flag.p) {
-    SCN_TRY(cs->flag.reserve(2));
-    SCN_TRY(scn_fill32(ctx, cs->flag.p, 0u, 4));
+  // Pass A: a wavefront per (sample, level, slab), each level from the source's
+  // rows, where those are short enough for registers; else one per sample, level
+  // after level
+  const int RW = pyr_set_fold(a);
+  long long wordsA = (8 * maskWords + 15) / 16 * 2 + PYR_A_GEO / 8;
+  a.slabs = 1;
+  if (RW) {
+    // (at most 8: 12 us for 33 samples of 47^3; a wavefront a level: 27)
+    for (int most = a.batch < 64 ? 8 : a.batch < 512 ? 512 / a.batch : 1;; most /= 2) {
+      a.slabs = most;
+      a.nSlabs = 0;
+      wordsA = 0;
+      for (int x = 0; x < a.nMasks; ++x) {
+        const int slabs = pyr_slabs(d, src->n, a.lv[x], most);
+        for (int z = 0; z < slabs; ++z, ++a.nSlabs) {
+          if (a.nSlabs < PYR_MAX_SLABS) {
+            a.slabLevel[a.nSlabs] = (unsigned char)x;
+            a.slabOf[a.nSlabs] = (unsigned char)z;
+          }
+          const long long words = pyr_slab_words(d, RW, src->n, a.lv[x], pyr_slab(d, a.lv[x], a.lv[x].magicN, z, slabs));
+          wordsA = x > 0 && words > wordsA ? words : wordsA;
+        }
+      }
+      if (a.nSlabs <= PYR_MAX_SLABS)
+        break;
+    }
   }
+  SCN_TRY(cs->pyramid.reserve((size_t)a.batch * (size_t)maskWords + 2));
+  SCN_TRY(cs->counts.reserve((size_t)a.nMasks * a.batch * a.slabs + 2));
   a.pyramid = cs->pyramid.p;
   a.counts = cs->counts.p;
-  a.flag = cs->flag.p;
-  a.ticket = (unsigned long long)++ctx->ticket;
   a.scalars = (long long *)ctx->d_pinned;
   a.badSites = (const long long *)(ctx->d_scalars + 15);
   cs->pyrSource = src;
@@ -1460,32 +1653,49 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
     std::call_once(once, [] {
-      const void *k[6] = {reinterpret_cast<const void *>(&k_pyr_masks<1>),
+      const void *k[10] = {reinterpret_cast<const void *>(&k_pyr_levels<2, 1>),
+                          reinterpret_cast<const void *>(&k_pyr_levels<2, 2>),
+                          reinterpret_cast<const void *>(&k_pyr_levels<2, 4>),
+                          reinterpret_cast<const void *>(&k_pyr_levels<3, 1>),
+                          reinterpret_cast<const void *>(&k_pyr_masks<1>),
                           reinterpret_cast<const void *>(&k_pyr_masks<2>),
                           reinterpret_cast<const void *>(&k_pyr_masks<3>),
                           reinterpret_cast<const void *>(&k_pyr_rules<1>),
                           reinterpret_cast<const void *>(&k_pyr_rules<2>),
                           reinterpret_cast<const void *>(&k_pyr_rules<3>)};
-      for (int i = 0; i < 6 && attr == hipSuccess; ++i)
+      for (int i = 0; i < 10 && attr == hipSuccess; ++i)
         attr = hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize,
                                    CHAIN_LDS_MAX);
     });
     SCN_HIP_CHECK(attr);
   }
-  const size_t ldsA = (size_t)(8 * pyrStride + PYR_A_EXTRA);
-  const dim3 grid((unsigned)a.batch);
+  const size_t ldsA = (size_t)(8 * wordsA + 16);
+  const dim3 grid((unsigned)a.batch), levels((unsigned)a.batch, (unsigned)a.nSlabs);
+  const dim3 gridB((unsigned)(a.batch * a.nParts + 1));
+  if (RW == 1 && d == 3)
+    hipLaunchKernelGGL((k_pyr_levels<3, 1>), levels, dim3(64), ldsA, ctx->stream, a);
+  else if (RW == 1)
+    hipLaunchKernelGGL((k_pyr_levels<2, 1>), levels, dim3(64), ldsA, ctx->stream, a);
+  else if (RW == 2)
+    hipLaunchKernelGGL((k_pyr_levels<2, 2>), levels, dim3(64), ldsA, ctx->stream, a);
+  else if (RW == 4)
+    hipLaunchKernelGGL((k_pyr_levels<2, 4>), levels, dim3(64), ldsA, ctx->stream, a);
+  else if (d == 1)
+    hipLaunchKernelGGL(k_pyr_masks<1>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
+  else if (d == 2)
+    hipLaunchKernelGGL(k_pyr_masks<2>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
+  else
+    hipLaunchKernelGGL(k_pyr_masks<3>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
+  SCN_HIP_CHECK(hipGetLastError());
   switch (d) {
   case 1:
-    hipLaunchKernelGGL(k_pyr_masks<1>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
-    hipLaunchKernelGGL(k_pyr_rules<1>, grid, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
+    hipLaunchKernelGGL(k_pyr_rules<1>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
     break;
   case 2:
-    hipLaunchKernelGGL(k_pyr_masks<2>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
-    hipLaunchKernelGGL(k_pyr_rules<2>, grid, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
+    hipLaunchKernelGGL(k_pyr_rules<2>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
     break;
   default:
-    hipLaunchKernelGGL(k_pyr_masks<3>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
-    hipLaunchKernelGGL(k_pyr_rules<3>, grid, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
+    hipLaunchKernelGGL(k_pyr_rules<3>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
     break;
   }
   SCN_HIP_CHECK(hipGetLastError());

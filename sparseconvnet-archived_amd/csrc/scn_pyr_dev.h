@@ -8,14 +8,15 @@
 // their rows in the order (owner's key, output's key).  Everything a layer's
 // rule book needs therefore follows from occupancy masks alone:
 //
-//   pass A  the masks of all layers of the sample: each is its input mask
-//           OR-ed over the window and thinned by the stride, up to 64 sites of
-//           a row at a time (pyr_dilate_pieces), plus a popcount prefix per
-//           word (the rank of a site = its position in iteration order);
-//   pass B  per output site, in five sweeps over ALL layers at once (or, for a
-//           sample too large for that, over as many consecutive layers as
-//           the LDS holds, window after window) with one barrier between
-//           them: enumerate the sites by rank; find each
+//   pass A  the masks of all layers of the sample: each is the source's rows
+//           OR-ed over the windows of all layers up to it and thinned by their
+//           strides (pyr_sweep_fold), or its input mask over one window, up to
+//           64 sites of a row at a time (pyr_dilate_pieces);
+//   pass B  a popcount prefix per mask word (the rank of a site = its position
+//           in iteration order), then per output site, in five sweeps over ALL
+//           layers of a part at once (or, for a sample too large for that, over
+//           as many consecutive layers as the LDS holds, window after window)
+//           with one barrier between them: enumerate the sites by rank; find each
 //           site's owner (first set bit of its window) and mark, in the owner's
 //           16-bit ownership mask, which of its candidates this is (an LDS
 //           atomic OR); prefix sums of the owned counts per layer; a site's row
@@ -38,7 +39,7 @@
 #endif
 
 #define PYR_MAX_LEVELS 24  // recorded layers of a chain
-#define PYR_HDR_BYTES 5248 // pass B's header and level tables in LDS
+#define PYR_HDR_BYTES 6528 // pass B's header and level tables in LDS
 #define PYR_CUBE_MAX 16    // ownership masks are 16 bits
 #define PYR_ROWS_MAX 65000 // rows of one sample at one layer (16-bit rows)
 enum { PYR_REGIONS = 0, PYR_TERMINAL = 1 };
@@ -54,6 +55,7 @@ struct PyrLevel {
   int maskOff; // of the mask in a sample's pyramid, in 64-bit words
   unsigned magicN, magicS; // floor(2^32 / nOut) + 1, floor(2^32 / size) + 1
   unsigned seg;    // output sites a piece of the dilation covers (the last piece of a row: what is left)
+  int foldS;       // the windows of all layers up to this one taken together: stride
   long long volOut, fullSize;
   // where the layer's results go
   int *rules;
@@ -65,7 +67,17 @@ struct PyrLevel {
   long long boundRows, boundActive;
   int slot;
   unsigned segs, magicSegs; // pieces in a row of the output field, floor(2^32 / segs) + 1
+  int foldW;                // ... and side
 };
+
+// What a workgroup of pass B does of a sample: layers la .. lb, or (F > 1, la ==
+// lb) the f-th of F slabs of one layer's output field along its first axis.
+struct PyrPart {
+  unsigned char la, lb, f, F;
+};
+#define PYR_MAX_PARTS 24
+#define PYR_MAX_SLABS 48
+#define PYR_MAX_CHUNKS 88
 
 struct PyrArgs {
   int nLevels; // recorded layers: levels 1 .. nLevels
@@ -77,14 +89,20 @@ struct PyrArgs {
   const pyr_u64 *bits; // the source batch's occupancy mask
   const int *bg;       // and background rows
   int maskWords;       // 64-bit words of all masks of a sample, spares included
-  int pyrStride;       // 64-bit words a sample takes in `pyramid`: masks, then 16-bit prefixes
-  pyr_u64 *pyramid;
-  int *counts; // [nLevels + 1][batch][2]: sites, has a background row
-  unsigned long long *flag;
-  unsigned long long ticket;
+  int pyrStride;       // 64-bit words of a sample's masks and 16-bit prefixes
+  pyr_u64 *pyramid; // [batch][maskWords]
+  int slabs;        // wavefronts of pass A a level may be shared out among
+  int nSlabs;       // levels and slabs there are
+  unsigned char slabLevel[PYR_MAX_SLABS], slabOf[PYR_MAX_SLABS];
+  int *counts;      // [nMasks][batch][slabs]: sites
   long long *scalars;
   const long long *badSites;
   int ldsBytesB; // dynamic LDS pass B is launched with
+  // rank prefixes are made a chunk of a level's mask words at a time
+  int nChunks;
+  unsigned char chunkLevel[PYR_MAX_CHUNKS], chunkOf[PYR_MAX_CHUNKS];
+  int nParts;
+  PyrPart parts[PYR_MAX_PARTS];
   PyrLevel lv[PYR_MAX_LEVELS + 1];
 };
 
@@ -298,6 +316,240 @@ PYR_FN pyr_u64 pyr_source_word(const pyr_u64 *bits, long long vol, int b, unsign
   return v;
 }
 
+// ------------------------------------------- pass A, a wavefront per level
+// Square windows compose: site j of level x is active iff the source has an
+// active site in [j S, j S + W) along every axis, S the product of the strides
+// up to x and W = 1 + the sum of (side - 1) times the stride before.  So a level
+// can be made from the source directly, and no level waits for the one before.
+// (Unless windows leave gaps that a later window would bridge, pyr_set_fold.  What
+// it costs: W / S source rows more or less a row of the field, two or three for
+// the usual chains at any depth.)
+// The source's rows of a sample, each on words of its own: RW of 64 bits.
+template <int RW>
+PYR_FN void pyr_stage_row(const pyr_u64 *bits, long long p, int n0, pyr_u64 (&out)[RW]) {
+  const unsigned char *w = reinterpret_cast<const unsigned char *>(bits) + 4 * (p >> 5);
+  const int sh = (int)(p & 31), last = (sh + n0 - 1) >> 5; // (nothing past the row's last word is read)
+  unsigned d[2 * RW + 1];
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 0; i <= 2 * RW; ++i)
+    __builtin_memcpy(&d[i], w + 4 * (i < last ? i : last), 4);
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 0; i < RW; ++i) {
+    pyr_u64 v = (pyr_u64)pyr_alignbit(d[2 * i + 1], d[2 * i], (unsigned)sh) |
+                ((pyr_u64)pyr_alignbit(d[2 * i + 2], d[2 * i + 1], (unsigned)sh) << 32);
+    const int left = n0 - 64 * i;
+    out[i] = left >= 64 ? v : left <= 0 ? 0ull : v & ((1ull << left) - 1ull);
+  }
+}
+// y |= y >> k over RW words (k < 64 RW)
+template <int RW> PYR_FN void pyr_or_shifted(pyr_u64 (&y)[RW], unsigned k) {
+  if (RW == 1) {
+    y[0] |= y[0] >> k;
+    return;
+  }
+  const unsigned words = k >> 6, sh = k & 63u;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 0; i < RW; ++i) {
+    pyr_u64 v = 0;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (int j = i; j < RW; ++j) {
+      if ((unsigned)(j - i) == words)
+        v |= y[j] >> sh;
+      if ((unsigned)(j - i) == words + 1 && sh)
+        v |= y[j] << (64u - sh);
+    }
+    y[i] |= v; // (the words above are still as they were)
+  }
+}
+// A row of the source OR-ed over the windows' other axes -> bits of an output row
+template <int RW> PYR_FN void pyr_fold_row(pyr_u64 (&y)[RW], int W, int S, int nOut) {
+  int k = 1; // bit t: any of the k sites from t on
+  for (; 2 * k <= W; k *= 2)
+    pyr_or_shifted<RW>(y, (unsigned)k);
+  if (k < W)
+    pyr_or_shifted<RW>(y, (unsigned)(W - k));
+  if ((S & (S - 1)) == 0) {
+    for (int s = S; s > 1; s >>= 1)
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+      for (int i = 0; i < RW; ++i) {
+        const pyr_u64 lo = 2 * i < RW ? pyr_even_bits(y[2 * i % RW]) : 0ull;
+        y[i] = lo | (2 * i + 1 < RW ? pyr_even_bits(y[(2 * i + 1) % RW]) << 32 : 0ull);
+      }
+  } else {
+    pyr_u64 r[RW];
+    for (int i = 0; i < RW; ++i)
+      r[i] = 0;
+    for (int j = 0; j < nOut; ++j) {
+      const int at = j * S;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+      for (int i = 0; i < RW; ++i) {
+        pyr_u64 bit = 0;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+        for (int q = 0; q < RW; ++q)
+          bit = q == at >> 6 ? (y[q] >> (at & 63)) & 1ull : bit;
+        if (i == j >> 6)
+          r[i] |= bit << (j & 63);
+      }
+    }
+    for (int i = 0; i < RW; ++i)
+      y[i] = r[i];
+  }
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+  for (int i = 0; i < RW; ++i) {
+    const int left = nOut - 64 * i;
+    y[i] = left >= 64 ? y[i] : left <= 0 ? 0ull : y[i] & ((1ull << left) - 1ull);
+  }
+}
+#define PYR_FOLD_DIRECT 2 // (three dimensions) sides up to this are OR-ed over two axes at once
+// Sets the layers' foldW, foldS.  Returns the words a source row takes in a lane's
+// registers, or 0: rows too long for that, one dimension, or windows with gaps.
+PYR_FN int pyr_set_fold(PyrArgs &a) {
+  const int n0 = a.lv[0].nOut;
+  a.lv[0].foldW = a.lv[0].foldS = 1;
+  for (int x = 1; x < a.nMasks; ++x) {
+    const PyrLevel &P = a.lv[x - 1];
+    PyrLevel &L = a.lv[x];
+    if (L.size > 1 && P.foldS > P.foldW)
+      return 0;
+    L.foldW = P.foldW + (L.size - 1) * P.foldS;
+    // (a stride beyond the field: a single site, whatever the stride)
+    const long long S = (long long)P.foldS * L.stride;
+    L.foldS = (int)(S < n0 ? S : n0);
+  }
+  if (a.d == 3)
+    return n0 <= 64 ? 1 : 0;
+  return a.d < 2 || n0 > 256 ? 0 : n0 <= 64 ? 1 : n0 <= 128 ? 2 : 4;
+}
+// A wavefront makes the words w0 .. w1 - 1 of a level's mask (slabs of the larger
+// fields' levels, so that one wavefront has not all of the work): the output rows
+// row0 .. row1 - 1 that reach into them, and for those the planes p0 .. p1 - 1 of
+// the source's rows (two dimensions: rows p0 .. p1 - 1).
+struct PyrSlab {
+  int w0, w1, row0, row1, p0, p1;
+};
+PYR_FN PyrSlab pyr_slab(int d, const PyrLevel &L, unsigned nOutMagic, int slab, int slabs) {
+  PyrSlab z;
+  z.w0 = (int)((long long)L.words * slab / slabs);
+  z.w1 = (int)((long long)L.words * (slab + 1) / slabs);
+  const int rows = d == 3 ? L.nOut * L.nOut : L.nOut;
+  z.row0 = (int)pyr_div(64u * (unsigned)z.w0, (unsigned)L.nOut, nOutMagic);
+  z.row1 = (int)pyr_div(64u * (unsigned)z.w1 + (unsigned)L.nOut - 1u, (unsigned)L.nOut, nOutMagic);
+  z.row1 = z.row1 < rows ? z.row1 : rows;
+  const int j0 = d == 3 ? (int)pyr_div((unsigned)z.row0, (unsigned)L.nOut, nOutMagic) : z.row0;
+  const int j1 = d == 3 ? (int)pyr_div((unsigned)z.row1 - 1u, (unsigned)L.nOut, nOutMagic) : z.row1 - 1;
+  z.p0 = j0 * L.foldS;
+  z.p1 = j1 * L.foldS + L.foldW;
+  return z;
+}
+// 64-bit words of LDS it takes: the source's rows, in three dimensions where
+// windows overlap much the rows OR-ed over the second axis, the mask
+PYR_FN long long pyr_slab_words(int d, int RW, int n0, const PyrLevel &L, const PyrSlab &z) {
+  const long long planes = z.p1 - z.p0;
+  return RW * planes * ((d == 3 ? n0 : 1) + (d == 3 && L.foldW > PYR_FOLD_DIRECT ? L.nOut : 0)) + (z.w1 - z.w0);
+}
+// How many slabs a level is worth, of `most`: the rows that a wavefront fetches and
+// makes set the pace, 512 of each or so
+PYR_FN int pyr_slabs(int d, int n0, const PyrLevel &L, int most) {
+  const int rows = d == 3 ? n0 * n0 : n0, own = d == 3 ? L.nOut : 4 * L.nOut;
+  int n = (rows + 511) / 512;
+  n = n < own / 4 ? n : own / 4; // (a few planes each)
+  n = n < L.words ? n : L.words;
+  n = n < most ? n : most;
+  return n > 0 ? n : 1;
+}
+template <int RW>
+PYR_FN void pyr_sweep_stage(const pyr_u64 *bits, long long first, int n0, int rows, pyr_u64 *dst, int t, int T) {
+#if defined(__HIPCC__)
+#pragma unroll 8
+#endif
+  for (int r = t; r < rows; r += T) {
+    pyr_u64 v[RW];
+    pyr_stage_row<RW>(bits, first + (long long)r * n0, n0, v);
+    for (int i = 0; i < RW; ++i)
+      dst[r * RW + i] = v[i];
+  }
+}
+// three dimensions: mid[p0][j1] = the source's rows [p0][j1 S .. + W), for `planes` planes
+template <int RW>
+PYR_FN void pyr_sweep_mid(const pyr_u64 *rows, pyr_u64 *mid, int planes, int n0, int nOut, unsigned magicN, int W,
+                          int S, int t, int T) {
+  for (unsigned m = (unsigned)t; m < (unsigned)(planes * nOut); m += (unsigned)T) {
+    const unsigned p0 = pyr_div(m, (unsigned)nOut, magicN), j1 = m - p0 * (unsigned)nOut;
+    const pyr_u64 *src = rows + (p0 * (unsigned)n0 + j1 * (unsigned)S) * RW;
+    pyr_u64 y[RW];
+    for (int i = 0; i < RW; ++i)
+      y[i] = src[i];
+    for (int q = 1; q < W; ++q)
+      for (int i = 0; i < RW; ++i)
+        y[i] |= src[q * RW + i];
+    for (int i = 0; i < RW; ++i)
+      mid[m * RW + i] = y[i];
+  }
+}
+// Words z.w0 .. of a level's mask (out: they start as zero) from the source's rows
+// (and `mid`), both from plane z.p0 on
+template <int D, int RW>
+PYR_FN void pyr_sweep_fold(const pyr_u64 *rows, const pyr_u64 *mid, pyr_u64 *out, const PyrSlab &z, int n0, int nOut,
+                           unsigned magicN, int W, int S, int t, int T) {
+  for (unsigned row = (unsigned)(z.row0 + t); row < (unsigned)z.row1; row += (unsigned)T) {
+    pyr_u64 y[RW];
+    for (int i = 0; i < RW; ++i)
+      y[i] = 0;
+    const pyr_u64 *src;
+    unsigned step; // between the rows to be OR-ed
+    int sides = 1; // of `step` 1
+    if (D == 2) {
+      src = rows + (row * (unsigned)S - (unsigned)z.p0) * RW;
+      step = RW;
+    } else {
+      const unsigned j0 = pyr_div(row, (unsigned)nOut, magicN), j1 = row - j0 * (unsigned)nOut;
+      const unsigned plane = j0 * (unsigned)S - (unsigned)z.p0;
+      if (W > PYR_FOLD_DIRECT) {
+        src = mid + (plane * (unsigned)nOut + j1) * RW;
+        step = (unsigned)nOut * RW;
+      } else {
+        src = rows + (plane * (unsigned)n0 + j1 * (unsigned)S) * RW;
+        step = (unsigned)n0 * RW;
+        sides = W;
+      }
+    }
+    for (int q = 0; q < W; ++q)
+      for (int u = 0; u < sides; ++u)
+        for (int i = 0; i < RW; ++i)
+          y[i] |= src[(unsigned)q * step + (unsigned)(u * RW + i)];
+    pyr_fold_row<RW>(y, W, S, nOut);
+    const unsigned pos = row * (unsigned)nOut, sh = pos & 63u;
+    const int at = (int)(pos >> 6);
+    pyr_u64 carry = 0;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (int i = 0; i <= RW; ++i) {
+      const pyr_u64 here = i < RW ? y[i % RW] : 0ull;
+      const pyr_u64 v = carry | (here << sh);
+      carry = sh ? here >> (64u - sh) : 0ull;
+      if (v && at + i >= z.w0 && at + i < z.w1) // (the other words are other slabs')
+        PYR_ATOMIC_OR64(&out[at + i - z.w0], v);
+    }
+  }
+}
+
 // Pass B takes a sample's layers a WINDOW of levels xa .. xb at a time: level
 // xa as input only (its rows known: the source's, or from the window before),
 // layers xa + 1 .. xb built.  LDS bytes of a window for a sample with n[x]
@@ -312,27 +564,51 @@ PYR_FN long long pyr_lds_window(const PyrArgs &a, const int *n, int xa, int xb) 
 }
 // The window that starts at level xa: as many layers as fit (at least one,
 // when there is one)
-PYR_FN int pyr_window_end(const PyrArgs &a, const int *n, int xa) {
-  int xb = xa + 1 < a.nMasks ? xa + 1 : xa;
+PYR_FN int pyr_window_end(const PyrArgs &a, const int *n, int xa, int xLast = -1) {
+  if (xLast < 0)
+    xLast = a.nMasks - 1;
+  int xb = xa < xLast ? xa + 1 : xa;
   long long total = n[xa] + (xb > xa ? n[xb] : 0);
   const long long fixed = PYR_HDR_BYTES + 8ll * a.pyrStride + 4ll * n[xa] + 6 * 16;
-  while (xb + 1 < a.nMasks && fixed + 11ll * (total + n[xb + 1]) <= a.ldsBytesB) {
+  while (xb < xLast && fixed + 11ll * (total + n[xb + 1]) <= a.ldsBytesB) {
     total += n[xb + 1];
     ++xb;
   }
   return xb;
 }
-// Whether every layer of the sample fits by itself
-PYR_FN bool pyr_fits(const PyrArgs &a, const int *n) {
-  bool fits = pyr_lds_window(a, n, 0, a.nMasks > 1 ? 1 : 0) <= a.ldsBytesB;
-  for (int x = 1; x + 1 < a.nMasks; ++x)
-    fits = fits && pyr_lds_window(a, n, x, x + 1) <= a.ldsBytesB;
+// Whether level x fits with the one after it, n0 and n1 sites
+PYR_FN bool pyr_pair_fits(const PyrArgs &a, int n0, int n1) {
+  return PYR_HDR_BYTES + 8ll * a.pyrStride + 11ll * ((long long)n0 + n1) + 4ll * n0 + 6 * 16 <= a.ldsBytesB;
+}
+// Whether every layer of the sample fits by itself; sites(x): of level x
+template <typename N> PYR_FN bool pyr_fits_of(const PyrArgs &a, N sites) {
+  bool fits = true;
+  for (int x = 0; x == 0 || x + 1 < a.nMasks; ++x)
+    fits = fits && pyr_pair_fits(a, sites(x), x + 1 < a.nMasks ? sites(x + 1) : 0);
   return fits;
+}
+PYR_FN bool pyr_fits(const PyrArgs &a, const int *n) {
+  return pyr_fits_of(a, [n](int x) { return n[x]; });
 }
 
 // ------------------------------------------------------------------- pass B
+// Sets the list of chunks, of 256 words (false: too many of them)
+#define PYR_CHUNK 256
+PYR_FN bool pyr_set_chunks(PyrArgs &a) {
+  a.nChunks = 0;
+  for (int x = 0; x < a.nMasks; ++x)
+    for (int c = 0; PYR_CHUNK * c < a.lv[x].words + 2; ++c, ++a.nChunks) {
+      if (a.nChunks == PYR_MAX_CHUNKS)
+        return false;
+      a.chunkLevel[a.nChunks] = (unsigned char)x;
+      a.chunkOf[a.nChunks] = (unsigned char)c;
+    }
+  return true;
+}
+
 struct PyrHdr {
   int n[PYR_MAX_LEVELS + 1];       // this sample's sites at level x
+  int words[PYR_MAX_LEVELS + 1], maskOff[PYR_MAX_LEVELS + 1]; // its mask's words and where they are (with prefixes to make)
   int hasBg[PYR_MAX_LEVELS + 1];   // and whether it has a background row there
   int siteOff[PYR_MAX_LEVELS + 2]; // where level x of the current window starts in the per-site arrays
   int itemOff[PYR_MAX_LEVELS + 2]; // output sites of the window's layers before layer l (index l)
@@ -341,7 +617,19 @@ struct PyrHdr {
   long long actAll[PYR_MAX_LEVELS + 1], bgAll[PYR_MAX_LEVELS + 1];
   int over; // some layer outgrew its bounds, or a sample the LDS
   int total; // sites of this sample over the levels of the current window
+  // What a part of a sample takes (cut: otherwise all of it).  Ranks lo .. lo +
+  // held - 1 of a level are held in LDS; as the input of the next layer, ranks
+  // own .. ownEnd - 1 count what they own; layers from emitFrom on are written,
+  // of a layer in slabs its output ranks emit .. emitEnd - 1.
+  int cut, emitFrom, slab;
+  int lo[PYR_MAX_LEVELS + 1], held[PYR_MAX_LEVELS + 1];
+  int own[PYR_MAX_LEVELS + 1], ownEnd[PYR_MAX_LEVELS + 1];
+  int before[PYR_MAX_LEVELS + 1]; // held outputs of level x that inputs before `own` own
+  int emit, emitEnd;
+  int plane[2]; // where this part's slab starts and ends along the first axis
 };
+PYR_FN int pyr_held(const PyrHdr *h, int x) { return h->cut ? h->held[x] : h->n[x]; }
+PYR_FN int pyr_lo(const PyrHdr *h, int x) { return h->cut ? h->lo[x] : 0; }
 // What the sweeps need of layer l, once per item: kept in LDS (the kernel
 // arguments are far away for a lane that wants the entry of ITS layer), the
 // geometry in one 16-byte read, the rest as the sweeps come to it.
@@ -349,10 +637,14 @@ struct PyrLv {
   int size, stride, nIn, nOut;
   int width;
   unsigned magicS;
-  int inMaskOff, inSiteOff; // mask and sites of the layer's input (level l - 1)
-  int siteOff, n;           // sites of the layer's output (level l)
+  int inMaskOff, inSiteOff; // mask and sites of the layer's input (level l - 1): rank r is at inSiteOff + r
+  int siteOff, n;           // sites of the layer's output (level l) that are held
   int bgIn;                 // batch-global row of the input's background row, or -1
-  int flags;                // PYR_LV_SOURCE: the input is the window's first level, its rows are in srcRow; PYR_LV_TERMINAL
+  int flags;                // PYR_LV_*
+  int inLo;                 // rank of the first input site that is held
+  int own, ownEnd;          // input ranks that count what they own
+  int emit, emitEnd;        // the held output sites that are written
+  int pad[3];
   long long rowBase;        // batch-global row of this sample's row 0 at level l
   long long actBefore;      // entries of the samples before this one at level l
   long long inRowBase;      // rowBase of the input level (0 for the source)
@@ -364,14 +656,16 @@ struct PyrLv {
   long long boundActive;
   int *bg;
 };
-enum { PYR_LV_SOURCE = 1, PYR_LV_TERMINAL = 2 };
+// SOURCE: the input is the window's first level, its rows are in srcRow; QUIET:
+// the layer's rows are wanted by the next one, another workgroup writes it
+enum { PYR_LV_SOURCE = 1, PYR_LV_TERMINAL = 2, PYR_LV_QUIET = 4 };
 // What the enumeration needs of level x (x < nMasks), in one 16-byte read
 struct PyrEn {
   int maskOff, nOut;
   unsigned magicN;
   int siteOff;
 };
-#define PYR_LV_AT 1536
+#define PYR_LV_AT 2048
 #define PYR_EN_AT (PYR_LV_AT + (PYR_MAX_LEVELS + 1) * (int)sizeof(PyrLv))
 static_assert(sizeof(PyrHdr) <= PYR_LV_AT, "header");
 static_assert(PYR_EN_AT + (PYR_MAX_LEVELS + 1) * sizeof(PyrEn) <= PYR_HDR_BYTES, "level tables");
@@ -432,18 +726,25 @@ PYR_FN void pyr_fill_level(const PyrLevel &L, int inMaskOff, int bgSource, const
   v.width = L.width;
   v.magicS = L.magicS;
   v.inMaskOff = inMaskOff;
-  v.inSiteOff = h->siteOff[l - 1];
+  v.inLo = pyr_lo(h, l - 1);
+  v.inSiteOff = h->siteOff[l - 1] - v.inLo;
   const bool region = L.kind == PYR_REGIONS;
   v.siteOff = region ? h->siteOff[l] : 0;
-  v.n = region ? h->n[l] : 0;
+  v.n = region ? pyr_held(h, l) : 0;
   const int x = l - 1;
-  v.flags = (x == xa ? PYR_LV_SOURCE : 0) | (region ? 0 : PYR_LV_TERMINAL);
+  const bool quiet = l < h->emitFrom;
+  v.flags = (x == xa ? PYR_LV_SOURCE : 0) | (region ? 0 : PYR_LV_TERMINAL) | (quiet ? PYR_LV_QUIET : 0);
+  v.own = h->cut ? h->own[x] : 0;
+  v.ownEnd = h->cut ? h->ownEnd[x] : h->n[x];
+  v.emit = h->cut && region ? h->emit - h->lo[l] : 0;
+  v.emitEnd = h->cut && region ? h->emitEnd - h->lo[l] : v.n;
+  v.pad[0] = v.pad[1] = v.pad[2] = 0;
   v.inRowBase = x == 0 ? 0 : h->actBefore[x] + h->bgBefore[x];
   v.bgIn = x == 0 ? bgSource : (h->hasBg[x] ? (int)v.inRowBase + h->n[x] : -1);
   v.rowBase = region ? h->actBefore[l] + h->bgBefore[l] : 0;
   v.actBefore = region ? h->actBefore[l] : 0;
   v.volOut = L.volOut;
-  v.rules = L.rules;
+  v.rules = quiet ? nullptr : L.rules;
   v.capacity = L.capacity;
   v.ekey = L.ekey;
   v.erow = L.erow;
@@ -459,11 +760,158 @@ PYR_FN void pyr_fill_offsets(PyrHdr *h, int xa, int xb, int t) {
     return;
   int sum = 0;
   for (int x = xa; x < t; ++x)
-    sum += h->n[x];
+    sum += pyr_held(h, x);
   h->siteOff[t] = sum;
-  h->itemOff[t] = t > xa ? sum - h->n[xa] : 0;
+  h->itemOff[t] = t > xa ? sum - pyr_held(h, xa) : 0;
   if (t == xb + 1)
     h->total = sum;
+}
+
+// rank of the first site of level x at leading coordinate j (all of them: j = nOut)
+PYR_FN int pyr_rank_of_plane(const PyrArgs &a, const PyrLds &s, int x, int j) {
+  const PyrLevel &L = a.lv[x];
+  unsigned p = (unsigned)j;
+  for (int q = 1; q < a.d; ++q)
+    p *= (unsigned)L.nOut;
+  return (int)pyr_rank(s.masks + L.maskOff, s.pref + L.maskOff, p);
+}
+// The slabs of a level start at the planes that hold the f-th parts of its sites
+// (a surface in the middle of its field leaves a field's equal parts unequal
+// work): a lane a plane looks whether this part's slab starts or ends there.
+// Lane 0 has set h->plane to {f ? nOut : 0, nOut} before.
+PYR_FN void pyr_sweep_planes(const PyrArgs &a, const PyrLds &s, const PyrPart &p, int t, int T) {
+  PyrHdr *h = s.h;
+  const int x = p.la, nOut = a.lv[x].nOut;
+  const int r0 = (int)((long long)h->n[x] * p.f / p.F), r1 = (int)((long long)h->n[x] * (p.f + 1) / p.F);
+  for (int j = t; j < nOut; j += T) {
+    const int from = pyr_rank_of_plane(a, s, x, j), to = pyr_rank_of_plane(a, s, x, j + 1);
+    if (p.f > 0 && from <= r0 && r0 < to)
+      h->plane[0] = j;
+    if (p.f + 1 < p.F && from <= r1 && r1 < to)
+      h->plane[1] = j;
+  }
+}
+// What a part in slabs holds, a lane a number (t < PYR_CUT_LANES; the masks and
+// their prefixes are in LDS, h->n and h->plane are set).  A slab of layer l's
+// outputs, planes [J0, J1), has windows over the input planes I = [J0 stride,
+// (J1 - 1) stride + side).  A row is the number of outputs owned by inputs before
+// the output's owner, and by the owner itself through later candidates: all
+// outputs whose windows end before I belong to inputs before I; those whose
+// windows meet I are held and looked at one by one.  The rows of I are wanted too:
+// the same again for layer l - 1 with I in the place of [J0, J1).
+#define PYR_CUT_LANES 10
+PYR_FN void pyr_fill_cut(const PyrArgs &a, const PyrLds &s, const PyrPart &p, int t) {
+  PyrHdr *h = s.h;
+  if (t >= PYR_CUT_LANES)
+    return;
+  const int back = t < 6 ? 0 : 1; // lanes 0 .. 5: layer l, and 6 .. 9 the one before
+  const int l = p.la - back;
+  if (l < 1)
+    return;
+  int j0 = h->plane[0], j1 = h->plane[1], i0 = 0, i1 = 0, o0 = 0, o1 = 0;
+  for (int u = 0; u <= back; ++u) {
+    if (u)
+      j0 = i0, j1 = i1;
+    const PyrLevel &L = a.lv[p.la - u];
+    if (j0 < j1) {
+      i0 = j0 * L.stride;
+      i1 = (j1 - 1) * L.stride + L.size;
+      o0 = i0 < L.size ? 0 : (i0 - L.size) / L.stride + 1; // the first window that ends behind i0
+      o1 = (i1 - 1) / L.stride + 1;                        // the first that starts at i1 or later
+      o1 = o1 < L.nOut ? o1 : L.nOut;
+    }
+  }
+  const int lane = t < 6 ? t : t - 4; // 0, 1: what is written; 2, 3: held outputs; 4, 5: input ranks
+  const int at = lane == 0 ? j0 : lane == 1 ? j1 : lane == 2 ? o0 : lane == 3 ? o1 : lane == 4 ? i0 : i1;
+  const int rank = pyr_rank_of_plane(a, s, lane < 4 ? l : l - 1, at);
+  if (lane == 0)
+    h->emit = rank;
+  else if (lane == 1)
+    h->emitEnd = rank;
+  else if (lane == 2)
+    h->lo[l] = rank;
+  else if (lane == 3)
+    h->held[l] = rank; // (its end: pyr_fix_cut)
+  else if (lane == 4)
+    h->own[l - 1] = rank;
+  else
+    h->ownEnd[l - 1] = rank;
+}
+// (after a barrier; lane 0)
+PYR_FN void pyr_fix_cut(PyrHdr *h, const PyrPart &p) {
+  const int last = p.la > 1 ? p.la - 1 : p.la;
+  for (int l = p.la; l >= last; --l)
+    h->held[l] -= h->lo[l];
+  h->lo[last - 1] = h->own[last - 1];
+  h->held[last - 1] = h->ownEnd[last - 1] - h->own[last - 1];
+}
+// the rows owned by the inputs before level x's own ones: where its bases start
+PYR_FN int pyr_base_start(const PyrHdr *h, int x) { return h->cut ? h->lo[x + 1] + h->before[x + 1] : 0; }
+
+// How many workgroups a sample is worth, and which layers each of them takes.
+// n[x]: sites of a typical sample at level x.  A workgroup's cost is taken as its
+// sites, weighted by what the sweeps were measured to issue per site; a part
+// that starts behind the first layer works the rows of the layer before out again.
+PYR_FN long long pyr_part_cost(const PyrArgs &a, const long long *n, int la, int lb) {
+  const int ENUM = 18, OWNER = 14, ROWS = 9, BASES = 8;
+  long long c = la > 1 ? n[la - 1] * (ENUM + OWNER + ROWS) + n[la - 2] * BASES : n[0] * ENUM;
+  for (int l = la; l <= lb; ++l)
+    c += n[l] * (ENUM + OWNER + ROWS + 10 + 3 * a.lv[l].width) + n[l - 1] * BASES;
+  return c;
+}
+// parts of at most `most` cost each (slabs where a layer costs more); their number
+PYR_FN int pyr_cut_parts(const PyrArgs &a, const long long *n, long long most, PyrPart *parts, int room) {
+  int count = 0;
+  const int last = a.nMasks - 1;
+  for (int la = 1; la <= last;) {
+    int lb = la, F = 1;
+    const long long c = pyr_part_cost(a, n, la, la);
+    if (c > most) {
+      long long want = (c + most - 1) / most;
+      want = want < a.lv[la].nOut ? want : a.lv[la].nOut;
+      // (the terminal layer lists all rows of the last level: that one stays whole)
+      F = la == last && a.nLevels > last ? 1 : want < 255 ? (int)want : 255;
+    } else {
+      while (lb < last && pyr_part_cost(a, n, la, lb + 1) <= most)
+        ++lb;
+    }
+    for (int f = 0; f < F; ++f, ++count)
+      if (count < room) {
+        PyrPart p = {(unsigned char)la, (unsigned char)lb, (unsigned char)f, (unsigned char)F};
+        parts[count] = p;
+      }
+    la = lb + 1;
+  }
+  return count;
+}
+// Sets a.parts: at most `want` parts, none cheaper than it is worth (512 sites
+// or so: half a round of a workgroup's lanes).  n: null when nothing is known.
+#ifndef PYR_PART_MIN
+#define PYR_PART_MIN (128 * 64)
+#endif
+PYR_FN void pyr_plan_parts(PyrArgs &a, const long long *n, int want) {
+  const PyrPart all = {1, (unsigned char)(a.nMasks - 1), 0, 1};
+  a.nParts = 1;
+  a.parts[0] = all;
+  want = want < PYR_MAX_PARTS ? want : PYR_MAX_PARTS;
+  if (!n || want <= 1 || a.nMasks <= 1)
+    return;
+  long long lo = PYR_PART_MIN, hi = pyr_part_cost(a, n, 1, a.nMasks - 1);
+  if (hi <= lo)
+    return;
+  // (the smallest cost that cuts into few enough parts, within a sixteenth)
+  while (hi - lo > lo / 16) {
+    const long long mid = lo + (hi - lo) / 2;
+    if (pyr_cut_parts(a, n, mid, a.parts, 0) <= want)
+      hi = mid;
+    else
+      lo = mid;
+  }
+  const int count = pyr_cut_parts(a, n, hi, a.parts, PYR_MAX_PARTS);
+  if (count <= PYR_MAX_PARTS)
+    a.nParts = count;
+  else
+    a.parts[0] = all;
 }
 
 // Entry x of the enumeration's table (x < nMasks; siteOff: in the current window)
@@ -579,8 +1027,10 @@ PYR_FN void pyr_owner(const PyrLv &v, const PyrLds &s, int r, int *kStar, unsign
 
 #if defined(__HIP_DEVICE_COMPILE__)
 #define PYR_ATOMIC_OR(ptr, v) atomicOr((ptr), (v))
+#define PYR_ATOMIC_ADD(ptr, v) atomicAdd((ptr), (v))
 #else
 #define PYR_ATOMIC_OR(ptr, v) (*(ptr) |= (v))
+#define PYR_ATOMIC_ADD(ptr, v) (*(ptr) += (v))
 #endif
 
 // ---- sweep 0: the ownership masks start empty (no barrier is needed between
@@ -636,11 +1086,11 @@ template <int D>
 PYR_FN void pyr_sweep_enumerate(const PyrArgs &a, const PyrLds &s, int xa, int xb, int t, int T) {
   const int total = s.h->total;
   int x = xa;
-  for (int i = (xa > 0 ? s.h->n[xa] : 0) + t; i < total; i += T) {
+  for (int i = (xa > 0 || s.h->emitFrom > 1 ? pyr_held(s.h, xa) : 0) + t; i < total; i += T) {
     while (x + 1 <= xb && i >= s.en[x + 1].siteOff)
       ++x;
     const PyrEn e = s.en[x];
-    const unsigned r = (unsigned)(i - e.siteOff);
+    const unsigned r = (unsigned)(i - e.siteOff + pyr_lo(s.h, x));
     // (the level's two spare words have the level's count as prefix: > r)
     const int span = (x + 1 < a.nMasks ? s.en[x + 1].maskOff : a.maskWords) - e.maskOff;
     const unsigned short *pref = s.pref + e.maskOff;
@@ -663,10 +1113,13 @@ PYR_FN void pyr_sweep_enumerate(const PyrArgs &a, const PyrLds &s, int xa, int x
   }
 }
 
-// ---- sweep 2: every output site tells its owner which candidate it is
+// ---- sweep 2: every output site tells its owner which candidate it is.  (Of a
+// part's outputs some are owned by inputs before its own: counted; some by
+// inputs behind them: nobody here asks for their rows.)
+#define PYR_NOT_MINE 255
 template <int D>
 PYR_FN void pyr_sweep_owners(const PyrLds &s, int la, int lb, int t, int T) {
-  const PyrHdr *h = s.h;
+  PyrHdr *h = s.h;
   const int items = h->itemOff[lb + 1];
   int l = la;
   for (int it = t; it < items; it += T) {
@@ -676,6 +1129,12 @@ PYR_FN void pyr_sweep_owners(const PyrLds &s, int la, int lb, int t, int T) {
     unsigned rank;
     const int r = it - h->itemOff[l];
     pyr_owner<D>(v, s, r, &k, &rank);
+    if ((int)rank < v.own || (int)rank >= v.ownEnd) {
+      if ((int)rank < v.own)
+        PYR_ATOMIC_ADD(&h->before[l], 1);
+      s.kOf[v.siteOff + r] = PYR_NOT_MINE;
+      continue;
+    }
     const unsigned at = (unsigned)v.inSiteOff + rank;
     PYR_ATOMIC_OR(&s.own[at >> 1], 1u << (k + 16 * (int)(at & 1u)));
     // (kept for sweep 4, which then has no window to look at)
@@ -699,10 +1158,14 @@ PYR_FN void pyr_sweep_rows(const PyrLds &s, int la, int lb, int b, int t, int T)
     const PyrLv &v = s.lv[l];
     const int r = it - h->itemOff[l];
     const int k = s.kOf[v.siteOff + r];
+    if (k == PYR_NOT_MINE)
+      continue;
     const unsigned at = (unsigned)v.inSiteOff + s.row[v.siteOff + r];
     // the owner's candidates after this one are the outputs before it
     const unsigned row = s.base[at] + (unsigned)pyr_popc32(pyr_own_mask(s, at) >> (k + 1));
     s.row[v.siteOff + r] = (unsigned short)row;
+    if ((v.flags & PYR_LV_QUIET) || r < v.emit || r >= v.emitEnd)
+      continue;
     int j[D];
     pyr_unpack<D>(s.key[v.siteOff + r], j);
     const long long entry = v.actBefore + row;
@@ -716,8 +1179,8 @@ PYR_FN void pyr_sweep_rows(const PyrLds &s, int la, int lb, int b, int t, int T)
 // batch-global row of the input site with rank `rank` of layer v
 PYR_FN int pyr_in_row(const PyrLv &v, const PyrLds &s, unsigned rank) {
   if (v.flags & PYR_LV_SOURCE)
-    return (int)s.srcRow[rank];
-  return (int)v.inRowBase + (int)s.row[v.inSiteOff + rank];
+    return (int)s.srcRow[rank - (unsigned)v.inLo];
+  return (int)v.inRowBase + (int)s.row[(unsigned)v.inSiteOff + rank];
 }
 // batch-global row of level x's background row of this sample (-1: none)
 PYR_FN int pyr_bg_row(const PyrArgs &a, const PyrLds &s, int x, int b) {
@@ -739,13 +1202,17 @@ template <int D>
 PYR_FN void pyr_sweep_rules(const PyrLds &s, int la, int lb, int t, int T) {
   const PyrHdr *h = s.h;
   const int items = h->itemOff[lb + 1];
-  int l = la;
-  for (int it = t; it < items; it += T) {
+  int l = la > h->emitFrom ? la : h->emitFrom; // (the layers before are another workgroup's)
+  if (l > lb)
+    return;
+  for (int it = h->itemOff[l] + t; it < items; it += T) {
     l = pyr_item_level(h, lb, it, l);
     const PyrLv &v = s.lv[l];
     if (!v.rules)
       continue;
     const int r = it - h->itemOff[l];
+    if (r < v.emit || r >= v.emitEnd)
+      continue;
     const pyr_u64 *in = s.masks + v.inMaskOff;
     const unsigned short *pref = s.pref + v.inMaskOff;
     int j[D];
@@ -809,7 +1276,7 @@ PYR_FN void pyr_sweep_carry(const PyrLds &s, unsigned char *lds, const PyrArgs &
   const unsigned short *row = s.row + h->siteOff[xb];
   unsigned *dst = reinterpret_cast<unsigned *>(lds + PYR_HDR_BYTES + 8ll * a.pyrStride);
   const long long rowBase = h->actBefore[xb] + h->bgBefore[xb];
-  for (int i = t; i < h->n[xb]; i += T)
+  for (int i = t; i < pyr_held(h, xb); i += T)
     dst[i] = (unsigned)(rowBase + row[i]);
 }
 
@@ -820,8 +1287,12 @@ PYR_FN void pyr_sweep_tail(const PyrArgs &a, const PyrLds &s, int la, int lb, in
   const PyrHdr *h = s.h;
   const int W = T >= 64 ? 64 : T;
   const int lane = t % W, wave = t / W, waves = T / W;
+  if (h->slab > 0) // (the first slab of a layer does this)
+    return;
   for (int l = la + wave; l <= lb; l += waves) {
     const PyrLv &v = s.lv[l];
+    if (v.flags & PYR_LV_QUIET)
+      continue;
     const int bgOut = pyr_bg_row(a, s, l, b);
     if (h->hasBg[l] && v.rules && bgOut >= 0 &&
         ((long long)bgOut + 1) * v.width <= v.capacity) { // Regions.cu:647-652
