@@ -330,6 +330,17 @@ int scn_maxpool_checked(scn_ctx *ctx, const float *d_in, int64_t nInRows,
  * before the first negative rule, summed in rule order. */
 int scn_terminal_pool(scn_ctx *ctx, const float *d_in, float *d_out,
                       const int32_t *d_rules, int64_t count, int S, int C);
+/* scn_terminal_pool into d_pooled [M x K], scn_nin_forward with SCN_SOFTMAX on it
+ * into d_probs [M x N], and a copy of the probabilities to `copy` (pinned host or
+ * device memory; null: none), in one launch and to the same bits.  Where
+ * scn_terminal_classifier_supported says 0 the three calls stay three:
+ * SCN_ERR_ARG. */
+int scn_terminal_classifier_supported(int64_t M, int K, int N);
+int scn_terminal_classifier(scn_ctx *ctx, const float *d_in,
+                            const int32_t *d_rules, int64_t M, int S,
+                            float *d_pooled, const float *d_W,
+                            const float *d_B, float *d_probs, float *copy,
+                            int K, int N, float p);
 /* dSigmoidSoftmax (SigmoidLayer.cu:160-177). */
 int scn_softmax_rows(scn_ctx *ctx, const float *d_in, float *d_out, int64_t M,
                      int N);

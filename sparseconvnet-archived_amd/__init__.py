@@ -122,6 +122,8 @@ def lib():
         "scn_maxpool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp]),
         "scn_maxpool_checked": (C.c_int, [vp, vp, i64, vp, vp, i64, C.c_int, C.c_int, vp]),
         "scn_terminal_pool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_terminal_classifier_supported": (C.c_int, [i64, C.c_int, C.c_int]),
+        "scn_terminal_classifier": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float]),
         "scn_softmax_rows": (C.c_int, [vp, vp, vp, i64, C.c_int]),
         "scn_softmax_grad": (C.c_int, [vp, vp, vp, vp, i64, C.c_int]),
         "scn_activation_backward": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),
@@ -310,6 +312,10 @@ class Context:
 
     def terminal_pool(self, d_in, d_out, d_rules, count, S, Cn):
         _check(lib().scn_terminal_pool(self.h, d_in.ptr, d_out.ptr, d_rules.ptr, count, S, Cn))
+
+    def terminal_classifier(self, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, p=1.0):
+        _check(lib().scn_terminal_classifier(self.h, d_in.ptr, d_rules.ptr, M, S, d_pooled.ptr, d_W.ptr, d_B.ptr,
+                                             d_probs.ptr, copy.ptr if copy is not None else None, K, N, p))
 
     def softmax_rows(self, d_in, d_out, M, N):
         _check(lib().scn_softmax_rows(self.h, d_in.ptr, d_out.ptr, M, N))

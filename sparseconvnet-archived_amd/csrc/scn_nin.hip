@@ -269,6 +269,185 @@ __global__ void __launch_bounds__(FR_THREADS)
   }
 }
 
+// ---- the classifier: few rows, at most 128 classes, soft-max --------------------
+// What bounds it is the work of the few compute units it runs on, each of which
+// reads all of W through a path that takes sixteen cycles an instruction whatever
+// that fetches: 17.5 us for 61 rows of 800 x 100 with eight rows a workgroup and a
+// float a lane.  So a workgroup has two rows, a lane four neighbouring classes and
+// half of its wavefront's share of K, sixteen bytes a load, and the next loads are
+// under way while a batch is multiplied.  The soft-max of a row is taken by one
+// wavefront (running maximum from -10000, lanes striding over the classes, as in
+// the kernel that does it as a pass of its own).
+// TERMINAL: the rows are the means of a terminal pooling, taken on the way into
+// LDS with the arithmetic of k_terminal_pool and written down too, and the
+// probabilities also go where the host reads them: a net's last three launches,
+// each a few microseconds of launch, trips to memory and drain, in one (1 x 192 x
+// 100: 3.1 + 6.7 + 2.3 us and two gaps -> 5.8; 100 rows 4.0 + 8.7 + 2.4 -> 6.1; 33
+// x 128 x 40 4.4 + 5.5 + 2.6 -> 6.4; 61 x 800 x 100 4.9 + 17.5 + 3.3 -> 11.0).
+#define CL_DEPTH 12
+#define CL_ROWS 2
+struct TerminalSource {
+  const int *rules; // [M x S]
+  int S;
+  const long long *meta;
+  float *pooled; // [M x K]
+  float *copy;   // [M x N], or null
+};
+template <bool TERMINAL>
+__global__ void __launch_bounds__(FR_THREADS)
+    k_classifier(const float *__restrict__ A, const float *__restrict__ W, float *__restrict__ out, long long M, int K,
+                 int N, Epilogue ep, const long long *dRows, TerminalSource ts) {
+  M = live_rows(M, dRows);
+  if ((long long)blockIdx.x * CL_ROWS >= M)
+    return;
+  __shared__ __attribute__((aligned(16))) float sA[CL_ROWS][FR_MAX_K];
+  __shared__ __attribute__((aligned(16))) float part[FR_WAVES][CL_ROWS][128];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long long m0 = (long long)blockIdx.x * CL_ROWS;
+  // a row of A and four of its channels; TERMINAL: the first of its rules are asked
+  // for before W
+  const int k = 4 * (tid & 255), row = tid >> 8;
+  const long long mRow = m0 + row;
+  static_assert(FR_THREADS == 256 * CL_ROWS, "a quarter of FR_MAX_K lanes a row");
+  constexpr int RULES = 8; // at a time
+  int S = ts.S, rule[RULES];
+  auto load_rules = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < RULES; ++u)
+      rule[u] = mRow < M && p0 + u < S ? ts.rules[mRow * S + p0 + u] : -1;
+  };
+  if constexpr (TERMINAL) {
+    if (ts.meta) // (the width is a bound, the rows lie at the true one)
+      S = ts.meta[META_OVERFLOW] ? 0 : (int)(ts.meta[META_WIDTH] < S ? ts.meta[META_WIDTH] : S);
+    load_rules(0);
+  }
+  const int half = lane >> 5, n = 4 * (lane & 31) < N ? 4 * (lane & 31) : 0; // (past the end: not used)
+  const int per = (K + 2 * FR_WAVES - 1) / (2 * FR_WAVES) * 2; // k of a wavefront, two a load
+  const int k0 = wave * per < K ? wave * per : K, k1 = min(K, k0 + per);
+  const float *const w = W + n;
+  float4 wv[2][CL_DEPTH];
+  auto load_w = [&](int b, int k) {
+#pragma unroll
+    for (int i = 0; i < CL_DEPTH; ++i) {
+      int kk = k + 2 * i + half;
+      kk = kk < K ? kk : K - 1; // (the product is dropped below)
+      wv[b][i] = *reinterpret_cast<const float4 *>(w + (long long)kk * N);
+    }
+  };
+  load_w(0, k0);
+  if constexpr (TERMINAL) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    int rows = 0;
+    bool more = true;
+    for (int p0 = 0; p0 < S && more; p0 += RULES) { // (added in rule order, up to the first negative one)
+      if (p0)
+        load_rules(p0);
+      float4 x[RULES];
+#pragma unroll
+      for (int u = 0; u < RULES; ++u) {
+        more = more && rule[u] >= 0;
+        if (more && k < K)
+          x[u] = *reinterpret_cast<const float4 *>(A + (long long)rule[u] * K + k);
+      }
+      bool on = true;
+#pragma unroll
+      for (int u = 0; u < RULES; ++u) {
+        on = on && rule[u] >= 0;
+        if (on) {
+          v.x += x[u].x, v.y += x[u].y, v.z += x[u].z, v.w += x[u].w;
+          ++rows;
+        }
+      }
+    }
+    const float count = (float)rows;
+    const float4 mean = make_float4(v.x / count, v.y / count, v.z / count, v.w / count);
+    if (k < K) {
+      if (mRow < M)
+        *reinterpret_cast<float4 *>(ts.pooled + mRow * K + k) = mean;
+      *reinterpret_cast<float4 *>(&sA[row][k]) = mRow < M ? mean : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  } else if (k < K) {
+    *reinterpret_cast<float4 *>(&sA[row][k]) =
+        mRow < M ? *reinterpret_cast<const float4 *>(A + mRow * K + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __syncthreads();
+  float4 acc[CL_ROWS];
+#pragma unroll
+  for (int r = 0; r < CL_ROWS; ++r)
+    acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto multiply = [&](int b, int from) {
+#pragma unroll
+    for (int i = 0; i < CL_DEPTH; ++i)
+      if (from + 2 * i + half < k1) {
+#pragma unroll
+        for (int r = 0; r < CL_ROWS; ++r) {
+          const float a = sA[r][from + 2 * i + half];
+          acc[r].x = fmaf(a, wv[b][i].x, acc[r].x);
+          acc[r].y = fmaf(a, wv[b][i].y, acc[r].y);
+          acc[r].z = fmaf(a, wv[b][i].z, acc[r].z);
+          acc[r].w = fmaf(a, wv[b][i].w, acc[r].w);
+        }
+      }
+  };
+  for (int from = k0; from < k1; from += 4 * CL_DEPTH) {
+    if (from + 2 * CL_DEPTH < k1)
+      load_w(1, from + 2 * CL_DEPTH);
+    multiply(0, from);
+    if (from + 2 * CL_DEPTH >= k1)
+      break;
+    if (from + 4 * CL_DEPTH < k1)
+      load_w(0, from + 4 * CL_DEPTH);
+    multiply(1, from + 2 * CL_DEPTH);
+  }
+#pragma unroll
+  for (int r = 0; r < CL_ROWS; ++r) {
+    acc[r].x += __shfl_xor(acc[r].x, 32, 64);
+    acc[r].y += __shfl_xor(acc[r].y, 32, 64);
+    acc[r].z += __shfl_xor(acc[r].z, 32, 64);
+    acc[r].w += __shfl_xor(acc[r].w, 32, 64);
+    if (half == 0)
+      *reinterpret_cast<float4 *>(&part[wave][r][4 * lane]) = acc[r];
+  }
+  __syncthreads();
+  // the partial sums are always added in wavefront order
+  const long long m = m0 + wave;
+  if (wave >= CL_ROWS || m >= M)
+    return;
+  float z[2], mx = -10000.0f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int c = 64 * j + lane;
+    float v = part[0][wave][c];
+#pragma unroll
+    for (int u = 1; u < FR_WAVES; ++u)
+      v += part[u][wave][c];
+    z[j] = 0.f;
+    if (c < N) {
+      z[j] = apply_act(v, c, ep); // bias and scale; the activation itself is the soft-max below
+      mx = fmaxf(mx, z[j]);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1)
+    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (64 * j + lane < N) {
+      z[j] = expf(z[j] - mx);
+      sum += z[j];
+    }
+  for (int off = 32; off > 0; off >>= 1)
+    sum += __shfl_xor(sum, off, 64);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (64 * j + lane < N) {
+      const float y = z[j] / sum;
+      out[m * N + 64 * j + lane] = y;
+      if (TERMINAL && ts.copy)
+        ts.copy[m * N + 64 * j + lane] = y;
+    }
+}
+
 // ---- few input channels: one lane per four outputs ------------------------
 // The first NiN layer of a net multiplies a tall matrix by a tiny W (K = 3 fs
 // or so): bandwidth only.  W sits in LDS; a lane reads its row of A (16-byte
@@ -1683,7 +1862,11 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
     if (act == SCN_SOFTMAX && N <= 128) {
       // whole rows in one workgroup: the soft-max rides along
       softmaxDone = true;
-      hipLaunchKernelGGL((k_nin_fewrows<2, true>), dim3(scn_ceil_div(M, FR_ROWS), 1),
+      if (vec && !gs)
+        hipLaunchKernelGGL((k_classifier<false>), dim3(scn_ceil_div(M, CL_ROWS)), dim3(FR_THREADS), 0, ctx->stream, d_A,
+                           d_W, d_out, (long long)M, K, N, ep, dRows, TerminalSource());
+      else // (classes or channels in other than fours)
+        hipLaunchKernelGGL((k_nin_fewrows<2, true>), dim3(scn_ceil_div(M, FR_ROWS), 1),
                          dim3(FR_THREADS), 0, ctx->stream, d_A, d_W, d_out,
                          (long long)M, K, N, ep, gs ? *gs : none, gs != nullptr, dRows);
     } else {
@@ -1860,4 +2043,31 @@ extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
   gs.zeros = ctx->d_zeros;
   return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p,
                      act, precision, &gs);
+}
+
+// Where scn_nin_forward takes the classifier to k_classifier
+extern "C" int scn_terminal_classifier_supported(int64_t M, int K, int N) {
+  return M >= 1 && M <= FR_MAX_M && K >= 1 && K <= FR_MAX_K && N >= 1 && N <= 128 && K % 4 == 0 && N % 4 == 0 &&
+         !(N % 16 == 0 && scn_planes_shape(K));
+}
+extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
+                                       float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
+                                       float *copy, int K, int N, float p) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_terminal_classifier: null context");
+  SCN_REQUIRE(S >= 1 && scn_terminal_classifier_supported(M, K, N), SCN_ERR_ARG,
+              "scn_terminal_classifier: M %lld S %d K %d N %d", (long long)M, S, K, N);
+  // (d_in may be null: an input without rows, every rule negative)
+  SCN_REQUIRE(d_rules && d_pooled && d_W && d_B && d_probs, SCN_ERR_ARG, "scn_terminal_classifier: null buffer");
+  SCN_REQUIRE((((uintptr_t)d_in | (uintptr_t)d_W | (uintptr_t)d_pooled) & 15) == 0, SCN_ERR_ARG,
+              "scn_terminal_classifier: matrices start on 16 bytes");
+  Epilogue ep = Epilogue();
+  ep.bias = d_B;
+  ep.p = p;
+  ep.act = SCN_SOFTMAX;
+  ProfScope prof(ctx, SCN_K_NIN);
+  TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy};
+  hipLaunchKernelGGL((k_classifier<true>), dim3(scn_ceil_div(M, CL_ROWS)), dim3(FR_THREADS), 0, ctx->stream, d_in, d_W,
+                     d_probs, (long long)M, K, N, ep, ctx->d_meta ? ctx->d_meta + META_SITES : nullptr, ts);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
 }

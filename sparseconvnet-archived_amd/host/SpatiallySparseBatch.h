@@ -13,6 +13,7 @@
 struct BatchResultStage {
   float *pinned;
   size_t capacity; // floats
+  bool copied; // the forward pass has left the probabilities in `pinned` already
   scn_event *arrived;
   bool pending;
   // a training batch: the point of the net's stream behind the backward pass,

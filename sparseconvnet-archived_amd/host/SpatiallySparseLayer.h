@@ -334,6 +334,16 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
 void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
                               SpatiallySparseBatch &batch, int nTop);
 
+// the last two layers of a test batch's forward pass and that copy in one launch,
+// where they are a terminal pooling and a classifier that it takes
+bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
+                               SpatiallySparseLayer *pooling,
+                               SpatiallySparseLayer *classifier,
+                               SpatiallySparseBatchInterface &input,
+                               SpatiallySparseBatchInterface &middle,
+                               SpatiallySparseBatchInterface &output,
+                               cudaMemStream &ms);
+
 // utilities.h
 int ipow(int base, int exp);
 int triangleSize(int linearSize, int dimension);

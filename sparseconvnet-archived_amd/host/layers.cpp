@@ -980,6 +980,51 @@ int TerminalPoolingLayer::calculateInputSpatialSize(int outputSpatialSize) {
 // In two halves, so that a caller may queue the next batch's forward pass
 // between them: the copy of the probabilities to the host is only queued
 // (SoftmaxClassifier.cu:24, copyToCPUAsync), the statistics are computed once
+// pinned memory for the probabilities of a batch
+static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream) {
+  if (n <= r.capacity)
+    return;
+  if (r.pinned)
+    SCN_CHECKED(scn_host_free(memStream.ctx, r.pinned));
+  r.capacity = n + n / 2;
+  SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
+                             (void **)&r.pinned));
+}
+// A net's end, a terminal pooling and the classifier, in one launch that also
+// leaves the probabilities where the host reads them.  False: not of that kind,
+// nothing done.
+bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
+                               SpatiallySparseLayer *pooling,
+                               SpatiallySparseLayer *classifier,
+                               SpatiallySparseBatchInterface &input,
+                               SpatiallySparseBatchInterface &middle,
+                               SpatiallySparseBatchInterface &output,
+                               cudaMemStream &ms) {
+  auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
+  if (batch.type == TRAINBATCH || batch.type == RESCALEBATCH || !n ||
+      n->fn != SOFTMAX ||
+      !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
+      middle.nSpatialSites != batch.batchSize ||
+      !scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn,
+                                         n->nFeaturesOut))
+    return false;
+  const size_t K = n->nFeaturesIn, N = n->nFeaturesOut, M = batch.batchSize;
+  output.sub->reset();
+  middle.sub->poolingChoices.resize64(M * K, kBoundRows * K);
+  middle.sub->features.resize64(M * K, kBoundRows * K);
+  output.sub->features.resize64(M * N, kBoundRows * N);
+  result_room(*batch.result, M * N, ms);
+  SCN_CHECKED(scn_terminal_classifier(
+      ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
+      (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
+      n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
+      (int)N, 1.0f - n->dropout));
+  batch.result->copied = true;
+  if (!batch.countsPending) // (else counted when they are settled)
+    addMultiplyAdds((__int128_t)M * K * N);
+  return true;
+}
+
 // it has arrived (:27 onwards).
 void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
                              SpatiallySparseBatch &batch,
@@ -1002,18 +1047,14 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
   }
   BatchResultStage &r = *batch.result;
   const size_t n = (size_t)batch.batchSize * input.nFeatures;
-  if (n > r.capacity) {
-    if (r.pinned)
-      SCN_CHECKED(scn_host_free(memStream.ctx, r.pinned));
-    r.capacity = n + n / 2;
-    SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
-                               (void **)&r.pinned));
-  }
+  result_room(r, n, memStream);
   if (!r.arrived)
     SCN_CHECKED(scn_event_create(memStream.ctx, &r.arrived));
   // a kernel copies what a batch usually has: queueing it takes the host a
   // fifth of the time of an asynchronous memcpy
-  if (n <= ((size_t)1 << 18))
+  if (r.copied)
+    r.copied = false;
+  else if (n <= ((size_t)1 << 18))
     SCN_CHECKED(scn_copy(memStream.ctx, r.pinned, input.sub->features.dPtr(),
                          n * sizeof(float)));
   else

@@ -492,11 +492,17 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   // a RESCALEBATCH rescales every layer's weights right after its forward
   // pass (SparseConvNetCUDA.cu:230-241)
   float scalingUnderneath = 1;
+  batch.result->copied = false;
   for (size_t i = 0; i < layers.size(); i++) {
     batch.interfaces[i + 1].sub->reset();
     scn_prof_tag(ms.ctx, (int)i);
     if (batch.countsPending)
       SCN_CHECKED(scn_ctx_rows_from(ms.ctx, batch.interfaces[i + 1].deviceGrids));
+    if (i + 2 == layers.size() &&
+        forwardTerminalClassifier(batch, layers[i], layers[i + 1],
+                                  batch.interfaces[i], batch.interfaces[i + 1],
+                                  batch.interfaces[i + 2], ms))
+      break;
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);
     if (batch.type == RESCALEBATCH) {
       std::cout << i << ":"
