@@ -401,7 +401,7 @@ int scn_nag_update(scn_ctx *ctx, const float *d_delta, float *d_momentum,
  * NetworkInNetworkLayer.cu:274-287, NetworkInNetworkPReLULayer.cu:211-214 and
  * :262-275).  With clearGradients the gradients are left zero, which is what
  * the accumulating products below expect of the next batch. */
-#define SCN_NAG_MAX 4
+#define SCN_NAG_MAX 48
 typedef struct scn_nag_item {
   float *d_delta;
   float *d_momentum;
@@ -420,6 +420,16 @@ int scn_activation_backward_acc(scn_ctx *ctx, const float *d_out,
                                 float *d_delta, int64_t M, int N, int act,
                                 const float *d_prelu, float *d_db,
                                 float *d_dprelu);
+/* The same with the product in a buffer of its own, d_dst, and d_delta left as
+ * it is (accumulate: as _acc).  With a max-pooling behind the layer: an output of
+ * the pooling is the activation it chose, so the derivative can be taken, and the
+ * bias gradient summed, over the pooling's outputs (d_out and d_delta those of the
+ * pooling, M its rows), of which there are fewer, before scn_maxpool_backward
+ * spreads d_dst. */
+int scn_activation_backward_to(scn_ctx *ctx, const float *d_out,
+                               const float *d_delta, float *d_dst, int64_t M,
+                               int N, int act, const float *d_prelu,
+                               float *d_db, float *d_dprelu, int accumulate);
 int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
                       float *d_dW, int64_t M, int K, int N);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout

@@ -29,7 +29,7 @@ class ScnError(RuntimeError):
     pass
 
 
-NAG_MAX = 4
+NAG_MAX = 48
 
 
 class NagItem(C.Structure):
@@ -135,6 +135,7 @@ def lib():
         "scn_nag_update": (C.c_int, [vp, vp, vp, vp, i64, f32, f32, C.c_int]),
         "scn_nag_update_many": (C.c_int, [vp, P(NagItem), C.c_int, f32, f32, C.c_int]),
         "scn_activation_backward_acc": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),
+        "scn_activation_backward_to": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp, C.c_int]),
         "scn_sgemm_AtB_acc": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
         "scn_shrink_matrix": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int]),
         "scn_nag_update_shrunk": (C.c_int, [vp, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, f32, f32]),
@@ -329,6 +330,11 @@ class Context:
         _check(f(self.h, d_out.ptr, d_delta.ptr, M, N, act,
                  d_prelu.ptr if d_prelu is not None else None, d_db.ptr,
                  d_dprelu.ptr if d_dprelu is not None else None))
+
+    def activation_backward_to(self, d_out, d_delta, d_dst, M, N, act, d_prelu, d_db, d_dprelu, accumulate=False):
+        _check(lib().scn_activation_backward_to(self.h, d_out.ptr, d_delta.ptr, d_dst.ptr, M, N, act,
+                                                d_prelu.ptr if d_prelu is not None else None, d_db.ptr,
+                                                d_dprelu.ptr if d_dprelu is not None else None, int(accumulate)))
 
     def sgemm_AtB(self, d_A, d_D, d_dW, M, K, N, accumulate=False):
         f = lib().scn_sgemm_AtB_acc if accumulate else lib().scn_sgemm_AtB

@@ -76,7 +76,7 @@ __device__ __forceinline__ float act_derivative(int act, float b, float d,
 #define ACTB_THREADS 512
 template <int V>
 __global__ __launch_bounds__(ACTB_THREADS) void k_act_backward(
-    const float *__restrict__ out, float *__restrict__ delta, long long M,
+    const float *__restrict__ out, const float *delta, float *dst, long long M,
     int N, int act, const float *__restrict__ prelu, float *__restrict__ db,
     float *__restrict__ dprelu, int P) {
   typedef float vec __attribute__((ext_vector_type(V)));
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(ACTB_THREADS) void k_act_backward(
           d[u][i] = act_derivative(act, b[u][i], d[u][i], alpha[i], t[i]);
           s[i] += d[u][i];
         }
-        *reinterpret_cast<vec *>(delta + (r + u * step) * N + c) = d[u];
+        *reinterpret_cast<vec *>(dst + (r + u * step) * N + c) = d[u];
       }
     }
     for (; r < M; r += step) {
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(ACTB_THREADS) void k_act_backward(
         d[i] = act_derivative(act, b[i], d[i], alpha[i], t[i]);
         s[i] += d[i];
       }
-      *reinterpret_cast<vec *>(delta + r * N + c) = d;
+      *reinterpret_cast<vec *>(dst + r * N + c) = d;
     }
   }
 #pragma unroll
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(ACTB_THREADS) void k_act_backward(
 }
 
 static int activation_backward(scn_ctx *ctx, const float *d_out,
-                               float *d_delta, int64_t M, int N, int act,
+                               const float *d_delta, float *d_dst, int64_t M, int N, int act,
                                const float *d_prelu, float *d_db,
                                float *d_dprelu, bool clear) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_activation_backward: null context");
@@ -166,9 +166,9 @@ static int activation_backward(scn_ctx *ctx, const float *d_out,
   }
   if (M == 0)
     return SCN_OK;
-  SCN_REQUIRE(d_out && d_delta, SCN_ERR_ARG,
+  SCN_REQUIRE(d_out && d_delta && d_dst, SCN_ERR_ARG,
               "scn_activation_backward: null buffer");
-  const int V = N % 4 == 0 && (((uintptr_t)d_out | (uintptr_t)d_delta) & 15) == 0 ? 4 : 1;
+  const int V = N % 4 == 0 && (((uintptr_t)d_out | (uintptr_t)d_delta | (uintptr_t)d_dst) & 15) == 0 ? 4 : 1;
   // (a row of up to 64 lanes: with fewer rows of lanes the sums below are short)
   const int colBlocks = scn_ceil_div(N, V * 64);
   const int P = scn_ceil_div(N / V, colBlocks);
@@ -181,7 +181,7 @@ static int activation_backward(scn_ctx *ctx, const float *d_out,
   if (rowBlocks > cap)
     rowBlocks = cap;
   hipLaunchKernelGGL((V == 4 ? k_act_backward<4> : k_act_backward<1>), dim3(colBlocks, rowBlocks),
-                     dim3(ACTB_THREADS), 0, ctx->stream, d_out, d_delta, (long long)M, N, act,
+                     dim3(ACTB_THREADS), 0, ctx->stream, d_out, d_delta, d_dst, (long long)M, N, act,
                      d_prelu, d_db, d_dprelu, P);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
@@ -191,16 +191,24 @@ extern "C" int scn_activation_backward(scn_ctx *ctx, const float *d_out,
                                        float *d_delta, int64_t M, int N,
                                        int act, const float *d_prelu,
                                        float *d_db, float *d_dprelu) {
-  return activation_backward(ctx, d_out, d_delta, M, N, act, d_prelu, d_db,
-                             d_dprelu, true);
+  return activation_backward(ctx, d_out, d_delta, d_delta, M, N, act, d_prelu,
+                             d_db, d_dprelu, true);
 }
 
 extern "C" int scn_activation_backward_acc(scn_ctx *ctx, const float *d_out,
                                            float *d_delta, int64_t M, int N,
                                            int act, const float *d_prelu,
                                            float *d_db, float *d_dprelu) {
-  return activation_backward(ctx, d_out, d_delta, M, N, act, d_prelu, d_db,
-                             d_dprelu, false);
+  return activation_backward(ctx, d_out, d_delta, d_delta, M, N, act, d_prelu,
+                             d_db, d_dprelu, false);
+}
+extern "C" int scn_activation_backward_to(scn_ctx *ctx, const float *d_out,
+                                          const float *d_delta, float *d_dst,
+                                          int64_t M, int N, int act,
+                                          const float *d_prelu, float *d_db,
+                                          float *d_dprelu, int accumulate) {
+  return activation_backward(ctx, d_out, d_delta, d_dst, M, N, act, d_prelu,
+                             d_db, d_dprelu, !accumulate);
 }
 
 // ---------------------------------------------- dW = A^T D (scn_planes.hip)
@@ -431,8 +439,9 @@ extern "C" int scn_nag_update(scn_ctx *ctx, const float *d_delta,
   return SCN_OK;
 }
 
-// The momentum step of several tensors (a layer's W, B and PReLU slopes) in
-// one launch: a workgroup finds its tensor from the running workgroup counts.
+// The momentum step of several tensors (all layers' W, B and PReLU slopes) in
+// one launch: a workgroup finds its tensor from the running workgroup counts (a
+// lane a count: a walk over them in the arguments is a trip a cache line).
 // With `clear` the gradient is left zero, so the next batch's accumulating
 // products need no clearing launch.
 struct NagList {
@@ -447,9 +456,9 @@ struct NagList {
 
 __global__ __launch_bounds__(256) void k_nag_update_many(NagList l, float lr,
                                                          float mu, int clear) {
-  int t = 0;
-  while (t + 1 < l.count && blockIdx.x >= l.firstBlock[t + 1])
-    ++t;
+  static_assert(SCN_NAG_MAX <= 64, "a lane an item");
+  const int lane = threadIdx.x & 63;
+  const int t = __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_NAG_MAX ? lane : 0])) - 1;
   const long long i =
       (long long)(blockIdx.x - l.firstBlock[t]) * blockDim.x + threadIdx.x;
   if (i >= l.n[t])

@@ -83,5 +83,9 @@ public:
   PinnedStage hostFeatures;
   size_t hostFeatureCount;
   std::unique_ptr<BatchResultStage> result;
+  // SparseConvNetCUDA::backwardBatch: the layers' momentum steps, put off to the
+  // end of the backward pass and queued together (elsewhere every layer queues its own)
+  std::vector<scn_nag_item> updates;
+  bool collectUpdates = false;
   void reset();
 };

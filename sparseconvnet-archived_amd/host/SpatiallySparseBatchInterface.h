@@ -10,6 +10,7 @@ class SpatiallySparseBatchSubInterface {
 public:
   vectorCUDA<float> features;
   vectorCUDA<float> dfeatures; // gradient of the cost, training batches only
+  vectorCUDA<float> dactivated; // of a pooling's output: that, times the derivative of the layer below
   vectorCUDA<int> poolingChoices;
   // room for a bf16 copy of `features` (two bytes an element), made by a
   // following fused convolution with bf16 operands whose window is large
@@ -30,6 +31,10 @@ public:
   // sub->dfeatures has been cleared for the layer that adds to it next
   // (SparseConvNetCUDA::backwardBatch clears those of a whole pass at once)
   bool gradientCleared = false;
+  // a layer's output: the activation's derivative is in dfeatures already (taken
+  // over the outputs of the pooling behind it); a pooling's: sub->dactivated holds
+  // what it is to spread
+  bool activationDone = false, activationAhead = false;
   // Host view of the sparse grids.  Filled by the Pictures for the input
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().

@@ -39,6 +39,18 @@ public:
   virtual int calculateInputSpatialSize(int outputSpatialSize) = 0;
   // backwards() adds to the input's gradient (and does not assign it)
   virtual bool addsInputGradient() const { return false; }
+  // every output is one of its inputs, and backwards() adds the output's gradient
+  // (or sub->dactivated in its place) to that input's
+  virtual bool choosesInputs() const { return false; }
+  // The derivative of this layer's activation (and the sums that go with it) over
+  // the outputs of a pooling that chooses from this layer's: `pooled` gets what the
+  // pooling is to spread.  Nothing, where the layer has to do that itself.
+  virtual void activationAhead(SpatiallySparseBatch &batch,
+                               SpatiallySparseBatchInterface &input,
+                               SpatiallySparseBatchInterface &output,
+                               SpatiallySparseBatchInterface &pooled) {
+    (void)batch, (void)input, (void)output, (void)pooled;
+  }
 };
 
 // ConvolutionalLayer.h:3-33 -- gathers each output site's receptive field
@@ -115,7 +127,7 @@ private:
   RNG rng;
   std::mutex rngMutex; // preprocess() runs on several producer threads
   vectorCUDA<float> dw, db, workspace; // gradients; W transposed for dA
-  bool gradsClean = false; // dw and db hold zeros (the momentum step left them so)
+  bool gradsClean = false; // dw and db hold zeros (the momentum step leaves them so)
   vectorCUDA<float> w, b; // sub-matrix of a training batch with dropout
 
 public:
@@ -146,6 +158,10 @@ public:
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
                  float momentum);
+  void activationAhead(SpatiallySparseBatch &batch,
+                       SpatiallySparseBatchInterface &input,
+                       SpatiallySparseBatchInterface &output,
+                       SpatiallySparseBatchInterface &pooled);
   int calculateInputSpatialSize(int outputSpatialSize);
 };
 
@@ -187,6 +203,10 @@ public:
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
                  float momentum);
+  void activationAhead(SpatiallySparseBatch &batch,
+                       SpatiallySparseBatchInterface &input,
+                       SpatiallySparseBatchInterface &output,
+                       SpatiallySparseBatchInterface &pooled);
   int calculateInputSpatialSize(int outputSpatialSize);
 };
 
@@ -208,6 +228,7 @@ public:
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
   bool addsInputGradient() const { return true; }
+  bool choosesInputs() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -233,6 +254,7 @@ public:
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
   bool addsInputGradient() const { return true; }
+  bool choosesInputs() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -275,6 +297,7 @@ public:
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
   bool addsInputGradient() const { return true; }
+  bool choosesInputs() const { return true; }
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,

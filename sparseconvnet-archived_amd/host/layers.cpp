@@ -362,7 +362,44 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
 // leaves the gradients zero (gradsClean), so the next batch's products add to
 // them without clearing launches of their own; the reference updates the
 // slopes before the products, which nothing after that point reads.
+//
+// The gradients' buffers for a matrix of K x N; whether they hold zeros
+static bool nin_gradients(vectorCUDA<float> &dw, vectorCUDA<float> &db,
+                          vectorCUDA<float> *dprelu, int K, int N,
+                          bool &gradsClean) {
+  gradsClean = gradsClean && dw.size64() == (size_t)K * N &&
+               db.size64() == (size_t)N &&
+               (!dprelu || dprelu->size64() == (size_t)N);
+  dw.resize64((size_t)K * N);
+  db.resize64((size_t)N);
+  if (dprelu)
+    dprelu->resize64((size_t)N);
+  return gradsClean;
+}
+static void nin_activation_ahead(cudaMemStream &ms,
+                                 SpatiallySparseBatchInterface &input,
+                                 SpatiallySparseBatchInterface &output,
+                                 SpatiallySparseBatchInterface &pooled, int act,
+                                 vectorCUDA<float> *PReLU, vectorCUDA<float> &dw,
+                                 vectorCUDA<float> &db, vectorCUDA<float> *dprelu,
+                                 bool &gradsClean) {
+  const int K = (int)input.featuresPresent.size();
+  const int N = (int)output.featuresPresent.size();
+  if (!output.backpropErrors || (int)pooled.featuresPresent.size() != N ||
+      pooled.sub->features.size64() != (size_t)pooled.nSpatialSites * N)
+    return;
+  const bool clean = nin_gradients(dw, db, dprelu, K, N, gradsClean);
+  pooled.sub->dactivated.resize64((size_t)pooled.nSpatialSites * N);
+  SCN_CHECKED(scn_activation_backward_to(
+      ms.ctx, pooled.sub->features.dPtr(), pooled.sub->dfeatures.dPtr(),
+      pooled.sub->dactivated.dPtr(), pooled.nSpatialSites, N, act,
+      PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
+      dprelu ? dprelu->dPtr() : nullptr, clean));
+  pooled.activationAhead = true;
+  output.activationDone = true;
+}
 static void nin_backwards(cudaMemStream &ms,
+                          std::vector<scn_nag_item> *updates,
                           SpatiallySparseBatchInterface &input,
                           SpatiallySparseBatchInterface &output, int nFeaturesIn,
                           int nFeaturesOut, vectorCUDA<float> *shrunkW,
@@ -378,18 +415,14 @@ static void nin_backwards(cudaMemStream &ms,
   const int64_t M = output.nSpatialSites;
   const int K = (int)input.featuresPresent.size();
   const int N = (int)output.featuresPresent.size();
-  const bool clean = gradsClean && dw.size64() == (size_t)K * N &&
-                     db.size64() == (size_t)N &&
-                     (!dprelu || dprelu->size64() == (size_t)N);
+  const bool clean = nin_gradients(dw, db, dprelu, K, N, gradsClean);
   gradsClean = false;
-  dw.resize64((size_t)K * N);
-  db.resize64((size_t)N);
-  if (dprelu)
-    dprelu->resize64((size_t)N);
-  SCN_CHECKED((clean ? scn_activation_backward_acc : scn_activation_backward)(
-      ms.ctx, output.sub->features.dPtr(), output.sub->dfeatures.dPtr(), M, N,
-      act, PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
-      dprelu ? dprelu->dPtr() : nullptr));
+  if (!output.activationDone)
+    SCN_CHECKED((clean ? scn_activation_backward_acc : scn_activation_backward)(
+        ms.ctx, output.sub->features.dPtr(), output.sub->dfeatures.dPtr(), M, N,
+        act, PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
+        dprelu ? dprelu->dPtr() : nullptr));
+  output.activationDone = false;
   SCN_CHECKED((clean ? scn_sgemm_AtB_acc : scn_sgemm_AtB)(
       ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(),
       dw.dPtr(), M, K, N));
@@ -422,8 +455,11 @@ static void nin_backwards(cudaMemStream &ms,
       items[n++] = {dprelu->dPtr(), MPReLU->dPtr(), PReLU->dPtr(), N, 1};
     items[n++] = {dw.dPtr(), MW.dPtr(), W.dPtr(), (int64_t)K * N, 0};
     items[n++] = {db.dPtr(), MB.dPtr(), B.dPtr(), N, 0};
-    SCN_CHECKED(
-        scn_nag_update_many(ms.ctx, items, n, learningRate, momentum, 1));
+    if (updates)
+      updates->insert(updates->end(), items, items + n);
+    else
+      SCN_CHECKED(
+          scn_nag_update_many(ms.ctx, items, n, learningRate, momentum, 1));
     gradsClean = true;
   }
   (void)nFeaturesIn;
@@ -491,12 +527,20 @@ void NetworkInNetworkLayer::backwards(SpatiallySparseBatch &batch,
                                       SpatiallySparseBatchInterface &input,
                                       SpatiallySparseBatchInterface &output,
                                       float learningRate, float momentum) {
-  nin_backwards(memStream, input, output, nFeaturesIn, nFeaturesOut,
+  nin_backwards(memStream, batch.collectUpdates ? &batch.updates : nullptr,
+                input, output, nFeaturesIn, nFeaturesOut,
                 nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output)
                     ? &w
                     : nullptr,
                 (int)fn, W, MW, B, MB, nullptr, nullptr, dw, db, nullptr,
                 workspace, gradsClean, learningRate, momentum);
+}
+void NetworkInNetworkLayer::activationAhead(
+    SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+    SpatiallySparseBatchInterface &output, SpatiallySparseBatchInterface &pooled) {
+  if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    nin_activation_ahead(memStream, input, output, pooled, (int)fn, nullptr, dw,
+                         db, nullptr, gradsClean);
 }
 // scaleWeights (NetworkInNetworkLayer.cu:203-218; the PReLU layer's is the
 // same, NetworkInNetworkPReLULayer.cu:175-189): bring the mean magnitude of
@@ -622,12 +666,20 @@ void NetworkInNetworkPReLULayer::forwards(
 void NetworkInNetworkPReLULayer::backwards(
     SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
     SpatiallySparseBatchInterface &output, float learningRate, float momentum) {
-  nin_backwards(memStream, input, output, nFeaturesIn, nFeaturesOut,
+  nin_backwards(memStream, batch.collectUpdates ? &batch.updates : nullptr,
+                input, output, nFeaturesIn, nFeaturesOut,
                 nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output)
                     ? &w
                     : nullptr,
                 (int)PRELU, W, MW, B, MB, &PReLU, &MPReLU, dw, db, &dprelu,
                 workspace, gradsClean, learningRate, momentum);
+}
+void NetworkInNetworkPReLULayer::activationAhead(
+    SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+    SpatiallySparseBatchInterface &output, SpatiallySparseBatchInterface &pooled) {
+  if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    nin_activation_ahead(memStream, input, output, pooled, (int)PRELU, &PReLU,
+                         dw, db, &dprelu, gradsClean);
 }
 void NetworkInNetworkPReLULayer::loadWeightsFromStream(std::ifstream &f,
                                                        bool momentum) {
@@ -706,8 +758,10 @@ static void pool_backwards(cudaMemStream &ms,
     return;
   const size_t nf = output.featuresPresent.size();
   clear_gradient(ms, input, nf);
+  vectorCUDA<float> &d = output.activationAhead ? output.sub->dactivated : output.sub->dfeatures;
+  output.activationAhead = false;
   SCN_CHECKED(scn_maxpool_backward(
-      ms.ctx, input.sub->dfeatures.dPtr(), output.sub->dfeatures.dPtr(),
+      ms.ctx, input.sub->dfeatures.dPtr(), d.dPtr(),
       output.nSpatialSites, (int)nf, output.sub->poolingChoices.dPtr()));
 }
 void MaxPoolingLayer::backwards(SpatiallySparseBatch &batch,

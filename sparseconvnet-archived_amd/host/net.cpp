@@ -462,11 +462,22 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
     grads[n++] = input.sub->dfeatures.dPtr();
   }
   SCN_CHECKED(scn_fill32_many(memStream.ctx, grads, sizes, n, 0u));
+  batch.updates.clear();
+  batch.collectUpdates = true;
   for (int i = (int)layers.size() - 1; i >= 0; i--) {
     scn_prof_tag(memStream.ctx, i);
+    if (i > 0 && layers[i]->choosesInputs())
+      layers[i - 1]->activationAhead(batch, batch.interfaces[i - 1],
+                                     batch.interfaces[i], batch.interfaces[i + 1]);
     layers[i]->backwards(batch, batch.interfaces[i], batch.interfaces[i + 1],
                          learningRate, momentum);
   }
+  batch.collectUpdates = false;
+  for (size_t i = 0; i < batch.updates.size(); i += SCN_NAG_MAX)
+    SCN_CHECKED(scn_nag_update_many(
+        memStream.ctx, batch.updates.data() + i,
+        (int)std::min<size_t>(SCN_NAG_MAX, batch.updates.size() - i),
+        learningRate, momentum, 1));
   // the backward kernels read the slot's rule books and features: the slot
   // stays with the consumer until the stream has passed this point
   BatchResultStage &r = *batch.result;
