@@ -1346,6 +1346,7 @@ static void chain_mark_output(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   out->d = in->d;
   out->n = n;
   out->vol = vol;
+  out->rankStateFor = 0;
   out->nActive = boundActive;
   out->nSites = (int)boundRows;
   out->rankValid = false;

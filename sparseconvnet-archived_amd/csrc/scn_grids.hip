@@ -25,6 +25,7 @@
 //          + #background rows appended for earlier samples,
 // which needs no sort: count owned outputs per input, scatter the counts to
 // iteration order through the rank, prefix-sum, emit.
+#include <algorithm>
 #include "scn_common.h"
 #include <atomic>
 #include "scn_scan_dev.h"
@@ -537,12 +538,13 @@ __device__ __forceinline__ unsigned long long even_bits(unsigned long long x) {
 template <int D, int S>
 __global__ void __launch_bounds__(256)
     k_mask_dilate(GridView in, Geom g, unsigned long long *outBits,
-                  long long nWords, long long totalBits) {
+                  long long nWords, long long totalBits, ScanState rank) {
   // (runs of blocks to one XCD: the rows and planes a word's windows reach into
   // are the ones its neighbours in the same L2 have just read)
   const long long w = xcd_contiguous_block((nWords + 255) / 256) * blockDim.x + threadIdx.x;
   if (w >= nWords)
     return;
+  rank.clear((size_t)w);
   const int size = S ? S : g.size;
   constexpr int UN = S ? S : 1; // (no unrolling of loops whose length is not known here)
   unsigned long long res = 0;
@@ -799,10 +801,12 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// clears a hash table (all-ones = empty slots) and an occupancy mask at once
+// clears a hash table (all-ones = empty slots) and an occupancy mask at once (and
+// the state of the scan for the mask's ranks)
 __global__ void k_clear_grid(uint4 *slots, size_t nSlots,
-                             unsigned long long *bits, size_t nWords) {
+                             unsigned long long *bits, size_t nWords, ScanState rank) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  rank.clear(i);
   size_t step = (size_t)gridDim.x * blockDim.x;
   for (size_t k = i; k < nSlots; k += step)
     slots[k] = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
@@ -1215,8 +1219,7 @@ static long long ipow_ll(long long b, int e) {
 // (re)shape a grids object for `batch` samples of an n^d field holding up to
 // nActive sites; clears the mask, unless the caller writes every word of it
 // (wholeMask), and the hash table when the caller is about to fill it (withTable)
-static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
-                         long long nActive, bool withTable = false, bool wholeMask = false) {
+static int grids_check(int batch, int d, int n) {
   SCN_REQUIRE(batch >= 0 && d >= 1 && d <= 3 && n >= 1, SCN_ERR_ARG,
               "grids: batch %d dimension %d spatialSize %d (dimension must be 1..3)",
               batch, d, n);
@@ -1228,6 +1231,13 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
   // (the rows of a rule-book plan carry their sample above 40 bits of coordinates)
   SCN_REQUIRE(batch < (1 << 22) && (d == 1 || n < (d == 3 ? (1 << 13) : (1 << 20))),
               SCN_ERR_CAPACITY, "grids: %d samples of side %d", batch, n);
+  return SCN_OK;
+}
+static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
+                         long long nActive, bool withTable = false, bool wholeMask = false) {
+  SCN_TRY(grids_check(batch, d, n));
+  const long long vol = ipow_ll(n, d);
+  g->rankStateFor = 0;
   g->batch = batch;
   g->d = d;
   g->n = n;
@@ -1275,9 +1285,18 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
     size_t blocks = (most + 255) / 256;
     if (blocks > 16384)
       blocks = 16384;
+    ScanState rank = {nullptr, 0};
+    if (clearWords) { // (as many lanes as words, or 16384 x 256: more than tiles)
+      SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
+      rank = scn_scan_state(g->nWords + 1, g->scanTmp.p);
+      if (rank.words <= blocks * 256)
+        g->rankStateFor = g->nWords + 1;
+      else
+        rank.words = 0;
+    }
     hipLaunchKernelGGL(k_clear_grid, dim3((unsigned)blocks), dim3(256), 0,
                        ctx->stream, (uint4 *)g->table.p, clearSlots, g->bits.p,
-                       clearWords);
+                       clearWords, rank);
     SCN_HIP_CHECK(hipGetLastError());
   }
   return SCN_OK;
@@ -1403,11 +1422,13 @@ static int ensure_index(scn_ctx *ctx, scn_grids *g) {
 static int ensure_rank(scn_ctx *ctx, scn_grids *g) {
   SCN_TRY(ensure_index(ctx, g));
   if (!g->rankValid) {
+    const bool cleared = g->rankStateFor == g->nWords + 1; // (by the kernel that wrote or cleared the mask)
+    g->rankStateFor = 0;
     SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
     // one word past the mask so that the rank of the end position is defined
     SCN_TRY(scn_scan_exclusive_popc64(ctx->stream,
                                       (const uint64_t *)g->bits.p, g->prefix.p,
-                                      g->nWords + 1, g->scanTmp.p));
+                                      g->nWords + 1, g->scanTmp.p, cleared));
     g->rankValid = true;
   }
   if (!g->rankRowValid) {
@@ -1443,7 +1464,7 @@ int scn_grids_ensure_table(scn_ctx *ctx, scn_grids *g) {
         blocks = 16384;
       hipLaunchKernelGGL(k_clear_grid, dim3((unsigned)blocks), dim3(256), 0,
                          ctx->stream, (uint4 *)g->table.p, cap,
-                         (unsigned long long *)nullptr, (size_t)0);
+                         (unsigned long long *)nullptr, (size_t)0, ScanState{nullptr, 0});
       SCN_HIP_CHECK(hipGetLastError());
     }
     g->cleanSlots = 0;
@@ -1795,7 +1816,13 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   SCN_TRY(out->bgBefore.reserve((size_t)in->batch + 2));
   SCN_TRY(out->sampleStart.reserve((size_t)in->batch + 2));
   SCN_TRY(out->bg.reserve((size_t)in->batch + 1));
-  SCN_TRY(out->scanTmp.reserve(scn_scan_tmp_elems((size_t)nE + 1)));
+  // the output mask: word by word from the input mask where the mode allows
+  // it, else bit by bit as the emit pass finds the sites
+  const bool dilated = g.mode == MODE_SQ_NOMIN && g.size <= 64;
+  const size_t outWords = (size_t)((volOutAll + 63) / 64);
+  SCN_TRY(grids_check(in->batch, g.d, g.nOut));
+  out->rankStateFor = 0;
+  SCN_TRY(out->scanTmp.reserve(scn_scan_tmp_elems(std::max((size_t)nE + 1, dilated ? outWords + 1 : 0))));
   GridView vin = view_of(in);
   // number of candidates of one input: (ceil(size / stride))^d at most
   long long maxCand = 1;
@@ -1856,6 +1883,21 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
                          inMeta, boundRows, boundActive, slot);
   }
   SCN_HIP_CHECK(hipGetLastError());
+  size_t rankStateFor = 0;
+  if (dilated) {
+    // (needs no count: runs while the host waits for them.  It also clears the
+    // state of the scan that gives the mask its ranks)
+    SCN_TRY(out->bits.reserve(outWords + 8)); // the scan reads whole 32-byte groups
+    const long long words = (long long)outWords + 2; // all that grids_prepare would clear
+    const long long blocks = (scn_ceil_div(words, 256) + 7) / 8 * 8; // whole rounds of the 8 XCDs
+    auto dilate = g.size == 2 ? k_mask_dilate<D, 2>
+                              : (g.size == 3 ? k_mask_dilate<D, 3> : k_mask_dilate<D, 0>);
+    hipLaunchKernelGGL(dilate, dim3((unsigned)blocks), dim3(256),
+                       0, ctx->stream, vin, g, out->bits.p, words, volOutAll,
+                       scn_scan_state(outWords + 1, out->scanTmp.p));
+    SCN_HIP_CHECK(hipGetLastError());
+    rankStateFor = outWords + 1;
+  }
   long long nSites = boundRows, nOutActive = boundActive;
   if (!deferred) {
     SCN_TRY(read_scalars(ctx, ticket));
@@ -1868,27 +1910,17 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
               "rules: %lld output rows do not fit 32-bit row numbers", nSites);
   // out->bg already holds what k_plan_samples wrote: grids_prepare only
   // reserves it (no reallocation at the same size) and clears table and mask
-  const bool dilated = g.mode == MODE_SQ_NOMIN && g.size <= 64;
   SCN_TRY(grids_prepare(ctx, out, in->batch, g.d, g.nOut, nOutActive, false, dilated));
+  if (dilated)
+    out->rankStateFor = rankStateFor;
   out->nSites = (int)nSites;
   if (deferred)
     mark_pending(ctx, out, slot);
   SCN_TRY(out->siteKey.reserve((size_t)nSites + 1));
   long long nThreads = nE > in->batch ? nE : in->batch;
-  // the output mask: word by word from the input mask where the mode allows
-  // it, else bit by bit as the emit pass finds the sites
   GridView vout = view_of(out);
-  if (dilated) {
-    const long long words = (long long)out->nWords + 2; // all that grids_prepare would clear
-    const long long blocks = (scn_ceil_div(words, 256) + 7) / 8 * 8; // whole rounds of the 8 XCDs
-    auto dilate = g.size == 2 ? k_mask_dilate<D, 2>
-                              : (g.size == 3 ? k_mask_dilate<D, 3> : k_mask_dilate<D, 0>);
-    hipLaunchKernelGGL(dilate, dim3((unsigned)blocks), dim3(256),
-                       0, ctx->stream, vin, g, out->bits.p, words,
-                       (long long)in->batch * g.volOut);
-    SCN_HIP_CHECK(hipGetLastError());
+  if (dilated)
     vout.bits = nullptr;
-  }
   if (tiled) {
     const long long lanes = ownWords > in->batch ? ownWords : in->batch;
     hipLaunchKernelGGL(k_tile2_emit<D>, dim3(xcd_grid(scn_ceil_div(lanes, 256))), dim3(256),

@@ -130,6 +130,7 @@ struct scn_grids {
   DevBuf<int> erow;
   DevBuf<int> bg;
   DevBuf<unsigned> scanTmp;
+  size_t rankStateFor = 0; // a scan of that many elements finds its state in scanTmp clear
   // state of the plan that produced this object
   int planKind = PLAN_NONE;
   const scn_grids *planIn = nullptr;
