@@ -152,6 +152,14 @@ int scn_grids_build(scn_ctx *ctx, scn_grids *grids, int batch, int dimension,
                     int spatialSize, const int32_t *d_sample,
                     const int64_t *d_key, const int32_t *d_row, int64_t n,
                     const int32_t *d_background, int32_t nSpatialSites);
+/* The same, and a copy of `bytes` from src to dst (device or pinned host memory,
+ * not overlapping) in the same launch: a batch's features beside its sites. */
+int scn_grids_build_copy(scn_ctx *ctx, scn_grids *grids, int batch,
+                         int dimension, int spatialSize,
+                         const int32_t *d_sample, const int64_t *d_key,
+                         const int32_t *d_row, int64_t nActive,
+                         const int32_t *d_background, int32_t nSpatialSites,
+                         void *dst, const void *src, size_t bytes);
 int scn_grids_info(const scn_grids *grids, int *batch, int *dimension,
                    int *spatialSize, int64_t *nActive, int32_t *nSpatialSites);
 /* Every entry in map iteration order (sample, then ascending key), and

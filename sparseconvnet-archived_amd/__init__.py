@@ -101,6 +101,8 @@ def lib():
         "scn_ctx_rows_held": (C.c_int, [vp, P(C.c_int)]),
         "scn_grids_destroy": (C.c_int, [vp, vp]),
         "scn_grids_build": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_int, vp, vp, vp, i64, vp, i32]),
+        "scn_grids_build_copy": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_int, vp, vp, vp, i64, vp, i32, vp, vp,
+                                           C.c_size_t]),
         "scn_grids_info": (C.c_int, [vp, P(C.c_int), P(C.c_int), P(C.c_int), P(i64), P(i32)]),
         "scn_grids_download": (C.c_int, [vp, vp, vp, vp, vp, vp]),
         "scn_grids_find": (C.c_int, [vp, vp, vp, vp, i64, vp]),

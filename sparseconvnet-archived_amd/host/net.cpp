@@ -409,18 +409,16 @@ void SparseConvNetCUDA::preprocessResident(int cc, const ResidentBatch &input,
     d_key = (const int64_t *)b.stagingKey.dPtr();
     d_row = b.stagingRow.dPtr();
   }
-  SCN_CHECKED(scn_grids_build(ctx, in.deviceGrids, input.batchSize, dimension,
-                              in.spatialSize, d_sample, d_key, d_row,
-                              input.nActive, d_background,
-                              input.nSpatialSites));
   in.sub->features.copyToGPU();
   in.sub->features.resize64(nElems);
+  SCN_CHECKED(scn_grids_build_copy(
+      ctx, in.deviceGrids, input.batchSize, dimension, in.spatialSize, d_sample,
+      d_key, d_row, input.nActive, d_background, input.nSpatialSites,
+      in.sub->features.dPtr(), input.d_features,
+      byCopyEngine ? 0 : nElems * sizeof(float)));
   if (byCopyEngine)
     SCN_CHECKED(scn_h2d_async(ctx, in.sub->features.dPtr(), input.d_features,
                               nElems * sizeof(float)));
-  else
-    SCN_CHECKED(scn_copy(ctx, in.sub->features.dPtr(), input.d_features,
-                         nElems * sizeof(float)));
   buildRuleBooks(*this, ctx, b, mayRunAhead);
   if (!b.countsPending)
     SCN_CHECKED(scn_sync(ctx));
