@@ -132,13 +132,28 @@ __device__ __forceinline__ floatx16 tile_f32(const float *A, const GatherSource 
   return sum;
 }
 
-// A workgroup of four wavefronts owns 128 MT rows x 32 NT columns, a wavefront
-// 32 MT rows of them, and walks k in blocks of 32, two MFMA steps.
-// W passes through two LDS buffers, a block each, split into planes on the way
-// in and laid out as the MFMA reads it, [plane][16 k][tile][lane]: every
-// operand read is a contiguous kilobyte.  A goes from global memory (GATHER:
-// through the rules of the workgroup's rows, staged in LDS) straight into
-// registers, PD blocks ahead as W does, and is split there.
+enum { W_PLAIN, W_IMAGE, W_STREAM }; // how W comes: see k_nin_planes
+// Of the loads a wavefront has asked for, all but the last N have landed, and its
+// LDS reads too: what another wavefront asks for next may take their place.
+template <int N> __device__ __forceinline__ void w_landed() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N < 63 ? N : 63) : "memory");
+}
+// A barrier for LDS accesses; loads under way stay so.
+__device__ __forceinline__ void barrier_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A workgroup of WAVES wavefronts owns 32 WAVES MT rows x 32 NT columns, a
+// wavefront 32 MT rows of them, and walks k in blocks of 32, two MFMA steps.
+// W passes through LDS buffers, a block each, split into planes on the way in
+// (W_PLAIN) or copied from an image of it, through registers (W_IMAGE) or without
+// a stop there (W_STREAM: three buffers, filled two blocks ahead), and laid out
+// as the MFMA reads it, [plane][16 k][tile][lane]: every operand read is a
+// contiguous kilobyte.  A goes from global memory (GATHER: through the rules of
+// the workgroup's rows, staged in LDS) straight into registers, PD blocks ahead
+// as W does, and is split there.
 // Lane (c, q) supplies k = 8 q .. 8 q + 7 of a step's sixteen for row c of A
 // and for its columns of W; it owns the NT adjacent columns NT c .. NT c + NT -
 // 1 (tile j of the MFMA = columns {NT c + j}).
@@ -155,22 +170,24 @@ __device__ __forceinline__ floatx16 tile_f32(const float *A, const GatherSource 
 // K is a multiple of 32.  GATHER 1: so are a gathered row's channels, and a
 // block lies within one filter position; GATHER 2: they are a multiple of 4 and
 // every four of them are looked up.  A16: the rows are bf16 already.
-template <int PL, int MT, int NT, int PD, int GATHER, bool A16, bool IMG>
-__global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 : 4)
+template <int PL, int MT, int NT, int PD, int GATHER, bool A16, int WM, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 : 4)
     k_nin_planes(const float *__restrict__ A, const float *__restrict__ W,
                  float *__restrict__ out, long long M, int K, int N,
                  Epilogue ep, GatherSource gs, int nSplits, RowRange rows, PlainW plain) {
   M = rows.live(M);
-  if ((long long)(blockIdx.x / nSplits) * (128 * MT) >= M)
+  if ((long long)(blockIdx.x / nSplits) * (32 * WAVES * MT) >= M)
     return;
   constexpr int ES = A16 ? 2 : 4;
-  constexpr int WAVES = 4, THREADS = 64 * WAVES;
+  constexpr int THREADS = 64 * WAVES;
   constexpr int ROWS = 32 * MT * WAVES, NW = 32 * NT;
   constexpr int STEP_BYTES = NT * 1024;       // one plane of 16 k
   constexpr int PLANE_BYTES = 2 * STEP_BYTES; // ... of a block
   constexpr int BUF_BYTES = PL * PLANE_BYTES;
+  constexpr bool STREAM = WM == W_STREAM;
+  constexpr int BUFS = STREAM ? 3 : 2;
   constexpr int UNITS = 2 * MT; // of a block: (step, row tile)
-  extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [2][BUF_BYTES], then the rules
+  extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [BUFS][BUF_BYTES], then the rules
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
@@ -180,13 +197,14 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
   const int n0 = split * NW;
   const int T = K / 32;
 
-  // ---- W.  One item = 8 consecutive k of one column; IMG: 16 bytes of the image
+  // ---- W.  One item = 8 consecutive k of one column, or 16 bytes of the image
+  constexpr bool IMG = WM == W_IMAGE;
   constexpr int ITEMS = IMG ? BUF_BYTES / 16 : 4 * NW;
-  constexpr int WPER = (ITEMS + THREADS - 1) / THREADS;
+  constexpr int WPER = STREAM ? 0 : (ITEMS + THREADS - 1) / THREADS;
   constexpr int WREGS = IMG ? 4 : 8;
-  float wv[PD][WPER][WREGS];
-  int wDst[WPER];
-  const float *wSrc[WPER];
+  float wv[PD][WPER + 1][WREGS];
+  int wDst[WPER + 1];
+  const float *wSrc[WPER + 1];
 #pragma unroll
   for (int u = 0; u < WPER; ++u) {
     int x = tid + THREADS * u;
@@ -235,9 +253,37 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
     }
   };
 
+  // W_STREAM: a block of the image goes straight into LDS, a kilobyte an instruction,
+  // each wavefront every WAVES-th of them.  (The compiler does not know of these
+  // loads: what it waits for of its own, the loads being counted in order, it
+  // waits a little longer for.)
+  constexpr int CHUNKS = BUF_BYTES / 1024;
+  const unsigned char *const image =
+      reinterpret_cast<const unsigned char *>(W) + (long long)split * T * BUF_BYTES + 16 * lane;
+  const int wave0 = __builtin_amdgcn_readfirstlane(wave);
+  const unsigned ldsW = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)sW;
+  auto w_fetch = [&](int t, int buf) {
+    if constexpr (STREAM) {
+      t = t < T ? t : T - 1; // (past the last block: that one again, where nobody reads)
+      const unsigned char *const src = image + (long long)t * BUF_BYTES;
+#pragma unroll
+      for (int u = 0; u < (CHUNKS + WAVES - 1) / WAVES; ++u) {
+        const int chunk = wave0 + WAVES * u;
+        if ((u + 1) * WAVES <= CHUNKS || chunk < CHUNKS) {
+          const unsigned lds = ldsW + (unsigned)(buf * BUF_BYTES + chunk * 1024);
+          const unsigned char *const from = src + chunk * 1024;
+          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                       :
+                       : "s"(lds), "v"(from)
+                       : "memory", "m0");
+        }
+      }
+    }
+  };
+
   // ---- A
   const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
-  int *const sRules = reinterpret_cast<int *>(sW + 2 * BUF_BYTES);
+  int *const sRules = reinterpret_cast<int *>(sW + BUFS * BUF_BYTES);
   const unsigned char *rowPtr[MT]; // this lane's rows at the filter position of the block to fetch
   int fetchT = 0, f = 0, ch = 0;   // the block to fetch
   auto aim = [&]() {
@@ -274,8 +320,14 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
   };
   bf16x8 ap[2][PL]; // the unit in hand and the next one
   auto a_split = [&](int slot, int u, int dst) {
-    if (A16) {
+    if (A16 && !STREAM) {
       ap[dst][0] = __builtin_bit_cast(bf16x8, raw[slot][u][0]);
+    } else if (A16) {
+      floatx4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) // (a copy that stays one: see the loads)
+        asm("v_mov_b32 %0, %1" : "=v"(x[i]) : "v"(raw[slot][u][0][i]));
+      ap[dst][0] = __builtin_bit_cast(bf16x8, x);
     } else {
       const floatx4 x = raw[slot][u][0], y = raw[slot][u][A16 ? 0 : 1];
       const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
@@ -287,12 +339,21 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
 #pragma unroll
   for (int p = 0; p < PD; ++p)
     w_load(p, p);
+#pragma unroll
+  for (int p = 0; p < (STREAM ? 3 : 0); ++p)
+    w_fetch(p, p);
+  if (STREAM && !GATHER) { // (GATHER: with the rules)
+    w_landed<0>();
+    barrier_lds();
+  }
   if (GATHER) {
     const long long first = wgRow0 * gs.fs, last = M * gs.fs - 1;
     for (int i = tid; i < ROWS * gs.fs; i += THREADS) {
       const long long r = first + i;
       sRules[i] = gs.rules[r < last ? r : last];
     }
+    if (STREAM)
+      w_landed<0>();
     __syncthreads();
     if (GATHER == 1)
       aim();
@@ -313,7 +374,8 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
       a_load(p, u);
   }
   w_store(0, 0);
-  __syncthreads();
+  if (!STREAM)
+    __syncthreads();
 
   constexpr int NACC = PL > 1 ? 2 : 1;
   floatx16 acc[NACC][MT][NT];
@@ -331,6 +393,7 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
   constexpr int BB = NT == 1 ? 2 : 1; // a single tile has no other's MFMAs to be read under
   bf16x8 b[BB][NT][PL];
   int cur = 0;
+  auto other = [&]() { return STREAM ? (cur == 2 ? 0 : cur + 1) : cur ^ 1; };
   auto read_b = [&](int buf, int s, int j) {
 #pragma unroll
     for (int l = 0; l < PL; ++l)
@@ -362,7 +425,9 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr int PRODUCTS = PL * (PL + 1) / 2;
-  auto block = [&](int p, bool firstOfAll) {
+  // (loads of A a block, and image loads that every wavefront makes)
+  constexpr int A_LOADS = UNITS * (A16 ? 1 : 2), W_LOADS = CHUNKS / WAVES;
+  auto block = [&](int p, int t, bool firstOfAll) {
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
       const int s = u / MT, i = u % MT, src = u & 1; // (UNITS is even)
@@ -373,19 +438,38 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
         a_split((p + 1) % PD, 0, src ^ 1);
       if (u == 0) {
         next_block();
-        a_load(p, 0); // (unit 0 was split a unit ago)
+        if (!STREAM)
+          a_load(p, 0); // (unit 0 was split a unit ago)
       }
-      if (u + 1 < UNITS)
+      // (W_STREAM: into registers whose last use lies behind the last unit's
+      // scheduling barrier: were both in one region the load would get others,
+      // copied back at the end of the loop, where the copy waits for a load just
+      // made)
+      if (STREAM)
+        a_load(p, u);
+      else if (u + 1 < UNITS)
         a_load(p, u + 1);
-      else
+      if (u == UNITS - 1)
         w_store((p + 1) % PD, cur ^ 1);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         if (u == UNITS - 1 && j == (NT > 1)) { // before the first read of the next block's W
           if (NT > 1)
             deal(PRODUCTS);
-          __syncthreads();
-          cur ^= 1;
+          if constexpr (STREAM) {
+            // The next block's W was asked for two blocks ago (the first three
+            // blocks' before the loop, and waited for there); since then this
+            // wavefront has asked for two blocks of A, wherever in the loop the
+            // compiler has put those, and one of W, of which a block each may
+            // still be under way.  Behind the barrier nobody reads this block's W
+            // any more: its place takes the third.
+            w_landed<A_LOADS + W_LOADS>();
+            barrier_lds();
+            w_fetch(t + 3, cur);
+          } else {
+            __syncthreads();
+          }
+          cur = other();
         }
         // a tile's W is read as soon as its registers are free
         if (NT == 1) {
@@ -406,9 +490,11 @@ __global__ void __launch_bounds__(256, MT * NT >= 3 ? 2 : MT * NT * PD >= 2 ? 3 
     for (int p = 0; p < PD; ++p)
       if (t + p < T) { // uniform
         w_load(p, t + p + PD);
-        block(p, t + p == 0);
+        block(p, t + p, t + p == 0);
       }
   }
+  if (STREAM)
+    w_landed<0>(); // (before the wavefront gives its LDS back)
 
   // ---- epilogue: register v of a tile is row 8 (v / 4) + 4 q + v % 4
   const int n = n0 + NT * c;
@@ -677,31 +763,37 @@ static bool planes_image(scn_ctx *ctx) {
 constexpr int planes_depth(int PL, int MT, int NT) {
   return PL * MT * NT <= 4 || (PL < 3 && MT == 1) ? 2 : 1;
 }
-template <int PL, int MT, int NT, bool IMG, bool FINE = false>
+// (W_STREAM: gathered rows, with one plane bf16 ones)
+template <int PL, int MT, int NT, int WM, bool FINE = false, int WAVES = 4>
 static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
                          const Epilogue &ep, const GatherSource *gs, bool a16, bool wT,
                          const RowRange &rows) {
   const int nSplits = scn_ceil_div(N, 32 * NT);
-  const size_t lds = (size_t)2 * PL * 2 * NT * 1024 + (gs ? (size_t)128 * MT * gs->fs * 4 : 0);
+  const size_t lds = (size_t)(WM == W_STREAM ? 3 : 2) * PL * 2 * NT * 1024 +
+                     (gs ? (size_t)32 * WAVES * MT * gs->fs * 4 : 0);
   constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     int rc = SCN_OK;
 #define SCN_PLANES_LDS(G, H)                                                   \
   if (hipFuncSetAttribute(                                                     \
-          reinterpret_cast<const void *>(k_nin_planes<PL, MT, NT, PD, G, H, IMG>), \
+          reinterpret_cast<const void *>(k_nin_planes<PL, MT, NT, PD, G, H, WM, WAVES>), \
           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) \
     rc = SCN_ERR_HIP;
-    SCN_PLANES_LDS(0, false) SCN_PLANES_LDS(G, false)
-    if (PL == 1)
+    if constexpr (WM == W_STREAM) {
       SCN_PLANES_LDS(G, PL == 1)
+    } else {
+      SCN_PLANES_LDS(0, false) SCN_PLANES_LDS(G, false)
+      if (PL == 1)
+        SCN_PLANES_LDS(G, PL == 1)
+    }
 #undef SCN_PLANES_LDS
     return rc;
   });
   SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
   const PlainW plain = {W, wT};
-  if (IMG) {
+  if (WM != W_PLAIN) {
     const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;
     if (PL == 3 && wT)
       hipLaunchKernelGGL((k_planes_image<PL, NT, PL == 3>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream,
@@ -711,12 +803,14 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
                          ctx->d_image, K, N, nSplits);
     W = reinterpret_cast<const float *>(ctx->d_image);
   }
-  const dim3 grid((unsigned)(scn_ceil_div(M, 128 * MT) * (long long)nSplits));
+  const dim3 grid((unsigned)(scn_ceil_div(M, 32 * WAVES * MT) * (long long)nSplits));
 #define SCN_PLANES_GO(G, H, src)                                               \
-  hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, IMG>), grid,       \
-                     dim3(256), lds, ctx->stream, A, W, out, M, K, N,   \
+  hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, WM, WAVES>), grid,   \
+                     dim3(64 * WAVES), lds, ctx->stream, A, W, out, M, K, N,   \
                      ep, src, nSplits, rows, plain)
-  if (!gs)
+  if constexpr (WM == W_STREAM)
+    SCN_PLANES_GO(G, PL == 1, *gs);
+  else if (!gs)
     SCN_PLANES_GO(0, false, GatherSource());
   else if (PL == 1 && a16)
     SCN_PLANES_GO(G, PL == 1, *gs);
@@ -850,12 +944,24 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   }
   // (channels in other than 32s, seldom met: one tile)
   if (gs && gs->nIn % 32 != 0)
-    return launch_planes<PL, 1, 2, false, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
+    return launch_planes<PL, 1, 2, W_PLAIN, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
+  // W_STREAM where the chip is full and the contraction long: the widest tile, W
+  // from its image, rows gathered (by no more than 27 positions: with the third
+  // buffer two workgroups still fit a compute unit's LDS).  The registers it frees let bf16 rows go eight
+  // wavefronts to a workgroup, half the reading of W: 596000 x 2592 x 128 433 ->
+  // 406 us, and of ten layers of 57 to 395 GFLOP 0.99 to 1.10 times as fast.
+  // 1.36 M x 1728 x 64 in three planes 1386 -> 1347.  Everywhere else what the
+  // third buffer costs is not made good: (3, 1, 1) 58.8 -> 61.6 us, one plane
+  // (1, 2) 40 -> 47, rows that are not gathered 141 -> 148.
+  if constexpr (PL != 2)
+    if (choice.tile == 3 && choice.image && gs && (PL > 1 || a16))
+      return launch_planes<PL, (PL > 1 ? 2 : 1), (PL > 1 ? 2 : 4), W_STREAM, false, (PL > 1 ? 4 : 8)>(
+          ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
 #define SCN_PLANES_CASE(I, MT, NT)                                             \
   case I:                                                                      \
     return choice.image                                                        \
-               ? launch_planes<PL, MT, NT, true>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows) \
-               : launch_planes<PL, MT, NT, false>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
+               ? launch_planes<PL, MT, NT, W_IMAGE>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows) \
+               : launch_planes<PL, MT, NT, W_PLAIN>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
   switch (choice.tile) {
     SCN_PLANES_CASE(0, 1, 1)
     SCN_PLANES_CASE(1, 1, 2)

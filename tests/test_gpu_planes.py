@@ -43,6 +43,30 @@ def test_planes_against_float64(scn, ctx, rows, fs, nIn, N, act):
     assert err.max() <= 2e-6 and np.sqrt((err ** 2).mean()) <= np.sqrt((plain ** 2).mean()) + 1e-8
 
 
+# rows gathered, W streamed from its image: whole and broken groups of rows, an odd and an even number of blocks, columns
+# that are no whole slice
+@pytest.mark.parametrize("rows,fs,nIn,N", [(70144, 9, 64, 128), (70145, 27, 32, 128), (65791, 27, 64, 64), (40001, 27, 96, 160),
+                                           (33024, 12, 160, 224)])
+@pytest.mark.parametrize("a16", [False, True])
+def test_streamed_weights_give_the_same_bits(scn, ctx, rows, fs, nIn, N, a16):
+    rng = np.random.default_rng(rows + fs)
+    d_in = ctx.array(rng.standard_normal((900, nIn), dtype=np.float32))
+    d_rules = ctx.array(rng.integers(-1, 900, (rows, fs)).astype(np.int32))
+    d_W = ctx.array(rng.standard_normal((fs * nIn, N), dtype=np.float32))
+    d_B = ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+    one, two = (ctx.array(np.full((rows, N), 7, np.float32)) for _ in range(2))
+    print("streamed", rows, fs, nIn, N, a16, flush=True)
+    if a16:
+        ctx.conv_nin_forward_a16(d_in, 900, ctx.empty((900, nIn), np.float32), d_rules, fs, nIn, d_W, d_B, None, one, rows, N,
+                                 1.0, scn.RELU)
+    else:
+        ctx.conv_nin_forward(d_in, d_rules, fs, nIn, d_W, d_B, None, one, rows, N, 1.0, scn.RELU, scn.FP32_PLANES)
+    g = ctx.empty((rows, fs * nIn), np.float32)
+    ctx.gather_rows(d_in, g, d_rules, rows * fs, nIn)
+    ctx.nin_forward(g, d_W, d_B, None, two, rows, fs * nIn, N, 1.0, scn.RELU, scn.BF16 if a16 else scn.FP32_PLANES)
+    assert np.array_equal(one.download(), two.download())
+
+
 def test_fp32_takes_the_planes_where_they_pay(scn, ctx):
     """few rows and long contractions: the same bits as SCN_FP32_PLANES"""
     rng = np.random.default_rng(5)
