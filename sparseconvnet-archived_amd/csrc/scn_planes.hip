@@ -23,26 +23,27 @@
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
+// The PL planes of two floats, a word each.
+template <int PL> __device__ __forceinline__ void split2(float a, float b, unsigned (&w)[PL]) {
+#pragma unroll
+  for (int l = 0; l < PL; ++l) {
+    w[l] = pack_bf16x2(a, b);
+    if (l + 1 < PL) {
+      a -= __uint_as_float(w[l] << 16);
+      b -= __uint_as_float(w[l] & 0xffff0000u);
+    }
+  }
+}
 // The PL planes of eight floats, each as an MFMA operand.
 template <int PL>
 __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[PL]) {
-  unsigned w[PL][4];
+  unsigned w[4][PL];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float a = x[2 * i], b = x[2 * i + 1];
-#pragma unroll
-    for (int l = 0; l < PL; ++l) {
-      const unsigned h = pack_bf16x2(a, b);
-      w[l][i] = h;
-      if (l + 1 < PL) {
-        a -= __uint_as_float(h << 16);
-        b -= __uint_as_float(h & 0xffff0000u);
-      }
-    }
-  }
+  for (int i = 0; i < 4; ++i)
+    split2<PL>(x[2 * i], x[2 * i + 1], w[i]);
 #pragma unroll
   for (int l = 0; l < PL; ++l)
-    p[l] = __builtin_bit_cast(bf16x8, uint4{w[l][0], w[l][1], w[l][2], w[l][3]});
+    p[l] = __builtin_bit_cast(bf16x8, uint4{w[0][l], w[1][l], w[2][l], w[3][l]});
 }
 
 // Rows that are known on the device only.  Which kernel takes a layer depends
@@ -197,43 +198,54 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
   const int n0 = split * NW;
   const int T = K / 32;
 
-  // ---- W.  One item = 8 consecutive k of one column, or 16 bytes of the image
+  // ---- W.  One item = V adjacent columns of two consecutive k, or 16 bytes of the
+  // image.  (Every instruction occupies the vector memory path for 16 cycles or
+  // more: with the eight k of a column to an item, a dword each, 100 drawings'
+  // layers of 128 and 256 k took 5 % longer.  N is a multiple of 4; a scratch
+  // matrix W may be aligned to no more than a float.)
   constexpr bool IMG = WM == W_IMAGE;
-  constexpr int ITEMS = IMG ? BUF_BYTES / 16 : 4 * NW;
+  constexpr int V = NT % 2 ? 2 : 4;
+  constexpr int ITEMS = IMG ? BUF_BYTES / 16 : 16 * NW / V;
   constexpr int WPER = STREAM ? 0 : (ITEMS + THREADS - 1) / THREADS;
-  constexpr int WREGS = IMG ? 4 : 8;
+  constexpr int WREGS = IMG ? 4 : 2 * V;
   float wv[PD][WPER + 1][WREGS];
-  int wDst[WPER + 1];
+  int wDst[WPER + 1][IMG ? 1 : V];
   const float *wSrc[WPER + 1];
 #pragma unroll
   for (int u = 0; u < WPER; ++u) {
     int x = tid + THREADS * u;
     x = x < ITEMS ? x : ITEMS - 1; // past the end: the last item again (same value, same place)
-    if (IMG) {
-      wDst[u] = x * 16;
+    if constexpr (IMG) {
+      wDst[u][0] = x * 16;
       wSrc[u] = W + (long long)split * T * (BUF_BYTES / 4) + x * 4;
     } else {
-      const int kg = x / NW, tile = (x % NW) / 32, cc = x % 32;
-      int n = n0 + NT * cc + tile;
-      n = n < N ? n : N - 1; // (a column past the end is not stored)
-      wDst[u] = (kg / 2) * STEP_BYTES + tile * 1024 + (kg & 1) * 512 + cc * 16;
-      wSrc[u] = W + (long long)(8 * kg) * N + n;
+      const int kp = x / (NW / V), at = V * (x % (NW / V));
+#pragma unroll
+      for (int e = 0; e < V; ++e)
+        wDst[u][e] = (kp / 8) * STEP_BYTES + (at + e) % NT * 1024 + (kp / 4 & 1) * 512 + (at + e) / NT * 16 + (kp & 3) * 4;
+      // (columns past the end are not stored)
+      wSrc[u] = W + (long long)(2 * kp) * N + (n0 + at < N ? n0 + at : N - V);
     }
   }
   auto w_load = [&](int slot, int t) {
     t = t < T ? t : T - 1;
 #pragma unroll
     for (int u = 0; u < WPER; ++u) {
-      if (IMG) {
+      if constexpr (IMG) {
         const floatx4 v = *reinterpret_cast<const floatx4 *>(wSrc[u] + (long long)t * (BUF_BYTES / 4));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           wv[slot][u][i] = v[i];
       } else {
+        typedef float floatxv __attribute__((ext_vector_type(V), aligned(4)));
         const float *p = wSrc[u] + (long long)t * 32 * N;
 #pragma unroll
-        for (int i = 0; i < WREGS; ++i)
-          wv[slot][u][i] = p[(long long)i * N];
+        for (int h = 0; h < 2; ++h) {
+          const floatxv v = *reinterpret_cast<const floatxv *>(p + (long long)h * N);
+#pragma unroll
+          for (int e = 0; e < V; ++e)
+            wv[slot][u][2 * e + h] = v[e];
+        }
       }
     }
   };
@@ -241,18 +253,20 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
 #pragma unroll
     for (int u = 0; u < WPER; ++u) {
       if constexpr (IMG) {
-        *reinterpret_cast<floatx4 *>(sW + buf * BUF_BYTES + wDst[u]) =
+        *reinterpret_cast<floatx4 *>(sW + buf * BUF_BYTES + wDst[u][0]) =
             floatx4{wv[slot][u][0], wv[slot][u][1], wv[slot][u][2], wv[slot][u][3]};
       } else {
-        bf16x8 p[PL];
-        split8<PL>(wv[slot][u], p);
 #pragma unroll
-        for (int l = 0; l < PL; ++l)
-          *reinterpret_cast<bf16x8 *>(sW + buf * BUF_BYTES + l * PLANE_BYTES + wDst[u]) = p[l];
+        for (int e = 0; e < V; ++e) {
+          unsigned w[PL];
+          split2<PL>(wv[slot][u][2 * e], wv[slot][u][2 * e + 1], w);
+#pragma unroll
+          for (int l = 0; l < PL; ++l)
+            *reinterpret_cast<unsigned *>(sW + buf * BUF_BYTES + l * PLANE_BYTES + wDst[u][e]) = w[l];
+        }
       }
     }
   };
-
   // W_STREAM: a block of the image goes straight into LDS, a kilobyte an instruction,
   // each wavefront every WAVES-th of them.  (The compiler does not know of these
   // loads: what it waits for of its own, the loads being counted in order, it

@@ -284,3 +284,30 @@ def test_a_context_without_room_for_weights_gives_the_same_bits(scn, ctx):
             c.sync()
         assert all(np.array_equal(x.download(), y.download()) for x, y in zip(*outs))
     scn.lib().scn_ctx_destroy(h)
+
+
+@pytest.mark.parametrize("M,N,K", [(60000, 256, 512), (20001, 64, 100), (20001, 96, 36), (40001, 128, 260)])
+def test_scratch_that_begins_at_any_float(scn, ctx, M, N, K):
+    """a context without room for weights transposes W into the caller's scratch, wherever that begins"""
+    import ctypes as C
+    h = C.c_void_p()
+    assert scn.lib().scn_ctx_create_for_plans(0, C.byref(h)) == scn.OK
+    plain = scn.Context(handle=h.value)
+    rng = np.random.default_rng(K)
+    D, W = ctx.array(rng.standard_normal((M, N), dtype=np.float32)), ctx.array(rng.standard_normal((K, N), dtype=np.float32))
+    room = ctx.empty(scn.lib().scn_sgemm_ABt_workspace(N, K) + 4, np.float32)
+    got = []
+    print("scratch", M, N, K, flush=True)
+    for c, at in ((ctx, 0), (plain, 0), (plain, 1), (plain, 2)):
+        out = ctx.empty((M, K), np.float32)
+        ctx.sync()
+        scn._check(scn.lib().scn_sgemm_ABt(c.h, D.ptr, W.ptr, out.ptr, M, N, K, C.c_void_p(room.ptr + 4 * at)))
+        c.sync()
+        got.append(out.download())
+    f64 = D.download()[:500].astype(np.float64) @ W.download().astype(np.float64).T
+    scale = np.abs(D.download()[:500]).astype(np.float64) @ np.abs(W.download()).astype(np.float64).T
+    # (fp32's own accumulation, or the planes': a rounding every few of the N)
+    assert all(np.all(np.abs(g[:500] - f64) <= 2e-6 * scale) for g in got)
+    if N >= 256:  # the planes whatever the scratch
+        assert all(np.array_equal(got[0], g) for g in got[1:])
+    scn.lib().scn_ctx_destroy(h)
