@@ -375,3 +375,5 @@ int intRoundUp(int a, int d);
 std::vector<int> range(int n);
 template <typename t>
 std::vector<int> vectorTopIndices(std::vector<t> &test, int k);
+template <typename t> // ... into a vector that is there
+void vectorTopIndices(std::vector<t> &test, int k, std::vector<int> &indices);

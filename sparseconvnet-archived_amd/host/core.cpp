@@ -51,8 +51,15 @@ int intRound(int a, int d) { return (int)(round(a * 1.0 / d) * d); }
 
 // Top-k indices, best first; on ties the lower index stays ahead.
 template <typename t>
-std::vector<int> vectorTopIndices(std::vector<t> &test, int k) {
-  std::vector<int> indices(k);
+void vectorTopIndices(std::vector<t> &test, int k, std::vector<int> &indices) {
+  indices.assign(k, 0);
+  if (k == 1) {
+    t most = test[0];
+    for (int i = 1; i < (int)test.size(); i++)
+      if (test[i] > most)
+        most = test[i], indices[0] = i;
+    return;
+  }
   std::vector<t> best(k);
   best[0] = test[0];
   for (int i = 1; i < (int)test.size(); i++) {
@@ -71,8 +78,14 @@ std::vector<int> vectorTopIndices(std::vector<t> &test, int k) {
       indices[j] = i;
     }
   }
+}
+template <typename t>
+std::vector<int> vectorTopIndices(std::vector<t> &test, int k) {
+  std::vector<int> indices;
+  vectorTopIndices(test, k, indices);
   return indices;
 }
+template void vectorTopIndices<float>(std::vector<float> &, int, std::vector<int> &);
 template std::vector<int> vectorTopIndices<float>(std::vector<float> &, int);
 
 // ---- RNG ------------------------------------------------------------------------
@@ -409,6 +422,8 @@ void SpatiallySparseBatch::reset() {
   labels.resize(0);
   labels.copyToCPU();
   result->labels.clear();
+  sparePredictions.swap(predictions);
+  spareProbabilities.swap(probabilities);
   predictions.resize(0);
   probabilities.resize(0);
   negativeLogLikelihood = 0;

@@ -1126,11 +1126,18 @@ void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
   r.pending = false;
   const int nClasses = input.nFeatures;
   const float *probs = r.pinned;
+  const size_t had = batch.probabilities.size(), had2 = batch.predictions.size();
+  if (had == 0)
+    batch.probabilities.swap(batch.spareProbabilities);
+  if (had2 == 0)
+    batch.predictions.swap(batch.sparePredictions);
+  batch.probabilities.resize(had + batch.batchSize);
+  batch.predictions.resize(had2 + batch.batchSize);
   for (int i = 0; i < batch.batchSize; ++i)
-    batch.probabilities.push_back(std::vector<float>(
-        probs + (size_t)i * nClasses, probs + (size_t)(i + 1) * nClasses));
+    batch.probabilities[had + i].assign(probs + (size_t)i * nClasses,
+                                        probs + (size_t)(i + 1) * nClasses);
   for (int i = 0; i < batch.batchSize; i++)
-    batch.predictions.push_back(vectorTopIndices(batch.probabilities[i], nTop));
+    vectorTopIndices(batch.probabilities[i], nTop, batch.predictions[had2 + i]);
   if (batch.type != UNLABELEDBATCH) {
     const std::vector<int> &labels = r.labels;
     batch.mistakes += batch.batchSize;
