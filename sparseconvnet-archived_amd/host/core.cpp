@@ -375,7 +375,8 @@ void SpatiallySparseBatchInterface::summary() {
 }
 
 BatchResultStage::BatchResultStage()
-    : pinned(nullptr), capacity(0), copied(false), arrived(nullptr), pending(false),
+    : pinned(nullptr), capacity(0), copied(false), stamps(nullptr),
+      stamp(0), stamped(0), arrived(nullptr), pending(false),
       consumed(nullptr), consumedPending(false), enqueued(true) {}
 BatchResultStage::~BatchResultStage() {
   if (arrived)
@@ -384,6 +385,8 @@ BatchResultStage::~BatchResultStage() {
     scn_event_destroy(consumed);
   if (pinned)
     scn_host_free(scnDefaultContext(), pinned);
+  if (stamps)
+    scn_host_free(scnDefaultContext(), stamps);
 }
 
 PinnedStage::~PinnedStage() {

@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include "SpatiallySparseLayer.h"
 
 static void unsupported(const char *what) {
@@ -1044,6 +1045,23 @@ static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream)
   SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
                              (void **)&r.pinned));
 }
+static const int kStampRows = 512; // the most that scn_terminal_classifier_supported allows
+// Watches a stamped batch's words.  False: it has none, or they were not written
+// within milliseconds (the stream has to be waited for, which also surfaces an error).
+bool resultsArrived(BatchResultStage &r) {
+  if (!r.pending || !r.stamped)
+    return false;
+  const volatile unsigned *words = r.stamps;
+  int row = 0;
+  for (int spin = 0; spin < 400000 && row < r.stamped; ++spin) {
+    while (row < r.stamped && words[row] == r.stamp)
+      ++row;
+    if (row < r.stamped)
+      __builtin_ia32_pause();
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return row == r.stamped;
+}
 // A net's end, a terminal pooling and the classifier, in one launch that also
 // leaves the probabilities where the host reads them.  False: not of that kind,
 // nothing done.
@@ -1060,7 +1078,8 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
       !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
       middle.nSpatialSites != batch.batchSize ||
       !scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn,
-                                         n->nFeaturesOut))
+                                         n->nFeaturesOut) ||
+      batch.batchSize > kStampRows)
     return false;
   const size_t K = n->nFeaturesIn, N = n->nFeaturesOut, M = batch.batchSize;
   output.sub->reset();
@@ -1068,12 +1087,20 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   middle.sub->features.resize64(M * K, kBoundRows * K);
   output.sub->features.resize64(M * N, kBoundRows * N);
   result_room(*batch.result, M * N, ms);
-  SCN_CHECKED(scn_terminal_classifier(
+  BatchResultStage &r = *batch.result;
+  r.stamped = batch.countsPending ? (int)M : 0; // (a batch on the net's own stream, read at once)
+  if (r.stamped && !r.stamps) {
+    SCN_CHECKED(scn_host_alloc(ms.ctx, kStampRows * sizeof(unsigned), (void **)&r.stamps));
+    memset(r.stamps, 0, kStampRows * sizeof(unsigned));
+  }
+  if (++r.stamp == 0) // (the words begin as zeros)
+    ++r.stamp;
+  SCN_CHECKED(scn_terminal_classifier_stamped(
       ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
       (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
       n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
-      (int)N, 1.0f - n->dropout));
-  batch.result->copied = true;
+      (int)N, 1.0f - n->dropout, r.stamped ? r.stamps : nullptr, r.stamp));
+  r.copied = true;
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)M * K * N);
   return true;
@@ -1101,6 +1128,8 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
   }
   BatchResultStage &r = *batch.result;
   const size_t n = (size_t)batch.batchSize * input.nFeatures;
+  if (!r.copied)
+    r.stamped = 0;
   result_room(r, n, memStream);
   if (!r.arrived)
     SCN_CHECKED(scn_event_create(memStream.ctx, &r.arrived));
@@ -1122,7 +1151,8 @@ void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
   BatchResultStage &r = *batch.result;
   if (!r.pending)
     return;
-  SCN_CHECKED(scn_event_wait(r.arrived));
+  if (!resultsArrived(r))
+    SCN_CHECKED(scn_event_wait(r.arrived));
   r.pending = false;
   const int nClasses = input.nFeatures;
   const float *probs = r.pinned;
