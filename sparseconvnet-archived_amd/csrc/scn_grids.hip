@@ -1319,7 +1319,8 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
     if (blocks > 16384)
       blocks = 16384;
     ScanState rank = {nullptr, 0};
-    if (clearWords) { // (as many lanes as words, or 16384 x 256: more than tiles)
+    // (as many lanes as words, or 16384 x 256: more than tiles)
+    if (clearWords && scn_scan_state(g->nWords + 1, nullptr).words) {
       SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
       rank = scn_scan_state(g->nWords + 1, g->scanTmp.p);
       if (rank.words <= blocks * 256)

@@ -787,25 +787,8 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
   const size_t lds = (size_t)(WM == W_STREAM ? 3 : 2) * PL * 2 * NT * 1024 +
                      (gs ? (size_t)32 * WAVES * MT * gs->fs * 4 : 0);
   constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
-  static OncePerDevice configured;
-  const int rc = configured.run(ctx->device, [&]() {
-    int rc = SCN_OK;
-#define SCN_PLANES_LDS(G, H)                                                   \
-  if (hipFuncSetAttribute(                                                     \
-          reinterpret_cast<const void *>(k_nin_planes<PL, MT, NT, PD, G, H, WM, WAVES>), \
-          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) \
-    rc = SCN_ERR_HIP;
-    if constexpr (WM == W_STREAM) {
-      SCN_PLANES_LDS(G, PL == 1)
-    } else {
-      SCN_PLANES_LDS(0, false) SCN_PLANES_LDS(G, false)
-      if (PL == 1)
-        SCN_PLANES_LDS(G, PL == 1)
-    }
-#undef SCN_PLANES_LDS
-    return rc;
-  });
-  SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  // (what a launch may ask for without saying so: saying it costs 0.1 ms and more a kernel)
+  SCN_REQUIRE(lds <= 64 * 1024, SCN_ERR_ARG, "planes: %d filter positions", gs ? gs->fs : 0);
   const PlainW plain = {W, wT};
   if (WM != W_PLAIN) {
     const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;

@@ -16,7 +16,7 @@ struct BatchResultStage {
   bool copied; // the forward pass has left the probabilities in `pinned` already
   // ... and writes `stamp` into a word a row as it does, `stamped` of them: watching
   // those takes a microsecond or two where waiting for the stream takes ten
-  unsigned *stamps;
+  unsigned *stamps; // behind `pinned`, of its allocation
   unsigned stamp;
   int stamped;
   scn_event *arrived;

@@ -385,8 +385,6 @@ BatchResultStage::~BatchResultStage() {
     scn_event_destroy(consumed);
   if (pinned)
     scn_host_free(scnDefaultContext(), pinned);
-  if (stamps)
-    scn_host_free(scnDefaultContext(), stamps);
 }
 
 PinnedStage::~PinnedStage() {

@@ -1035,17 +1035,20 @@ int TerminalPoolingLayer::calculateInputSpatialSize(int outputSpatialSize) {
 // In two halves, so that a caller may queue the next batch's forward pass
 // between them: the copy of the probabilities to the host is only queued
 // (SoftmaxClassifier.cu:24, copyToCPUAsync), the statistics are computed once
-// pinned memory for the probabilities of a batch
+static const int kStampRows = 512; // the most that scn_terminal_classifier_supported allows
+// pinned memory for the probabilities of a batch, and the words that say which of
+// its rows have arrived
 static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream) {
   if (n <= r.capacity)
     return;
   if (r.pinned)
     SCN_CHECKED(scn_host_free(memStream.ctx, r.pinned));
   r.capacity = n + n / 2;
-  SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
+  SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float) + kStampRows * sizeof(unsigned),
                              (void **)&r.pinned));
+  r.stamps = (unsigned *)(r.pinned + r.capacity);
+  memset(r.stamps, 0, kStampRows * sizeof(unsigned));
 }
-static const int kStampRows = 512; // the most that scn_terminal_classifier_supported allows
 // Watches a stamped batch's words.  False: it has none, or they were not written
 // within milliseconds (the stream has to be waited for, which also surfaces an error).
 bool resultsArrived(BatchResultStage &r) {
@@ -1089,10 +1092,6 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   result_room(*batch.result, M * N, ms);
   BatchResultStage &r = *batch.result;
   r.stamped = batch.countsPending ? (int)M : 0; // (a batch on the net's own stream, read at once)
-  if (r.stamped && !r.stamps) {
-    SCN_CHECKED(scn_host_alloc(ms.ctx, kStampRows * sizeof(unsigned), (void **)&r.stamps));
-    memset(r.stamps, 0, kStampRows * sizeof(unsigned));
-  }
   if (++r.stamp == 0) // (the words begin as zeros)
     ++r.stamp;
   SCN_CHECKED(scn_terminal_classifier_stamped(
