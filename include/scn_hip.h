@@ -223,9 +223,6 @@ int scn_rules_terminal_plan(scn_ctx *ctx, const scn_grids *in, scn_grids *out,
  * plans the batch again with deferral off (that also raises the bounds). */
 int scn_ctx_defer_counts(scn_ctx *ctx, int on);
 int scn_rules_settle(scn_ctx *ctx);
-/* The same without waiting, for a caller that has seen on the host what a kernel
- * queued on the context behind all of its plans has written there. */
-int scn_rules_settle_arrived(scn_ctx *ctx);
 /* The layers' kernels ahead of the counts.  Until it is called with null, the
  * feature calls that follow on the context (scn_gather_rows, scn_nin_forward,
  * scn_conv_nin_forward*, scn_maxpool*, scn_terminal_pool) take the number of
@@ -352,14 +349,6 @@ int scn_terminal_classifier(scn_ctx *ctx, const float *d_in,
                             float *d_pooled, const float *d_W,
                             const float *d_B, float *d_probs, float *copy,
                             int K, int N, float p);
-/* The same; stamps[m] (M words of pinned host memory, 32-bit) becomes `stamp` once
- * row m of `copy` can be read by the host. */
-int scn_terminal_classifier_stamped(scn_ctx *ctx, const float *d_in,
-                                    const int32_t *d_rules, int64_t M, int S,
-                                    float *d_pooled, const float *d_W,
-                                    const float *d_B, float *d_probs,
-                                    float *copy, int K, int N, float p,
-                                    uint32_t *stamps, uint32_t stamp);
 /* dSigmoidSoftmax (SigmoidLayer.cu:160-177). */
 int scn_softmax_rows(scn_ctx *ctx, const float *d_in, float *d_out, int64_t M,
                      int N);

@@ -97,7 +97,6 @@ def lib():
         "scn_ctx_chain_rules": (C.c_int, [vp, C.c_int]),
         "scn_ctx_chain_count": (C.c_int, [vp, P(i64), P(i64)]),
         "scn_rules_settle": (C.c_int, [vp]),
-        "scn_rules_settle_arrived": (C.c_int, [vp]),
         "scn_ctx_rows_from": (C.c_int, [vp, vp]),
         "scn_ctx_rows_held": (C.c_int, [vp, P(C.c_int)]),
         "scn_grids_destroy": (C.c_int, [vp, vp]),
@@ -127,8 +126,6 @@ def lib():
         "scn_terminal_pool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
         "scn_terminal_classifier_supported": (C.c_int, [i64, C.c_int, C.c_int]),
         "scn_terminal_classifier": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float]),
-        "scn_terminal_classifier_stamped": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int,
-                                                      C.c_float, vp, C.c_uint32]),
         "scn_softmax_rows": (C.c_int, [vp, vp, vp, i64, C.c_int]),
         "scn_softmax_grad": (C.c_int, [vp, vp, vp, vp, i64, C.c_int]),
         "scn_activation_backward": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),

@@ -1581,15 +1581,14 @@ extern "C" int scn_ctx_defer_counts(scn_ctx *ctx, int on) {
   ctx->deferCounts = on != 0;
   return SCN_OK;
 }
-static int settle(scn_ctx *ctx, bool wait) {
+extern "C" int scn_rules_settle(scn_ctx *ctx) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_rules_settle: null context");
   SCN_TRY(scn_chain_flush(ctx));
   ctx->d_meta = nullptr; // (the counts that scn_ctx_rows_from spoke of are the host's from here on)
   ctx->rowsHeld = true; // (of the passes settled here: none, when nothing is pending)
   if (ctx->pendingGrids.empty())
     return SCN_OK;
-  if (wait)
-    SCN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+  SCN_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   std::atomic_thread_fence(std::memory_order_acquire);
   bool overflowed = false;
   for (const auto &c : ctx->rowsChosen) {
@@ -1634,8 +1633,6 @@ static int settle(scn_ctx *ctx, bool wait) {
               "plans; plan it again with deferral off");
   return SCN_OK;
 }
-extern "C" int scn_rules_settle(scn_ctx *ctx) { return settle(ctx, true); }
-extern "C" int scn_rules_settle_arrived(scn_ctx *ctx) { return settle(ctx, false); }
 extern "C" int scn_ctx_rows_from(scn_ctx *ctx, const scn_grids *g) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_ctx_rows_from: null context");
   ctx->d_meta = nullptr;

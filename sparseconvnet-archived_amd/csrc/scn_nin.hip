@@ -284,9 +284,6 @@ __global__ void __launch_bounds__(FR_THREADS)
 // each a few microseconds of launch, trips to memory and drain, in one (1 x 192 x
 // 100: 3.1 + 6.7 + 2.3 us and two gaps -> 5.8; 100 rows 4.0 + 8.7 + 2.4 -> 6.1; 33
 // x 128 x 40 4.4 + 5.5 + 2.6 -> 6.4; 61 x 800 x 100 4.9 + 17.5 + 3.3 -> 11.0).
-// Stamps: the host sees a row's word 10 to 35 us before a wait for the stream comes
-// back (one drawing 115 -> 102 us, 100 drawings 214 -> 189, 61 images of the wide
-// net 429 -> 394), so a wavefront writes its row's when the row is out.
 #define CL_DEPTH 12
 #define CL_ROWS 2
 struct TerminalSource {
@@ -295,21 +292,12 @@ struct TerminalSource {
   const long long *meta;
   float *pooled; // [M x K]
   float *copy;   // [M x N], or null
-  // a word a row in host memory, or null: `stamp` once the row's copy is there
-  unsigned *stamps;
-  unsigned stamp;
 };
 template <bool TERMINAL>
 __global__ void __launch_bounds__(FR_THREADS)
     k_classifier(const float *__restrict__ A, const float *__restrict__ W, float *__restrict__ out, long long M, int K,
                  int N, Epilogue ep, const long long *dRows, TerminalSource ts) {
-  const long long bound = M;
   M = live_rows(M, dRows);
-  if (TERMINAL && ts.stamps && threadIdx.x < CL_ROWS) { // (rows that there are not: nothing to wait for)
-    const long long m = (long long)blockIdx.x * CL_ROWS + threadIdx.x;
-    if (m >= M && m < bound)
-      *(volatile unsigned *)(ts.stamps + m) = ts.stamp;
-  }
   if ((long long)blockIdx.x * CL_ROWS >= M)
     return;
   __shared__ __attribute__((aligned(16))) float sA[CL_ROWS][FR_MAX_K];
@@ -458,11 +446,6 @@ __global__ void __launch_bounds__(FR_THREADS)
       if (TERMINAL && ts.copy)
         ts.copy[m * N + 64 * j + lane] = y;
     }
-  if (TERMINAL && ts.stamps) {
-    __threadfence_system();
-    if (lane == 0)
-      *(volatile unsigned *)(ts.stamps + m) = ts.stamp;
-  }
 }
 
 // ---- few input channels: one lane per four outputs ------------------------
@@ -2070,12 +2053,6 @@ extern "C" int scn_terminal_classifier_supported(int64_t M, int K, int N) {
 extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
                                        float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
                                        float *copy, int K, int N, float p) {
-  return scn_terminal_classifier_stamped(ctx, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, p, nullptr,
-                                         0);
-}
-extern "C" int scn_terminal_classifier_stamped(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
-                                               float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
-                                               float *copy, int K, int N, float p, uint32_t *stamps, uint32_t stamp) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_terminal_classifier: null context");
   SCN_REQUIRE(S >= 1 && scn_terminal_classifier_supported(M, K, N), SCN_ERR_ARG,
               "scn_terminal_classifier: M %lld S %d K %d N %d", (long long)M, S, K, N);
@@ -2088,7 +2065,7 @@ extern "C" int scn_terminal_classifier_stamped(scn_ctx *ctx, const float *d_in, 
   ep.p = p;
   ep.act = SCN_SOFTMAX;
   ProfScope prof(ctx, SCN_K_NIN);
-  TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy, stamps, stamp};
+  TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy};
   hipLaunchKernelGGL((k_classifier<true>), dim3(scn_ceil_div(M, CL_ROWS)), dim3(FR_THREADS), 0, ctx->stream, d_in, d_W,
                      d_probs, (long long)M, K, N, ep, ctx->d_meta ? ctx->d_meta + META_SITES : nullptr, ts);
   SCN_HIP_CHECK(hipGetLastError());

@@ -14,11 +14,6 @@ struct BatchResultStage {
   float *pinned;
   size_t capacity; // floats
   bool copied; // the forward pass has left the probabilities in `pinned` already
-  // ... and writes `stamp` into a word a row as it does, `stamped` of them: watching
-  // those takes a microsecond or two where waiting for the stream takes ten
-  unsigned *stamps; // behind `pinned`, of its allocation
-  unsigned stamp;
-  int stamped;
   scn_event *arrived;
   bool pending;
   // a training batch: the point of the net's stream behind the backward pass,

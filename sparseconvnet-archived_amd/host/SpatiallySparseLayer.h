@@ -367,8 +367,6 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &output,
                                cudaMemStream &ms);
 
-bool resultsArrived(BatchResultStage &r);
-
 // utilities.h
 int ipow(int base, int exp);
 int triangleSize(int linearSize, int dimension);

@@ -375,8 +375,7 @@ void SpatiallySparseBatchInterface::summary() {
 }
 
 BatchResultStage::BatchResultStage()
-    : pinned(nullptr), capacity(0), copied(false), stamps(nullptr),
-      stamp(0), stamped(0), arrived(nullptr), pending(false),
+    : pinned(nullptr), capacity(0), copied(false), arrived(nullptr), pending(false),
       consumed(nullptr), consumedPending(false), enqueued(true) {}
 BatchResultStage::~BatchResultStage() {
   if (arrived)

@@ -5,7 +5,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include "SpatiallySparseLayer.h"
 
 static void unsupported(const char *what) {
@@ -1035,35 +1034,15 @@ int TerminalPoolingLayer::calculateInputSpatialSize(int outputSpatialSize) {
 // In two halves, so that a caller may queue the next batch's forward pass
 // between them: the copy of the probabilities to the host is only queued
 // (SoftmaxClassifier.cu:24, copyToCPUAsync), the statistics are computed once
-static const int kStampRows = 512; // the most that scn_terminal_classifier_supported allows
-// pinned memory for the probabilities of a batch, and the words that say which of
-// its rows have arrived
+// pinned memory for the probabilities of a batch
 static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream) {
   if (n <= r.capacity)
     return;
   if (r.pinned)
     SCN_CHECKED(scn_host_free(memStream.ctx, r.pinned));
   r.capacity = n + n / 2;
-  SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float) + kStampRows * sizeof(unsigned),
+  SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
                              (void **)&r.pinned));
-  r.stamps = (unsigned *)(r.pinned + r.capacity);
-  memset(r.stamps, 0, kStampRows * sizeof(unsigned));
-}
-// Watches a stamped batch's words.  False: it has none, or they were not written
-// within milliseconds (the stream has to be waited for, which also surfaces an error).
-bool resultsArrived(BatchResultStage &r) {
-  if (!r.pending || !r.stamped)
-    return false;
-  const volatile unsigned *words = r.stamps;
-  int row = 0;
-  for (int spin = 0; spin < 400000 && row < r.stamped; ++spin) {
-    while (row < r.stamped && words[row] == r.stamp)
-      ++row;
-    if (row < r.stamped)
-      __builtin_ia32_pause();
-  }
-  std::atomic_thread_fence(std::memory_order_acquire);
-  return row == r.stamped;
 }
 // A net's end, a terminal pooling and the classifier, in one launch that also
 // leaves the probabilities where the host reads them.  False: not of that kind,
@@ -1081,8 +1060,7 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
       !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
       middle.nSpatialSites != batch.batchSize ||
       !scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn,
-                                         n->nFeaturesOut) ||
-      batch.batchSize > kStampRows)
+                                         n->nFeaturesOut))
     return false;
   const size_t K = n->nFeaturesIn, N = n->nFeaturesOut, M = batch.batchSize;
   output.sub->reset();
@@ -1090,16 +1068,12 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   middle.sub->features.resize64(M * K, kBoundRows * K);
   output.sub->features.resize64(M * N, kBoundRows * N);
   result_room(*batch.result, M * N, ms);
-  BatchResultStage &r = *batch.result;
-  r.stamped = batch.countsPending ? (int)M : 0; // (a batch on the net's own stream, read at once)
-  if (++r.stamp == 0) // (the words begin as zeros)
-    ++r.stamp;
-  SCN_CHECKED(scn_terminal_classifier_stamped(
+  SCN_CHECKED(scn_terminal_classifier(
       ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
       (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
       n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
-      (int)N, 1.0f - n->dropout, r.stamped ? r.stamps : nullptr, r.stamp));
-  r.copied = true;
+      (int)N, 1.0f - n->dropout));
+  batch.result->copied = true;
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)M * K * N);
   return true;
@@ -1127,8 +1101,6 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
   }
   BatchResultStage &r = *batch.result;
   const size_t n = (size_t)batch.batchSize * input.nFeatures;
-  if (!r.copied)
-    r.stamped = 0;
   result_room(r, n, memStream);
   if (!r.arrived)
     SCN_CHECKED(scn_event_create(memStream.ctx, &r.arrived));
@@ -1150,8 +1122,7 @@ void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
   BatchResultStage &r = *batch.result;
   if (!r.pending)
     return;
-  if (!resultsArrived(r))
-    SCN_CHECKED(scn_event_wait(r.arrived));
+  SCN_CHECKED(scn_event_wait(r.arrived));
   r.pending = false;
   const int nClasses = input.nFeatures;
   const float *probs = r.pinned;

@@ -321,8 +321,7 @@ bool SparseConvNetCUDA::settleRuleBooks(SpatiallySparseBatch &b) {
   scn_ctx *ctx = b.preprocessStream ? b.preprocessStream->ctx : memStream.ctx;
   const bool ahead = b.countsPending;
   b.countsPending = false;
-  const int rc = ahead && resultsArrived(*b.result) ? scn_rules_settle_arrived(ctx)
-                                                    : scn_rules_settle(ctx);
+  const int rc = scn_rules_settle(ctx);
   if (rc == SCN_ERR_CAPACITY) {
     planAllLayers(cnn, ctx, b); // every plan empties its own output tables again
     return false;

@@ -1,5 +1,5 @@
 """Results of batches of changing sizes through one net, whose vectors are written over: the probabilities, predictions
-and counts are those of nets that have seen no other batch, for one prediction a sample and for several.  And the words that say on the host that a row of them has arrived."""
+and counts are those of nets that have seen no other batch, for one prediction a sample and for several."""
 import numpy as np
 import pytest
 
@@ -37,29 +37,3 @@ def test_results_of_batches_in_turn(scn, nTop):
         assert np.array_equal(again[:b], p) and np.all(again[b] == 7) and np.all(pred[b] == -1)
         assert np.array_equal(pred[:b], _ranked(p, nTop))
     net.close()
-
-
-@pytest.mark.parametrize("M", [1, 2, 3, 511, 512])
-def test_stamps_say_that_a_row_has_arrived(scn, ctx, M):
-    import time
-    K, N, S = 64, 20, 3
-    rng = np.random.default_rng(M)
-    x = ctx.array(rng.standard_normal((M * S, K)).astype(np.float32))
-    rules = ctx.array(np.arange(M * S, dtype=np.int32))
-    W, B = ctx.array(rng.standard_normal((K, N)).astype(np.float32)), ctx.array(rng.standard_normal(N).astype(np.float32))
-    pooled, probs = ctx.empty((M, K), np.float32), ctx.empty((M, N), np.float32)
-    room, words = ctx.host_alloc(M * N * 4), ctx.host_alloc((M + 1) * 4)
-    copy, stamps = np.frombuffer(room.buffer(), np.float32).reshape(M, N), np.frombuffer(words.buffer(), np.uint32)
-    stamps[:] = 0
-    print("stamps", M, flush=True)
-    for stamp in (1, 2, 0xffffffff):
-        copy[:] = 7
-        ctx.sync()
-        scn._check(scn.lib().scn_terminal_classifier_stamped(ctx.h, x.ptr, rules.ptr, M, S, pooled.ptr, W.ptr, B.ptr, probs.ptr,
-                                                             room.ptr, K, N, 1.0, words.ptr, stamp))
-        end = time.time() + 20
-        while not np.all(stamps[:M] == stamp) and time.time() < end:
-            pass
-        seen = copy.copy()  # (before any wait for the stream)
-        assert np.all(stamps[:M] == stamp) and stamps[M] == 0
-        assert np.array_equal(seen, probs.download())
