@@ -46,7 +46,6 @@
 #include "scn_pyr_dev.h"
 #include <stdlib.h>
 #include <string.h>
-#include <mutex>
 
 #define CHAIN_MAX_LEVELS 24
 #ifndef CHAIN_THREADS
@@ -1477,6 +1476,26 @@ int scn_chain_record_fill(scn_ctx *ctx, const scn_grids *in, scn_grids *out,
   return SCN_OK;
 }
 
+// One launch.  Above 64 KB of LDS a kernel has to be told so, once on every
+// device; the first chain of a process waits for that, so only the kernels that
+// are launched with as much are told (a net's chain takes two of the thirteen).
+template <auto Kernel, typename Args>
+static int launch_lds(scn_ctx *ctx, dim3 grid, int threads, size_t lds, const Args &a) {
+  if (lds > 64 * 1024) {
+    static OncePerDevice told;
+    const int rc = told.run(ctx->device, [] {
+      return hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 CHAIN_LDS_MAX) == hipSuccess
+                 ? SCN_OK
+                 : SCN_ERR_HIP;
+    });
+    SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  }
+  hipLaunchKernelGGL(Kernel, grid, dim3((unsigned)threads), lds, ctx->stream, a);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 // Chains of square layers without a minimum (and a terminal layer at the end)
 // are built from the output side by k_pyr_masks / k_pyr_rules.  *done = false:
 // this chain is not of that kind (or its masks do not fit), run it the other way.
@@ -1649,58 +1668,31 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   a.scalars = (long long *)ctx->d_pinned;
   a.badSites = (const long long *)(ctx->d_scalars + 15);
   cs->pyrSource = src;
-  {
-    // (above 64 KB of LDS a kernel has to be told so once)
-    static std::once_flag once;
-    static hipError_t attr = hipSuccess;
-    std::call_once(once, [] {
-      const void *k[10] = {reinterpret_cast<const void *>(&k_pyr_levels<2, 1>),
-                          reinterpret_cast<const void *>(&k_pyr_levels<2, 2>),
-                          reinterpret_cast<const void *>(&k_pyr_levels<2, 4>),
-                          reinterpret_cast<const void *>(&k_pyr_levels<3, 1>),
-                          reinterpret_cast<const void *>(&k_pyr_masks<1>),
-                          reinterpret_cast<const void *>(&k_pyr_masks<2>),
-                          reinterpret_cast<const void *>(&k_pyr_masks<3>),
-                          reinterpret_cast<const void *>(&k_pyr_rules<1>),
-                          reinterpret_cast<const void *>(&k_pyr_rules<2>),
-                          reinterpret_cast<const void *>(&k_pyr_rules<3>)};
-      for (int i = 0; i < 10 && attr == hipSuccess; ++i)
-        attr = hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   CHAIN_LDS_MAX);
-    });
-    SCN_HIP_CHECK(attr);
-  }
   const size_t ldsA = (size_t)(8 * wordsA + 16);
   const dim3 grid((unsigned)a.batch), levels((unsigned)a.batch, (unsigned)a.nSlabs);
   const dim3 gridB((unsigned)(a.batch * a.nParts + 1));
   if (RW == 1 && d == 3)
-    hipLaunchKernelGGL((k_pyr_levels<3, 1>), levels, dim3(64), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_levels<3, 1>>(ctx, levels, 64, ldsA, a)));
   else if (RW == 1)
-    hipLaunchKernelGGL((k_pyr_levels<2, 1>), levels, dim3(64), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_levels<2, 1>>(ctx, levels, 64, ldsA, a)));
   else if (RW == 2)
-    hipLaunchKernelGGL((k_pyr_levels<2, 2>), levels, dim3(64), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_levels<2, 2>>(ctx, levels, 64, ldsA, a)));
   else if (RW == 4)
-    hipLaunchKernelGGL((k_pyr_levels<2, 4>), levels, dim3(64), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_levels<2, 4>>(ctx, levels, 64, ldsA, a)));
   else if (d == 1)
-    hipLaunchKernelGGL(k_pyr_masks<1>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_masks<1>>(ctx, grid, PYR_A_THREADS, ldsA, a)));
   else if (d == 2)
-    hipLaunchKernelGGL(k_pyr_masks<2>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
+    SCN_TRY((launch_lds<k_pyr_masks<2>>(ctx, grid, PYR_A_THREADS, ldsA, a)));
   else
-    hipLaunchKernelGGL(k_pyr_masks<3>, grid, dim3(PYR_A_THREADS), ldsA, ctx->stream, a);
-  SCN_HIP_CHECK(hipGetLastError());
+    SCN_TRY((launch_lds<k_pyr_masks<3>>(ctx, grid, PYR_A_THREADS, ldsA, a)));
   switch (d) {
   case 1:
-    hipLaunchKernelGGL(k_pyr_rules<1>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
-    break;
+    return launch_lds<k_pyr_rules<1>>(ctx, gridB, PYR_B_THREADS, (size_t)ldsB, a);
   case 2:
-    hipLaunchKernelGGL(k_pyr_rules<2>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
-    break;
+    return launch_lds<k_pyr_rules<2>>(ctx, gridB, PYR_B_THREADS, (size_t)ldsB, a);
   default:
-    hipLaunchKernelGGL(k_pyr_rules<3>, gridB, dim3(PYR_B_THREADS), (size_t)ldsB, ctx->stream, a);
-    break;
+    return launch_lds<k_pyr_rules<3>>(ctx, gridB, PYR_B_THREADS, (size_t)ldsB, a);
   }
-  SCN_HIP_CHECK(hipGetLastError());
-  return SCN_OK;
 }
 
 int scn_chain_flush(scn_ctx *ctx) {
@@ -1790,33 +1782,18 @@ int scn_chain_flush(scn_ctx *ctx) {
   a.scalars = (long long *)ctx->d_pinned;
   a.badSites = (const long long *)(ctx->d_scalars + 15);
   const size_t ldsBytes = (size_t)(fixed + arena);
-  {
-    // (above 64 KB of LDS a kernel has to be told so once)
-    static std::once_flag once;
-    static hipError_t attr = hipSuccess;
-    std::call_once(once, [] {
-      const void *k[3] = {reinterpret_cast<const void *>(&k_chain_sample<1>),
-                          reinterpret_cast<const void *>(&k_chain_sample<2>),
-                          reinterpret_cast<const void *>(&k_chain_sample<3>)};
-      for (int i = 0; i < 3 && attr == hipSuccess; ++i)
-        attr = hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   CHAIN_LDS_MAX);
-    });
-    SCN_HIP_CHECK(attr);
-  }
-  const dim3 grid((unsigned)a.batch), block(CHAIN_THREADS);
+  const dim3 grid((unsigned)a.batch);
   switch (a.d) {
   case 1:
-    hipLaunchKernelGGL(k_chain_sample<1>, grid, block, ldsBytes, ctx->stream, a);
+    SCN_TRY((launch_lds<k_chain_sample<1>>(ctx, grid, CHAIN_THREADS, ldsBytes, a)));
     break;
   case 2:
-    hipLaunchKernelGGL(k_chain_sample<2>, grid, block, ldsBytes, ctx->stream, a);
+    SCN_TRY((launch_lds<k_chain_sample<2>>(ctx, grid, CHAIN_THREADS, ldsBytes, a)));
     break;
   default:
-    hipLaunchKernelGGL(k_chain_sample<3>, grid, block, ldsBytes, ctx->stream, a);
+    SCN_TRY((launch_lds<k_chain_sample<3>>(ctx, grid, CHAIN_THREADS, ldsBytes, a)));
     break;
   }
-  SCN_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(k_chain_place, dim3((unsigned)a.batch, (unsigned)a.nLevels),
                      dim3(PLACE_THREADS), 0, ctx->stream, a);
   SCN_HIP_CHECK(hipGetLastError());

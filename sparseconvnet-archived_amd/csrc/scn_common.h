@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <mutex>
 #include <vector>
 #include "scn_hip.h"
 
@@ -152,6 +153,22 @@ __device__ __forceinline__ long long live_rows(long long bound, const long long 
   const long long n = *d_rows;
   return n < bound ? n : bound;
 }
+
+// Kernel attributes (the dynamic LDS limit) are set per device: fn runs once for
+// every device a context of this process lives on, and again if it failed.
+struct OncePerDevice {
+  std::mutex m;
+  unsigned long long done = 0;
+  template <class F> int run(int device, F fn) {
+    std::lock_guard<std::mutex> lock(m);
+    if (device >= 0 && device < 64 && ((done >> device) & 1ull))
+      return SCN_OK;
+    const int rc = fn();
+    if (rc == SCN_OK && device >= 0 && device < 64)
+      done |= 1ull << device;
+    return rc;
+  }
+};
 
 // runs the recorded rule-book plans of the context, if any (scn_chain.hip)
 int scn_chain_flush(scn_ctx *ctx);

@@ -2,23 +2,6 @@
 // constants, the source of a gathered matrix, bf16 conversions.
 #pragma once
 #include "scn_common.h"
-#include <mutex>
-
-// Kernel attributes (the dynamic LDS limit) are set per device: fn runs once for
-// every device a context of this process lives on, and again if it failed.
-struct OncePerDevice {
-  std::mutex m;
-  unsigned long long done = 0;
-  template <class F> int run(int device, F fn) {
-    std::lock_guard<std::mutex> lock(m);
-    if (device >= 0 && device < 64 && ((done >> device) & 1ull))
-      return SCN_OK;
-    const int rc = fn();
-    if (rc == SCN_OK && device >= 0 && device < 64)
-      done |= 1ull << device;
-    return rc;
-  }
-};
 
 struct Epilogue {
   const float *bias;
