@@ -257,6 +257,10 @@ int scn_ctx_chain_rules(scn_ctx *ctx, int on);
 /* how many chains of recorded plans the context has run, and how many plans
  * they held in all (a plan that could not join is not counted) */
 int scn_ctx_chain_count(scn_ctx *ctx, int64_t *chains, int64_t *plans);
+/* how the last chain shared out each sample: the workgroups that made its rule
+ * rows, and the wavefronts that made its masks (0: one after the other, a
+ * wavefront a sample; both 0: a chain built from the input side) */
+int scn_ctx_chain_split(scn_ctx *ctx, int *parts, int *slabs);
 int scn_rules_width(const scn_grids *out, int64_t *width);
 /* Writes nOutputSpatialSites * width int32 rules; capacity in int32s. */
 int scn_rules_fill(scn_ctx *ctx, const scn_grids *in, scn_grids *out,

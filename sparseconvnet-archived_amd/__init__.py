@@ -96,6 +96,7 @@ def lib():
         "scn_ctx_defer_counts": (C.c_int, [vp, C.c_int]),
         "scn_ctx_chain_rules": (C.c_int, [vp, C.c_int]),
         "scn_ctx_chain_count": (C.c_int, [vp, P(i64), P(i64)]),
+        "scn_ctx_chain_split": (C.c_int, [vp, P(C.c_int), P(C.c_int)]),
         "scn_rules_settle": (C.c_int, [vp]),
         "scn_ctx_rows_from": (C.c_int, [vp, vp]),
         "scn_ctx_rows_held": (C.c_int, [vp, P(C.c_int)]),
@@ -491,6 +492,13 @@ def chain_count(ctx):
     """(chains run, plans they held) so far on this context"""
     a, b = C.c_int64(), C.c_int64()
     _check(lib().scn_ctx_chain_count(ctx.h, C.byref(a), C.byref(b)))
+    return a.value, b.value
+
+
+def chain_split(ctx):
+    """(workgroups, wavefronts) the last chain shared each sample out among, for its rule rows and its masks"""
+    a, b = C.c_int(), C.c_int()
+    _check(lib().scn_ctx_chain_split(ctx.h, C.byref(a), C.byref(b)))
     return a.value, b.value
 
 

@@ -125,6 +125,7 @@ struct ChainState {
   int pyrMisses = 0;     // such chains in a row that still outgrew it
   scn_grids *pyrSource = nullptr; // source of the last such chain: its largest sample comes back in h_pinned[13]
   long long nPyramids = 0;
+  int parts = 0, slabs = 0; // of a sample, in the last chain (scn_ctx_chain_split)
 };
 
 // ------------------------------------------------------------------ device
@@ -1267,6 +1268,15 @@ extern "C" int scn_ctx_chain_count(scn_ctx *ctx, int64_t *chains, int64_t *plans
   return SCN_OK;
 }
 
+extern "C" int scn_ctx_chain_split(scn_ctx *ctx, int *parts, int *slabs) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_ctx_chain_split: null context");
+  if (parts)
+    *parts = ctx->chain ? ctx->chain->parts : 0;
+  if (slabs)
+    *slabs = ctx->chain ? ctx->chain->slabs : 0;
+  return SCN_OK;
+}
+
 // LDS bytes of everything but the arena for a chain over grids of these
 // volumes (the source first); fills the layout when `a` is given
 static long long chain_fixed_lds(const std::vector<long long> &vols, ChainArgs *a) {
@@ -1587,9 +1597,11 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
     long long n[PYR_MAX_LEVELS + 1];
     n[0] = src->nActive / a.batch + 1;
     for (int l = 1; l < a.nMasks; ++l)
-      n[l] = recs[l - 1].out->seenActive / a.batch + 1;
+      n[l] = pyr_typical(recs[l - 1].out->meanSites, src->meanSites, n[0], a.lv[l].volOut);
+    src->saw(src->nActive, a.batch);
     const int want = PYR_CUS / a.batch;
     pyr_plan_parts(a, n, want < 3 ? 1 : want);
+    cs->parts = a.nParts;
   }
   // pass B's LDS: from the largest samples seen at every level, or all there is.
   // What a part needs is what lets several workgroups share a compute unit; every
@@ -1661,6 +1673,7 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
         break;
     }
   }
+  cs->slabs = RW ? a.nSlabs : 0;
   SCN_TRY(cs->pyramid.reserve((size_t)a.batch * (size_t)maskWords + 2));
   SCN_TRY(cs->counts.reserve((size_t)a.nMasks * a.batch * a.slabs + 2));
   a.pyramid = cs->pyramid.p;
@@ -1703,6 +1716,7 @@ int scn_chain_flush(scn_ctx *ctx) {
   recs.swap(cs->recs);
   cs->nChains += 1;
   cs->nPlans += (long long)recs.size();
+  cs->parts = cs->slabs = 0;
   ProfScope ps(ctx, SCN_K_RULES);
   scn_grids *src = recs[0].in;
   if (cs->pyramids) {

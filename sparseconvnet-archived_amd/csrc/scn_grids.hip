@@ -1612,6 +1612,7 @@ extern "C" int scn_rules_settle(scn_ctx *ctx) {
       g->lastRows = slot[0];
       g->lastBatch = g->batch;
       g->seenActive = slot[1] > g->seenActive ? slot[1] : g->seenActive;
+      g->saw(slot[1], g->batch);
       if (g->planKind == PLAN_TERMINAL) {
         g->termS = slot[3];
         g->seenWidth = slot[3] > g->seenWidth ? slot[3] : g->seenWidth;
@@ -1953,6 +1954,8 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
     nOutActive = ctx->h_pinned[1];
     out->seenRows = nSites > out->seenRows ? nSites : out->seenRows;
     out->seenActive = nOutActive > out->seenActive ? nOutActive : out->seenActive;
+    in->saw(nE, in->batch);
+    out->saw(nOutActive, in->batch);
   }
   SCN_REQUIRE(nSites < 2147483647ll, SCN_ERR_CAPACITY,
               "rules: %lld output rows do not fit 32-bit row numbers", nSites);

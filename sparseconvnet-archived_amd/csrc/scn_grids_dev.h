@@ -108,6 +108,11 @@ struct scn_grids {
   bool atOnce = false; // ... and all of its plans overflow together or not at all
   bool chained = false; // plan and rules came from a chain of recorded plans
   long long seenSample = 0; // most active sites one sample has had (chained plans)
+  long long meanSites = 0;  // active sites a sample of the last batch that is known to have had any, on average
+  void saw(long long active, int samples) {
+    if (active > 0)
+      meanSites = active / samples + 1;
+  }
   // how much of table / bits is known to be empty right now (scn_grids_clear_many)
   size_t cleanSlots = 0, cleanWords = 0;
   // Deferred counts: while pending, nActive / nSites / termS hold upper bounds

@@ -884,6 +884,13 @@ PYR_FN int pyr_cut_parts(const PyrArgs &a, const long long *n, long long most, P
   }
   return count;
 }
+// Sites of a typical sample of this batch at a level, before they are counted: as many
+// as a sample of the batch before had there (`then`), by how many the source has now
+// and had.  (Means over the samples: two batches need not be of one size.)
+PYR_FN long long pyr_typical(long long then, long long thenSource, long long nowSource, long long field) {
+  const long long n = thenSource > 0 ? then * nowSource / thenSource : then;
+  return 1 + (n < field ? n : field);
+}
 // Sets a.parts: at most `want` parts, none cheaper than it is worth (512 sites
 // or so: half a round of a workgroup's lanes).  n: null when nothing is known.
 #ifndef PYR_PART_MIN

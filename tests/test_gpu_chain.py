@@ -261,3 +261,25 @@ def test_find_on_recorded_grids(scn, ctx):
             assert scn.settle(ctx)
         # sample 0: outputs in first-touch order 0,1,4,5 (key 6), 2,6 (key 7), 11,15 (key 19); then its background row
         assert g.find([0, 0, 0, 0, 1, 1], [0, 5, 2, 15, 0, 1]).tolist() == [0, 3, 4, 7, 9, -1]
+
+
+def test_a_sample_is_shared_out_by_its_own_size_not_the_last_batch_s(scn):
+    """How many workgroups a sample is worth is planned from the sites a sample of the batch before had at each level:
+    one small drawing after a batch of forty is shared out as after a single one."""
+    layers = [("sq", 2, 1, 1), ("sq", 3, 2, 1)] * 5
+    sample = {126 * (40 + i % 5) + 40 + i: i + 1 for i in range(24)}
+    splits = []
+    for before in (1, 40):
+        ctx = scn.Context()
+        st = Stack(scn, ctx, 2, layers)
+        sizes = st.sizes(2)
+        many = [(25 * b, {k: r + 25 * b for k, r in sample.items()}) for b in range(before)]
+        st.build(many, 25 * before, sizes[0])
+        st.run(many, sizes)
+        one = [(0, dict(sample))]
+        st.build(one, 25, sizes[0])
+        got, ok = st.run_chained(one, sizes)
+        assert ok
+        st.check(got, st.oracle(one, sizes), 1)
+        splits.append(scn.chain_split(ctx))
+    assert splits[0] == splits[1] and 1 <= splits[0][0] < 24, splits
