@@ -55,7 +55,6 @@
 #define CHAIN_LDS_MAX (152 * 1024)
 // most LDS a workgroup of k_pyr_rules asks for
 #define PYR_LDS_MAX CHAIN_LDS_MAX
-#define PYR_CUS 256 // compute units: one workgroup of k_pyr_rules each
 #define CHAIN_HEADER_BYTES 512
 #define CHAIN_MIN_ARENA (16 * 1024)
 // bytes of arena per entry of the input grid (key, row, ownership mask, base)
@@ -1599,7 +1598,7 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
     for (int l = 1; l < a.nMasks; ++l)
       n[l] = pyr_typical(recs[l - 1].out->meanSites, src->meanSites, n[0], a.lv[l].volOut);
     src->saw(src->nActive, a.batch);
-    const int want = PYR_CUS / a.batch;
+    const int want = ctx->numCU / a.batch;
     pyr_plan_parts(a, n, want < 3 ? 1 : want);
     cs->parts = a.nParts;
   }
