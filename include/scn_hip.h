@@ -496,7 +496,8 @@ enum {
   SCN_K_CONV_NIN = 7, /* gather fused into the NiN contraction */
   SCN_K_PROBE = 8,    /* scn_prof_probe: what a span costs by itself */
   SCN_K_BACKWARD = 9, /* every kernel of the backward pass and the update */
-  SCN_K_COUNT = 10
+  SCN_K_NET_END = 10, /* scn_terminal_classifier; the host classes tag it with the classifier's layer */
+  SCN_K_COUNT = 11
 };
 int scn_prof_enable(scn_ctx *ctx, int on);
 /* label attached to the spans recorded from now on (e.g. the layer index) */

@@ -20,9 +20,10 @@ HEADER = os.path.join(ROOT, "include", "scn_hip.h")
 NOSIGMOID, RELU, VLEAKYRELU, LEAKYRELU, TANH, SOFTMAX, PRELU, SIGMOID = range(8)
 FP32, BF16, BF16X3, FP32_PLANES = 0, 1, 2, 3
 OK, ERR_ARG, ERR_HIP, ERR_CAPACITY, ERR_STATE = range(5)
-K_GRID_BUILD, K_RULES, K_GATHER, K_NIN, K_MAXPOOL, K_TERMINAL, K_SOFTMAX, K_CONV_NIN, K_PROBE, K_BACKWARD = range(10)
+K_GRID_BUILD, K_RULES, K_GATHER, K_NIN, K_MAXPOOL, K_TERMINAL, K_SOFTMAX, K_CONV_NIN, K_PROBE, K_BACKWARD, \
+    K_NET_END = range(11)
 KERNEL_FAMILIES = ["grid_build", "rules", "gather", "nin", "maxpool", "terminal", "softmax", "conv_nin", "probe",
-                   "backward"]
+                   "backward", "net_end"]
 
 
 class ScnError(RuntimeError):

@@ -2064,7 +2064,7 @@ extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const in
   ep.bias = d_B;
   ep.p = p;
   ep.act = SCN_SOFTMAX;
-  ProfScope prof(ctx, SCN_K_NIN);
+  ProfScope prof(ctx, SCN_K_NET_END);
   TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy};
   hipLaunchKernelGGL((k_classifier<true>), dim3(scn_ceil_div(M, CL_ROWS)), dim3(FR_THREADS), 0, ctx->stream, d_in, d_W,
                      d_probs, (long long)M, K, N, ep, ctx->d_meta ? ctx->d_meta + META_SITES : nullptr, ts);

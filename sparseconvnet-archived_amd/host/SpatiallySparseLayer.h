@@ -358,14 +358,14 @@ void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
                               SpatiallySparseBatch &batch, int nTop);
 
 // the last two layers of a test batch's forward pass and that copy in one launch,
-// where they are a terminal pooling and a classifier that it takes
+// where they are a terminal pooling and a classifier (layer `last`) that it takes
 bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseLayer *pooling,
                                SpatiallySparseLayer *classifier,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
-                               cudaMemStream &ms);
+                               cudaMemStream &ms, int last);
 
 // utilities.h
 int ipow(int base, int exp);

@@ -1053,7 +1053,7 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
-                               cudaMemStream &ms) {
+                               cudaMemStream &ms, int last) {
   auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
   if (batch.type == TRAINBATCH || batch.type == RESCALEBATCH || !n ||
       n->fn != SOFTMAX ||
@@ -1068,6 +1068,7 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   middle.sub->features.resize64(M * K, kBoundRows * K);
   output.sub->features.resize64(M * N, kBoundRows * N);
   result_room(*batch.result, M * N, ms);
+  scn_prof_tag(ms.ctx, last);
   SCN_CHECKED(scn_terminal_classifier(
       ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
       (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),

@@ -510,7 +510,7 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
     if (i + 2 == layers.size() &&
         forwardTerminalClassifier(batch, layers[i], layers[i + 1],
                                   batch.interfaces[i], batch.interfaces[i + 1],
-                                  batch.interfaces[i + 2], ms))
+                                  batch.interfaces[i + 2], ms, (int)i + 1))
       break;
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);
     if (batch.type == RESCALEBATCH) {

@@ -45,3 +45,22 @@ def test_shapes_it_does_not_take(scn, ctx):
     for M, K, N in ((0, 64, 100), (513, 64, 100), (8, 1028, 100), (8, 66, 100), (8, 64, 10), (8, 64, 132), (8, 64, 96)):
         assert not lib.scn_terminal_classifier_supported(M, K, N)
         assert lib.scn_terminal_classifier(ctx.h, None, None, M, 1, None, None, None, None, None, K, N, 1.0) != 0
+
+
+def test_the_last_launch_has_a_row_of_its_own_in_a_profile(scn):
+    """a net's spans by family and layer: the terminal pooling and the classifier in one, under the classifier"""
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    cfg = synthetic.config(2, batch=3)
+    net = hostapi.Net(cfg.dimension, cfg.nInputFeatures, cfg.nClasses, threads=1)
+    cfg.build(net)
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TESTBATCH)
+    for pts, f, label in synthetic.make_samples(cfg, 5):
+        ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
+    c = scn.Context(handle=net.context_handle())
+    c.prof_enable(True)
+    net.begin(ds, cfg.batch)
+    assert net.next_batch()
+    net.end()
+    rows = [(fam, tag) for fam, tag, _ in c.prof_spans() if tag >= len(net.layers()) - 2]
+    c.prof_enable(False)
+    assert net.layers()[-2]["kind"] == "terminal" and rows == [("net_end", len(net.layers()) - 1)], rows
