@@ -384,10 +384,10 @@ def measure(scn, hostapi, synthetic, args, number, precision, headline):
                            launches_per_step=r_launches, bound="hbm", achieved=round(a, 3), peak=HBM_PEAK_GBS,
                            unit="GB/s", frac=round(a / HBM_PEAK_GBS, 5), algorithmic_bytes=int(r_bytes), traffic=None)
         if r_launches <= 2.5:
-            rules_entry["note"] = ("every layer's rule book in two launches, one workgroup per sample: all layers' "
-                                   "occupancy masks by dilation, then owners, rows and rule rows per output site "
-                                   "in LDS; integer work bound by instruction issue on one compute unit per sample, "
-                                   "the HBM roofline is far from binding")
+            rules_entry["note"] = ("every layer's rule book in two launches: all layers' occupancy masks from the "
+                                   "source's, a wavefront a sample, layer and slab; then owners, rows and rule rows per "
+                                   "output site in LDS, one workgroup a sample or, for few samples, several; integer "
+                                   "work bound by instruction issue, the HBM roofline is far from binding")
         else:
             rules_entry["note"] = ("layer by layer through masks, rank prefixes and rows by rank in HBM: a dozen "
                                    "launches per layer; the rule rows themselves leave at 4-6 TB/s")

@@ -1030,10 +1030,7 @@ int TerminalPoolingLayer::calculateInputSpatialSize(int outputSpatialSize) {
   return inSpatialSize;
 }
 
-// ---- SoftmaxClassifier (SoftmaxClassifier.cu:16-58) ---------------------------
-// In two halves, so that a caller may queue the next batch's forward pass
-// between them: the copy of the probabilities to the host is only queued
-// (SoftmaxClassifier.cu:24, copyToCPUAsync), the statistics are computed once
+// ---- the end of a net ---------------------------------------------------------
 // pinned memory for the probabilities of a batch
 static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream) {
   if (n <= r.capacity)
@@ -1080,6 +1077,10 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   return true;
 }
 
+// ---- SoftmaxClassifier (SoftmaxClassifier.cu:16-58) ---------------------------
+// In two halves, so that a caller may queue the next batch's forward pass
+// between them: the copy of the probabilities to the host is only queued
+// (SoftmaxClassifier.cu:24, copyToCPUAsync), the statistics are computed once
 // it has arrived (:27 onwards).
 void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
                              SpatiallySparseBatch &batch,
