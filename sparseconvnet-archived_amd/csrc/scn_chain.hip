@@ -43,7 +43,7 @@
 // recorded layers get their entry lists, backgroundCol and counts; their hash
 // tables and masks are only built if somebody asks (ensure_index).
 #include "scn_grids_dev.h"
-#include "scn_pyr_dev.h"
+#include "scn_pyr_body.h"
 #include <stdlib.h>
 #include <string.h>
 
@@ -803,7 +803,7 @@ __global__ void __launch_bounds__(PLACE_THREADS) k_chain_place(ChainArgs a) {
 
 // ------------------------------------------------ chains built from the output side
 //
-// scn_pyr_dev.h has the per-lane bodies; here are the two kernels around them.
+// scn_pyr_body.h and scn_pyr_dev.h have what they do; here they are launched.
 // Pass A: the occupancy masks of all layers and the sample's site counts, left
 // in global memory.  k_pyr_levels makes each layer's mask from the source's rows
 // (the windows of all layers before it taken together), so that its wavefronts do
@@ -826,403 +826,68 @@ __global__ void __launch_bounds__(PLACE_THREADS) k_chain_place(ChainArgs a) {
 // barrier to pass and gave no wrong word in any run; it costs a 126 x 126 field
 // about 2 us and a 47^3 one about 20.
 #define PYR_A_THREADS 64
-#define PYR_A_BARRIER() lds_barrier()
 #define PYR_B_THREADS 1024
 static_assert(sizeof(PyrArgs) <= 4096, "kernel arguments");
 
-// A layer's geometry as k_pyr_masks keeps it in LDS: one broadcast read a layer
-// instead of trips to the kernel arguments
-struct PyrGeoA {
-  int nIn, nOut, size, stride;
-  int words, offIn, offOut;
-  unsigned magicN, seg, segs, magicSegs;
-  int pad;
+static_assert(PYR_META_SITES == META_SITES && PYR_META_ACTIVE == META_ACTIVE && PYR_META_OVERFLOW == META_OVERFLOW &&
+                  PYR_META_WIDTH == META_WIDTH,
+              "meta words");
+
+// The executor of scn_pyr_body.h: the workgroup itself, a lane's values in its
+// registers
+template <int THREADS> struct PyrWorkgroup {
+  static constexpr int T = THREADS;
+  template <typename V> struct Lane {
+    V v;
+    __device__ __forceinline__ V &operator[](int) { return v; }
+    __device__ __forceinline__ const V &operator[](int) const { return v; }
+  };
+  template <typename V> using Wave = Lane<V>;
+  static __device__ __forceinline__ int lane() { return threadIdx.x & 63; }
+  __device__ __forceinline__ int threads() const { return THREADS; }
+  template <typename F> __device__ __forceinline__ void lanes(F f) const { f((int)threadIdx.x); }
+  template <typename F> __device__ __forceinline__ void waves(int n, F f) const {
+    for (int i = (int)threadIdx.x >> 6; i < n; i += THREADS / 64)
+      f(i);
+  }
+  template <typename F> __device__ __forceinline__ void wave(F f) const { f(lane()); }
+  template <typename F> __device__ __forceinline__ unsigned sum(F f) const {
+    return wave_last(wave_scan_incl_dpp(f(lane())));
+  }
+  template <typename F> __device__ __forceinline__ int max(F f) const {
+    return (int)wave_last((unsigned)wave_max_dpp(f(lane())));
+  }
+  template <typename F> __device__ __forceinline__ Wave<unsigned> scan(F f) const {
+    return {wave_scan_incl_dpp(f(lane()))};
+  }
+  template <typename F> __device__ __forceinline__ int count(F f) const { return __popcll(__ballot(f(lane()))); }
+  template <typename V> __device__ __forceinline__ int at(const Wave<V> &w, int lane) const {
+    return __builtin_amdgcn_readlane((int)w.v, lane);
+  }
+  __device__ __forceinline__ int uniform(int x) const { return __builtin_amdgcn_readfirstlane(x); }
+  __device__ __forceinline__ void sync() const { lds_barrier(); }
+  __device__ __forceinline__ int row(const PyrArgs &a, long long p) const {
+    return a.dense ? a.dense[p] : hash_find(reinterpret_cast<const Slot *>(a.table), a.shift, a.mask, p);
+  }
+  __device__ __forceinline__ void check(bool) const {}
+  __device__ __forceinline__ void window() const {}
 };
-static_assert(sizeof(PyrGeoA) == 48, "three 16-byte reads");
-#define PYR_A_GEO ((PYR_MAX_LEVELS + 1) * (int)sizeof(PyrGeoA)) // geometry: after the masks
 
-template <int D>
-__global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
+template <int D> __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_masks(PyrArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  pyr_u64 *masks = reinterpret_cast<pyr_u64 *>(lds);
-  PyrGeoA *geo = reinterpret_cast<PyrGeoA *>(lds + (8ll * a.maskWords + 15) / 16 * 16);
-  int *const counts = a.counts + (long long)blockIdx.x * a.slabs; // (slabs: 1)
-  const int b = blockIdx.x, t = threadIdx.x;
-  static_assert(PYR_A_THREADS == 64, "one wavefront: the levels below pass no barrier");
-  if (t >= 1 && t < a.nMasks) {
-    const PyrLevel &L = a.lv[t];
-    PyrGeoA g;
-    g.nIn = L.nIn;
-    g.nOut = L.nOut;
-    g.size = L.size;
-    g.stride = L.stride;
-    g.words = L.words;
-    g.offIn = a.lv[t - 1].maskOff;
-    g.offOut = L.maskOff;
-    g.magicN = L.magicN;
-    g.seg = L.seg;
-    g.segs = L.segs;
-    g.magicSegs = L.magicSegs;
-    g.pad = 0;
-    geo[t] = g;
-  }
-  { // level 0: the sample's slice of the source mask, four words a lane at a time
-    const PyrLevel &L = a.lv[0];
-    const int words = L.words;
-    const long long vol = L.volOut;
-    unsigned n = 0;
-    for (int w0 = 0; w0 < words + 2; w0 += 256) {
-      pyr_u64 v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int w = w0 + 64 * u + t;
-        v[u] = w < words ? pyr_source_word(a.bits, vol, b, (unsigned)w) : 0ull;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int w = w0 + 64 * u + t;
-        n += (unsigned)pyr_popc64(v[u]);
-        if (w < words + 2)
-          masks[w] = v[u];
-      }
-    }
-    n = wave_last(wave_scan_incl_dpp(n));
-    if (t == 0)
-      counts[0] = (int)n;
-    // the other levels start empty: their pieces are OR-ed in
-    for (int w = words + 2 + t; w < a.maskWords; w += PYR_A_THREADS)
-      masks[w] = 0ull;
-  }
-  PYR_A_BARRIER();
-  for (int x = 1; x < a.nMasks; ++x) {
-    // (wavefront-uniform values, told to the compiler: the loops over a window's
-    // rows then branch on scalars)
-    PyrGeoA g = geo[x];
-    g.nIn = __builtin_amdgcn_readfirstlane(g.nIn);
-    g.nOut = __builtin_amdgcn_readfirstlane(g.nOut);
-    g.size = __builtin_amdgcn_readfirstlane(g.size);
-    g.stride = __builtin_amdgcn_readfirstlane(g.stride);
-    g.words = __builtin_amdgcn_readfirstlane(g.words);
-    g.offIn = __builtin_amdgcn_readfirstlane(g.offIn);
-    g.offOut = __builtin_amdgcn_readfirstlane(g.offOut);
-    g.magicN = (unsigned)__builtin_amdgcn_readfirstlane((int)g.magicN);
-    g.seg = (unsigned)__builtin_amdgcn_readfirstlane((int)g.seg);
-    g.segs = (unsigned)__builtin_amdgcn_readfirstlane((int)g.segs);
-    g.magicSegs = (unsigned)__builtin_amdgcn_readfirstlane((int)g.magicSegs);
-    pyr_sweep_dilate<D>(masks + g.offIn, masks + g.offOut, g.nIn, g.nOut, g.size, g.stride, g.magicN, g.seg, g.segs,
-                        g.magicSegs, t, PYR_A_THREADS);
-    PYR_A_BARRIER();
-    unsigned n = 0;
-    for (int w = t; w < g.words; w += 64)
-      n += (unsigned)pyr_popc64(masks[g.offOut + w]);
-    n = wave_last(wave_scan_incl_dpp(n));
-    if (t == 0)
-      counts[(long long)x * a.batch * a.slabs] = (int)n;
-  }
-  pyr_u64 *dst = a.pyramid + (long long)b * a.maskWords;
-  for (int i = t; i < a.maskWords; i += PYR_A_THREADS)
-    dst[i] = masks[i];
+  PyrWorkgroup<PYR_A_THREADS> e;
+  pyr_masks_body<D>(e, a, lds, blockIdx.x);
 }
-
-// Pass A with a wavefront per (sample, level, slab): blockIdx.x the sample, .y the
-// level and slab.
-template <int D, int RW>
-__global__ void __launch_bounds__(64) k_pyr_levels(PyrArgs a) {
+// blockIdx.x the sample, .y the level and slab
+template <int D, int RW> __global__ void __launch_bounds__(PYR_A_THREADS) k_pyr_levels(PyrArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int b = blockIdx.x, x = a.slabLevel[blockIdx.y], slab = a.slabOf[blockIdx.y], t = threadIdx.x;
-  const PyrLevel &L = a.lv[x];
-  const int nOut = L.nOut, n0 = a.lv[0].nOut;
-  const long long vol0 = a.lv[0].volOut;
-  int *const count = a.counts + ((long long)x * a.batch + b) * a.slabs + slab;
-  const PyrSlab z = pyr_slab(D, L, L.magicN, slab, pyr_slabs(D, n0, L, a.slabs));
-  const int words = z.w1 - z.w0;
-  pyr_u64 *const out = a.pyramid + (long long)b * a.maskWords + L.maskOff + z.w0;
-  pyr_u64 *const rows = reinterpret_cast<pyr_u64 *>(lds);
-  const int plane = D == 3 ? n0 : 1;
-  const bool deep = D == 3 && L.foldW > PYR_FOLD_DIRECT;
-  pyr_u64 *const mid = rows + RW * plane * (z.p1 - z.p0);
-  pyr_u64 *const mask = mid + (deep ? RW * (z.p1 - z.p0) * nOut : 0);
-  if (x > 0) {
-    for (int w = t; w < words; w += 64)
-      mask[w] = 0ull;
-    pyr_sweep_stage<RW>(a.bits, (long long)b * vol0 + (long long)z.p0 * plane * n0, n0, plane * (z.p1 - z.p0), rows, t,
-                        64);
-    PYR_A_BARRIER();
-    if (deep) {
-      pyr_sweep_mid<RW>(rows, mid, z.p1 - z.p0, n0, nOut, L.magicN, L.foldW, L.foldS, t, 64);
-      PYR_A_BARRIER();
-    }
-    pyr_sweep_fold<D, RW>(rows, mid, mask, z, n0, nOut, L.magicN, L.foldW, L.foldS, t, 64);
-    PYR_A_BARRIER();
-  }
-  unsigned n = 0;
-#pragma unroll 4
-  for (int w = t; w < words; w += 64) {
-    const pyr_u64 v = x > 0 ? mask[w] : pyr_source_word(a.bits, vol0, b, (unsigned)(z.w0 + w));
-    n += (unsigned)pyr_popc64(v);
-    out[w] = v;
-  }
-  if (z.w1 == L.words && t < 2) // (two spare words)
-    out[words + t] = 0ull;
-  n = wave_last(wave_scan_incl_dpp(n));
-  if (t == 0)
-    *count = (int)n;
+  PyrWorkgroup<PYR_A_THREADS> e;
+  pyr_levels_body<D, RW>(e, a, lds, blockIdx.x, blockIdx.y);
 }
-
-template <int D>
-__global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
+template <int D> __global__ void __launch_bounds__(PYR_B_THREADS) k_pyr_rules(PyrArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  PyrHdr *h = reinterpret_cast<PyrHdr *>(lds);
-  // (the last workgroup has no sample: it reports the counts to the host)
-  const bool reports = blockIdx.x == (unsigned)(a.batch * a.nParts);
-  const int b = reports ? 0 : blockIdx.x % a.batch, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const PyrPart part = a.parts[reports ? 0 : blockIdx.x / a.batch];
-  constexpr int T = PYR_B_THREADS;
-  // lane t keeps layer t's arguments from here on: fetched while the masks
-  // come in, not when the level table wants them
-  PyrLevel mine;
-  int inMaskOff = 0;
-  const int bgSource = a.bg[b];
-  if (t <= a.nLevels) {
-    mine = a.lv[t];
-    inMaskOff = a.lv[t > 0 ? t - 1 : 0].maskOff;
-  }
-  if (t == 0) {
-    h->over = 0;
-    h->cut = part.F > 1;
-    h->emitFrom = part.la;
-    h->slab = part.f;
-    h->plane[0] = part.f ? a.lv[part.la].nOut : 0;
-    h->plane[1] = a.lv[part.la].nOut;
-  }
-  if (t < a.nMasks) {
-    h->before[t] = 0;
-    h->words[t] = mine.words + 2;
-    h->maskOff[t] = mine.maskOff;
-  }
-  // the masks of the part's levels and of the two before it
-  const int xFirst = part.la >= 3 ? part.la - 2 : 0, xLast = part.lb;
-  pyr_u64 *const masks = reinterpret_cast<pyr_u64 *>(lds + PYR_HDR_BYTES);
-  unsigned short *const pref = reinterpret_cast<unsigned short *>(masks + a.maskWords);
-  {
-    const pyr_u64 *src = a.pyramid + (long long)b * a.maskWords;
-    const int end = xLast + 1 < a.nMasks ? a.lv[xLast + 1].maskOff : a.maskWords;
-    for (int i = a.lv[xFirst].maskOff + t; i < end; i += T)
-      masks[i] = src[i];
-  }
-  // sums over the samples, a wavefront per level
-  for (int x = wave; x < a.nMasks; x += T / 64) {
-    const int *cnt = a.counts + (long long)x * a.batch * a.slabs;
-    const long long full = a.lv[x].fullSize;
-    const int slabs = a.slabs == 1 ? 1 : pyr_slabs(a.d, a.lv[0].nOut, a.lv[x], a.slabs);
-    // (a batch's rows are numbered in 32 bits, so these sums fit)
-    unsigned v0 = 0, v1 = 0, v2 = 0, v3 = 0, own = 0;
-    int mx = 0;
-    for (int s = lane; s < a.batch; s += 64) {
-      int n = 0;
-      for (int z = 0; z < slabs; ++z)
-        n += cnt[s * a.slabs + z];
-      const int hb = n < full;
-      if (s < b) {
-        v0 += n;
-        v1 += hb;
-      }
-      own = s == b ? n : own;
-      v2 += n;
-      v3 += hb;
-      mx = n > mx ? n : mx;
-    }
-    v0 = wave_last(wave_scan_incl_dpp(v0));
-    v1 = wave_last(wave_scan_incl_dpp(v1));
-    v2 = wave_last(wave_scan_incl_dpp(v2));
-    v3 = wave_last(wave_scan_incl_dpp(v3));
-    own = wave_last(wave_scan_incl_dpp(own));
-    mx = (int)wave_last((unsigned)wave_max_dpp(mx));
-    if (lane == 0) {
-      h->n[x] = (int)own;
-      h->hasBg[x] = (int)own < full;
-      h->actBefore[x] = v0;
-      h->bgBefore[x] = v1;
-      h->actAll[x] = v2;
-      h->bgAll[x] = v3;
-      h->maxAct[x] = mx;
-    }
-  }
-  lds_barrier();
-  if (t >= 1 && t <= a.nLevels && pyr_report(a, mine, h, t).over)
-    atomicOr(&h->over, 1);
-  // (a sample that does not fit: the whole batch is planned another way.  The
-  // largest counts of two levels need not be one sample's: they only say whether
-  // the samples have to be asked)
-  if (t < a.nMasks && (h->maxAct[t] > PYR_ROWS_MAX ||
-                       !pyr_pair_fits(a, h->maxAct[t], t + 1 < a.nMasks ? h->maxAct[t + 1] : 0)))
-    atomicOr(&h->over, 4);
-  // rank prefixes, a wavefront per chunk of 256 words of a level: within the
-  // chunk now, what lies before it once the chunks' sums are there
-  unsigned *const sums = reinterpret_cast<unsigned *>(lds + PYR_HDR_BYTES + 8ll * a.pyrStride);
-  for (int i = wave; i < a.nChunks; i += T / 64) {
-    const int x = a.chunkLevel[i];
-    if (x < xFirst || x > xLast)
-      continue;
-    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * a.chunkOf[i] + 4 * lane;
-    unsigned pc[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      pc[u] = w0 + u < words ? (unsigned)pyr_popc64(masks[at + w0 + u]) : 0u;
-    const unsigned four = pc[0] + pc[1] + pc[2] + pc[3];
-    const unsigned incl = wave_scan_incl_dpp(four);
-    unsigned run = incl - four;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (w0 + u < words)
-        pref[at + w0 + u] = (unsigned short)run;
-      run += pc[u];
-    }
-    if (lane == 63)
-      sums[i] = incl;
-  }
-  lds_barrier();
-  for (int i = wave; i < a.nChunks; i += T / 64) {
-    const int x = a.chunkLevel[i], c = a.chunkOf[i];
-    if (c == 0 || x < xFirst || x > xLast)
-      continue;
-    unsigned before = 0;
-    for (int k = lane; k < c; k += 64)
-      before += sums[i - c + k];
-    before = wave_last(wave_scan_incl_dpp(before));
-    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * c + 4 * lane;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (w0 + u < words)
-        pref[at + w0 + u] = (unsigned short)(pref[at + w0 + u] + before);
-  }
-  if (h->over & 4) {
-    for (int sample = t; sample < a.batch; sample += T) {
-      const int *c = a.counts + (long long)sample * a.slabs;
-      auto sites = [&](int x) {
-        int n = 0;
-        for (int z = 0; z < pyr_slabs(a.d, a.lv[0].nOut, a.lv[x], a.slabs); ++z)
-          n += c[(long long)x * a.batch * a.slabs + z];
-        return n;
-      };
-      bool fits = pyr_fits_of(a, sites);
-      for (int x = 0; x < a.nMasks; ++x)
-        fits = fits && sites(x) <= PYR_ROWS_MAX;
-      if (!fits)
-        atomicOr(&h->over, 2);
-    }
-  }
-  lds_barrier();
-  const bool over = (h->over & 3) != 0;
-  if (reports && t >= 1 && t <= a.nLevels) {
-    const PyrLevel &L = mine;
-    const PyrReport r = pyr_report(a, mine, h, t);
-    L.meta[META_SITES] = over ? 0 : r.nSites;
-    L.meta[META_ACTIVE] = over ? 0 : r.nActive;
-    L.meta[META_OVERFLOW] = over;
-    L.meta[META_WIDTH] = L.kind == PYR_TERMINAL ? r.extra : 0;
-    volatile long long *slot = a.scalars + 16 + 4 * L.slot;
-    slot[0] = r.nSites;
-    slot[1] = r.nActive;
-    slot[2] = over;
-    slot[3] = r.extra;
-  }
-  if (reports && t == 0) {
-    a.scalars[15] = *a.badSites;
-    a.scalars[13] = h->maxAct[0];
-  }
-  if (over || reports)
-    return;
-  if (part.F > 1) {
-    const PyrLds all = pyr_lds_view(a, lds, 0, 0);
-    pyr_sweep_planes(a, all, part, t, T);
-    lds_barrier();
-    pyr_fill_cut(a, all, part, t);
-    lds_barrier();
-    if (t == 0)
-      pyr_fix_cut(h, part);
-    lds_barrier();
-  }
-  // the part's layers a window of levels at a time: as many as the LDS holds (all
-  // of them, for all but the largest samples); the rows of the layer before the
-  // first of them are worked out here once more
-  for (int xa = part.la >= 3 ? part.la - 2 : 0;;) {
-    // (pyr_window_end and pyr_fill_offsets, a lane a level: every wavefront by itself)
-    const int levelSites = lane >= xa && lane <= part.lb ? pyr_held(h, lane) : 0;
-    const int sitesTo = (int)wave_scan_incl_dpp((unsigned)levelSites);
-    const int firstSites = __builtin_amdgcn_readlane(levelSites, xa);
-    const long long room = a.ldsBytesB - (PYR_HDR_BYTES + 8ll * a.pyrStride + 4ll * firstSites + 6 * 16);
-    const int fit = __popcll(__ballot(lane > xa + 1 && lane <= part.lb && 11ll * sitesTo <= room));
-    const int xb = xa < part.lb ? xa + 1 + fit : xa;
-    const int la = xa + 1, lb = xb;
-    const bool last = xb == part.lb;
-    if (t >= xa && t <= xb + 1) {
-      const int sum = sitesTo - levelSites;
-      h->siteOff[t] = sum;
-      h->itemOff[t] = t > xa ? sum - firstSites : 0;
-      if (t == xb + 1)
-        h->total = sum;
-    }
-    lds_barrier();
-    if (t < a.nMasks)
-      pyr_fill_en(mine, lds, t, h->siteOff[t]);
-    const PyrLds s = pyr_lds_view(a, lds, h->total, pyr_held(h, xa));
-    if ((t >= la && t <= lb) || (last && lb == a.nMasks - 1 && t == a.nLevels && t > lb))
-      pyr_fill_level(mine, inMaskOff, bgSource, s, t, xa);
-    pyr_sweep_clear(s, t, T);
-    lds_barrier();
-    pyr_sweep_enumerate<D>(a, s, xa, xb, t, T);
-    lds_barrier();
-    if (xa == 0 && part.la == 1) { // the batch's rows of the source's sites: their loads go out first
-      const PyrLevel &L = a.lv[0];
-      const long long p0 = (long long)b * L.volOut;
-      const Slot *table = reinterpret_cast<const Slot *>(a.table);
-      for (int r = t; r < pyr_held(h, 0); r += T) {
-        int c[D];
-        pyr_unpack<D>(s.key[r], c);
-        long long p = p0 + pyr_key<D>(c, L.nOut);
-        p = p < (long long)a.batch * L.volOut ? p : 0; // (a mask never has a site beyond the field)
-        s.srcRow[r] = (unsigned)(a.dense ? a.dense[p] : hash_find(table, a.shift, a.mask, p));
-      }
-    }
-    pyr_sweep_owners<D>(s, la, lb, t, T);
-    lds_barrier();
-    // rows owned by the sites before, a wavefront per level
-    for (int x = xa + wave; x < xb; x += T / 64) {
-      const int from = h->cut ? h->own[x] : 0;
-      const int n = (h->cut ? h->ownEnd[x] : h->n[x]) - from;
-      const unsigned off = (unsigned)(h->siteOff[x] + from - pyr_lo(h, x));
-      unsigned carry = (unsigned)pyr_base_start(h, x);
-      for (int r0 = 0; r0 < n; r0 += 256) { // (four sites a lane: the chain of sums is what this takes)
-        const int r = r0 + 4 * lane;
-        unsigned v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          v[u] = r + u < n ? (unsigned)pyr_popc32(pyr_own_mask(s, off + r + u)) : 0u;
-        const unsigned four = v[0] + v[1] + v[2] + v[3];
-        const unsigned incl = wave_scan_incl_dpp(four);
-        unsigned run = carry + incl - four;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (r + u < n)
-            s.base[off + r + u] = (unsigned short)run;
-          run += v[u];
-        }
-        carry += wave_last(incl);
-      }
-    }
-    lds_barrier();
-    pyr_sweep_rows<D>(s, la, lb, b, t, T);
-    lds_barrier();
-    pyr_sweep_rules<D>(s, la, lb, t, T);
-    pyr_sweep_tail(a, s, la, lb, b, t, T);
-    if (last)
-      break;
-    lds_barrier();
-    pyr_sweep_carry(s, lds, a, xb, t, T);
-    lds_barrier();
-    xa = xb;
-  }
+  PyrWorkgroup<PYR_B_THREADS> e;
+  pyr_rules_body<D>(e, a, lds, blockIdx.x);
 }
 
 // -------------------------------------------------------------------- host
@@ -1533,36 +1198,13 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   a.nLevels = (int)recs.size();
   a.batch = src->batch;
   a.d = d;
-  auto magic = [](long long x) { return (unsigned)((1ull << 32) / (unsigned long long)(x > 0 ? x : 1) + 1); };
-  long long maskWords = 0;
-  {
-    PyrLevel &L = a.lv[0];
-    L.kind = PYR_REGIONS;
-    L.nIn = L.nOut = src->n;
-    L.size = L.stride = L.width = 1;
-    L.volOut = src->vol;
-    L.fullSize = src->vol + 1; // (the source's background rows are the caller's)
-    L.words = (int)((src->vol + 63) / 64);
-    L.maskOff = 0;
-    L.magicN = magic(src->n);
-    L.magicS = magic(1);
-    maskWords = L.words + 2;
-  }
-  a.nMasks = 1;
+  // (the source's background rows are the caller's: no count of sites is a full one)
+  pyr_add_level(a, 0, PYR_REGIONS, src->n, src->n, 1, 1, 1, src->vol, src->vol + 1);
   for (int l = 1; l <= a.nLevels; ++l) {
     const ChainRec &r = recs[l - 1];
+    pyr_add_level(a, l, r.lv.kind == CH_TERMINAL ? PYR_TERMINAL : PYR_REGIONS, r.lv.nIn, r.lv.nOut, r.lv.size,
+                  r.lv.stride, r.lv.width, r.geom.volOut, r.lv.fullSize);
     PyrLevel &L = a.lv[l];
-    L.kind = r.lv.kind == CH_TERMINAL ? PYR_TERMINAL : PYR_REGIONS;
-    L.nIn = r.lv.nIn;
-    L.nOut = r.lv.nOut;
-    L.size = r.lv.size;
-    L.stride = r.lv.stride;
-    L.width = r.lv.width;
-    L.volOut = r.geom.volOut;
-    L.fullSize = r.lv.fullSize;
-    L.magicN = magic(L.nOut);
-    L.magicS = magic(L.size);
-    pyr_set_pieces(L);
     L.rules = r.lv.rules;
     L.capacity = r.lv.capacity;
     L.ekey = r.lv.ekey;
@@ -1572,20 +1214,9 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
     L.boundRows = r.lv.boundRows;
     L.boundActive = r.lv.boundActive;
     L.slot = r.lv.slot;
-    if (L.kind == PYR_REGIONS) {
-      L.words = (int)((L.volOut + 63) / 64);
-      L.maskOff = (int)maskWords;
-      maskWords += L.words + 2;
-      a.nMasks = l + 1;
-    }
   }
-  long long pyrStride = maskWords + (maskWords + 3) / 4;
-  pyrStride = (pyrStride + 1) / 2 * 2;
-  const long long fixedB = PYR_HDR_BYTES + 8 * pyrStride + 6 * 16;
-  if (fixedB + CHAIN_MIN_ARENA > PYR_LDS_MAX || !pyr_set_chunks(a))
+  if (!pyr_set_layout(a) || pyr_fixed_lds(a) + CHAIN_MIN_ARENA > PYR_LDS_MAX)
     return SCN_OK;
-  a.maskWords = (int)maskWords;
-  a.pyrStride = (int)pyrStride;
   {
     // A workgroup of pass B has a compute unit to itself (sixteen wavefronts of 82
     // registers) and issues what there is to issue: a batch of few samples leaves
@@ -1615,20 +1246,7 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
       known = known && seen > 0;
       n[x] = seen + seen / 2 + 64;
     }
-    long long need = 4 * a.nChunks; // (the sums of the prefixes' chunks)
-    for (int x = 0; x < a.nMasks; ++x) {
-      const long long pair = 15 * n[x] + (x + 1 < a.nMasks ? 11 * n[x + 1] : 0);
-      need = pair > need ? pair : need;
-    }
-    for (int p = 0; p < a.nParts; ++p) {
-      const PyrPart &part = a.parts[p];
-      const int xa = part.la >= 3 ? part.la - 2 : 0;
-      long long sites = 4 * n[xa];
-      for (int x = xa; x <= part.lb; ++x)
-        sites += 11 * (part.F > 1 ? n[x] / part.F + n[x] / (2 * part.F) + 64 : n[x]);
-      need = sites > need ? sites : need;
-    }
-    need += fixedB;
+    const long long need = pyr_rules_lds(a, n);
     ldsB = known && need < ldsB ? need : ldsB;
   }
   ldsB = (ldsB + 15) / 16 * 16;
@@ -1649,31 +1267,9 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   // rows, where those are short enough for registers; else one per sample, level
   // after level
   const int RW = pyr_set_fold(a);
-  long long wordsA = (8 * maskWords + 15) / 16 * 2 + PYR_A_GEO / 8;
-  a.slabs = 1;
-  if (RW) {
-    // (at most 8: 12 us for 33 samples of 47^3; a wavefront a level: 27)
-    for (int most = a.batch < 64 ? 8 : a.batch < 512 ? 512 / a.batch : 1;; most /= 2) {
-      a.slabs = most;
-      a.nSlabs = 0;
-      wordsA = 0;
-      for (int x = 0; x < a.nMasks; ++x) {
-        const int slabs = pyr_slabs(d, src->n, a.lv[x], most);
-        for (int z = 0; z < slabs; ++z, ++a.nSlabs) {
-          if (a.nSlabs < PYR_MAX_SLABS) {
-            a.slabLevel[a.nSlabs] = (unsigned char)x;
-            a.slabOf[a.nSlabs] = (unsigned char)z;
-          }
-          const long long words = pyr_slab_words(d, RW, src->n, a.lv[x], pyr_slab(d, a.lv[x], a.lv[x].magicN, z, slabs));
-          wordsA = x > 0 && words > wordsA ? words : wordsA;
-        }
-      }
-      if (a.nSlabs <= PYR_MAX_SLABS)
-        break;
-    }
-  }
+  const long long wordsA = RW ? pyr_plan_slabs(a, RW) : pyr_plan_whole(a);
   cs->slabs = RW ? a.nSlabs : 0;
-  SCN_TRY(cs->pyramid.reserve((size_t)a.batch * (size_t)maskWords + 2));
+  SCN_TRY(cs->pyramid.reserve((size_t)a.batch * (size_t)a.maskWords + 2));
   SCN_TRY(cs->counts.reserve((size_t)a.nMasks * a.batch * a.slabs + 2));
   a.pyramid = cs->pyramid.p;
   a.counts = cs->counts.p;

@@ -24,10 +24,11 @@
 //           (a later candidate is an earlier output); and the rule rows, which
 //           look the input sites' rows up by rank.
 //
-// The code below is the per-lane body of every sweep.  It is written against
-// plain pointers ("lds" is just memory) so that the same text compiles for the
-// device (scn_chain.hip) and for the host, where a harness runs the lanes one
-// after the other with the barriers between sweeps (tests/chain_cpu_harness.cpp).
+// The code below is the per-lane body of every sweep, and what the planning works
+// out from a chain's geometry.  It is written against plain pointers ("lds" is just
+// memory); scn_pyr_body.h puts the sweeps together to kernels.  The same text
+// compiles for the device (scn_chain.hip) and for the host, where a harness runs the
+// lanes one after the other (tests/chain_cpu_harness.cpp).
 #pragma once
 #include <stdint.h>
 #include <type_traits>
@@ -118,6 +119,7 @@ PYR_FN unsigned pyr_mulhi(unsigned a, unsigned b) {
 PYR_FN unsigned pyr_div(unsigned x, unsigned d, unsigned magic) {
   return d == 1 ? x : pyr_mulhi(x, magic);
 }
+PYR_FN unsigned pyr_magic(long long d) { return (unsigned)((1ull << 32) / (pyr_u64)(d > 0 ? d : 1) + 1); }
 PYR_FN pyr_u64 pyr_even_bits(pyr_u64 x) {
   x &= 0x5555555555555555ull;
   x = (x | (x >> 1)) & 0x3333333333333333ull;
@@ -212,7 +214,32 @@ PYR_FN unsigned pyr_seg(int size, int stride) {
 PYR_FN void pyr_set_pieces(PyrLevel &L) {
   L.seg = pyr_seg(L.size, L.stride);
   L.segs = ((unsigned)L.nOut + L.seg - 1u) / L.seg;
-  L.magicSegs = (unsigned)((1ull << 32) / (L.segs > 0 ? L.segs : 1u) + 1ull);
+  L.magicSegs = pyr_magic(L.segs);
+}
+// Level l of a chain (the levels in order, the terminal layer, which has no mask,
+// last): its geometry and where its mask lies
+PYR_FN void pyr_add_level(PyrArgs &a, int l, int kind, int nIn, int nOut, int size, int stride, int width,
+                          long long volOut, long long fullSize) {
+  PyrLevel &L = a.lv[l];
+  L.kind = kind;
+  L.nIn = nIn;
+  L.nOut = nOut;
+  L.size = size;
+  L.stride = stride;
+  L.width = width;
+  L.volOut = volOut;
+  L.fullSize = fullSize;
+  L.magicN = pyr_magic(nOut);
+  L.magicS = pyr_magic(size);
+  pyr_set_pieces(L);
+  if (l == 0)
+    a.maskWords = 0;
+  if (kind == PYR_REGIONS) {
+    L.words = (int)((volOut + 63) / 64);
+    L.maskOff = a.maskWords;
+    a.maskWords += L.words + 2;
+    a.nMasks = l + 1;
+  }
 }
 #if defined(__HIPCC__) && defined(__HIP_DEVICE_COMPILE__)
 #define PYR_ATOMIC_OR64(ptr, v) atomicOr(reinterpret_cast<unsigned long long *>(ptr), (unsigned long long)(v))
@@ -465,13 +492,41 @@ PYR_FN long long pyr_slab_words(int d, int RW, int n0, const PyrLevel &L, const 
 }
 // How many slabs a level is worth, of `most`: the rows that a wavefront fetches and
 // makes set the pace, 512 of each or so
+#ifndef PYR_SLAB_ROWS
+#define PYR_SLAB_ROWS 512
+#endif
 PYR_FN int pyr_slabs(int d, int n0, const PyrLevel &L, int most) {
   const int rows = d == 3 ? n0 * n0 : n0, own = d == 3 ? L.nOut : 4 * L.nOut;
-  int n = (rows + 511) / 512;
+  int n = (rows + PYR_SLAB_ROWS - 1) / PYR_SLAB_ROWS;
   n = n < own / 4 ? n : own / 4; // (a few planes each)
   n = n < L.words ? n : L.words;
   n = n < most ? n : most;
   return n > 0 ? n : 1;
+}
+// Shares the levels out: a.slabs at most, a.nSlabs in all.  Returns the words of LDS
+// a wavefront needs.  (At most 8: 12 us for 33 samples of 47^3; a wavefront a level:
+// 27)
+PYR_FN long long pyr_plan_slabs(PyrArgs &a, int RW) {
+  const int n0 = a.lv[0].nOut;
+  for (int most = a.batch < 64 ? 8 : a.batch < 512 ? 512 / a.batch : 1;; most /= 2) {
+    long long need = 0;
+    a.slabs = most;
+    a.nSlabs = 0;
+    for (int x = 0; x < a.nMasks; ++x) {
+      const PyrLevel &L = a.lv[x];
+      const int slabs = pyr_slabs(a.d, n0, L, most);
+      for (int z = 0; z < slabs; ++z, ++a.nSlabs) {
+        if (a.nSlabs < PYR_MAX_SLABS) {
+          a.slabLevel[a.nSlabs] = (unsigned char)x;
+          a.slabOf[a.nSlabs] = (unsigned char)z;
+        }
+        const long long words = pyr_slab_words(a.d, RW, n0, L, pyr_slab(a.d, L, L.magicN, z, slabs));
+        need = x > 0 && words > need ? words : need;
+      }
+    }
+    if (a.nSlabs <= PYR_MAX_SLABS)
+      return need;
+  }
 }
 template <int RW>
 PYR_FN void pyr_sweep_stage(const pyr_u64 *bits, long long first, int n0, int rows, pyr_u64 *dst, int t, int T) {
@@ -552,33 +607,14 @@ PYR_FN void pyr_sweep_fold(const pyr_u64 *rows, const pyr_u64 *mid, pyr_u64 *out
 
 // Pass B takes a sample's layers a WINDOW of levels xa .. xb at a time: level
 // xa as input only (its rows known: the source's, or from the window before),
-// layers xa + 1 .. xb built.  LDS bytes of a window for a sample with n[x]
-// sites at level x: per site key (4), row, ownership mask, base (2 each),
-// which candidate of its owner it is (1); the input level's batch-global rows
-// (4 more); every array padded to 16 bytes
-PYR_FN long long pyr_lds_window(const PyrArgs &a, const int *n, int xa, int xb) {
-  long long total = 0;
-  for (int x = xa; x <= xb; ++x)
-    total += n[x];
-  return PYR_HDR_BYTES + 8ll * a.pyrStride + 11ll * total + 4ll * n[xa] + 6 * 16;
-}
-// The window that starts at level xa: as many layers as fit (at least one,
-// when there is one)
-PYR_FN int pyr_window_end(const PyrArgs &a, const int *n, int xa, int xLast = -1) {
-  if (xLast < 0)
-    xLast = a.nMasks - 1;
-  int xb = xa < xLast ? xa + 1 : xa;
-  long long total = n[xa] + (xb > xa ? n[xb] : 0);
-  const long long fixed = PYR_HDR_BYTES + 8ll * a.pyrStride + 4ll * n[xa] + 6 * 16;
-  while (xb < xLast && fixed + 11ll * (total + n[xb + 1]) <= a.ldsBytesB) {
-    total += n[xb + 1];
-    ++xb;
-  }
-  return xb;
-}
+// layers xa + 1 .. xb built, as many as fit.  LDS bytes of a window for a sample
+// with n[x] sites at level x, beside the fixed ones: per site key (4), row,
+// ownership mask, base (2 each), which candidate of its owner it is (1); the input
+// level's batch-global rows (4 more); every array padded to 16 bytes
+PYR_FN long long pyr_fixed_lds(const PyrArgs &a) { return PYR_HDR_BYTES + 8ll * a.pyrStride + 6 * 16; }
 // Whether level x fits with the one after it, n0 and n1 sites
 PYR_FN bool pyr_pair_fits(const PyrArgs &a, int n0, int n1) {
-  return PYR_HDR_BYTES + 8ll * a.pyrStride + 11ll * ((long long)n0 + n1) + 4ll * n0 + 6 * 16 <= a.ldsBytesB;
+  return pyr_fixed_lds(a) + 11ll * ((long long)n0 + n1) + 4ll * n0 <= a.ldsBytesB;
 }
 // Whether every layer of the sample fits by itself; sites(x): of level x
 template <typename N> PYR_FN bool pyr_fits_of(const PyrArgs &a, N sites) {
@@ -586,9 +622,6 @@ template <typename N> PYR_FN bool pyr_fits_of(const PyrArgs &a, N sites) {
   for (int x = 0; x == 0 || x + 1 < a.nMasks; ++x)
     fits = fits && pyr_pair_fits(a, sites(x), x + 1 < a.nMasks ? sites(x + 1) : 0);
   return fits;
-}
-PYR_FN bool pyr_fits(const PyrArgs &a, const int *n) {
-  return pyr_fits_of(a, [n](int x) { return n[x]; });
 }
 
 // ------------------------------------------------------------------- pass B
@@ -604,6 +637,29 @@ PYR_FN bool pyr_set_chunks(PyrArgs &a) {
       a.chunkOf[a.nChunks] = (unsigned char)c;
     }
   return true;
+}
+// After the levels: how a sample's masks and prefixes lie in LDS, and those chunks
+PYR_FN bool pyr_set_layout(PyrArgs &a) {
+  const long long words = a.maskWords + (a.maskWords + 3ll) / 4;
+  a.pyrStride = (int)((words + 1) / 2 * 2);
+  return pyr_set_chunks(a);
+}
+// LDS bytes of pass B in a.parts, for samples of up to n[x] sites at level x
+PYR_FN long long pyr_rules_lds(const PyrArgs &a, const long long *n) {
+  long long need = 4 * a.nChunks; // (the sums of the prefixes' chunks)
+  for (int x = 0; x < a.nMasks; ++x) {
+    const long long pair = 15 * n[x] + (x + 1 < a.nMasks ? 11 * n[x + 1] : 0);
+    need = pair > need ? pair : need;
+  }
+  for (int p = 0; p < a.nParts; ++p) {
+    const PyrPart &part = a.parts[p];
+    const int xa = part.la >= 3 ? part.la - 2 : 0;
+    long long sites = 4 * n[xa];
+    for (int x = xa; x <= part.lb; ++x)
+      sites += 11 * (part.F > 1 ? n[x] / part.F + n[x] / (2 * part.F) + 64 : n[x]);
+    need = sites > need ? sites : need;
+  }
+  return need + pyr_fixed_lds(a);
 }
 
 struct PyrHdr {
@@ -751,20 +807,6 @@ PYR_FN void pyr_fill_level(const PyrLevel &L, int inMaskOff, int bgSource, const
   v.boundActive = L.boundActive;
   v.bg = L.bg;
   s.lv[l] = v;
-}
-
-// Where the levels of the window xa .. xb start in the per-site arrays, and
-// the window's layers among its items: lane t does entry t (t <= nMasks)
-PYR_FN void pyr_fill_offsets(PyrHdr *h, int xa, int xb, int t) {
-  if (t < xa || t > xb + 1)
-    return;
-  int sum = 0;
-  for (int x = xa; x < t; ++x)
-    sum += pyr_held(h, x);
-  h->siteOff[t] = sum;
-  h->itemOff[t] = t > xa ? sum - pyr_held(h, xa) : 0;
-  if (t == xb + 1)
-    h->total = sum;
 }
 
 // rank of the first site of level x at leading coordinate j (all of them: j = nOut)

@@ -1,181 +1,183 @@
-// Host harness for csrc/scn_pyr_dev.h: the per-lane bodies of the kernels that
-// build a net's rule books from the output side, run here lane after lane with
-// the barriers between the sweeps, on plain memory.  Built with the address and
-// undefined-behaviour sanitizers by tests/test_chain_cpu.py, which compares
-// what comes out with the oracle: every index the kernels compute is computed
-// here first, on the CPU, with bounds checked.
+// The kernels that build a net's rule books from the output side
+// (csrc/scn_pyr_body.h, scn_pyr_dev.h) on the host: the text the device runs, with
+// an executor that does the lanes of a workgroup one after the other.  Built with
+// the undefined-behaviour sanitizer by tests/test_chain_cpu.py, which compares what
+// comes out with the oracle: every index the kernels compute is computed here
+// first, on the CPU.  What the planning in csrc/scn_chain.hip does with a chain
+// is done here by the same functions.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
-#include "scn_pyr_dev.h"
+#include "scn_pyr_body.h"
 
 namespace {
 
-unsigned magic(long long x) { return (unsigned)((1ull << 32) / (unsigned long long)(x > 0 ? x : 1) + 1); }
+// An executor of scn_pyr_body.h.  Backwards: the lanes and wavefronts in descending
+// order (between two barriers none may matter to another).
+struct HostLanes {
+  static constexpr int T = 0;
+  int nLanes;
+  bool backwards;
+  int windows = 0;
+  HostLanes(int lanes, bool backwards) : nLanes(lanes), backwards(backwards) {}
+  template <typename V> struct Lane { // (of the lanes that have a layer)
+    V v[PYR_MAX_LEVELS + 1];
+    V &operator[](int t) {
+      if (t < 0 || t > PYR_MAX_LEVELS)
+        abort();
+      return v[t];
+    }
+  };
+  template <typename V> struct Wave {
+    V v[64];
+    V &operator[](int t) { return v[t]; }
+    const V &operator[](int t) const { return v[t]; }
+  };
+  int threads() const { return nLanes; }
+  template <typename F> void each(int n, F f) const {
+    for (int i = 0; i < n; ++i)
+      f(backwards ? n - 1 - i : i);
+  }
+  template <typename F> void lanes(F f) const { each(nLanes, f); }
+  template <typename F> void waves(int n, F f) const { each(n, f); }
+  template <typename F> void wave(F f) const { each(64, f); }
+  template <typename F> unsigned sum(F f) const {
+    unsigned n = 0;
+    each(64, [&](int lane) { n += f(lane); });
+    return n;
+  }
+  template <typename F> int max(F f) const {
+    int n = 0;
+    each(64, [&](int lane) { n = f(lane) > n ? f(lane) : n; });
+    return n;
+  }
+  template <typename F> Wave<unsigned> scan(F f) const {
+    Wave<unsigned> w;
+    unsigned n = 0;
+    for (int lane = 0; lane < 64; ++lane)
+      w[lane] = n += f(lane);
+    return w;
+  }
+  template <typename F> int count(F f) const {
+    int n = 0;
+    each(64, [&](int lane) { n += f(lane) ? 1 : 0; });
+    return n;
+  }
+  template <typename V> int at(const Wave<V> &w, int lane) const { return (int)w[lane]; }
+  int uniform(int x) const { return x; }
+  void sync() const {}
+  int row(const PyrArgs &a, long long p) const { return a.dense[p]; }
+  void check(bool holds) const {
+    if (!holds) {
+      fprintf(stderr, "a workgroup's own check does not hold\n");
+      abort();
+    }
+  }
+  void window() { ++windows; }
+};
+
+// Memory with something behind it that has to stay as it is
+struct Guarded {
+  std::vector<pyr_u64> v;
+  size_t words;
+  explicit Guarded(size_t words) : v(words + 16, 0xA5A5A5A5A5A5A5A5ull), words(words) {}
+  pyr_u64 *words64() { return v.data(); }
+  unsigned char *bytes() { return reinterpret_cast<unsigned char *>(v.data()); }
+  ~Guarded() {
+    for (size_t i = words; i < v.size(); ++i)
+      if (v[i] != 0xA5A5A5A5A5A5A5A5ull) {
+        fprintf(stderr, "written beyond a buffer's end\n");
+        abort();
+      }
+  }
+};
+
+#ifndef PYR_HARNESS_PLAN
+// whole samples (n: the mean sites of the levels)
+void plan(PyrArgs &a, const long long *n) { pyr_plan_parts(a, n, 1); }
+#endif
+
+template <int D, int RW> void levels(const PyrArgs &a, long long words) {
+  for (int y = 0; y < a.nSlabs; ++y)
+    for (int b = 0; b < a.batch; ++b) {
+      Guarded lds((size_t)words + 2);
+      HostLanes e(64, y & 1);
+      pyr_levels_body<D, RW>(e, a, lds.bytes(), b, y);
+    }
+}
+
+// Both kinds of pass A, which have to agree; what they leave is then in a.pyramid
+// and a.counts as the library would have it
+template <int D> void pass_a(PyrArgs &a, std::vector<int> &counts) {
+  const size_t all = (size_t)a.batch * (size_t)a.maskWords;
+  long long words = pyr_plan_whole(a);
+  for (int b = 0; b < a.batch; ++b) {
+    Guarded lds((size_t)words + 2);
+    HostLanes e(64, b & 1);
+    pyr_masks_body<D>(e, a, lds.bytes(), b);
+  }
+  const int RW = pyr_set_fold(a);
+  if (D == 1 || !RW)
+    return;
+  const std::vector<int> whole(counts);
+  const std::vector<pyr_u64> masks(a.pyramid, a.pyramid + all);
+  std::fill(counts.begin(), counts.end(), -1);
+  std::fill(a.pyramid, a.pyramid + all, 0x3C3C3C3C3C3C3C3Cull);
+  words = pyr_plan_slabs(a, RW);
+  if (D == 3)
+    levels<3, 1>(a, words);
+  else if (RW == 1)
+    levels<2, 1>(a, words);
+  else if (RW == 2)
+    levels<2, 2>(a, words);
+  else
+    levels<2, 4>(a, words);
+  bool same = !memcmp(masks.data(), a.pyramid, 8 * all);
+  for (int x = 0; x < a.nMasks; ++x)
+    for (int b = 0; b < a.batch; ++b) {
+      int n = 0;
+      for (int z = 0; z < pyr_slabs(D, a.lv[0].nOut, a.lv[x], a.slabs); ++z)
+        n += counts[((size_t)x * a.batch + b) * a.slabs + z];
+      same = same && n == whole[(size_t)x * a.batch + b];
+    }
+  if (!same) {
+    fprintf(stderr, "levels from the source differ\n");
+    abort();
+  }
+}
+
+// report: [nLevels + 1][4]
+template <int D> int run(PyrArgs &a, int T, std::vector<int> &counts, long long *report) {
+  pass_a<D>(a, counts);
+  long long mean[PYR_MAX_LEVELS + 1];
+  for (int x = 0; x < a.nMasks; ++x) {
+    mean[x] = 0;
+    for (int b = 0; b < a.batch; ++b)
+      for (int z = 0; z < (a.slabs == 1 ? 1 : pyr_slabs(D, a.lv[0].nOut, a.lv[x], a.slabs)); ++z)
+        mean[x] += counts[((size_t)x * a.batch + b) * a.slabs + z];
+    mean[x] = mean[x] / a.batch + 1;
+  }
+  plan(a, mean);
+  int over = 0;
+  for (int block = a.batch * a.nParts; block >= 0; --block) {
+    Guarded lds((size_t)a.ldsBytesB / 8);
+    HostLanes e(T, block & 1);
+    pyr_rules_body<D>(e, a, lds.bytes(), block);
+    over |= reinterpret_cast<PyrHdr *>(lds.bytes())->over;
+    report[0] = e.windows > report[0] ? e.windows : report[0]; // (the most windows a part took)
+  }
+  for (int l = 1; l <= a.nLevels; ++l)
+    memcpy(report + 4 * l, a.scalars + 16 + 4 * a.lv[l].slot, 32);
+  return (over & 2 ? 1 : 0) | (over & 1 ? 2 : 0);
+}
+
 long long ipow(long long a, int d) {
   long long r = 1;
   for (int i = 0; i < d; ++i)
     r *= a;
   return r;
-}
-
-// k_pyr_masks for sample b with T lanes
-template <int D> void pass_a(const PyrArgs &a, int b, int T, bool *gaveUp) {
-  std::vector<pyr_u64> lds((size_t)a.pyrStride + 64, 0);
-  pyr_u64 *masks = lds.data();
-  unsigned short *pref = reinterpret_cast<unsigned short *>(lds.data() + a.maskWords);
-  int cnt[PYR_MAX_LEVELS + 1] = {0};
-  {
-    const PyrLevel &L = a.lv[0];
-    for (int t = 0; t < T; ++t)
-      for (int w = t; w < L.words + 2; w += T)
-        masks[w] = w < L.words ? pyr_source_word(a.bits, L.volOut, b, (unsigned)w) : 0ull;
-  }
-  for (int x = 1; x < a.nMasks; ++x) { // (the masks start as zero: the pieces are OR-ed in)
-    const PyrLevel &L = a.lv[x];
-    const pyr_u64 *in = masks + a.lv[x - 1].maskOff;
-    pyr_u64 *out = masks + L.maskOff;
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_dilate<D>(in, out, L.nIn, L.nOut, L.size, L.stride, L.magicN, L.seg, L.segs, L.magicSegs, t, T);
-  }
-  for (int x = 0; x < a.nMasks; ++x) {
-    const PyrLevel &L = a.lv[x];
-    unsigned carry = 0;
-    for (int w = 0; w < L.words + 2; ++w) {
-      pref[L.maskOff + w] = (unsigned short)carry;
-      carry += (unsigned)pyr_popc64(masks[L.maskOff + w]);
-    }
-    cnt[x] = (int)carry;
-  }
-  memcpy(a.pyramid + (long long)b * a.pyrStride, lds.data(), 8ll * a.pyrStride);
-  for (int x = 0; x < a.nMasks; ++x) {
-    int *c = a.counts + ((long long)x * a.batch + b) * 2;
-    c[0] = cnt[x];
-    c[1] = (long long)cnt[x] < a.lv[x].fullSize;
-  }
-  bool fits = pyr_fits(a, cnt);
-  for (int x = 0; x < a.nMasks; ++x)
-    fits = fits && cnt[x] <= PYR_ROWS_MAX;
-  if (!fits)
-    *gaveUp = true;
-}
-
-// k_pyr_rules for sample b with T lanes; report: [nLevels + 1][4]
-template <int D> void pass_b(const PyrArgs &a, int b, int T, bool gaveUp, long long *report, bool *overOut) {
-  std::vector<unsigned char> ldsv((size_t)a.ldsBytesB);
-  unsigned char *lds = ldsv.data();
-  PyrHdr *h = reinterpret_cast<PyrHdr *>(lds);
-  h->over = 0;
-  memcpy(lds + PYR_HDR_BYTES, a.pyramid + (long long)b * a.pyrStride, 8ll * a.pyrStride);
-  for (int x = 0; x < a.nMasks; ++x) {
-    const int *cnt = a.counts + (long long)x * a.batch * 2;
-    long long v0 = 0, v1 = 0, v2 = 0, v3 = 0;
-    int mx = 0;
-    for (int s = 0; s < a.batch; ++s) {
-      const int n = cnt[2 * s], hb = cnt[2 * s + 1];
-      if (s < b) {
-        v0 += n;
-        v1 += hb;
-      }
-      v2 += n;
-      v3 += hb;
-      mx = n > mx ? n : mx;
-    }
-    h->n[x] = cnt[2 * b];
-    h->hasBg[x] = cnt[2 * b + 1];
-    h->actBefore[x] = v0;
-    h->bgBefore[x] = v1;
-    h->actAll[x] = v2;
-    h->bgAll[x] = v3;
-    h->maxAct[x] = mx;
-  }
-  for (int t = 1; t <= a.nLevels; ++t)
-    if (pyr_report(a, a.lv[t], h, t).over)
-      h->over |= 1;
-  if (!pyr_fits(a, h->n))
-    h->over |= 2;
-  const bool over = h->over != 0 || gaveUp;
-  if (b == 0)
-    for (int t = 1; t <= a.nLevels; ++t) {
-      const PyrReport r = pyr_report(a, a.lv[t], h, t);
-      report[4 * t + 0] = r.nSites;
-      report[4 * t + 1] = r.nActive;
-      report[4 * t + 2] = over;
-      report[4 * t + 3] = r.extra;
-    }
-  if (over) {
-    *overOut = true;
-    return;
-  }
-  int windows = 0;
-  for (int xa = 0;;) {
-    const int xb = pyr_window_end(a, h->n, xa);
-    const int la = xa + 1, lb = xb;
-    const bool last = xb == a.nMasks - 1;
-    ++windows;
-    for (int t = 0; t <= a.nMasks; ++t)
-      pyr_fill_offsets(h, xa, xb, t);
-    for (int t = 0; t < a.nMasks; ++t)
-      pyr_fill_en(a.lv[t], lds, t, h->siteOff[t]);
-    const PyrLds s = pyr_lds_view(a, lds, h->total, h->n[xa]);
-    // (the last array must end inside what pass B was launched with)
-    if (s.kOf + h->total > lds + a.ldsBytesB || pyr_lds_window(a, h->n, xa, xb) > a.ldsBytesB) {
-      fprintf(stderr, "a window takes more LDS than pass B was launched with\n");
-      abort();
-    }
-    for (int t = 1; t <= a.nLevels; ++t)
-      if ((t >= la && t <= lb) || (last && t == a.nLevels && t > lb))
-        pyr_fill_level(a.lv[t], a.lv[t - 1].maskOff, a.bg[b], s, t, xa);
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_clear(s, t, T);
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_enumerate<D>(a, s, xa, xb, t, T);
-    if (xa == 0) {
-      const PyrLevel &L = a.lv[0];
-      const long long p0 = (long long)b * L.volOut;
-      for (int r = 0; r < h->n[0]; ++r) {
-        int c[D];
-        pyr_unpack<D>(s.key[r], c);
-        s.srcRow[r] = (unsigned)a.dense[p0 + pyr_key<D>(c, L.nOut)];
-      }
-    }
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_owners<D>(s, la, lb, t, T);
-    for (int x = xa; x < xb; ++x) {
-      unsigned carry = 0;
-      for (int r = 0; r < h->n[x]; ++r) {
-        s.base[h->siteOff[x] + r] = (unsigned short)carry;
-        carry += (unsigned)pyr_popc32(pyr_own_mask(s, (unsigned)(h->siteOff[x] + r)));
-      }
-      if ((int)carry != h->n[x + 1]) {
-        fprintf(stderr, "level %d: %u sites owned, %d sites exist\n", x + 1, carry, h->n[x + 1]);
-        abort();
-      }
-    }
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_rows<D>(s, la, lb, b, t, T);
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_rules<D>(s, la, lb, t, T);
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_tail(a, s, la, lb, b, t, T);
-    if (last)
-      break;
-    for (int t = 0; t < T; ++t)
-      pyr_sweep_carry(s, lds, a, xb, t, T);
-    xa = xb;
-  }
-  if (windows > report[0])
-    report[0] = windows; // (the most windows a sample took)
-}
-
-template <int D> int run(PyrArgs &a, int T, long long *report) {
-  bool gaveUp = false, over = false;
-  for (int b = 0; b < a.batch; ++b)
-    pass_a<D>(a, b, T / 2 > 0 ? T / 2 : 1, &gaveUp);
-  for (int b = 0; b < a.batch; ++b)
-    pass_b<D>(a, b, T, gaveUp, report, &over);
-  return (gaveUp ? 1 : 0) | (over ? 2 : 0);
 }
 
 } // namespace
@@ -198,8 +200,8 @@ extern "C" int pyr_cpu_chain(int d, int batch, int n0, int nLevels, const int *g
   std::vector<int> dense((size_t)(batch * vol0), -7);
   for (long long i = 0; i < nActive; ++i) {
     const long long p = (long long)sample[i] * vol0 + key[i];
-    bits[p >> 6] |= 1ull << (p & 63);
-    dense[p] = row[i];
+    bits[(size_t)(p >> 6)] |= 1ull << (p & 63);
+    dense[(size_t)p] = row[i];
   }
   a.nLevels = nLevels;
   a.batch = batch;
@@ -207,66 +209,40 @@ extern "C" int pyr_cpu_chain(int d, int batch, int n0, int nLevels, const int *g
   a.dense = dense.data();
   a.bits = bits.data();
   a.bg = bg;
-  long long maskWords = 0;
-  {
-    PyrLevel &L = a.lv[0];
-    L.kind = PYR_REGIONS;
-    L.nIn = L.nOut = n0;
-    L.size = L.stride = L.width = 1;
-    L.volOut = vol0;
-    L.fullSize = vol0 + 1;
-    L.words = (int)((vol0 + 63) / 64);
-    L.maskOff = 0;
-    L.magicN = magic(n0);
-    L.magicS = magic(1);
-    maskWords = L.words + 2;
-  }
-  a.nMasks = 1;
+  std::vector<long long> meta((size_t)nLevels * 4), scalars((size_t)(16 + 4 * nLevels));
+  const long long badSites = 0;
+  a.scalars = scalars.data();
+  a.badSites = &badSites;
+  pyr_add_level(a, 0, PYR_REGIONS, n0, n0, 1, 1, 1, vol0, vol0 + 1);
   for (int l = 1; l <= nLevels; ++l) {
     const int *g = geo + 5 * (l - 1);
+    const bool terminal = g[0] == PYR_TERMINAL;
+    const long long vol = terminal ? 1 : ipow(g[2], d);
+    pyr_add_level(a, l, g[0], g[1], g[2], g[3], g[4], terminal ? 1 : (int)ipow(g[3], d), vol, vol);
     PyrLevel &L = a.lv[l];
-    L.kind = g[0];
-    L.nIn = g[1];
-    L.nOut = g[2];
-    L.size = g[3];
-    L.stride = g[4];
-    L.width = L.kind == PYR_TERMINAL ? 1 : (int)ipow(L.size, d);
-    L.volOut = L.kind == PYR_TERMINAL ? 1 : ipow(L.nOut, d);
-    L.fullSize = L.volOut;
-    L.magicN = magic(L.nOut);
-    L.magicS = magic(L.size);
-    pyr_set_pieces(L);
     L.rules = rules[l - 1];
     L.capacity = rulesCap[l - 1];
     L.ekey = ekey[l - 1];
     L.erow = erow[l - 1];
     L.bg = bgOut[l - 1];
+    L.meta = meta.data() + 4 * (l - 1);
+    L.slot = l - 1;
     L.boundRows = bounds[2 * (l - 1)];
     L.boundActive = bounds[2 * (l - 1) + 1];
-    if (L.kind == PYR_REGIONS) {
-      L.words = (int)((L.volOut + 63) / 64);
-      L.maskOff = (int)maskWords;
-      maskWords += L.words + 2;
-      a.nMasks = l + 1;
-    }
   }
-  long long pyrStride = maskWords + (maskWords + 3) / 4;
-  pyrStride = (pyrStride + 1) / 2 * 2;
-  a.maskWords = (int)maskWords;
-  a.pyrStride = (int)pyrStride;
-  a.ldsBytesB = ldsBytesB;
-  std::vector<pyr_u64> pyramid((size_t)(batch * pyrStride));
-  std::vector<int> counts((size_t)a.nMasks * batch * 2);
-  a.pyramid = pyramid.data();
-  a.counts = counts.data();
-  if (PYR_HDR_BYTES + 8 * pyrStride > ldsBytesB)
+  if (!pyr_set_layout(a) || pyr_fixed_lds(a) + 4 * a.nChunks > ldsBytesB)
     return 4;
+  a.ldsBytesB = ldsBytesB;
+  Guarded pyramid((size_t)batch * (size_t)a.maskWords);
+  std::vector<int> counts((size_t)a.nMasks * batch * 8, -1);
+  a.pyramid = pyramid.words64();
+  a.counts = counts.data();
   switch (d) {
   case 1:
-    return run<1>(a, T, report);
+    return run<1>(a, T, counts, report);
   case 2:
-    return run<2>(a, T, report);
+    return run<2>(a, T, counts, report);
   default:
-    return run<3>(a, T, report);
+    return run<3>(a, T, counts, report);
   }
 }

@@ -1,6 +1,6 @@
-"""csrc/scn_pyr_dev.h on the CPU: the per-lane bodies of the kernels that build a whole net's rule books from the
-output side (k_pyr_masks / k_pyr_rules), compiled for the host and run lane after lane by tests/chain_cpu_harness.cpp,
-against the oracle's gridRules (Regions.cu:528-653) layer by layer and its terminal rules
+"""csrc/scn_pyr_body.h and scn_pyr_dev.h on the CPU: the kernels that build a whole net's rule books from the output
+side (k_pyr_masks, k_pyr_levels, k_pyr_rules), compiled for the host and run lane after lane by
+tests/chain_cpu_harness.cpp, against the oracle's gridRules (Regions.cu:528-653) layer by layer and its terminal rules
 (TerminalPoolingLayer.cu:8-20).  Every buffer the harness writes is allocated with guard words that must come back
 untouched."""
 import ctypes as C
@@ -16,17 +16,18 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRC = os.path.join(HERE, "chain_cpu_harness.cpp")
 LIB = os.path.join(HERE, "libchain_cpu.so")
+CSRC = os.path.join(ROOT, "sparseconvnet-archived_amd", "csrc")
+HEADERS = tuple(os.path.join(CSRC, h) for h in ("scn_pyr_dev.h", "scn_pyr_body.h"))
 GUARD = 64
 REGIONS, TERMINAL = 0, 1
 
 
 def build(force=False):
-    hdr = os.path.join(ROOT, "sparseconvnet-archived_amd", "csrc", "scn_pyr_dev.h")
-    stale = not os.path.exists(LIB) or os.path.getmtime(LIB) < max(os.path.getmtime(SRC), os.path.getmtime(hdr))
+    stale = not os.path.exists(LIB) or os.path.getmtime(LIB) < max(os.path.getmtime(p) for p in (SRC,) + HEADERS)
     if force or stale:
         subprocess.check_call(["g++", "-O1", "-g", "-std=c++17", "-shared", "-fPIC", "-Wall", "-fsanitize=undefined",
                                "-fno-sanitize-recover=undefined", "-static-libubsan",
-                               "-I", os.path.dirname(hdr), SRC, "-o", LIB])
+                               "-I", CSRC, SRC, "-o", LIB])
 
 
 @pytest.fixture(scope="module")

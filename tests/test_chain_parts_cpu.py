@@ -1,5 +1,5 @@
-"""What csrc/scn_pyr_dev.h does beside the sweeps over whole samples, on the CPU under the sanitizer: every level's mask
-from the source directly, and a sample's rule books by several workgroups, each with some of the layers or with a slab
+"""The same with more shared out than such small fields would be, on the CPU under the sanitizer: every level's mask
+by several wavefronts, and a sample's rule books by several workgroups, each with some of the layers or with a slab
 of one of them (chain_parts_harness.cpp).  The chains, the oracle and the guard words are test_chain_cpu.py's."""
 import ctypes as C
 import os
@@ -16,11 +16,11 @@ LIB = os.path.join(whole.HERE, "libchain_parts_cpu.so")
 
 @pytest.fixture(scope="module")
 def harness():
-    hdr = os.path.join(whole.ROOT, "sparseconvnet-archived_amd", "csrc", "scn_pyr_dev.h")
-    if not os.path.exists(LIB) or os.path.getmtime(LIB) < max(os.path.getmtime(p) for p in (SRC, whole.SRC, hdr)):
+    if not os.path.exists(LIB) or os.path.getmtime(LIB) < max(os.path.getmtime(p)
+                                                              for p in (SRC, whole.SRC) + whole.HEADERS):
         subprocess.check_call(["g++", "-O1", "-g", "-std=c++17", "-shared", "-fPIC", "-Wall", "-fsanitize=undefined",
                                "-fno-sanitize-recover=undefined", "-static-libubsan",
-                               "-I", os.path.dirname(hdr), "-I", whole.HERE, SRC, "-o", LIB])
+                               "-I", whole.CSRC, "-I", whole.HERE, SRC, "-o", LIB])
     lib = C.CDLL(LIB)
     lib.pyr_cpu_chain.restype = C.c_int
     return lib

@@ -283,3 +283,31 @@ def test_a_sample_is_shared_out_by_its_own_size_not_the_last_batch_s(scn):
         st.check(got, st.oracle(one, sizes), 1)
         splits.append(scn.chain_split(ctx))
     assert splits[0] == splits[1] and 1 <= splits[0][0] < 24, splits
+
+
+@pytest.mark.parametrize("d,layers,batch,parts,slabs", [
+    (3, [("sq", 2, 1, 1), ("sq", 2, 2, 1)] * 4, 5, (12, 24), (14, 48)),  # 47^3: layers in slabs, levels in slabs
+    (2, [("sq", 2, 1, 1), ("sq", 3, 2, 1)] * 5, 3, (4, 24), (11, 11)),   # 126 x 126, ten layers: a wavefront a level
+    (2, [("sq", 2, 1, 1), ("sq", 3, 2, 1)] * 5, 100, (1, 1), (11, 11)),  # enough samples: a workgroup each
+    (1, [("sq", 3, 1, 1), ("sq", 2, 2, 1)], 4, (1, 24), (0, 0))])        # one dimension: level after level
+def test_samples_are_shared_out_and_stay_the_same(scn, d, layers, batch, parts, slabs):
+    ctx = scn.Context()
+    st = Stack(scn, ctx, d, layers)
+    sizes = st.sizes(2)
+    n, rng, samples, row = sizes[0], np.random.default_rng(d + batch), [], 0
+    for b in range(batch):  # thick shells and strokes, in rows of no order; samples unlike in size
+        at = np.stack(np.meshgrid(*[np.arange(n)] * d, indexing="ij"), -1).reshape(-1, d)
+        off = np.abs(np.linalg.norm(at - rng.uniform(0.4, 0.6, d) * n, axis=1) - rng.uniform(0.15, 0.25) * n)
+        keys = rng.permutation(np.flatnonzero(off < 0.5 + 0.1 * (b % 3)))
+        samples.append((row, {int(k): row + 1 + i for i, k in enumerate(keys)}))
+        row += len(keys) + 1
+    st.build(samples, row, n)
+    st.run(samples, sizes)
+    for _ in range(2):  # the second time with LDS for what was seen
+        st.build(samples, row, n)
+        got, ok = st.run_chained(samples, sizes)
+        assert ok
+        split = scn.chain_split(ctx)
+        print("split", split, flush=True)
+        assert parts[0] <= split[0] <= parts[1] and slabs[0] <= split[1] <= slabs[1], split
+        st.check(got, st.oracle(samples, sizes), batch)
