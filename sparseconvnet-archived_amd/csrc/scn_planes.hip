@@ -200,9 +200,12 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
 
   // ---- W.  One item = V adjacent columns of two consecutive k, or 16 bytes of the
   // image.  (Every instruction occupies the vector memory path for 16 cycles or
-  // more: with the eight k of a column to an item, a dword each, 100 drawings'
-  // layers of 128 and 256 k took 5 % longer.  N is a multiple of 4; a scratch
-  // matrix W may be aligned to no more than a float.)
+  // more: with the eight k of a column to an item, a dword each, the (1, 2) tiles of
+  // 100 drawings' layers took 15.7 us and not 14.5, the (1, 1) tiles 20.6 and not
+  // 20.2.  Such an item was stored 16 bytes a plane; the dwords that this one stores
+  // meet on their banks, in half of the cycles that the LDS is in use (5 % before);
+  // with them that is an eighth of all.  N is a multiple of 4; a scratch matrix W may
+  // be aligned to no more than a float.)
   constexpr bool IMG = WM == W_IMAGE;
   constexpr int V = NT % 2 ? 2 : 4;
   constexpr int ITEMS = IMG ? BUF_BYTES / 16 : 16 * NW / V;
@@ -944,12 +947,15 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
     return launch_planes<PL, 1, 2, W_PLAIN, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
   // W_STREAM where the chip is full and the contraction long: the widest tile, W
   // from its image, rows gathered (by no more than 27 positions: with the third
-  // buffer two workgroups still fit a compute unit's LDS).  The registers it frees let bf16 rows go eight
-  // wavefronts to a workgroup, half the reading of W: 596000 x 2592 x 128 433 ->
-  // 406 us, and of ten layers of 57 to 395 GFLOP 0.99 to 1.10 times as fast.
-  // 1.36 M x 1728 x 64 in three planes 1386 -> 1347.  Everywhere else what the
-  // third buffer costs is not made good: (3, 1, 1) 58.8 -> 61.6 us, one plane
-  // (1, 2) 40 -> 47, rows that are not gathered 141 -> 148.
+  // buffer two workgroups still fit a compute unit's LDS).  The registers it frees
+  // let bf16 rows go eight wavefronts to a workgroup, half the reading of W:
+  // 596000 x 2592 x 128 433 -> 406 us, and of ten layers of 57 to 395 GFLOP 0.99 to
+  // 1.10 times as fast.  In three planes it is 1 % of layers of 1728 k and more,
+  // whose loop is all they are (1.36 M x 1728 x 64 1422 -> 1398 us, 596000 x 2592 x
+  // 128 1808 -> 1788, 3456 k 889 -> 876: means of each side's runs, in turn on one
+  // card), and nothing that shows on shorter ones (512 to 1280 k, 66 to 970 us: 0.97
+  // to 1.03).  Everywhere else what the third buffer costs is not made good: (3, 1, 1)
+  // 58.8 -> 61.6 us, one plane (1, 2) 40 -> 47, rows that are not gathered 141 -> 148.
   if constexpr (PL != 2)
     if (choice.tile == 3 && choice.image && gs && (PL > 1 || a16))
       return launch_planes<PL, (PL > 1 ? 2 : 1), (PL > 1 ? 2 : 4), W_STREAM, false, (PL > 1 ? 4 : 8)>(
