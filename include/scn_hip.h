@@ -248,8 +248,8 @@ int scn_ctx_rows_held(scn_ctx *ctx, int *held);
  * plan before -- are only noted, provided every `out` has held a plan before
  * and a sample's grids fit the LDS of a compute unit (2-D and small 3-D
  * fields); scn_ctx_chain_rules(ctx, 0), scn_rules_settle or any call that
- * cannot join then runs all of them in two launches, one workgroup carrying
- * one sample through every layer.  Results (rules, counts, grids as seen
+ * cannot join then runs all of them in two launches, which share the samples
+ * out among workgroups (scn_ctx_chain_split).  Results (rules, counts, grids as seen
  * through scn_grids_download / scn_grids_find) are those of the calls made one
  * by one; a sample too large for the LDS is reported by scn_rules_settle as
  * SCN_ERR_CAPACITY like any outgrown bound. */

@@ -1218,7 +1218,7 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   if (!pyr_set_layout(a) || pyr_fixed_lds(a) + CHAIN_MIN_ARENA > PYR_LDS_MAX)
     return SCN_OK;
   {
-    // A workgroup of pass B has a compute unit to itself (sixteen wavefronts of 82
+    // A workgroup of pass B has a compute unit to itself (sixteen wavefronts of 85
     // registers) and issues what there is to issue: a batch of few samples leaves
     // units idle.  One drawing 26.5 us with a workgroup a sample, 14 with as many
     // as it is worth; 61 images 24 and 16.5 with four; 33 samples of a 47^3 field 73

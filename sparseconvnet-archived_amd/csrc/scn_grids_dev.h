@@ -1,6 +1,6 @@
 // Types and device helpers shared by the translation units that build sparse
 // grids and rule books (scn_grids.hip: one layer at a time through tables in
-// HBM; scn_chain.hip: all layers of a net at once, one workgroup per sample).
+// HBM; scn_chain.hip: all layers of a net at once, samples side by side).
 #pragma once
 #include "scn_common.h"
 #include "scn_scan_dev.h"

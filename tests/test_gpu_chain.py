@@ -1,5 +1,5 @@
 """Recorded plans (scn_ctx_chain_rules): the rule books of consecutive layers
-built together, one workgroup per sample, against the CPU oracle -- bit-exact
+built together, samples side by side, against the CPU oracle -- bit-exact
 rules, counts, grids (table and mask built on demand from the entry lists) --
 and against the same calls run one by one."""
 import numpy as np
