@@ -110,8 +110,11 @@ __global__ void __launch_bounds__(256)
               const int *__restrict__ rules, long long nOutSites, int ps,
               int C, int chunks, int *__restrict__ choice,
               const float *__restrict__ spare, const long long *dRows) {
-  long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   nOutSites = live_rows(nOutSites, dRows);
+  const unsigned tiles = (unsigned)((nOutSites * chunks + 255) / 256);
+  if (blockIdx.x >= tiles)
+    return;
+  const long long idx = (long long)xcd_eighth(blockIdx.x, tiles) * 256 + threadIdx.x;
   if (idx >= nOutSites * chunks)
     return;
   long long r = idx / chunks;

@@ -512,8 +512,10 @@ __global__ void __launch_bounds__(256)
                 float *__restrict__ out, long long M, int K, int N, Epilogue ep,
                 GatherSource gs, const long long *dRows) {
   M = live_rows(M, dRows);
-  if ((long long)blockIdx.x * (32 * CT_GROUPS) >= M)
+  const unsigned tiles = (unsigned)((M + 32 * CT_GROUPS - 1) / (32 * CT_GROUPS));
+  if (blockIdx.x >= tiles)
     return;
+  const long long tile = xcd_eighth(blockIdx.x, tiles);
   // LDS: the gathered rows, then this workgroup's columns of W at pitch wp
   extern __shared__ __attribute__((aligned(16))) float ctLds[];
   float *const sA = ctLds;
@@ -523,7 +525,7 @@ __global__ void __launch_bounds__(256)
   const int n0 = blockIdx.y * CT_COLS;
   const int cols = N - n0 < CT_COLS ? N - n0 : CT_COLS; // a multiple of 4
   const int r = tid >> 3;
-  const long long mFirst = (long long)blockIdx.x * (32 * CT_GROUPS) + r;
+  const long long mFirst = tile * (32 * CT_GROUPS) + r;
   int rule[CT_GROUPS][TK_MAX_K / 8];
 #pragma unroll
   for (int g = 0; g < CT_GROUPS; ++g)

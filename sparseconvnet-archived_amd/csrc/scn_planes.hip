@@ -177,8 +177,10 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
                  float *__restrict__ out, long long M, int K, int N,
                  Epilogue ep, GatherSource gs, int nSplits, RowRange rows, PlainW plain) {
   M = rows.live(M);
-  if ((long long)(blockIdx.x / nSplits) * (32 * WAVES * MT) >= M)
+  const unsigned tiles = (unsigned)((M + 32 * WAVES * MT - 1) / (32 * WAVES * MT)) * nSplits;
+  if (blockIdx.x >= tiles)
     return;
+  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
   constexpr int ES = A16 ? 2 : 4;
   constexpr int THREADS = 64 * WAVES;
   constexpr int ROWS = 32 * MT * WAVES, NW = 32 * NT;
@@ -192,8 +194,8 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
-  const int split = blockIdx.x % nSplits; // workgroups that share rows are neighbours
-  const long long wgRow0 = (long long)(blockIdx.x / nSplits) * ROWS;
+  const int split = tileOf % nSplits; // workgroups that share rows are neighbours
+  const long long wgRow0 = (long long)(tileOf / nSplits) * ROWS;
   const long long row0 = wgRow0 + wave * 32 * MT;
   const int n0 = split * NW;
   const int T = K / 32;
@@ -602,16 +604,18 @@ __global__ void __launch_bounds__(512, 2)
                         float *__restrict__ out, long long M, int K, int N,
                         Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
   M = rows.live(M);
-  if ((long long)(blockIdx.x / nSplits) * 32 >= M)
+  const unsigned tiles = (unsigned)((M + 31) / 32) * nSplits;
+  if (blockIdx.x >= tiles)
     return;
+  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
   constexpr int ES = A16 ? 2 : 4;
   __shared__ __attribute__((aligned(16))) float sPart[8 * 16 * 64];
   __shared__ int sRules[GATHER ? 32 * GF_MAX_FS : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
-  const int split = blockIdx.x % nSplits;
-  const long long row0 = (long long)(blockIdx.x / nSplits) * 32;
+  const int split = tileOf % nSplits;
+  const long long row0 = (long long)(tileOf / nSplits) * 32;
   const int n0 = split * 32;
   const int T = K / 32;
   const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
@@ -1027,9 +1031,11 @@ __global__ void __launch_bounds__(512, 2)
   int *const sAgain = reinterpret_cast<int *>(sTile + 8 * TILE);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
-  const int k0 = (blockIdx.x / nTiles) * 32 * MT;
-  const int n0 = (blockIdx.x % nTiles) * 32 * NT;
-  const long long m0 = (long long)blockIdx.y * rowsPerSplit;
+  // (the tiles of a range of rows, which read the same, to one XCD)
+  const unsigned at = xcd_eighth(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  const int k0 = (int)(at % gridDim.x / nTiles) * 32 * MT;
+  const int n0 = (int)(at % gridDim.x % nTiles) * 32 * NT;
+  const long long m0 = (long long)(at / gridDim.x) * rowsPerSplit;
   const long long m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
   // this lane's columns (past the end: the last ones, not stored)
   int ka = k0 + MT * c, na = n0 + NT * c;

@@ -741,8 +741,9 @@ __global__ __launch_bounds__(256) void k_maxpool_backward(
   __shared__ float sSum[ROOM];
   __shared__ int sRows;
   const int tid = threadIdx.x, P = 1 << shift;
-  const long long r0 = (long long)(blockIdx.x / slices) * (T * EPT >> shift);
-  const int j = (int)(blockIdx.x % slices) * P + (tid & (P - 1)); // (P divides T)
+  const unsigned tileOf = xcd_eighth(blockIdx.x, gridDim.x);
+  const long long r0 = (long long)(tileOf / slices) * (T * EPT >> shift);
+  const int j = (int)(tileOf % slices) * P + (tid & (P - 1)); // (P divides T)
   int tg[EPT], slot[EPT];
   float dv[EPT];
 #pragma unroll
