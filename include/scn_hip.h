@@ -444,6 +444,51 @@ int scn_activation_backward_to(scn_ctx *ctx, const float *d_out,
                                float *d_db, float *d_dprelu, int accumulate);
 int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
                       float *d_dW, int64_t M, int K, int N);
+/* The backward pass of a convolution without its gathered matrix (no
+ * counterpart in the reference, which keeps that matrix and its gradient).
+ * scn_rules_inverse_many turns the rules of up to SCN_INVERSE_MAX layers round:
+ *   d_positions [fs x scn_positions_pitch(rows)]: the rules position by position,
+ *     padded with -1;
+ *   d_inverse [inputRows x fs]: which of the `rows` output rows names an input row
+ *     at each filter position (-1: none); for the background row of sample s, which
+ *     any number may name, that is rows + s fs + f;
+ *   d_background [rows + 2 batch]: a bit for every position at which a row names
+ *     its sample's background row, then for every sample the first and the last of
+ *     its rows with any (2^31 - 1 and -1: none).
+ * (d_positions, d_background, and d_inverse and d_background may be null: not
+ * wanted; fs <= 32.)
+ * scn_conv_AtB: scn_sgemm_AtB of what scn_gather_rows would make of d_in through
+ * the rules (nIn <= 4096; d_positions aligned to 16 bytes).
+ * The gradient of the input is a convolution of d_D with the rules turned round.
+ * d_delta has rows + batch fs rows, those behind the layer's own cleared by the
+ * caller; scn_background_sums adds what is to be there.
+ * scn_transpose_filters_many gives the weights, Wt [fs N x nIn] of W [fs nIn x
+ * N], and scn_conv_input_gradient writes every input row's gradient, d_din
+ * [inputRows x nIn], from d_delta (where scn_conv_nin_supported_p(fs, N, nIn,
+ * SCN_FP32)). */
+#define SCN_INVERSE_MAX 16
+typedef struct scn_inverse_item {
+  const scn_grids *input; /* the convolution's input grids, counts settled */
+  const int32_t *d_rules; /* [rows x fs] */
+  int32_t *d_inverse, *d_background, *d_positions;
+  int64_t rows, inputRows;
+  int32_t fs;
+} scn_inverse_item;
+int64_t scn_positions_pitch(int64_t rows);
+int scn_rules_inverse_many(scn_ctx *ctx, const scn_inverse_item *items, int nItems);
+int scn_background_sums(scn_ctx *ctx, float *d_delta, int64_t rows, int N,
+                        const int32_t *d_background, int fs, int batch);
+#define SCN_FILTERS_MAX 32
+typedef struct scn_filter_item {
+  const float *d_W;
+  float *d_Wt;
+  int32_t fs, nIn, N;
+} scn_filter_item;
+int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *items, int nItems);
+int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
+                            const float *d_Wt, float *d_din, int64_t inputRows, int nIn);
+int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,
+                 const float *d_D, float *d_dW, int64_t M, int N, int accumulate);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout
  * (NetworkInNetworkLayer.cu:7-25): w[i][j] = W[inPresent[i]][outPresent[j]],
  * W with rows of nOut floats; a null d_inPresent keeps the rows (row i of w

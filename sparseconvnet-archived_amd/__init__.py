@@ -33,6 +33,15 @@ class ScnError(RuntimeError):
 NAG_MAX = 48
 
 
+class InverseItem(C.Structure):
+    _fields_ = [("input", C.c_void_p), ("d_rules", C.c_void_p), ("d_inverse", C.c_void_p),
+                ("d_background", C.c_void_p), ("d_positions", C.c_void_p), ("rows", C.c_int64), ("inputRows", C.c_int64), ("fs", C.c_int32)]
+
+
+class FilterItem(C.Structure):
+    _fields_ = [("d_W", C.c_void_p), ("d_Wt", C.c_void_p), ("fs", C.c_int32), ("nIn", C.c_int32), ("N", C.c_int32)]
+
+
 class NagItem(C.Structure):
     """scn_nag_item of the C header."""
     _fields_ = [("d_delta", C.c_void_p), ("d_momentum", C.c_void_p), ("d_weights", C.c_void_p),
@@ -141,6 +150,12 @@ def lib():
         "scn_activation_backward_acc": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),
         "scn_activation_backward_to": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp, C.c_int]),
         "scn_sgemm_AtB_acc": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_conv_AtB": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
+        "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, i64, C.c_int]),
+        "scn_background_sums": (C.c_int, [vp, vp, i64, C.c_int, vp, C.c_int, C.c_int]),
+        "scn_positions_pitch": (i64, [i64]),
+        "scn_transpose_filters_many": (C.c_int, [vp, P(FilterItem), C.c_int]),
         "scn_shrink_matrix": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int]),
         "scn_nag_update_shrunk": (C.c_int, [vp, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int, f32, f32]),
         "scn_sum_abs": (C.c_int, [vp, vp, i64, P(C.c_double)]),
@@ -343,6 +358,32 @@ class Context:
     def sgemm_AtB(self, d_A, d_D, d_dW, M, K, N, accumulate=False):
         f = lib().scn_sgemm_AtB_acc if accumulate else lib().scn_sgemm_AtB
         _check(f(self.h, d_A.ptr, d_D.ptr, d_dW.ptr, M, K, N))
+
+    def conv_AtB(self, d_in, d_positions, fs, nIn, d_D, d_dW, M, N, accumulate=False):
+        _check(lib().scn_conv_AtB(self.h, d_in.ptr if d_in is not None else None, d_positions.ptr, fs, nIn, d_D.ptr,
+                                  d_dW.ptr, M, N, int(accumulate)))
+
+    def rules_inverse_many(self, items):
+        """items: (input Grids, d_rules, d_inverse, d_background, d_positions, rows, inputRows, fs) tuples; the three
+        outputs may be None"""
+        arr = (InverseItem * max(1, len(items)))()
+        for k, (g, rules, inverse, background, positions, rows, inputRows, fs) in enumerate(items):
+            out = [x.ptr if x is not None else None for x in (inverse, background, positions)]
+            arr[k] = InverseItem(g.h, rules.ptr, *out, rows, inputRows, fs)
+        _check(lib().scn_rules_inverse_many(self.h, arr, len(items)))
+
+    def conv_input_gradient(self, d_delta, d_inverse, fs, N, d_Wt, d_din, inputRows, nIn):
+        _check(lib().scn_conv_input_gradient(self.h, d_delta.ptr, d_inverse.ptr, fs, N, d_Wt.ptr, d_din.ptr, inputRows, nIn))
+
+    def background_sums(self, d_delta, M, N, d_background, fs, batch):
+        _check(lib().scn_background_sums(self.h, d_delta.ptr, M, N, d_background.ptr, fs, batch))
+
+    def transpose_filters_many(self, items):
+        """items: (d_W, d_Wt, fs, nIn, N) tuples"""
+        arr = (FilterItem * max(1, len(items)))()
+        for k, (w, wt, fs, nIn, n) in enumerate(items):
+            arr[k] = FilterItem(w.ptr, wt.ptr, fs, nIn, n)
+        _check(lib().scn_transpose_filters_many(self.h, arr, len(items)))
 
     def nag_update_many(self, items, learningRate, momentum, clearGradients=False):
         """items: (d_delta, d_momentum, d_weights, n, keepPositive) tuples, at most NAG_MAX of them."""

@@ -1019,12 +1019,15 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // rows as that leaves it.  29827 x 256 x 96 in 23 us (32 on the fp32 MFMA with
 // a thousand workgroups), 200000 x 1728 x 64 in 350 (470): A from HBM at 3.9
 // TB/s.
+// GATHER: the rows of A through rules, which lie position by position, so that
+// a lane's eight are two loads (eight of them through row by row rules: 17.8 us
+// where this is 15.6 and a gathered matrix 14.5, and 8.2 to gather it).
 #define ATB_STEP 16
-template <int MT, int NT>
+template <int MT, int NT, bool GATHER>
 __global__ void __launch_bounds__(512, 2)
     k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
                  float *__restrict__ dW, long long M, int K, int N, int nTiles,
-                 long long rowsPerSplit) {
+                 long long rowsPerSplit, GatherSource gs) {
   constexpr int PL = 3, GM = 8;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
   extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], then a flag
@@ -1042,9 +1045,24 @@ __global__ void __launch_bounds__(512, 2)
   ka = ka + MT <= K ? ka : K - MT;
   na = na + NT <= N ? na : N - NT;
   const unsigned offA = (unsigned)(8 * q) * K + ka, offD = (unsigned)(8 * q) * N + na;
+  // GATHER: this lane's filter position and channel, the same for all rows
+  const int f = GATHER ? ka / gs.nIn : 0, ch = GATHER ? ka - f * gs.nIn : 0;
 
   struct Step {
     float a[8][MT], d[8][NT];
+    int rule[GATHER ? 8 : 1];
+  };
+  // GATHER: the rules of a step are asked for a step before its rows are
+  auto look_up = [&](Step &s, long long m) {
+#pragma unroll
+    for (int h = 0; h < (GATHER ? 2 : 0); ++h) {
+      // (the positions' pitch: the last rows of one are padded with none)
+      const long long pitch = (M + ATB_STEP - 1) / ATB_STEP * ATB_STEP;
+      const long long at = m + 8 * q + 4 * h;
+      const int4 v = *reinterpret_cast<const int4 *>(gs.rules + f * pitch + (at < pitch ? at : pitch - 4));
+      s.rule[(4 * h) % (GATHER ? 8 : 1)] = v.x, s.rule[(4 * h + 1) % (GATHER ? 8 : 1)] = v.y;
+      s.rule[(4 * h + 2) % (GATHER ? 8 : 1)] = v.z, s.rule[(4 * h + 3) % (GATHER ? 8 : 1)] = v.w;
+    }
   };
   auto load = [&](Step &s, long long m, bool guard) {
 #pragma unroll
@@ -1059,6 +1077,8 @@ __global__ void __launch_bounds__(512, 2)
         pa = A + (m + i) * K + offA;
         pd = D + (m + i) * N + offD;
       }
+      if constexpr (GATHER)
+        pa = s.rule[i] >= 0 ? A + (long long)s.rule[i] * gs.nIn + ch : gs.zeros;
       if constexpr (MT == 2) {
         const floatx2 v = *reinterpret_cast<const floatx2 *>(pa);
         s.a[i][0] = v[0], s.a[i][1] = v[1];
@@ -1125,17 +1145,24 @@ __global__ void __launch_bounds__(512, 2)
       load(s, at < m1 ? at : m1 - 1, true);
   };
   if (m < m1) {
+    look_up(s0, m);
+    look_up(s1, m + ATB_STEP * GM);
     fetch(s0, m);
+    look_up(s0, m + 2 * ATB_STEP * GM);
     for (;;) {
       const long long ma = m + ATB_STEP * GM;
-      if (ma < m1)
+      if (ma < m1) {
         fetch(s1, ma);
+        look_up(s1, ma + 2 * ATB_STEP * GM);
+      }
       compute(s0);
       if (ma >= m1)
         break;
       const long long mb = ma + ATB_STEP * GM;
-      if (mb < m1)
+      if (mb < m1) {
         fetch(s0, mb);
+        look_up(s0, mb + 2 * ATB_STEP * GM);
+      }
       compute(s1);
       if (mb >= m1)
         break;
@@ -1198,7 +1225,12 @@ __global__ void __launch_bounds__(512, 2)
       float a[MT], d[NT];
 #pragma unroll
       for (int i = 0; i < MT; ++i)
-        a[i] = r < m1 ? A[r * K + ka + i] : 0.f;
+        if constexpr (GATHER) {
+          const int rule = r < m1 ? gs.rules[ka / gs.nIn * ((M + ATB_STEP - 1) / ATB_STEP * ATB_STEP) + r] : -1;
+          a[i] = rule >= 0 ? A[(long long)rule * gs.nIn + ka % gs.nIn + i] : 0.f;
+        } else {
+          a[i] = r < m1 ? A[r * K + ka + i] : 0.f;
+        }
 #pragma unroll
       for (int j = 0; j < NT; ++j)
         d[j] = r < m1 ? D[r * N + na + j] : 0.f;
@@ -1222,13 +1254,13 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
-template <int MT, int NT>
+template <int MT, int NT, bool GATHER>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
-                      long long M, int K, int N, long long splits) {
+                      long long M, int K, int N, long long splits, const GatherSource &gs) {
   const size_t lds = ((size_t)8 * 32 * MT * 32 * NT + 1) * sizeof(float);
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
                ? SCN_OK
                : SCN_ERR_HIP;
@@ -1238,9 +1270,18 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
   const long long tiles = (long long)scn_ceil_div(K, 32 * MT) * nTiles;
   long long rows = (M + splits - 1) / splits;
   rows = (rows + 8 * ATB_STEP - 1) / (8 * ATB_STEP) * (8 * ATB_STEP);
-  hipLaunchKernelGGL((k_atb_planes<MT, NT>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)), dim3(512),
-                     lds, ctx->stream, A, D, dW, M, K, N, nTiles, rows);
+  hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
+                     dim3(512), lds, ctx->stream, A, D, dW, M, K, N, nTiles, rows, gs);
   return SCN_OK;
+}
+template <int MT, int NT>
+static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, long long M, int K, int N,
+                      long long splits, const GatherSource *gs) {
+  if constexpr (MT == 2 && NT == 2) // (not gathered: see below)
+    return launch_atb<MT, NT, false>(ctx, A, D, dW, M, K, N, splits, GatherSource());
+  else
+    return gs ? launch_atb<MT, NT, true>(ctx, A, D, dW, M, K, N, splits, *gs)
+              : launch_atb<MT, NT, false>(ctx, A, D, dW, M, K, N, splits, GatherSource());
 }
 
 // The tile and the number of row ranges that cost least: rounds of one workgroup
@@ -1249,7 +1290,7 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
 // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
 // (The search is 0.1 to 2 us of the host's time, a launch some 5.)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
-                   long long M, int K, int N) {
+                   long long M, int K, int N, const GatherSource *gs) {
   static const struct {
     int mt, nt;
     double ti, f;
@@ -1257,8 +1298,8 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
   int best = 0;
   long long splits = 1;
   double least = 1e300;
-  for (int i = 0; i < 4; ++i) {
-    if ((tile[i].mt == 2 && (K % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
+  for (int i = 0; i < (gs ? 3 : 4); ++i) { // (two by two tiles of gathered rows: 264 bytes a lane spilled)
+    if ((tile[i].mt == 2 && ((gs ? gs->nIn : K) % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
       continue;
     const long long tiles = (long long)scn_ceil_div(K, 32 * tile[i].mt) * scn_ceil_div(N, 32 * tile[i].nt);
     if (tiles > 0x7fffffffll)
@@ -1278,11 +1319,11 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
   SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
   switch (best) {
   case 1:
-    return launch_atb<2, 1>(ctx, A, D, dW, M, K, N, splits);
+    return launch_atb<2, 1>(ctx, A, D, dW, M, K, N, splits, gs);
   case 2:
-    return launch_atb<1, 2>(ctx, A, D, dW, M, K, N, splits);
+    return launch_atb<1, 2>(ctx, A, D, dW, M, K, N, splits, gs);
   case 3:
-    return launch_atb<2, 2>(ctx, A, D, dW, M, K, N, splits);
+    return launch_atb<2, 2>(ctx, A, D, dW, M, K, N, splits, gs);
   }
-  return launch_atb<1, 1>(ctx, A, D, dW, M, K, N, splits);
+  return launch_atb<1, 1>(ctx, A, D, dW, M, K, N, splits, gs);
 }

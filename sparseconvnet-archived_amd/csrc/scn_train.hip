@@ -10,6 +10,7 @@
 //   max-pooling                dMaxPoolBackProp, MaxPoolingLayer.cu:74-82
 //   terminal pooling           dTerminalPoolBackProp, TerminalPoolingLayer.cu:48-62
 #include <mutex>
+#include "scn_grids_dev.h"
 #include "scn_nin_dev.h"
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
@@ -211,6 +212,15 @@ extern "C" int scn_activation_backward_to(scn_ctx *ctx, const float *d_out,
                              d_db, d_dprelu, !accumulate);
 }
 
+// The number of rows is the caller's, whatever scn_ctx_rows_from says to the
+// forward calls, whose kernels run in some of the backward ones
+struct OwnRows {
+  scn_ctx *ctx;
+  const long long *meta;
+  explicit OwnRows(scn_ctx *c) : ctx(c), meta(c->d_meta) { c->d_meta = nullptr; }
+  ~OwnRows() { ctx->d_meta = meta; }
+};
+
 // ---------------------------------------------- dW = A^T D (scn_planes.hip)
 static int sgemm_AtB(scn_ctx *ctx, const float *d_A, const float *d_D,
                      float *d_dW, int64_t M, int K, int N, bool clear) {
@@ -240,6 +250,345 @@ extern "C" int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A,
                                  const float *d_D, float *d_dW, int64_t M,
                                  int K, int N) {
   return sgemm_AtB(ctx, d_A, d_D, d_dW, M, K, N, false);
+}
+
+// The same product with A left ungathered: row m of it is what scn_gather_rows
+// would make of the rules of output row m, given position by position.
+extern "C" int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,
+                            const float *d_D, float *d_dW, int64_t M, int N, int accumulate) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_AtB: null context");
+  SCN_REQUIRE(M >= 0 && fs >= 1 && nIn >= 1 && nIn <= SCN_ZERO_FLOATS && (int64_t)fs * nIn <= 0x7fffffff && N >= 1,
+              SCN_ERR_ARG, "scn_conv_AtB: M %lld fs %d nIn %d N %d", (long long)M, fs, nIn, N);
+  SCN_REQUIRE(d_dW, SCN_ERR_ARG, "scn_conv_AtB: null d_dW");
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  if (!accumulate)
+    SCN_TRY(scn_fill32(ctx, d_dW, 0, (size_t)fs * nIn * N));
+  if (M == 0)
+    return SCN_OK;
+  // (d_in may be null: an input without rows, every rule negative)
+  SCN_REQUIRE(d_positions && d_D, SCN_ERR_ARG, "scn_conv_AtB: null buffer");
+  SCN_REQUIRE(((uintptr_t)d_positions & 15) == 0, SCN_ERR_ARG, "scn_conv_AtB: positions start on 16 bytes");
+  GatherSource gs = GatherSource();
+  gs.rules = d_positions;
+  gs.fs = fs;
+  gs.nIn = nIn;
+  gs.zeros = ctx->d_zeros;
+  SCN_TRY(scn_atb_planes(ctx, d_in, d_D, d_dW, (long long)M, fs * nIn, N, &gs));
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
+// ------------------------------------- the gradient of a convolution's input
+// dA = D W^T scattered through the rules is itself a convolution: row r of the
+// input gets, for every filter position f at which an output row o names it,
+// D[o] W_f^T.  There is one such o at most, unless r is a background row, which
+// any number of windows names.  So a layer's rules are turned round once
+// (inverse[r * fs + f] = o, -1: none); the rows of D that name a sample's
+// background row (background[o]: at which positions) are summed per position
+// (k_background_sums) into rows behind D's own, which the background row's
+// inverse names; and the forward kernels do
+// the rest on W with every position's block transposed: no matrix of M x K is
+// written and read again, none is cleared, and no float is added atomically but
+// those few.  (Where W holds an infinity, a position that no row names adds 0
+// times it: NaN, and not nothing.  Such a net's forward pass is full of them.)
+// Of a batch of 100 drawings the backward kernels of the layer 57000 x 128 -> 64
+// take 4.4 + 17.2 + 22.5 + 14.7 us with the matrix (image, dW, dA, scatter; 8.2
+// for the gathering besides) and 15.6 + 6.3 + 19.3 without (dW, sums, gradient);
+// 12 batches 7570 -> 6620 us of kernels, of voxel models 5650 -> 5000.  Turning
+// the rules round, on the producers' streams, is 10 us of a batch.
+#define POSITIONS_PITCH(rows) (((rows) + 15) & ~15ll)
+struct InverseList {
+  const int *rules[SCN_INVERSE_MAX], *bg[SCN_INVERSE_MAX];
+  int *inverse[SCN_INVERSE_MAX], *positions[SCN_INVERSE_MAX];
+  int *background[SCN_INVERSE_MAX];
+  int rows[SCN_INVERSE_MAX], inRows[SCN_INVERSE_MAX];
+  unsigned firstBlock[SCN_INVERSE_MAX + 1];
+  int fs[SCN_INVERSE_MAX], batch[SCN_INVERSE_MAX];
+  int count;
+};
+// a workgroup an item
+__global__ __launch_bounds__(256) void k_inverse_background(InverseList l) {
+  const int t = blockIdx.x, fs = l.fs[t];
+  if (!l.inverse[t])
+    return;
+  if (l.background[t])
+    for (int s = threadIdx.x; s < l.batch[t]; s += 256) {
+      l.background[t][l.rows[t] + 2 * s] = 0x7fffffff;
+      l.background[t][l.rows[t] + 2 * s + 1] = -1;
+    }
+  for (int x = threadIdx.x; x < l.batch[t] * fs; x += 256) {
+    const int r = l.bg[t][x / fs];
+    if (r >= 0 && r < l.inRows[t])
+      l.inverse[t][(long long)r * fs + x % fs] = l.rows[t] + x;
+  }
+}
+// a lane a row of the output
+__global__ __launch_bounds__(256) void k_inverse_rules(InverseList l) {
+  static_assert(SCN_INVERSE_MAX <= 64, "a lane an item");
+  const int lane = threadIdx.x & 63;
+  const int t =
+      __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_INVERSE_MAX ? lane : 0])) - 1;
+  const long long o = (long long)(blockIdx.x - l.firstBlock[t]) * 256 + threadIdx.x;
+  const int rows = l.rows[t], inRows = l.inRows[t], fs = l.fs[t];
+  const long long pitch = POSITIONS_PITCH((long long)rows);
+  const int *const rules = l.rules[t];
+  int *const inverse = l.inverse[t], *const positions = l.positions[t];
+  if (o >= pitch)
+    return;
+  unsigned mask = 0;
+  int sample = 0;
+  for (int f = 0; f < fs; ++f) {
+    const int r = o < rows ? rules[o * fs + f] : -1;
+    if (positions)
+      positions[f * pitch + o] = r;
+    if (!inverse || r < 0 || r >= inRows)
+      continue;
+    int *const at = inverse + (long long)r * fs + f;
+    const int was = *at;
+    if (was < rows) { // (the background rows' are named already)
+      *at = (int)o;
+    } else {
+      mask |= 1u << f;
+      sample = (was - rows) / fs;
+    }
+  }
+  if (!l.background[t])
+    return;
+  if (o < rows)
+    l.background[t][o] = (int)mask;
+  // the first and the last row of a sample that name its background: of the rows of
+  // a wavefront only those at the ends of a sample's run (all of them: 22 us a batch
+  // of 100 drawings and not 8, some 400 atomics on a line)
+  int *const ends = l.background[t] + rows;
+  const unsigned long long named = __ballot(mask != 0);
+  const unsigned long long below = named & ((1ull << lane) - 1), above = named & ~((2ull << lane) - 1);
+  const int before = __shfl(sample, below ? 63 - __builtin_clzll(below) : lane);
+  const int behind = __shfl(sample, above ? __builtin_ctzll(above) : lane);
+  if (!mask)
+    return;
+  if (!below || before != sample)
+    atomicMin(&ends[2 * sample], (int)o);
+  if (!above || behind != sample)
+    atomicMax(&ends[2 * sample + 1], (int)o);
+}
+extern "C" int64_t scn_positions_pitch(int64_t rows) { return POSITIONS_PITCH(rows); }
+extern "C" int scn_rules_inverse_many(scn_ctx *ctx, const scn_inverse_item *items, int nItems) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_rules_inverse_many: null context");
+  SCN_REQUIRE(nItems >= 0 && nItems <= SCN_INVERSE_MAX && (items || nItems == 0), SCN_ERR_ARG,
+              "scn_rules_inverse_many: %d items (at most %d)", nItems, SCN_INVERSE_MAX);
+  InverseList l;
+  void *fill[SCN_INVERSE_MAX];
+  size_t words[SCN_INVERSE_MAX];
+  long long blocks = 0; // (16 items of no more than 2^23 workgroups)
+  int fills = 0;
+  l.count = 0;
+  for (int k = 0; k < nItems; ++k) {
+    const scn_inverse_item &it = items[k];
+    SCN_REQUIRE(it.input && it.rows >= 0 && it.inputRows >= 0 && it.inputRows <= 0x7fffffffll && it.fs >= 1 &&
+                    it.fs <= 32,
+                SCN_ERR_ARG, "scn_rules_inverse_many: item %d rows %lld of %lld fs %d", k, (long long)it.rows,
+                (long long)it.inputRows, it.fs);
+    SCN_REQUIRE(!it.input->pending, SCN_ERR_STATE, "scn_rules_inverse_many: item %d: counts not settled", k);
+    SCN_REQUIRE(it.rows + (int64_t)it.input->batch * it.fs <= 0x7fffffffll, SCN_ERR_CAPACITY,
+                "scn_rules_inverse_many: item %d: %lld rows", k, (long long)it.rows);
+    SCN_REQUIRE((it.d_rules || it.rows == 0) && (it.d_inverse || !it.d_background), SCN_ERR_ARG,
+                "scn_rules_inverse_many: item %d null buffer", k);
+    const int c = l.count++;
+    l.rules[c] = it.d_rules;
+    l.bg[c] = it.input->bg.p;
+    l.inverse[c] = it.inputRows ? it.d_inverse : nullptr;
+    l.positions[c] = it.d_positions;
+    l.background[c] = it.d_background;
+    l.rows[c] = (int)it.rows;
+    l.inRows[c] = (int)it.inputRows;
+    l.fs[c] = it.fs;
+    l.batch[c] = it.input->batch;
+    l.firstBlock[c] = (unsigned)blocks;
+    blocks += scn_ceil_div(scn_positions_pitch(it.rows), 256);
+    if (l.inverse[c]) {
+      fill[fills] = it.d_inverse;
+      words[fills++] = (size_t)it.inputRows * it.fs;
+    }
+  }
+  if (l.count == 0)
+    return SCN_OK;
+  l.firstBlock[l.count] = (unsigned)blocks;
+  ProfScope prof(ctx, SCN_K_RULES);
+  if (fills) {
+    SCN_TRY(scn_fill32_many(ctx, fill, words, fills, 0xffffffffu));
+    hipLaunchKernelGGL(k_inverse_background, dim3(l.count), dim3(256), 0, ctx->stream, l);
+  }
+  if (blocks)
+    hipLaunchKernelGGL(k_inverse_rules, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, l);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
+// A workgroup takes a part of the rows of D between the first and the last that
+// name a sample's background.  A lane keeps the sums of V columns at FS positions
+// over every rows-th row, as the row's mask says, the workgroup's lanes of one
+// column are put together in LDS, and each sum is added to memory once.  (Ranges
+// of rows without regard to samples, with the sums given up where the sample
+// changes: 9.4 us a layer of 100 drawings on average.)
+template <int V, int FS>
+__global__ __launch_bounds__(256) void k_background_sums(float *delta, long long M, int N,
+                                                         const int *__restrict__ background, int fs, int parts,
+                                                         int P) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  __shared__ float sSum[256 * V * FS];
+  const int tid = threadIdx.x;
+  const int rows = 256 / P; // lanes beyond the last whole row idle
+  const int tx = tid % P, ty = tid / P;
+  const int c = (blockIdx.y * P + tx) * V;
+  const unsigned at = xcd_eighth(blockIdx.x, gridDim.x);
+  const int sample = (int)(at / parts), part = (int)(at % parts);
+  int first = background[M + 2 * sample], end = background[M + 2 * sample + 1] + 1;
+  const int range = (end - first + parts - 1) / parts;
+  if (end <= first || first + part * range >= end)
+    return;
+  first += part * range;
+  end = first + range < end ? first + range : end;
+  for (int f0 = 0; f0 < fs; f0 += FS) {
+    vec acc[FS];
+#pragma unroll
+    for (int f = 0; f < FS; ++f)
+      acc[f] = vec(0.f);
+    // (the rows are asked for before it is known whether they are wanted: most are)
+    constexpr int AHEAD = 4;
+    if (c < N && ty < rows)
+      for (int r = first + ty; r < end; r += AHEAD * rows) {
+        unsigned mask[AHEAD];
+        vec d[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+          const int ru = r + u * rows < end ? r + u * rows : end - 1;
+          mask[u] = r + u * rows < end ? (unsigned)background[ru] >> f0 : 0;
+          d[u] = *reinterpret_cast<const vec *>(delta + (long long)ru * N + c);
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+          for (int f = 0; f < FS; ++f)
+            acc[f] += mask[u] >> f & 1 ? d[u] : vec(0.f);
+      }
+#pragma unroll
+    for (int f = 0; f < FS; ++f)
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+        sSum[(f * V + v) * 256 + tid] = acc[f][v];
+    __syncthreads();
+    for (int x = tid; x < P * V * FS; x += 256) {
+      const int f = x / (P * V), col = x % (P * V), lane = col / V, v = col % V;
+      const int n = (blockIdx.y * P + lane) * V + v;
+      if (n >= N || f0 + f >= fs)
+        continue;
+      float sum = 0.f;
+      for (int k = 0; k < rows; ++k)
+        sum += sSum[(f * V + v) * 256 + k * P + lane];
+      unsafeAtomicAdd(delta + (M + (long long)sample * fs + f0 + f) * N + n, sum);
+    }
+    __syncthreads();
+  }
+}
+extern "C" int scn_background_sums(scn_ctx *ctx, float *d_delta, int64_t M, int N, const int32_t *d_background,
+                                   int fs, int batch) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_background_sums: null context");
+  SCN_REQUIRE(M >= 0 && M <= 0x7fffffffll && N >= 1 && fs >= 1 && fs <= 32 && batch >= 0, SCN_ERR_ARG,
+              "scn_background_sums: M %lld N %d fs %d batch %d", (long long)M, N, fs, batch);
+  if (M == 0 || batch == 0)
+    return SCN_OK;
+  SCN_REQUIRE(d_delta && d_background, SCN_ERR_ARG, "scn_background_sums: null buffer");
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  const int V = N % 4 == 0 && ((uintptr_t)d_delta & 15) == 0 ? 4 : 1;
+  const int colBlocks = scn_ceil_div(N, V * 64);
+  const int P = scn_ceil_div(scn_ceil_div(N, V), colBlocks);
+  // two workgroups a compute unit, of 32 rows at least: what it costs to begin and to end
+  long long parts = scn_ceil_div(2 * ctx->numCU, (int64_t)batch * colBlocks);
+  const long long most = scn_ceil_div(M, 32ll * batch);
+  parts = parts < most ? parts : most;
+  SCN_REQUIRE(batch * parts <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_background_sums: batch %d", batch);
+  const dim3 grid((unsigned)(batch * parts), (unsigned)colBlocks);
+#define SCN_BGS_GO(V, FS)                                                                                     \
+  hipLaunchKernelGGL((k_background_sums<V, FS>), grid, dim3(256), 0, ctx->stream, d_delta, (long long)M, N,   \
+                     d_background, fs, (int)parts, P)
+  if (V == 4 && fs <= 4)
+    SCN_BGS_GO(4, 4);
+  else if (V == 4)
+    SCN_BGS_GO(4, 8);
+  else
+    SCN_BGS_GO(1, 8);
+#undef SCN_BGS_GO
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
+// Wt[(f N + n) nIn + c] = W[(f nIn + c) N + n]: the weights of that convolution,
+// all layers' in one launch, a workgroup a tile of 32 x 32
+struct FilterList {
+  const float *W[SCN_FILTERS_MAX];
+  float *Wt[SCN_FILTERS_MAX];
+  unsigned firstBlock[SCN_FILTERS_MAX + 1];
+  int nIn[SCN_FILTERS_MAX], N[SCN_FILTERS_MAX];
+  int count;
+};
+__global__ __launch_bounds__(256) void k_transpose_filters(FilterList l) {
+  __shared__ float tile[32][33];
+  const int lane = threadIdx.x & 63;
+  const int t =
+      __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_FILTERS_MAX ? lane : 0])) - 1;
+  const int nIn = l.nIn[t], N = l.N[t], across = (N + 31) / 32, down = (nIn + 31) / 32;
+  const unsigned b = blockIdx.x - l.firstBlock[t];
+  const int f = (int)(b / (across * down)), n0 = (int)(b % across) * 32, c0 = (int)(b / across % down) * 32;
+  const float *const W = l.W[t] + (long long)f * nIn * N;
+  float *const Wt = l.Wt[t] + (long long)f * nIn * N;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5; // 32 x 8
+  for (int i = ty; i < 32; i += 8)
+    if (c0 + i < nIn && n0 + tx < N)
+      tile[i][tx] = W[(long long)(c0 + i) * N + n0 + tx];
+  __syncthreads();
+  for (int i = ty; i < 32; i += 8)
+    if (n0 + i < N && c0 + tx < nIn)
+      Wt[(long long)(n0 + i) * nIn + c0 + tx] = tile[tx][i];
+}
+extern "C" int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *items, int nItems) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_transpose_filters_many: null context");
+  SCN_REQUIRE(nItems >= 0 && nItems <= SCN_FILTERS_MAX && (items || nItems == 0), SCN_ERR_ARG,
+              "scn_transpose_filters_many: %d items (at most %d)", nItems, SCN_FILTERS_MAX);
+  static_assert(SCN_FILTERS_MAX <= 64, "a lane an item");
+  FilterList l;
+  long long blocks = 0;
+  for (int k = 0; k < nItems; ++k) {
+    const scn_filter_item &it = items[k];
+    SCN_REQUIRE(it.d_W && it.d_Wt && it.fs >= 1 && it.nIn >= 1 && it.N >= 1, SCN_ERR_ARG,
+                "scn_transpose_filters_many: item %d fs %d nIn %d N %d", k, it.fs, it.nIn, it.N);
+    l.W[k] = it.d_W;
+    l.Wt[k] = it.d_Wt;
+    l.nIn[k] = it.nIn;
+    l.N[k] = it.N;
+    l.firstBlock[k] = (unsigned)blocks;
+    blocks += (long long)it.fs * scn_ceil_div(it.N, 32) * scn_ceil_div(it.nIn, 32);
+    SCN_REQUIRE(blocks <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_transpose_filters_many: %lld workgroups", blocks);
+  }
+  l.count = nItems;
+  l.firstBlock[nItems] = (unsigned)blocks;
+  if (blocks == 0)
+    return SCN_OK;
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  hipLaunchKernelGGL(k_transpose_filters, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, l);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
+extern "C" int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
+                                       const float *d_Wt, float *d_din, int64_t inputRows, int nIn) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_input_gradient: null context");
+  SCN_REQUIRE(inputRows >= 0 && nIn >= 1 && nIn <= SCN_ZERO_FLOATS && N <= SCN_ZERO_FLOATS, SCN_ERR_ARG,
+              "scn_conv_input_gradient: %lld rows nIn %d N %d", (long long)inputRows, nIn, N);
+  if (inputRows == 0)
+    return SCN_OK;
+  OwnRows ownRows(ctx);
+  return scn_conv_nin_forward_p(ctx, d_delta, d_inverse, fs, N, d_Wt, ctx->d_zeros, nullptr, d_din, inputRows, nIn,
+                                1.f, SCN_NOSIGMOID, SCN_FP32_PLANES);
 }
 
 // ------------------------------------------------------------ dA = D W^T
@@ -275,14 +624,7 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
     return SCN_OK;
   SCN_REQUIRE(d_D && d_W && d_dA && d_workspace, SCN_ERR_ARG,
               "scn_sgemm_ABt: null buffer");
-  // (M is the caller's number of rows, whatever scn_ctx_rows_from says to the
-  // forward calls, whose kernels run here)
-  struct OwnRows {
-    scn_ctx *ctx;
-    const long long *meta;
-    explicit OwnRows(scn_ctx *c) : ctx(c), meta(c->d_meta) { c->d_meta = nullptr; }
-    ~OwnRows() { ctx->d_meta = meta; }
-  } ownRows(ctx);
+  OwnRows ownRows(ctx);
   bool transpose = false;
   Epilogue ep = Epilogue();
   ep.bias = ctx->d_zeros;

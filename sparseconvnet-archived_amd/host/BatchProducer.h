@@ -60,8 +60,9 @@ public:
   int batchSize;
   int spatialSize;
   std::vector<int> permutation;
+  // unseen: see SpatiallySparseBatch
   BatchProducer(SparseConvNetCUDA &cnn, SpatiallySparseDataset &dataset,
-                int spatialSize, int batchSize);
+                int spatialSize, int batchSize, bool unseen = false);
   // nBatches passes over one batch that is resident in HBM (benchmarking), or
   // over several taken in turn
   BatchProducer(SparseConvNetCUDA &cnn, const ResidentBatch &resident,
@@ -84,6 +85,7 @@ public:
 
 private:
   static SpatiallySparseDataset emptyDataset;
+  bool unseen = false;
   std::vector<ResidentBatch> residents; // empty: batches come from the dataset
   void start();
   std::vector<char> slotFull;

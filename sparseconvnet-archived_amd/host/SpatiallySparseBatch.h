@@ -77,6 +77,9 @@ public:
   // the rule books' counts are still on the device: the interfaces hold bounds
   // until SparseConvNetCUDA::settleRuleBooks
   bool countsPending;
+  // a training batch between whose layers nobody looks (processDataset's): what
+  // only its layers' kernels would read need not be there
+  bool unseen;
   // device staging of the input sites (sample, key as two ints, row,
   // backgroundCol), reused from batch to batch
   vectorCUDA<int> stagingSample, stagingKey, stagingRow, stagingBackground;

@@ -35,6 +35,15 @@ public:
   // over the outputs of the pooling behind it); a pooling's: sub->dactivated holds
   // what it is to spread
   bool activationDone = false, activationAhead = false;
+  // A convolution's output in a batch nobody looks into (SpatiallySparseBatch::
+  // unseen) whose matrix and gradient are left out: the rules turned round
+  // (scn_rules_inverse_many; all but the positions empty where no gradient of its
+  // input is wanted).
+  bool leftOut = false;
+  vectorCUDA<int> inverse, background, positions;
+  // rows of sub->dfeatures behind the layer's own: sums over the background of
+  // such a convolution's input
+  size_t gradientSums = 0;
   // Host view of the sparse grids.  Filled by the Pictures for the input
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().

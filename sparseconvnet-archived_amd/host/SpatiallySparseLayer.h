@@ -51,6 +51,12 @@ public:
                                SpatiallySparseBatchInterface &pooled) {
     (void)batch, (void)input, (void)output, (void)pooled;
   }
+  // the weights that the gradient of a left out convolution's input is made with
+  // (input.leftOut), for scn_transpose_filters_many
+  virtual void transposedFilters(SpatiallySparseBatchInterface &input,
+                                 std::vector<scn_filter_item> &items) {
+    (void)input, (void)items;
+  }
 };
 
 // ConvolutionalLayer.h:3-33 -- gathers each output site's receptive field
@@ -162,6 +168,8 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  void transposedFilters(SpatiallySparseBatchInterface &input,
+                         std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);
 };
 
@@ -207,6 +215,8 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  void transposedFilters(SpatiallySparseBatchInterface &input,
+                         std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);
 };
 

@@ -322,7 +322,8 @@ void SpatiallySparseBatchSubInterface::reset() {
 SpatiallySparseBatchInterface::SpatiallySparseBatchInterface(
     SpatiallySparseBatchSubInterface *s)
     : sub(s), featuresPresent(false, 0), deviceGrids(nullptr),
-      ownsDeviceGrids(false), rules(true, 0), deferredGatherFrom(nullptr) {
+      ownsDeviceGrids(false), rules(true, 0), inverse(true, 0), background(true, 0), positions(true, 0),
+      deferredGatherFrom(nullptr) {
   reset();
 }
 SpatiallySparseBatchInterface::SpatiallySparseBatchInterface(
@@ -332,7 +333,8 @@ SpatiallySparseBatchInterface::SpatiallySparseBatchInterface(
       nSpatialSites(o.nSpatialSites), spatialSize(o.spatialSize),
       backpropErrors(o.backpropErrors), grids(std::move(o.grids)),
       deviceGrids(o.deviceGrids), ownsDeviceGrids(o.ownsDeviceGrids),
-      rules(std::move(o.rules)), deferredGatherFrom(nullptr) {
+      rules(std::move(o.rules)), inverse(std::move(o.inverse)), background(std::move(o.background)),
+      positions(std::move(o.positions)), deferredGatherFrom(nullptr) {
   o.deviceGrids = nullptr;
   o.ownsDeviceGrids = false;
 }
@@ -346,6 +348,11 @@ void SpatiallySparseBatchInterface::reset() {
   grids.resize(0);
   rules.resize(0);
   backpropErrors = false;
+  leftOut = false;
+  gradientSums = 0;
+  inverse.resize(0);
+  background.resize(0);
+  positions.resize(0);
   deferredGatherFrom = nullptr;
   // deviceGrids keeps its tables for the next batch
 }
@@ -412,6 +419,7 @@ SpatiallySparseBatch::SpatiallySparseBatch(
 }
 void SpatiallySparseBatch::reset() {
   countsPending = false;
+  unseen = false;
   batchSize = 0;
   sampleNumbers.resize(0);
   for (auto &i : interfaces)

@@ -87,7 +87,7 @@ static void gather_now(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
 // the input's gradient at nf features a site, zero
 static void clear_gradient(cudaMemStream &ms,
                            SpatiallySparseBatchInterface &input, size_t nf) {
-  const size_t n = (size_t)input.nSpatialSites * nf;
+  const size_t n = ((size_t)input.nSpatialSites + input.gradientSums) * nf;
   const bool cleared = input.gradientCleared && input.sub->dfeatures.size64() == n;
   input.gradientCleared = false;
   if (cleared)
@@ -101,7 +101,7 @@ static void clear_gradient(cudaMemStream &ms,
 static void conv_backwards(SpatiallySparseBatchInterface &input,
                            SpatiallySparseBatchInterface &output,
                            cudaMemStream &ms) {
-  if (!input.backpropErrors)
+  if (!input.backpropErrors || output.deferredGatherFrom) // (done by the layer behind)
     return;
   const size_t nIn = input.featuresPresent.size();
   const size_t width = output.featuresPresent.size();
@@ -165,8 +165,9 @@ void ConvolutionalLayer::preprocess(SpatiallySparseBatch &batch,
 void ConvolutionalLayer::forwards(SpatiallySparseBatch &batch,
                                   SpatiallySparseBatchInterface &input,
                                   SpatiallySparseBatchInterface &output) {
-  // (the backward pass needs the gathered matrix: no deferral while training)
-  if (deferGather && batch.type != TRAINBATCH) {
+  // (the backward pass needs the gathered matrix: no deferral while training,
+  // unless that pass does without it)
+  if (batch.type == TRAINBATCH ? output.leftOut : deferGather) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -229,7 +230,7 @@ void ConvolutionalTriangularLayer::preprocess(
 void ConvolutionalTriangularLayer::forwards(
     SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
     SpatiallySparseBatchInterface &output) {
-  if (deferGather && batch.type != TRAINBATCH) {
+  if (batch.type == TRAINBATCH ? output.leftOut : deferGather) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -398,8 +399,36 @@ static void nin_activation_ahead(cudaMemStream &ms,
   pooled.activationAhead = true;
   output.activationDone = true;
 }
-static void nin_backwards(cudaMemStream &ms,
-                          std::vector<scn_nag_item> *updates,
+// A layer behind a convolution that was left out: dW from the convolution's
+// input, and that input's gradient from this layer's output's, through the rules
+// turned round (transposed: the weights for that, scn_transpose_filters_many).
+static void conv_nin_gradients(cudaMemStream &ms, SpatiallySparseBatchInterface &middle,
+                               SpatiallySparseBatchInterface &output, vectorCUDA<float> &dw,
+                               vectorCUDA<float> &transposed, bool clean, int batchSize) {
+  SpatiallySparseBatchInterface &src = *middle.deferredGatherFrom;
+  const int64_t M = output.nSpatialSites;
+  const int N = output.nFeatures, nIn = src.nFeatures, fs = middle.nFeatures / nIn;
+  SCN_CHECKED(scn_conv_AtB(ms.ctx, src.sub->features.dPtr(), middle.positions.dPtr(), fs, nIn,
+                           output.sub->dfeatures.dPtr(), dw.dPtr(), M, N, clean));
+  addMultiplyAdds((__int128_t)M * fs * nIn * N);
+  if (!src.backpropErrors)
+    return;
+  SCN_CHECKED(scn_background_sums(ms.ctx, output.sub->dfeatures.dPtr(), M, N,
+                                  middle.background.dPtr(), fs, batchSize));
+  src.sub->dfeatures.resize64(((size_t)src.nSpatialSites + src.gradientSums) * nIn);
+  SCN_CHECKED(scn_conv_input_gradient(ms.ctx, output.sub->dfeatures.dPtr(), middle.inverse.dPtr(), fs, N,
+                                      transposed.dPtr(), src.sub->dfeatures.dPtr(), src.nSpatialSites, nIn));
+  addMultiplyAdds((__int128_t)M * fs * nIn * N); // (what the reference's count holds for it)
+}
+static void nin_transposed_filters(SpatiallySparseBatchInterface &input, int nFeaturesOut, vectorCUDA<float> &W,
+                                   vectorCUDA<float> &transposed, std::vector<scn_filter_item> &items) {
+  if (!input.deferredGatherFrom || !input.backpropErrors)
+    return;
+  const int nIn = input.deferredGatherFrom->nFeatures;
+  transposed.resize64((size_t)input.nFeatures * nFeaturesOut);
+  items.push_back({W.dPtr(), transposed.dPtr(), input.nFeatures / nIn, nIn, nFeaturesOut});
+}
+static void nin_backwards(cudaMemStream &ms, SpatiallySparseBatch &batch,
                           SpatiallySparseBatchInterface &input,
                           SpatiallySparseBatchInterface &output, int nFeaturesIn,
                           int nFeaturesOut, vectorCUDA<float> *shrunkW,
@@ -423,12 +452,16 @@ static void nin_backwards(cudaMemStream &ms,
         act, PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
         dprelu ? dprelu->dPtr() : nullptr));
   output.activationDone = false;
-  SCN_CHECKED((clean ? scn_sgemm_AtB_acc : scn_sgemm_AtB)(
-      ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(),
-      dw.dPtr(), M, K, N));
-  addMultiplyAdds((__int128_t)M * K * N);
-  if (input.backpropErrors) {
-    input.sub->dfeatures.resize64((size_t)input.nSpatialSites * K);
+  if (input.deferredGatherFrom) {
+    conv_nin_gradients(ms, input, output, dw, workspace, clean, batch.batchSize);
+  } else {
+    SCN_CHECKED((clean ? scn_sgemm_AtB_acc : scn_sgemm_AtB)(
+        ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(),
+        dw.dPtr(), M, K, N));
+    addMultiplyAdds((__int128_t)M * K * N);
+  }
+  if (input.backpropErrors && !input.deferredGatherFrom) {
+    input.sub->dfeatures.resize64(((size_t)input.nSpatialSites + input.gradientSums) * K);
     workspace.resize64((size_t)scn_sgemm_ABt_workspace(N, K));
     SCN_CHECKED(scn_sgemm_ABt(ms.ctx, output.sub->dfeatures.dPtr(),
                               shrunkW ? shrunkW->dPtr() : W.dPtr(),
@@ -455,8 +488,8 @@ static void nin_backwards(cudaMemStream &ms,
       items[n++] = {dprelu->dPtr(), MPReLU->dPtr(), PReLU->dPtr(), N, 1};
     items[n++] = {dw.dPtr(), MW.dPtr(), W.dPtr(), (int64_t)K * N, 0};
     items[n++] = {db.dPtr(), MB.dPtr(), B.dPtr(), N, 0};
-    if (updates)
-      updates->insert(updates->end(), items, items + n);
+    if (batch.collectUpdates)
+      batch.updates.insert(batch.updates.end(), items, items + n);
     else
       SCN_CHECKED(
           scn_nag_update_many(ms.ctx, items, n, learningRate, momentum, 1));
@@ -527,7 +560,7 @@ void NetworkInNetworkLayer::backwards(SpatiallySparseBatch &batch,
                                       SpatiallySparseBatchInterface &input,
                                       SpatiallySparseBatchInterface &output,
                                       float learningRate, float momentum) {
-  nin_backwards(memStream, batch.collectUpdates ? &batch.updates : nullptr,
+  nin_backwards(memStream, batch,
                 input, output, nFeaturesIn, nFeaturesOut,
                 nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output)
                     ? &w
@@ -541,6 +574,14 @@ void NetworkInNetworkLayer::activationAhead(
   if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
     nin_activation_ahead(memStream, input, output, pooled, (int)fn, nullptr, dw,
                          db, nullptr, gradsClean);
+}
+void NetworkInNetworkLayer::transposedFilters(SpatiallySparseBatchInterface &input,
+                                              std::vector<scn_filter_item> &items) {
+  nin_transposed_filters(input, nFeaturesOut, W, workspace, items);
+}
+void NetworkInNetworkPReLULayer::transposedFilters(SpatiallySparseBatchInterface &input,
+                                                   std::vector<scn_filter_item> &items) {
+  nin_transposed_filters(input, nFeaturesOut, W, workspace, items);
 }
 // scaleWeights (NetworkInNetworkLayer.cu:203-218; the PReLU layer's is the
 // same, NetworkInNetworkPReLULayer.cu:175-189): bring the mean magnitude of
@@ -666,7 +707,7 @@ void NetworkInNetworkPReLULayer::forwards(
 void NetworkInNetworkPReLULayer::backwards(
     SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
     SpatiallySparseBatchInterface &output, float learningRate, float momentum) {
-  nin_backwards(memStream, batch.collectUpdates ? &batch.updates : nullptr,
+  nin_backwards(memStream, batch,
                 input, output, nFeaturesIn, nFeaturesOut,
                 nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output)
                     ? &w

@@ -450,16 +450,32 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   void *grads[SCN_FILL_MAX];
   size_t sizes[SCN_FILL_MAX];
   int n = 0;
-  for (size_t i = 0; i < layers.size() && n < SCN_FILL_MAX; i++) {
+  for (size_t i = 0; i < layers.size(); i++) {
     SpatiallySparseBatchInterface &input = batch.interfaces[i];
-    input.gradientCleared = layers[i]->addsInputGradient() && input.backpropErrors;
-    if (!input.gradientCleared)
+    const size_t nf = input.featuresPresent.size();
+    // (rows of a left out convolution that was gathered all the same are not used)
+    if (i == 0 || !batch.interfaces[i - 1].deferredGatherFrom)
+      input.gradientSums = 0;
+    const size_t own = (size_t)input.nSpatialSites * nf, sums = input.gradientSums * nf;
+    input.gradientCleared = layers[i]->addsInputGradient() && input.backpropErrors &&
+                            !batch.interfaces[i + 1].deferredGatherFrom;
+    if (!input.gradientCleared && !sums)
       continue;
-    sizes[n] = (size_t)input.nSpatialSites * input.featuresPresent.size();
-    input.sub->dfeatures.resize64(sizes[n]);
-    grads[n++] = input.sub->dfeatures.dPtr();
+    input.sub->dfeatures.resize64(own + sums);
+    sizes[n] = input.gradientCleared ? own + sums : sums;
+    grads[n++] = input.sub->dfeatures.dPtr() + (input.gradientCleared ? 0 : own);
+    if (n == SCN_FILL_MAX) {
+      SCN_CHECKED(scn_fill32_many(memStream.ctx, grads, sizes, n, 0u));
+      n = 0;
+    }
   }
   SCN_CHECKED(scn_fill32_many(memStream.ctx, grads, sizes, n, 0u));
+  std::vector<scn_filter_item> filters;
+  for (size_t i = 0; i < layers.size(); i++)
+    layers[i]->transposedFilters(batch.interfaces[i], filters);
+  for (size_t i = 0; i < filters.size(); i += SCN_FILTERS_MAX)
+    SCN_CHECKED(scn_transpose_filters_many(memStream.ctx, filters.data() + i,
+                                           (int)std::min<size_t>(SCN_FILTERS_MAX, filters.size() - i)));
   batch.updates.clear();
   batch.collectUpdates = true;
   for (int i = (int)layers.size() - 1; i >= 0; i--) {
@@ -633,7 +649,7 @@ float SparseConvNetCUDA::processDataset(SpatiallySparseDataset &dataset,
   multiplyAddCount = 0;
   auto start = std::chrono::system_clock::now();
   std::ofstream f, g;
-  BatchProducer bp(*this, dataset, inputSpatialSize, batchSize);
+  BatchProducer bp(*this, dataset, inputSpatialSize, batchSize, dataset.type == TRAINBATCH);
   if (dataset.type == UNLABELEDBATCH) {
     f.open("unlabelledData.predictions");
     g.open("unlabelledData.probabilities");
@@ -850,9 +866,9 @@ SpatiallySparseDataset BatchProducer::emptyDataset;
 
 BatchProducer::BatchProducer(SparseConvNetCUDA &cnn,
                              SpatiallySparseDataset &dataset, int spatialSize,
-                             int batchSize)
+                             int batchSize, bool unseen)
     : cnn(cnn), batchCounter(-1), dataset(dataset), batchSize(batchSize),
-      spatialSize(spatialSize), stopping(false) {
+      spatialSize(spatialSize), unseen(unseen), stopping(false) {
   assert(batchSize > 0);
   nBatches = ((int)dataset.pictures.size() + batchSize - 1) / batchSize;
   permutation = range((int)dataset.pictures.size());
@@ -897,6 +913,7 @@ void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
   SpatiallySparseBatch &b = cnn.batchPool[cc];
   b.reset();
   b.type = dataset.type;
+  b.unseen = unseen;
   SpatiallySparseBatchInterface &in = b.interfaces[0];
   in.nFeatures = dataset.nFeatures;
   in.spatialSize = spatialSize;
@@ -951,6 +968,38 @@ void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
     std::memcpy(b.hostFeatures.p, features.data(), features.size() * sizeof(float));
   features.clear();
 }
+// Of an unseen training batch the convolutions whose gathered matrix, and that
+// matrix's gradient, the layer behind can do without: no dropout on either side,
+// and shapes that the fused kernels take, forwards and (turned round) backwards.
+static void leaveOutConvolutions(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBatch &b) {
+  std::vector<scn_inverse_item> items;
+  for (size_t i = 0; i + 2 < cnn.layers.size(); ++i) { // (the classifier's gradient has no rows for sums)
+    SpatiallySparseBatchInterface &in = b.interfaces[i], &middle = b.interfaces[i + 1], &out = b.interfaces[i + 2];
+    if ((!dynamic_cast<ConvolutionalLayer *>(cnn.layers[i]) &&
+         !dynamic_cast<ConvolutionalTriangularLayer *>(cnn.layers[i])) ||
+        (!dynamic_cast<NetworkInNetworkLayer *>(cnn.layers[i + 1]) &&
+         !dynamic_cast<NetworkInNetworkPReLULayer *>(cnn.layers[i + 1])))
+      continue;
+    const int nIn = in.nFeatures, N = out.nFeatures, fs = middle.nFeatures / nIn;
+    if ((int)middle.featuresPresent.size() != middle.nFeatures || (int)out.featuresPresent.size() != N ||
+        nIn > 4096 || N > 4096 || !scn_conv_nin_supported_p(fs, nIn, N, SCN_FP32) ||
+        (in.backpropErrors && !scn_conv_nin_supported_p(fs, N, nIn, SCN_FP32)))
+      continue;
+    middle.leftOut = true;
+    const size_t rows = (size_t)middle.nSpatialSites;
+    middle.positions.resize64(scn_positions_pitch(rows) * fs);
+    if (in.backpropErrors) {
+      out.gradientSums = (size_t)b.batchSize * fs;
+      middle.inverse.resize64((size_t)in.nSpatialSites * fs);
+      middle.background.resize64(rows + 2 * (size_t)b.batchSize);
+    }
+    items.push_back({in.deviceGrids, middle.rules.dPtr(), in.backpropErrors ? middle.inverse.dPtr() : nullptr,
+                     in.backpropErrors ? middle.background.dPtr() : nullptr, middle.positions.dPtr(),
+                     (int64_t)rows, in.nSpatialSites, fs});
+  }
+  for (size_t i = 0; i < items.size(); i += SCN_INVERSE_MAX)
+    SCN_CHECKED(scn_rules_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
+}
 // GPU half: the input grids go to HBM, then every layer builds its rule book,
 // all on the slot's stream
 void BatchProducer::preprocessBatchOnDevice(int cc) {
@@ -991,6 +1040,8 @@ void BatchProducer::preprocessBatchOnDevice(int cc) {
     b.labels.copyToGPUAsync(ms);
   }
   buildRuleBooks(cnn, ctx, b);
+  if (b.unseen)
+    leaveOutConvolutions(cnn, ctx, b);
   SCN_CHECKED(scn_sync(ctx));
 }
 void BatchProducer::batchProducerThread(int nThread) {

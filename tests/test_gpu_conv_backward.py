@@ -1,0 +1,183 @@
+"""The backward pass of a convolution without its gathered matrix: dW through the rules, and the input's gradient as a
+convolution of the output's through the rules turned round, background rows included; then whole epochs, in which the
+host classes take that way, against the net-level oracle."""
+import numpy as np
+import pytest
+
+import oracle_net
+from test_gpu_training import pair, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def layer(scn, ctx, d, field, window, batch, density, seed, stride=1):
+    """input grids, their rows, the rules of a convolution [rows x window^d]; sample 1 has no site, sample 2 is full"""
+    rng = np.random.default_rng(seed)
+    vol = field ** d
+    S, K, R, bg, n = [], [], [], [], 0
+    for s in range(batch):
+        keys = np.nonzero(rng.random(vol) < density)[0] if s != 2 else np.arange(vol)
+        keys = keys[:0] if s == 1 else keys
+        full = len(keys) == vol
+        bg.append(-1 if full else n + len(keys))
+        S += [s] * len(keys)
+        K += list(keys)
+        R += list(range(n, n + len(keys)))
+        n += len(keys) + (not full)
+    g, h = scn.Grids(ctx), scn.Grids(ctx)
+    g.build(batch, d, field, np.array(S, np.int32), np.array(K, np.int64), np.array(R, np.int32), np.array(bg, np.int32), n)
+    out = (field - window) // stride + 1
+    rows = g.plan_square(h, field, out, window, stride)
+    fs = window ** d
+    rules = ctx.empty((rows, fs), np.int32)
+    g.fill(h, rules, rows * fs)
+    return g, n, rows, fs, rules, bg
+
+
+@pytest.mark.parametrize("d,field,window,batch,density,nIn,N,stride", [
+    (2, 9, 2, 1, 0.3, 32, 32, 1), (2, 11, 3, 4, 0.2, 32, 36, 1), (3, 6, 2, 5, 0.1, 64, 96, 1), (3, 7, 3, 3, 0.05, 32, 64, 1),
+    (2, 40, 2, 30, 0.15, 96, 128, 1), (2, 13, 3, 6, 0.4, 4, 300, 1), (1, 50, 2, 3, 0.2, 32, 32, 1), (2, 12, 2, 5, 0.3, 160, 64, 2),
+    (3, 20, 2, 9, 0.02, 32, 64, 1)])
+def test_gradients_through_rules(scn, ctx, d, field, window, batch, density, nIn, N, stride):
+    rng = np.random.default_rng(field * window + N)
+    g, n, rows, fs, d_rules, bg = layer(scn, ctx, d, field, window, batch, density, field + N, stride)
+    print("conv backward", d, field, window, batch, nIn, N, "rows", rows, "of", n, flush=True)
+    rules = d_rules.download()
+    x, D = rng.standard_normal((n, nIn), dtype=np.float32), rng.standard_normal((rows, N), dtype=np.float32)
+    W = rng.standard_normal((fs * nIn, N), dtype=np.float32)
+    d_x, d_W = ctx.array(x), ctx.array(W)
+    # the rules turned round
+    inverse = ctx.array(np.full((n, fs), 7, np.int32))
+    pitch = (rows + 15) // 16 * 16
+    background, positions = ctx.array(np.full(rows + 2 * batch, 7, np.int32)), ctx.array(np.full((fs, pitch), 7, np.int32))
+    ctx.rules_inverse_many([(g, d_rules, inverse, background, positions, rows, n, fs)])
+    want = np.full((n, fs), -1, np.int64)
+    for s, b in enumerate(bg):
+        if b >= 0:
+            want[b] = rows + s * fs + np.arange(fs)
+    isBg = np.isin(rules, [b for b in bg if b >= 0])
+    o, f = np.nonzero((rules >= 0) & ~isBg)
+    want[rules[o, f], f] = o
+    assert np.array_equal(inverse.download(), want)
+    assert np.array_equal(positions.download(), np.pad(rules.T, ((0, 0), (0, pitch - rows)), constant_values=-1))
+    got = background.download()
+    assert np.array_equal(got[:rows].astype(np.uint32), (isBg * (1 << np.arange(fs, dtype=np.uint32))).sum(1))
+    for s, b in enumerate(bg):
+        mine = np.nonzero((rules == b).any(1))[0] if b >= 0 else []
+        assert tuple(got[rows + 2 * s:rows + 2 * s + 2]) == ((mine[0], mine[-1]) if len(mine) else (2 ** 31 - 1, -1))
+    only = ctx.array(np.full((fs, pitch), 7, np.int32))  # (what a net's first convolution wants)
+    ctx.rules_inverse_many([(g, d_rules, None, None, only, rows, n, fs)])
+    assert np.array_equal(only.download(), positions.download())
+    # dW, from zero and added to
+    dense = np.where(rules[:, :, None] >= 0, x[np.maximum(rules, 0)], 0).reshape(rows, fs * nIn).astype(np.float64)
+    start = rng.standard_normal(W.shape, dtype=np.float32)
+    for add in (False, True):
+        dW = ctx.array(start)
+        ctx.conv_AtB(d_x, positions, fs, nIn, ctx.array(D), dW, rows, N, accumulate=add)
+        scale = np.abs(dense).T @ np.abs(D) + np.abs(start)
+        assert np.all(np.abs(dW.download() - add * start - dense.T @ D) <= 2e-6 * scale)
+    # the input's gradient
+    Wt = ctx.array(np.full(W.size, 7, np.float32))
+    ctx.transpose_filters_many([(d_W, Wt, fs, nIn, N)])
+    assert np.array_equal(Wt.download().reshape(fs, N, nIn), W.reshape(fs, nIn, N).transpose(0, 2, 1))
+    delta = ctx.array(np.concatenate([D, np.zeros((batch * fs, N), np.float32)]))
+    ctx.background_sums(delta, rows, N, background, fs, batch)
+    got = delta.download()
+    assert np.array_equal(got[:rows], D)
+    sums, size = np.zeros((batch * fs, N)), np.zeros((batch * fs, N))
+    for s, b in enumerate(bg):
+        for q in range(fs):
+            sums[s * fs + q] = D[rules[:, q] == b].astype(np.float64).sum(0) if b >= 0 else 0
+            size[s * fs + q] = np.abs(D[rules[:, q] == b]).astype(np.float64).sum(0) if b >= 0 else 0
+    assert np.all(np.abs(got[rows:] - sums) <= 2e-6 * size)
+    dx = ctx.array(np.full((n, nIn), 7, np.float32))
+    ctx.conv_input_gradient(delta, inverse, fs, N, Wt, dx, n, nIn)
+    want, size = np.zeros((n, nIn)), np.zeros((n, nIn))
+    o, f = np.nonzero(rules >= 0)
+    dA = (D.astype(np.float64) @ W.astype(np.float64).T).reshape(rows, fs, nIn)
+    absA = (np.abs(D).astype(np.float64) @ np.abs(W).astype(np.float64).T).reshape(rows, fs, nIn)
+    np.add.at(want, rules[o, f], dA[o, f])
+    np.add.at(size, rules[o, f], absA[o, f])
+    assert np.all(np.abs(dx.download() - want) <= 4e-6 * size)
+
+
+def test_many_layers_in_one_call(scn, ctx):
+    layers = [layer(scn, ctx, 2, 8 + 3 * k, 2 + k % 2, 1 + k, 0.3, k) for k in range(6)]
+    one = [ctx.array(np.full((n, fs), 7, np.int32)) for _, n, _, fs, _, _ in layers]
+    many = [ctx.array(np.full((n, fs), 7, np.int32)) for _, n, _, fs, _, _ in layers]
+    items = [[(g, rules, inv, None, None, rows, n, fs) for (g, n, rows, fs, rules, _), inv in zip(layers, to)] for to in (one, many)]
+    for it in items[0]:
+        ctx.rules_inverse_many([it])
+    ctx.rules_inverse_many(items[1])
+    for a, b in zip(one, many):
+        assert np.array_equal(a.download(), b.download())
+
+
+def test_refusals(scn, ctx):
+    g, n, rows, fs, rules, _ = layer(scn, ctx, 2, 8, 2, 2, 0.3, 1)
+    buf = ctx.empty((64, 64), np.float32)
+    with pytest.raises(scn.ScnError):
+        ctx.conv_AtB(buf, rules, 0, 32, buf, buf, 4, 4)
+    with pytest.raises(scn.ScnError):
+        ctx.conv_AtB(buf, rules, 4, 5000, buf, buf, 4, 4)  # more channels than the zero row has
+    with pytest.raises(scn.ScnError):
+        ctx.rules_inverse_many([(g, rules, rules, None, None, rows, n, fs)] * 17)
+    with pytest.raises(scn.ScnError):
+        ctx.background_sums(buf, 4, 0, rules, fs, 2)
+
+
+STACKS = {
+    "tri": (True, [("addLeNetLayerMP", 32, 2, 1, 2, 2, 4), ("addLeNetLayerMP", 64, 2, 1, 2, 2, 1), ("addLeNetLayerMP", 64, 2, 1, 1, 1, 3),
+                   ("addTerminalPoolingLayer", 2), ("addSoftmaxLayer",)]),
+    # convolutions one behind the other, without a pooling between them; the last one's output is one site a sample
+    "unpooled": (False, [("addLeNetLayerMP", 32, 3, 1, 1, 1, 1), ("addLeNetLayerMP", 64, 2, 1, 1, 1, 6),
+                         ("addLeNetLayerMP", 32, 2, 1, 3, 2, 1), ("addLeNetLayerMP", 32, 2, 1, 1, 1, 1), ("addSoftmaxLayer",)])}
+
+
+@pytest.mark.parametrize("what,batch,epochs", [(2, 8, 2), (3, 5, 1), (4, 2, 1), ("tri", 4, 2), ("unpooled", 4, 2)])
+def test_epochs_against_the_oracle(scn, what, batch, epochs):
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    rng = np.random.default_rng(5)
+    if isinstance(what, int):
+        cfg = synthetic.config(what, batch=2 * batch + 1)
+        samples = synthetic.make_samples(cfg, 41)
+        triangular = False
+    else:
+        triangular, stack = STACKS[what]
+        lattice = 12
+        cfg = synthetic.Config(what, 2, 3, 10, 2 * batch + 1, lattice, stack)
+        cfg.number = 2
+        samples = []
+        for _ in range(2 * batch + 1):
+            pts = np.array([(a, b) for a in range(lattice) for b in range(lattice - (a if triangular else 0))
+                            if rng.random() < 0.3], np.int32)
+            samples.append((pts, rng.uniform(-1, 1, (len(pts), 3)).astype(np.float32), int(rng.integers(0, 10))))
+    pts, f, label = samples[1]
+    samples[1] = (pts[:0], f[:0], label)  # a sample without a site
+    net, ora = pair(cfg, hostapi, 51, triangular)
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TRAINBATCH)
+    for pts, f, label in samples:
+        ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
+    lr, mu = 0.01, 0.9
+    net.set_training(lr, mu, shuffle=False)
+    for _ in range(epochs):
+        net.processDatasetTrain(ds, batch, lr, mu)
+        for b in range(0, len(samples), batch):  # (the last batch is not full)
+            mine = samples[b:b + batch]
+            S, K, R, bg, feats, n = synthetic.codify(mine, cfg.dimension, cfg.lattice, net.inputSpatialSize,
+                                                     cfg.nInputFeatures)
+            labels = np.array([s[2] for s in mine], np.int32)
+            fwd = ora.forward(len(mine), S, K, R, bg, feats, n, labels)
+            ora.train_step(fwd, labels, lr, mu)
+    for i, l in enumerate(net.layers()):
+        if not l["kind"].startswith("nin"):
+            continue
+        M, W = net.get_weights(i, momentum=True), net.get_weights(i)
+        err = [rel_l2(a, b) for a, b in zip(M, ora.momentum[i]) if a is not None]
+        print("layer", i, "momentum off by", err, flush=True)
+        # (the bar of one batch, a batch's share of rectifiers that a rounding turns among them)
+        assert max(err) <= 1e-4 * epochs * 3
+        for a, b in zip(W, ora.weights[i]):
+            if a is not None:
+                assert np.allclose(a, b, rtol=1e-4 * epochs * 3, atol=3e-6 * epochs)
+    net.close()
