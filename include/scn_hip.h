@@ -444,6 +444,10 @@ int scn_activation_backward_to(scn_ctx *ctx, const float *d_out,
                                float *d_db, float *d_dprelu, int accumulate);
 int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
                       float *d_dW, int64_t M, int K, int N);
+/* scn_sgemm_AtB (accumulate: _acc) and the bias gradient in one: d_db[N] = (or
+ * +=) the column sums of D, where the activation's derivative is in D already. */
+int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *d_dW,
+                       float *d_db, int64_t M, int K, int N, int accumulate);
 /* The backward pass of a convolution without its gathered matrix (no
  * counterpart in the reference, which keeps that matrix and its gradient).
  * scn_rules_inverse_many turns the rules of up to SCN_INVERSE_MAX layers round:
@@ -458,7 +462,8 @@ int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
  * (d_positions, d_background, and d_inverse and d_background may be null: not
  * wanted; fs <= 32.)
  * scn_conv_AtB: scn_sgemm_AtB of what scn_gather_rows would make of d_in through
- * the rules (nIn <= 4096; d_positions aligned to 16 bytes).
+ * the rules, with d_db as scn_sgemm_AtB_sums or null (nIn <= 4096; d_positions
+ * aligned to 16 bytes).
  * The gradient of the input is a convolution of d_D with the rules turned round.
  * d_delta has rows + batch fs rows, those behind the layer's own cleared by the
  * caller; scn_background_sums adds what is to be there.
@@ -488,7 +493,7 @@ int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *items, int n
 int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
                             const float *d_Wt, float *d_din, int64_t inputRows, int nIn);
 int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,
-                 const float *d_D, float *d_dW, int64_t M, int N, int accumulate);
+                 const float *d_D, float *d_dW, float *d_db, int64_t M, int N, int accumulate);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout
  * (NetworkInNetworkLayer.cu:7-25): w[i][j] = W[inPresent[i]][outPresent[j]],
  * W with rows of nOut floats; a null d_inPresent keeps the rows (row i of w
@@ -519,6 +524,10 @@ int scn_gather_rows_backward(scn_ctx *ctx, float *d_din, const float *d_dconv,
  * the count x C elements of dout; the caller zeroes din first. */
 int scn_maxpool_backward(scn_ctx *ctx, float *d_din, const float *d_dout,
                          int64_t count, int C, const int32_t *d_choice);
+/* ... of a pooling behind an activation (any but PReLU), whose derivative it takes
+ * on the way: d_out are the pooling's outputs, each of them the activation it chose. */
+int scn_maxpool_backward_through(scn_ctx *ctx, float *d_din, const float *d_dout, int64_t count,
+                                 int C, const int32_t *d_choice, const float *d_out, int act);
 /* terminalPoolBackProp (TerminalPoolingLayer.cu:48-73): every row listed for
  * sample b before the first negative rule is assigned dout[b] / (number of
  * rows listed); the caller zeroes din first. */

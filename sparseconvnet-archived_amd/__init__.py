@@ -150,7 +150,9 @@ def lib():
         "scn_activation_backward_acc": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),
         "scn_activation_backward_to": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp, C.c_int]),
         "scn_sgemm_AtB_acc": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
-        "scn_conv_AtB": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_conv_AtB": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_sgemm_AtB_sums": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, C.c_int, C.c_int]),
+        "scn_maxpool_backward_through": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, C.c_int]),
         "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
         "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, i64, C.c_int]),
         "scn_background_sums": (C.c_int, [vp, vp, i64, C.c_int, vp, C.c_int, C.c_int]),
@@ -359,9 +361,15 @@ class Context:
         f = lib().scn_sgemm_AtB_acc if accumulate else lib().scn_sgemm_AtB
         _check(f(self.h, d_A.ptr, d_D.ptr, d_dW.ptr, M, K, N))
 
-    def conv_AtB(self, d_in, d_positions, fs, nIn, d_D, d_dW, M, N, accumulate=False):
+    def conv_AtB(self, d_in, d_positions, fs, nIn, d_D, d_dW, M, N, accumulate=False, d_db=None):
         _check(lib().scn_conv_AtB(self.h, d_in.ptr if d_in is not None else None, d_positions.ptr, fs, nIn, d_D.ptr,
-                                  d_dW.ptr, M, N, int(accumulate)))
+                                  d_dW.ptr, d_db.ptr if d_db is not None else None, M, N, int(accumulate)))
+
+    def sgemm_AtB_sums(self, d_A, d_D, d_dW, d_db, M, K, N, accumulate=False):
+        _check(lib().scn_sgemm_AtB_sums(self.h, d_A.ptr, d_D.ptr, d_dW.ptr, d_db.ptr, M, K, N, int(accumulate)))
+
+    def maxpool_backward_through(self, d_din, d_dout, count, C, d_choice, d_out, act):
+        _check(lib().scn_maxpool_backward_through(self.h, d_din.ptr, d_dout.ptr, count, C, d_choice.ptr, d_out.ptr, act))
 
     def rules_inverse_many(self, items):
         """items: (input Grids, d_rules, d_inverse, d_background, d_positions, rows, inputRows, fs) tuples; the three

@@ -63,8 +63,9 @@ bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N);
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
                        const Epilogue &ep, const GatherSource *gs, bool a16);
-// dW += A^T D (gs: the rows of A through rules)
-int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
+// dW += A^T D, db (may be null) += the column sums of D (gs: the rows of A through
+// rules, position by position)
+int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                    long long M, int K, int N, const GatherSource *gs = nullptr);
 // out = A Wt^T; false: the caller's other way, or (transpose) scn_planes_forward
 // on the transpose

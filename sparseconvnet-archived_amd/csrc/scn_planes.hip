@@ -1026,12 +1026,13 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 template <int MT, int NT, bool GATHER>
 __global__ void __launch_bounds__(512, 2)
     k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
-                 float *__restrict__ dW, long long M, int K, int N, int nTiles,
+                 float *__restrict__ dW, float *__restrict__ db, long long M, int K, int N, int nTiles,
                  long long rowsPerSplit, GatherSource gs) {
   constexpr int PL = 3, GM = 8;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
-  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], then a flag
-  int *const sAgain = reinterpret_cast<int *>(sTile + 8 * TILE);
+  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], [8][32 NT], a flag
+  float *const sBias = sTile + 8 * TILE;
+  int *const sAgain = reinterpret_cast<int *>(sBias + 8 * 32 * NT);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
   // (the tiles of a range of rows, which read the same, to one XCD)
@@ -1111,7 +1112,18 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
           acc[h][i][j][v] = 0.f;
+  // the column sums of D, by the workgroups of the first tile of K
+  // (not by two by two tiles, whose registers are full)
+  const bool sums = MT * NT < 4 && db && k0 == 0;
+  float ds[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    ds[j] = 0.f;
   auto compute = [&](const Step &s) {
+    if (sums)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        ds[j] += ((s.d[0][j] + s.d[1][j]) + (s.d[2][j] + s.d[3][j])) + ((s.d[4][j] + s.d[5][j]) + (s.d[6][j] + s.d[7][j]));
     bf16x8 ap[MT][PL], dp[NT][PL];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -1178,7 +1190,21 @@ __global__ void __launch_bounds__(512, 2)
         sTile[wave * TILE + ((i * NT + j) * 16 + v) * 64 + lane] = acc[0][i][j][v] + acc[1][i][j][v];
   if (tid == 0)
     *sAgain = 0;
+  if (sums)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const float both = ds[j] + __shfl_xor(ds[j], 32);
+      if (q == 0)
+        sBias[wave * 32 * NT + NT * c + j] = both;
+    }
   __syncthreads();
+  if (sums && tid < 32 * NT && n0 + tid < N) {
+    float sum = 0.f;
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+      sum += sBias[g * 32 * NT + tid];
+    unsafeAtomicAdd(db + n0 + tid, sum);
+  }
   // element e of the tile: register v of lane l of sub-tile (i, j): row (of dW)
   // MT (8 (v / 4) + 4 (l / 32) + v % 4) + i, column NT (l % 32) + j
   auto add = [&](int e) {
@@ -1255,9 +1281,9 @@ __global__ void __launch_bounds__(512, 2)
 }
 
 template <int MT, int NT, bool GATHER>
-static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
+static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                       long long M, int K, int N, long long splits, const GatherSource &gs) {
-  const size_t lds = ((size_t)8 * 32 * MT * 32 * NT + 1) * sizeof(float);
+  const size_t lds = ((size_t)8 * 32 * MT * 32 * NT + 8 * 32 * NT + 1) * sizeof(float);
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER>),
@@ -1271,17 +1297,17 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW,
   long long rows = (M + splits - 1) / splits;
   rows = (rows + 8 * ATB_STEP - 1) / (8 * ATB_STEP) * (8 * ATB_STEP);
   hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
-                     dim3(512), lds, ctx->stream, A, D, dW, M, K, N, nTiles, rows, gs);
+                     dim3(512), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs);
   return SCN_OK;
 }
 template <int MT, int NT>
-static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, long long M, int K, int N,
+static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db, long long M, int K, int N,
                       long long splits, const GatherSource *gs) {
   if constexpr (MT == 2 && NT == 2) // (not gathered: see below)
-    return launch_atb<MT, NT, false>(ctx, A, D, dW, M, K, N, splits, GatherSource());
+    return launch_atb<MT, NT, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
   else
-    return gs ? launch_atb<MT, NT, true>(ctx, A, D, dW, M, K, N, splits, *gs)
-              : launch_atb<MT, NT, false>(ctx, A, D, dW, M, K, N, splits, GatherSource());
+    return gs ? launch_atb<MT, NT, true>(ctx, A, D, dW, db, M, K, N, splits, *gs)
+              : launch_atb<MT, NT, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
 }
 
 // The tile and the number of row ranges that cost least: rounds of one workgroup
@@ -1289,7 +1315,7 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, l
 // waiting for memory) and `f` to start, to sum and to store, and the atomics.
 // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
 // (The search is 0.1 to 2 us of the host's time, a launch some 5.)
-int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
+int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                    long long M, int K, int N, const GatherSource *gs) {
   static const struct {
     int mt, nt;
@@ -1298,7 +1324,7 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
   int best = 0;
   long long splits = 1;
   double least = 1e300;
-  for (int i = 0; i < (gs ? 3 : 4); ++i) { // (two by two tiles of gathered rows: 264 bytes a lane spilled)
+  for (int i = 0; i < (gs || db ? 3 : 4); ++i) { // (two by two tiles of gathered rows: 264 bytes a lane spilled)
     if ((tile[i].mt == 2 && ((gs ? gs->nIn : K) % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
       continue;
     const long long tiles = (long long)scn_ceil_div(K, 32 * tile[i].mt) * scn_ceil_div(N, 32 * tile[i].nt);
@@ -1319,11 +1345,11 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW,
   SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
   switch (best) {
   case 1:
-    return launch_atb<2, 1>(ctx, A, D, dW, M, K, N, splits, gs);
+    return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, splits, gs);
   case 2:
-    return launch_atb<1, 2>(ctx, A, D, dW, M, K, N, splits, gs);
+    return launch_atb<1, 2>(ctx, A, D, dW, db, M, K, N, splits, gs);
   case 3:
-    return launch_atb<2, 2>(ctx, A, D, dW, M, K, N, splits, gs);
+    return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, splits, gs);
   }
-  return launch_atb<1, 1>(ctx, A, D, dW, M, K, N, splits, gs);
+  return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, splits, gs);
 }

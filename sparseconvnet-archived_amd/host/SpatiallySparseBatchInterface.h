@@ -32,9 +32,11 @@ public:
   // (SparseConvNetCUDA::backwardBatch clears those of a whole pass at once)
   bool gradientCleared = false;
   // a layer's output: the activation's derivative is in dfeatures already (taken
-  // over the outputs of the pooling behind it); a pooling's: sub->dactivated holds
-  // what it is to spread
+  // over the outputs of the pooling behind it), and, with activationAhead, the bias
+  // gradient has been summed; a pooling's: sub->dactivated holds what it is to
+  // spread (activationAhead), or it takes the derivative of `through` itself
   bool activationDone = false, activationAhead = false;
+  int through = -1;
   // A convolution's output in a batch nobody looks into (SpatiallySparseBatch::
   // unseen) whose matrix and gradient are left out: the rules turned round
   // (scn_rules_inverse_many; all but the positions empty where no gradient of its

@@ -389,27 +389,30 @@ static void nin_activation_ahead(cudaMemStream &ms,
   if (!output.backpropErrors || (int)pooled.featuresPresent.size() != N ||
       pooled.sub->features.size64() != (size_t)pooled.nSpatialSites * N)
     return;
+  output.activationDone = true;
+  if (!PReLU) {
+    pooled.through = act;
+    return;
+  }
   const bool clean = nin_gradients(dw, db, dprelu, K, N, gradsClean);
   pooled.sub->dactivated.resize64((size_t)pooled.nSpatialSites * N);
   SCN_CHECKED(scn_activation_backward_to(
       ms.ctx, pooled.sub->features.dPtr(), pooled.sub->dfeatures.dPtr(),
       pooled.sub->dactivated.dPtr(), pooled.nSpatialSites, N, act,
-      PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
-      dprelu ? dprelu->dPtr() : nullptr, clean));
-  pooled.activationAhead = true;
-  output.activationDone = true;
+      PReLU->dPtr(), db.dPtr(), dprelu->dPtr(), clean));
+  pooled.activationAhead = output.activationAhead = true;
 }
 // A layer behind a convolution that was left out: dW from the convolution's
 // input, and that input's gradient from this layer's output's, through the rules
 // turned round (transposed: the weights for that, scn_transpose_filters_many).
 static void conv_nin_gradients(cudaMemStream &ms, SpatiallySparseBatchInterface &middle,
-                               SpatiallySparseBatchInterface &output, vectorCUDA<float> &dw,
+                               SpatiallySparseBatchInterface &output, vectorCUDA<float> &dw, float *db,
                                vectorCUDA<float> &transposed, bool clean, int batchSize) {
   SpatiallySparseBatchInterface &src = *middle.deferredGatherFrom;
   const int64_t M = output.nSpatialSites;
   const int N = output.nFeatures, nIn = src.nFeatures, fs = middle.nFeatures / nIn;
   SCN_CHECKED(scn_conv_AtB(ms.ctx, src.sub->features.dPtr(), middle.positions.dPtr(), fs, nIn,
-                           output.sub->dfeatures.dPtr(), dw.dPtr(), M, N, clean));
+                           output.sub->dfeatures.dPtr(), dw.dPtr(), db, M, N, clean));
   addMultiplyAdds((__int128_t)M * fs * nIn * N);
   if (!src.backpropErrors)
     return;
@@ -446,14 +449,20 @@ static void nin_backwards(cudaMemStream &ms, SpatiallySparseBatch &batch,
   const int N = (int)output.featuresPresent.size();
   const bool clean = nin_gradients(dw, db, dprelu, K, N, gradsClean);
   gradsClean = false;
-  if (!output.activationDone)
+  // (the bias gradient goes with dW where the derivative has been taken, or is 1)
+  const bool sums = output.activationDone ? !output.activationAhead : act == SOFTMAX || act == NOSIGMOID;
+  if (!output.activationDone && !sums)
     SCN_CHECKED((clean ? scn_activation_backward_acc : scn_activation_backward)(
         ms.ctx, output.sub->features.dPtr(), output.sub->dfeatures.dPtr(), M, N,
         act, PReLU ? PReLU->dPtr() : nullptr, db.dPtr(),
         dprelu ? dprelu->dPtr() : nullptr));
-  output.activationDone = false;
+  output.activationDone = output.activationAhead = false;
   if (input.deferredGatherFrom) {
-    conv_nin_gradients(ms, input, output, dw, workspace, clean, batch.batchSize);
+    conv_nin_gradients(ms, input, output, dw, sums ? db.dPtr() : nullptr, workspace, clean, batch.batchSize);
+  } else if (sums) {
+    SCN_CHECKED(scn_sgemm_AtB_sums(ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(), dw.dPtr(),
+                                   db.dPtr(), M, K, N, clean));
+    addMultiplyAdds((__int128_t)M * K * N);
   } else {
     SCN_CHECKED((clean ? scn_sgemm_AtB_acc : scn_sgemm_AtB)(
         ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(),
@@ -800,10 +809,16 @@ static void pool_backwards(cudaMemStream &ms,
   const size_t nf = output.featuresPresent.size();
   clear_gradient(ms, input, nf);
   vectorCUDA<float> &d = output.activationAhead ? output.sub->dactivated : output.sub->dfeatures;
+  if (output.through >= 0)
+    SCN_CHECKED(scn_maxpool_backward_through(
+        ms.ctx, input.sub->dfeatures.dPtr(), d.dPtr(), output.nSpatialSites, (int)nf,
+        output.sub->poolingChoices.dPtr(), output.sub->features.dPtr(), output.through));
+  else
+    SCN_CHECKED(scn_maxpool_backward(
+        ms.ctx, input.sub->dfeatures.dPtr(), d.dPtr(),
+        output.nSpatialSites, (int)nf, output.sub->poolingChoices.dPtr()));
   output.activationAhead = false;
-  SCN_CHECKED(scn_maxpool_backward(
-      ms.ctx, input.sub->dfeatures.dPtr(), d.dPtr(),
-      output.nSpatialSites, (int)nf, output.sub->poolingChoices.dPtr()));
+  output.through = -1;
 }
 void MaxPoolingLayer::backwards(SpatiallySparseBatch &batch,
                                 SpatiallySparseBatchInterface &input,

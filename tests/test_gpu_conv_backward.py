@@ -76,6 +76,10 @@ def test_gradients_through_rules(scn, ctx, d, field, window, batch, density, nIn
         ctx.conv_AtB(d_x, positions, fs, nIn, ctx.array(D), dW, rows, N, accumulate=add)
         scale = np.abs(dense).T @ np.abs(D) + np.abs(start)
         assert np.all(np.abs(dW.download() - add * start - dense.T @ D) <= 2e-6 * scale)
+    dW, db = ctx.array(start), ctx.array(start[0])
+    ctx.conv_AtB(d_x, positions, fs, nIn, ctx.array(D), dW, rows, N, d_db=db)
+    assert np.all(np.abs(dW.download() - dense.T @ D) <= 2e-6 * scale)
+    assert np.all(np.abs(db.download() - D.astype(np.float64).sum(0)) <= 2e-6 * np.abs(D).astype(np.float64).sum(0))
     # the input's gradient
     Wt = ctx.array(np.full(W.size, 7, np.float32))
     ctx.transpose_filters_many([(d_W, Wt, fs, nIn, N)])
@@ -101,6 +105,43 @@ def test_gradients_through_rules(scn, ctx, d, field, window, batch, density, nIn
     assert np.all(np.abs(dx.download() - want) <= 4e-6 * size)
 
 
+# every tile that sums take; ragged rows and columns; added to and not
+@pytest.mark.parametrize("M,K,N", [(1, 32, 32), (130, 34, 31), (1000, 66, 100), (40001, 12, 32), (30011, 256, 96), (70003, 432, 128)])
+def test_weight_and_bias_gradients_in_one(scn, ctx, M, K, N):
+    rng = np.random.default_rng(M + K + N)
+    A, D = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((M, N), dtype=np.float32)
+    start = rng.standard_normal((K + 1, N), dtype=np.float32)
+    print("products with sums", M, K, N, flush=True)
+    for add in (False, True):
+        dW, db = ctx.array(start[:K]), ctx.array(start[K])
+        ctx.sgemm_AtB_sums(ctx.array(A), ctx.array(D), dW, db, M, K, N, accumulate=add)
+        scale = np.abs(A).astype(np.float64).T @ np.abs(D).astype(np.float64) + np.abs(start[:K])
+        assert np.all(np.abs(dW.download() - add * start[:K] - A.astype(np.float64).T @ D) <= 2e-6 * scale)
+        size = np.abs(D).astype(np.float64).sum(0) + np.abs(start[K])
+        assert np.all(np.abs(db.download() - add * start[K] - D.astype(np.float64).sum(0)) <= 2e-6 * size)
+
+
+@pytest.mark.parametrize("n,C", [(1, 4), (2001, 32), (9000, 3), (20000, 96)])
+@pytest.mark.parametrize("act", ["NOSIGMOID", "RELU", "VLEAKYRELU", "LEAKYRELU", "TANH", "SIGMOID"])
+def test_pooling_gradient_takes_the_derivative(scn, ctx, n, C, act):
+    rng = np.random.default_rng(n + C)
+    a = getattr(scn, act)
+    out = rng.uniform(-1, 1, (n, C)).astype(np.float32)
+    out[rng.random((n, C)) < 0.3] = 0
+    g = rng.standard_normal((n, C)).astype(np.float32)
+    choice = ctx.array((rng.integers(0, 700, (n, C)) * C + np.arange(C)).astype(np.int32))
+    dB = ctx.array(np.zeros(C, np.float32))
+    two, one = (ctx.array(np.zeros((700, C), np.float32)) for _ in range(2))
+    d = ctx.array(g)
+    ctx.activation_backward(ctx.array(out), d, n, C, a, None, dB, None)
+    ctx.maxpool_backward(two, d, n, C, choice)
+    ctx.maxpool_backward_through(one, ctx.array(g), n, C, choice, ctx.array(out), a)
+    # (the same products, added in another order)
+    size = np.zeros(700 * C)
+    np.add.at(size, choice.download().ravel(), np.abs(g).ravel().astype(np.float64))
+    assert np.all(np.abs(one.download().ravel() - two.download().ravel()) <= 1e-6 * size)
+
+
 def test_many_layers_in_one_call(scn, ctx):
     layers = [layer(scn, ctx, 2, 8 + 3 * k, 2 + k % 2, 1 + k, 0.3, k) for k in range(6)]
     one = [ctx.array(np.full((n, fs), 7, np.int32)) for _, n, _, fs, _, _ in layers]
@@ -124,6 +165,8 @@ def test_refusals(scn, ctx):
         ctx.rules_inverse_many([(g, rules, rules, None, None, rows, n, fs)] * 17)
     with pytest.raises(scn.ScnError):
         ctx.background_sums(buf, 4, 0, rules, fs, 2)
+    with pytest.raises(scn.ScnError):
+        ctx.maxpool_backward_through(buf, buf, 4, 4, rules, buf, scn.PRELU)  # its slopes' gradient needs a pass of its own
 
 
 STACKS = {
