@@ -50,6 +50,10 @@ public:
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().
   std::vector<SparseGrid> grids;
+  // the last batch's, empty, for the next one's to be built in: ten producers that
+  // allocate and free a hundred grids each hold one another up (a batch's half on
+  // the CPU 0.6 to 1.7 ms, and 0.45 to 0.65 for most of them without)
+  std::vector<SparseGrid> spareGrids;
   scn_grids *deviceGrids;
   bool ownsDeviceGrids;
   vectorCUDA<int> rules;

@@ -345,6 +345,11 @@ SpatiallySparseBatchInterface::~SpatiallySparseBatchInterface() {
 void SpatiallySparseBatchInterface::reset() {
   featuresPresent.resize(0);
   nSpatialSites = 0;
+  for (auto &g : grids) {
+    g.backgroundCol = -1;
+    g.mp.clear();
+    spareGrids.push_back(std::move(g));
+  }
   grids.resize(0);
   rules.resize(0);
   backpropErrors = false;

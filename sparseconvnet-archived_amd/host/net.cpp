@@ -923,7 +923,12 @@ void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
     Picture *pic = dataset.pictures[permutation[i]]->distort(rng, dataset.type);
     b.sampleNumbers.push_back(permutation[i]);
     b.batchSize++;
-    in.grids.push_back(SparseGrid());
+    if (in.spareGrids.empty()) {
+      in.grids.push_back(SparseGrid());
+    } else {
+      in.grids.push_back(std::move(in.spareGrids.back()));
+      in.spareGrids.pop_back();
+    }
     b.labels.hVector().push_back(pic->label);
     pic->codifyInputData(in.grids.back(), in.sub->features.hVector(),
                          in.nSpatialSites, in.spatialSize);

@@ -7,7 +7,10 @@
 
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 #include <memory>
+#include <mutex>
+#include <utility>
 #include "BatchProducer.h"
 #include "SparseConvNet.h"
 #include "SparseConvNetCUDA.h"
@@ -24,6 +27,8 @@ struct scnh_net {
   int readyAtStart = 0;  // slots that held a finished batch when the clock started
   float *allProbs = nullptr; // where a stream pass leaves every batch's probabilities
   int64_t allProbsCapacity = 0;
+  PinnedStage readBack; // what scnh_get_weights reads through
+  std::mutex readBackMutex;
 };
 struct scnh_dataset {
   SpatiallySparseDataset ds;
@@ -158,24 +163,44 @@ static void put(vectorCUDA<float> &v, const float *src) {
   std::copy(src, src + h.size(), h.begin());
   v.copyToGPU();
 }
-static void get(vectorCUDA<float> &v, float *out) {
-  if (!out)
+// A layer's vectors, written to pinned memory by kernels and waited for once (a
+// blocking copy of each to ordinary memory takes 18 us, whatever its size: 0.6 ms
+// of reading a net of seven such layers back)
+static void get(scnh_net *net, std::initializer_list<std::pair<vectorCUDA<float> *, float *>> vectors) {
+  std::lock_guard<std::mutex> lock(net->readBackMutex);
+  scn_ctx *ctx = net->cnn->memStream.ctx;
+  auto room = [](size_t n) { return (n + 3) & ~(size_t)3; };
+  size_t total = 0;
+  for (auto &v : vectors)
+    if (v.second)
+      total += room(v.first->size64());
+  if (total == 0)
     return;
-  SCN_CHECKED(scn_d2h(scnDefaultContext(), out, v.dPtr(),
-                      v.size64() * sizeof(float)));
+  net->readBack.reserve(total * sizeof(float));
+  float *at = net->readBack.as<float>();
+  for (auto &v : vectors)
+    if (v.second) {
+      SCN_CHECKED(scn_copy(ctx, at, v.first->dPtr(), v.first->size64() * sizeof(float)));
+      at += room(v.first->size64());
+    }
+  SCN_CHECKED(scn_sync(ctx));
+  at = net->readBack.as<float>();
+  for (auto &v : vectors)
+    if (v.second) {
+      std::copy(at, at + v.first->size64(), v.second);
+      at += room(v.first->size64());
+    }
 }
 int scnh_get_weights(scnh_net *net, int layer, int momentum, float *W,
                      float *B, float *prelu) {
   SpatiallySparseLayer *l = net->cnn->layers.at(layer);
   if (auto *c = dynamic_cast<NetworkInNetworkLayer *>(l)) {
-    get(momentum ? c->MW : c->W, W);
-    get(momentum ? c->MB : c->B, B);
+    get(net, {{momentum ? &c->MW : &c->W, W}, {momentum ? &c->MB : &c->B, B}});
     return 0;
   }
   if (auto *c = dynamic_cast<NetworkInNetworkPReLULayer *>(l)) {
-    get(momentum ? c->MW : c->W, W);
-    get(momentum ? c->MB : c->B, B);
-    get(momentum ? c->MPReLU : c->PReLU, prelu);
+    get(net, {{momentum ? &c->MW : &c->W, W}, {momentum ? &c->MB : &c->B, B},
+              {momentum ? &c->MPReLU : &c->PReLU, prelu}});
     return 0;
   }
   return -1;

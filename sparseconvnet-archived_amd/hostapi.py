@@ -275,12 +275,12 @@ class Net:
         return lib().scnh_input_spatial_size(self.h)
 
     def layers(self):
-        out = []
-        for i in range(lib().scnh_n_layers(self.h)):
-            a, b, c = C.c_int(), C.c_int(), C.c_int()
-            kind = lib().scnh_layer_info(self.h, i, C.byref(a), C.byref(b), C.byref(c))
-            out.append(dict(kind=LAYER_KINDS[kind], nIn=a.value, nOut=b.value, act=c.value))
-        return out
+        return [self._layer(i) for i in range(lib().scnh_n_layers(self.h))]
+
+    def _layer(self, i):
+        a, b, c = C.c_int(), C.c_int(), C.c_int()
+        kind = lib().scnh_layer_info(self.h, i, C.byref(a), C.byref(b), C.byref(c))
+        return dict(kind=LAYER_KINDS[kind], nIn=a.value, nOut=b.value, act=c.value)
 
     def set_weights(self, layer, W, B, prelu=None):
         W = np.ascontiguousarray(W, np.float32)
@@ -291,7 +291,7 @@ class Net:
 
     def get_weights(self, layer, momentum=False):
         """(W [K x N], B [N], PReLU slopes [N] or None) of a NiN layer, or their momentum vectors"""
-        l = self.layers()[layer]
+        l = self._layer(range(lib().scnh_n_layers(self.h))[layer])
         W = np.empty((l["nIn"], l["nOut"]), np.float32)
         B = np.empty(l["nOut"], np.float32)
         pr = np.empty(l["nOut"], np.float32) if l["kind"] == "nin_prelu" else None
