@@ -448,6 +448,7 @@ int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
  * +=) the column sums of D, where the activation's derivative is in D already. */
 int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *d_dW,
                        float *d_db, int64_t M, int K, int N, int accumulate);
+#define SCN_IMAGES_MAX 32
 /* The backward pass of a convolution without its gathered matrix (no
  * counterpart in the reference, which keeps that matrix and its gradient).
  * scn_rules_inverse_many turns the rules of up to SCN_INVERSE_MAX layers round:

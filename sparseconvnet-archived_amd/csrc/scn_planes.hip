@@ -46,6 +46,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[PL]) {
     p[l] = __builtin_bit_cast(bf16x8, uint4{w[0][l], w[1][l], w[2][l], w[3][l]});
 }
 
+bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
+
 // Rows that are known on the device only.  Which kernel takes a layer depends
 // on their number; where either may be right both are launched, and one of them
 // finds that it is not its.
@@ -144,6 +146,12 @@ __device__ __forceinline__ void barrier_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A kilobyte of global memory straight into LDS, 16 bytes a lane, lane after lane
+// from `lds`.  (The compiler does not know of it: see lines_landed and w_landed.)
+__device__ __forceinline__ void dma_kilobyte(unsigned lds, const unsigned char *from) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(from) : "memory", "m0");
 }
 
 // A workgroup of WAVES wavefronts owns 32 WAVES MT rows x 32 NT columns, a
@@ -289,12 +297,7 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
       for (int u = 0; u < (CHUNKS + WAVES - 1) / WAVES; ++u) {
         const int chunk = wave0 + WAVES * u;
         if ((u + 1) * WAVES <= CHUNKS || chunk < CHUNKS) {
-          const unsigned lds = ldsW + (unsigned)(buf * BUF_BYTES + chunk * 1024);
-          const unsigned char *const from = src + chunk * 1024;
-          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                       :
-                       : "s"(lds), "v"(from)
-                       : "memory", "m0");
+          dma_kilobyte(ldsW + (unsigned)(buf * BUF_BYTES + chunk * 1024), src + chunk * 1024);
         }
       }
     }
@@ -734,6 +737,363 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
+// Of the requests a wavefront has made, all but the last N have landed.
+template <int N> __device__ __forceinline__ void lines_landed() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N < 63 ? N : 63) : "memory");
+}
+
+// The same contraction with both operands through LDS: the rows of A by whole
+// lines, W from its image, by requests that need no registers (dma_kilobyte), D - 1
+// blocks of 32 k ahead.  k_nin_planes fetches a row 16 bytes a lane, 32 rows to an
+// instruction, and a block ahead: layers of some 10000 rows spent their time waiting
+// for those loads, and wide ones went through their rows once for every 32 or 64
+// columns.  Here a workgroup of RW by CW wavefronts owns 32 MT RW rows x 32 NT CW
+// columns, a wavefront 32 MT x 32 NT of them.
+//
+// A block's slot: its rows, a line (128 bytes) each, whose eight pieces are stored
+// rotated by the row (piece ^ row % 8, by what each lane asks for), so that eight
+// rows' reads of one piece lie on all banks; then its chunks of the image.  Units,
+// splitting under the MFMAs and the order of all sums are k_nin_planes': the same
+// bits.  One barrier a block, before its second step's MFMAs: behind it the next
+// block may be read and the last one's slot is asked for again.
+//
+// Straight code that is run once is fetched from L2 by every compute unit: an
+// epilogue with a branch an element took 1.1 us a tile, and takes 0.4.
+//
+// Microseconds, the rows written by a kernel before, k_nin_planes with its image
+// (where it takes one) -> here with the image made: three planes, through rules,
+// 28400 x 256 x 96 20.6 -> 16.1, 11400 x 384 x 128 17.7 -> 14.4, 6160 x 1280 x 480
+// 71 -> 45, 2250 x 1920 x 640 61 -> 43; not gathered 11434 x 512 x 96 30 -> 21,
+// 139000 x 128 x 384 136 -> 116; one plane, 41600 x 640 x 320 60 -> 46, 2176 x 2560 x
+// 800 46 -> 25, 140000 x 384 x 128 47 -> 37.  With the chip full k_nin_planes' (2, 2)
+// tiles of three planes stay ahead on gathered rows: 1.36 M x 1728 x 64 1483 against
+// 1797.
+
+template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER>
+__global__ void __launch_bounds__(64 * RW * CW, 2)
+    k_nin_lines(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
+                int K, int N, Epilogue ep, GatherSource gs, int nSplits, RowRange rows, PlainW plain) {
+  constexpr int WAVES = RW * CW, THREADS = 64 * WAVES;
+  constexpr int ROWS = 32 * MT * RW, TW = NT * CW, NW = 32 * TW;
+  constexpr int A_CHUNKS = ROWS / 8, W_CHUNKS = TW * PL * 2;
+  constexpr int A_PER = (A_CHUNKS + WAVES - 1) / WAVES, W_PER = (W_CHUNKS + WAVES - 1) / WAVES, PER = A_PER + W_PER;
+  constexpr int A_BYTES = A_CHUNKS * 1024, SLOT = (A_CHUNKS + W_CHUNKS) * 1024;
+  extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [D][SLOT], then the rules
+  M = rows.live(M);
+  const unsigned tiles = (unsigned)((M + ROWS - 1) / ROWS) * nSplits;
+  if (blockIdx.x >= tiles)
+    return;
+  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, q = lane >> 5;
+  const int cg = wave % CW, rg = wave / CW;
+  const int split = tileOf % nSplits;
+  const long long wgRow0 = (long long)(tileOf / nSplits) * ROWS;
+  const long long row0 = wgRow0 + rg * 32 * MT;
+  const int n0 = split * NW + cg * 32 * NT; // this wavefront's columns
+  const int T = K / 32;
+  int *const sRules = reinterpret_cast<int *>(sW + D * SLOT);
+  const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)sW;
+
+  // ---- requests
+  const unsigned char *wSrc[W_PER];
+  unsigned wDst[W_PER];
+  const int lastTile = (N + 31) / 32 - 1;
+#pragma unroll
+  for (int u = 0; u < W_PER; ++u) {
+    int x = wave + WAVES * u;
+    x = x < W_CHUNKS ? x : W_CHUNKS - 1; // (past the end: the last one again)
+    int tile = split * TW + x / (2 * PL);
+    tile = tile < lastTile ? tile : lastTile;
+    wSrc[u] = image + ((long long)tile * T * (2 * PL) + x % (2 * PL)) * 1024 + 16 * lane;
+    wDst[u] = A_BYTES + x * 1024;
+  }
+  const unsigned char *rowPtr[A_PER];
+  int f = 0, ch = 0;
+  const int piece = 16 * ((lane & 7) ^ (lane >> 3));
+  auto aim = [&]() {
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u) {
+      const int x = wave + WAVES * u;
+      const int r = 8 * (x < A_CHUNKS ? x : A_CHUNKS - 1) + (lane >> 3);
+      if (GATHER) {
+        const int rule = sRules[r * gs.fs + f];
+        rowPtr[u] = (rule >= 0 ? Ab + (long long)rule * gs.nIn * 4 : reinterpret_cast<const unsigned char *>(gs.zeros)) + piece;
+      } else {
+        long long m = wgRow0 + r;
+        m = m < M ? m : M - 1;
+        rowPtr[u] = Ab + m * K * 4 + piece;
+      }
+    }
+  };
+  auto fetch_w = [&](int t, int slot, int u) {
+    dma_kilobyte(lds0 + slot * SLOT + wDst[u], wSrc[u] + (long long)t * (2 * PL * 1024));
+  };
+  auto fetch_a = [&](int slot, int u) {
+    const int x = wave + WAVES * u;
+    dma_kilobyte(lds0 + slot * SLOT + (x < A_CHUNKS ? x : A_CHUNKS - 1) * 1024, rowPtr[u] + ch * 4);
+  };
+  auto advance = [&]() { // to the next block's rows
+    ch += 32;
+    if (GATHER && ch == gs.nIn) {
+      ch = 0;
+      if (++f < gs.fs)
+        aim();
+    }
+  };
+
+  // ---- operands
+  const unsigned char *const aLane = sW + (rg * 32 * MT + c) * 128;
+  const int swizzle = c & 7;
+  const unsigned char *const wLane = sW + A_BYTES + cg * NT * PL * 2048 + lane * 16;
+  floatx4 raw[2];
+  auto read_a = [&](int slot, int u) { // unit u of a block: (step, row tile)
+    const unsigned char *const p = aLane + slot * SLOT + (u % MT) * 4096;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      raw[h] = *reinterpret_cast<const floatx4 *>(p + (((4 * (u / MT) + 2 * q + h) ^ swizzle) * 16));
+  };
+  unsigned ap[2][PL][4]; // words of an MFMA operand: two k each
+  auto a_split = [&](int dst, int p) { // a quarter of it
+    const floatx4 x = raw[p / 2];
+    unsigned w[PL];
+    split2<PL>(x[2 * (p % 2)], x[2 * (p % 2) + 1], w);
+#pragma unroll
+    for (int l = 0; l < PL; ++l) {
+      asm volatile("" : "+v"(w[l])); // (here, and not where it is used)
+      ap[dst][l][p] = w[l];
+    }
+  };
+  auto operand = [&](int src, int l) {
+    return __builtin_bit_cast(bf16x8, uint4{ap[src][l][0], ap[src][l][1], ap[src][l][2], ap[src][l][3]});
+  };
+  constexpr int BB = NT == 1 ? 2 : 1; // a single tile has no other's MFMAs to be read under
+  bf16x8 b[BB][NT][PL];
+  auto read_b = [&](int slot, int s, int j) {
+#pragma unroll
+    for (int l = 0; l < PL; ++l)
+      b[s % BB][j][l] = *reinterpret_cast<const bf16x8 *>(wLane + slot * SLOT + ((j * PL + l) * 2 + s) * 1024);
+  };
+
+  // ---- prologue
+  ColEpilogue col[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + 32 * j + c;
+    col[j] = load_col(ep, n < N ? n : N - 1);
+  }
+  const int first = T < D - 1 ? T : D - 1;
+  if (GATHER) {
+    const long long begin = wgRow0 * gs.fs, last = M * gs.fs - 1;
+    for (int i = tid; i < ROWS * gs.fs; i += THREADS) {
+      const long long r = begin + i;
+      sRules[i] = gs.rules[r < last ? r : last];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) // (asked for now: they come with the rules)
+    asm volatile("" : "+v"(col[j].pb), "+v"(col[j].slope));
+  __syncthreads();
+  aim();
+#pragma unroll 1
+  for (int t = 0; t < first; ++t) {
+#pragma unroll
+    for (int u = 0; u < W_PER; ++u)
+      fetch_w(t, t, u);
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u)
+      fetch_a(t, u);
+    advance();
+  }
+  if (first == D - 1)
+    lines_landed<PER *(D - 2)>();
+  else
+    lines_landed<0>();
+  barrier_lds();
+
+  constexpr int NACC = PL > 1 ? 2 : 1;
+  floatx16 acc[NACC][MT][NT];
+#pragma unroll
+  for (int h = 0; h < NACC; ++h)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[h][i][j][v] = 0.f;
+
+  int last = D - 1, cur = 0, next = 1; // slots of blocks t - 1, t and t + 1
+  read_a(0, 0);
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    read_b(0, 0, j);
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    a_split(0, p);
+  read_a(0, 1);
+
+  constexpr int PRODUCTS = PL * (PL + 1) / 2;
+  auto tile = [&](int s, int i, int j, int src) {
+#pragma unroll
+    for (int x = 0; x < PL; ++x)
+#pragma unroll
+      for (int y = 0; x + y < PL; ++y) {
+        floatx16 &d = acc[x + y == 0 ? 0 : NACC - 1][i][j];
+        d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(src, x), b[s % BB][j][y], d, 0, 0, 0);
+      }
+  };
+  // vector instructions to go with an MFMA: the splitting, dealt out to all tiles but the first
+  constexpr int VALU = ((PL == 1 ? 4 : PL == 2 ? 24 : 44) + PRODUCTS * (NT > 1 ? NT - 1 : 1) - 1) / (PRODUCTS * (NT > 1 ? NT - 1 : 1)) + 1;
+  auto deal = [&]() {
+#pragma unroll
+    for (int i = 0; i < PRODUCTS; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x320, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int UNITS = 2 * MT, SECOND = MT; // the first unit of the second step: the barrier before it
+  auto block = [&](int t, auto steady) {     // steady: with a block to ask for
+    const bool more = steady || t + D - 1 < T; // uniform
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int s = u / MT, i = u % MT, src = u & 1;
+      if (u == SECOND) {
+        // The next block has landed (those asked for behind it may be under way), and
+        // nobody reads the last one any more.
+        if (steady || t + D - 1 <= T) // uniform
+          lines_landed<PER *(D - 3)>();
+        else
+          lines_landed<0>();
+        asm volatile("s_barrier" ::: "memory");
+      }
+      if (MT == 1 && u == SECOND)
+        read_a(next, 0);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (NT == 1) {
+          if (i == MT - 1)
+            read_b(s ? next : cur, s ^ 1, 0);
+        }
+        tile(s, i, j, src);
+        if (NT > 1 && i == MT - 1)
+          read_b(s ? next : cur, s ^ 1, j);
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (j == (NT == 1 || !(MT == 1 && u == SECOND) ? p * NT / 4 : 1 + p * (NT - 1) / 4))
+            a_split(src ^ 1, p);
+        if (j == NT - 1) // (split: its registers take the next but one)
+          if (MT > 1)
+            read_a(u + 2 < UNITS ? cur : next, (u + 2) % UNITS);
+          else if (u == SECOND)
+            read_a(next, 1);
+        deal();
+        if (more && u >= SECOND) {
+          constexpr int G = MT * NT;
+          const int g = i * NT + j;
+#pragma unroll
+          for (int x = g * PER / G; x < (g + 1) * PER / G; ++x) {
+            if (x < W_PER)
+              fetch_w(t + D - 1, last, x);
+            else
+              fetch_a(last, x - W_PER);
+          }
+        }
+      }
+    }
+    if (more)
+      advance();
+    last = cur, cur = next, next = next == D - 1 ? 0 : next + 1;
+  };
+  int t = 0;
+#pragma unroll 1
+  for (; t + D - 1 < T; ++t)
+    block(t, std::true_type());
+#pragma unroll 1
+  for (; t < T; ++t)
+    block(t, std::false_type());
+
+  // ---- epilogue: register v of a tile is row 8 (v / 4) + 4 q + v % 4
+  if constexpr (NACC == 2) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[0][i][j][v] += acc[NACC - 1][i][j][v];
+  }
+  unsigned long long again = 0; // results to be taken from the operands themselves
+  if constexpr (PL == 3) {
+    float none[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; // 0 sum: NaN for a sum that is not finite
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          none[v % 8] = fmaf(acc[0][i][j][v], 0.f, none[v % 8]);
+    if (((none[0] + none[1]) + (none[2] + none[3])) + ((none[4] + none[5]) + (none[6] + none[7])) != 0.f) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (doubtful<PL>(acc[0][i][j][v]))
+              again |= 1ull << ((i * NT + j) * 16 + v);
+    }
+  }
+  {
+    // (what lies past the last row, or in no column, is past the buffer's end: not
+    // stored, without a branch to each)
+    const long long left = ((M - row0) * N - n0) * 4;
+    const __amdgpu_buffer_rsrc_t to =
+        __builtin_amdgcn_make_buffer_rsrc(out + row0 * N + n0, 0, (int)(left < 0 ? 0 : left < 0x40000000 ? left : 0x40000000),
+                                          0x00020000);
+    const unsigned pitch = 4u * (unsigned)N;
+    unsigned at[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      at[j] = n0 + 32 * j + c < N ? (unsigned)(4 * q) * pitch + 128u * j + 4u * c : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[0][i][j][v], col[j])), to, at[j], 0, 0);
+          at[j] += v % 4 == 3 ? 5 * pitch : pitch;
+        }
+  }
+  if constexpr (PL == 3) {
+    if (!__any(again != 0))
+      return;
+#pragma unroll 1
+    for (int e = 0; e < MT * NT; ++e) {
+      const unsigned mine = (unsigned)(again >> (16 * e)) & 0xffffu;
+      if (!__any(mine != 0))
+        continue;
+      const int i = e / NT, j = e % NT;
+      long long m = row0 + 32 * i + c;
+      m = m < M ? m : M - 1;
+      const int n = n0 + 32 * j + c, nn = n < N ? n : N - 1;
+      const floatx16 exact = tile_f32<GATHER>(A, gs, sRules + (m - wgRow0) * gs.fs, plain, m, nn, K, N, mine);
+      const ColEpilogue last = load_col(ep, nn);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const long long r = row0 + 32 * i + 8 * (v / 4) + 4 * q + v % 4;
+        if ((mine >> v & 1) && r < M && n < N)
+          out[r * N + n] = finish(exact[v], last);
+      }
+    }
+  }
+}
+
 // The image of W that the long contractions stream: for every slice of 32 NT
 // columns and every block of 32 k what w_store leaves in LDS, in that order.
 // WT: W is given as its transpose, [N x K].
@@ -763,6 +1123,60 @@ __global__ void __launch_bounds__(256)
   for (int l = 0; l < PL; ++l)
     *reinterpret_cast<bf16x8 *>(image + st * BUF_BYTES + l * 2 * NT * 1024 + (kg / 2) * NT * 1024 + tile * 1024 +
                                 (kg & 1) * 512 + cc * 16) = p[l];
+}
+
+// The image of W that k_nin_lines reads: a chunk of 1 KB for every tile of 32
+// columns, block of 32 k, plane and step of 16 k, in that order.  Those of several
+// layers in one launch (each by itself takes 3 us, whatever it holds).
+//   fs 0: W is [K x N]; -1: [N x K]; more: the filters of the layer whose input's
+//   gradient this is, [fs N x K / fs], its rule positions in the same order.
+struct ImageList {
+  const float *W[SCN_IMAGES_MAX];
+  unsigned char *image[SCN_IMAGES_MAX];
+  unsigned firstBlock[SCN_IMAGES_MAX + 1];
+  int K[SCN_IMAGES_MAX], N[SCN_IMAGES_MAX], fs[SCN_IMAGES_MAX], planes[SCN_IMAGES_MAX];
+  int count;
+};
+template <int PL>
+__device__ __forceinline__ void weight_image(const float *__restrict__ W, unsigned char *__restrict__ image, int K, int N,
+                                             int fs, long long item) {
+  const int T = K / 32, columns = (N + 31) / 32 * 32;
+  if (item >= (long long)T * 4 * columns)
+    return;
+  const int column = (int)(item % columns), kg = (int)(item / columns); // (eight k, column)
+  const int n = column < N ? column : N - 1, k = 8 * kg;
+  float v[8];
+  if (fs == 0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[i] = W[(long long)(k + i) * N + n];
+  } else {
+    const int width = fs < 0 ? K : K / fs, f = k / width; // (a multiple of 8)
+    const float *const src = W + ((long long)f * N + n) * width + (k - f * width);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[i] = src[i];
+  }
+  bf16x8 p[PL];
+  split8<PL>(v, p);
+#pragma unroll
+  for (int l = 0; l < PL; ++l)
+    *reinterpret_cast<bf16x8 *>(image + ((((long long)(column / 32) * T + kg / 4) * PL + l) * 2 + kg / 2 % 2) * 1024 +
+                                (kg & 1) * 512 + (column & 31) * 16) = p[l];
+}
+__global__ void __launch_bounds__(256) k_weight_images(ImageList l) {
+  const int lane = threadIdx.x & 63;
+  const int x = __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_IMAGES_MAX ? lane : 0])) - 1;
+  const long long item = (long long)(blockIdx.x - l.firstBlock[x]) * 256 + threadIdx.x;
+  if (l.planes[x] == 3)
+    weight_image<3>(l.W[x], l.image[x], l.K[x], l.N[x], l.fs[x], item);
+  else
+    weight_image<1>(l.W[x], l.image[x], l.K[x], l.N[x], l.fs[x], item);
+}
+static int64_t image_bytes(int planes, int K, int N) { return (int64_t)scn_ceil_div(N, 32) * 32 * K * 2 * planes; }
+// What k_nin_lines takes: three planes or one, blocks within one filter position.
+static bool lines_shape(int planes, int K, int nIn) {
+  return planes != 2 && scn_planes_shape(K) && nIn % 32 == 0;
 }
 
 // False: convert on the way instead -- the stream is being captured (a graph may
@@ -823,6 +1237,41 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
 #undef SCN_PLANES_GO
   return SCN_OK;
 }
+static int weight_images(scn_ctx *ctx, const ImageList &l) {
+  if (l.firstBlock[l.count] == 0)
+    return SCN_OK;
+  hipLaunchKernelGGL(k_weight_images, dim3(l.firstBlock[l.count]), dim3(256), 0, ctx->stream, l);
+  return SCN_OK;
+}
+static void add_image(ImageList &l, const float *W, unsigned char *image, int planes, int K, int N, int fs) {
+  const int i = l.count++;
+  l.W[i] = W, l.image[i] = image, l.K[i] = K, l.N[i] = N, l.fs[i] = fs, l.planes[i] = planes;
+  l.firstBlock[i + 1] = l.firstBlock[i] + (unsigned)scn_ceil_div((int64_t)K / 8 * ((N + 31) / 32 * 32), 256);
+}
+template <int PL, int MT, int NT, int RW, int CW, int D>
+static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
+                        const Epilogue &ep, const GatherSource *gs, bool wT, const RowRange &rows,
+                        const unsigned char *image) {
+  if (!image) {
+    ImageList l;
+    l.count = 0, l.firstBlock[0] = 0;
+    add_image(l, W, ctx->d_image, PL, K, N, wT ? -1 : 0);
+    SCN_TRY(weight_images(ctx, l));
+    image = ctx->d_image;
+  }
+  constexpr int ROWS = 32 * MT * RW, COLUMNS = 32 * NT * CW;
+  const size_t lds = (size_t)D * (ROWS / 8 + NT * CW * PL * 2) * 1024 + (gs ? (size_t)ROWS * gs->fs * 4 : 0);
+  SCN_REQUIRE(lds <= 160 * 1024, SCN_ERR_ARG, "planes: %d filter positions", gs ? gs->fs : 0);
+  const int nSplits = scn_ceil_div(N, COLUMNS);
+  const dim3 grid((unsigned)(scn_ceil_div(M, ROWS) * (long long)nSplits));
+  if (gs)
+    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, true>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
+                       out, M, K, N, ep, *gs, nSplits, rows, PlainW{W, wT});
+  else
+    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
+                       out, M, K, N, ep, GatherSource(), nSplits, rows, PlainW{W, wT});
+  return SCN_OK;
+}
 template <int PL>
 static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
@@ -844,8 +1293,6 @@ static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
 #undef SCN_SPLITK_GO
   return SCN_OK;
 }
-
-bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
 
 // Which tile.  With n workgroups on every compute unit a block of 32 k takes tn
 // n microseconds, and no less than t1 (its chain: request, split, barrier).
@@ -890,14 +1337,17 @@ static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
 struct PlanesChoice {
   int tile; // index into planesTiles, -1: split contraction
   bool image;
+  float cost; // microseconds, about
+  int lines = -1; // k_nin_lines, a tile of its own: index into linesTiles
+  const unsigned char *weights = nullptr; // the image it reads, null: to be made
 };
 // needImage: of the tiles, only from the image
 static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16,
                                    bool needImage = false) {
   if (M <= split_rows(ctx, planes, K, N))
-    return {-1, false};
+    return {-1, false, 0.f};
   const int T = K / 32;
-  PlanesChoice best = {0, false};
+  PlanesChoice best = {0, false, 0.f};
   float least = 1e30f;
   for (int i = 0; i < 4; ++i) {
     const int mt = planesTiles[planes > 1][i][0], nt = planesTiles[planes > 1][i][1];
@@ -911,10 +1361,45 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
       const PlanesCost &c = planesCost[planes > 1 ? 2 : a16][i][img];
       const float cost = T * fmaxf(c.t1, c.tn * n) + 3.f + units * (.2f + .17f * n) + (img ? 5.f : 0.f);
       if (cost < least)
-        least = cost, best = {i, img != 0};
+        least = cost, best = {i, img != 0, cost};
     }
   }
   return best;
+}
+// k_nin_lines' tiles.  A workgroup alone on its compute unit takes f + T t1
+// microseconds for T blocks of 32 k, with `resident` of them there (LDS) a block
+// takes all of them tn.  Fitted to 26 shapes (1037 to 1.36 M rows, 128 to 2592 k, 64
+// to 800 columns; 10 % rms), of which it takes 25 to the fastest of these tiles or
+// one within 5 %.  Taller or wider tiles, one wavefront in place of two a SIMD, and
+// deeper rings gained nothing.
+struct LinesTile {
+  int mt, nt, rw, cw, d, resident;
+  float f, t1, tn;
+};
+static const LinesTile linesTiles[2][5] = {
+    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f}}, // one plane
+    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f},
+     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f}}};
+static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool gather, int *tile) {
+  const int T = K / 32;
+  float least = 1e30f;
+  for (int i = 0; i < (planes == 3 ? 5 : 3); ++i) {
+    const LinesTile &x = linesTiles[planes == 3][i];
+    const float n = (float)scn_ceil_div(M, 32 * x.mt * x.rw) * scn_ceil_div(N, 32 * x.nt * x.cw) / ctx->numCU;
+    float cost;
+    if (n <= x.resident) {
+      const float shared = x.resident > 1 ? (fmaxf(ceilf(n), 1.f) - 1.f) / (x.resident - 1) : 0.f;
+      cost = x.f + T * (x.t1 + shared * (x.tn - x.t1));
+    } else {
+      const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
+      cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));
+    }
+    if (planes == 3 && gather && n > 4.f) // (rows that few workgroups share, and the clock)
+      cost *= 1.12f;
+    if (cost < least)
+      least = cost, *tile = i;
+  }
+  return least + 4.f;
 }
 bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
   return M <= split_rows(ctx, planes, K, N);
@@ -946,6 +1431,25 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   } else if (choice.tile < 0) {
     return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
   }
+#define SCN_LINES_CASE(I, MT, NT, RW, CW, D)                                                                             \
+  case I:                                                                                                               \
+    return launch_lines<PL, MT, NT, RW, CW, D>(ctx, A, W, out, M, K, N, ep, gs, wT, rows, choice.weights);
+  if constexpr (PL == 3) {
+    switch (choice.lines) { // (as in linesTiles)
+      SCN_LINES_CASE(0, 1, 2, 4, 2, 3)
+      SCN_LINES_CASE(1, 2, 1, 4, 2, 3)
+      SCN_LINES_CASE(2, 1, 3, 4, 1, 4)
+      SCN_LINES_CASE(3, 1, 2, 2, 2, 4)
+      SCN_LINES_CASE(4, 1, 1, 2, 2, 3)
+    }
+  } else if constexpr (PL == 1) {
+    switch (choice.lines) {
+      SCN_LINES_CASE(0, 1, 2, 4, 2, 3)
+      SCN_LINES_CASE(1, 1, 2, 2, 2, 4)
+      SCN_LINES_CASE(2, 1, 1, 2, 2, 3)
+    }
+  }
+#undef SCN_LINES_CASE
   // (channels in other than 32s, seldom met: one tile)
   if (gs && gs->nIn % 32 != 0)
     return launch_planes<PL, 1, 2, W_PLAIN, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
@@ -979,13 +1483,33 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   return SCN_ERR_ARG;
 }
 
+// k_nin_lines where it is the faster (the same bits): for rows that are not gathered
+// wherever it can run, as k_nin_planes' costs are too low for those.
+static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, const GatherSource *gs, const void *image,
+                          bool room, PlanesChoice &choice) {
+  if (!lines_shape(planes, K, gs ? gs->nIn : K) ||
+      !(image || (room && image_bytes(planes, K, N) <= (int64_t)SCN_IMAGE_BYTES)))
+    return;
+  int tile = 0;
+  const float cost = lines_choose(ctx, planes, M, K, N, gs != nullptr, &tile) + (image ? 0.f : 4.f);
+  if (gs && cost >= choice.cost + 2.f) // (2: what the other's leave out of a launch)
+    return;
+  choice.lines = tile;
+  choice.weights = (const unsigned char *)image;
+}
+
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
-                       const Epilogue &ep, const GatherSource *gs, bool a16) {
+                       const Epilogue &ep, const GatherSource *gs, bool a16,
+                       const void *image) {
   // (rows guessed: a tile in any case, they may be more)
   const long long split = split_rows(ctx, planes, K, N), hint = scn_rows_hint(ctx, M);
-  PlanesChoice choice = planes_choose(ctx, planes, M > split && hint <= split ? split + 1 : hint, K, N, a16);
-  choice.image = choice.image && planes_image(ctx);
+  const long long rows = M > split && hint <= split ? split + 1 : hint;
+  PlanesChoice choice = planes_choose(ctx, planes, rows, K, N, a16);
+  const bool room = planes_image(ctx);
+  choice.image = choice.image && room;
+  if (choice.tile >= 0 && !a16)
+    lines_instead(ctx, planes, rows, K, N, gs, image, room, choice);
   return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
          : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
                        : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16, choice);
@@ -999,8 +1523,11 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
   *transpose = false;
   if (!scn_planes_shape(K) || ((uintptr_t)A & 15) || ((uintptr_t)out & 15) || N % 4 != 0)
     return false;
-  const PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
-  if (choice.tile >= 0 && !(choice.image && planes_image(ctx))) {
+  PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
+  const bool room = planes_image(ctx);
+  if (choice.tile >= 0)
+    lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, choice);
+  if (choice.tile >= 0 && !(room && (choice.image || choice.lines >= 0))) {
     *transpose = choice.image;
     return false;
   }
