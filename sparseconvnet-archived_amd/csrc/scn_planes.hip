@@ -601,8 +601,10 @@ __global__ void __launch_bounds__(64 * WAVES, WAVES == 8 ? 4 : MT * NT >= 3 ? 2 
 // or two trips to memory long, whatever it is wide: W comes straight from
 // global memory (no two wavefronts want the same piece of it), and the eight
 // partial tiles meet in LDS.
-template <int PL, bool GATHER, bool A16, bool WT>
-__global__ void __launch_bounds__(512, 2)
+// GATHER 1: a gathered row's channels are a multiple of 32 (a block lies within one
+// filter position), 2: of 4.
+template <int PL, int GATHER, bool A16, bool WT>
+__global__ void __launch_bounds__(512, GATHER == 2 && PL > 1 ? 2 : 4)
     k_nin_planes_splitk(const float *__restrict__ A, const float *__restrict__ W,
                         float *__restrict__ out, long long M, int K, int N,
                         Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
@@ -615,7 +617,7 @@ __global__ void __launch_bounds__(512, 2)
   __shared__ __attribute__((aligned(16))) float sPart[8 * 16 * 64];
   __shared__ int sRules[GATHER ? 32 * GF_MAX_FS : 1];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, q = lane >> 5;
   const int split = tileOf % nSplits;
   const long long row0 = (long long)(tileOf / nSplits) * 32;
@@ -623,7 +625,10 @@ __global__ void __launch_bounds__(512, 2)
   const int T = K / 32;
   const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
   const int n = n0 + c < N ? n0 + c : N - 1; // (a column past the end is not stored)
-  const float *const wCol = WT ? W + (long long)n * K + 8 * q : W + (long long)(8 * q) * N + n;
+  // this lane's place in a step's eight rows of W, in bytes (the rows' own addresses
+  // are the wavefront's)
+  const unsigned wLane = WT ? 32u * q : 4u * ((unsigned)(8 * q) * N + n);
+  const float *const wRow = WT ? W + (long long)n * K : W;
   struct Block {
     floatx4 a[2][A16 ? 1 : 2];
     float w[2][8];
@@ -635,16 +640,25 @@ __global__ void __launch_bounds__(512, 2)
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        b.w[s][i] = wCol[(long long)(32 * t + 16 * s + i) * (WT ? 1 : N)];
+        b.w[s][i] = *reinterpret_cast<const float *>(
+            reinterpret_cast<const unsigned char *>(wRow + (long long)(32 * t + 16 * s + i) * (WT ? 1 : N)) + wLane);
   };
   auto load_a = [&](Block &b, int t) {
+    const unsigned char *row = nullptr;
+    if (GATHER == 1) {
+      const int f = (int)__umulhi((unsigned)(32 * t), gs.magic); // uniform
+      const int rule = sRules[c * gs.fs + f];
+      row = (rule >= 0 ? Ab + (long long)rule * gs.nIn * ES : reinterpret_cast<const unsigned char *>(gs.zeros)) +
+            (32 * t - f * gs.nIn + 8 * q) * ES;
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int h = 0; h < (A16 ? 1 : 2); ++h) {
         const int k = 32 * t + 16 * s + 8 * q + 4 * h;
-        b.a[s][h] = GATHER ? gathered_piece<A16>(Ab, gs, sRules + c * gs.fs, k)
-                           : *reinterpret_cast<const floatx4 *>(Ab + (m * K + k) * ES);
+        b.a[s][h] = GATHER == 1   ? *reinterpret_cast<const floatx4 *>(row + (16 * s + 4 * h) * ES)
+                    : GATHER == 2 ? gathered_piece<A16>(Ab, gs, sRules + c * gs.fs, k)
+                                  : *reinterpret_cast<const floatx4 *>(Ab + (m * K + k) * ES);
       }
   };
   constexpr int NACC = PL > 1 ? 2 : 1;
@@ -700,9 +714,12 @@ __global__ void __launch_bounds__(512, 2)
     load_a(b0, t2);
     compute(b1);
   }
+  // (the lane's numbers anew: the loop has no registers to keep them in)
+  const int at = __lane_id(), c1 = at & 31, q1 = at >> 5;
+  const ColEpilogue col = load_col(ep, n0 + c1 < N ? n0 + c1 : N - 1);
 #pragma unroll
   for (int v = 0; v < 16; ++v)
-    sPart[(wave * 16 + v) * 64 + lane] = NACC == 2 ? acc[0][v] + acc[NACC - 1][v] : acc[0][v];
+    sPart[(wave * 16 + v) * 64 + at] = NACC == 2 ? acc[0][v] + acc[NACC - 1][v] : acc[0][v];
   __syncthreads();
   // register v of lane (c, q) is row 8 (v / 4) + 4 q + v % 4; this wavefront's
   // are v = wave and wave + 8
@@ -711,17 +728,19 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int v = 8 * h + wave;
-    sum[h] = sPart[v * 64 + lane];
+    sum[h] = sPart[v * 64 + at];
 #pragma unroll
     for (int w = 1; w < 8; ++w)
-      sum[h] += sPart[(w * 16 + v) * 64 + lane];
+      sum[h] += sPart[(w * 16 + v) * 64 + at];
     if (doubtful<PL>(sum[h]))
       again |= 1u << v;
   }
   if constexpr (PL == 3) {
     if (__any(again != 0)) {
+      const long long m1 = row0 + c1 < M ? row0 + c1 : M - 1;
+      const int n1 = n0 + c1 < N ? n0 + c1 : N - 1;
       const floatx16 plain =
-          tile_f32<GATHER>(A, gs, sRules + (GATHER ? (int)(m - row0) * gs.fs : 0), PlainW{W, WT}, m, n, K, N, again);
+          tile_f32<GATHER != 0>(A, gs, sRules + (GATHER ? (int)(m1 - row0) * gs.fs : 0), PlainW{W, WT}, m1, n1, K, N, again);
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         if (again >> v & 1)
@@ -731,9 +750,9 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int v = 8 * h + wave;
-    const int dr = 8 * (v / 4) + 4 * q + v % 4;
-    if (row0 + dr < M && n0 + c < N)
-      out[(row0 + dr) * N + n0 + c] = finish(sum[h], load_col(ep, n0 + c));
+    const int dr = 8 * (v / 4) + 4 * q1 + v % 4;
+    if (row0 + dr < M && n0 + c1 < N)
+      out[(row0 + dr) * N + n0 + c1] = finish(sum[h], col);
   }
 }
 
@@ -1283,13 +1302,15 @@ static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
   hipLaunchKernelGGL((k_nin_planes_splitk<PL, G, H, T>), grid, dim3(512), 0,   \
                      ctx->stream, A, W, out, M, K, N, ep, src, nSplits, rows)
   if (PL == 3 && wT)
-    SCN_SPLITK_GO(false, false, PL == 3, GatherSource());
+    SCN_SPLITK_GO(0, false, PL == 3, GatherSource());
   else if (!gs)
-    SCN_SPLITK_GO(false, false, false, GatherSource());
+    SCN_SPLITK_GO(0, false, false, GatherSource());
   else if (PL == 1 && a16)
-    SCN_SPLITK_GO(true, PL == 1, false, *gs);
+    SCN_SPLITK_GO(2, PL == 1, false, *gs);
+  else if (gs->nIn % 32 == 0)
+    SCN_SPLITK_GO(1, false, false, *gs);
   else
-    SCN_SPLITK_GO(true, false, false, *gs);
+    SCN_SPLITK_GO(2, false, false, *gs);
 #undef SCN_SPLITK_GO
   return SCN_OK;
 }
@@ -1325,11 +1346,15 @@ static const PlanesCost planesCost[3][4][2] = {
     {{{.64f, .46f}, {.54f, .39f}}, {{.96f, .72f}, {.95f, .64f}}, {{1.6f, 1.16f}, {1.23f, .99f}}, {{1.36f, 1.29f}, {1.22f, 1.16f}}}};
 
 // The split contraction takes up to this many rows: one or two trips to memory
-// while its workgroups are up to so many a compute unit (measured: three planes,
-// 390 workgroups of 512 k 10.2 us against 14.2 for the tile, 1460 of 384 k 23.9
-// against 16); every 32 rows read the whole of W, out of L2 up to about 512 k.
+// while its workgroups are up to so many a compute unit.  Two fit (with 158
+// registers, until the rows of whole blocks were looked up once and W's addresses
+// left to the scalar unit, it was one: 2600 x 512 x 160 11.0 us, now 8.4).  Measured
+// against k_nin_lines with its image made, us at so many a compute unit: three
+// planes, 512 k 2.4 11.2, 12.2, and 3.1 14.5, 12.8; 768 k 2.5 15.0, 17.0, and 3.2
+// 19.4, 17.6; 256 k 1.8 6.2, 7.7, and 2.4 8.5, 8.0; 2560 k 2.2 41.7, 45.9, and 3.1
+// 51.7, 46.5; one plane, 512 k 1.6 6.9, 7.2, and 2.0 9.3, 7.4; 256 k 1.8 5.4, 5.4.
 static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
-  const float perCU = planes == 1 ? (K <= 512 ? 1.4f + K / 160.f : 3.3f) : fminf(1.f + K / 230.f, 3.1f);
+  const float perCU = planes == 1 ? 2.f : fminf(1.f + K / 230.f, planes == 2 ? 3.1f : 2.6f);
   const long long rows = (long long)(perCU * ctx->numCU / scn_ceil_div(N, 32));
   return 32 * (rows < 1 ? 1 : rows);
 }
