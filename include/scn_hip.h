@@ -448,7 +448,29 @@ int scn_sgemm_AtB_acc(scn_ctx *ctx, const float *d_A, const float *d_D,
  * +=) the column sums of D, where the activation's derivative is in D already. */
 int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *d_dW,
                        float *d_db, int64_t M, int K, int N, int accumulate);
+/* Weights laid out as the contractions of middle layers read them (planes of the
+ * matrix cores' operands), for those that a program runs many of: up to
+ * SCN_IMAGES_MAX layers' in one launch, where a call without makes its own in one.
+ * The same results, bit for bit.
+ * scn_weight_image_bytes: the room that W [K x N] takes, 0 where a contraction of M
+ * rows would not read it (nIn: channels of the rows that the rules name, K where
+ * the matrix is there; precision as scn_nin_forward_p's).
+ * scn_weight_images_many: d_image (aligned to 16 bytes) from d_W; with fs > 0 d_W are
+ * the filters of a layer, [fs N x K / fs], and the image that of the weights
+ * scn_transpose_filters_many makes of them.
+ * scn_conv_nin_forward_image: scn_conv_nin_forward_p (d_rules null: scn_nin_forward_p
+ * of a matrix of fs nIn columns) with d_W and its image, or null. */
 #define SCN_IMAGES_MAX 32
+typedef struct scn_image_item {
+  const float *d_W;
+  void *d_image;
+  int32_t K, N, fs, precision;
+} scn_image_item;
+int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N, int nIn, int precision);
+int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items, int nItems);
+int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn, const float *d_W,
+                               const void *d_image, const float *d_B, const float *d_prelu, float *d_out, int64_t M, int N,
+                               float p, int act, int precision);
 /* The backward pass of a convolution without its gathered matrix (no
  * counterpart in the reference, which keeps that matrix and its gradient).
  * scn_rules_inverse_many turns the rules of up to SCN_INVERSE_MAX layers round:
@@ -471,7 +493,7 @@ int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *
  * scn_transpose_filters_many gives the weights, Wt [fs N x nIn] of W [fs nIn x
  * N], and scn_conv_input_gradient writes every input row's gradient, d_din
  * [inputRows x nIn], from d_delta (where scn_conv_nin_supported_p(fs, N, nIn,
- * SCN_FP32)). */
+ * SCN_FP32); d_image: of Wt, SCN_FP32_PLANES, or null). */
 #define SCN_INVERSE_MAX 16
 typedef struct scn_inverse_item {
   const scn_grids *input; /* the convolution's input grids, counts settled */
@@ -492,7 +514,7 @@ typedef struct scn_filter_item {
 } scn_filter_item;
 int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *items, int nItems);
 int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
-                            const float *d_Wt, float *d_din, int64_t inputRows, int nIn);
+                            const float *d_Wt, const void *d_image, float *d_din, int64_t inputRows, int nIn);
 int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,
                  const float *d_D, float *d_dW, float *d_db, int64_t M, int N, int accumulate);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout

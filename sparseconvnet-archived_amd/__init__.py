@@ -42,6 +42,11 @@ class FilterItem(C.Structure):
     _fields_ = [("d_W", C.c_void_p), ("d_Wt", C.c_void_p), ("fs", C.c_int32), ("nIn", C.c_int32), ("N", C.c_int32)]
 
 
+class ImageItem(C.Structure):
+    _fields_ = [("d_W", C.c_void_p), ("d_image", C.c_void_p), ("K", C.c_int32), ("N", C.c_int32), ("fs", C.c_int32),
+                ("precision", C.c_int32)]
+
+
 class NagItem(C.Structure):
     """scn_nag_item of the C header."""
     _fields_ = [("d_delta", C.c_void_p), ("d_momentum", C.c_void_p), ("d_weights", C.c_void_p),
@@ -154,7 +159,10 @@ def lib():
         "scn_sgemm_AtB_sums": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, C.c_int, C.c_int]),
         "scn_maxpool_backward_through": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, C.c_int]),
         "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
-        "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, i64, C.c_int]),
+        "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, i64, C.c_int]),
+        "scn_weight_image_bytes": (i64, [vp, i64, C.c_int, C.c_int, C.c_int, C.c_int]),
+        "scn_weight_images_many": (C.c_int, [vp, P(ImageItem), C.c_int]),
+        "scn_conv_nin_forward_image": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, C.c_int, f32, C.c_int, C.c_int]),
         "scn_background_sums": (C.c_int, [vp, vp, i64, C.c_int, vp, C.c_int, C.c_int]),
         "scn_positions_pitch": (i64, [i64]),
         "scn_transpose_filters_many": (C.c_int, [vp, P(FilterItem), C.c_int]),
@@ -380,8 +388,20 @@ class Context:
             arr[k] = InverseItem(g.h, rules.ptr, *out, rows, inputRows, fs)
         _check(lib().scn_rules_inverse_many(self.h, arr, len(items)))
 
-    def conv_input_gradient(self, d_delta, d_inverse, fs, N, d_Wt, d_din, inputRows, nIn):
-        _check(lib().scn_conv_input_gradient(self.h, d_delta.ptr, d_inverse.ptr, fs, N, d_Wt.ptr, d_din.ptr, inputRows, nIn))
+    def conv_input_gradient(self, d_delta, d_inverse, fs, N, d_Wt, d_din, inputRows, nIn, d_image=None):
+        _check(lib().scn_conv_input_gradient(self.h, d_delta.ptr, d_inverse.ptr, fs, N, d_Wt.ptr, d_image.ptr if d_image is not None else None, d_din.ptr,
+                                             inputRows, nIn))
+
+    def weight_images_many(self, items):
+        """items: (d_W, d_image, K, N, fs, precision) tuples"""
+        arr = (ImageItem * max(1, len(items)))()
+        for k, (w, image, K, n, fs, precision) in enumerate(items):
+            arr[k] = ImageItem(w.ptr, image.ptr, K, n, fs, precision)
+        _check(lib().scn_weight_images_many(self.h, arr, len(items)))
+
+    def conv_nin_forward_image(self, d_in, d_rules, fs, nIn, d_W, d_image, d_B, d_prelu, d_out, M, N, p, act, precision):
+        _check(lib().scn_conv_nin_forward_image(self.h, d_in.ptr, d_rules.ptr if d_rules is not None else None, fs, nIn, d_W.ptr, d_image.ptr if d_image is not None else None, d_B.ptr,
+                                                d_prelu.ptr if d_prelu is not None else None, d_out.ptr, M, N, p, act, precision))
 
     def background_sums(self, d_delta, M, N, d_background, fs, batch):
         _check(lib().scn_background_sums(self.h, d_delta.ptr, M, N, d_background.ptr, fs, batch))

@@ -1786,11 +1786,13 @@ static void launch_mfma(scn_ctx *ctx, const float *A, const float *W,
 // 1920 x 640 186, 140).  SCN_FP32_PLANES, which the host classes ask for, takes
 // the planes at every size.
 #define PLANES_MIN_FLOPS 4e10
-// rows16: a bf16 copy of the matrix the rules point into, or null
+// rows16: a bf16 copy of the matrix the rules point into, or null; image: the
+// weights for the planes (scn_weight_images_many), or null
 static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
                        const float *d_B, const float *d_prelu, float *d_out,
                        int64_t M, int K, int N, float p, int act, int precision,
-                       const GatherSource *gs, const void *rows16 = nullptr) {
+                       const GatherSource *gs, const void *rows16 = nullptr,
+                       const void *image = nullptr) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_nin_forward: null context");
   SCN_REQUIRE(M >= 0 && K >= 1 && N >= 1, SCN_ERR_ARG,
               "scn_nin_forward: M %lld K %d N %d", (long long)M, K, N);
@@ -1846,7 +1848,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   if (planes && rounded && act != SCN_SOFTMAX) {
     const bool a16 = precision == SCN_BF16 && rows16 && gs && gs->nIn % 8 == 0 && ((uintptr_t)rows16 & 15) == 0;
     SCN_TRY(scn_planes_forward(ctx, precision == SCN_BF16 ? 1 : 2, a16 ? (const float *)rows16 : d_A, d_W, d_out, M,
-                               K, N, ep, gs, a16));
+                               K, N, ep, gs, a16, image));
   } else if (tiledBf16) {
     SCN_REQUIRE(!gs, SCN_ERR_ARG,
                 "fused convolution: shape outside the bf16 kernel's range");
@@ -1888,7 +1890,8 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
                        dim3(256), 0, ctx->stream, d_A, d_W, d_out, (long long)M,
                        K, N, ep, dRows);
   } else if (planes) {
-    SCN_TRY(scn_planes_forward(ctx, 3, d_A, d_W, d_out, M, K, N, ep, gs, false));
+    SCN_TRY(scn_planes_forward(ctx, 3, d_A, d_W, d_out, M, K, N, ep, gs, false,
+                               precision == SCN_FP32_PLANES ? image : nullptr));
   } else if (vec && wres_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
     // W-resident kernel took it
   } else if (vec && ctx->wstream && wstream_forward(ctx, d_A, d_W, d_out, M, K, N, ep, gs)) {
@@ -2021,12 +2024,9 @@ extern "C" int scn_conv_nin_forward(scn_ctx *ctx, const float *d_in,
   return scn_conv_nin_forward_p(ctx, d_in, d_rules, fs, nIn, d_W, d_B, d_prelu,
                                 d_out, M, N, p, act, SCN_FP32);
 }
-extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
-                                      const int32_t *d_rules, int fs, int nIn,
-                                      const float *d_W, const float *d_B,
-                                      const float *d_prelu, float *d_out,
-                                      int64_t M, int N, float p, int act,
-                                      int precision) {
+static int conv_nin_forward(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn,
+                            const float *d_W, const void *d_image, const float *d_B, const float *d_prelu,
+                            float *d_out, int64_t M, int N, float p, int act, int precision) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_nin_forward: null context");
   SCN_REQUIRE(scn_conv_nin_supported_p(fs, nIn, N, precision), SCN_ERR_ARG,
               "scn_conv_nin_forward: fs %d nIn %d N %d precision %d is outside "
@@ -2044,7 +2044,27 @@ extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
   gs.magic = (unsigned)((1ull << 32) / (unsigned)nIn + 1);
   gs.zeros = ctx->d_zeros;
   return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p,
-                     act, precision, &gs);
+                     act, precision, &gs, nullptr, d_image);
+}
+extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
+                                      const int32_t *d_rules, int fs, int nIn,
+                                      const float *d_W, const float *d_B,
+                                      const float *d_prelu, float *d_out,
+                                      int64_t M, int N, float p, int act,
+                                      int precision) {
+  return conv_nin_forward(ctx, d_in, d_rules, fs, nIn, d_W, nullptr, d_B, d_prelu, d_out, M, N, p, act, precision);
+}
+extern "C" int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in,
+                                          const int32_t *d_rules, int fs, int nIn,
+                                          const float *d_W, const void *d_image, const float *d_B,
+                                          const float *d_prelu, float *d_out,
+                                          int64_t M, int N, float p, int act,
+                                          int precision) {
+  SCN_REQUIRE(((uintptr_t)d_image & 15) == 0, SCN_ERR_ARG, "scn_conv_nin_forward: the image starts on 16 bytes");
+  if (d_rules)
+    return conv_nin_forward(ctx, d_in, d_rules, fs, nIn, d_W, d_image, d_B, d_prelu, d_out, M, N, p, act, precision);
+  SCN_REQUIRE(fs >= 1 && nIn >= 1, SCN_ERR_ARG, "scn_conv_nin_forward: fs %d nIn %d", fs, nIn);
+  return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p, act, precision, nullptr, nullptr, d_image);
 }
 
 // Where scn_nin_forward takes the classifier to k_classifier

@@ -1540,6 +1540,48 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16, choice);
 }
 
+// The planes of a call of that precision, 0: none that take an image
+static int image_planes(int precision) {
+  return precision == SCN_FP32_PLANES ? 3 : precision == SCN_BF16 ? 1 : 0;
+}
+extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N, int nIn, int precision) {
+  const int planes = image_planes(precision);
+  if (!ctx || M < 1 || K < 1 || N < 1 || nIn < 1 || planes == 0 || N % 4 != 0 || !lines_shape(planes, K, nIn))
+    return 0;
+  const long long hint = scn_rows_hint(ctx, M), split = split_rows(ctx, planes, K, N);
+  if (6 * hint <= 5 * split)
+    return 0;
+  int tile;
+  const PlanesChoice choice = planes_choose(ctx, planes, hint > split ? hint : split + 1, K, N, false);
+  if (nIn != K && lines_choose(ctx, planes, hint, K, N, true, &tile) >= choice.cost + 2.f)
+    return 0;
+  return image_bytes(planes, K, N);
+}
+extern "C" int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items, int nItems) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_weight_images_many: null context");
+  SCN_REQUIRE(nItems >= 0 && nItems <= SCN_IMAGES_MAX && (items || nItems == 0), SCN_ERR_ARG,
+              "scn_weight_images_many: %d items (at most %d)", nItems, SCN_IMAGES_MAX);
+  static_assert(SCN_IMAGES_MAX <= 64, "a lane an item");
+  ImageList l;
+  l.count = 0, l.firstBlock[0] = 0;
+  long long blocks = 0;
+  for (int k = 0; k < nItems; ++k) {
+    const scn_image_item &it = items[k];
+    const int planes = image_planes(it.precision);
+    SCN_REQUIRE(it.d_W && it.d_image && planes && scn_planes_shape(it.K) && it.N >= 1 && it.fs >= 0 &&
+                    (it.fs == 0 || (it.K % it.fs == 0 && it.K / it.fs % 8 == 0)) && ((uintptr_t)it.d_image & 15) == 0,
+                SCN_ERR_ARG, "scn_weight_images_many: item %d K %d N %d fs %d precision %d", k, it.K, it.N, it.fs,
+                it.precision);
+    blocks += scn_ceil_div((int64_t)it.K / 8 * (((int64_t)it.N + 31) / 32 * 32), 256);
+    SCN_REQUIRE(blocks <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_weight_images_many: %lld workgroups", blocks);
+    add_image(l, it.d_W, (unsigned char *)it.d_image, planes, it.K, it.N, it.fs);
+  }
+  ProfScope prof(ctx, SCN_K_NIN);
+  SCN_TRY(weight_images(ctx, l));
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 // out = A Wt^T for Wt [N x K].  False: nothing has been launched; not a shape for
 // it, or (transpose) one that scn_planes_forward takes to the same bits from the
 // transpose, because the image may not be used now.

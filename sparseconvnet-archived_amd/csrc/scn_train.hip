@@ -593,15 +593,17 @@ extern "C" int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *i
 }
 
 extern "C" int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
-                                       const float *d_Wt, float *d_din, int64_t inputRows, int nIn) {
+                                       const float *d_Wt, const void *d_image, float *d_din, int64_t inputRows,
+                                       int nIn) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_input_gradient: null context");
   SCN_REQUIRE(inputRows >= 0 && nIn >= 1 && nIn <= SCN_ZERO_FLOATS && N <= SCN_ZERO_FLOATS, SCN_ERR_ARG,
               "scn_conv_input_gradient: %lld rows nIn %d N %d", (long long)inputRows, nIn, N);
   if (inputRows == 0)
     return SCN_OK;
   OwnRows ownRows(ctx);
-  return scn_conv_nin_forward_p(ctx, d_delta, d_inverse, fs, N, d_Wt, ctx->d_zeros, nullptr, d_din, inputRows, nIn,
-                                1.f, SCN_NOSIGMOID, SCN_FP32_PLANES);
+  SCN_REQUIRE(d_inverse, SCN_ERR_ARG, "scn_conv_input_gradient: null rules");
+  return scn_conv_nin_forward_image(ctx, d_delta, d_inverse, fs, N, d_Wt, d_image, ctx->d_zeros, nullptr, d_din,
+                                    inputRows, nIn, 1.f, SCN_NOSIGMOID, SCN_FP32_PLANES);
 }
 
 // ------------------------------------------------------------ dA = D W^T

@@ -105,6 +105,7 @@ public:
                     int nBatchProducerThreads = 10);
   ~SparseConvNetCUDA();
   void forwardBatch(SpatiallySparseBatch &batch, int lane = 0);
+  void makeWeightImages(SpatiallySparseBatch &batch, cudaMemStream &ms);
   void backwardBatch(SpatiallySparseBatch &batch, float learningRate,
                      float momentum);
   // training batches are drawn in shuffled order (BatchProducer.cu:23-26);

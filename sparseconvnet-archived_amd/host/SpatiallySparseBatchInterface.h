@@ -16,6 +16,10 @@ public:
   // following fused convolution with bf16 operands whose window is large
   // enough for the rows to be read many times over
   vectorCUDA<float> features16;
+  // the weights of the layer whose output this is, laid out for its forward pass
+  // and, turned round, for the gradient of its input: made for one batch by
+  // SparseConvNetCUDA::makeWeightImages and used up by the layer (empty: none)
+  vectorCUDA<float> weightImage, turnedImage;
   SpatiallySparseBatchSubInterface();
   void reset();
 };

@@ -51,6 +51,21 @@ public:
                                SpatiallySparseBatchInterface &pooled) {
     (void)batch, (void)input, (void)output, (void)pooled;
   }
+  // The layouts of the weights that this pass over the batch is to read
+  // (output.sub->weightImage, turnedImage), for scn_weight_images_many; `before`:
+  // the input of the convolution in front whose gather is deferred, or null.
+  virtual void weightImages(SpatiallySparseBatch &batch,
+                            SpatiallySparseBatchInterface &input,
+                            SpatiallySparseBatchInterface &output,
+                            const SpatiallySparseBatchInterface *before,
+                            std::vector<scn_image_item> &items) {
+    (void)batch, (void)input, (void)output, (void)before, (void)items;
+  }
+  // convolutions: the layer behind will gather (deferGather, or a batch without the matrix)
+  virtual bool defersGather(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &output) const {
+    (void)batch, (void)output;
+    return false;
+  }
   // the weights that the gradient of a left out convolution's input is made with
   // (input.leftOut), for scn_transpose_filters_many
   virtual void transposedFilters(SpatiallySparseBatchInterface &input,
@@ -87,6 +102,7 @@ public:
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
   bool addsInputGradient() const { return true; }
+  bool defersGather(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &output) const;
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -119,6 +135,7 @@ public:
                 SpatiallySparseBatchInterface &input,
                 SpatiallySparseBatchInterface &output);
   bool addsInputGradient() const { return true; }
+  bool defersGather(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &output) const;
   void backwards(SpatiallySparseBatch &batch,
                  SpatiallySparseBatchInterface &input,
                  SpatiallySparseBatchInterface &output, float learningRate,
@@ -168,6 +185,11 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  void weightImages(SpatiallySparseBatch &batch,
+                    SpatiallySparseBatchInterface &input,
+                    SpatiallySparseBatchInterface &output,
+                    const SpatiallySparseBatchInterface *before,
+                    std::vector<scn_image_item> &items);
   void transposedFilters(SpatiallySparseBatchInterface &input,
                          std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);
@@ -215,6 +237,11 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  void weightImages(SpatiallySparseBatch &batch,
+                    SpatiallySparseBatchInterface &input,
+                    SpatiallySparseBatchInterface &output,
+                    const SpatiallySparseBatchInterface *before,
+                    std::vector<scn_image_item> &items);
   void transposedFilters(SpatiallySparseBatchInterface &input,
                          std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);

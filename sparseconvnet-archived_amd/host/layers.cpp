@@ -162,12 +162,19 @@ void ConvolutionalLayer::preprocess(SpatiallySparseBatch &batch,
                              output.featuresPresent.hVector(), input.nFeatures,
                              (int)input.featuresPresent.size(), fs);
 }
+// (the backward pass needs the gathered matrix: no deferral while training,
+// unless that pass does without it)
+bool ConvolutionalLayer::defersGather(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &output) const {
+  return batch.type == TRAINBATCH ? output.leftOut : deferGather;
+}
+bool ConvolutionalTriangularLayer::defersGather(SpatiallySparseBatch &batch,
+                                                SpatiallySparseBatchInterface &output) const {
+  return batch.type == TRAINBATCH ? output.leftOut : deferGather;
+}
 void ConvolutionalLayer::forwards(SpatiallySparseBatch &batch,
                                   SpatiallySparseBatchInterface &input,
                                   SpatiallySparseBatchInterface &output) {
-  // (the backward pass needs the gathered matrix: no deferral while training,
-  // unless that pass does without it)
-  if (batch.type == TRAINBATCH ? output.leftOut : deferGather) {
+  if (defersGather(batch, output)) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -230,7 +237,7 @@ void ConvolutionalTriangularLayer::preprocess(
 void ConvolutionalTriangularLayer::forwards(
     SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
     SpatiallySparseBatchInterface &output) {
-  if (batch.type == TRAINBATCH ? output.leftOut : deferGather) {
+  if (defersGather(batch, output)) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -317,6 +324,37 @@ static void nin_forwards_shrunk(cudaMemStream &ms,
                               Kp, Np, 1.0f, act, abi_precision(precision)));
   addMultiplyAdds((__int128_t)output.nSpatialSites * Kp * Np);
 }
+// bf16 operands, a window of eight or more sites and a matrix worth the pass:
+// round the input once and let the contraction read the bf16 rows (the same
+// result bit for bit, half the bytes through the caches)
+static bool rounds_rows(int precision, int fs, int nIn, int rows) {
+  return precision == SCN_BF16 && fs >= 8 && nIn % 8 == 0 && (int64_t)rows * fs >= (int64_t)1 << 20;
+}
+// The layout of the weights that was made for this pass, or null: used once
+static const void *take_image(vectorCUDA<float> &image) {
+  const void *const p = image.size64() ? image.dPtr() : nullptr;
+  image.resize64(0);
+  return p;
+}
+static void nin_weight_images(SpatiallySparseBatch &batch, cudaMemStream &ms, SpatiallySparseBatchInterface &input,
+                              SpatiallySparseBatchInterface &output, const SpatiallySparseBatchInterface *before,
+                              vectorCUDA<float> &W, int K, int N, int precision, std::vector<scn_image_item> &items) {
+  const int nIn = before ? before->nFeatures : K, fs = K / nIn, p = abi_precision(precision);
+  const int64_t bytes = before && rounds_rows(precision, fs, nIn, output.nSpatialSites)
+                            ? 0
+                            : scn_weight_image_bytes(ms.ctx, output.nSpatialSites, K, N, nIn, p);
+  if (bytes) {
+    output.sub->weightImage.resize64((size_t)bytes / 4);
+    items.push_back({W.dPtr(), output.sub->weightImage.dPtr(), K, N, 0, p});
+  }
+  if (batch.type != TRAINBATCH || !input.leftOut || !before || !before->backpropErrors)
+    return;
+  const int64_t turned = scn_weight_image_bytes(ms.ctx, before->nSpatialSites, fs * N, nIn, N, SCN_FP32_PLANES);
+  if (turned) {
+    output.sub->turnedImage.resize64((size_t)turned / 4);
+    items.push_back({W.dPtr(), output.sub->turnedImage.dPtr(), fs * N, nIn, fs, SCN_FP32_PLANES});
+  }
+}
 // When the preceding convolutional layer deferred its gather: run the fused
 // kernel (fp32 operands), or gather now if this layer wants bf16 operands.
 // Returns false when the input is an ordinary feature matrix.
@@ -324,7 +362,7 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
                       SpatiallySparseBatchInterface &output,
                       vectorCUDA<float> &W, vectorCUDA<float> &B,
                       vectorCUDA<float> *prelu, int nFeaturesOut, float p,
-                      int act, int precision) {
+                      int act, int precision, const void *image) {
   SpatiallySparseBatchInterface *src = input.deferredGatherFrom;
   if (!src)
     return false;
@@ -334,11 +372,7 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
     gather_now(ms, *src, input);
     return false;
   }
-  // bf16 operands, a window of eight or more sites and a matrix worth the
-  // pass: round the input once and let the contraction read the bf16 rows
-  // (the same result bit for bit, half the bytes through the caches)
-  if (precision == SCN_BF16 && fs >= 8 && nIn % 8 == 0 &&
-      (int64_t)output.nSpatialSites * fs >= (int64_t)1 << 20) {
+  if (rounds_rows(precision, fs, nIn, output.nSpatialSites)) {
     const size_t elems = (size_t)src->nSpatialSites * nIn;
     src->sub->features16.resize64(elems / 2 + 8, kBoundRows * nIn / 2);
     SCN_CHECKED(scn_conv_nin_forward_a16(
@@ -348,9 +382,9 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
         output.nSpatialSites, nFeaturesOut, p, act));
     return true;
   }
-  SCN_CHECKED(scn_conv_nin_forward_p(
+  SCN_CHECKED(scn_conv_nin_forward_image(
       ms.ctx, src->sub->features.dPtr(), input.rules.dPtr(), fs, nIn, W.dPtr(),
-      B.dPtr(), prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(),
+      image, B.dPtr(), prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(),
       output.nSpatialSites, nFeaturesOut, p, act, abi_precision(precision)));
   return true;
 }
@@ -420,7 +454,7 @@ static void conv_nin_gradients(cudaMemStream &ms, SpatiallySparseBatchInterface 
                                   middle.background.dPtr(), fs, batchSize));
   src.sub->dfeatures.resize64(((size_t)src.nSpatialSites + src.gradientSums) * nIn);
   SCN_CHECKED(scn_conv_input_gradient(ms.ctx, output.sub->dfeatures.dPtr(), middle.inverse.dPtr(), fs, N,
-                                      transposed.dPtr(), src.sub->dfeatures.dPtr(), src.nSpatialSites, nIn));
+                                      transposed.dPtr(), take_image(output.sub->turnedImage), src.sub->dfeatures.dPtr(), src.nSpatialSites, nIn));
   addMultiplyAdds((__int128_t)M * fs * nIn * N); // (what the reference's count holds for it)
 }
 static void nin_transposed_filters(SpatiallySparseBatchInterface &input, int nFeaturesOut, vectorCUDA<float> &W,
@@ -555,13 +589,13 @@ void NetworkInNetworkLayer::forwards(SpatiallySparseBatch &batch,
   // test-time scaling by the kept fraction (NetworkInNetworkLayer.cu:188)
   float p = 1.0f - (batch.type != RESCALEBATCH ? dropout : 0.0f);
   cudaMemStream &ms = fwd_stream(batch, memStream);
+  const void *const image = take_image(output.sub->weightImage);
   if (!nin_fused(ms, input, output, W, B, nullptr, nFeaturesOut, p,
-                 (int)fn, precision))
-    SCN_CHECKED(scn_nin_forward(ms.ctx, input.sub->features.dPtr(),
-                                W.dPtr(), B.dPtr(), nullptr,
-                                output.sub->features.dPtr(),
-                                output.nSpatialSites, nFeaturesIn, nFeaturesOut,
-                                p, (int)fn, abi_precision(precision)));
+                 (int)fn, precision, image))
+    SCN_CHECKED(scn_conv_nin_forward_image(
+        ms.ctx, input.sub->features.dPtr(), nullptr, 1, nFeaturesIn, W.dPtr(),
+        image, B.dPtr(), nullptr, output.sub->features.dPtr(),
+        output.nSpatialSites, nFeaturesOut, p, (int)fn, abi_precision(precision)));
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)output.nSpatialSites * nFeaturesIn * nFeaturesOut);
 }
@@ -583,6 +617,22 @@ void NetworkInNetworkLayer::activationAhead(
   if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
     nin_activation_ahead(memStream, input, output, pooled, (int)fn, nullptr, dw,
                          db, nullptr, gradsClean);
+}
+void NetworkInNetworkLayer::weightImages(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                                         SpatiallySparseBatchInterface &output,
+                                         const SpatiallySparseBatchInterface *before,
+                                         std::vector<scn_image_item> &items) {
+  if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    nin_weight_images(batch, fwd_stream(batch, memStream), input, output, before, W, nFeaturesIn, nFeaturesOut, precision,
+                      items);
+}
+void NetworkInNetworkPReLULayer::weightImages(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                                              SpatiallySparseBatchInterface &output,
+                                              const SpatiallySparseBatchInterface *before,
+                                              std::vector<scn_image_item> &items) {
+  if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    nin_weight_images(batch, fwd_stream(batch, memStream), input, output, before, W, nFeaturesIn, nFeaturesOut, precision,
+                      items);
 }
 void NetworkInNetworkLayer::transposedFilters(SpatiallySparseBatchInterface &input,
                                               std::vector<scn_filter_item> &items) {
@@ -703,13 +753,13 @@ void NetworkInNetworkPReLULayer::forwards(
   }
   float p = 1.0f - (batch.type != RESCALEBATCH ? dropout : 0.0f);
   cudaMemStream &ms = fwd_stream(batch, memStream);
+  const void *const image = take_image(output.sub->weightImage);
   if (!nin_fused(ms, input, output, W, B, &PReLU, nFeaturesOut, p,
-                 (int)PRELU, precision))
-    SCN_CHECKED(scn_nin_forward(ms.ctx, input.sub->features.dPtr(),
-                                W.dPtr(), B.dPtr(), PReLU.dPtr(),
-                                output.sub->features.dPtr(),
-                                output.nSpatialSites, nFeaturesIn, nFeaturesOut,
-                                p, (int)PRELU, abi_precision(precision)));
+                 (int)PRELU, precision, image))
+    SCN_CHECKED(scn_conv_nin_forward_image(
+        ms.ctx, input.sub->features.dPtr(), nullptr, 1, nFeaturesIn, W.dPtr(),
+        image, B.dPtr(), PReLU.dPtr(), output.sub->features.dPtr(),
+        output.nSpatialSites, nFeaturesOut, p, (int)PRELU, abi_precision(precision)));
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)output.nSpatialSites * nFeaturesIn * nFeaturesOut);
 }

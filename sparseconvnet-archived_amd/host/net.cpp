@@ -487,6 +487,8 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
                          learningRate, momentum);
   }
   batch.collectUpdates = false;
+  for (size_t i = 1; i < batch.interfaces.size(); i++)
+    batch.interfaces[i].sub->turnedImage.resize64(0);
   for (size_t i = 0; i < batch.updates.size(); i += SCN_NAG_MAX)
     SCN_CHECKED(scn_nag_update_many(
         memStream.ctx, batch.updates.data() + i,
@@ -499,6 +501,27 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
     SCN_CHECKED(scn_event_create(memStream.ctx, &r.consumed));
   SCN_CHECKED(scn_event_record(memStream.ctx, r.consumed));
   r.consumedPending = true;
+}
+// The weights as the contractions of this pass read them, all layers' in one
+// launch (by themselves 3 to 5 us a layer).  Made for every batch: nothing is
+// kept that a change of the weights could leave behind.
+void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStream &ms) {
+  std::vector<scn_image_item> items;
+  for (size_t i = 0; i < layers.size(); i++) {
+    SpatiallySparseBatchInterface &input = batch.interfaces[i], &output = batch.interfaces[i + 1];
+    output.sub->weightImage.resize64(0);
+    output.sub->turnedImage.resize64(0);
+    if (batch.type == RESCALEBATCH) // (whose weights change on the way)
+      continue;
+    if (batch.countsPending)
+      SCN_CHECKED(scn_ctx_rows_from(ms.ctx, output.deviceGrids));
+    const bool gathers = i > 0 && layers[i - 1]->defersGather(batch, input);
+    layers[i]->weightImages(batch, input, output, gathers ? &batch.interfaces[i - 1] : nullptr, items);
+  }
+  if (batch.countsPending)
+    SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
+  for (size_t i = 0; i < items.size(); i += SCN_IMAGES_MAX)
+    SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, (int)std::min<size_t>(SCN_IMAGES_MAX, items.size() - i)));
 }
 // The two halves of processBatch.  forwardBatch only queues work on the net's
 // stream (every layer, then the copy of the probabilities to the host);
@@ -514,6 +537,7 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   for (size_t i = 0; i < layers.size(); i++)
     batch.interfaces[i + 1].sub =
         lane == 0 ? sharedSubInterfaces[i] : laneSubInterfaces[lane - 1][i];
+  makeWeightImages(batch, ms);
   // a RESCALEBATCH rescales every layer's weights right after its forward
   // pass (SparseConvNetCUDA.cu:230-241)
   float scalingUnderneath = 1;
@@ -540,6 +564,8 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   }
   if (batch.countsPending)
     SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
+  for (size_t i = 1; i < batch.interfaces.size(); i++) // (what no layer has taken)
+    batch.interfaces[i].sub->weightImage.resize64(0);
   SoftmaxClassifierLaunch(batch.interfaces.back(), batch, ms);
 }
 void SparseConvNetCUDA::finishBatch(SpatiallySparseBatch &batch,

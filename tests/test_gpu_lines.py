@@ -52,6 +52,57 @@ def test_lines_give_the_same_bits(scn, ctx, rows, fs, nIn, N, precision, gathere
     assert np.isfinite(got).all() and np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("rows,fs,nIn,N", [(20011, 8, 64, 96), (70145, 9, 64, 128), (33025, 8, 32, 64), (9001, 8, 160, 256)])
+def test_bf16_rows(scn, ctx, rows, fs, nIn, N):
+    rng = np.random.default_rng(rows)
+    K = fs * nIn
+    d_in, d_in16 = ctx.array(rng.standard_normal((900, nIn), dtype=np.float32)), ctx.empty((900, nIn), np.float32)
+    d_rules = ctx.array(rng.integers(-1, 900, (rows, fs)).astype(np.int32))
+    d_W, d_B = ctx.array((0.1 * rng.standard_normal((K, N))).astype(np.float32)), ctx.array(np.zeros(N, np.float32))
+    one, two = (ctx.array(np.full((rows + 256, N), 7, np.float32)) for _ in range(2))
+    print("lines of bf16 rows", rows, fs, nIn, N, flush=True)
+    ctx.conv_nin_forward_a16(d_in, 900, d_in16, d_rules, fs, nIn, d_W, d_B, None, one, rows, N, 1.0, scn.RELU)
+    with Graph(ctx) as g:
+        ctx.conv_nin_forward_a16(d_in, 900, d_in16, d_rules, fs, nIn, d_W, d_B, None, two, rows, N, 1.0, scn.RELU)
+    g.replay(ctx)
+    got, want = one.download(), two.download()
+    g.close()
+    assert np.all(got[rows:] == 7) and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("rows,fs,nIn,N", [(28415, 4, 64, 96), (9001, 8, 32, 36), (33001, 2, 64, 160), (20001, 27, 32, 64)])
+@pytest.mark.parametrize("precision", ["FP32_PLANES", "BF16"])
+def test_weights_laid_out_ahead(scn, ctx, rows, fs, nIn, N, precision):
+    """several layers' in one launch, as they stand and as the filters of the layer they are turned from"""
+    rng = np.random.default_rng(rows)
+    K, p = fs * nIn, getattr(scn, precision)
+    N = (N + 31) // 32 * 32 if precision == "BF16" else N
+    d_in = ctx.array(rng.standard_normal((500, nIn), dtype=np.float32))
+    d_rules = ctx.array(rng.integers(-1, 500, (rows, fs)).astype(np.int32))
+    W = (rng.standard_normal((fs, nIn, N)) * 0.1).astype(np.float32)
+    d_W, d_turned = ctx.array(W.reshape(K, N)), ctx.array(np.ascontiguousarray(W.transpose(0, 2, 1)).reshape(fs * N, nIn))
+    d_B = ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+    size = (N + 31) // 32 * 32 * K * (6 if precision == "FP32_PLANES" else 2)
+    # (the wider of these shapes are faster with their weights converted on the way)
+    assert scn.lib().scn_weight_image_bytes(ctx.h, rows, K, N, nIn, p) in (0, size)
+    assert scn.lib().scn_weight_image_bytes(ctx.h, 28415, 256, 96, 64, p) == 96 * 256 * (6 if precision == "FP32_PLANES" else 2)
+    assert scn.lib().scn_weight_image_bytes(ctx.h, 32, K, N, nIn, p) == 0  # (the split contraction: W as it stands)
+    images = [ctx.empty((size // 4,), np.float32) for _ in range(3)]
+    print("images", precision, rows, fs, nIn, N, flush=True)
+    ctx.weight_images_many([(d_W, images[0], K, N, 0, p), (d_turned, images[1], K, N, fs, p), (d_W, images[2], K, N, 0, p)])
+    outs = [ctx.array(np.full((rows, N), 7, np.float32)) for _ in range(4)]
+    ctx.conv_nin_forward(d_in, d_rules, fs, nIn, d_W, d_B, None, outs[3], rows, N, 1.0, scn.RELU, p)
+    for image, out in zip(images, outs):
+        ctx.conv_nin_forward_image(d_in, d_rules, fs, nIn, d_W, image, d_B, None, out, rows, N, 1.0, scn.RELU, p)
+    want = outs[3].download()
+    for out in outs[:3]:
+        assert np.array_equal(out.download(), want)
+    matrix, plain = ctx.empty((rows, K), np.float32), ctx.array(np.full((rows, N), 7, np.float32))
+    ctx.gather_rows(d_in, matrix, d_rules, rows * fs, nIn)
+    ctx.conv_nin_forward_image(matrix, None, 1, K, d_W, images[0], d_B, None, plain, rows, N, 1.0, scn.RELU, p)
+    assert np.array_equal(plain.download(), want)
+
+
 @pytest.mark.parametrize("M,N,K", [(4001, 64, 96), (33333, 128, 384), (9000, 96, 512)])
 def test_products_with_the_transpose(scn, ctx, M, N, K):
     rng = np.random.default_rng(M)
