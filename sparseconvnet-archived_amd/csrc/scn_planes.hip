@@ -788,13 +788,14 @@ template <int N> __device__ __forceinline__ void lines_landed() {
 // tiles of three planes stay ahead on gathered rows: 1.36 M x 1728 x 64 1483 against
 // 1797.
 
-template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER>
+template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16>
 __global__ void __launch_bounds__(64 * RW * CW, 2)
     k_nin_lines(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
-                int K, int N, Epilogue ep, GatherSource gs, int nSplits, RowRange rows, PlainW plain) {
+                int K, int N, Epilogue ep, GatherSource gs, int nSplits, bool byColumns, RowRange rows, PlainW plain) {
   constexpr int WAVES = RW * CW, THREADS = 64 * WAVES;
   constexpr int ROWS = 32 * MT * RW, TW = NT * CW, NW = 32 * TW;
-  constexpr int A_CHUNKS = ROWS / 8, W_CHUNKS = TW * PL * 2;
+  constexpr int ES = A16 ? 2 : 4, LINE = 32 * ES, LANES = LINE / 16; // a row's part of a block, and lanes that fetch it
+  constexpr int A_CHUNKS = ROWS * LINE / 1024, W_CHUNKS = TW * PL * 2;
   constexpr int A_PER = (A_CHUNKS + WAVES - 1) / WAVES, W_PER = (W_CHUNKS + WAVES - 1) / WAVES, PER = A_PER + W_PER;
   constexpr int A_BYTES = A_CHUNKS * 1024, SLOT = (A_CHUNKS + W_CHUNKS) * 1024;
   extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [D][SLOT], then the rules
@@ -807,8 +808,9 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, q = lane >> 5;
   const int cg = wave % CW, rg = wave / CW;
-  const int split = tileOf % nSplits;
-  const long long wgRow0 = (long long)(tileOf / nSplits) * ROWS;
+  const unsigned rowTiles = tiles / nSplits;
+  const int split = byColumns ? tileOf / rowTiles : tileOf % nSplits;
+  const long long wgRow0 = (long long)(byColumns ? tileOf % rowTiles : tileOf / nSplits) * ROWS;
   const long long row0 = wgRow0 + rg * 32 * MT;
   const int n0 = split * NW + cg * 32 * NT; // this wavefront's columns
   const int T = K / 32;
@@ -831,19 +833,20 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   }
   const unsigned char *rowPtr[A_PER];
   int f = 0, ch = 0;
-  const int piece = 16 * ((lane & 7) ^ (lane >> 3));
+  // (A16: two rows lie on all banks, so that they are rotated by pairs)
+  const int piece = 16 * ((lane % LANES) ^ (A16 ? lane >> 3 & 3 : lane >> 3));
   auto aim = [&]() {
 #pragma unroll
     for (int u = 0; u < A_PER; ++u) {
       const int x = wave + WAVES * u;
-      const int r = 8 * (x < A_CHUNKS ? x : A_CHUNKS - 1) + (lane >> 3);
+      const int r = 64 / LANES * (x < A_CHUNKS ? x : A_CHUNKS - 1) + lane / LANES;
       if (GATHER) {
         const int rule = sRules[r * gs.fs + f];
-        rowPtr[u] = (rule >= 0 ? Ab + (long long)rule * gs.nIn * 4 : reinterpret_cast<const unsigned char *>(gs.zeros)) + piece;
+        rowPtr[u] = (rule >= 0 ? Ab + (long long)rule * gs.nIn * ES : reinterpret_cast<const unsigned char *>(gs.zeros)) + piece;
       } else {
         long long m = wgRow0 + r;
         m = m < M ? m : M - 1;
-        rowPtr[u] = Ab + m * K * 4 + piece;
+        rowPtr[u] = Ab + m * K * ES + piece;
       }
     }
   };
@@ -852,7 +855,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   };
   auto fetch_a = [&](int slot, int u) {
     const int x = wave + WAVES * u;
-    dma_kilobyte(lds0 + slot * SLOT + (x < A_CHUNKS ? x : A_CHUNKS - 1) * 1024, rowPtr[u] + ch * 4);
+    dma_kilobyte(lds0 + slot * SLOT + (x < A_CHUNKS ? x : A_CHUNKS - 1) * 1024, rowPtr[u] + ch * ES);
   };
   auto advance = [&]() { // to the next block's rows
     ch += 32;
@@ -864,17 +867,22 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   };
 
   // ---- operands
-  const unsigned char *const aLane = sW + (rg * 32 * MT + c) * 128;
-  const int swizzle = c & 7;
+  const unsigned char *const aLane = sW + (rg * 32 * MT + c) * LINE;
+  const int swizzle = A16 ? c >> 1 & 3 : c & 7;
   const unsigned char *const wLane = sW + A_BYTES + cg * NT * PL * 2048 + lane * 16;
   floatx4 raw[2];
-  auto read_a = [&](int slot, int u) { // unit u of a block: (step, row tile)
-    const unsigned char *const p = aLane + slot * SLOT + (u % MT) * 4096;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      raw[h] = *reinterpret_cast<const floatx4 *>(p + (((4 * (u / MT) + 2 * q + h) ^ swizzle) * 16));
-  };
   unsigned ap[2][PL][4]; // words of an MFMA operand: two k each
+  auto read_a = [&](int slot, int u) { // unit u of a block: (step, row tile)
+    const unsigned char *const p = aLane + slot * SLOT + (u % MT) * 32 * LINE;
+    if constexpr (A16) {
+      const uint4 w = *reinterpret_cast<const uint4 *>(p + (((2 * (u / MT) + q) ^ swizzle) * 16));
+      ap[u & 1][0][0] = w.x, ap[u & 1][0][1] = w.y, ap[u & 1][0][2] = w.z, ap[u & 1][0][3] = w.w;
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        raw[h] = *reinterpret_cast<const floatx4 *>(p + (((4 * (u / MT) + 2 * q + h) ^ swizzle) * 16));
+    }
+  };
   auto a_split = [&](int dst, int p) { // a quarter of it
     const floatx4 x = raw[p / 2];
     unsigned w[PL];
@@ -949,10 +957,12 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     read_b(0, 0, j);
+  if (!A16) {
 #pragma unroll
-  for (int p = 0; p < 4; ++p)
-    a_split(0, p);
-  read_a(0, 1);
+    for (int p = 0; p < 4; ++p)
+      a_split(0, p);
+    read_a(0, 1);
+  }
 
   constexpr int PRODUCTS = PL * (PL + 1) / 2;
   auto tile = [&](int s, int i, int j, int src) {
@@ -990,7 +1000,9 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
           lines_landed<0>();
         asm volatile("s_barrier" ::: "memory");
       }
-      if (MT == 1 && u == SECOND)
+      if (A16) // (where the last unit but one's operand was)
+        read_a(u + 1 < UNITS ? cur : next, (u + 1) % UNITS);
+      else if (MT == 1 && u == SECOND)
         read_a(next, 0);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
@@ -1002,14 +1014,15 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
         if (NT > 1 && i == MT - 1)
           read_b(s ? next : cur, s ^ 1, j);
 #pragma unroll
-        for (int p = 0; p < 4; ++p)
+        for (int p = 0; p < (A16 ? 0 : 4); ++p)
           if (j == (NT == 1 || !(MT == 1 && u == SECOND) ? p * NT / 4 : 1 + p * (NT - 1) / 4))
             a_split(src ^ 1, p);
-        if (j == NT - 1) // (split: its registers take the next but one)
+        if (!A16 && j == NT - 1) { // (split: its registers take the next but one)
           if (MT > 1)
             read_a(u + 2 < UNITS ? cur : next, (u + 2) % UNITS);
           else if (u == SECOND)
             read_a(next, 1);
+        }
         deal();
         if (more && u >= SECOND) {
           constexpr int G = MT * NT;
@@ -1267,7 +1280,7 @@ static void add_image(ImageList &l, const float *W, unsigned char *image, int pl
   l.W[i] = W, l.image[i] = image, l.K[i] = K, l.N[i] = N, l.fs[i] = fs, l.planes[i] = planes;
   l.firstBlock[i + 1] = l.firstBlock[i] + (unsigned)scn_ceil_div((int64_t)K / 8 * ((N + 31) / 32 * 32), 256);
 }
-template <int PL, int MT, int NT, int RW, int CW, int D>
+template <int PL, int MT, int NT, int RW, int CW, int D, bool A16 = false>
 static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
                         const Epilogue &ep, const GatherSource *gs, bool wT, const RowRange &rows,
                         const unsigned char *image) {
@@ -1279,16 +1292,19 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
     image = ctx->d_image;
   }
   constexpr int ROWS = 32 * MT * RW, COLUMNS = 32 * NT * CW;
-  const size_t lds = (size_t)D * (ROWS / 8 + NT * CW * PL * 2) * 1024 + (gs ? (size_t)ROWS * gs->fs * 4 : 0);
+  const size_t lds = (size_t)D * (ROWS / (A16 ? 16 : 8) + NT * CW * PL * 2) * 1024 + (gs ? (size_t)ROWS * gs->fs * 4 : 0);
   SCN_REQUIRE(lds <= 160 * 1024, SCN_ERR_ARG, "planes: %d filter positions", gs ? gs->fs : 0);
   const int nSplits = scn_ceil_div(N, COLUMNS);
   const dim3 grid((unsigned)(scn_ceil_div(M, ROWS) * (long long)nSplits));
+  // An XCD takes neighbouring tiles: rows with all their columns, so that they come
+  // to its L2 once, or, where the image is the larger part, columns with all rows.
+  const bool byColumns = image_bytes(PL, K, N) > (long long)scn_rows_hint(ctx, M) * (gs ? gs->nIn : K) * 4;
   if (gs)
-    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, true>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
-                       out, M, K, N, ep, *gs, nSplits, rows, PlainW{W, wT});
-  else
-    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
-                       out, M, K, N, ep, GatherSource(), nSplits, rows, PlainW{W, wT});
+    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, true, A16>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
+                       out, M, K, N, ep, *gs, nSplits, byColumns, rows, PlainW{W, wT});
+  else if constexpr (!A16)
+    hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false, false>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
+                       out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
   return SCN_OK;
 }
 template <int PL>
@@ -1401,14 +1417,14 @@ struct LinesTile {
   int mt, nt, rw, cw, d, resident;
   float f, t1, tn;
 };
-static const LinesTile linesTiles[2][5] = {
+static const LinesTile linesTiles[2][6] = {
     {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f}}, // one plane
     {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f},
-     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f}}};
+     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f}}};
 static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool gather, int *tile) {
   const int T = K / 32;
   float least = 1e30f;
-  for (int i = 0; i < (planes == 3 ? 5 : 3); ++i) {
+  for (int i = 0; i < (planes == 3 ? 6 : 3); ++i) {
     const LinesTile &x = linesTiles[planes == 3][i];
     const float n = (float)scn_ceil_div(M, 32 * x.mt * x.rw) * scn_ceil_div(N, 32 * x.nt * x.cw) / ctx->numCU;
     float cost;
@@ -1466,12 +1482,17 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
       SCN_LINES_CASE(2, 1, 3, 4, 1, 4)
       SCN_LINES_CASE(3, 1, 2, 2, 2, 4)
       SCN_LINES_CASE(4, 1, 1, 2, 2, 3)
+      SCN_LINES_CASE(5, 1, 1, 2, 2, 6)
     }
   } else if constexpr (PL == 1) {
     switch (choice.lines) {
       SCN_LINES_CASE(0, 1, 2, 4, 2, 3)
       SCN_LINES_CASE(1, 1, 2, 2, 2, 4)
       SCN_LINES_CASE(2, 1, 1, 2, 2, 3)
+    case 3: // (of bf16 rows)
+      return launch_lines<PL, 1, 2, 4, 2, 3, true>(ctx, A, W, out, M, K, N, ep, gs, wT, rows, choice.weights);
+    case 4:
+      return launch_lines<PL, 1, 1, 4, 2, 4, true>(ctx, A, W, out, M, K, N, ep, gs, wT, rows, choice.weights);
     }
   }
 #undef SCN_LINES_CASE
@@ -1533,6 +1554,15 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
   PlanesChoice choice = planes_choose(ctx, planes, rows, K, N, a16);
   const bool room = planes_image(ctx);
   choice.image = choice.image && room;
+  // (bf16 rows: a block takes half a line of each; long
+  // contractions, of 27 positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444
+  // us against 474, 400000 x 512 x 96 90 against 72, 140000 x 1024 x 256 111 against
+  // 85, 131071 x 256 x 64 20.8 against 15.9)
+  if (a16 && choice.tile >= 0 && K <= 1280 && N > 32 && lines_shape(1, K, gs->nIn) &&
+      (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES))) {
+    choice.lines = N <= 64 ? 4 : 3;
+    choice.weights = (const unsigned char *)image;
+  }
   if (choice.tile >= 0 && !a16)
     lines_instead(ctx, planes, rows, K, N, gs, image, room, choice);
   return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
