@@ -1647,11 +1647,18 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // a lane's eight are two loads (eight of them through row by row rules: 17.8 us
 // where this is 15.6 and a gathered matrix 14.5, and 8.2 to gather it).
 #define ATB_STEP 16
-template <int MT, int NT, bool GATHER>
+// LINES: the rows come into LDS by whole lines, a ring of steps for each wavefront,
+// which waits for nobody: a kilobyte to a request, where the loads above take 256 or
+// 512 bytes and every request occupies the path for 16 cycles or more, twice what the
+// splitting takes.  A backward layer with dW of 139000 x 384 x 128 384 -> 370 us;
+// dW of 28000 x 256 x 96 and its like 16.5 -> 15.6, of which some 5 are the start and
+// the atomics.
+constexpr int atb_ring(int MT, int NT) { return MT * NT >= 4 ? 2 : 3; }
+template <int MT, int NT, bool GATHER, bool LINES>
 __global__ void __launch_bounds__(512, 2)
     k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
                  float *__restrict__ dW, float *__restrict__ db, long long M, int K, int N, int nTiles,
-                 long long rowsPerSplit, GatherSource gs) {
+                 long long rowsPerSplit, GatherSource gs, const float *zeros) {
   constexpr int PL = 3, GM = 8;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
   extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], [8][32 NT], a flag
@@ -1771,38 +1778,147 @@ __global__ void __launch_bounds__(512, 2)
             d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[i][x], dp[j][y], d, 0, 0, 0);
           }
   };
-  const long long whole = m1 - ATB_STEP; // last start of a step without a guard
-  Step s0, s1;
-  long long m = m0 + ATB_STEP * wave; // a step in eight is this wavefront's
-  auto fetch = [&](Step &s, long long at) {
-    if (at <= whole)
-      load(s, at, false);
-    else
-      load(s, at < m1 ? at : m1 - 1, true);
-  };
-  if (m < m1) {
-    look_up(s0, m);
-    look_up(s1, m + ATB_STEP * GM);
-    fetch(s0, m);
-    look_up(s0, m + 2 * ATB_STEP * GM);
-    for (;;) {
-      const long long ma = m + ATB_STEP * GM;
-      if (ma < m1) {
-        fetch(s1, ma);
-        look_up(s1, ma + 2 * ATB_STEP * GM);
+  if constexpr (LINES) {
+    constexpr int RING = atb_ring(MT, NT), AU = 2 * MT, DU = 2 * NT, FETCH = AU + DU;
+    constexpr int SLOT = FETCH * 1024;
+    const int wave0 = __builtin_amdgcn_readfirstlane(wave);
+    unsigned char *const ring = reinterpret_cast<unsigned char *>(sTile) + wave0 * RING * SLOT;
+    const unsigned ldsRing = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)ring;
+    const long long pitch = (M + ATB_STEP - 1) / ATB_STEP * ATB_STEP;
+    // what this lane asks for: four columns of every 8 / MT-th (8 / NT-th) row
+    int ca = k0 + 4 * (lane % (8 * MT)), cd = n0 + 4 * (lane % (8 * NT));
+    ca = ca < K ? ca : K - 4, cd = cd < N ? cd : N - 4; // (past the end: not stored)
+    const int ra = lane / (8 * MT), rd = lane / (8 * NT);
+    const int f4 = GATHER ? ca / gs.nIn : 0, ch4 = GATHER ? ca - f4 * gs.nIn : 0;
+    const int steps = (int)((m1 - m0 - ATB_STEP * wave0 + ATB_STEP * GM - 1) / (ATB_STEP * GM));
+    auto place = [&](int t) { return m0 + ATB_STEP * (wave0 + (long long)GM * (t < steps ? t : steps - 1)); };
+    struct Rules {
+      int r[GATHER ? AU : 1];
+    };
+    auto ask = [&](Rules &x, int t) { // (the positions' pitch: whole steps)
+#pragma unroll
+      for (int u = 0; u < (GATHER ? AU : 0); ++u)
+        asm volatile("global_load_dword %0, %1, off"
+                     : "=v"(x.r[u % (GATHER ? AU : 1)])
+                     : "v"(gs.rules + f4 * pitch + place(t) + 8 / MT * u + ra)
+                     : "memory");
+    };
+    auto settle = [&](Rules &x) { // (asked for by then: their registers hold them from here on)
+#pragma unroll
+      for (int u = 0; u < (GATHER ? AU : 0); ++u)
+        asm volatile("" : "+v"(x.r[u % (GATHER ? AU : 1)]));
+    };
+    const float *const none = GATHER ? gs.zeros : zeros;
+    auto fetch = [&](const Rules &x, int t, int slot) {
+      const long long m = place(t);
+      const unsigned lds = ldsRing + slot * SLOT;
+#pragma unroll
+      for (int u = 0; u < AU; ++u) {
+        const long long row = m + 8 / MT * u + ra;
+        const int rule = x.r[GATHER ? u % AU : 0];
+        const float *const from = GATHER ? (rule >= 0 ? A + (long long)rule * gs.nIn + ch4 : none)
+                                         : (row < m1 ? A + row * K + ca : none);
+        dma_kilobyte(lds + u * 1024, reinterpret_cast<const unsigned char *>(from));
       }
-      compute(s0);
-      if (ma >= m1)
-        break;
-      const long long mb = ma + ATB_STEP * GM;
-      if (mb < m1) {
-        fetch(s0, mb);
-        look_up(s0, mb + 2 * ATB_STEP * GM);
+#pragma unroll
+      for (int u = 0; u < DU; ++u) {
+        const long long row = m + 8 / NT * u + rd;
+        dma_kilobyte(lds + (AU + u) * 1024, reinterpret_cast<const unsigned char *>(row < m1 ? D + row * N + cd : none));
       }
-      compute(s1);
-      if (mb >= m1)
-        break;
-      m = mb;
+    };
+    auto take = [&](Step &s, int slot) {
+      const unsigned char *const at = ring + slot * SLOT;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float *const pa = reinterpret_cast<const float *>(at) + (8 * q + i) * 32 * MT + MT * c;
+        const float *const pd = reinterpret_cast<const float *>(at + AU * 1024) + (8 * q + i) * 32 * NT + NT * c;
+        if constexpr (MT == 2) {
+          const floatx2 v = *reinterpret_cast<const floatx2 *>(pa);
+          s.a[i][0] = v[0], s.a[i][1] = v[1];
+        } else {
+          s.a[i][0] = *pa;
+        }
+        if constexpr (NT == 2) {
+          const floatx2 v = *reinterpret_cast<const floatx2 *>(pd);
+          s.d[i][0] = v[0], s.d[i][1] = v[1];
+        } else {
+          s.d[i][0] = *pd;
+        }
+      }
+    };
+    if (steps > 0) { // uniform
+      // Rules are asked for a step before their rows, in front of the rows asked for
+      // then: what has landed when all but the last step's rows have holds a step's
+      // rows and the next request's rules.
+      Rules x, y;
+      {
+        Rules first, second;
+        ask(first, 0);
+        ask(second, 1);
+        ask(x, RING - 1);
+        w_landed<0>();
+        settle(first);
+        settle(second);
+        fetch(first, 0, 0);
+        if (RING == 3)
+          fetch(second, 1, 1);
+      }
+      int slot = 0, into = RING - 1;
+      auto step = [&](int t, Rules &have, Rules &next) {
+        w_landed<RING == 3 ? FETCH : 0>(); // (and this wavefront's reads of the slot that is asked for again)
+        settle(have);
+        ask(next, t + RING);
+        fetch(have, t + RING - 1, into);
+        Step s;
+        take(s, slot);
+        compute(s);
+        slot = slot == RING - 1 ? 0 : slot + 1, into = into == RING - 1 ? 0 : into + 1;
+      };
+#pragma unroll 1
+      for (int t = 0; t < steps; t += 2) {
+        step(t, x, y);
+        if (t + 1 < steps)
+          step(t + 1, y, x);
+      }
+      w_landed<0>();
+      settle(x); // (rules that nobody needs have their registers until they have come)
+      settle(y);
+    }
+    __syncthreads(); // (the sums take the rings' place)
+  } else {
+    const long long whole = m1 - ATB_STEP; // last start of a step without a guard
+    Step s0, s1;
+    long long m = m0 + ATB_STEP * wave; // a step in eight is this wavefront's
+    auto fetch = [&](Step &s, long long at) {
+      if (at <= whole)
+        load(s, at, false);
+      else
+        load(s, at < m1 ? at : m1 - 1, true);
+    };
+    if (m < m1) {
+      look_up(s0, m);
+      look_up(s1, m + ATB_STEP * GM);
+      fetch(s0, m);
+      look_up(s0, m + 2 * ATB_STEP * GM);
+      for (;;) {
+        const long long ma = m + ATB_STEP * GM;
+        if (ma < m1) {
+          fetch(s1, ma);
+          look_up(s1, ma + 2 * ATB_STEP * GM);
+        }
+        compute(s0);
+        if (ma >= m1)
+          break;
+        const long long mb = ma + ATB_STEP * GM;
+        if (mb < m1) {
+          fetch(s0, mb);
+          look_up(s0, mb + 2 * ATB_STEP * GM);
+        }
+        compute(s1);
+        if (mb >= m1)
+          break;
+        m = mb;
+      }
     }
   }
 #pragma unroll
@@ -1904,13 +2020,14 @@ __global__ void __launch_bounds__(512, 2)
   }
 }
 
-template <int MT, int NT, bool GATHER>
+template <int MT, int NT, bool GATHER, bool LINES>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                       long long M, int K, int N, long long splits, const GatherSource &gs) {
-  const size_t lds = ((size_t)8 * 32 * MT * 32 * NT + 8 * 32 * NT + 1) * sizeof(float);
+  const size_t sums = ((size_t)8 * 32 * MT * 32 * NT + 8 * 32 * NT + 1) * sizeof(float);
+  const size_t rings = (size_t)8 * atb_ring(MT, NT) * 2048 * (MT + NT), lds = LINES && rings > sums ? rings : sums;
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER>),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER, LINES>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
                ? SCN_OK
                : SCN_ERR_HIP;
@@ -1920,18 +2037,22 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, f
   const long long tiles = (long long)scn_ceil_div(K, 32 * MT) * nTiles;
   long long rows = (M + splits - 1) / splits;
   rows = (rows + 8 * ATB_STEP - 1) / (8 * ATB_STEP) * (8 * ATB_STEP);
-  hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
-                     dim3(512), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs);
+  hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER, LINES>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
+                     dim3(512), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs, ctx->d_zeros);
   return SCN_OK;
 }
 template <int MT, int NT>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db, long long M, int K, int N,
-                      long long splits, const GatherSource *gs) {
+                      long long splits, const GatherSource *gs, bool lines) {
   if constexpr (MT == 2 && NT == 2) // (not gathered: see below)
-    return launch_atb<MT, NT, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
+    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, splits, GatherSource())
+                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
+  else if (gs)
+    return lines ? launch_atb<MT, NT, true, true>(ctx, A, D, dW, db, M, K, N, splits, *gs)
+                 : launch_atb<MT, NT, true, false>(ctx, A, D, dW, db, M, K, N, splits, *gs);
   else
-    return gs ? launch_atb<MT, NT, true>(ctx, A, D, dW, db, M, K, N, splits, *gs)
-              : launch_atb<MT, NT, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
+    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, splits, GatherSource())
+                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
 }
 
 // The tile and the number of row ranges that cost least: rounds of one workgroup
@@ -1967,13 +2088,15 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
     }
   }
   SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
+  // (requests of four columns, in one filter position each)
+  const bool lines = K % 4 == 0 && N % 4 == 0 && (!gs || gs->nIn % 4 == 0) && (((uintptr_t)A | (uintptr_t)D) & 15) == 0;
   switch (best) {
   case 1:
-    return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, splits, gs);
+    return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
   case 2:
-    return launch_atb<1, 2>(ctx, A, D, dW, db, M, K, N, splits, gs);
+    return launch_atb<1, 2>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
   case 3:
-    return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, splits, gs);
+    return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
   }
-  return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, splits, gs);
+  return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
 }

@@ -116,3 +116,27 @@ def test_products_with_the_transpose(scn, ctx, M, N, K):
     assert np.all(got[M:] == 7)
     # products to 2^-25, one rounding of the sum every few k (as in test_gpu_planes.py)
     assert (np.abs(got[:M] - want) / scale).max() <= 2e-6
+
+
+# rows: part of a step of sixteen, a step and a row more, fewer steps than the ring holds, several ranges of rows;
+# columns that are no whole tile, two filter positions to a tile of 64 (or, in fours, three)
+@pytest.mark.parametrize("M", [1, 15, 17, 129, 391, 2051, 40003])
+@pytest.mark.parametrize("fs,nIn,N", [(3, 36, 44), (4, 32, 64), (2, 96, 160), (9, 8, 4)])
+def test_weight_gradients_by_lines(scn, ctx, M, fs, nIn, N):
+    rng = np.random.default_rng(M + nIn)
+    K = fs * nIn
+    x, D = rng.standard_normal((300, nIn), dtype=np.float32), rng.standard_normal((M, N), dtype=np.float32)
+    rules = rng.integers(-1, 300, (M, fs)).astype(np.int32)
+    pitch = (M + 15) // 16 * 16
+    positions = ctx.array(np.ascontiguousarray(np.pad(rules.T, ((0, 0), (0, pitch - M)), constant_values=-1)))
+    dense = np.where(rules[:, :, None] >= 0, x[np.maximum(rules, 0)], 0).reshape(M, K).astype(np.float32)
+    want, scale = dense.T.astype(np.float64) @ D, np.abs(dense.T).astype(np.float64) @ np.abs(D) + 1e-30
+    d_x, d_D, d_A = ctx.array(x), ctx.array(D), ctx.array(dense)
+    dW, dB, plain = ctx.array(np.full((K, N), 7, np.float32)), ctx.array(np.full(N, 7, np.float32)), ctx.empty((K, N), np.float32)
+    print("dW by lines", M, fs, nIn, N, flush=True)
+    ctx.conv_AtB(d_x, positions, fs, nIn, d_D, dW, M, N, d_db=dB)
+    ctx.sgemm_AtB(d_A, d_D, plain, M, K, N)
+    # products to 2^-25 and one rounding of a sum every few rows, as in test_gpu_planes.py
+    for got in (dW, plain):
+        assert (np.abs(got.download() - want) / scale).max() <= 2e-6
+    assert (np.abs(dB.download() - D.sum(0, dtype=np.float64)) / (np.abs(D).sum(0) + 1e-30)).max() <= 2e-6
