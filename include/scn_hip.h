@@ -20,10 +20,12 @@
  *     row-major int32 [output rows x rule width]; rows are batch-global;
  *   - numeric kernels never allocate: every buffer is the caller's
  *     (SpatiallySparseBatchSubInterface, SpatiallySparseBatchInterface.h:8-17).
- *     A long contraction puts its layer's weights, laid out for the matrix
+ *     A contraction in planes puts its layer's weights, laid out for the matrix
  *     cores, into room that scn_ctx_create has made for the context (16 MB;
- *     never while its stream is being captured, or where there was no memory
- *     for it: the weights are then converted on the way, to the same bits).
+ *     never while its stream is being captured, where there was no memory
+ *     for it or they are more: the weights are then converted on the way, to
+ *     the same bits), unless the caller has laid them out
+ *     (scn_weight_images_many).
  *     scn_grids objects own their tables and only ever grow them.
  */
 #ifndef SCN_HIP_H

@@ -56,7 +56,7 @@ struct scn_ctx {
   int64_t *d_pinned; // the same memory as the device sees it
   int64_t *d_scalars; // 16 int64
   float *d_zeros;     // SCN_ZERO_FLOATS zeros: the row a negative rule stands for
-  unsigned char *d_image; // SCN_IMAGE_BYTES or null: a layer's weights as a long contraction streams them
+  unsigned char *d_image; // SCN_IMAGE_BYTES or null: a layer's weights as its contraction reads them
   long long ticket;   // number of the last count readback (h_pinned[14] echoes it)
   // deferred counts (scn_ctx_defer_counts): plans whose counts are still on
   // their way; slot i of them reports into h_pinned[16 + 4 i ..]

@@ -1126,10 +1126,9 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   }
 }
 
-// The image of W that the long contractions stream: for every slice of 32 NT
+// The image of W that k_nin_planes reads: for every slice of 32 NT
 // columns and every block of 32 k what w_store leaves in LDS, in that order.
-// WT: W is given as its transpose, [N x K].
-template <int PL, int NT, bool WT>
+template <int PL, int NT>
 __global__ void __launch_bounds__(256)
     k_planes_image(const float *__restrict__ W, unsigned char *__restrict__ image,
                    int K, int N, int nSplits) {
@@ -1144,11 +1143,11 @@ __global__ void __launch_bounds__(256)
   const int kg = x / NW, tile = (x % NW) / 32, cc = x % 32;
   int n = split * NW + NT * cc + tile;
   n = n < N ? n : N - 1;
-  const float *const src = WT ? W + (long long)n * K + 32 * t + 8 * kg : W + (long long)(32 * t + 8 * kg) * N + n;
+  const float *const src = W + (long long)(32 * t + 8 * kg) * N + n;
   float v[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    v[i] = src[WT ? i : (long long)i * N];
+    v[i] = src[(long long)i * N];
   bf16x8 p[PL];
   split8<PL>(v, p);
 #pragma unroll
@@ -1230,27 +1229,25 @@ static bool planes_image(scn_ctx *ctx) {
 constexpr int planes_depth(int PL, int MT, int NT) {
   return PL * MT * NT <= 4 || (PL < 3 && MT == 1) ? 2 : 1;
 }
-// (W_STREAM: gathered rows, with one plane bf16 ones)
+// (W_STREAM: gathered rows, with one plane bf16 ones.  W_IMAGE: gathered rows, with
+// two planes any; k_nin_lines takes the others.)
 template <int PL, int MT, int NT, int WM, bool FINE = false, int WAVES = 4>
 static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
-                         const Epilogue &ep, const GatherSource *gs, bool a16, bool wT,
-                         const RowRange &rows) {
+                         const Epilogue &ep, const GatherSource *gs, bool a16, const RowRange &rows) {
   const int nSplits = scn_ceil_div(N, 32 * NT);
   const size_t lds = (size_t)(WM == W_STREAM ? 3 : 2) * PL * 2 * NT * 1024 +
                      (gs ? (size_t)32 * WAVES * MT * gs->fs * 4 : 0);
   constexpr int G = FINE ? 2 : 1, PD = planes_depth(PL, MT, NT);
   // (what a launch may ask for without saying so: saying it costs 0.1 ms and more a kernel)
   SCN_REQUIRE(lds <= 64 * 1024, SCN_ERR_ARG, "planes: %d filter positions", gs ? gs->fs : 0);
-  const PlainW plain = {W, wT};
+  const PlainW plain = {W, 0};
+  constexpr bool GATHERED = WM == W_STREAM || (WM == W_IMAGE && PL != 2);
+  SCN_REQUIRE(gs || !GATHERED, SCN_ERR_ARG, "planes: no rules");
   if (WM != W_PLAIN) {
     const long long items = (long long)nSplits * (K / 32) * 4 * 32 * NT;
-    if (PL == 3 && wT)
-      hipLaunchKernelGGL((k_planes_image<PL, NT, PL == 3>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream,
-                         W, ctx->d_image, K, N, nSplits);
-    else
-      hipLaunchKernelGGL((k_planes_image<PL, NT, false>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream, W,
-                         ctx->d_image, K, N, nSplits);
+    hipLaunchKernelGGL((k_planes_image<PL, NT>), dim3(scn_ceil_div(items, 256)), dim3(256), 0, ctx->stream, W, ctx->d_image,
+                       K, N, nSplits);
     W = reinterpret_cast<const float *>(ctx->d_image);
   }
   const dim3 grid((unsigned)(scn_ceil_div(M, 32 * WAVES * MT) * (long long)nSplits));
@@ -1258,13 +1255,14 @@ static int launch_planes(scn_ctx *ctx, const float *A, const float *W,
   hipLaunchKernelGGL((k_nin_planes<PL, MT, NT, PD, G, H, WM, WAVES>), grid,   \
                      dim3(64 * WAVES), lds, ctx->stream, A, W, out, M, K, N,   \
                      ep, src, nSplits, rows, plain)
-  if constexpr (WM == W_STREAM)
+  if constexpr (!GATHERED)
+    if (!gs) {
+      SCN_PLANES_GO(0, false, GatherSource());
+      return SCN_OK;
+    }
+  if (WM == W_STREAM || (PL == 1 && a16))
     SCN_PLANES_GO(G, PL == 1, *gs);
-  else if (!gs)
-    SCN_PLANES_GO(0, false, GatherSource());
-  else if (PL == 1 && a16)
-    SCN_PLANES_GO(G, PL == 1, *gs);
-  else
+  else if constexpr (WM != W_STREAM)
     SCN_PLANES_GO(G, false, *gs);
 #undef SCN_PLANES_GO
   return SCN_OK;
@@ -1382,7 +1380,7 @@ struct PlanesChoice {
   int lines = -1; // k_nin_lines, a tile of its own: index into linesTiles
   const unsigned char *weights = nullptr; // the image it reads, null: to be made
 };
-// needImage: of the tiles, only from the image
+// needImage: of the tiles, only from the image (scn_planes_abt: whether there is one)
 static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16,
                                    bool needImage = false) {
   if (M <= split_rows(ctx, planes, K, N))
@@ -1498,7 +1496,7 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
 #undef SCN_LINES_CASE
   // (channels in other than 32s, seldom met: one tile)
   if (gs && gs->nIn % 32 != 0)
-    return launch_planes<PL, 1, 2, W_PLAIN, true>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
+    return launch_planes<PL, 1, 2, W_PLAIN, true>(ctx, A, W, out, M, K, N, ep, gs, a16, rows);
   // W_STREAM where the chip is full and the contraction long: the widest tile, W
   // from its image, rows gathered (by no more than 27 positions: with the third
   // buffer two workgroups still fit a compute unit's LDS).  The registers it frees
@@ -1513,12 +1511,12 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   if constexpr (PL != 2)
     if (choice.tile == 3 && choice.image && gs && (PL > 1 || a16))
       return launch_planes<PL, (PL > 1 ? 2 : 1), (PL > 1 ? 2 : 4), W_STREAM, false, (PL > 1 ? 4 : 8)>(
-          ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
+          ctx, A, W, out, M, K, N, ep, gs, a16, rows);
 #define SCN_PLANES_CASE(I, MT, NT)                                             \
   case I:                                                                      \
     return choice.image                                                        \
-               ? launch_planes<PL, MT, NT, W_IMAGE>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows) \
-               : launch_planes<PL, MT, NT, W_PLAIN>(ctx, A, W, out, M, K, N, ep, gs, a16, false, rows);
+               ? launch_planes<PL, MT, NT, W_IMAGE>(ctx, A, W, out, M, K, N, ep, gs, a16, rows) \
+               : launch_planes<PL, MT, NT, W_PLAIN>(ctx, A, W, out, M, K, N, ep, gs, a16, rows);
   switch (choice.tile) {
     SCN_PLANES_CASE(0, 1, 1)
     SCN_PLANES_CASE(1, 1, 2)
@@ -1624,7 +1622,7 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
   const bool room = planes_image(ctx);
   if (choice.tile >= 0)
     lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, choice);
-  if (choice.tile >= 0 && !(room && (choice.image || choice.lines >= 0))) {
+  if (choice.tile >= 0 && choice.lines < 0) {
     *transpose = choice.image;
     return false;
   }
