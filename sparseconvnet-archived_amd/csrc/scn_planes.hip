@@ -1433,12 +1433,25 @@ static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, b
       const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
       cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));
     }
-    if (planes == 3 && gather && n > 4.f) // (rows that few workgroups share, and the clock)
+    // (rows that few workgroups share, and the clock: 130000 x 512 x 64 63 us in the
+    // second tile, 58 in k_nin_planes)
+    if (planes == 3 && gather && n > (x.mt > 1 ? 1.f : 4.f))
       cost *= 1.12f;
     if (cost < least)
       least = cost, *tile = i;
   }
   return least + 4.f;
+}
+// The same of bf16 rows, whose tile goes by the columns, and with the image where it
+// is not made yet.  Fitted to 49 shapes (3500 to 120000 rows, 256 to 1152 k, 64 to
+// 320 columns).  Making the image is what small layers would lose by: us in
+// k_nin_planes -> here, 9000 x 576 x 160 11.1 -> 13.9, 30000 x 256 x 64 8.7 -> 9.1;
+// 9000 x 1024 x 320 30 -> 21, 60000 x 512 x 128 25 -> 21, 120000 x 576 x 160 61 -> 54.
+static float lines_rows16(scn_ctx *ctx, long long M, int K, int N, bool image) {
+  const float n = (float)scn_ceil_div(M, 128) * scn_ceil_div(N, N <= 64 ? 64 : 128) / ctx->numCU;
+  const float x = fmaxf(n - .5f, 0.f), T = K / 32;
+  return (N <= 64 ? 3.f + 2.6f * x + T * (.2f + .15f * x) : 2.3f + 1.6f * x + T * (.37f + .22f * x)) +
+         (image ? 0.f : 3.f + (float)K * N / 150000.f);
 }
 bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
   return M <= split_rows(ctx, planes, K, N);
@@ -1552,12 +1565,13 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
   PlanesChoice choice = planes_choose(ctx, planes, rows, K, N, a16);
   const bool room = planes_image(ctx);
   choice.image = choice.image && room;
-  // (bf16 rows: a block takes half a line of each; long
-  // contractions, of 27 positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444
-  // us against 474, 400000 x 512 x 96 90 against 72, 140000 x 1024 x 256 111 against
-  // 85, 131071 x 256 x 64 20.8 against 15.9)
+  // (bf16 rows: a block takes half a line of each; long contractions, of 27
+  // positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444 us against 474.
+  // k_nin_planes' cost is 2 too high where it converts W on the way, of layers that
+  // small.)
   if (a16 && choice.tile >= 0 && K <= 1280 && N > 32 && lines_shape(1, K, gs->nIn) &&
-      (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES))) {
+      (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES)) &&
+      lines_rows16(ctx, rows, K, N, image != nullptr) < choice.cost - (choice.image ? 0.f : 2.f)) {
     choice.lines = N <= 64 ? 4 : 3;
     choice.weights = (const unsigned char *)image;
   }
