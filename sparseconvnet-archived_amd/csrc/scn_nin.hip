@@ -505,8 +505,16 @@ __global__ void __launch_bounds__(256)
 // values a lane) and walks all of its columns, CT_COLS at most, in blocks of
 // 32; the products of an output are those of the plain kernel on the gathered
 // matrix, in the same order.
+// LDS is what it waits for: with a read of A, on four rows' banks, for every read of
+// W 139500 x 12 x 160 took 34 us (2.6 TB/s written).  A lane takes four k of a row at
+// once and holds CT_GROUPS rows against what it reads of W: two 24.7 us, four 23.0,
+// but 66500 rows 15.8 and 18.5 (21.1 before), 83597 x 12 x 32 7.3 and 8.1 (8.9).
+// Few rows want workgroups and a short chain of loads, one group: 900 x 12 x 32 5.1 ->
+// 3.5 us (two groups 4.3), 30000 5.9 -> 4.5 (4.9), 40001 x 12 x 64 9.3 -> 6.8 (7.5);
+// at 66500 x 12 x 160 and 83597 x 12 x 32 two are ahead (16.8, 8.3 with one).
 #define CT_COLS 256
-#define CT_GROUPS 2 // groups of 32 rows a workgroup takes: all their loads are in flight together
+#define CT_PITCH (TK_MAX_K + 4) // floats: eight rows' reads of four k lie on all banks
+template <int CT_GROUPS>
 __global__ void __launch_bounds__(256)
     k_conv_thin(const float *__restrict__ A, const float *__restrict__ W,
                 float *__restrict__ out, long long M, int K, int N, Epilogue ep,
@@ -519,7 +527,7 @@ __global__ void __launch_bounds__(256)
   // LDS: the gathered rows, then this workgroup's columns of W at pitch wp
   extern __shared__ __attribute__((aligned(16))) float ctLds[];
   float *const sA = ctLds;
-  float *const sW = ctLds + CT_GROUPS * 32 * TK_MAX_K;
+  float *const sW = ctLds + CT_GROUPS * 32 * CT_PITCH;
   const int wp = N < CT_COLS ? N : CT_COLS;
   const int tid = threadIdx.x;
   const int n0 = blockIdx.y * CT_COLS;
@@ -547,34 +555,56 @@ __global__ void __launch_bounds__(256)
       float v = 0.f;
       if (rule[g][j] >= 0)
         v = A[(long long)rule[g][j] * gs.nIn + (k - gather_rule_of(gs, k) * gs.nIn)];
-      sA[(32 * g + r) * TK_MAX_K + k] = v;
+      sA[(32 * g + r) * CT_PITCH + k] = v;
     }
   __syncthreads();
+  const float *const arow = sA + r * CT_PITCH;
+  for (int c4 = (tid & 7) * 4; c4 < cols; c4 += 32) {
+    float4 acc[CT_GROUPS];
 #pragma unroll
-  for (int g = 0; g < CT_GROUPS; ++g) {
-    const long long m = mFirst + 32 * g;
-    if (m >= M)
-      break;
-    const float *arow = sA + (32 * g + r) * TK_MAX_K;
-    for (int c4 = (tid & 7) * 4; c4 < cols; c4 += 32) {
-      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int k = 0; k < K; ++k) {
-        const float a = arow[k];
-        const float4 wv = *reinterpret_cast<const float4 *>(&sW[k * wp + c4]);
-        acc.x = fmaf(a, wv.x, acc.x);
-        acc.y = fmaf(a, wv.y, acc.y);
-        acc.z = fmaf(a, wv.z, acc.z);
-        acc.w = fmaf(a, wv.w, acc.w);
+    for (int g = 0; g < CT_GROUPS; ++g)
+      acc[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k = 0; k < K; k += 4) { // K % 4 == 0
+      float a[CT_GROUPS][4];
+#pragma unroll
+      for (int g = 0; g < CT_GROUPS; ++g) {
+        const float4 v = *reinterpret_cast<const float4 *>(arow + 32 * g * CT_PITCH + k);
+        a[g][0] = v.x, a[g][1] = v.y, a[g][2] = v.z, a[g][3] = v.w;
       }
-      const int n = n0 + c4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 wv = *reinterpret_cast<const float4 *>(&sW[(k + i) * wp + c4]);
+#pragma unroll
+        for (int g = 0; g < CT_GROUPS; ++g) {
+          acc[g].x = fmaf(a[g][i], wv.x, acc[g].x);
+          acc[g].y = fmaf(a[g][i], wv.y, acc[g].y);
+          acc[g].z = fmaf(a[g][i], wv.z, acc[g].z);
+          acc[g].w = fmaf(a[g][i], wv.w, acc[g].w);
+        }
+      }
+    }
+    const int n = n0 + c4;
+#pragma unroll
+    for (int g = 0; g < CT_GROUPS; ++g) {
+      const long long m = mFirst + 32 * g;
+      if (m >= M)
+        break;
       float4 o;
-      o.x = apply_act(acc.x, n, ep);
-      o.y = apply_act(acc.y, n + 1, ep);
-      o.z = apply_act(acc.z, n + 2, ep);
-      o.w = apply_act(acc.w, n + 3, ep);
+      o.x = apply_act(acc[g].x, n, ep);
+      o.y = apply_act(acc[g].y, n + 1, ep);
+      o.z = apply_act(acc[g].z, n + 2, ep);
+      o.w = apply_act(acc[g].w, n + 3, ep);
       *reinterpret_cast<float4 *>(out + m * N + n) = o;
     }
   }
+}
+
+template <int G>
+static void launch_conv_thin(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
+                             const Epilogue &ep, const GatherSource &gs, const long long *dRows) {
+  const size_t lds = (size_t)(G * 32 * CT_PITCH + K * (N < CT_COLS ? N : CT_COLS)) * sizeof(float);
+  hipLaunchKernelGGL(k_conv_thin<G>, dim3(scn_ceil_div(M, 32 * G), scn_ceil_div(N, CT_COLS)), dim3(256), lds, ctx->stream,
+                     A, W, out, M, K, N, ep, gs, dRows);
 }
 
 // ---- MFMA path: fp32 operands, v_mfma_f32_32x32x2_f32 ----------------------
@@ -1881,10 +1911,10 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
     }
   } else if (vec && gs && gs->nIn % 4 != 0) {
     // channels in other than fours: K <= TK_MAX_K (scn_conv_nin_supported)
-    const size_t lds = (size_t)(CT_GROUPS * 32 * TK_MAX_K + K * (N < CT_COLS ? N : CT_COLS)) * sizeof(float);
-    hipLaunchKernelGGL(k_conv_thin, dim3(scn_ceil_div(M, 32 * CT_GROUPS), scn_ceil_div(N, CT_COLS)),
-                       dim3(256), lds, ctx->stream, d_A, d_W, d_out, (long long)M,
-                       K, N, ep, *gs, dRows);
+    if (scn_rows_hint(ctx, M) <= 6ll * 32 * ctx->numCU)
+      launch_conv_thin<1>(ctx, d_A, d_W, d_out, (long long)M, K, N, ep, *gs, dRows);
+    else
+      launch_conv_thin<2>(ctx, d_A, d_W, d_out, (long long)M, K, N, ep, *gs, dRows);
   } else if (vec && !gs && K <= TK_MAX_K) {
     hipLaunchKernelGGL(k_nin_thin, dim3(scn_ceil_div(M, 32), scn_ceil_div(N, 32)),
                        dim3(256), 0, ctx->stream, d_A, d_W, d_out, (long long)M,
