@@ -479,8 +479,8 @@ int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in, const int32_t *d
  *   d_positions [fs x scn_positions_pitch(rows)]: the rules position by position,
  *     padded with -1;
  *   d_inverse [inputRows x fs]: which of the `rows` output rows names an input row
- *     at each filter position (-1: none); for the background row of sample s, which
- *     any number may name, that is rows + s fs + f;
+ *     at each filter position (negative: none); for the background row of sample s,
+ *     which any number may name, that is rows + s fs + f;
  *   d_background [rows + 2 batch]: a bit for every position at which a row names
  *     its sample's background row, then for every sample the first and the last of
  *     its rows with any (2^31 - 1 and -1: none).
@@ -495,7 +495,8 @@ int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in, const int32_t *d
  * scn_transpose_filters_many gives the weights, Wt [fs N x nIn] of W [fs nIn x
  * N], and scn_conv_input_gradient writes every input row's gradient, d_din
  * [inputRows x nIn], from d_delta (where scn_conv_nin_supported_p(fs, N, nIn,
- * SCN_FP32); d_image: of Wt, SCN_FP32_PLANES, or null). */
+ * SCN_FP32); d_image: of Wt, SCN_FP32_PLANES, or null); a position at which no row
+ * names an input row adds nothing to it, whatever the weights. */
 #define SCN_INVERSE_MAX 16
 typedef struct scn_inverse_item {
   const scn_grids *input; /* the convolution's input grids, counts settled */

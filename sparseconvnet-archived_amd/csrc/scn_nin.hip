@@ -2056,7 +2056,7 @@ extern "C" int scn_conv_nin_forward(scn_ctx *ctx, const float *d_in,
 }
 static int conv_nin_forward(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn,
                             const float *d_W, const void *d_image, const float *d_B, const float *d_prelu,
-                            float *d_out, int64_t M, int N, float p, int act, int precision) {
+                            float *d_out, int64_t M, int N, float p, int act, int precision, bool namedOnly = false) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_nin_forward: null context");
   SCN_REQUIRE(scn_conv_nin_supported_p(fs, nIn, N, precision), SCN_ERR_ARG,
               "scn_conv_nin_forward: fs %d nIn %d N %d precision %d is outside "
@@ -2073,8 +2073,19 @@ static int conv_nin_forward(scn_ctx *ctx, const float *d_in, const int32_t *d_ru
   gs.nIn = nIn;
   gs.magic = (unsigned)((1ull << 32) / (unsigned)nIn + 1);
   gs.zeros = ctx->d_zeros;
+  gs.namedOnly = namedOnly;
   return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p,
                      act, precision, &gs, nullptr, d_image);
+}
+bool scn_conv_takes_planes(const float *A, const float *W, const float *out, int K, int N) {
+  return scn_planes_shape(K) && (N % 16 == 0 || (N % 4 == 0 && K > FR_MAX_K)) &&
+         (((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) & 15) == 0;
+}
+int scn_conv_named(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn, const float *d_W,
+                   const void *d_image, float *d_out, int64_t M, int N) {
+  SCN_REQUIRE(((uintptr_t)d_image & 15) == 0, SCN_ERR_ARG, "scn_conv_nin_forward: the image starts on 16 bytes");
+  return conv_nin_forward(ctx, d_in, d_rules, fs, nIn, d_W, d_image, ctx->d_zeros, nullptr, d_out, M, N, 1.f,
+                          SCN_NOSIGMOID, SCN_FP32_PLANES, true);
 }
 extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
                                       const int32_t *d_rules, int fs, int nIn,

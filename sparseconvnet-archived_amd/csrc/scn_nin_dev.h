@@ -45,6 +45,9 @@ struct GatherSource {
   int nIn;            // channels of the gathered matrix, nIn % 4 == 0
   unsigned magic;     // floor(2^32 / nIn) + 1: k / nIn == mulhi(k, magic) for k nIn < 2^32
   const float *zeros; // at least nIn zeros: the row a negative rule stands for
+  // a negative rule adds nothing, and not 0 times its weights: the same but for
+  // weights that are not finite (scn_planes_forward with three planes only)
+  int namedOnly;
 };
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -56,6 +59,13 @@ __device__ __forceinline__ unsigned pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(unsigned, h);
 }
 
+// scn_nin.hip: nin_forward takes the fused convolution of SCN_FP32_PLANES to
+// scn_planes_forward, whatever the rows
+bool scn_conv_takes_planes(const float *A, const float *W, const float *out, int K, int N);
+// scn_conv_nin_forward_image without bias and activation, in SCN_FP32_PLANES;
+// with scn_conv_takes_planes, GatherSource::namedOnly
+int scn_conv_named(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn, const float *d_W,
+                   const void *d_image, float *d_out, int64_t M, int N);
 // scn_planes.hip: the contraction with fp32 operands as `planes` bf16 planes
 bool scn_planes_shape(int K);
 // ... takes the split contraction: few rows

@@ -107,6 +107,44 @@ __device__ __forceinline__ floatx16 tile_f32(const float *A, const GatherSource 
 #pragma unroll
   for (int v = 0; v < 16; ++v)
     sum[v] = 0.f;
+  if (GATHER && gs.namedOnly) {
+    // position by position, each of which the rows that it is named for take
+    for (int f = 0; f < gs.fs; ++f) {
+      const unsigned named = (unsigned)__ballot(rules[f] >= 0); // row by row (the upper half holds them again)
+      if (!named)
+        continue;
+      floatx16 part;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        part[v] = 0.f;
+#pragma unroll 1
+      for (int t = 0; t < gs.nIn; t += 16) {
+        float a[8], b[8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = t + 8 * q + 4 * h;
+          const bool inside = k < gs.nIn; // (in fours)
+          const floatx4 x = gathered_piece<false>(reinterpret_cast<const unsigned char *>(A), gs, rules,
+                                                  f * gs.nIn + (inside ? k : 0));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            a[4 * h + i] = inside ? x[i] : 0.f;
+            b[4 * h + i] = inside ? w.W[(long long)(f * gs.nIn + k + i) * N + n] : 0.f;
+          }
+        }
+        mfma8_f32(a, b, part);
+      }
+      bool open = false;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        sum[v] += named >> (8 * (v / 4) + 4 * q + v % 4) & 1 ? part[v] : 0.f;
+        open |= (mine >> v & 1) && sum[v] == sum[v];
+      }
+      if (!__any(open))
+        break;
+    }
+    return sum;
+  }
 #pragma unroll 1
   for (int t = 0; t < K; t += 16) { // (K is a multiple of 32)
     const int k = t + 8 * q;

@@ -296,14 +296,15 @@ extern "C" int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_po
 // input gets, for every filter position f at which an output row o names it,
 // D[o] W_f^T.  There is one such o at most, unless r is a background row, which
 // any number of windows names.  So a layer's rules are turned round once
-// (inverse[r * fs + f] = o, -1: none); the rows of D that name a sample's
+// (inverse[r * fs + f] = o, negative: none); the rows of D that name a sample's
 // background row (background[o]: at which positions) are summed per position
 // (k_background_sums) into rows behind D's own, which the background row's
 // inverse names; and the forward kernels do
 // the rest on W with every position's block transposed: no matrix of M x K is
 // written and read again, none is cleared, and no float is added atomically but
-// those few.  (Where W holds an infinity, a position that no row names adds 0
-// times it: NaN, and not nothing.  Such a net's forward pass is full of them.)
+// those few.  (A position that no row names adds nothing, as in the scatter, and
+// not 0 times its weights, which may be infinite: GatherSource::namedOnly, and
+// k_input_gradient_again for the shapes that the planes do not take.)
 // Of a batch of 100 drawings the backward kernels of the layer 57000 x 128 -> 64
 // take 4.4 + 17.2 + 22.5 + 14.7 us with the matrix (image, dW, dA, scatter; 8.2
 // for the gathering besides) and 15.6 + 6.3 + 19.3 without (dW, sums, gradient);
@@ -329,10 +330,11 @@ __global__ __launch_bounds__(256) void k_inverse_background(InverseList l) {
       l.background[t][l.rows[t] + 2 * s] = 0x7fffffff;
       l.background[t][l.rows[t] + 2 * s + 1] = -1;
     }
+  // (-2 - x: a background row's, until a row that names it is met)
   for (int x = threadIdx.x; x < l.batch[t] * fs; x += 256) {
     const int r = l.bg[t][x / fs];
     if (r >= 0 && r < l.inRows[t])
-      l.inverse[t][(long long)r * fs + x % fs] = l.rows[t] + x;
+      l.inverse[t][(long long)r * fs + x % fs] = -2 - x;
   }
 }
 // a lane a row of the output
@@ -358,11 +360,13 @@ __global__ __launch_bounds__(256) void k_inverse_rules(InverseList l) {
       continue;
     int *const at = inverse + (long long)r * fs + f;
     const int was = *at;
-    if (was < rows) { // (the background rows' are named already)
+    if (was >= -1 && was < rows) {
       *at = (int)o;
-    } else {
+    } else { // (a background row's; those that find it unnamed all store the same)
       mask |= 1u << f;
-      sample = (was - rows) / fs;
+      sample = (was < 0 ? -2 - was : was - rows) / fs;
+      if (was < 0)
+        *at = rows - 2 - was;
     }
   }
   if (!l.background[t])
@@ -592,6 +596,27 @@ extern "C" int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *i
   return SCN_OK;
 }
 
+// Where the planes do not take the product (few shapes: rows in other than 32s): the
+// elements that are not finite again, without the positions that no row names.  A
+// sum of fs N products each, one after the other.
+__global__ __launch_bounds__(256) void k_input_gradient_again(const float *__restrict__ delta,
+                                                              const int *__restrict__ inverse, int fs, int N,
+                                                              const float *__restrict__ Wt, float *__restrict__ din,
+                                                              long long count, int nIn) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < count; i += (long long)gridDim.x * 256) {
+    if (fabsf(din[i]) <= 3.4028235e38f)
+      continue;
+    const long long r = i / nIn;
+    const int c = (int)(i - r * nIn);
+    float sum = 0.f;
+    for (int f = 0; f < fs; ++f) {
+      const int o = inverse[r * fs + f];
+      for (int n = 0; n < (o < 0 ? 0 : N); ++n)
+        sum = fmaf(delta[(long long)o * N + n], Wt[((long long)f * N + n) * nIn + c], sum);
+    }
+    din[i] = sum;
+  }
+}
 extern "C" int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
                                        const float *d_Wt, const void *d_image, float *d_din, int64_t inputRows,
                                        int nIn) {
@@ -602,8 +627,15 @@ extern "C" int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const
     return SCN_OK;
   OwnRows ownRows(ctx);
   SCN_REQUIRE(d_inverse, SCN_ERR_ARG, "scn_conv_input_gradient: null rules");
-  return scn_conv_nin_forward_image(ctx, d_delta, d_inverse, fs, N, d_Wt, d_image, ctx->d_zeros, nullptr, d_din,
-                                    inputRows, nIn, 1.f, SCN_NOSIGMOID, SCN_FP32_PLANES);
+  SCN_TRY(scn_conv_named(ctx, d_delta, d_inverse, fs, N, d_Wt, d_image, d_din, inputRows, nIn));
+  if (!scn_conv_takes_planes(d_delta, d_Wt, d_din, fs * N, nIn)) {
+    ProfScope prof(ctx, SCN_K_BACKWARD);
+    const long long count = (long long)inputRows * nIn, most = 16ll * ctx->numCU, blocks = (count + 255) / 256;
+    hipLaunchKernelGGL(k_input_gradient_again, dim3((unsigned)(blocks < most ? blocks : most)), dim3(256), 0,
+                       ctx->stream, d_delta, d_inverse, fs, N, d_Wt, d_din, count, nIn);
+    SCN_HIP_CHECK(hipGetLastError());
+  }
+  return SCN_OK;
 }
 
 // ------------------------------------------------------------ dA = D W^T

@@ -224,3 +224,123 @@ def test_epochs_against_the_oracle(scn, what, batch, epochs):
             if a is not None:
                 assert np.allclose(a, b, rtol=1e-4 * epochs * 3, atol=3e-6 * epochs)
     net.close()
+
+
+def products(a, b):
+    """a @ b by columns of a: infinities and NaN as plain sums of products give them, whatever the library does"""
+    with np.errstate(invalid="ignore", over="ignore"):
+        out = np.zeros((a.shape[0], b.shape[1]))
+        for k in range(a.shape[1]):
+            out += a[:, k:k + 1] * b[k]
+    return out
+
+
+# split contraction, tiles of whole lines, tiles of k_nin_planes (channels in fours of a position; few rows to a
+# workgroup); few rows, tiles and resident weights on the fp32 MFMA
+@pytest.mark.parametrize("d,field,window,batch,density,nIn,N", [
+    (2, 7, 2, 4, 0.3, 32, 32), (3, 6, 3, 3, 0.1, 32, 64), (2, 110, 2, 12, 0.15, 32, 64), (2, 120, 2, 24, 0.2, 64, 32),
+    (2, 110, 2, 12, 0.15, 64, 24), (2, 9, 2, 3, 0.3, 20, 36), (2, 60, 3, 6, 0.2, 32, 36), (2, 70, 2, 9, 0.2, 64, 36)])
+def test_infinite_weights_reach_the_rows_that_are_named(scn, ctx, d, field, window, batch, density, nIn, N):
+    """as a product per output row, added through the rules, has it: a filter position that no output row names an input
+    row at adds nothing to it, not 0 times its weights"""
+    rng = np.random.default_rng(field + N)
+    g, n, rows, fs, d_rules, bg = layer(scn, ctx, d, field, window, batch, density, field + nIn)
+    print("infinite weights", d, field, window, nIn, N, "rows", rows, "of", n, flush=True)
+    # (a sum of 250000 rows of D is below 1: what is finite in 64 bits, 3.4e38 times it included, is so in 32)
+    rules, D = d_rules.download(), (1e-4 * rng.standard_normal((rows, N))).astype(np.float32)
+    W = rng.standard_normal((fs, nIn, N)).astype(np.float32)
+    for value in (np.inf, -np.inf, np.nan, 3.4e38):
+        W[rng.integers(0, fs), rng.integers(0, nIn), rng.integers(0, N)] = value
+    D[rows // 2, 3], D[rows // 3, 1] = np.inf, np.nan
+    pitch = scn.lib().scn_positions_pitch(rows)
+    inverse, background = ctx.empty((n, fs), np.int32), ctx.empty(rows + 2 * batch, np.int32)
+    positions = ctx.empty((fs, pitch), np.int32)
+    ctx.rules_inverse_many([(g, d_rules, inverse, background, positions, rows, n, fs)])
+    Wt, delta = ctx.empty(W.size, np.float32), ctx.array(np.concatenate([D, np.zeros((batch * fs, N), np.float32)]))
+    ctx.transpose_filters_many([(ctx.array(W.reshape(fs * nIn, N)), Wt, fs, nIn, N)])
+    ctx.background_sums(delta, rows, N, background, fs, batch)
+    want, size = np.zeros((n, nIn)), np.zeros((n, nIn))
+    isBg = np.isin(rules, [b for b in bg if b >= 0])
+    with np.errstate(invalid="ignore", over="ignore"):
+        for f in range(fs):
+            Wf = W[f].T.astype(np.float64)
+            own = np.nonzero((rules[:, f] >= 0) & ~isBg[:, f])[0]
+            want[rules[own, f]] += products(D[own].astype(np.float64), Wf)
+            size[rules[own, f]] += products(np.abs(D[own]).astype(np.float64), np.abs(Wf))
+            for b in bg:
+                mine = np.nonzero(rules[:, f] == b)[0] if b >= 0 else []
+                if len(mine):
+                    want[b] += products(D[mine].astype(np.float64).sum(0, keepdims=True), Wf)[0]
+                    size[b] += products(np.abs(D[mine]).astype(np.float64).sum(0, keepdims=True), np.abs(Wf))[0]
+    outs = [ctx.array(np.full((n, nIn), 7, np.float32)) for _ in range(2)]
+    ctx.conv_input_gradient(delta, inverse, fs, N, Wt, outs[0], n, nIn)
+    if N % 32 == 0:  # (the weights laid out, as epochs have them: the same bits)
+        image = ctx.empty((nIn + 31) // 32 * 32 * fs * N * 6 // 4, np.float32)
+        ctx.weight_images_many([(ctx.array(W.reshape(fs * nIn, N)), image, fs * N, nIn, fs, scn.FP32_PLANES)])
+        ctx.conv_input_gradient(delta, inverse, fs, N, Wt, outs[1], n, nIn, d_image=image)
+        assert np.array_equal(outs[1].download(), outs[0].download(), equal_nan=True)
+    got, sure = outs[0].download(), np.isfinite(want)
+    assert sure.mean() > 0.5 and not sure.all() and size[sure].max() < 3.4e38
+    assert np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True)
+    assert np.all(np.abs(got[sure] - want[sure]) <= 4e-6 * size[sure])
+
+
+@pytest.mark.parametrize("M,fs,nIn,N", [(391, 3, 36, 44), (2051, 4, 32, 64), (391, 4, 7, 33), (9001, 4, 96, 160)])
+def test_infinite_operands_of_the_weight_gradient(scn, ctx, M, fs, nIn, N):
+    """through the rules (rows by lines, and not): what the gathered matrix's product has, zero rows included"""
+    rng = np.random.default_rng(M + nIn)
+    # (the sum of a column of D is below 1 in magnitude: what is finite in 64 bits is so in 32)
+    x, D = rng.standard_normal((300, nIn)).astype(np.float32), (0.1 / M * rng.standard_normal((M, N))).astype(np.float32)
+    x[3, 5], x[77, 2], x[5, 1], x[8, 0], D[M // 2, 11], D[M // 3, 2] = np.inf, -np.inf, np.nan, 3.4e38, np.inf, np.nan
+    rules = rng.integers(-1, 300, (M, fs)).astype(np.int32)
+    pitch = scn.lib().scn_positions_pitch(M)
+    positions = ctx.array(np.ascontiguousarray(np.pad(rules.T, ((0, 0), (0, pitch - M)), constant_values=-1)))
+    print("infinite operands of dW", M, fs, nIn, N, flush=True)
+    dense = np.where(rules[:, :, None] >= 0, x[np.maximum(rules, 0)], 0).reshape(M, fs * nIn).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = np.einsum("mk,mn->kn", dense, D.astype(np.float64))
+        size, sums = np.einsum("mk,mn->kn", np.abs(dense), np.abs(D).astype(np.float64)), D.astype(np.float64).sum(0)
+    dW, db = ctx.array(np.full((fs * nIn, N), 7, np.float32)), ctx.array(np.full(N, 7, np.float32))
+    ctx.conv_AtB(ctx.array(x), positions, fs, nIn, ctx.array(D), dW, M, N, d_db=db)
+    got, sure = dW.download(), np.isfinite(want)
+    assert np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True)
+    assert np.all(np.abs(got[sure] - want[sure]) <= 2e-6 * size[sure])
+    got, sure = db.download(), np.isfinite(sums)
+    assert np.array_equal(got[~sure], sums[~sure].astype(np.float32), equal_nan=True)
+    assert np.all(np.abs(got[sure] - sums[sure]) <= 2e-6 * np.abs(D).sum(0)[sure])
+
+
+def test_an_epoch_with_an_infinite_weight(scn):
+    """of a channel that is never above zero, so that the net's outputs are finite: an epoch leaves what single batches,
+    which gather, leave"""
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    cfg = synthetic.config(2, batch=8)
+    samples = synthetic.make_samples(cfg, 43)
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TRAINBATCH)
+    for pts, f, label in samples:
+        ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
+    left = []
+    for epoch in (True, False):
+        net, _ = pair(cfg, hostapi, 52)
+        nin = [i for i, l in enumerate(net.layers()) if l["kind"].startswith("nin")]
+        W, B, _ = net.get_weights(nin[0])
+        B[5] = -1e6
+        net.set_weights(nin[0], W, B)
+        W, B, _ = net.get_weights(nin[1])
+        W[32 + 5, 2] = np.inf  # (its second position)
+        net.set_weights(nin[1], W, B)
+        net.set_training(0.01, 0.9, shuffle=False)
+        if epoch:
+            net.processDatasetTrain(ds, 4, 0.01, 0.9)
+        else:
+            net.begin(ds, 4)
+            while net.next_batch():
+                pass
+        left.append([a for i in nin for m in (True, False) for a in net.get_weights(i, momentum=m) if a is not None])
+        net.close()
+    for k, (a, b) in enumerate(zip(*left)):
+        sure = np.isfinite(b)
+        print("tensor", k, "not finite", int((~sure).sum()), "of", b.size, flush=True)
+        assert np.array_equal(a[~sure], b[~sure], equal_nan=True)
+        # (the bar of the oracle's epochs: a batch's share of rectifiers that a rounding turns)
+        assert rel_l2(a[sure], b[sure]) <= 3e-4
