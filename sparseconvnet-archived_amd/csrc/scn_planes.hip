@@ -191,6 +191,12 @@ __device__ __forceinline__ void barrier_lds() {
 __device__ __forceinline__ void dma_kilobyte(unsigned lds, const unsigned char *from) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(from) : "memory", "m0");
 }
+// ... and 256 bytes, a word a lane.  (What is asked for behind the compiler's back
+// goes to LDS and never to a register of its: one promised by an asm before the data
+// is there may be copied or spilled on the way, with what it held before.)
+__device__ __forceinline__ void dma_words(unsigned lds, const int *from) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(from) : "memory", "m0");
+}
 
 // A workgroup of WAVES wavefronts owns 32 WAVES MT rows x 32 NT columns, a
 // wavefront 32 MT rows of them, and walks k in blocks of 32, two MFMA steps.
@@ -1842,21 +1848,24 @@ __global__ void __launch_bounds__(512, 2)
     const int f4 = GATHER ? ca / gs.nIn : 0, ch4 = GATHER ? ca - f4 * gs.nIn : 0;
     const int steps = (int)((m1 - m0 - ATB_STEP * wave0 + ATB_STEP * GM - 1) / (ATB_STEP * GM));
     auto place = [&](int t) { return m0 + ATB_STEP * (wave0 + (long long)GM * (t < steps ? t : steps - 1)); };
+    // Rules: a word a lane for each request of rows, behind the rings of all wavefronts
     struct Rules {
       int r[GATHER ? AU : 1];
     };
-    auto ask = [&](Rules &x, int t) { // (the positions' pitch: whole steps)
+    int *const sRule = reinterpret_cast<int *>(reinterpret_cast<unsigned char *>(sTile) + GM * RING * SLOT) + wave0 * AU * 64;
+    auto ask = [&](int t, int *to) { // (the positions' pitch: whole steps)
+      const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int *)to;
 #pragma unroll
       for (int u = 0; u < (GATHER ? AU : 0); ++u)
-        asm volatile("global_load_dword %0, %1, off"
-                     : "=v"(x.r[u % (GATHER ? AU : 1)])
-                     : "v"(gs.rules + f4 * pitch + place(t) + 8 / MT * u + ra)
-                     : "memory");
+        dma_words(lds + u * 256, gs.rules + f4 * pitch + place(t) + 8 / MT * u + ra);
     };
-    auto settle = [&](Rules &x) { // (asked for by then: their registers hold them from here on)
+    auto look = [&](Rules &x, const int *from) { // (read before the next ones take their place)
 #pragma unroll
       for (int u = 0; u < (GATHER ? AU : 0); ++u)
-        asm volatile("" : "+v"(x.r[u % (GATHER ? AU : 1)]));
+        x.r[u % (GATHER ? AU : 1)] = from[u * 64 + lane];
+#pragma unroll
+      for (int u = 0; u < (GATHER ? AU : 0); ++u)
+        asm volatile("" : "+v"(x.r[u % (GATHER ? AU : 1)]) : : "memory");
     };
     const float *const none = GATHER ? gs.zeros : zeros;
     auto fetch = [&](const Rules &x, int t, int slot) {
@@ -1900,39 +1909,34 @@ __global__ void __launch_bounds__(512, 2)
       // Rules are asked for a step before their rows, in front of the rows asked for
       // then: what has landed when all but the last step's rows have holds a step's
       // rows and the next request's rules.
-      Rules x, y;
+      static_assert(!GATHER || RING == 3, "the first two steps' rules come together");
+      Rules x;
       {
-        Rules first, second;
-        ask(first, 0);
-        ask(second, 1);
-        ask(x, RING - 1);
+        Rules second;
+        int *const spare = reinterpret_cast<int *>(ring + (RING - 1) * SLOT); // (nothing is asked for there yet)
+        ask(0, spare);
+        ask(1, spare + AU * 64);
+        ask(RING - 1, sRule);
         w_landed<0>();
-        settle(first);
-        settle(second);
-        fetch(first, 0, 0);
+        look(x, spare);
+        look(second, spare + AU * 64);
+        fetch(x, 0, 0);
         if (RING == 3)
           fetch(second, 1, 1);
       }
       int slot = 0, into = RING - 1;
-      auto step = [&](int t, Rules &have, Rules &next) {
+#pragma unroll 1
+      for (int t = 0; t < steps; ++t) {
         w_landed<RING == 3 ? FETCH : 0>(); // (and this wavefront's reads of the slot that is asked for again)
-        settle(have);
-        ask(next, t + RING);
-        fetch(have, t + RING - 1, into);
+        look(x, sRule);
+        ask(t + RING, sRule);
+        fetch(x, t + RING - 1, into);
         Step s;
         take(s, slot);
         compute(s);
         slot = slot == RING - 1 ? 0 : slot + 1, into = into == RING - 1 ? 0 : into + 1;
-      };
-#pragma unroll 1
-      for (int t = 0; t < steps; t += 2) {
-        step(t, x, y);
-        if (t + 1 < steps)
-          step(t + 1, y, x);
       }
       w_landed<0>();
-      settle(x); // (rules that nobody needs have their registers until they have come)
-      settle(y);
     }
     __syncthreads(); // (the sums take the rings' place)
   } else {
@@ -2074,7 +2078,8 @@ template <int MT, int NT, bool GATHER, bool LINES>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                       long long M, int K, int N, long long splits, const GatherSource &gs) {
   const size_t sums = ((size_t)8 * 32 * MT * 32 * NT + 8 * 32 * NT + 1) * sizeof(float);
-  const size_t rings = (size_t)8 * atb_ring(MT, NT) * 2048 * (MT + NT), lds = LINES && rings > sums ? rings : sums;
+  const size_t rings = (size_t)8 * (atb_ring(MT, NT) * 2048 * (MT + NT) + (GATHER ? 2 * MT * 256 : 0));
+  const size_t lds = LINES && rings > sums ? rings : sums;
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER, LINES>),
