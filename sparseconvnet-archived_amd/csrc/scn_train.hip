@@ -323,13 +323,13 @@ struct InverseList {
 // a workgroup an item
 __global__ __launch_bounds__(256) void k_inverse_background(InverseList l) {
   const int t = blockIdx.x, fs = l.fs[t];
-  if (!l.inverse[t])
-    return;
   if (l.background[t])
     for (int s = threadIdx.x; s < l.batch[t]; s += 256) {
       l.background[t][l.rows[t] + 2 * s] = 0x7fffffff;
       l.background[t][l.rows[t] + 2 * s + 1] = -1;
     }
+  if (!l.inverse[t]) // (not wanted, or an input without rows)
+    return;
   // (-2 - x: a background row's, until a row that names it is met)
   for (int x = threadIdx.x; x < l.batch[t] * fs; x += 256) {
     const int r = l.bg[t][x / fs];
@@ -398,6 +398,7 @@ extern "C" int scn_rules_inverse_many(scn_ctx *ctx, const scn_inverse_item *item
   size_t words[SCN_INVERSE_MAX];
   long long blocks = 0; // (16 items of no more than 2^23 workgroups)
   int fills = 0;
+  bool ends = false;
   l.count = 0;
   for (int k = 0; k < nItems; ++k) {
     const scn_inverse_item &it = items[k];
@@ -422,6 +423,7 @@ extern "C" int scn_rules_inverse_many(scn_ctx *ctx, const scn_inverse_item *item
     l.batch[c] = it.input->batch;
     l.firstBlock[c] = (unsigned)blocks;
     blocks += scn_ceil_div(scn_positions_pitch(it.rows), 256);
+    ends |= it.d_background != nullptr;
     if (l.inverse[c]) {
       fill[fills] = it.d_inverse;
       words[fills++] = (size_t)it.inputRows * it.fs;
@@ -431,10 +433,10 @@ extern "C" int scn_rules_inverse_many(scn_ctx *ctx, const scn_inverse_item *item
     return SCN_OK;
   l.firstBlock[l.count] = (unsigned)blocks;
   ProfScope prof(ctx, SCN_K_RULES);
-  if (fills) {
+  if (fills)
     SCN_TRY(scn_fill32_many(ctx, fill, words, fills, 0xffffffffu));
+  if (fills || ends)
     hipLaunchKernelGGL(k_inverse_background, dim3(l.count), dim3(256), 0, ctx->stream, l);
-  }
   if (blocks)
     hipLaunchKernelGGL(k_inverse_rules, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, l);
   SCN_HIP_CHECK(hipGetLastError());

@@ -154,6 +154,28 @@ def test_many_layers_in_one_call(scn, ctx):
         assert np.array_equal(a.download(), b.download())
 
 
+def test_an_input_without_rows(scn, ctx):
+    """rows that name nothing: every sample's first and last row with a background are "none", alone and beside a layer
+    that has an inverse; its sums add nothing"""
+    g, n, rows, fs, rules, _ = layer(scn, ctx, 2, 8, 2, 3, 0.3, 1)
+    batch, N = 3, 8
+    none = ctx.array(np.full((rows, fs), -1, np.int32))
+    inverse = ctx.array(np.full((n, fs), 7, np.int32))
+    for beside in (False, True):
+        background, other = (ctx.array(np.full(rows + 2 * batch, 7, np.int32)) for _ in range(2))
+        items = [(g, none, inverse, background, None, rows, 0, fs)]
+        ctx.rules_inverse_many(items + [(g, rules, inverse, other, None, rows, n, fs)] * beside)
+        got = background.download()
+        assert np.all(got[:rows] == 0)
+        # (only then may they be taken for rows: a kernel walks from the first to the last)
+        assert np.array_equal(got[rows:], np.tile(np.array([2 ** 31 - 1, -1], np.int32), batch))
+        delta = np.zeros((rows + batch * fs, N), np.float32)
+        delta[:rows] = 1
+        d_delta = ctx.array(delta)
+        ctx.background_sums(d_delta, rows, N, background, fs, batch)
+        assert np.array_equal(d_delta.download(), delta)
+
+
 def test_refusals(scn, ctx):
     g, n, rows, fs, rules, _ = layer(scn, ctx, 2, 8, 2, 2, 0.3, 1)
     buf = ctx.empty((64, 64), np.float32)
