@@ -54,9 +54,10 @@ public:
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().
   std::vector<SparseGrid> grids;
-  // the last batch's, empty, for the next one's to be built in: ten producers that
-  // allocate and free a hundred grids each hold one another up (a batch's half on
-  // the CPU 0.6 to 1.7 ms, and 0.45 to 0.65 for most of them without)
+  // A picture batch's input: the last batch's grids, empty, for the next one's to be
+  // built in (keepGrids, by the producer that fills them; no more than a batch has).
+  // Ten producers that allocate and free a hundred grids each hold one another up (a
+  // batch's half on the CPU 0.6 to 1.7 ms, and 0.45 to 0.65 for most of them without).
   std::vector<SparseGrid> spareGrids;
   scn_grids *deviceGrids;
   bool ownsDeviceGrids;
@@ -72,6 +73,7 @@ public:
   SpatiallySparseBatchInterface(SpatiallySparseBatchInterface &&o);
   ~SpatiallySparseBatchInterface();
   void downloadGrids(int batchSize);
+  void keepGrids(size_t most); // grids become spare ones
   void summary();
   void reset();
 };

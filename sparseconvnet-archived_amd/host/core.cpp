@@ -345,11 +345,6 @@ SpatiallySparseBatchInterface::~SpatiallySparseBatchInterface() {
 void SpatiallySparseBatchInterface::reset() {
   featuresPresent.resize(0);
   nSpatialSites = 0;
-  for (auto &g : grids) {
-    g.backgroundCol = -1;
-    g.mp.clear();
-    spareGrids.push_back(std::move(g));
-  }
   grids.resize(0);
   rules.resize(0);
   backpropErrors = false;
@@ -360,6 +355,18 @@ void SpatiallySparseBatchInterface::reset() {
   positions.resize(0);
   deferredGatherFrom = nullptr;
   // deviceGrids keeps its tables for the next batch
+}
+void SpatiallySparseBatchInterface::keepGrids(size_t most) {
+  for (auto &g : grids) {
+    if (spareGrids.size() >= most)
+      break;
+    g.backgroundCol = -1;
+    g.mp.clear();
+    spareGrids.push_back(std::move(g));
+  }
+  grids.resize(0);
+  if (spareGrids.size() > most)
+    spareGrids.resize(most);
 }
 // Rebuilds the host SparseGrid view from the tables in HBM.
 void SpatiallySparseBatchInterface::downloadGrids(int batchSize) {

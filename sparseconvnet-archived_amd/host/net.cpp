@@ -937,10 +937,11 @@ BatchProducer::~BatchProducer() {
 // CPU half of BatchProducer.cu:40-87: distort, codify, normalise
 void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
   SpatiallySparseBatch &b = cnn.batchPool[cc];
+  SpatiallySparseBatchInterface &in = b.interfaces[0];
+  in.keepGrids(batchSize);
   b.reset();
   b.type = dataset.type;
   b.unseen = unseen;
-  SpatiallySparseBatchInterface &in = b.interfaces[0];
   in.nFeatures = dataset.nFeatures;
   in.spatialSize = spatialSize;
   in.featuresPresent.hVector() = range(dataset.nFeatures);
