@@ -111,7 +111,10 @@ extern "C" int scn_malloc(scn_ctx *c, size_t bytes, void **d_ptr) {
   *d_ptr = nullptr;
   if (bytes == 0)
     bytes = 16;
-  SCN_HIP_CHECK(hipMalloc(d_ptr, bytes));
+  const hipError_t e = hipMalloc(d_ptr, bytes);
+  if (e != hipSuccess)
+    (void)hipGetLastError(); // (the caller's to deal with, and not the next launch's)
+  SCN_HIP_CHECK(e);
   return SCN_OK;
 }
 

@@ -18,8 +18,9 @@ public:
   vectorCUDA<float> features16;
   // the weights of the layer whose output this is, laid out for its forward pass
   // and, turned round, for the gradient of its input: made for one batch by
-  // SparseConvNetCUDA::makeWeightImages and used up by the layer (empty: none)
-  vectorCUDA<float> weightImage, turnedImage;
+  // SparseConvNetCUDA::makeWeightImages, in the stream's room for them, and used up
+  // by the layer (null: none)
+  void *weightImage = nullptr, *turnedImage = nullptr;
   SpatiallySparseBatchSubInterface();
   void reset();
 };

@@ -16,6 +16,14 @@
 #include "SpatiallySparseBatch.h"
 #include "SpatiallySparseBatchInterface.h"
 
+// A layer's weights laid out for one pass: what to make, the room it takes, and
+// where the layer looks for it
+struct WeightImage {
+  scn_image_item item;
+  int64_t bytes;
+  void **image;
+};
+
 class SpatiallySparseLayer {
 public:
   cudaMemStream &memStream;
@@ -58,7 +66,7 @@ public:
                             SpatiallySparseBatchInterface &input,
                             SpatiallySparseBatchInterface &output,
                             const SpatiallySparseBatchInterface *before,
-                            std::vector<scn_image_item> &items) {
+                            std::vector<WeightImage> &items) {
     (void)batch, (void)input, (void)output, (void)before, (void)items;
   }
   // convolutions: the layer behind will gather (deferGather, or a batch without the matrix)
@@ -189,7 +197,7 @@ public:
                     SpatiallySparseBatchInterface &input,
                     SpatiallySparseBatchInterface &output,
                     const SpatiallySparseBatchInterface *before,
-                    std::vector<scn_image_item> &items);
+                    std::vector<WeightImage> &items);
   void transposedFilters(SpatiallySparseBatchInterface &input,
                          std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);
@@ -241,7 +249,7 @@ public:
                     SpatiallySparseBatchInterface &input,
                     SpatiallySparseBatchInterface &output,
                     const SpatiallySparseBatchInterface *before,
-                    std::vector<scn_image_item> &items);
+                    std::vector<WeightImage> &items);
   void transposedFilters(SpatiallySparseBatchInterface &input,
                          std::vector<scn_filter_item> &items);
   int calculateInputSpatialSize(int outputSpatialSize);

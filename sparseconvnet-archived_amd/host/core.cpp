@@ -158,9 +158,22 @@ cudaMemStream::cudaMemStream(bool layers) : ctx(nullptr) {
   SCN_CHECKED(layers ? scn_ctx_create(-1, &ctx) : scn_ctx_create_for_plans(-1, &ctx));
   g_liveCtx.push_back(ctx);
   g_defaultCtx = g_liveCtx.front();
+  if (layers && scn_malloc(ctx, ROOM, &images) == SCN_OK)
+    imageBytes = ROOM;
+}
+void *cudaMemStream::imageRoom(size_t bytes) {
+  if (bytes > imageBytes) {
+    SCN_CHECKED(scn_free(nullptr, images)); // (waits for what reads it)
+    images = nullptr;
+    imageBytes = 0;
+    SCN_CHECKED(scn_malloc(ctx, bytes + bytes / 4, &images));
+    imageBytes = bytes + bytes / 4;
+  }
+  return images;
 }
 cudaMemStream::~cudaMemStream() {
   std::lock_guard<std::mutex> lock(g_ctxMutex);
+  scn_free(nullptr, images);
   g_liveCtx.erase(std::find(g_liveCtx.begin(), g_liveCtx.end(), ctx));
   g_defaultCtx = g_liveCtx.empty() ? nullptr : g_liveCtx.front();
   scn_ctx_destroy(ctx);

@@ -331,29 +331,25 @@ static bool rounds_rows(int precision, int fs, int nIn, int rows) {
   return precision == SCN_BF16 && fs >= 8 && nIn % 8 == 0 && (int64_t)rows * fs >= (int64_t)1 << 20;
 }
 // The layout of the weights that was made for this pass, or null: used once
-static const void *take_image(vectorCUDA<float> &image) {
-  const void *const p = image.size64() ? image.dPtr() : nullptr;
-  image.resize64(0);
+static const void *take_image(void *&image) {
+  const void *const p = image;
+  image = nullptr;
   return p;
 }
 static void nin_weight_images(SpatiallySparseBatch &batch, cudaMemStream &ms, SpatiallySparseBatchInterface &input,
                               SpatiallySparseBatchInterface &output, const SpatiallySparseBatchInterface *before,
-                              vectorCUDA<float> &W, int K, int N, int precision, std::vector<scn_image_item> &items) {
+                              vectorCUDA<float> &W, int K, int N, int precision, std::vector<WeightImage> &items) {
   const int nIn = before ? before->nFeatures : K, fs = K / nIn, p = abi_precision(precision);
   const int64_t bytes = before && rounds_rows(precision, fs, nIn, output.nSpatialSites)
                             ? 0
                             : scn_weight_image_bytes(ms.ctx, output.nSpatialSites, K, N, nIn, p);
-  if (bytes) {
-    output.sub->weightImage.resize64((size_t)bytes / 4);
-    items.push_back({W.dPtr(), output.sub->weightImage.dPtr(), K, N, 0, p});
-  }
+  if (bytes)
+    items.push_back({{W.dPtr(), nullptr, K, N, 0, p}, bytes, &output.sub->weightImage});
   if (batch.type != TRAINBATCH || !input.leftOut || !before || !before->backpropErrors)
     return;
   const int64_t turned = scn_weight_image_bytes(ms.ctx, before->nSpatialSites, fs * N, nIn, N, SCN_FP32_PLANES);
-  if (turned) {
-    output.sub->turnedImage.resize64((size_t)turned / 4);
-    items.push_back({W.dPtr(), output.sub->turnedImage.dPtr(), fs * N, nIn, fs, SCN_FP32_PLANES});
-  }
+  if (turned)
+    items.push_back({{W.dPtr(), nullptr, fs * N, nIn, fs, SCN_FP32_PLANES}, turned, &output.sub->turnedImage});
 }
 // When the preceding convolutional layer deferred its gather: run the fused
 // kernel (fp32 operands), or gather now if this layer wants bf16 operands.
@@ -621,7 +617,7 @@ void NetworkInNetworkLayer::activationAhead(
 void NetworkInNetworkLayer::weightImages(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
                                          SpatiallySparseBatchInterface &output,
                                          const SpatiallySparseBatchInterface *before,
-                                         std::vector<scn_image_item> &items) {
+                                         std::vector<WeightImage> &items) {
   if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
     nin_weight_images(batch, fwd_stream(batch, memStream), input, output, before, W, nFeaturesIn, nFeaturesOut, precision,
                       items);
@@ -629,7 +625,7 @@ void NetworkInNetworkLayer::weightImages(SpatiallySparseBatch &batch, SpatiallyS
 void NetworkInNetworkPReLULayer::weightImages(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
                                               SpatiallySparseBatchInterface &output,
                                               const SpatiallySparseBatchInterface *before,
-                                              std::vector<scn_image_item> &items) {
+                                              std::vector<WeightImage> &items) {
   if (!nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
     nin_weight_images(batch, fwd_stream(batch, memStream), input, output, before, W, nFeaturesIn, nFeaturesOut, precision,
                       items);

@@ -488,7 +488,7 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   }
   batch.collectUpdates = false;
   for (size_t i = 1; i < batch.interfaces.size(); i++)
-    batch.interfaces[i].sub->turnedImage.resize64(0);
+    batch.interfaces[i].sub->turnedImage = nullptr;
   for (size_t i = 0; i < batch.updates.size(); i += SCN_NAG_MAX)
     SCN_CHECKED(scn_nag_update_many(
         memStream.ctx, batch.updates.data() + i,
@@ -503,23 +503,34 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   r.consumedPending = true;
 }
 // The weights as the contractions of this pass read them, all layers' in one
-// launch (by themselves 3 to 5 us a layer).  Made for every batch: nothing is
-// kept that a change of the weights could leave behind.
+// launch (by themselves 3 to 5 us a layer), side by side in the stream's room: one
+// pass at a time reads them.  Made for every batch: nothing is kept that a change
+// of the weights could leave behind.
 void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStream &ms) {
-  std::vector<scn_image_item> items;
+  std::vector<WeightImage> images;
   for (size_t i = 0; i < layers.size(); i++) {
     SpatiallySparseBatchInterface &input = batch.interfaces[i], &output = batch.interfaces[i + 1];
-    output.sub->weightImage.resize64(0);
-    output.sub->turnedImage.resize64(0);
+    output.sub->weightImage = output.sub->turnedImage = nullptr;
     if (batch.type == RESCALEBATCH) // (whose weights change on the way)
       continue;
     if (batch.countsPending)
       SCN_CHECKED(scn_ctx_rows_from(ms.ctx, output.deviceGrids));
     const bool gathers = i > 0 && layers[i - 1]->defersGather(batch, input);
-    layers[i]->weightImages(batch, input, output, gathers ? &batch.interfaces[i - 1] : nullptr, items);
+    layers[i]->weightImages(batch, input, output, gathers ? &batch.interfaces[i - 1] : nullptr, images);
   }
   if (batch.countsPending)
     SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
+  size_t total = 0;
+  auto room = [](int64_t bytes) { return ((size_t)bytes + 255) & ~(size_t)255; };
+  for (auto &x : images)
+    total += room(x.bytes);
+  char *at = total ? (char *)ms.imageRoom(total) : nullptr;
+  std::vector<scn_image_item> items;
+  for (auto &x : images) {
+    x.item.d_image = *x.image = at;
+    items.push_back(x.item);
+    at += room(x.bytes);
+  }
   for (size_t i = 0; i < items.size(); i += SCN_IMAGES_MAX)
     SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, (int)std::min<size_t>(SCN_IMAGES_MAX, items.size() - i)));
 }
@@ -565,7 +576,7 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   if (batch.countsPending)
     SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
   for (size_t i = 1; i < batch.interfaces.size(); i++) // (what no layer has taken)
-    batch.interfaces[i].sub->weightImage.resize64(0);
+    batch.interfaces[i].sub->weightImage = nullptr;
   SoftmaxClassifierLaunch(batch.interfaces.back(), batch, ms);
 }
 void SparseConvNetCUDA::finishBatch(SpatiallySparseBatch &batch,

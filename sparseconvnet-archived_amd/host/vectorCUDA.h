@@ -22,6 +22,17 @@ public:
   cudaMemStream &operator=(const cudaMemStream &) = delete;
   void *stream() const;
   void synchronize() const;
+  // Room for the weights of a pass over a batch as its contractions read them, in
+  // the order of the stream: a layers' stream has ROOM of it from the start, which
+  // holds those of a net of some 5 M weights (and so the first batch does not wait
+  // for allocations: an allocation a layer was 0.1 ms of the first 1.6 of a net with
+  // up to 800 channels), and more as soon as it is asked for.
+  void *imageRoom(size_t bytes);
+
+private:
+  static constexpr size_t ROOM = (size_t)32 << 20;
+  void *images = nullptr;
+  size_t imageBytes = 0;
 };
 
 // the context vectorCUDA objects use when no stream is named: the one of the
