@@ -1249,9 +1249,11 @@ __global__ void __launch_bounds__(256) k_weight_images(ImageList l) {
     weight_image<1>(l.W[x], l.image[x], l.K[x], l.N[x], l.fs[x], item);
 }
 static int64_t image_bytes(int planes, int K, int N) { return (int64_t)scn_ceil_div(N, 32) * 32 * K * 2 * planes; }
-// What k_nin_lines takes: three planes or one, blocks within one filter position.
-static bool lines_shape(int planes, int K, int nIn) {
-  return planes != 2 && scn_planes_shape(K) && nIn % 32 == 0;
+// What k_nin_lines takes: three planes or one, blocks within one filter position, 64
+// rows of the output within the gigabyte that its stores reach (columns that there are
+// none of lie from 2 GB on, and have to stay there).
+static bool lines_shape(int planes, int K, int N, int nIn) {
+  return planes != 2 && scn_planes_shape(K) && nIn % 32 == 0 && N <= 1 << 22;
 }
 
 // False: convert on the way instead -- the stream is being captured (a graph may
@@ -1412,6 +1414,8 @@ static const PlanesCost planesCost[3][4][2] = {
 // 19.4, 17.6; 256 k 1.8 6.2, 7.7, and 2.4 8.5, 8.0; 2560 k 2.2 41.7, 45.9, and 3.1
 // 51.7, 46.5; one plane, 512 k 1.6 6.9, 7.2, and 2.0 9.3, 7.4; 256 k 1.8 5.4, 5.4.
 static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
+  if (N > 1 << 26) // (a lane's place in nine rows of W has 32 bits)
+    return 0;
   const float perCU = planes == 1 ? 2.f : fminf(1.f + K / 230.f, planes == 2 ? 3.1f : 2.6f);
   const long long rows = (long long)(perCU * ctx->numCU / scn_ceil_div(N, 32));
   return 32 * (rows < 1 ? 1 : rows);
@@ -1588,7 +1592,7 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
 // wherever it can run, as k_nin_planes' costs are too low for those.
 static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, const GatherSource *gs, const void *image,
                           bool room, PlanesChoice &choice) {
-  if (!lines_shape(planes, K, gs ? gs->nIn : K) ||
+  if (!lines_shape(planes, K, N, gs ? gs->nIn : K) ||
       !(image || (room && image_bytes(planes, K, N) <= (int64_t)SCN_IMAGE_BYTES)))
     return;
   int tile = 0;
@@ -1613,7 +1617,7 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
   // positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444 us against 474.
   // k_nin_planes' cost is 2 too high where it converts W on the way, of layers that
   // small.)
-  if (a16 && choice.tile >= 0 && K <= 1280 && N > 32 && lines_shape(1, K, gs->nIn) &&
+  if (a16 && choice.tile >= 0 && K <= 1280 && N > 32 && lines_shape(1, K, N, gs->nIn) &&
       (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES)) &&
       lines_rows16(ctx, rows, K, N, image != nullptr) < choice.cost - (choice.image ? 0.f : 2.f)) {
     choice.lines = N <= 64 ? 4 : 3;
@@ -1632,7 +1636,7 @@ static int image_planes(int precision) {
 }
 extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N, int nIn, int precision) {
   const int planes = image_planes(precision);
-  if (!ctx || M < 1 || K < 1 || N < 1 || nIn < 1 || planes == 0 || N % 4 != 0 || !lines_shape(planes, K, nIn))
+  if (!ctx || M < 1 || K < 1 || N < 1 || nIn < 1 || planes == 0 || N % 4 != 0 || !lines_shape(planes, K, N, nIn))
     return 0;
   const long long hint = scn_rows_hint(ctx, M), split = split_rows(ctx, planes, K, N);
   if (6 * hint <= 5 * split)

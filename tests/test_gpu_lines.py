@@ -103,6 +103,13 @@ def test_weights_laid_out_ahead(scn, ctx, rows, fs, nIn, N, precision):
     assert np.array_equal(plain.download(), want)
 
 
+def test_no_image_of_more_columns_than_the_stores_reach(scn, ctx):
+    """64 rows of the output in a gigabyte"""
+    for p in (scn.FP32_PLANES, scn.BF16):
+        assert scn.lib().scn_weight_image_bytes(ctx.h, 10000, 64, 1 << 22, 64, p) > 0
+        assert scn.lib().scn_weight_image_bytes(ctx.h, 10000, 64, (1 << 22) + 32, 64, p) == 0
+
+
 @pytest.mark.parametrize("M,N,K", [(4001, 64, 96), (33333, 128, 384), (9000, 96, 512)])
 def test_products_with_the_transpose(scn, ctx, M, N, K):
     rng = np.random.default_rng(M)
