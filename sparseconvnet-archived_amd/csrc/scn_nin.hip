@@ -2104,7 +2104,8 @@ extern "C" int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in,
   SCN_REQUIRE(((uintptr_t)d_image & 15) == 0, SCN_ERR_ARG, "scn_conv_nin_forward: the image starts on 16 bytes");
   if (d_rules)
     return conv_nin_forward(ctx, d_in, d_rules, fs, nIn, d_W, d_image, d_B, d_prelu, d_out, M, N, p, act, precision);
-  SCN_REQUIRE(fs >= 1 && nIn >= 1, SCN_ERR_ARG, "scn_conv_nin_forward: fs %d nIn %d", fs, nIn);
+  SCN_REQUIRE(fs >= 1 && nIn >= 1 && (int64_t)fs * nIn <= 0x7fffffff, SCN_ERR_ARG, "scn_conv_nin_forward: fs %d nIn %d", fs,
+              nIn);
   return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p, act, precision, nullptr, nullptr, d_image);
 }
 

@@ -103,6 +103,13 @@ def test_weights_laid_out_ahead(scn, ctx, rows, fs, nIn, N, precision):
     assert np.array_equal(plain.download(), want)
 
 
+def test_a_matrix_of_more_columns_than_there_are_numbers_is_refused(scn, ctx):
+    buf = ctx.empty((64, 64), np.float32)
+    for fs, nIn in ((1 << 16, (1 << 16) + 1), (1 << 30, 4), (0, 32), (4, 0)):
+        with pytest.raises(scn.ScnError):  # (without rows: nothing is launched either way)
+            ctx.conv_nin_forward_image(buf, None, fs, nIn, buf, None, buf, None, buf, 0, 64, 1.0, scn.RELU, scn.FP32_PLANES)
+
+
 def test_no_image_of_more_columns_than_the_stores_reach(scn, ctx):
     """64 rows of the output in a gigabyte"""
     for p in (scn.FP32_PLANES, scn.BF16):
