@@ -1,6 +1,8 @@
 """The backward pass of a convolution without its gathered matrix: dW through the rules, and the input's gradient as a
 convolution of the output's through the rules turned round, background rows included; then whole epochs, in which the
 host classes take that way, against the net-level oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -105,6 +107,28 @@ def test_gradients_through_rules(scn, ctx, d, field, window, batch, density, nIn
     assert np.all(np.abs(dx.download() - want) <= 4e-6 * size)
 
 
+@pytest.mark.parametrize("d,field,window,batch,density,nIn,N", [(2, 110, 2, 12, 0.15, 64, 64), (2, 110, 2, 12, 0.15, 96, 64)])
+def test_gradient_with_the_filters_laid_out(scn, ctx, d, field, window, batch, density, nIn, N):
+    """as epochs have it: through inverse rules, the rows of sums behind delta's own among them, the bits without"""
+    rng = np.random.default_rng(field)
+    g, n, rows, fs, d_rules, bg = layer(scn, ctx, d, field, window, batch, density, field + N)
+    print("turned image", d, field, window, nIn, N, "rows", rows, "of", n, flush=True)
+    d_W = ctx.array(rng.standard_normal((fs * nIn, N), dtype=np.float32))
+    delta = ctx.array(np.concatenate([rng.standard_normal((rows, N), dtype=np.float32), np.zeros((batch * fs, N), np.float32)]))
+    inverse, background, Wt = ctx.empty((n, fs), np.int32), ctx.empty(rows + 2 * batch, np.int32), ctx.empty(fs * nIn * N, np.float32)
+    ctx.rules_inverse_many([(g, d_rules, inverse, background, None, rows, n, fs)])
+    assert (inverse.download() >= rows).any()
+    ctx.background_sums(delta, rows, N, background, fs, batch)
+    ctx.transpose_filters_many([(d_W, Wt, fs, nIn, N)])
+    size = scn.lib().scn_weight_image_bytes(ctx.h, n, fs * N, nIn, N, scn.FP32_PLANES)
+    assert size > 0
+    image, outs = ctx.empty(size // 4, np.float32), [ctx.array(np.full((n, nIn), 7, np.float32)) for _ in range(2)]
+    ctx.weight_images_many([(d_W, image, fs * N, nIn, fs, scn.FP32_PLANES)])
+    for out, im in zip(outs, (None, image)):
+        ctx.conv_input_gradient(delta, inverse, fs, N, Wt, out, n, nIn, d_image=im)
+    assert np.array_equal(outs[0].download(), outs[1].download())
+
+
 # every tile that sums take; ragged rows and columns; added to and not
 @pytest.mark.parametrize("M,K,N", [(1, 32, 32), (130, 34, 31), (1000, 66, 100), (40001, 12, 32), (30011, 256, 96), (70003, 432, 128)])
 def test_weight_and_bias_gradients_in_one(scn, ctx, M, K, N):
@@ -196,10 +220,36 @@ STACKS = {
                    ("addTerminalPoolingLayer", 2), ("addSoftmaxLayer",)]),
     # convolutions one behind the other, without a pooling between them; the last one's output is one site a sample
     "unpooled": (False, [("addLeNetLayerMP", 32, 3, 1, 1, 1, 1), ("addLeNetLayerMP", 64, 2, 1, 1, 1, 6),
-                         ("addLeNetLayerMP", 32, 2, 1, 3, 2, 1), ("addLeNetLayerMP", 32, 2, 1, 1, 1, 1), ("addSoftmaxLayer",)])}
+                         ("addLeNetLayerMP", 32, 2, 1, 3, 2, 1), ("addLeNetLayerMP", 32, 2, 1, 1, 1, 1), ("addSoftmaxLayer",)]),
+    # rows enough for weights laid out ahead, forwards and turned round
+    "laid out": (False, [("addLeNetLayerMP", 64, 3, 1, 2, 2, 4), ("addLeNetLayerMP", 64, 2, 1, 2, 2, 4),
+                         ("addLeNetLayerMP", 64, 3, 1, 2, 2, 4), ("addLeNetLayerMP", 64, 2, 1, 1, 1, 4), ("addSoftmaxLayer",)])}
 
 
-@pytest.mark.parametrize("what,batch,epochs", [(2, 8, 2), (3, 5, 1), (4, 2, 1), ("tri", 4, 2), ("unpooled", 4, 2)])
+def laid_out(scn, net, cfg, hostapi, samples):
+    """of a batch's convolutions: are there layouts of the weights for one of them forwards, and turned round?"""
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TESTBATCH)
+    for pts, f, label in samples:
+        ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
+    net.begin(ds, len(samples))
+    assert net.next_batch()
+    info = [net.interface(i, want_features=False) for i in range(len(net.layers()) + 1)]
+    net.end()
+    size, layers = scn.lib().scn_weight_image_bytes, net.layers()
+    forwards = turned = 0
+    ctx = C.c_void_p(net.context_handle())
+    for i, l in enumerate(layers[1:], 1):
+        if l["kind"].startswith("nin") and layers[i - 1]["kind"] == "conv" and i > 1:
+            src, out, N = info[i - 1], info[i + 1], l["nOut"]
+            nIn, fs = src["nFeatures"], l["nIn"] // src["nFeatures"]
+            forwards = max(forwards, size(ctx, out["nSpatialSites"], l["nIn"], N, nIn, scn.FP32_PLANES))
+            turned = max(turned, size(ctx, src["nSpatialSites"], fs * N, nIn, N, scn.FP32_PLANES))
+            print("rows", out["nSpatialSites"], "of", src["nSpatialSites"], "layouts", forwards, turned, flush=True)
+    return forwards, turned
+
+
+@pytest.mark.parametrize("what,batch,epochs", [(2, 8, 2), (3, 5, 1), (4, 2, 1), ("tri", 4, 2), ("unpooled", 4, 2),
+                                               ("laid out", 100, 1)])
 def test_epochs_against_the_oracle(scn, what, batch, epochs):
     from sparseconvnet_archived_amd import hostapi, synthetic
     rng = np.random.default_rng(5)
@@ -209,7 +259,7 @@ def test_epochs_against_the_oracle(scn, what, batch, epochs):
         triangular = False
     else:
         triangular, stack = STACKS[what]
-        lattice = 12
+        lattice = 30 if what == "laid out" else 12
         cfg = synthetic.Config(what, 2, 3, 10, 2 * batch + 1, lattice, stack)
         cfg.number = 2
         samples = []
@@ -220,6 +270,8 @@ def test_epochs_against_the_oracle(scn, what, batch, epochs):
     pts, f, label = samples[1]
     samples[1] = (pts[:0], f[:0], label)  # a sample without a site
     net, ora = pair(cfg, hostapi, 51, triangular)
+    if what == "laid out":
+        assert all(laid_out(scn, net, cfg, hostapi, samples[:batch]))
     ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TRAINBATCH)
     for pts, f, label in samples:
         ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
