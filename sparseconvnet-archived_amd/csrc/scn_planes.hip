@@ -1700,9 +1700,8 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // eight wavefronts take sixteen rows each in turn and their sums meet in LDS.
 // The workgroups of one tile add to dW with float atomics, some 200 of which
 // retire in a nanosecond: few workgroups (one a compute unit), each with as many
-// rows as that leaves it.  29827 x 256 x 96 in 23 us (32 on the fp32 MFMA with
-// a thousand workgroups), 200000 x 1728 x 64 in 350 (470): A from HBM at 3.9
-// TB/s.
+// rows as that leaves it (29827 x 256 x 96 in 23 us, where the fp32 MFMA with a
+// thousand workgroups took 32; 200000 x 1728 x 64 in 350, 470).
 // GATHER: the rows of A through rules, which lie position by position, so that
 // a lane's eight are two loads (eight of them through row by row rules: 17.8 us
 // where this is 15.6 and a gathered matrix 14.5, and 8.2 to gather it).
@@ -1712,7 +1711,7 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // 512 bytes and every request occupies the path for 16 cycles or more, twice what the
 // splitting takes.  A backward layer with dW of 139000 x 384 x 128 384 -> 370 us;
 // dW of 28000 x 256 x 96 and its like 16.5 -> 15.6, of which some 5 are the start and
-// the atomics.
+// the atomics; 35461 x 256 x 96 20, 198759 x 1728 x 64 328 (A from HBM at 4.2 TB/s).
 constexpr int atb_ring(int MT, int NT) { return MT * NT >= 4 ? 2 : 3; }
 template <int MT, int NT, bool GATHER, bool LINES>
 __global__ void __launch_bounds__(512, 2)
@@ -1804,8 +1803,8 @@ __global__ void __launch_bounds__(512, 2)
         for (int v = 0; v < 16; ++v)
           acc[h][i][j][v] = 0.f;
   // the column sums of D, by the workgroups of the first tile of K
-  // (not by two by two tiles, whose registers are full)
-  const bool sums = MT * NT < 4 && db && k0 == 0;
+  // (not by two by two tiles without LINES, whose registers are full)
+  const bool sums = (LINES || MT * NT < 4) && db && k0 == 0;
   float ds[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -2115,9 +2114,13 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, f
 }
 
 // The tile and the number of row ranges that cost least: rounds of one workgroup
-// a compute unit, each `ti` microseconds for every 128 rows (two thirds of it
-// waiting for memory) and `f` to start, to sum and to store, and the atomics.
+// a compute unit, each `ti` microseconds for every 128 rows and `f` to start, to sum
+// and to store, and the atomics.  (Fitted where the rows were loaded into registers;
+// by lines it is 0.9 of `ti` for all of them, so that the choice is the same.)
 // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
+// Two by two tiles, us against two by one: 126507 x 1728 x 64 208, 255; 53325 x 640 x
+// 320 138, 177; 17223 x 1280 x 480 148, 174; 153345 x 384 x 128 106, 130; with the sums
+// of D the same.
 // (The search is 0.1 to 2 us of the host's time, a launch some 5.)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                    long long M, int K, int N, const GatherSource *gs) {
@@ -2128,7 +2131,10 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
   int best = 0;
   long long splits = 1;
   double least = 1e300;
-  for (int i = 0; i < (gs || db ? 3 : 4); ++i) { // (two by two tiles of gathered rows: 264 bytes a lane spilled)
+  // (requests of four columns, in one filter position each)
+  const bool lines = K % 4 == 0 && N % 4 == 0 && (!gs || gs->nIn % 4 == 0) && (((uintptr_t)A | (uintptr_t)D) & 15) == 0;
+  // (two by two tiles of gathered rows, and with sums but not by lines: 264 bytes a lane spilled)
+  for (int i = 0; i < (gs || (db && !lines) ? 3 : 4); ++i) {
     if ((tile[i].mt == 2 && ((gs ? gs->nIn : K) % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
       continue;
     const long long tiles = (long long)scn_ceil_div(K, 32 * tile[i].mt) * scn_ceil_div(N, 32 * tile[i].nt);
@@ -2147,8 +2153,6 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
     }
   }
   SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
-  // (requests of four columns, in one filter position each)
-  const bool lines = K % 4 == 0 && N % 4 == 0 && (!gs || gs->nIn % 4 == 0) && (((uintptr_t)A | (uintptr_t)D) & 15) == 0;
   switch (best) {
   case 1:
     return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);

@@ -130,7 +130,8 @@ def test_gradient_with_the_filters_laid_out(scn, ctx, d, field, window, batch, d
 
 
 # every tile that sums take; ragged rows and columns; added to and not
-@pytest.mark.parametrize("M,K,N", [(1, 32, 32), (130, 34, 31), (1000, 66, 100), (40001, 12, 32), (30011, 256, 96), (70003, 432, 128)])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 32), (130, 34, 31), (1000, 66, 100), (40001, 12, 32), (30011, 256, 96), (70003, 432, 128),
+                                   (53327, 644, 324)])
 def test_weight_and_bias_gradients_in_one(scn, ctx, M, K, N):
     rng = np.random.default_rng(M + K + N)
     A, D = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((M, N), dtype=np.float32)
