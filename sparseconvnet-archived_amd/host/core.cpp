@@ -153,21 +153,22 @@ scn_ctx *scnDefaultContext() {
   }
   return g_defaultCtx;
 }
-cudaMemStream::cudaMemStream(bool layers) : ctx(nullptr) {
+cudaMemStream::cudaMemStream(bool layers, size_t imageRoom) : ctx(nullptr) {
   std::lock_guard<std::mutex> lock(g_ctxMutex);
   SCN_CHECKED(layers ? scn_ctx_create(-1, &ctx) : scn_ctx_create_for_plans(-1, &ctx));
   g_liveCtx.push_back(ctx);
   g_defaultCtx = g_liveCtx.front();
-  if (layers && scn_malloc(ctx, ROOM, &images) == SCN_OK)
-    imageBytes = ROOM;
+  if (layers && imageRoom && scn_malloc(ctx, imageRoom, &images) == SCN_OK)
+    imageBytes = imageRoom;
 }
 void *cudaMemStream::imageRoom(size_t bytes) {
   if (bytes > imageBytes) {
     SCN_CHECKED(scn_free(nullptr, images)); // (waits for what reads it)
     images = nullptr;
     imageBytes = 0;
-    SCN_CHECKED(scn_malloc(ctx, bytes + bytes / 4, &images));
-    imageBytes = bytes + bytes / 4;
+    const size_t want = std::max(bytes + bytes / 4, ROOM);
+    SCN_CHECKED(scn_malloc(ctx, want, &images));
+    imageBytes = want;
   }
   return images;
 }

@@ -33,7 +33,7 @@ SparseConvNetCUDA::SparseConvNetCUDA(int dimension, int nInputFeatures,
   // and the forward passes should not share theirs with producer streams)
   nForwardLanes = nBatchProducerThreads >= 4 ? 2 : 1;
   for (int lane = 1; lane < nForwardLanes; ++lane)
-    laneStreams.emplace_back(new cudaMemStream());
+    laneStreams.emplace_back(new cudaMemStream(true, 0));
   batchPool.reserve(nBatchProducerThreads);
   const int nStreams = std::min(nBatchProducerThreads, N_PRODUCER_STREAMS);
   for (int c = 0; c < nStreams; c++) {

@@ -16,21 +16,23 @@ public:
   // layers: the stream runs layers, and not only the producers' rule books
   // (16 MB for each of those would be memory that nothing uses, and 1 ms of a
   // new net's first batch)
-  explicit cudaMemStream(bool layers = true);
+  explicit cudaMemStream(bool layers = true, size_t imageRoom = ROOM);
   ~cudaMemStream();
   cudaMemStream(const cudaMemStream &) = delete;
   cudaMemStream &operator=(const cudaMemStream &) = delete;
   void *stream() const;
   void synchronize() const;
   // Room for the weights of a pass over a batch as its contractions read them, in
-  // the order of the stream: a layers' stream has ROOM of it from the start, which
+  // the order of the stream: a net's own stream has ROOM of it from the start, which
   // holds those of a net of some 5 M weights (and so the first batch does not wait
   // for allocations: an allocation a layer was 0.1 ms of the first 1.6 of a net with
-  // up to 800 channels), and more as soon as it is asked for.
+  // up to 800 channels), the other lanes' streams, which a net may never use, make
+  // it with their first batch (0.1 ms of a new net for each), and all make more as
+  // soon as it is asked for.
+  static constexpr size_t ROOM = (size_t)32 << 20;
   void *imageRoom(size_t bytes);
 
 private:
-  static constexpr size_t ROOM = (size_t)32 << 20;
   void *images = nullptr;
   size_t imageBytes = 0;
 };
