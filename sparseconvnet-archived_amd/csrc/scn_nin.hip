@@ -1810,11 +1810,13 @@ static void launch_mfma(scn_ctx *ctx, const float *A, const float *W,
 // SCN_FP32 goes to the bf16 matrix cores where the contraction is long (40
 // GFLOP: 1.36 M x 1728 x 64 and its pooling 2.24 -> 1.41 ms) or its rows are few
 // (the split contraction: 600 x 384 x 128 in 5.0 us for 9.5).  In between it
-// keeps to fp32 MFMA, and so to the bits it has always given, whichever is the
-// faster (fp32 MFMA, planes, in us: 30000 x 256 x 96 19.8, 24.6; 66000 x 1728 x
-// 64 169, 209; 150000 x 1728 x 64 306, 277; 41600 x 640 x 320 151, 128; 9000 x
-// 1920 x 640 186, 140).  SCN_FP32_PLANES, which the host classes ask for, takes
-// the planes at every size.
+// keeps to fp32 MFMA, and so to the bits it has always given, though the planes,
+// their image made by the call, have become the faster there but for the shortest
+// contractions of plain rows (us, fp32 MFMA and planes, rows through rules: 35461 x
+// 256 x 96 35, 23; 17223 x 384 x 128 39, 22; 53325 x 640 x 320 220, 127; 11742 x 1920 x
+// 640 269, 144; 126507 x 1728 x 64 233, 142; 118775 x 128 x 32 19.5, 15.8, plain 16.8,
+// 26.5).  SCN_FP32_PLANES, which the host classes ask for, takes the planes at every
+// size.
 #define PLANES_MIN_FLOPS 4e10
 // rows16: a bf16 copy of the matrix the rules point into, or null; image: the
 // weights for the planes (scn_weight_images_many), or null
