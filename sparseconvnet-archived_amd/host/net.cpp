@@ -531,6 +531,7 @@ void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStr
     items.push_back(x.item);
     at += room(x.bytes);
   }
+  scn_prof_tag(ms.ctx, -1); // (no layer's)
   for (size_t i = 0; i < items.size(); i += SCN_IMAGES_MAX)
     SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, (int)std::min<size_t>(SCN_IMAGES_MAX, items.size() - i)));
 }
