@@ -386,8 +386,8 @@ def test_infinite_operands_of_the_weight_gradient(scn, ctx, M, fs, nIn, N):
 
 
 def test_an_epoch_with_an_infinite_weight(scn):
-    """of a channel that is never above zero, so that the net's outputs are finite: an epoch leaves what single batches,
-    which gather, leave"""
+    """of a channel that is never above zero, so that the net's outputs are finite: an epoch of one batch leaves what the
+    batch by itself, which gathers, leaves"""
     from sparseconvnet_archived_amd import hostapi, synthetic
     cfg = synthetic.config(2, batch=8)
     samples = synthetic.make_samples(cfg, 43)
@@ -406,16 +406,16 @@ def test_an_epoch_with_an_infinite_weight(scn):
         net.set_weights(nin[1], W, B)
         net.set_training(0.01, 0.9, shuffle=False)
         if epoch:
-            net.processDatasetTrain(ds, 4, 0.01, 0.9)
+            net.processDatasetTrain(ds, 8, 0.01, 0.9)
         else:
-            net.begin(ds, 4)
+            net.begin(ds, 8)
             while net.next_batch():
                 pass
         left.append([a for i in nin for m in (True, False) for a in net.get_weights(i, momentum=m) if a is not None])
         net.close()
     for k, (a, b) in enumerate(zip(*left)):
         sure = np.isfinite(b)
-        print("tensor", k, "not finite", int((~sure).sum()), "of", b.size, flush=True)
+        print("tensor", k, "not finite", int((~sure).sum()), "of", b.size, "off by", rel_l2(a[sure], b[sure]), flush=True)
         assert np.array_equal(a[~sure], b[~sure], equal_nan=True)
-        # (the bar of the oracle's epochs: a batch's share of rectifiers that a rounding turns)
-        assert rel_l2(a[sure], b[sure]) <= 3e-4
+        # (the same forward pass, bit for bit, so the same rectifiers: what is left are fp32 sums in other orders)
+        assert rel_l2(a[sure], b[sure]) <= 1e-5
