@@ -520,6 +520,19 @@ int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d
                             const float *d_Wt, const void *d_image, float *d_din, int64_t inputRows, int nIn);
 int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,
                  const float *d_D, float *d_dW, float *d_db, int64_t M, int N, int accumulate);
+/* The weight gradients of several layers in one launch: each as scn_conv_AtB
+ * gives it, or with null d_positions and fs = 1 as scn_sgemm_AtB_sums does for
+ * K = nIn (d_db may be null), always added. */
+#define SCN_ATB_MAX 24
+typedef struct scn_atb_item {
+  const float *d_in;
+  const int32_t *d_positions;
+  const float *d_D;
+  float *d_dW, *d_db;
+  int64_t M;
+  int32_t fs, nIn, N;
+} scn_atb_item;
+int scn_AtB_many(scn_ctx *ctx, const scn_atb_item *items, int nItems);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout
  * (NetworkInNetworkLayer.cu:7-25): w[i][j] = W[inPresent[i]][outPresent[j]],
  * W with rows of nOut floats; a null d_inPresent keeps the rows (row i of w

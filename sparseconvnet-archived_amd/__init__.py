@@ -47,6 +47,12 @@ class ImageItem(C.Structure):
                 ("precision", C.c_int32)]
 
 
+class AtbItem(C.Structure):
+    """scn_atb_item of the C header."""
+    _fields_ = [("d_in", C.c_void_p), ("d_positions", C.c_void_p), ("d_D", C.c_void_p), ("d_dW", C.c_void_p),
+                ("d_db", C.c_void_p), ("M", C.c_int64), ("fs", C.c_int32), ("nIn", C.c_int32), ("N", C.c_int32)]
+
+
 class NagItem(C.Structure):
     """scn_nag_item of the C header."""
     _fields_ = [("d_delta", C.c_void_p), ("d_momentum", C.c_void_p), ("d_weights", C.c_void_p),
@@ -156,6 +162,7 @@ def lib():
         "scn_activation_backward_to": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp, C.c_int]),
         "scn_sgemm_AtB_acc": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
         "scn_conv_AtB": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, i64, C.c_int, C.c_int]),
+        "scn_AtB_many": (C.c_int, [vp, P(AtbItem), C.c_int]),
         "scn_sgemm_AtB_sums": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, C.c_int, C.c_int]),
         "scn_maxpool_backward_through": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, C.c_int]),
         "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
@@ -372,6 +379,14 @@ class Context:
     def conv_AtB(self, d_in, d_positions, fs, nIn, d_D, d_dW, M, N, accumulate=False, d_db=None):
         _check(lib().scn_conv_AtB(self.h, d_in.ptr if d_in is not None else None, d_positions.ptr, fs, nIn, d_D.ptr,
                                   d_dW.ptr, d_db.ptr if d_db is not None else None, M, N, int(accumulate)))
+
+    def AtB_many(self, items):
+        """[(d_in, d_positions or None, fs, nIn, d_D, d_dW, d_db or None, M, N)]"""
+        arr = (AtbItem * max(1, len(items)))()
+        for k, (x, p, fs, nIn, D, dW, db, M, N) in enumerate(items):
+            arr[k] = AtbItem(x.ptr if x is not None else None, p.ptr if p is not None else None, D.ptr, dW.ptr,
+                             db.ptr if db is not None else None, M, fs, nIn, N)
+        _check(lib().scn_AtB_many(self.h, arr, len(items)))
 
     def sgemm_AtB_sums(self, d_A, d_D, d_dW, d_db, M, K, N, accumulate=False):
         _check(lib().scn_sgemm_AtB_sums(self.h, d_A.ptr, d_D.ptr, d_dW.ptr, d_db.ptr, M, K, N, int(accumulate)))

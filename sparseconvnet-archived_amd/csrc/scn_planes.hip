@@ -1712,25 +1712,29 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // splitting takes.  A backward layer with dW of 139000 x 384 x 128 384 -> 370 us;
 // dW of 28000 x 256 x 96 and its like 16.5 -> 15.6, of which some 5 are the start and
 // the atomics; 35461 x 256 x 96 20, 198759 x 1728 x 64 328 (A from HBM at 4.2 TB/s).
-constexpr int atb_ring(int MT, int NT) { return MT * NT >= 4 ? 2 : 3; }
-template <int MT, int NT, bool GATHER, bool LINES>
-__global__ void __launch_bounds__(512, 2)
-    k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
-                 float *__restrict__ dW, float *__restrict__ db, long long M, int K, int N, int nTiles,
-                 long long rowsPerSplit, GatherSource gs, const float *zeros) {
-  constexpr int PL = 3, GM = 8;
+// A step's planes are made among the MFMAs of the step before, and where registers
+// and LDS have room there are three wavefronts to a SIMD: the two together 55 -> 50 us
+// for six layers of a batch of drawings in one launch.
+constexpr int atb_ring(int MT, int NT) { return MT * NT >= 2 ? 2 : 3; }
+// wavefronts of a workgroup: three a SIMD where registers and LDS have room
+constexpr int atb_waves(int MT, int NT, bool LINES) { return LINES && MT * NT < 4 ? 12 : 8; }
+// (one tile of dW, of the rows from m0 to m1: m0 a multiple of ATB_STEP; GM wavefronts)
+template <int MT, int NT, bool GATHER, bool LINES, int GM>
+__device__ __forceinline__ void atb_tile(const float *__restrict__ A, const float *__restrict__ D, float *__restrict__ dW,
+                                         float *__restrict__ db, long long M, int K, int N, int nTiles,
+                                         GatherSource gs, const float *zeros, unsigned tile, long long m0,
+                                         long long m1) {
+  constexpr int PL = 3;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
-  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [8][TILE], [8][32 NT], a flag
-  float *const sBias = sTile + 8 * TILE;
-  int *const sAgain = reinterpret_cast<int *>(sBias + 8 * 32 * NT);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  extern __shared__ __attribute__((aligned(16))) float sTile[]; // [GM][TILE], [GM][32 NT], a flag
+  float *const sBias = sTile + GM * TILE;
+  int *const sAgain = reinterpret_cast<int *>(sBias + GM * 32 * NT);
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid)); // (what follows from it is not kept from one tile to the next)
+  const int lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
-  // (the tiles of a range of rows, which read the same, to one XCD)
-  const unsigned at = xcd_eighth(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-  const int k0 = (int)(at % gridDim.x / nTiles) * 32 * MT;
-  const int n0 = (int)(at % gridDim.x % nTiles) * 32 * NT;
-  const long long m0 = (long long)(at / gridDim.x) * rowsPerSplit;
-  const long long m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
+  const int k0 = (int)(tile / nTiles) * 32 * MT;
+  const int n0 = (int)(tile % nTiles) * 32 * NT;
   // this lane's columns (past the end: the last ones, not stored)
   int ka = k0 + MT * c, na = n0 + NT * c;
   ka = ka + MT <= K ? ka : K - MT;
@@ -1809,22 +1813,28 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
   for (int j = 0; j < NT; ++j)
     ds[j] = 0.f;
-  auto compute = [&](const Step &s) {
-    if (sums)
+  struct Planes {
+    bf16x8 a[MT][PL], d[NT][PL];
+  };
+  auto split = [&](const Step &s, Planes &p, bool counts) { // (counts: whether the step's D is to be summed)
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        ds[j] += ((s.d[0][j] + s.d[1][j]) + (s.d[2][j] + s.d[3][j])) + ((s.d[4][j] + s.d[5][j]) + (s.d[6][j] + s.d[7][j]));
-    bf16x8 ap[MT][PL], dp[NT][PL];
+    for (int j = 0; j < NT; ++j) {
+      const float sum =
+          ((s.d[0][j] + s.d[1][j]) + (s.d[2][j] + s.d[3][j])) + ((s.d[4][j] + s.d[5][j]) + (s.d[6][j] + s.d[7][j]));
+      ds[j] += counts ? sum : 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const float v[8] = {s.a[0][i], s.a[1][i], s.a[2][i], s.a[3][i], s.a[4][i], s.a[5][i], s.a[6][i], s.a[7][i]};
-      split8<PL>(v, ap[i]);
+      split8<PL>(v, p.a[i]);
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const float v[8] = {s.d[0][j], s.d[1][j], s.d[2][j], s.d[3][j], s.d[4][j], s.d[5][j], s.d[6][j], s.d[7][j]};
-      split8<PL>(v, dp[j]);
+      split8<PL>(v, p.d[j]);
     }
+  };
+  auto multiply = [&](const Planes &p) {
 #pragma unroll
     for (int x = 0; x < PL; ++x)
 #pragma unroll
@@ -1834,8 +1844,13 @@ __global__ void __launch_bounds__(512, 2)
 #pragma unroll
           for (int j = 0; j < NT; ++j) {
             floatx16 &d = acc[x + y == 0 ? 0 : 1][i][j];
-            d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ap[i][x], dp[j][y], d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p.a[i][x], p.d[j][y], d, 0, 0, 0);
           }
+  };
+  auto compute = [&](const Step &s) {
+    Planes p;
+    split(s, p, sums);
+    multiply(p);
   };
   if constexpr (LINES) {
     constexpr int RING = atb_ring(MT, NT), AU = 2 * MT, DU = 2 * NT, FETCH = AU + DU;
@@ -1870,23 +1885,33 @@ __global__ void __launch_bounds__(512, 2)
       for (int u = 0; u < (GATHER ? AU : 0); ++u)
         asm volatile("" : "+v"(x.r[u % (GATHER ? AU : 1)]) : : "memory");
     };
-    const float *const none = GATHER ? gs.zeros : zeros;
+    // (byte addresses: a multiplication a request of gathered rows, none of plain ones)
+    typedef unsigned long long u64;
+    const u64 none = (u64)(uintptr_t)(GATHER ? gs.zeros : zeros);
+    const u64 fromA = (u64)(uintptr_t)(GATHER ? A + ch4 : A + (m0 + ra) * K + ca);
+    const u64 fromD = (u64)(uintptr_t)(D + (m0 + rd) * N + cd);
+    const unsigned rowA = (GATHER ? gs.nIn : K) * 4u;
+    const int left = (int)(m1 - m0);
     auto fetch = [&](const Rules &x, int t, int slot) {
-      const long long m = place(t);
+      const int m = (int)(place(t) - m0); // uniform
       const unsigned lds = ldsRing + slot * SLOT;
+      const u64 stepA = fromA + (u64)m * K * 4, stepD = fromD + (u64)m * N * 4;
+      // (chosen, not jumped to: the MFMAs beside are dealt out in one block of code)
+      auto request = [&](int u, bool live, u64 from) {
+        asm volatile("" : "+v"(from));
+        dma_kilobyte(lds + u * 1024, reinterpret_cast<const unsigned char *>((uintptr_t)(live ? from : none)));
+      };
 #pragma unroll
       for (int u = 0; u < AU; ++u) {
-        const long long row = m + 8 / MT * u + ra;
         const int rule = x.r[GATHER ? u % AU : 0];
-        const float *const from = GATHER ? (rule >= 0 ? A + (long long)rule * gs.nIn + ch4 : none)
-                                         : (row < m1 ? A + row * K + ca : none);
-        dma_kilobyte(lds + u * 1024, reinterpret_cast<const unsigned char *>(from));
+        if constexpr (GATHER)
+          request(u, rule >= 0, fromA + (u64)(unsigned)rule * rowA);
+        else
+          request(u, m + 8 / MT * u + ra < left, stepA + (u64)(8 / MT * u) * K * 4);
       }
 #pragma unroll
-      for (int u = 0; u < DU; ++u) {
-        const long long row = m + 8 / NT * u + rd;
-        dma_kilobyte(lds + (AU + u) * 1024, reinterpret_cast<const unsigned char *>(row < m1 ? D + row * N + cd : none));
-      }
+      for (int u = 0; u < DU; ++u)
+        request(AU + u, m + 8 / NT * u + rd < left, stepD + (u64)(8 / NT * u) * N * 4);
     };
     auto take = [&](Step &s, int slot) {
       const unsigned char *const at = ring + slot * SLOT;
@@ -1912,32 +1937,80 @@ __global__ void __launch_bounds__(512, 2)
       // Rules are asked for a step before their rows, in front of the rows asked for
       // then: what has landed when all but the last step's rows have holds a step's
       // rows and the next request's rules.
-      static_assert(!GATHER || RING == 3, "the first two steps' rules come together");
-      Rules x;
-      {
-        Rules second;
+      if constexpr (MT * NT < 4) {
+        // A step's planes are made while the MFMAs of the one before run, dealt out
+        // among them.  So a slot is free when its planes have been made, and RING steps
+        // are under way.
+        Rules first[RING];
         int *const spare = reinterpret_cast<int *>(ring + (RING - 1) * SLOT); // (nothing is asked for there yet)
-        ask(0, spare);
-        ask(1, spare + AU * 64);
-        ask(RING - 1, sRule);
+        static_assert(RING * AU * 256 <= SLOT, "a slot holds the first rules");
+#pragma unroll
+        for (int r = 0; r < RING; ++r)
+          ask(r, spare + r * AU * 64);
+        ask(RING, sRule);
         w_landed<0>();
-        look(x, spare);
-        look(second, spare + AU * 64);
-        fetch(x, 0, 0);
-        if (RING == 3)
-          fetch(second, 1, 1);
-      }
-      int slot = 0, into = RING - 1;
+#pragma unroll
+        for (int r = 0; r < RING; ++r)
+          look(first[r], spare + r * AU * 64);
+        w_landed<0>(); // (the words have been read: their place is asked for again)
+#pragma unroll
+        for (int r = 0; r < RING; ++r)
+          fetch(first[r], r, r);
+        int slot = 1, into = 0;
+        Planes even, odd;
+        Rules x;
+        {
+          Step s;
+          w_landed<(RING - 1) * FETCH>();
+          take(s, 0);
+          split(s, even, true);
+        }
+        auto step = [&](const Planes &now, Planes &next, int t) {
+          w_landed<(RING - 2) * FETCH>(); // (and this wavefront's reads of the slot that is asked for again)
+          look(x, sRule);
+          Step s;
+          take(s, slot);
+          ask(t + RING + 1, sRule);
+          fetch(x, t + RING, into);
+          split(s, next, t + 1 < steps);
+          multiply(now);
+#pragma unroll
+          for (int k = 0; k < 6 * MT * NT; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                   // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x2, (44 * (MT + NT) + 6 * MT * NT - 1) / (6 * MT * NT), 0); // VALU
+          }
+          // (here and not where they are used)
+#pragma unroll
+          for (int l = 0; l < PL; ++l) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+              asm volatile("" : "+v"(next.a[i][l]));
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+              asm volatile("" : "+v"(next.d[j][l]));
+          }
+          slot = slot == RING - 1 ? 0 : slot + 1, into = into == RING - 1 ? 0 : into + 1;
+        };
 #pragma unroll 1
-      for (int t = 0; t < steps; ++t) {
-        w_landed<RING == 3 ? FETCH : 0>(); // (and this wavefront's reads of the slot that is asked for again)
-        look(x, sRule);
-        ask(t + RING, sRule);
-        fetch(x, t + RING - 1, into);
-        Step s;
-        take(s, slot);
-        compute(s);
-        slot = slot == RING - 1 ? 0 : slot + 1, into = into == RING - 1 ? 0 : into + 1;
+        for (int t = 0; t < steps; ++t) {
+          step(even, odd, t);
+          if (++t == steps)
+            break;
+          step(odd, even, t);
+        }
+      } else {
+        Rules x = {};
+        fetch(x, 0, 0);
+        int slot = 0, into = RING - 1;
+#pragma unroll 1
+        for (int t = 0; t < steps; ++t) {
+          w_landed<0>(); // (and this wavefront's reads of the slot that is asked for again)
+          fetch(x, t + RING - 1, into);
+          Step s;
+          take(s, slot);
+          compute(s);
+          slot = slot == RING - 1 ? 0 : slot + 1, into = into == RING - 1 ? 0 : into + 1;
+        }
       }
       w_landed<0>();
     }
@@ -2019,10 +2092,10 @@ __global__ void __launch_bounds__(512, 2)
       unsafeAtomicAdd(dW + (long long)kk * N + nn, sum);
   };
   unsigned again = 0; // this lane's elements that are to be taken again
-  for (int e = tid; e < TILE; e += 512) {
+  for (int e = tid; e < TILE; e += 64 * GM) {
     const float sum = add(e);
     if (doubtful<PL>(sum))
-      again |= 1u << (e / 512);
+      again |= 1u << (e / (64 * GM));
     else
       put(e, sum);
   }
@@ -2071,18 +2144,34 @@ __global__ void __launch_bounds__(512, 2)
         for (int v = 0; v < 16; ++v)
           sTile[wave * TILE + ((i * NT + j) * 16 + v) * 64 + lane] = plain[i][j][v];
     __syncthreads();
-    for (int e = tid; e < TILE; e += 512)
-      if (again >> (e / 512) & 1)
+    for (int e = tid; e < TILE; e += 64 * GM)
+      if (again >> (e / (64 * GM)) & 1)
         put(e, add(e));
   }
 }
 
 template <int MT, int NT, bool GATHER, bool LINES>
+__global__ void __launch_bounds__(64 * atb_waves(MT, NT, LINES), atb_waves(MT, NT, LINES) / 4)
+    k_atb_planes(const float *__restrict__ A, const float *__restrict__ D,
+                 float *__restrict__ dW, float *__restrict__ db, long long M, int K, int N, int nTiles,
+                 long long rowsPerSplit, GatherSource gs, const float *zeros) {
+  // (the tiles of a range of rows, which read the same, to one XCD)
+  const unsigned at = xcd_eighth(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  const long long m0 = at / gridDim.x * rowsPerSplit, m1 = m0 + rowsPerSplit < M ? m0 + rowsPerSplit : M;
+  atb_tile<MT, NT, GATHER, LINES, atb_waves(MT, NT, LINES)>(A, D, dW, db, M, K, N, nTiles, gs, zeros, at % gridDim.x,
+                                                            m0, m1);
+}
+constexpr size_t atb_lds(int MT, int NT, bool GATHER, bool LINES, int GM) {
+  const size_t sums = ((size_t)GM * 32 * MT * 32 * NT + GM * 32 * NT + 1) * sizeof(float);
+  const size_t rings = (size_t)GM * (atb_ring(MT, NT) * 2048 * (MT + NT) + (GATHER ? 2 * MT * 256 : 0));
+  return LINES && rings > sums ? rings : sums;
+}
+
+template <int MT, int NT, bool GATHER, bool LINES>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                       long long M, int K, int N, long long splits, const GatherSource &gs) {
-  const size_t sums = ((size_t)8 * 32 * MT * 32 * NT + 8 * 32 * NT + 1) * sizeof(float);
-  const size_t rings = (size_t)8 * (atb_ring(MT, NT) * 2048 * (MT + NT) + (GATHER ? 2 * MT * 256 : 0));
-  const size_t lds = LINES && rings > sums ? rings : sums;
+  constexpr int GM = atb_waves(MT, NT, LINES);
+  constexpr size_t lds = atb_lds(MT, NT, GATHER, LINES, GM);
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_planes<MT, NT, GATHER, LINES>),
@@ -2094,9 +2183,9 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, f
   const int nTiles = scn_ceil_div(N, 32 * NT);
   const long long tiles = (long long)scn_ceil_div(K, 32 * MT) * nTiles;
   long long rows = (M + splits - 1) / splits;
-  rows = (rows + 8 * ATB_STEP - 1) / (8 * ATB_STEP) * (8 * ATB_STEP);
+  rows = (rows + GM * ATB_STEP - 1) / (GM * ATB_STEP) * (GM * ATB_STEP);
   hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER, LINES>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
-                     dim3(512), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs, ctx->d_zeros);
+                     dim3(64 * GM), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs, ctx->d_zeros);
   return SCN_OK;
 }
 template <int MT, int NT>
@@ -2162,4 +2251,148 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
     return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
   }
   return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
+}
+
+// ---- the weight gradients of all layers of a net in one launch.  Each by itself is
+// a wave of workgroups that begins (some 4 us of trips to memory and of sums), has
+// a few microseconds of rows and ends in as many atomics again.  Here the tiles of
+// all of them, cut into ranges of rows, lie end to end, and every compute unit has
+// one workgroup that takes an equal part of that line: the end of one tile's range,
+// whole ones, the beginning of another.  So all end together, which workgroups of
+// one range each do not: their number is that of the compute units only by chance,
+// and a layer's ranges are shorter or longer than the next one's.  The seven layers of
+// a batch of 100 drawings (83597 x 12 x 32 to 100 x 192 x 100): 81 us in launches of
+// their own, 57 with workgroups of one range each, 51 so; without the first layer 65,
+// 50, 48.  12 batches of drawings 6515 -> 6260 us, of voxel models 5430 -> 5285.
+// What is left of it: 0.13 us a wavefront's step on a compute unit, in which vector
+// instructions are issued for half of the time, MFMAs run for a fifth and the
+// address unit works for a third; with any one of the three left out 0.11.
+// Tiles of two by one, by lines, through rules and without; one by one of rows that
+// are no whole requests, a net's first layer.
+struct AtbList {
+  const float *A[SCN_ATB_MAX], *D[SCN_ATB_MAX];
+  float *dW[SCN_ATB_MAX], *db[SCN_ATB_MAX];
+  const int *rules[SCN_ATB_MAX]; // null: plain rows
+  const float *zeros;
+  int M[SCN_ATB_MAX], K[SCN_ATB_MAX], N[SCN_ATB_MAX], fs[SCN_ATB_MAX];
+  int steps[SCN_ATB_MAX]; // of a range, ATB_MANY ATB_STEP rows each
+  int first[SCN_ATB_MAX]; // place in the line
+  int count, length, part; // of the line; of a workgroup
+};
+constexpr int ATB_MANY = atb_waves(2, 1, true); // wavefronts
+// What a step and a tile's beginning and end take, in sixteenths of a microsecond
+// (measured by the clock in the kernel, layers of 2500 to 84000 rows: by lines 1.42
+// to 1.68 us a step, a first layer's 1.3, and 4.7)
+constexpr int ATB_LINES_COST = 25, ATB_FIRST_COST = 21, ATB_TILE_COST = 75;
+__device__ __host__ __forceinline__ int atb_step_cost(const int *rules, int nIn) {
+  return rules && nIn % 4 ? ATB_FIRST_COST : ATB_LINES_COST;
+}
+__global__ void __launch_bounds__(64 * ATB_MANY, ATB_MANY / 4) k_atb_many(AtbList l) {
+  static_assert(SCN_ATB_MAX <= 64, "a lane an item");
+  int pos = (int)xcd_eighth(blockIdx.x, gridDim.x) * l.part; // (neighbours to one XCD)
+  const int end = pos + l.part < l.length ? pos + l.part : l.length;
+#pragma unroll 1
+  while (pos < end) { // uniform
+    const int lane = __lane_id(); // (anew)
+    const int t = __popcll(__ballot(lane < l.count && pos >= l.first[lane < SCN_ATB_MAX ? lane : 0])) - 1;
+    const int K = l.K[t], N = l.N[t], steps = l.steps[t], M = l.M[t];
+    GatherSource gs = GatherSource();
+    gs.rules = l.rules[t];
+    gs.fs = l.fs[t];
+    gs.nIn = K / gs.fs;
+    gs.zeros = l.zeros;
+    const int cost = atb_step_cost(gs.rules, gs.nIn), whole = ATB_TILE_COST + steps * cost;
+    // the range of a tile that this is in, tile after tile of one range of rows
+    const unsigned unit = (unsigned)(pos - l.first[t]) / whole;
+    const int from = pos - l.first[t] - (int)unit * whole;
+    const int to = whole - from < end - pos ? whole : from + end - pos;
+    auto step = [&](int place) { return place <= ATB_TILE_COST ? 0 : (place - ATB_TILE_COST + cost - 1) / cost; };
+    pos += to - from;
+    const int nTiles = (N + 31) / 32;
+#define SCN_ATB_TILE(MT, GATHER, LINES)                                                                         \
+  const unsigned tiles = (K + 32 * MT - 1) / (32 * MT) * nTiles;                                                \
+  const long long r0 = (long long)(unit / tiles) * steps;                                                       \
+  const long long m0 = (r0 + step(from)) * (ATB_MANY * ATB_STEP), m1 = (r0 + step(to)) * (ATB_MANY * ATB_STEP); \
+  if (m0 < (m1 < M ? m1 : M)) {                                                                                 \
+    __syncthreads(); /* (the one before is done with LDS) */                                                    \
+    atb_tile<MT, 1, GATHER, LINES, ATB_MANY>(l.A[t], l.D[t], l.dW[t], l.db[t], M, K, N, nTiles, gs, l.zeros,    \
+                                             unit % tiles, m0, m1 < M ? m1 : M);                                \
+  }
+    if (gs.rules && gs.nIn % 4 == 0) {
+      SCN_ATB_TILE(2, true, true);
+    } else if (gs.rules) {
+      SCN_ATB_TILE(1, true, false);
+    } else {
+      SCN_ATB_TILE(2, false, true);
+    }
+#undef SCN_ATB_TILE
+  }
+}
+// the tile that an item takes among many, or 0: not one for it
+static int atb_many_tile(const scn_atb_item &it) {
+  const int K = it.fs * it.nIn;
+  if (it.M > (1 << 30) || it.N % 4 || (((uintptr_t)it.d_in | (uintptr_t)it.d_D) & 15))
+    return 0;
+  if (it.d_positions)
+    return it.nIn % 4 == 0 ? 2 : K <= 32 ? 1 : 0;
+  return K % 4 == 0 ? 2 : 0;
+}
+int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
+  AtbList l;
+  l.count = 0;
+  l.zeros = ctx->d_zeros;
+  long long tiles[SCN_ATB_MAX], steps[SCN_ATB_MAX], work = 0;
+  int cost[SCN_ATB_MAX];
+  for (int k = 0; k < nItems; ++k) {
+    const scn_atb_item &it = items[k];
+    if (it.M == 0)
+      continue;
+    const int m = atb_many_tile(it), K = it.fs * it.nIn;
+    const long long n = m ? (long long)scn_ceil_div(K, 32 * m) * scn_ceil_div(it.N, 32) : 0;
+    const long long s = scn_ceil_div(it.M, ATB_MANY * ATB_STEP);
+    const int each = atb_step_cost(it.d_positions, it.nIn);
+    // one that keeps the chip busy by itself (some 60 us) gains nothing, and two by
+    // two tiles may be better for it
+    if (!m || n > 4096 || n * (s * each + ATB_TILE_COST) > 64ll * 16 * ctx->numCU) {
+      GatherSource gs = GatherSource();
+      gs.rules = it.d_positions;
+      gs.fs = it.fs;
+      gs.nIn = it.nIn;
+      gs.zeros = ctx->d_zeros;
+      SCN_TRY(scn_atb_planes(ctx, it.d_in, it.d_D, it.d_dW, it.d_db, it.M, K, it.N, it.d_positions ? &gs : nullptr));
+      continue;
+    }
+    const int c = l.count++;
+    l.A[c] = it.d_in, l.D[c] = it.d_D, l.dW[c] = it.d_dW, l.db[c] = it.d_db, l.rules[c] = it.d_positions;
+    l.M[c] = (int)it.M, l.K[c] = K, l.N[c] = it.N, l.fs[c] = it.fs;
+    tiles[c] = n, steps[c] = s, cost[c] = each;
+    work += n * s * each;
+  }
+  if (l.count == 0)
+    return SCN_OK;
+  // ranges about as long as a workgroup's part, all tiles of one side by side: they
+  // read the same rows
+  const long long part = scn_ceil_div(work, ctx->numCU);
+  long long length = 0;
+  for (int c = 0; c < l.count; ++c) {
+    long long ranges = (steps[c] * cost[c] + part / 2) / part;
+    ranges = ranges < 1 ? 1 : ranges > steps[c] ? steps[c] : ranges;
+    l.steps[c] = (int)scn_ceil_div(steps[c], ranges);
+    l.first[c] = (int)length;
+    length += tiles[c] * scn_ceil_div(steps[c], l.steps[c]) * (ATB_TILE_COST + (long long)l.steps[c] * cost[c]);
+  }
+  l.length = (int)length; // (at most SCN_ATB_MAX times what an item may be, and a range more of each)
+  l.part = scn_ceil_div(length, ctx->numCU);
+  constexpr size_t lds = atb_lds(2, 1, true, true, ATB_MANY);
+  static_assert(lds >= atb_lds(2, 1, false, true, ATB_MANY) && lds >= atb_lds(1, 1, true, false, ATB_MANY), "one size for all");
+  static OncePerDevice configured;
+  const int rc = configured.run(ctx->device, [&]() {
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_many), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds) == hipSuccess
+               ? SCN_OK
+               : SCN_ERR_HIP;
+  });
+  SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
+  hipLaunchKernelGGL(k_atb_many, dim3((unsigned)scn_ceil_div(length, l.part)), dim3(64 * ATB_MANY), lds, ctx->stream, l);
+  return SCN_OK;
 }

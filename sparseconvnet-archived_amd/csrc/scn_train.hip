@@ -291,6 +291,26 @@ extern "C" int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_po
   return SCN_OK;
 }
 
+extern "C" int scn_AtB_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_AtB_many: null context");
+  SCN_REQUIRE(nItems >= 0 && nItems <= SCN_ATB_MAX && (items || nItems == 0), SCN_ERR_ARG,
+              "scn_AtB_many: %d items (at most %d)", nItems, SCN_ATB_MAX);
+  for (int k = 0; k < nItems; ++k) {
+    const scn_atb_item &it = items[k];
+    SCN_REQUIRE(it.M >= 0 && it.fs >= 1 && it.nIn >= 1 && (int64_t)it.fs * it.nIn <= 0x7fffffff && it.N >= 1 &&
+                    (it.d_positions ? it.nIn <= SCN_ZERO_FLOATS : it.fs == 1 || it.M == 0),
+                SCN_ERR_ARG, "scn_AtB_many: item %d M %lld fs %d nIn %d N %d", k, (long long)it.M, it.fs, it.nIn, it.N);
+    // (d_in may be null where there are rules, all negative)
+    SCN_REQUIRE(it.M == 0 || (it.d_dW && it.d_D && (it.d_in || it.d_positions)), SCN_ERR_ARG,
+                "scn_AtB_many: item %d null buffer", k);
+    SCN_REQUIRE(((uintptr_t)it.d_positions & 15) == 0, SCN_ERR_ARG, "scn_AtB_many: positions start on 16 bytes");
+  }
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  SCN_TRY(scn_atb_planes_many(ctx, items, nItems));
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 // ------------------------------------- the gradient of a convolution's input
 // dA = D W^T scattered through the rules is itself a convolution: row r of the
 // input gets, for every filter position f at which an output row o names it,

@@ -91,8 +91,10 @@ public:
   size_t hostFeatureCount;
   std::unique_ptr<BatchResultStage> result;
   // SparseConvNetCUDA::backwardBatch: the layers' momentum steps, put off to the
-  // end of the backward pass and queued together (elsewhere every layer queues its own)
+  // end of the backward pass and queued together (elsewhere every layer queues its
+  // own), and the products that they wait for
   std::vector<scn_nag_item> updates;
+  std::vector<scn_atb_item> products;
   bool collectUpdates = false;
   void reset();
 };

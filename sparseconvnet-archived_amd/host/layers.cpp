@@ -432,22 +432,38 @@ static void nin_activation_ahead(cudaMemStream &ms,
       PReLU->dPtr(), db.dPtr(), dprelu->dPtr(), clean));
   pooled.activationAhead = output.activationAhead = true;
 }
+// dW, and with d_db the bias gradient: where the batch collects its updates, with
+// all other layers' at the end of its backward pass, before which nothing reads it
+// (later: what a step on the spot needs).  Until then the matrices stay as they are:
+// every interface has its own.
+static void nin_product(cudaMemStream &ms, SpatiallySparseBatch &batch, const scn_atb_item &it, bool clean,
+                        bool later) {
+  if (!clean) {
+    SCN_CHECKED(scn_fill32(ms.ctx, it.d_dW, 0, (size_t)it.fs * it.nIn * it.N));
+    if (it.d_db)
+      SCN_CHECKED(scn_fill32(ms.ctx, it.d_db, 0, (size_t)it.N));
+  }
+  if (batch.collectUpdates && later)
+    batch.products.push_back(it);
+  else
+    SCN_CHECKED(scn_AtB_many(ms.ctx, &it, 1));
+  addMultiplyAdds((__int128_t)it.M * it.fs * it.nIn * it.N);
+}
 // A layer behind a convolution that was left out: dW from the convolution's
 // input, and that input's gradient from this layer's output's, through the rules
 // turned round (transposed: the weights for that, scn_transpose_filters_many).
 static void conv_nin_gradients(cudaMemStream &ms, SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output, vectorCUDA<float> &dw, float *db,
-                               vectorCUDA<float> &transposed, bool clean, int batchSize) {
+                               vectorCUDA<float> &transposed, bool clean, SpatiallySparseBatch &batch, bool later) {
   SpatiallySparseBatchInterface &src = *middle.deferredGatherFrom;
   const int64_t M = output.nSpatialSites;
   const int N = output.nFeatures, nIn = src.nFeatures, fs = middle.nFeatures / nIn;
-  SCN_CHECKED(scn_conv_AtB(ms.ctx, src.sub->features.dPtr(), middle.positions.dPtr(), fs, nIn,
-                           output.sub->dfeatures.dPtr(), dw.dPtr(), db, M, N, clean));
-  addMultiplyAdds((__int128_t)M * fs * nIn * N);
+  nin_product(ms, batch, {src.sub->features.dPtr(), middle.positions.dPtr(), output.sub->dfeatures.dPtr(), dw.dPtr(), db,
+                          M, fs, nIn, N}, clean, later);
   if (!src.backpropErrors)
     return;
   SCN_CHECKED(scn_background_sums(ms.ctx, output.sub->dfeatures.dPtr(), M, N,
-                                  middle.background.dPtr(), fs, batchSize));
+                                  middle.background.dPtr(), fs, batch.batchSize));
   src.sub->dfeatures.resize64(((size_t)src.nSpatialSites + src.gradientSums) * nIn);
   SCN_CHECKED(scn_conv_input_gradient(ms.ctx, output.sub->dfeatures.dPtr(), middle.inverse.dPtr(), fs, N,
                                       transposed.dPtr(), take_image(output.sub->turnedImage), src.sub->dfeatures.dPtr(), src.nSpatialSites, nIn));
@@ -488,16 +504,10 @@ static void nin_backwards(cudaMemStream &ms, SpatiallySparseBatch &batch,
         dprelu ? dprelu->dPtr() : nullptr));
   output.activationDone = output.activationAhead = false;
   if (input.deferredGatherFrom) {
-    conv_nin_gradients(ms, input, output, dw, sums ? db.dPtr() : nullptr, workspace, clean, batch.batchSize);
-  } else if (sums) {
-    SCN_CHECKED(scn_sgemm_AtB_sums(ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(), dw.dPtr(),
-                                   db.dPtr(), M, K, N, clean));
-    addMultiplyAdds((__int128_t)M * K * N);
+    conv_nin_gradients(ms, input, output, dw, sums ? db.dPtr() : nullptr, workspace, clean, batch, !shrunkW);
   } else {
-    SCN_CHECKED((clean ? scn_sgemm_AtB_acc : scn_sgemm_AtB)(
-        ms.ctx, input.sub->features.dPtr(), output.sub->dfeatures.dPtr(),
-        dw.dPtr(), M, K, N));
-    addMultiplyAdds((__int128_t)M * K * N);
+    nin_product(ms, batch, {input.sub->features.dPtr(), nullptr, output.sub->dfeatures.dPtr(), dw.dPtr(),
+                            sums ? db.dPtr() : nullptr, M, 1, K, N}, clean, !shrunkW);
   }
   if (input.backpropErrors && !input.deferredGatherFrom) {
     input.sub->dfeatures.resize64(((size_t)input.nSpatialSites + input.gradientSums) * K);

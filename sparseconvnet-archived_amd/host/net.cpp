@@ -477,6 +477,7 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
     SCN_CHECKED(scn_transpose_filters_many(memStream.ctx, filters.data() + i,
                                            (int)std::min<size_t>(SCN_FILTERS_MAX, filters.size() - i)));
   batch.updates.clear();
+  batch.products.clear();
   batch.collectUpdates = true;
   for (int i = (int)layers.size() - 1; i >= 0; i--) {
     scn_prof_tag(memStream.ctx, i);
@@ -489,6 +490,10 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   batch.collectUpdates = false;
   for (size_t i = 1; i < batch.interfaces.size(); i++)
     batch.interfaces[i].sub->turnedImage = nullptr;
+  scn_prof_tag(memStream.ctx, -1); // (no layer's)
+  for (size_t i = 0; i < batch.products.size(); i += SCN_ATB_MAX)
+    SCN_CHECKED(scn_AtB_many(memStream.ctx, batch.products.data() + i,
+                             (int)std::min<size_t>(SCN_ATB_MAX, batch.products.size() - i)));
   for (size_t i = 0; i < batch.updates.size(); i += SCN_NAG_MAX)
     SCN_CHECKED(scn_nag_update_many(
         memStream.ctx, batch.updates.data() + i,

@@ -129,6 +129,39 @@ def test_gradient_with_the_filters_laid_out(scn, ctx, d, field, window, batch, d
     assert np.array_equal(outs[0].download(), outs[1].download())
 
 
+# all layers' weight gradients in one launch: rows through rules by lines (whole tiles and not), a first layer's of three
+# channels, plain rows; no rows, fewer than a step, more than a workgroup's share; a shape that goes by itself (N 31); more
+# tiles than compute units (1600 x 512: 400) beside others
+@pytest.mark.parametrize("plain", [[(1, 32, 32)], [(100, 160, 192), (0, 32, 32), (100, 192, 100), (130, 34, 31)],
+                                   [(5000, 1600, 512), (33, 64, 4), (20001, 96, 128)]])
+@pytest.mark.parametrize("convs", [[], [(2, 11, 3, 4, 0.2, 32, 36), (2, 40, 2, 9, 0.15, 3, 32), (3, 7, 3, 3, 0.05, 64, 64)],
+                                   [(2, 60, 2, 40, 0.15, 36, 64), (1, 50, 2, 3, 0.2, 32, 32)]])
+def test_weight_gradients_of_many_layers(scn, ctx, plain, convs):
+    rng = np.random.default_rng(len(plain) + 7 * len(convs))
+    items, checks = [], []
+    for M, K, N in plain:
+        A, D = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((M, N), dtype=np.float32)
+        items.append((ctx.array(A) if M else None, None, 1, K, ctx.array(D) if M else ctx.empty(1, np.float32), M, N))
+        checks.append((A, D))
+    for d, field, window, batch, density, nIn, N in convs:
+        g, n, rows, fs, d_rules, bg = layer(scn, ctx, d, field, window, batch, density, field + N)
+        positions = ctx.empty((fs, (rows + 15) // 16 * 16), np.int32)
+        ctx.rules_inverse_many([(g, d_rules, None, None, positions, rows, n, fs)])
+        rules = d_rules.download()
+        x, D = rng.standard_normal((n, nIn), dtype=np.float32), rng.standard_normal((rows, N), dtype=np.float32)
+        items.append((ctx.array(x), positions, fs, nIn, ctx.array(D), rows, N))
+        checks.append((np.where(rules[:, :, None] >= 0, x[np.maximum(rules, 0)], 0).reshape(rows, fs * nIn), D))
+    print("weight gradients of", [(i[2], i[3], i[5], i[6]) for i in items], flush=True)
+    starts = [rng.standard_normal((A.shape[1] + 1, D.shape[1]), dtype=np.float32) for A, D in checks]
+    out = [(ctx.array(s[:-1]), ctx.array(s[-1]) if k % 3 else None) for k, s in enumerate(starts)]
+    ctx.AtB_many([(x, p, fs, nIn, D, dW, db, M, N) for (x, p, fs, nIn, D, M, N), (dW, db) in zip(items, out)])
+    for (A, D), s, (dW, db) in zip(checks, starts, out):
+        A, D = A.astype(np.float64), D.astype(np.float64)
+        assert np.all(np.abs(dW.download() - s[:-1] - A.T @ D) <= 2e-6 * (np.abs(A).T @ np.abs(D) + np.abs(s[:-1])))
+        if db is not None:
+            assert np.all(np.abs(db.download() - s[-1] - D.sum(0)) <= 2e-6 * (np.abs(D).sum(0) + np.abs(s[-1])))
+
+
 # every tile that sums take; ragged rows and columns; added to and not
 @pytest.mark.parametrize("M,K,N", [(1, 32, 32), (130, 34, 31), (1000, 66, 100), (40001, 12, 32), (30011, 256, 96), (70003, 432, 128),
                                    (53327, 644, 324)])
