@@ -533,6 +533,31 @@ typedef struct scn_atb_item {
   int32_t fs, nIn, N;
 } scn_atb_item;
 int scn_AtB_many(scn_ctx *ctx, const scn_atb_item *items, int nItems);
+/* dMaxPoolBackProp by rows of the input, for square windows that overlap by no
+ * more than 1, 2, 4 or 8 to a row (scn_pool_inverse_slots: how many, 0: not a
+ * pooling for it).  scn_pool_inverse_many turns a pooling's rules round:
+ *   d_inverse [inputRows x slots]: the windows that a row lies in (-1: none; -2 all
+ *     through: a sample's background row);
+ *   d_samples [2 batch + 1]: where every sample's windows begin, and where the last
+ *     one's end; the samples' background rows (negative: none).
+ * output: the pooling's grids, as a plan made them; the counts of both are settled.
+ * scn_maxpool_gradient writes the whole of d_din [inputRows x C] (C a multiple of 4,
+ * buffers aligned to 16 bytes); d_out and act as scn_maxpool_backward_through has
+ * them, or null and SCN_NOSIGMOID; with d_background of a convolution whose rows
+ * are d_din's, at fs <= 8 positions (scn_rules_inverse_many), also the rows behind
+ * that scn_background_sums adds to, which need not be cleared. */
+typedef struct scn_pool_inverse_item {
+  const scn_grids *input, *output;
+  const int32_t *d_rules; /* [rows x size^dimension] */
+  int32_t *d_inverse, *d_samples;
+  int64_t rows, inputRows;
+  int32_t size, stride;
+} scn_pool_inverse_item;
+int scn_pool_inverse_slots(int dimension, int size, int stride);
+int scn_pool_inverse_many(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems);
+int scn_maxpool_gradient(scn_ctx *ctx, float *d_din, int64_t inputRows, const float *d_dout, int64_t rows, int C,
+                         const int32_t *d_choice, const float *d_out, int act, const int32_t *d_inverse, int slots,
+                         const int32_t *d_samples, int batch, const int32_t *d_background, int fs);
 /* Dropout during training.  dShrinkMatrixForDropout / dShrinkVectorForDropout
  * (NetworkInNetworkLayer.cu:7-25): w[i][j] = W[inPresent[i]][outPresent[j]],
  * W with rows of nOut floats; a null d_inPresent keeps the rows (row i of w

@@ -47,6 +47,13 @@ class ImageItem(C.Structure):
                 ("precision", C.c_int32)]
 
 
+class PoolInverseItem(C.Structure):
+    """scn_pool_inverse_item of the C header."""
+    _fields_ = [("input", C.c_void_p), ("output", C.c_void_p), ("d_rules", C.c_void_p), ("d_inverse", C.c_void_p),
+                ("d_samples", C.c_void_p), ("rows", C.c_int64), ("inputRows", C.c_int64), ("size", C.c_int32),
+                ("stride", C.c_int32)]
+
+
 class AtbItem(C.Structure):
     """scn_atb_item of the C header."""
     _fields_ = [("d_in", C.c_void_p), ("d_positions", C.c_void_p), ("d_D", C.c_void_p), ("d_dW", C.c_void_p),
@@ -165,6 +172,10 @@ def lib():
         "scn_AtB_many": (C.c_int, [vp, P(AtbItem), C.c_int]),
         "scn_sgemm_AtB_sums": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, C.c_int, C.c_int]),
         "scn_maxpool_backward_through": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, C.c_int]),
+        "scn_pool_inverse_slots": (C.c_int, [C.c_int, C.c_int, C.c_int]),
+        "scn_pool_inverse_many": (C.c_int, [vp, P(PoolInverseItem), C.c_int]),
+        "scn_maxpool_gradient": (C.c_int, [vp, vp, i64, vp, i64, C.c_int, vp, vp, C.c_int, vp, C.c_int, vp, C.c_int, vp,
+                                           C.c_int]),
         "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
         "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, i64, C.c_int]),
         "scn_weight_image_bytes": (i64, [vp, i64, C.c_int, C.c_int, C.c_int, C.c_int]),
@@ -393,6 +404,19 @@ class Context:
 
     def maxpool_backward_through(self, d_din, d_dout, count, C, d_choice, d_out, act):
         _check(lib().scn_maxpool_backward_through(self.h, d_din.ptr, d_dout.ptr, count, C, d_choice.ptr, d_out.ptr, act))
+
+    def pool_inverse_many(self, items):
+        """[(input grids, output grids, d_rules, d_inverse, d_samples, rows, inputRows, size, stride)]"""
+        arr = (PoolInverseItem * max(1, len(items)))()
+        for k, (g, h, rules, inverse, samples, rows, inputRows, size, stride) in enumerate(items):
+            arr[k] = PoolInverseItem(g.h, h.h, rules.ptr, inverse.ptr, samples.ptr, rows, inputRows, size, stride)
+        _check(lib().scn_pool_inverse_many(self.h, arr, len(items)))
+
+    def maxpool_gradient(self, d_din, inputRows, d_dout, rows, C_, d_choice, d_out, act, d_inverse, slots, d_samples, batch,
+                         d_background=None, fs=0):
+        _check(lib().scn_maxpool_gradient(self.h, d_din.ptr, inputRows, d_dout.ptr, rows, C_, d_choice.ptr,
+                                          d_out.ptr if d_out is not None else None, act, d_inverse.ptr, slots,
+                                          d_samples.ptr, batch, d_background.ptr if d_background is not None else None, fs))
 
     def rules_inverse_many(self, items):
         """items: (input Grids, d_rules, d_inverse, d_background, d_positions, rows, inputRows, fs) tuples; the three

@@ -1324,6 +1324,372 @@ extern "C" int scn_maxpool_backward_through(scn_ctx *ctx, float *d_din, const fl
   return maxpool_backward(ctx, d_din, d_dout, count, C, d_choice, d_out, act);
 }
 
+// ------------------------------------ the gradient of a pooling's input, by rows
+// The scatter above adds, where a row of the input has a window or a few: with the
+// pooling's rules turned round (inverse[r slots + j] = the window in which row r lies
+// at the j-th of the offsets that a row may have in a window; negative: none) every
+// row is read together and written once, nothing is cleared and no float is added
+// atomically.  A sample's background row may lie in any of its windows: those are
+// walked by one to eight wavefronts a sample and 16 channels, which also sums, where the layer
+// before the pooling is a convolution, what goes to the rows that name that
+// convolution's background, per position (what k_background_sums makes of din), from
+// the same windows: an output of the pooling has one row that it chose.
+//
+// A row's slot: ceil(size / stride) of them an axis.
+static int pool_slots(int dimension, int size, int stride, int *perAxis) {
+  *perAxis = stride >= 1 ? (size + stride - 1) / stride : 0;
+  int n = 1;
+  for (int a = 0; a < dimension; ++a)
+    n *= *perAxis;
+  return n == 1 || n == 2 || n == 4 || n == 8 ? n : 0;
+}
+extern "C" int scn_pool_inverse_slots(int dimension, int size, int stride) {
+  int k;
+  double width = 1; // (positions of a window)
+  for (int a = 0; a < dimension; ++a)
+    width *= size;
+  return dimension >= 1 && dimension <= 8 && size >= 1 && stride >= 1 && width <= 1024 ? pool_slots(dimension, size, stride, &k) : 0;
+}
+struct PoolInverseList {
+  const int *rules[SCN_INVERSE_MAX], *bg[SCN_INVERSE_MAX], *outBg[SCN_INVERSE_MAX];
+  int *inverse[SCN_INVERSE_MAX], *samples[SCN_INVERSE_MAX];
+  long long volume[SCN_INVERSE_MAX];
+  int rows[SCN_INVERSE_MAX], inRows[SCN_INVERSE_MAX], batch[SCN_INVERSE_MAX];
+  int dimension[SCN_INVERSE_MAX], size[SCN_INVERSE_MAX], stride[SCN_INVERSE_MAX], slots[SCN_INVERSE_MAX];
+  unsigned firstBlock[SCN_INVERSE_MAX + 1];
+  int count;
+};
+// a workgroup an item: where the samples' windows begin, and the background rows' marks
+__global__ __launch_bounds__(256) void k_pool_samples(PoolInverseList l) {
+  const int t = blockIdx.x, batch = l.batch[t], slots = l.slots[t];
+  // (a sample's rows are its sites and then, if it is not full, a background row)
+  auto end = [&](int s) {
+    long long full = 0;
+    int x = s;
+    for (; x >= 0 && l.outBg[t][x] < 0; --x)
+      full += l.volume[t];
+    const long long e = full + (x >= 0 ? l.outBg[t][x] + 1 : 0);
+    return (int)(e < l.rows[t] ? e : l.rows[t]);
+  };
+  for (int s = threadIdx.x; s <= batch; s += 256)
+    l.samples[t][s] = s == 0 ? 0 : end(s - 1);
+  for (int s = threadIdx.x; s < batch; s += 256) {
+    const int r = l.bg[t][s], mine = r >= 0 && r < l.inRows[t] ? r : -1;
+    l.samples[t][batch + 1 + s] = mine;
+    if (mine >= 0)
+      for (int j = 0; j < slots; ++j)
+        l.inverse[t][(long long)mine * slots + j] = -2;
+  }
+}
+// a lane a window
+__global__ __launch_bounds__(256) void k_pool_inverse(PoolInverseList l) {
+  static_assert(SCN_INVERSE_MAX <= 64, "a lane an item");
+  const int lane = threadIdx.x & 63;
+  const int t =
+      __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_INVERSE_MAX ? lane : 0])) - 1;
+  const long long o = (long long)(blockIdx.x - l.firstBlock[t]) * 256 + threadIdx.x;
+  if (o >= l.rows[t])
+    return;
+  const int dimension = l.dimension[t], size = l.size[t], stride = l.stride[t], slots = l.slots[t], inRows = l.inRows[t];
+  const int perAxis = (size + stride - 1) / stride;
+  int width = 1;
+  for (int a = 0; a < dimension; ++a)
+    width *= size;
+  int *const inverse = l.inverse[t];
+  for (int f = 0; f < width; ++f) { // (uniform; offsets along the last axis first)
+    int j = 0;
+    for (int a = 0, x = f, each = 1; a < dimension; ++a, x /= size, each *= perAxis)
+      j += x % size / stride * each;
+    const int r = l.rules[t][o * width + f];
+    if (r < 0 || r >= inRows)
+      continue;
+    int *const at = inverse + (long long)r * slots + j;
+    if (*at != -2)
+      *at = (int)o;
+  }
+}
+extern "C" int scn_pool_inverse_many(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_pool_inverse_many: null context");
+  SCN_REQUIRE(nItems >= 0 && nItems <= SCN_INVERSE_MAX && (items || nItems == 0), SCN_ERR_ARG,
+              "scn_pool_inverse_many: %d items (at most %d)", nItems, SCN_INVERSE_MAX);
+  PoolInverseList l;
+  void *fill[SCN_INVERSE_MAX];
+  size_t words[SCN_INVERSE_MAX];
+  long long blocks = 0; // (16 items of no more than 2^23 workgroups)
+  int fills = 0;
+  l.count = 0;
+  for (int k = 0; k < nItems; ++k) {
+    const scn_pool_inverse_item &it = items[k];
+    SCN_REQUIRE(it.input && it.output && it.rows >= 0 && it.rows <= 0x7fffffffll && it.inputRows >= 0, SCN_ERR_ARG,
+                "scn_pool_inverse_many: item %d rows %lld of %lld", k, (long long)it.rows, (long long)it.inputRows);
+    const int slots = scn_pool_inverse_slots(it.input->d, it.size, it.stride);
+    SCN_REQUIRE(slots > 0, SCN_ERR_ARG, "scn_pool_inverse_many: item %d size %d stride %d", k, it.size, it.stride);
+    SCN_REQUIRE(it.inputRows * slots <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_pool_inverse_many: item %d: %lld rows", k,
+                (long long)it.inputRows);
+    SCN_REQUIRE(!it.input->pending && !it.output->pending, SCN_ERR_STATE,
+                "scn_pool_inverse_many: item %d: counts not settled", k);
+    SCN_REQUIRE(it.input->batch == it.output->batch && it.input->d == it.output->d, SCN_ERR_ARG,
+                "scn_pool_inverse_many: item %d: grids of another pooling", k);
+    SCN_REQUIRE((it.d_rules || it.rows == 0) && (it.d_inverse || it.inputRows == 0) && it.d_samples, SCN_ERR_ARG,
+                "scn_pool_inverse_many: item %d null buffer", k);
+    const int c = l.count++;
+    l.rules[c] = it.d_rules;
+    l.bg[c] = it.input->bg.p;
+    l.outBg[c] = it.output->bg.p;
+    l.volume[c] = it.output->vol;
+    l.inverse[c] = it.d_inverse;
+    l.samples[c] = it.d_samples;
+    l.rows[c] = (int)it.rows;
+    l.inRows[c] = (int)it.inputRows;
+    l.batch[c] = it.input->batch;
+    l.dimension[c] = it.input->d;
+    l.size[c] = it.size;
+    l.stride[c] = it.stride;
+    l.slots[c] = slots;
+    l.firstBlock[c] = (unsigned)blocks;
+    blocks += scn_ceil_div(it.rows, 256);
+    if (it.inputRows) {
+      fill[fills] = it.d_inverse;
+      words[fills++] = (size_t)it.inputRows * slots;
+    }
+  }
+  if (l.count == 0)
+    return SCN_OK;
+  l.firstBlock[l.count] = (unsigned)blocks;
+  ProfScope prof(ctx, SCN_K_RULES);
+  if (fills)
+    SCN_TRY(scn_fill32_many(ctx, fill, words, fills, 0xffffffffu));
+  hipLaunchKernelGGL(k_pool_samples, dim3(l.count), dim3(256), 0, ctx->stream, l);
+  if (blocks)
+    hipLaunchKernelGGL(k_pool_inverse, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, l);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
+struct PoolGradient {
+  float *din;
+  const float *dout, *out; // out: the derivative of act is taken through it (null: has been)
+  const int *choice, *inverse, *samples, *background;
+  int rows, inRows, C, batch, act, fs, chunks;
+  int waves; // wavefronts to a sample and 16 channels: 1, 2, 4 or 8
+  unsigned sampleBlocks, magic; // choice / C = (choice * magic >> 32) >> shift
+  int shift;
+};
+// the sum over the two lanes of a row of sixteen that lie eight apart
+__device__ __forceinline__ float sum_eights(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false)); // row_ror:8
+}
+// (the activation is the same for all: one branch)
+template <int V>
+__device__ __forceinline__ void pool_gradient_of(const PoolGradient &g, float (&d)[V], const float (&o)[V]) {
+  float none = 0.f;
+  if (!g.out)
+    return;
+  if (g.act == SCN_RELU) {
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      d[k] = act_derivative(SCN_RELU, o[k], d[k], 0.f, none);
+  } else {
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      d[k] = act_derivative(g.act, o[k], d[k], g.act == SCN_LEAKYRELU ? 0.01f : 0.333f, none);
+  }
+}
+// Bound by the lines it asks for: of a row the windows that are there and no others
+// (asked for all the same: rows alone 20.8 us and not 11.8), of a sample's windows 64
+// bytes a request (32: 19 us for the samples alone and not 12).  57456 x 32 of 116619
+// rows of 100 samples, side 3: 16.9 us, with 4 sums, where clearing, scattering and
+// k_background_sums take 7 + 23 + 7; 27157 x 64 of 57508 16.9, 31; 39071 x 32 of 203375
+// voxels of 32 samples, side 2, with 8 sums, 22, 42.
+template <int W, int FS>
+__global__ __launch_bounds__(512, W == 8 ? 4 : 8) void k_maxpool_gradient(PoolGradient g) {
+  constexpr int T = 512;
+  const int tid = threadIdx.x, C = g.C;
+  if (blockIdx.x < g.sampleBlocks) { // samples, eight lanes of two channels
+    constexpr int SUMS = 2 * (FS + 1), AHEAD = 4;
+    __shared__ float sSum[T / 16][8][SUMS]; // [row of sixteen lanes][lane][position, channel]
+    const int waves = g.waves, STEP = 8 * waves;
+    // (a wavefront's item is the same in all its lanes)
+    const int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (T / 64 / waves) + (tid >> 6) / waves);
+    const int sample = item / g.chunks, j = tid & 7;
+    const int c = item % g.chunks * 16 + 2 * j;
+    const bool there = sample < g.batch;
+    const int first = there ? g.samples[sample] : 0, end = there ? g.samples[sample + 1] : 0;
+    const int bg = there ? g.samples[g.batch + 1 + sample] : -1;
+    float acc[FS + 1][2] = {};
+    if (c < C)
+      for (int w = first + (tid % (64 * waves) >> 3); w < end; w += AHEAD * STEP) {
+        int ch[AHEAD][2];
+        float d[AHEAD][2], o[AHEAD][2];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+          const int wu = w + u * STEP < end ? w + u * STEP : w;
+          const size_t at = (size_t)wu * C + c;
+          const int2 cc = *reinterpret_cast<const int2 *>(g.choice + at);
+          const float2 dd = *reinterpret_cast<const float2 *>(g.dout + at);
+          const float2 oo = g.out ? *reinterpret_cast<const float2 *>(g.out + at) : dd;
+          ch[u][0] = w + u * STEP < end ? cc.x : -1, ch[u][1] = w + u * STEP < end ? cc.y : -1;
+          d[u][0] = dd.x, d[u][1] = dd.y, o[u][0] = oo.x, o[u][1] = oo.y;
+        }
+        int mask[AHEAD][2];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const int row = ch[u][k] >= 0 ? (int)(__umulhi((unsigned)ch[u][k], g.magic) >> g.shift) : -1;
+            ch[u][k] = row;
+            if (FS > 0) {
+              const bool in = row >= 0 && row < g.inRows;
+              const int m = g.background[in ? row : 0];
+              mask[u][k] = in ? m : 0;
+            }
+          }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+          pool_gradient_of<2>(g, d[u], o[u]);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            acc[FS][k] += ch[u][k] >= 0 && ch[u][k] == bg ? d[u][k] : 0.f;
+#pragma unroll
+            for (int f = 0; f < FS; ++f)
+              acc[f][k] += mask[u][k] >> f & 1 ? d[u][k] : 0.f;
+          }
+        }
+      }
+#pragma unroll
+    for (int f = 0; f <= FS; ++f)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float v = sum_eights(acc[f][k]);
+        if ((tid & 15) < 8)
+          sSum[tid >> 4][j][2 * f + k] = v;
+      }
+    __syncthreads();
+    // a sum to a lane: the item's wavefronts share them
+    for (int x = tid % (64 * waves); x < 8 * SUMS; x += 64 * waves) {
+      const int k = x & 1, q = x >> 1 & 7, f = x >> 4;
+      const int cc = item % g.chunks * 16 + 2 * q + k;
+      if (!there || cc >= C || (f < FS && f >= g.fs) || (f == FS && bg < 0))
+        continue;
+      const int row0 = (tid >> 6) / waves * waves * 4;
+      float sum = 0.f;
+      for (int y = 0; y < 4 * waves; ++y)
+        sum += sSum[row0 + y][q][2 * f + k];
+      const long long row = f == FS ? bg : g.inRows + (long long)sample * g.fs + f;
+      g.din[row * C + cc] = sum;
+    }
+    return;
+  }
+  // a row and four channels to a lane
+  const unsigned quads = C / 4;
+  const unsigned at = xcd_eighth(blockIdx.x - g.sampleBlocks, gridDim.x - g.sampleBlocks) * T + tid;
+  const unsigned r = at / quads;
+  if (r >= (unsigned)g.inRows)
+    return;
+  const int c = (int)(at - r * quads) * 4, flat = (int)(r * C) + c;
+  int w[W];
+  const int *const from = g.inverse + (size_t)r * W;
+  if constexpr (W % 4 == 0) {
+#pragma unroll
+    for (int j = 0; j < W; j += 4) {
+      const int4 x = *reinterpret_cast<const int4 *>(from + j);
+      w[j] = x.x, w[j + 1] = x.y, w[j + 2] = x.z, w[j + 3] = x.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      w[j] = from[j];
+  }
+  if (w[0] == -2) // a background row
+    return;
+  // (all windows are asked for together)
+  int4 ch[W];
+  float4 d[W], o[W];
+#pragma unroll
+  for (int j = 0; j < W; ++j) {
+    ch[j] = make_int4(-1, -1, -1, -1);
+    if (w[j] >= 0) {
+      const size_t x = (size_t)(unsigned)(w[j] * C + c);
+      ch[j] = *reinterpret_cast<const int4 *>(g.choice + x);
+      d[j] = *reinterpret_cast<const float4 *>(g.dout + x);
+      if (g.out)
+        o[j] = *reinterpret_cast<const float4 *>(g.out + x);
+    }
+  }
+  float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < W; ++j) {
+    float v[4] = {d[j].x, d[j].y, d[j].z, d[j].w};
+    const float y[4] = {o[j].x, o[j].y, o[j].z, o[j].w};
+    pool_gradient_of<4>(g, v, y);
+    const int t[4] = {ch[j].x, ch[j].y, ch[j].z, ch[j].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      sum[k] += t[k] == flat + k ? v[k] : 0.f;
+  }
+  *reinterpret_cast<float4 *>(g.din + (size_t)r * C + c) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+}
+extern "C" int scn_maxpool_gradient(scn_ctx *ctx, float *d_din, int64_t inputRows, const float *d_dout, int64_t rows,
+                                    int C, const int32_t *d_choice, const float *d_out, int act,
+                                    const int32_t *d_inverse, int slots, const int32_t *d_samples, int batch,
+                                    const int32_t *d_background, int fs) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_maxpool_gradient: null context");
+  SCN_REQUIRE(rows >= 0 && inputRows >= 0 && C >= 4 && C % 4 == 0 && batch >= 0, SCN_ERR_ARG,
+              "scn_maxpool_gradient: rows %lld of %lld C %d batch %d", (long long)rows, (long long)inputRows, C, batch);
+  SCN_REQUIRE(slots == 1 || slots == 2 || slots == 4 || slots == 8, SCN_ERR_ARG, "scn_maxpool_gradient: %d slots", slots);
+  SCN_REQUIRE(!d_background || (fs >= 1 && fs <= 8), SCN_ERR_ARG, "scn_maxpool_gradient: fs %d", fs);
+  SCN_REQUIRE(act >= SCN_NOSIGMOID && act <= SCN_SIGMOID && act != SCN_PRELU, SCN_ERR_ARG,
+              "scn_maxpool_gradient: activation %d", act);
+  SCN_REQUIRE(inputRows * C <= 0x7fffffffll && rows * C <= 0x7fffffffll, SCN_ERR_CAPACITY,
+              "scn_maxpool_gradient: %lld x %d", (long long)inputRows, C);
+  const int64_t sums = d_background ? (int64_t)batch * fs : 0;
+  if (inputRows + sums == 0)
+    return SCN_OK;
+  SCN_REQUIRE(d_din, SCN_ERR_ARG, "scn_maxpool_gradient: null d_din");
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  if (rows == 0)
+    return scn_fill32(ctx, d_din, 0, (size_t)(inputRows + sums) * C);
+  SCN_REQUIRE(d_dout && d_choice && d_samples && (d_inverse || inputRows == 0), SCN_ERR_ARG,
+              "scn_maxpool_gradient: null buffer");
+  SCN_REQUIRE((((uintptr_t)d_din | (uintptr_t)d_dout | (uintptr_t)d_choice | (uintptr_t)d_out | (uintptr_t)d_inverse) & 15) == 0,
+              SCN_ERR_ARG, "scn_maxpool_gradient: buffers start on 16 bytes");
+  PoolGradient g = {d_din, d_dout, d_out, d_choice, d_inverse, d_samples, d_background, (int)rows, (int)inputRows, C,
+                    batch, act, d_background ? fs : 0, scn_ceil_div(C, 16), 1, 0u, 0u, 0};
+  SCN_REQUIRE((int64_t)batch * g.chunks <= 0x3fffffffll, SCN_ERR_CAPACITY, "scn_maxpool_gradient: batch %d", batch);
+  // (32 windows to a wavefront and round)
+  while (g.waves < 8 && rows > 32ll * g.waves * batch)
+    g.waves *= 2;
+  g.sampleBlocks = (unsigned)scn_ceil_div((int64_t)batch * g.chunks, 8 / g.waves);
+  // x / C for x < 2^31: ceil(2^(31 + s) / C), s = ceil(log2 C)
+  int s = 0;
+  while ((1ll << s) < C)
+    ++s;
+  g.magic = (unsigned)(((1ull << (31 + s)) + C - 1) / C);
+  g.shift = s - 1;
+  const dim3 grid(g.sampleBlocks + (unsigned)scn_ceil_div(inputRows * (C / 4), 512));
+#define SCN_PG_GO(W, FS) hipLaunchKernelGGL((k_maxpool_gradient<W, FS>), grid, dim3(512), 0, ctx->stream, g)
+#define SCN_PG_FS(W)     \
+  if (g.fs == 0)         \
+    SCN_PG_GO(W, 0);     \
+  else if (g.fs <= 4)    \
+    SCN_PG_GO(W, 4);     \
+  else                   \
+    SCN_PG_GO(W, 8)
+  if (slots == 1) {
+    SCN_PG_FS(1);
+  } else if (slots == 2) {
+    SCN_PG_FS(2);
+  } else if (slots == 4) {
+    SCN_PG_FS(4);
+  } else {
+    SCN_PG_FS(8);
+  }
+#undef SCN_PG_FS
+#undef SCN_PG_GO
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 // dTerminalPoolBackProp: every row listed for a sample receives (not
 // accumulates) the sample's gradient divided by the number of rows listed.
 __global__ void k_terminal_backward(float *__restrict__ din,

@@ -90,6 +90,8 @@ public:
   PinnedStage hostFeatures;
   size_t hostFeatureCount;
   std::unique_ptr<BatchResultStage> result;
+  // an unseen training batch: its poolings' rules turned round, one behind the other
+  vectorCUDA<int> poolInverses;
   // SparseConvNetCUDA::backwardBatch: the layers' momentum steps, put off to the
   // end of the backward pass and queued together (elsewhere every layer queues its
   // own), and the products that they wait for

@@ -49,8 +49,15 @@ public:
   bool leftOut = false;
   vectorCUDA<int> inverse, background, positions;
   // rows of sub->dfeatures behind the layer's own: sums over the background of
-  // such a convolution's input
+  // such a convolution's input; they are there, or cleared for scn_background_sums
+  // to add to
   size_t gradientSums = 0;
+  bool sumsDone = false, sumsCleared = false;
+  // A pooling's output in such a batch: its rules turned round (scn_pool_inverse_many;
+  // in the batch's room for them, for as long as it is this batch), null: the
+  // gradient is scattered
+  const int *poolInverse = nullptr, *poolSamples = nullptr;
+  int poolSlots = 0;
   // Host view of the sparse grids.  Filled by the Pictures for the input
   // interface; for deeper interfaces the grids are built in HBM
   // (deviceGrids) and this view is only materialised by downloadGrids().

@@ -364,6 +364,9 @@ void SpatiallySparseBatchInterface::reset() {
   backpropErrors = false;
   leftOut = false;
   gradientSums = 0;
+  sumsDone = sumsCleared = false;
+  poolInverse = poolSamples = nullptr;
+  poolSlots = 0;
   inverse.resize(0);
   background.resize(0);
   positions.resize(0);
@@ -439,7 +442,7 @@ SpatiallySparseBatch::SpatiallySparseBatch(
       labels(false, 0),
       stagingSample(true, 0), stagingKey(true, 0), stagingRow(true, 0),
       stagingBackground(true, 0), hostSites(0), hostFeatureCount(0),
-      result(new BatchResultStage()) {
+      result(new BatchResultStage()), poolInverses(true, 0) {
   interfaces.emplace_back(inputSub);
   reset();
 }

@@ -462,8 +462,12 @@ static void conv_nin_gradients(cudaMemStream &ms, SpatiallySparseBatchInterface 
                           M, fs, nIn, N}, clean, later);
   if (!src.backpropErrors)
     return;
-  SCN_CHECKED(scn_background_sums(ms.ctx, output.sub->dfeatures.dPtr(), M, N,
-                                  middle.background.dPtr(), fs, batch.batchSize));
+  if (!output.sumsDone) {
+    if (!output.sumsCleared)
+      SCN_CHECKED(scn_fill32(ms.ctx, output.sub->dfeatures.dPtr() + (size_t)M * N, 0, output.gradientSums * N));
+    SCN_CHECKED(scn_background_sums(ms.ctx, output.sub->dfeatures.dPtr(), M, N,
+                                    middle.background.dPtr(), fs, batch.batchSize));
+  }
   src.sub->dfeatures.resize64(((size_t)src.nSpatialSites + src.gradientSums) * nIn);
   SCN_CHECKED(scn_conv_input_gradient(ms.ctx, output.sub->dfeatures.dPtr(), middle.inverse.dPtr(), fs, N,
                                       transposed.dPtr(), take_image(output.sub->turnedImage), src.sub->dfeatures.dPtr(), src.nSpatialSites, nIn));
@@ -857,14 +861,34 @@ static void pool_forwards(cudaMemStream &ms,
                                   output.sub->poolingChoices.dPtr()));
 }
 // MaxPoolingLayer::backwards (MaxPoolingLayer.cu:134-146)
+// (middle: where the layer before is one behind a convolution that was left out, that
+// convolution's output, whose background the gradient is summed over)
 static void pool_backwards(cudaMemStream &ms,
                            SpatiallySparseBatchInterface &input,
-                           SpatiallySparseBatchInterface &output) {
+                           SpatiallySparseBatchInterface &output,
+                           const SpatiallySparseBatch *batch = nullptr,
+                           SpatiallySparseBatchInterface *middle = nullptr) {
   if (!input.backpropErrors)
     return;
   const size_t nf = output.featuresPresent.size();
-  clear_gradient(ms, input, nf);
   vectorCUDA<float> &d = output.activationAhead ? output.sub->dactivated : output.sub->dfeatures;
+  if (batch && output.poolInverse) {
+    input.gradientCleared = false;
+    input.sub->dfeatures.resize64(((size_t)input.nSpatialSites + input.gradientSums) * nf);
+    const int fs = input.gradientSums ? (int)(input.gradientSums / batch->batchSize) : 0;
+    // (without the derivative, which the layer before takes in place, nothing is summed yet)
+    const bool sums = fs > 0 && fs <= 8 && middle && input.activationDone;
+    SCN_CHECKED(scn_maxpool_gradient(
+        ms.ctx, input.sub->dfeatures.dPtr(), input.nSpatialSites, d.dPtr(), output.nSpatialSites, (int)nf,
+        output.sub->poolingChoices.dPtr(), output.through >= 0 ? output.sub->features.dPtr() : nullptr,
+        output.through >= 0 ? output.through : (int)NOSIGMOID, output.poolInverse, output.poolSlots,
+        output.poolSamples, batch->batchSize, sums ? middle->background.dPtr() : nullptr, fs));
+    input.sumsDone = sums;
+    output.activationAhead = false;
+    output.through = -1;
+    return;
+  }
+  clear_gradient(ms, input, nf);
   if (output.through >= 0)
     SCN_CHECKED(scn_maxpool_backward_through(
         ms.ctx, input.sub->dfeatures.dPtr(), d.dPtr(), output.nSpatialSites, (int)nf,
@@ -880,8 +904,11 @@ void MaxPoolingLayer::backwards(SpatiallySparseBatch &batch,
                                 SpatiallySparseBatchInterface &input,
                                 SpatiallySparseBatchInterface &output,
                                 float learningRate, float momentum) {
-  (void)batch, (void)learningRate, (void)momentum;
-  pool_backwards(memStream, input, output);
+  (void)learningRate, (void)momentum;
+  // (interfaces: .. convolution's output, its input's gradient, this one's output ..)
+  const size_t i = &input - batch.interfaces.data();
+  SpatiallySparseBatchInterface *middle = i > 0 ? &batch.interfaces[i - 1] : nullptr;
+  pool_backwards(memStream, input, output, &batch, middle && middle->deferredGatherFrom ? middle : nullptr);
 }
 void MaxPoolingLayer::forwards(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &input,

@@ -457,11 +457,18 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
     if (i == 0 || !batch.interfaces[i - 1].deferredGatherFrom)
       input.gradientSums = 0;
     const size_t own = (size_t)input.nSpatialSites * nf, sums = input.gradientSums * nf;
-    input.gradientCleared = layers[i]->addsInputGradient() && input.backpropErrors &&
+    // (a pooling whose rules are turned round writes the whole gradient, and the sums
+    // where it takes the activation's derivative)
+    const bool writes = batch.interfaces[i + 1].poolInverse;
+    input.gradientCleared = layers[i]->addsInputGradient() && input.backpropErrors && !writes &&
                             !batch.interfaces[i + 1].deferredGatherFrom;
+    input.sumsDone = false;
+    input.sumsCleared = sums && !writes;
     if (!input.gradientCleared && !sums)
       continue;
     input.sub->dfeatures.resize64(own + sums);
+    if (writes)
+      continue;
     sizes[n] = input.gradientCleared ? own + sums : sums;
     grads[n++] = input.sub->dfeatures.dPtr() + (input.gradientCleared ? 0 : own);
     if (n == SCN_FILL_MAX) {
@@ -1049,6 +1056,43 @@ static void leaveOutConvolutions(SparseConvNetCUDA &cnn, scn_ctx *ctx, Spatially
   for (size_t i = 0; i < items.size(); i += SCN_INVERSE_MAX)
     SCN_CHECKED(scn_rules_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
 }
+// ... and its poolings' rules turned round, where their windows overlap little: a
+// gradient that is read by rows and written once.  (A sample's windows are walked by
+// a workgroup for its background row: some 2 us for every 512 of them.)
+static void turnPoolings(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBatch &b) {
+  std::vector<scn_pool_inverse_item> items;
+  std::vector<SpatiallySparseBatchInterface *> outs;
+  auto room = [](size_t n) { return (n + 3) & ~(size_t)3; };
+  size_t total = 0;
+  for (size_t i = 0; i < cnn.layers.size(); ++i) {
+    MaxPoolingLayer *const pool = dynamic_cast<MaxPoolingLayer *>(cnn.layers[i]);
+    SpatiallySparseBatchInterface &in = b.interfaces[i], &out = b.interfaces[i + 1];
+    if (!pool || !in.backpropErrors)
+      continue;
+    const int slots = scn_pool_inverse_slots(pool->dimension, pool->poolSize, pool->poolStride);
+    const int64_t nf = (int64_t)out.featuresPresent.size();
+    if (slots == 0 || nf % 4 != 0 || nf == 0 || in.nSpatialSites * std::max<int64_t>(nf, slots) > 0x7fffffffll ||
+        out.nSpatialSites * nf > 0x7fffffffll || out.nSpatialSites > 2048ll * b.batchSize)
+      continue;
+    out.poolSlots = slots;
+    items.push_back({in.deviceGrids, out.deviceGrids, out.rules.dPtr(), nullptr, nullptr, out.nSpatialSites,
+                     in.nSpatialSites, pool->poolSize, pool->poolStride});
+    outs.push_back(&out);
+    total += room((size_t)in.nSpatialSites * slots) + room(2 * (size_t)b.batchSize + 1);
+  }
+  b.poolInverses.resize64(total);
+  int *at = b.poolInverses.dPtr();
+  for (size_t k = 0; k < items.size(); ++k) {
+    items[k].d_inverse = at;
+    at += room((size_t)items[k].inputRows * outs[k]->poolSlots);
+    items[k].d_samples = at;
+    at += room(2 * (size_t)b.batchSize + 1);
+    outs[k]->poolInverse = items[k].d_inverse;
+    outs[k]->poolSamples = items[k].d_samples;
+  }
+  for (size_t i = 0; i < items.size(); i += SCN_INVERSE_MAX)
+    SCN_CHECKED(scn_pool_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
+}
 // GPU half: the input grids go to HBM, then every layer builds its rule book,
 // all on the slot's stream
 void BatchProducer::preprocessBatchOnDevice(int cc) {
@@ -1089,8 +1133,10 @@ void BatchProducer::preprocessBatchOnDevice(int cc) {
     b.labels.copyToGPUAsync(ms);
   }
   buildRuleBooks(cnn, ctx, b);
-  if (b.unseen)
+  if (b.unseen) {
     leaveOutConvolutions(cnn, ctx, b);
+    turnPoolings(cnn, ctx, b);
+  }
   SCN_CHECKED(scn_sync(ctx));
 }
 void BatchProducer::batchProducerThread(int nThread) {

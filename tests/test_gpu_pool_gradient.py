@@ -1,0 +1,99 @@
+"""The gradient of a pooling's input by rows, through its rules turned round, and with it the sums over the background of
+the convolution before: against the scatter that the choices stand for, in float64."""
+import numpy as np
+import pytest
+
+from test_gpu_conv_backward import layer
+
+pytestmark = pytest.mark.gpu
+
+
+# one, two, four and eight windows to a row; a sample without sites and a full one (whose pooling's output is full, too);
+# a channel group of 16 that is not whole, rows that are no whole workgroups; more windows a sample than are asked for at
+# once (2-D, 90: a full sample has 1936); sums over 1, 4 and 8 positions, and none
+@pytest.mark.parametrize("d,field,window,size,stride,batch,density,C,act", [
+    (2, 10, 2, 3, 2, 4, 0.2, 32, "RELU"), (2, 9, 2, 2, 2, 5, 0.1, 4, "NOSIGMOID"), (3, 9, 2, 2, 2, 4, 0.05, 36, "RELU"),
+    (3, 8, 2, 3, 2, 3, 0.1, 20, "LEAKYRELU"), (2, 8, 2, 2, 1, 3, 0.3, 64, None), (1, 20, 2, 3, 2, 6, 0.2, 12, "TANH"),
+    (2, 90, 2, 3, 2, 3, 0.1, 32, "RELU"), (2, 9, 1, 3, 3, 4, 0.3, 300, "RELU"), (2, 14, 3, 2, 2, 40, 0.02, 32, "RELU")])
+def test_pool_gradient(scn, ctx, d, field, window, size, stride, batch, density, C, act):
+    rng = np.random.default_rng(field * size + C)
+    g, n, _, fs, _, bg = layer(scn, ctx, d, field, window, batch, density, field + C)
+    h, p = scn.Grids(ctx), scn.Grids(ctx)
+    mid = field - window + 1
+    inRows = g.plan_square(h, field, mid, window, 1)
+    d_conv = ctx.empty((inRows, fs), np.int32)
+    g.fill(h, d_conv, inRows * fs)
+    out = (mid - size) // stride + 1
+    width = size ** d
+    rows = h.plan_square(p, mid, out, size, stride)
+    d_rules = ctx.empty((rows, width), np.int32)
+    h.fill(p, d_rules, rows * width)
+    slots = scn.lib().scn_pool_inverse_slots(d, size, stride)
+    assert slots == (-(-size // stride)) ** d
+    print("pool gradient", d, field, window, size, stride, batch, C, "rows", rows, "of", inRows, flush=True)
+    x = rng.standard_normal((inRows, C), dtype=np.float32)
+    y, choice = ctx.empty((rows, C), np.float32), ctx.empty((rows, C), np.int32)
+    ctx.maxpool(ctx.array(x), y, d_rules, rows, width, C, choice)
+    D = rng.standard_normal((rows, C), dtype=np.float32)
+    inverse, samples = ctx.array(np.full((inRows, slots), 7, np.int32)), ctx.array(np.full(2 * batch + 1, 7, np.int32))
+    ctx.pool_inverse_many([(h, p, d_rules, inverse, samples, rows, inRows, size, stride)])
+    rules = d_rules.download().astype(np.int64)
+    got = samples.download()
+    inBg = got[batch + 1:]
+    assert got[0] == 0 and got[batch] == rows and np.all(np.diff(got[:batch + 1]) >= 0)
+    isBg = np.zeros(inRows, bool)
+    isBg[inBg[inBg >= 0]] = True
+    inv = inverse.download()
+    assert np.all(inv[isBg] == -2)
+    for r in rng.choice(np.nonzero(~isBg)[0], min(200, int((~isBg).sum())), replace=False):
+        assert sorted(w for w in inv[r] if w >= 0) == sorted(np.nonzero((rules == r).any(1))[0])
+    for s in range(batch):  # the windows that name a sample's background lie in its range
+        named = np.nonzero((rules == inBg[s]).any(1))[0] if inBg[s] >= 0 else []
+        assert all(got[s] <= w < got[s + 1] for w in named)
+    # the gradient, with and without sums
+    ch, v = choice.download().astype(np.int64), D.astype(np.float64)
+    o = y.download().astype(np.float64)
+    if act == "RELU":
+        v = v * (o > 0)
+    elif act == "LEAKYRELU":
+        v = np.where(o > 0, v, v * 0.01)
+    elif act == "TANH":
+        v = v * (1 + o) * (1 - o)
+    want, size_of = np.zeros(inRows * C), np.zeros(inRows * C)
+    np.add.at(want, ch[ch >= 0], v[ch >= 0])
+    np.add.at(size_of, ch[ch >= 0], np.abs(v[ch >= 0]))
+    want, size_of = want.reshape(inRows, C), size_of.reshape(inRows, C)
+    background = ctx.empty(inRows + 2 * batch, np.int32)
+    convInverse = ctx.empty((n, fs), np.int32)
+    ctx.rules_inverse_many([(g, d_conv, convInverse, background, None, inRows, n, fs)])
+    mask = background.download()[:inRows]
+    first = np.searchsorted(np.arange(rows), got[:batch + 1])
+    sums, sums_of = np.zeros((batch * fs, C)), np.zeros((batch * fs, C))
+    for s in range(batch):
+        w = slice(first[s], first[s + 1])
+        row, col = np.where(ch[w] >= 0, ch[w] // C, 0), np.broadcast_to(np.arange(C), ch[w].shape)
+        for f in range(fs):
+            hit = (ch[w] >= 0) & ((mask[row] >> f) & 1 == 1)
+            np.add.at(sums[s * fs + f], col[hit], v[w][hit])
+            np.add.at(sums_of[s * fs + f], col[hit], np.abs(v[w][hit]))
+    for withSums in (False, True) if fs <= 8 else (False,):
+        din = ctx.array(np.full((inRows + batch * fs, C), 7, np.float32))
+        ctx.maxpool_gradient(din, inRows, ctx.array(D), rows, C, choice, y if act else None,
+                             getattr(scn, act) if act else scn.NOSIGMOID, inverse, slots, samples, batch,
+                             background if withSums else None, fs if withSums else 0)
+        res = din.download()
+        # (the sums' longest chain: a lane's windows, six shuffles, eight wavefronts)
+        assert np.all(np.abs(res[:inRows] - want) <= 4e-6 * size_of + 1e-30)
+        assert np.all(res[inRows:] == 7) if not withSums else np.all(np.abs(res[inRows:] - sums) <= 4e-6 * sums_of + 1e-30)
+
+
+def test_pool_gradient_refusals(scn, ctx):
+    f = scn.lib().scn_pool_inverse_slots
+    assert [f(2, 3, 1), f(3, 3, 1), f(2, 4, 2), f(3, 4, 2), f(0, 2, 2), f(2, 2, 0)] == [0, 0, 4, 8, 0, 0]
+    b, i = ctx.empty((64, 64), np.float32), ctx.empty((64, 64), np.int32)
+    for kw in (dict(C_=6), dict(slots=3), dict(act=scn.PRELU), dict(fs=9, d_background=i)):
+        a = dict(d_din=b, inputRows=4, d_dout=b, rows=4, C_=4, d_choice=i, d_out=None, act=scn.NOSIGMOID, d_inverse=i, slots=1,
+                 d_samples=i, batch=1)
+        a.update(kw)
+        with pytest.raises(scn.ScnError):
+            ctx.maxpool_gradient(**a)
