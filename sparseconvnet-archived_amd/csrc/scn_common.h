@@ -210,3 +210,6 @@ int scn_scan_exclusive_u32(hipStream_t s, const uint32_t *in, uint32_t *out,
 // same, over popcounts of 64-bit words
 int scn_scan_exclusive_popc64(hipStream_t s, const uint64_t *words,
                               uint32_t *out, size_t n, uint32_t *tmp, bool cleared = false);
+// two of these at once, their states cleared
+int scn_scan_exclusive_popc64_pair(hipStream_t s, const uint64_t *wordsA, uint32_t *outA, size_t nA, uint32_t *tmpA,
+                                   const uint64_t *wordsB, uint32_t *outB, size_t nB, uint32_t *tmpB);

@@ -96,13 +96,29 @@ __global__ void __launch_bounds__(256) k_grid_build(GridView g, const int *sampl
     atomicOr(&g.bits[word], (unsigned long long)hi << 32 | lo);
 }
 
+struct RankRows {
+  const long long *ekey;
+  const int *erow;
+  Count n;
+  const long long *meta;
+  int *rankRow; // null: not wanted
+};
+// the rows by rank from the entry list
+__device__ __forceinline__ void rank_rows_body(const GridView &g, const RankRows &a, long long block) {
+  const long long e = xcd_contiguous_block(block, (count_now(a.n) + 255) / 256) * 256 + threadIdx.x;
+  if (e >= a.n.bound || (a.meta && a.meta[META_OVERFLOW]) || e >= count_now(a.n))
+    return;
+  a.rankRow[rank_of(g, a.ekey[e])] = a.erow[e];
+}
+
 // pass 1: number of output sites owned by each input, stored at the input's
 // position in iteration order
 template <int D>
 __global__ void k_plan_count(GridView in, Geom g, const long long *ekey,
                              Count nEntries, const long long *inMeta,
                              unsigned *cntByRank, unsigned long long *ownMask,
-                             unsigned *rankOf, ScanState scan) {
+                             unsigned *rankOf, ScanState scan,
+                             const int *erow, int *rankRow) {
   scan.clear((size_t)blockIdx.x * blockDim.x + threadIdx.x);
   long long e = xcd_contiguous_block((count_now(nEntries) + 255) / 256) * blockDim.x + threadIdx.x;
   if (e >= nEntries.bound)
@@ -117,7 +133,7 @@ __global__ void k_plan_count(GridView in, Geom g, const long long *ekey,
   }
   long long p = ekey[e];
   int i[D];
-  const int b = split_site<D>(p, g.volIn, g.nIn, i);
+  const int b = split_site<D>(p, g.volIn, g.nIn, g.divIn, i);
   unsigned n = 0;
   unsigned long long mask = 0;
   bool done = false;
@@ -147,6 +163,8 @@ __global__ void k_plan_count(GridView in, Geom g, const long long *ekey,
     });
   unsigned r = rank_of(in, p);
   cntByRank[r] = n;
+  if (rankRow) // the rows by rank, which the rule book is filled from (k_rank_rows)
+    rankRow[r] = erow[e];
   if (ownMask) { // only when a box never has more than 64 candidates
     ownMask[e] = mask; // kept per entry, with the rank, so that the emit pass
     rankOf[e] = r;     // reads them without walking the mask again
@@ -253,41 +271,6 @@ plan_samples_body(const GridView &in, const unsigned *base, long long nEntries,
   }
 }
 
-template <bool OWNERS>
-__global__ void __launch_bounds__(SCAN1_THREADS)
-    k_plan_samples(GridView in, const unsigned *base, long long nEntries,
-                   long long fullSize, int *outBg, int *bgBefore,
-                   unsigned *sampleStart, long long *scalars,
-                   const long long *badSites, long long ticket, long long *meta,
-                   const long long *inMeta, long long boundRows,
-                   long long boundActive, int pinnedSlot) {
-  unsigned rs0, re0;
-  sample_ranks(in, rs0, re0);
-  plan_samples_body<OWNERS>(in, base, nEntries, fullSize, outBg, bgBefore, sampleStart,
-                            scalars, badSites, ticket, meta, inMeta, boundRows,
-                            boundActive, pinnedSlot, rs0, re0);
-}
-
-// small batches: prefix sum of the owned counts and the per-sample pass in
-// one launch
-__global__ void __launch_bounds__(SCAN1_THREADS)
-    k_plan_scan_samples(GridView in, const unsigned *cnt, unsigned *base,
-                        long long nEntries, long long fullSize, int *outBg,
-                        int *bgBefore, unsigned *sampleStart,
-                        long long *scalars, const long long *badSites,
-                        long long ticket, long long *meta,
-                        const long long *inMeta, long long boundRows,
-                        long long boundActive, int pinnedSlot) {
-  __shared__ uint32_t ldsScan[SCAN1_LDS_WORDS];
-  unsigned rs0, re0;
-  sample_ranks(in, rs0, re0);
-  (void)block_scan_loop<false>(cnt, base, (size_t)nEntries, ldsScan);
-  __syncthreads(); // the block's own writes to base[] are visible to it
-  plan_samples_body(in, base, nEntries, fullSize, outBg, bgBefore, sampleStart,
-                    scalars, badSites, ticket, meta, inMeta, boundRows,
-                    boundActive, pinnedSlot, rs0, re0);
-}
-
 // pass 2: emit the owned outputs
 template <int D>
 __global__ void k_plan_emit(GridView in, GridView out, Geom g,
@@ -309,7 +292,7 @@ __global__ void k_plan_emit(GridView in, GridView out, Geom g,
     return;
   long long p = ekey[e];
   int i[D];
-  const int b = split_site<D>(p, g.volIn, g.nIn, i);
+  const int b = split_site<D>(p, g.volIn, g.nIn, g.divIn, i);
   unsigned idx = base[rank_of(in, p)];
   const int shiftRows = bgBefore[b];
   for_each_owned<D>(in, g, b, i, [&](long long outKey, int) {
@@ -358,7 +341,7 @@ __global__ void k_plan_emit_masked(GridView in, GridView out, Geom g,
   if (!((mask >> c) & 1ull))
     return;
   int i[D], lo[D], hi[D], j[D];
-  const int b = split_site<D>(p, g.volIn, g.nIn, i);
+  const int b = split_site<D>(p, g.volIn, g.nIn, g.divIn, i);
   (void)cand_box<D>(g, b, i, lo, hi);
   int rem = c;
 #pragma unroll
@@ -467,7 +450,7 @@ __global__ void __launch_bounds__(256)
     if (mask) {
       WalkItem &it = items[threadIdx.x];
       int i[D], lo[D], hi[D];
-      const int b = split_site<D>(p, g.volIn, g.nIn, i);
+      const int b = split_site<D>(p, g.volIn, g.nIn, g.divIn, i);
       (void)cand_box<D>(g, b, i, lo, hi);
       // a box is at most 64 candidates, so its sides are small: x / ext by a
       // multiplication (exact for x < 64: the error of the factor stays below 1 / 64 ext)
@@ -568,13 +551,20 @@ __device__ __forceinline__ unsigned long long even_bits(unsigned long long x) {
 }
 // S: the window's side when it is 2 or 3 (the loops over a window's rows unroll and all its rows are requested at
 // once), else 0 (read from g)
+struct Dilate {
+  unsigned long long *outBits;
+  long long nWords, totalBits;
+  ScanState rank;
+  unsigned blocks;
+};
 template <int D, int S>
-__global__ void __launch_bounds__(256)
-    k_mask_dilate(GridView in, Geom g, unsigned long long *outBits,
-                  long long nWords, long long totalBits, ScanState rank) {
+__device__ __forceinline__ void mask_dilate_body(const GridView &in, const Geom &g, const Dilate &to, long long block) {
+  unsigned long long *const outBits = to.outBits;
+  const long long nWords = to.nWords, totalBits = to.totalBits;
+  const ScanState rank = to.rank;
   // (runs of blocks to one XCD: the rows and planes a word's windows reach into
   // are the ones its neighbours in the same L2 have just read)
-  const long long w = xcd_contiguous_block((nWords + 255) / 256) * blockDim.x + threadIdx.x;
+  const long long w = xcd_contiguous_block(block, (nWords + 255) / 256) * 256 + threadIdx.x;
   if (w >= nWords)
     return;
   rank.clear((size_t)w);
@@ -586,7 +576,7 @@ __global__ void __launch_bounds__(256)
   // a piece reads (len - 1) stride + size input bits: at most 128
   const int lenMax = g.stride == 1 ? 64 : (128 - size) / g.stride + 1;
   int j[D];
-  int b = split_site<D>(pos, g.volOut, g.nOut, j);
+  int b = split_site<D>(pos, g.volOut, g.nOut, g.divOut, j);
   while (pos < end) {
     long long len = g.nOut - j[D - 1];
     len = len < end - pos ? len : end - pos;
@@ -703,6 +693,55 @@ __global__ void __launch_bounds__(256)
   }
   outBits[w] = res;
 }
+// The output's mask, and beside it what needs no more than a few workgroups: the
+// per-sample pass of k_plan_samples (KIND 0), the same over an owners' mask (1) or
+// behind a short scan (2, k_plan_scan_samples), and the rows by rank of the input.
+// By themselves these are 5.5 and 5 to 8 us in which most of the chip idles (40
+// samples of 126^3 lattice sites, 460 000 and 1.38 million of them active).  Eight
+// blocks for the samples, of which one works, so that the others keep their XCDs.
+struct PlanSamples {
+  GridView in; // (KIND 1: the owners' mask and its prefix)
+  unsigned *cnt, *base;
+  long long nEntries, fullSize;
+  int *outBg, *bgBefore;
+  unsigned *sampleStart;
+  long long *scalars;
+  const long long *badSites;
+  long long ticket;
+  long long *meta;
+  const long long *inMeta;
+  long long boundRows, boundActive;
+  int pinnedSlot;
+};
+template <int KIND> __device__ __forceinline__ void plan_samples_block(const PlanSamples &a) {
+  unsigned rs0, re0;
+  sample_ranks(a.in, rs0, re0);
+  if constexpr (KIND == 2) {
+    __shared__ uint32_t ldsScan[SCAN1_LDS_WORDS];
+    (void)block_scan_loop<false>(a.cnt, a.base, (size_t)a.nEntries, ldsScan);
+    __syncthreads(); // the block's own writes to base[] are visible to it
+  }
+  plan_samples_body<KIND == 1>(a.in, a.base, a.nEntries, a.fullSize, a.outBg, a.bgBefore, a.sampleStart, a.scalars,
+                               a.badSites, a.ticket, a.meta, a.inMeta, a.boundRows, a.boundActive, a.pinnedSlot, rs0, re0);
+}
+template <int KIND> __global__ void __launch_bounds__(SCAN1_THREADS) k_plan_samples(PlanSamples a) {
+  plan_samples_block<KIND>(a);
+}
+template <int D, int S, int KIND>
+__global__ void __launch_bounds__(SCAN1_THREADS)
+    k_plan_dilate(GridView in, Geom g, Dilate to, PlanSamples samples, RankRows rows) {
+  static_assert(SCAN1_THREADS == 256, "the dilation's");
+  if (blockIdx.x < 8) {
+    if (blockIdx.x == 0)
+      plan_samples_block<KIND>(samples);
+    return;
+  }
+  const unsigned block = blockIdx.x - 8;
+  if (block < to.blocks)
+    mask_dilate_body<D, S>(in, g, to, block);
+  else
+    rank_rows_body(in, rows, block - to.blocks);
+}
 
 // Windows of side 2 that tile the field (stride 2, no minimum): every input
 // lies in one window, a window's sites along the last axis are an even bit of
@@ -733,7 +772,7 @@ __global__ void __launch_bounds__(256)
   if (X) {
     const unsigned long long EVEN = 0x5555555555555555ull;
     int i[D];
-    (void)split_site<D>(pos, g.volIn, g.nIn, i);
+    (void)split_site<D>(pos, g.volIn, g.nIn, g.divIn, i);
     const long long plane = (long long)g.nIn * g.nIn;
     while (pos < end) {
       long long len = g.nIn - i[D - 1];
@@ -809,7 +848,7 @@ __global__ void __launch_bounds__(256)
   const long long w0 = w - lane; // the wavefront's first word, which exists as total > 0
   const unsigned idx0 = ownPrefix[w0];
   int i0[D];
-  const int b0 = split_site<D>(64 * w0, g.volIn, g.nIn, i0);
+  const int b0 = split_site<D>(64 * w0, g.volIn, g.nIn, g.divIn, i0);
   for (unsigned o = lane; o < total; o += 64) {
     const int l = wave_deal_find(sBefore + first, o);
     unsigned carry =
@@ -1406,14 +1445,7 @@ __global__ void k_grid_index(GridView g, const long long *ekey, const int *erow,
   const long long p = ekey[e];
   atomicOr(&g.bits[p >> 6], 1ull << (p & 63));
 }
-// the rows by rank from the entry list
-__global__ void k_rank_rows(GridView g, const long long *ekey, const int *erow,
-                            Count n, const long long *meta, int *rankRow) {
-  long long e = xcd_contiguous_block((count_now(n) + 255) / 256) * blockDim.x + threadIdx.x;
-  if (e >= n.bound || (meta && meta[META_OVERFLOW]) || e >= count_now(n))
-    return;
-  rankRow[rank_of(g, ekey[e])] = erow[e];
-}
+__global__ void k_rank_rows(GridView g, RankRows rows) { rank_rows_body(g, rows, blockIdx.x); }
 // the look-up table (dense rows or hash) from the entry list
 __global__ void k_grid_table(GridView g, const long long *ekey, const int *erow,
                              Count n, const long long *meta) {
@@ -1452,30 +1484,42 @@ static int ensure_index(scn_ctx *ctx, scn_grids *g) {
   return SCN_OK;
 }
 
+// mask and rank prefix
+static int ensure_prefix(scn_ctx *ctx, scn_grids *g) {
+  SCN_TRY(ensure_index(ctx, g));
+  if (g->rankValid)
+    return SCN_OK;
+  const bool cleared = g->rankStateFor == g->nWords + 1; // (by the kernel that wrote or cleared the mask)
+  g->rankStateFor = 0;
+  SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
+  // one word past the mask so that the rank of the end position is defined
+  SCN_TRY(scn_scan_exclusive_popc64(ctx->stream,
+                                    (const uint64_t *)g->bits.p, g->prefix.p,
+                                    g->nWords + 1, g->scanTmp.p, cleared));
+  g->rankValid = true;
+  return SCN_OK;
+}
+// the rows by rank that are still to be written (rankRow null: none)
+static int missing_rank_rows(scn_grids *g, RankRows *rows) {
+  *rows = RankRows{g->ekey.p, g->erow.p, count_active(g), g->pending ? g->meta.p : nullptr, nullptr};
+  if (g->rankRowValid)
+    return SCN_OK;
+  SCN_TRY(g->rankRow.reserve((size_t)g->nActive + 4));
+  if (g->nActive > 0)
+    rows->rankRow = g->rankRow.p;
+  return SCN_OK;
+}
 // mask, rank prefix and rows by rank: what a rule book needs of its input
 static int ensure_rank(scn_ctx *ctx, scn_grids *g) {
-  SCN_TRY(ensure_index(ctx, g));
-  if (!g->rankValid) {
-    const bool cleared = g->rankStateFor == g->nWords + 1; // (by the kernel that wrote or cleared the mask)
-    g->rankStateFor = 0;
-    SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
-    // one word past the mask so that the rank of the end position is defined
-    SCN_TRY(scn_scan_exclusive_popc64(ctx->stream,
-                                      (const uint64_t *)g->bits.p, g->prefix.p,
-                                      g->nWords + 1, g->scanTmp.p, cleared));
-    g->rankValid = true;
+  SCN_TRY(ensure_prefix(ctx, g));
+  RankRows rows;
+  SCN_TRY(missing_rank_rows(g, &rows));
+  if (rows.rankRow) {
+    hipLaunchKernelGGL(k_rank_rows, dim3(xcd_grid(scn_ceil_div(g->nActive, 256))), dim3(256), 0, ctx->stream,
+                       view_of(g), rows);
+    SCN_HIP_CHECK(hipGetLastError());
   }
-  if (!g->rankRowValid) {
-    SCN_TRY(g->rankRow.reserve((size_t)g->nActive + 4));
-    if (g->nActive > 0) {
-      hipLaunchKernelGGL(k_rank_rows, dim3(xcd_grid(scn_ceil_div(g->nActive, 256))),
-                         dim3(256), 0, ctx->stream, view_of(g), g->ekey.p,
-                         g->erow.p, count_active(g),
-                         g->pending ? g->meta.p : nullptr, g->rankRow.p);
-      SCN_HIP_CHECK(hipGetLastError());
-    }
-    g->rankRowValid = true;
-  }
+  g->rankRowValid = true;
   return SCN_OK;
 }
 
@@ -1840,10 +1884,22 @@ static bool tile2_enabled() {
   return on;
 }
 
+static FieldDivisors field_divisors(int batch, long long vol, int n) {
+  const FieldDivisors none = {{0, 0}, {0, 0}};
+  // (64 positions more: a lane past the end of the mask takes its word apart too)
+  return batch > 0 && vol <= (1ll << 31) && (long long)batch * vol + 256 < (1ll << 31)
+             ? FieldDivisors{divisor_of(vol), divisor_of(n)}
+             : none;
+}
+// What a plan of `in` needs of it.  The rows by rank are written on the way: by the
+// pass over its entries, or beside the dilation where there is none (tiled).
 template <int D>
 static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
-                          const Geom &g, long long fullSize,
+                          const Geom &geom, long long fullSize,
                           int64_t *nOutSites, long long fmpCand = 0) {
+  Geom g = geom;
+  g.divIn = field_divisors(in->batch, g.volIn, g.nIn);
+  g.divOut = field_divisors(in->batch, g.volOut, g.nOut);
   // deferred: size by bounds, leave the counts on the device (see scn_rules_settle)
   const bool deferred = ctx->deferCounts && out->seenRows > 0 &&
                         (int)ctx->pendingGrids.size() < SCN_MAX_PENDING;
@@ -1872,6 +1928,9 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   SCN_TRY(grids_check(in->batch, g.d, g.nOut));
   out->rankStateFor = 0;
   SCN_TRY(out->scanTmp.reserve(scn_scan_tmp_elems(std::max((size_t)nE + 1, dilated ? outWords + 1 : 0))));
+  RankRows rows;
+  SCN_TRY(ensure_index(ctx, in));
+  SCN_TRY(missing_rank_rows(in, &rows));
   GridView vin = view_of(in);
   // number of candidates of one input: (ceil(size / stride))^d at most
   long long maxCand = 1;
@@ -1894,59 +1953,86 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
                        ownWords, (long long)in->batch * g.volIn,
                        scn_scan_state((size_t)ownWords, out->scanTmp.p));
     SCN_HIP_CHECK(hipGetLastError());
-  } else if (masked) {
-    SCN_TRY(out->ownMask.reserve((size_t)nE + 2));
-    SCN_TRY(out->rankOf.reserve((size_t)nE + 2));
+  } else {
+    SCN_TRY(ensure_prefix(ctx, in));
+    if (masked) {
+      SCN_TRY(out->ownMask.reserve((size_t)nE + 2));
+      SCN_TRY(out->rankOf.reserve((size_t)nE + 2));
+    }
   }
   if (nE > 0 && !tiled) {
     hipLaunchKernelGGL(k_plan_count<D>, dim3(xcd_grid(scn_ceil_div(nE, 256))), dim3(256),
                        0, ctx->stream, vin, g, in->ekey.p, nEc, inMeta, out->cnt.p,
                        masked ? out->ownMask.p : nullptr, out->rankOf.p,
-                       scn_scan_state((size_t)nE, out->scanTmp.p));
+                       scn_scan_state((size_t)nE, out->scanTmp.p), rows.erow, rows.rankRow);
     SCN_HIP_CHECK(hipGetLastError());
+    in->rankRowValid = true;
   }
   const long long *bad = (const long long *)(ctx->d_scalars + 15);
   const long long ticket = ++ctx->ticket;
+  PlanSamples samples = {vin, out->cnt.p, out->base.p, nE, fullSize, out->bg.p, out->bgBefore.p, out->sampleStart.p,
+                         (long long *)ctx->d_pinned, bad, ticket, out->meta.p, inMeta, boundRows, boundActive, slot};
+  int kind = 0;
   if (tiled) {
-    SCN_TRY(scn_scan_exclusive_popc64(ctx->stream, (const uint64_t *)out->ownMask.p,
-                                      out->base.p, (size_t)ownWords, out->scanTmp.p, true));
-    GridView owners = vin;
-    owners.bits = out->ownMask.p;
-    owners.prefix = out->base.p;
-    hipLaunchKernelGGL(k_plan_samples<true>, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream,
-                       owners, (const unsigned *)nullptr, 0ll, fullSize, out->bg.p,
-                       out->bgBefore.p, out->sampleStart.p, (long long *)ctx->d_pinned, bad,
-                       ticket, out->meta.p, inMeta, boundRows, boundActive, slot);
+    // (the input's ranks wait until now, for one launch with the owners' ones)
+    const bool both = !in->rankValid && in->rankStateFor == in->nWords + 1;
+    if (both) {
+      SCN_TRY(scn_scan_exclusive_popc64_pair(ctx->stream, (const uint64_t *)out->ownMask.p, out->base.p, (size_t)ownWords,
+                                             out->scanTmp.p, (const uint64_t *)in->bits.p, in->prefix.p, in->nWords + 1,
+                                             in->scanTmp.p));
+      in->rankStateFor = 0;
+      in->rankValid = true;
+    } else {
+      SCN_TRY(scn_scan_exclusive_popc64(ctx->stream, (const uint64_t *)out->ownMask.p,
+                                        out->base.p, (size_t)ownWords, out->scanTmp.p, true));
+      SCN_TRY(ensure_prefix(ctx, in));
+    }
+    samples.in.bits = out->ownMask.p;
+    samples.in.prefix = out->base.p;
+    samples.nEntries = 0;
+    kind = 1;
   } else if ((size_t)nE <= SCAN1_MAX_ELEMS) {
-    hipLaunchKernelGGL(k_plan_scan_samples, dim3(1), dim3(SCAN1_THREADS), 0,
-                       ctx->stream, vin, out->cnt.p, out->base.p, nE, fullSize,
-                       out->bg.p, out->bgBefore.p, out->sampleStart.p,
-                       (long long *)ctx->d_pinned, bad, ticket, out->meta.p,
-                       inMeta, boundRows, boundActive, slot);
+    kind = 2;
   } else {
     SCN_TRY(scn_scan_exclusive_u32(ctx->stream, out->cnt.p, out->base.p,
                                    (size_t)nE, out->scanTmp.p, true));
-    hipLaunchKernelGGL(k_plan_samples<false>, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream, vin,
-                       out->base.p, nE, fullSize, out->bg.p, out->bgBefore.p,
-                       out->sampleStart.p, (long long *)ctx->d_pinned, bad, ticket, out->meta.p,
-                         inMeta, boundRows, boundActive, slot);
   }
-  SCN_HIP_CHECK(hipGetLastError());
   size_t rankStateFor = 0;
   if (dilated) {
     // (needs no count: runs while the host waits for them.  It also clears the
     // state of the scan that gives the mask its ranks)
     SCN_TRY(out->bits.reserve(outWords + 8)); // the scan reads whole 32-byte groups
     const long long words = (long long)outWords + 2; // all that grids_prepare would clear
-    const long long blocks = (scn_ceil_div(words, 256) + 7) / 8 * 8; // whole rounds of the 8 XCDs
-    auto dilate = g.size == 2 ? k_mask_dilate<D, 2>
-                              : (g.size == 3 ? k_mask_dilate<D, 3> : k_mask_dilate<D, 0>);
-    hipLaunchKernelGGL(dilate, dim3((unsigned)blocks), dim3(256),
-                       0, ctx->stream, vin, g, out->bits.p, words, volOutAll,
-                       scn_scan_state(outWords + 1, out->scanTmp.p));
-    SCN_HIP_CHECK(hipGetLastError());
+    const Dilate to = {out->bits.p, words, volOutAll, scn_scan_state(outWords + 1, out->scanTmp.p),
+                       xcd_grid(scn_ceil_div(words, 256))}; // (whole rounds of the 8 XCDs)
+    const RankRows beside = {rows.ekey, rows.erow, rows.n, rows.meta, in->rankRowValid ? nullptr : rows.rankRow};
+    const unsigned rowBlocks = beside.rankRow ? xcd_grid(scn_ceil_div(nE, 256)) : 0;
+    in->rankRowValid = true;
+    const dim3 grid(8 + to.blocks + rowBlocks);
+#define SCN_DILATE_GO(S, KIND) \
+  hipLaunchKernelGGL((k_plan_dilate<D, S, KIND>), grid, dim3(SCAN1_THREADS), 0, ctx->stream, vin, g, to, samples, beside)
+    if (kind == 1)
+      SCN_DILATE_GO(2, 1);
+    else if (g.size == 2 && kind == 0)
+      SCN_DILATE_GO(2, 0);
+    else if (g.size == 2)
+      SCN_DILATE_GO(2, 2);
+    else if (g.size == 3 && kind == 0)
+      SCN_DILATE_GO(3, 0);
+    else if (g.size == 3)
+      SCN_DILATE_GO(3, 2);
+    else if (kind == 0)
+      SCN_DILATE_GO(0, 0);
+    else
+      SCN_DILATE_GO(0, 2);
+#undef SCN_DILATE_GO
     rankStateFor = outWords + 1;
+  } else if (kind == 2) { // (tiled windows are always dilated)
+    hipLaunchKernelGGL(k_plan_samples<2>, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream, samples);
+  } else {
+    hipLaunchKernelGGL(k_plan_samples<0>, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream, samples);
   }
+  SCN_HIP_CHECK(hipGetLastError());
   long long nSites = boundRows, nOutActive = boundActive;
   if (!deferred) {
     SCN_TRY(read_scalars(ctx, ticket));
@@ -2034,6 +2120,7 @@ static int plan_regions(scn_ctx *ctx, const scn_grids *cin, scn_grids *out,
   g.volOut = ipow_ll(nOut, in->d);
   g.cube = (int)ipow_ll(size, in->d);
   g.magicStride = (unsigned)((1ull << 32) / (unsigned)stride + 1);
+  g.divIn = g.divOut = FieldDivisors();
   g.ticks = nullptr;
   g.tInR = g.tOutL = g.tOutR = 0;
   SCN_REQUIRE(ipow_ll(size, in->d) <= 32768, SCN_ERR_ARG,
@@ -2071,7 +2158,6 @@ static int plan_regions(scn_ctx *ctx, const scn_grids *cin, scn_grids *out,
     SCN_TRY(scn_chain_flush(ctx));
   }
   ProfScope ps(ctx, SCN_K_RULES);
-  SCN_TRY(ensure_rank(ctx, in));
   int rc;
   switch (in->d) {
   case 1:

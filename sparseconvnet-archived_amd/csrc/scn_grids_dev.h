@@ -15,6 +15,25 @@ struct __align__(16) Slot {
 enum { MODE_SQ_NOMIN = 0, MODE_SQ_MIN, MODE_SQ_VALID, MODE_TRI_NOMIN, MODE_TRI_MIN, MODE_SQ_FMP };
 enum { PLAN_NONE = 0, PLAN_REGIONS = 1, PLAN_TERMINAL = 2 };
 
+// x / d of 31-bit x by a multiplication: ceil(2^(31 + shift) / d), shift the least
+// with 2^shift >= d (a 32-bit division is some 22 instructions, a site's three of them)
+struct Divisor {
+  unsigned magic;
+  int shift;
+};
+__device__ __forceinline__ unsigned div31(unsigned x, const Divisor &d) { return __umulhi(x << 1, d.magic) >> d.shift; }
+static inline Divisor divisor_of(long long d) { // 1 <= d <= 2^31
+  Divisor r = {0, 0};
+  while ((1ll << r.shift) < d)
+    ++r.shift;
+  r.magic = (unsigned)(((1ull << (31 + r.shift)) + (unsigned long long)d - 1) / (unsigned long long)d);
+  return r;
+}
+// ... of a packed position by the field's volume and of a key by its side, where a
+// batch has no more than 2^31 of them (magic 0: it has)
+struct FieldDivisors {
+  Divisor vol, n;
+};
 struct Geom {
   int d;
   int nIn, nOut, size, stride, minActive, mode;
@@ -22,6 +41,7 @@ struct Geom {
   int width; // rule-row width: size^d or triangleSize(size, d)
   int cube;  // size^d
   unsigned magicStride; // floor(2^32 / stride) + 1 (div_magic)
+  FieldDivisors divIn, divOut; // set by plan_regions_d
   // MODE_SQ_FMP: per-sample, per-axis region tables (fractional max-pooling).
   // inputL at ticks[(b d + a) nOut + j], inputR the same at tInR; outputL and
   // outputR at tOutL / tOutR + (b d + a) nIn + i.  Null otherwise.
@@ -71,14 +91,14 @@ __device__ __forceinline__ long long count_now(const Count &c) {
 // without work keep their own numbers.  A permutation of the grid, which must
 // be a multiple of 8 blocks.
 #define XCD_RUN 32
-__device__ __forceinline__ long long xcd_contiguous_block(long long nLive) {
-  const long long b = blockIdx.x;
+__device__ __forceinline__ long long xcd_contiguous_block(long long b, long long nLive) {
   const long long whole = nLive / (8 * XCD_RUN) * (8 * XCD_RUN);
   if (b >= whole)
     return b;
   const long long turn = b / 8, xcd = b % 8;
   return ((turn / XCD_RUN) * 8 + xcd) * XCD_RUN + turn % XCD_RUN;
 }
+__device__ __forceinline__ long long xcd_contiguous_block(long long nLive) { return xcd_contiguous_block(blockIdx.x, nLive); }
 // (host side: the grid such kernels are launched with)
 static inline unsigned xcd_grid(long long blocks) {
   return (unsigned)((blocks + 7) / 8 * 8);
@@ -681,7 +701,19 @@ __device__ __forceinline__ int unpack_row_site(long long sk, int *j) {
 // key is taken apart in 32-bit arithmetic when the field allows it
 template <int D>
 __device__ __forceinline__ int split_site(long long p, long long vol, int n,
-                                          int *c) {
+                                          const FieldDivisors &div, int *c) {
+  if (div.vol.magic) { // uniform
+    const unsigned b = div31((unsigned)p, div.vol);
+    unsigned k = (unsigned)p - b * (unsigned)vol;
+#pragma unroll
+    for (int a = D - 1; a > 0; --a) {
+      const unsigned up = div31(k, div.n);
+      c[a] = (int)(k - up * (unsigned)n);
+      k = up;
+    }
+    c[0] = (int)k;
+    return (int)b;
+  }
   // (64-bit division is a long routine: most batches' masks have fewer than 2^32 bits)
   const int b = ((unsigned long long)(p | vol) >> 32) == 0 ? (int)((unsigned)p / (unsigned)vol)
                                                            : (int)(p / vol);

@@ -61,9 +61,8 @@ __device__ __forceinline__ uint32_t wave_incl_dpp(uint32_t v) {
 // lanes x 4 elements: every load and every store of a wavefront is one
 // contiguous kilobyte (two for 64-bit words).
 template <bool POPC>
-__global__ void __launch_bounds__(SCAN_THREADS)
-    k_scan_lookback(const void *in, uint32_t *out, size_t n, unsigned long long *state,
-                    unsigned nb) {
+__device__ __forceinline__ void scan_lookback_tile(const void *in, uint32_t *out, size_t n, unsigned long long *state,
+                                                   unsigned nb) {
   __shared__ uint32_t lds[SCAN_THREADS];
   __shared__ unsigned sTile;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -131,6 +130,27 @@ __global__ void __launch_bounds__(SCAN_THREADS)
 }
 
 template <bool POPC>
+__global__ void __launch_bounds__(SCAN_THREADS)
+    k_scan_lookback(const void *in, uint32_t *out, size_t n, unsigned long long *state,
+                    unsigned nb) {
+  scan_lookback_tile<POPC>(in, out, n, state, nb);
+}
+// Two of them side by side: 150 workgroups leave room for as many (7.7 us each of 1.25
+// million words; the pair 11.0).  A workgroup waits for those with lower tickets
+// of its own scan.
+struct ScanJob {
+  const void *in;
+  uint32_t *out;
+  size_t n;
+  unsigned long long *state;
+  unsigned nb;
+};
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_lookback_pair(ScanJob a, ScanJob b) {
+  const ScanJob &j = blockIdx.x < a.nb ? a : b;
+  scan_lookback_tile<true>(j.in, j.out, j.n, j.state, j.nb);
+}
+
+template <bool POPC>
 __global__ void __launch_bounds__(SCAN1_THREADS)
     k_scan_single(const void *in, uint32_t *out, size_t n) {
   __shared__ uint32_t lds[SCAN1_LDS_WORDS];
@@ -183,4 +203,21 @@ int scn_scan_exclusive_u32(hipStream_t s, const uint32_t *in, uint32_t *out,
 int scn_scan_exclusive_popc64(hipStream_t s, const uint64_t *words,
                               uint32_t *out, size_t n, uint32_t *tmp, bool cleared) {
   return scan_impl<true>(s, words, out, n, tmp, cleared);
+}
+
+int scn_scan_exclusive_popc64_pair(hipStream_t s, const uint64_t *wordsA, uint32_t *outA, size_t nA, uint32_t *tmpA,
+                                   const uint64_t *wordsB, uint32_t *outB, size_t nB, uint32_t *tmpB) {
+  if (nA <= SCAN1_MAX_ELEMS || nB <= SCAN1_MAX_ELEMS) {
+    SCN_TRY(scan_impl<true>(s, wordsA, outA, nA, tmpA, true));
+    return scan_impl<true>(s, wordsB, outB, nB, tmpB, true);
+  }
+  const size_t a = (nA + LB_TILE - 1) / LB_TILE, b = (nB + LB_TILE - 1) / LB_TILE;
+  SCN_REQUIRE(a + b < 0x7FFFFFFFull, SCN_ERR_CAPACITY, "scan: %zu and %zu elements", nA, nB);
+  SCN_REQUIRE((((uintptr_t)wordsA | (uintptr_t)outA | (uintptr_t)wordsB | (uintptr_t)outB) & 15) == 0, SCN_ERR_ARG,
+              "scan: buffers must be 16-byte aligned");
+  hipLaunchKernelGGL(k_scan_lookback_pair, dim3((unsigned)(a + b)), dim3(SCAN_THREADS), 0, s,
+                     (ScanJob{wordsA, outA, nA, scn_scan_state(nA, tmpA).state, (unsigned)a}),
+                     (ScanJob{wordsB, outB, nB, scn_scan_state(nB, tmpB).state, (unsigned)b}));
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
 }
