@@ -104,22 +104,53 @@ extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
 
 // dMaxPool (MaxPoolingLayer.cu:9-35): strict '<' so the first maximum wins,
 // negative rules skipped.  One lane owns VEC channels of one output row.
-template <int VEC>
+// A workgroup's rules come in one request a lane through LDS where they fit, and a
+// row is told from a lane by a multiplication (a 64-bit division is some 100
+// instructions): windows of 3 x 3 from 88000 x 32 7.1 -> 6.7 us, from 57500 x 64 7.9 ->
+// 7.3, few of them 3.7 -> 3.5, 246000 x 64 at a copy's rate either way (86.4, 87.8);
+// beside a contraction, whose path to memory has nine requests less a window to share,
+// more (a layer 596 000 x 2592 -> 128 with its pooling, among others, 458 -> 452).
+#define MP_RULES 1024
+struct PoolDivisor { // x / chunks = (x * magic >> 32) >> shift, x < 2^31 (magic 0: divided)
+  unsigned magic;
+  int shift;
+};
+template <int VEC, int PS>
 __global__ void __launch_bounds__(256)
     k_maxpool(const float *__restrict__ in, float *__restrict__ out,
-              const int *__restrict__ rules, long long nOutSites, int ps,
-              int C, int chunks, int *__restrict__ choice,
+              const int *__restrict__ rules, long long bound, int ps,
+              int C, int chunks, PoolDivisor div, int *__restrict__ choice,
               const float *__restrict__ spare, const long long *dRows) {
-  nOutSites = live_rows(nOutSites, dRows);
-  const unsigned tiles = (unsigned)((nOutSites * chunks + 255) / 256);
+  __shared__ int sRules[PS ? MP_RULES : 1];
+  if (PS)
+    ps = PS;
+  const long long nOutSites = live_rows(bound, dRows), all = nOutSites * chunks;
+  const unsigned tiles = (unsigned)((all + 255) / 256);
   if (blockIdx.x >= tiles)
     return;
-  const long long idx = (long long)xcd_eighth(blockIdx.x, tiles) * 256 + threadIdx.x;
-  if (idx >= nOutSites * chunks)
+  const long long tile = xcd_eighth(blockIdx.x, tiles);
+  const long long idx = tile * 256 + threadIdx.x;
+  long long r, r0; // this lane's row, the workgroup's first
+  if (div.magic) { // uniform
+    r = __umulhi((unsigned)idx << 1, div.magic) >> div.shift;
+    r0 = __umulhi((unsigned)(tile * 256) << 1, div.magic) >> div.shift;
+  } else {
+    r = idx / chunks;
+    r0 = tile * 256 / chunks;
+  }
+  if (PS) {
+    const long long last = tile * 256 + 255 < all ? tile * 256 + 255 : all - 1;
+    const int n = ((int)((div.magic ? (long long)(__umulhi((unsigned)last << 1, div.magic) >> div.shift) : last / chunks) - r0) + 1) * PS;
+    const int *const from = rules + r0 * PS;
+    for (int i = threadIdx.x; i < n; i += 256)
+      sRules[i] = from[i];
+  }
+  if (PS)
+    __syncthreads();
+  if (idx >= all)
     return;
-  long long r = idx / chunks;
-  int c0 = (int)(idx - r * chunks) * VEC;
-  const int *rr = rules + r * ps;
+  const int c0 = (int)(idx - r * chunks) * VEC;
+  const int *const rr = PS ? sRules + (int)(r - r0) * PS : rules + r * ps;
   float best[VEC];
   int arg[VEC];
 #pragma unroll
@@ -133,7 +164,7 @@ __global__ void __launch_bounds__(256)
   // which may have no rows at all -- and is dropped below), so that a window
   // costs two trips to memory rather than two per candidate; they are
   // compared in rule order.
-  constexpr int MP = 9;
+  constexpr int MP = PS && PS < 9 ? PS : 9;
   for (int p0 = 0; p0 < ps; p0 += MP) {
     int rule[MP];
 #pragma unroll
@@ -196,19 +227,31 @@ extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
               "scn_maxpool: null buffer");
   ProfScope prof(ctx, SCN_K_MAXPOOL);
   const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
-  if (C % 4 == 0 && aligned16(d_in) && aligned16(d_out) && aligned16(d_choice)) {
-    long long total = nOutSites * (C / 4);
-    hipLaunchKernelGGL(k_maxpool<4>, dim3(scn_ceil_div(total, 256)), dim3(256),
-                       0, ctx->stream, d_in, d_out, d_rules,
-                       (long long)nOutSites, ps, C, C / 4, d_choice,
-                       (const float *)ctx->d_zeros, dRows);
-  } else {
-    long long total = nOutSites * C;
-    hipLaunchKernelGGL(k_maxpool<1>, dim3(scn_ceil_div(total, 256)), dim3(256),
-                       0, ctx->stream, d_in, d_out, d_rules,
-                       (long long)nOutSites, ps, C, C, d_choice,
-                       (const float *)ctx->d_zeros, dRows);
+  const bool wide = C % 4 == 0 && aligned16(d_in) && aligned16(d_out) && aligned16(d_choice);
+  const int chunks = wide ? C / 4 : C;
+  const long long total = nOutSites * chunks;
+  PoolDivisor div = {0u, 0};
+  if (total + 256 < (1ll << 31)) { // ceil(2^(31 + shift) / chunks), 2^shift >= chunks
+    while ((1ll << div.shift) < chunks)
+      ++div.shift;
+    div.magic = (unsigned)(((1ull << (31 + div.shift)) + chunks - 1) / chunks);
   }
+  // (rows that a workgroup's 256 lanes may touch)
+  const bool fits = (256 / chunks + 2ll) * ps <= MP_RULES;
+#define SCN_MP_GO(VEC, PS)                                                                                       \
+  hipLaunchKernelGGL((k_maxpool<VEC, PS>), dim3(scn_ceil_div(total, 256)), dim3(256), 0, ctx->stream, d_in, d_out, \
+                     d_rules, (long long)nOutSites, ps, C, chunks, div, d_choice, (const float *)ctx->d_zeros, dRows)
+  if (!wide)
+    SCN_MP_GO(1, 0);
+  else if (fits && ps == 9)
+    SCN_MP_GO(4, 9);
+  else if (fits && ps == 8)
+    SCN_MP_GO(4, 8);
+  else if (fits && ps == 4)
+    SCN_MP_GO(4, 4);
+  else
+    SCN_MP_GO(4, 0);
+#undef SCN_MP_GO
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
 }
