@@ -1362,17 +1362,34 @@ struct PoolInverseList {
 // a workgroup an item: where the samples' windows begin, and the background rows' marks
 __global__ __launch_bounds__(256) void k_pool_samples(PoolInverseList l) {
   const int t = blockIdx.x, batch = l.batch[t], slots = l.slots[t];
-  // (a sample's rows are its sites and then, if it is not full, a background row)
-  auto end = [&](int s) {
-    long long full = 0;
-    int x = s;
-    for (; x >= 0 && l.outBg[t][x] < 0; --x)
-      full += l.volume[t];
-    const long long e = full + (x >= 0 ? l.outBg[t][x] + 1 : 0);
-    return (int)(e < l.rows[t] ? e : l.rows[t]);
-  };
-  for (int s = threadIdx.x; s <= batch; s += 256)
-    l.samples[t][s] = s == 0 ? 0 : end(s - 1);
+  // A sample's rows are its sites and then, if it is not full, a background row: its
+  // last row follows from that row of the last sample up to it that has one, and the
+  // full ones since.  (The last such sample by a running maximum; each looking back by
+  // itself: 18 us where the small fields of a batch of 100 drawings are full.)
+  __shared__ int sLast[256];
+  const int lane = threadIdx.x;
+  int carry = -1;
+  if (lane == 0)
+    l.samples[t][0] = 0;
+  for (int base = 0; base < batch; base += 256) { // uniform
+    const int s = base + lane, row = s < batch ? l.outBg[t][s] : -1;
+    int last = row >= 0 ? s : carry;
+    sLast[lane] = last;
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+      const int other = lane >= off ? sLast[lane - off] : -1;
+      last = other > last ? other : last;
+      __syncthreads();
+      sLast[lane] = last;
+      __syncthreads();
+    }
+    carry = sLast[255];
+    __syncthreads();
+    if (s < batch) {
+      const long long e = last >= 0 ? l.outBg[t][last] + 1 + (s - last) * l.volume[t] : (s + 1) * l.volume[t];
+      l.samples[t][s + 1] = (int)(e < l.rows[t] ? e : l.rows[t]);
+    }
+  }
   for (int s = threadIdx.x; s < batch; s += 256) {
     const int r = l.bg[t][s], mine = r >= 0 && r < l.inRows[t] ? r : -1;
     l.samples[t][batch + 1 + s] = mine;
