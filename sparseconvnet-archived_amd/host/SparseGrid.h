@@ -7,7 +7,9 @@
 // (SparseGrid.h:15-16, vectorHash.cpp:40-55); it is the order that fixes the
 // row numbering of every rule book.  Storage is an insertion-ordered entry
 // list with an open-addressing index, so codify stays O(1) per site on large
-// lattices; deeper layers never use this class (their grids live in HBM).
+// lattices; deeper layers never use this class (their grids live in HBM).  Entries
+// that are known to be new can be appended without the index, which the first look-up
+// afterwards makes (a batch is flattened from the entries and never looked up).
 #pragma once
 #include <stdint.h>
 #include <algorithm>
@@ -19,7 +21,7 @@ public:
   typedef std::pair<int64_t, int> value_type;
   typedef std::vector<value_type>::iterator iterator;
 
-  SparseGridMap() : live_(0), sorted_(true) {}
+  SparseGridMap() : live_(0), sorted_(true), stale_(false) {}
 
   int &operator[](int64_t key) {
     size_t slot = 0;
@@ -52,9 +54,19 @@ public:
     reindex();
   }
   size_t size() const { return entries_.size(); }
+  // n entries with keys of which none is here yet
+  void appendNew(const value_type *kv, size_t n) {
+    for (size_t i = 0; i < n; ++i)
+      if (i ? kv[i].first < kv[i - 1].first : !entries_.empty() && kv[0].first < entries_.back().first)
+        sorted_ = false;
+    entries_.insert(entries_.end(), kv, kv + n);
+    stale_ = stale_ || n > 0;
+  }
   // room for n sites without growing on the way (optional)
   void reserve(size_t n) {
     entries_.reserve(n);
+    if (stale_)
+      reindex();
     size_t cap = 16;
     while (cap < 2 * n + 2)
       cap *= 2;
@@ -68,6 +80,7 @@ public:
     entries_.clear();
     index_.clear();
     sorted_ = true;
+    stale_ = false;
   }
   // entries in insertion order unless an ordered view has been requested
   const std::vector<value_type> &entries() const { return entries_; }
@@ -77,13 +90,16 @@ private:
   std::vector<int> index_; // open addressing over entries_, -1 = empty
   size_t live_;
   bool sorted_;
+  bool stale_; // the index lacks entries (appendNew)
 
   static size_t mix(int64_t k) {
     uint64_t x = (uint64_t)k * 0x9E3779B97F4A7C15ull;
     return (size_t)(x ^ (x >> 29));
   }
   // the entry of `key`, or -1 and (if asked) the empty slot its probe ended at
-  int lookup(int64_t key, size_t *emptySlot = nullptr) const {
+  int lookup(int64_t key, size_t *emptySlot = nullptr) {
+    if (stale_)
+      reindex();
     if (index_.empty())
       return -1;
     size_t mask = index_.size() - 1, s = mix(key) & mask;
@@ -106,6 +122,7 @@ private:
     index_[s] = at;
   }
   void reindex() {
+    stale_ = false;
     size_t cap = 16;
     while (cap < 2 * entries_.size() + 2)
       cap *= 2;
