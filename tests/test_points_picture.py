@@ -32,7 +32,7 @@ def test_points(d, lattice, field, n):
         k, r, bg, f = ds.codify(i, field)
         shift = int((field - lattice) / 2)
         keys, rows, want = [], [], [np.zeros(3, np.float32)]
-        for p, f in zip(at + shift, feats):
+        for p, value in zip(at + shift, feats):
             if (p < 0).any() or (p >= field).any():
                 continue
             key = 0
@@ -41,7 +41,7 @@ def test_points(d, lattice, field, n):
             if key not in keys:
                 keys.append(key)
                 rows.append(len(want))
-                want.append(f)
+                want.append(value)
         assert bg == 0 and np.array_equal(f, np.array(want))
         assert dict(zip(k.tolist(), r.tolist())) == dict(zip(keys, rows))
 
