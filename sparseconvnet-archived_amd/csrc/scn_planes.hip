@@ -832,7 +832,13 @@ template <int N> __device__ __forceinline__ void lines_landed() {
 // tiles of three planes stay ahead on gathered rows: 1.36 M x 1728 x 64 1483 against
 // 1797.
 
-template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16>
+// LONG (plain rows): a workgroup goes through several tiles of the same columns, and
+// asks for the next one's rows before it is done with one, D - 1 blocks ahead across the
+// tiles.  Each tile by itself began with a trip to memory and ended in its stores, 4 of
+// the 10 us that one of 128 x 128 x 128 took.  The results go past the caches, which the
+// rows are wanted in: 139000 x 128 x 384 127 us -> 115, so 95; 139000 x 128 x 128 55 -> 37,
+// 400000 x 96 x 128 116 -> 73, 139000 x 256 x 192 109 -> 92, 50000 x 320 x 1280 265 -> 244.
+template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16, bool LONG = false>
 __global__ void __launch_bounds__(64 * RW * CW, 2)
     k_nin_lines(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
                 int K, int N, Epilogue ep, GatherSource gs, int nSplits, bool byColumns, RowRange rows, PlainW plain) {
@@ -844,21 +850,34 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   constexpr int A_BYTES = A_CHUNKS * 1024, SLOT = (A_CHUNKS + W_CHUNKS) * 1024;
   extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [D][SLOT], then the rules
   M = rows.live(M);
-  const unsigned tiles = (unsigned)((M + ROWS - 1) / ROWS) * nSplits;
-  if (blockIdx.x >= tiles)
-    return;
-  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
+  const unsigned rowTiles = (unsigned)((M + ROWS - 1) / ROWS), tiles = rowTiles * nSplits;
+  // LONG: the grid is eight times a multiple of nSplits; an XCD has an eighth of the rows
+  unsigned longFirst = 0, longStep = 0;
+  int mine = 1; // tiles of this workgroup
+  if constexpr (LONG) {
+    const unsigned x = blockIdx.x & 7, per = gridDim.x >> 3, rem = rowTiles & 7;
+    const unsigned group = (blockIdx.x >> 3) / nSplits, count = (rowTiles >> 3) + (x < rem);
+    longStep = per / nSplits;
+    if (group >= count)
+      return;
+    mine = (int)((count - group + longStep - 1) / longStep);
+    longFirst = x * (rowTiles >> 3) + (x < rem ? x : rem) + group;
+  } else {
+    if (blockIdx.x >= tiles)
+      return;
+  }
+  const unsigned tileOf = LONG ? 0 : xcd_eighth(blockIdx.x, tiles);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, q = lane >> 5;
   const int cg = wave % CW, rg = wave / CW;
-  const unsigned rowTiles = tiles / nSplits;
-  const int split = byColumns ? tileOf / rowTiles : tileOf % nSplits;
-  const long long wgRow0 = (long long)(byColumns ? tileOf % rowTiles : tileOf / nSplits) * ROWS;
-  const long long row0 = wgRow0 + rg * 32 * MT;
+  const int split = LONG ? (blockIdx.x >> 3) % nSplits : byColumns ? tileOf / rowTiles : tileOf % nSplits;
+  long long wgRow0 = (long long)(LONG ? longFirst : byColumns ? tileOf % rowTiles : tileOf / nSplits) * ROWS;
+  long long row0 = wgRow0 + rg * 32 * MT;
   const int n0 = split * NW + cg * 32 * NT; // this wavefront's columns
   const int T = K / 32;
   int *const sRules = reinterpret_cast<int *>(sW + D * SLOT);
+  static_assert(!LONG || !GATHER, "LONG: plain rows");
   const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)sW;
 
@@ -877,6 +896,9 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   }
   const unsigned char *rowPtr[A_PER];
   int f = 0, ch = 0;
+  // LONG: the tile whose rows are asked for, its first row, and the block of it
+  int asked = 0, askedBlock = 0;
+  long long askedRow0 = wgRow0;
   // (A16: two rows lie on all banks, so that they are rotated by pairs)
   const int piece = 16 * ((lane % LANES) ^ (A16 ? lane >> 3 & 3 : lane >> 3));
   auto aim = [&]() {
@@ -888,7 +910,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
         const int rule = sRules[r * gs.fs + f];
         rowPtr[u] = (rule >= 0 ? Ab + (long long)rule * gs.nIn * ES : reinterpret_cast<const unsigned char *>(gs.zeros)) + piece;
       } else {
-        long long m = wgRow0 + r;
+        long long m = (LONG ? askedRow0 : wgRow0) + r;
         m = m < M ? m : M - 1;
         rowPtr[u] = Ab + m * K * ES + piece;
       }
@@ -902,6 +924,16 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
     dma_kilobyte(lds0 + slot * SLOT + (x < A_CHUNKS ? x : A_CHUNKS - 1) * 1024, rowPtr[u] + ch * ES);
   };
   auto advance = [&]() { // to the next block's rows
+    if constexpr (LONG) {
+      ++askedBlock;
+      if (askedBlock == T) {
+        askedBlock = ch = 0;
+        askedRow0 += (long long)longStep * ROWS;
+        if (++asked < mine)
+          aim();
+        return;
+      }
+    }
     ch += 32;
     if (GATHER && ch == gs.nIn) {
       ch = 0;
@@ -1030,6 +1062,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
     __builtin_amdgcn_sched_barrier(0);
   };
   constexpr int UNITS = 2 * MT, SECOND = MT; // the first unit of the second step: the barrier before it
+  bool ahead = false;                        // LONG: not this workgroup's first tile
   auto block = [&](int t, auto steady) {     // steady: with a block to ask for
     const bool more = steady || t + D - 1 < T; // uniform
 #pragma unroll
@@ -1038,10 +1071,12 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
       if (u == SECOND) {
         // The next block has landed (those asked for behind it may be under way), and
         // nobody reads the last one any more.
-        if (steady || t + D - 1 <= T) // uniform
-          lines_landed<PER *(D - 3)>();
-        else
+        if (!(steady || t + D - 1 <= T)) // uniform
           lines_landed<0>();
+        else if (LONG && ahead && t + 1 <= D - 2) // asked for before the last tile's results were stored
+          lines_landed<PER *(D - 3) + MT * NT * 16>();
+        else
+          lines_landed<PER *(D - 3)>();
         asm volatile("s_barrier" ::: "memory");
       }
       if (A16) // (where the last unit but one's operand was)
@@ -1074,7 +1109,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
 #pragma unroll
           for (int x = g * PER / G; x < (g + 1) * PER / G; ++x) {
             if (x < W_PER)
-              fetch_w(t + D - 1, last, x);
+              fetch_w(LONG ? askedBlock : t + D - 1, last, x);
             else
               fetch_a(last, x - W_PER);
           }
@@ -1085,15 +1120,20 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
       advance();
     last = cur, cur = next, next = next == D - 1 ? 0 : next + 1;
   };
+  for (int at = 0;;) { // the tiles
   int t = 0;
 #pragma unroll 1
-  for (; t + D - 1 < T; ++t)
+  for (; t + (LONG && at + 1 < mine ? 0 : D - 1) < T; ++t)
     block(t, std::true_type());
 #pragma unroll 1
   for (; t < T; ++t)
     block(t, std::false_type());
 
   // ---- epilogue: register v of a tile is row 8 (v / 4) + 4 q + v % 4
+  int lane = tid & 63;
+  if constexpr (LONG) // (what follows from it is not kept from one tile to the next)
+    asm volatile("" : "+v"(lane));
+  const int c = lane & 31, q = lane >> 5;
   if constexpr (NACC == 2) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -1142,13 +1182,12 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
       for (int v = 0; v < 16; ++v)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[0][i][j][v], col[j])), to, at[j], 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[0][i][j][v], col[j])), to, at[j], 0, LONG ? 2 : 0);
           at[j] += v % 4 == 3 ? 5 * pitch : pitch;
         }
   }
   if constexpr (PL == 3) {
-    if (!__any(again != 0))
-      return;
+    if (__any(again != 0))
 #pragma unroll 1
     for (int e = 0; e < MT * NT; ++e) {
       const unsigned mine = (unsigned)(again >> (16 * e)) & 0xffffu;
@@ -1167,6 +1206,31 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
           out[r * N + n] = finish(exact[v], last);
       }
     }
+  }
+  if (!LONG || ++at == mine)
+    return;
+  if constexpr (LONG) {
+    wgRow0 += (long long)longStep * ROWS, row0 += (long long)longStep * ROWS;
+    ahead = true;
+#pragma unroll
+    for (int h = 0; h < NACC; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            acc[h][i][j][v] = 0.f;
+    // (the first operands anew: they need no registers while results are stored)
+    read_a(cur, 0);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      read_b(cur, 0, j);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      a_split(0, p);
+    read_a(cur, 1);
+  }
   }
 }
 
@@ -1324,6 +1388,11 @@ static void add_image(ImageList &l, const float *W, unsigned char *image, int pl
   l.W[i] = W, l.image[i] = image, l.K[i] = K, l.N[i] = N, l.fs[i] = fs, l.planes[i] = planes;
   l.firstBlock[i + 1] = l.firstBlock[i] + (unsigned)scn_ceil_div((int64_t)K / 8 * ((N + 31) / 32 * 32), 256);
 }
+// how many workgroups an XCD has of a LONG launch (0: none): a multiple of the slices of columns
+static int lines_long(const scn_ctx *ctx, int T, int splits, int d, bool gather) {
+  const int cus = ctx->numCU / 8;
+  return !gather && T >= d - 1 && splits <= cus ? cus / splits * splits : 0;
+}
 template <int PL, int MT, int NT, int RW, int CW, int D, bool A16 = false>
 static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
                         const Epilogue &ep, const GatherSource *gs, bool wT, const RowRange &rows,
@@ -1343,6 +1412,18 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
   // An XCD takes neighbouring tiles: rows with all their columns, so that they come
   // to its L2 once, or, where the image is the larger part, columns with all rows.
   const bool byColumns = image_bytes(PL, K, N) > (long long)scn_rows_hint(ctx, M) * (gs ? gs->nIn : K) * 4;
+  // LONG: plain rows, where a compute unit that has room for one workgroup has more than
+  // one tile.  (Gathered rows: 15948 x 1280 x 480 115 us for 110, 15003 x 1920 x 640 232
+  // for 220, with the rules of the next tiles under way; two workgroups to a compute unit
+  // see to that themselves: 139000 x 128 x 64 36 for 29.)
+  if constexpr (PL == 3 && !A16 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160) {
+    const int per = lines_long(ctx, K / 32, nSplits, D, gs != nullptr);
+    if (per && !byColumns && (int64_t)scn_ceil_div(scn_rows_hint(ctx, M), ROWS) * nSplits > ctx->numCU) {
+      hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false, false, true>), dim3(8 * per), dim3(64 * RW * CW), lds,
+                         ctx->stream, A, image, out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
+      return SCN_OK;
+    }
+  }
   if (gs)
     hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, true, A16>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
                        out, M, K, N, ep, *gs, nSplits, byColumns, rows, PlainW{W, wT});
@@ -1461,12 +1542,12 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
 // deeper rings gained nothing.
 struct LinesTile {
   int mt, nt, rw, cw, d, resident;
-  float f, t1, tn;
+  float f, t1, tn, next; // next: what a further tile of the same workgroup's begins and ends with (LONG)
 };
 static const LinesTile linesTiles[2][6] = {
-    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f}}, // one plane
-    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f},
-     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f}}};
+    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f}}, // one plane
+    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 3.3f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 3.4f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 4.5f},
+     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 2.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 1.2f}}};
 static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool gather, int *tile) {
   const int T = K / 32;
   float least = 1e30f;
@@ -1477,6 +1558,9 @@ static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, b
     if (n <= x.resident) {
       const float shared = x.resident > 1 ? (fmaxf(ceilf(n), 1.f) - 1.f) / (x.resident - 1) : 0.f;
       cost = x.f + T * (x.t1 + shared * (x.tn - x.t1));
+    } else if (const int per = x.next > 0.f ? lines_long(ctx, T, scn_ceil_div(N, 32 * x.nt * x.cw), x.d, gather) : 0) {
+      const float long_ = n * ctx->numCU / (8 * per), rounds = long_ <= 3.f ? ceilf(long_) : long_ + .5f;
+      cost = 1.f + rounds * (x.next + T * x.t1);
     } else {
       const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
       cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));

@@ -154,3 +154,26 @@ def test_weight_gradients_by_lines(scn, ctx, M, fs, nIn, N):
     for got in (dW, plain):
         assert (np.abs(got.download() - want) / scale).max() <= 2e-6
     assert (np.abs(dB.download() - D.sum(0, dtype=np.float64)) / (np.abs(D).sum(0) + 1e-30)).max() <= 2e-6
+
+
+# plain rows of which a compute unit has several tiles (k_nin_lines' LONG): two blocks of k, which a tile's requests are ahead
+# of its last block by, and more; slices of columns that do not divide an XCD's workgroups (640, 1280: 5 and 10); the last tile
+# of one row, of all but one; rows that are not finite in the first, a middle and the last tile, which are taken again there
+@pytest.mark.parametrize("M,K,N", [(128 * 300 + 1, 64, 384), (128 * 523 - 1, 128, 128), (256 * 300 + 77, 64, 64), (33001, 128, 256),
+                                   (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192)])
+def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
+    rng = np.random.default_rng(M + K + N)
+    A, W = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
+    odd = [0, M // 2, M - 1]
+    A[odd, 3] = [np.inf, np.nan, -np.inf]
+    print("several tiles", M, K, N, flush=True)
+    out, ws = ctx.array(np.full((M, N), 7, np.float32)), ctx.empty(int(scn.lib().scn_sgemm_ABt_workspace(K, N)), np.float32)
+    ctx.sgemm_ABt(ctx.array(A), ctx.array(W), out, M, K, N, ws)
+    got = out.download()
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(got[odd], A[odd, 3:4] * W[:, 3], equal_nan=True)
+    A[odd] = 0
+    got[odd] = 0
+    for r in range(0, M, 20000):
+        a = A[r:r + 20000].astype(np.float64)
+        assert np.all(np.abs(got[r:r + 20000] - a @ W.T.astype(np.float64)) <= 2e-6 * (np.abs(a) @ np.abs(W.T).astype(np.float64)))
