@@ -460,6 +460,11 @@ int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *
  * scn_weight_images_many: d_image (aligned to 16 bytes) from d_W; with fs > 0 d_W are
  * the filters of a layer, [fs N x K / fs], and the image that of the weights
  * scn_transpose_filters_many makes of them.
+ * scn_weight_images_later: the same beside the context's next launch that can take
+ * them along (a convolution over channels in other than fours, a net's first layer),
+ * or before the first call that is given an image; until then the images are not
+ * there, d_W and their room must stay, and no other stream may read them.  What an
+ * earlier call of it left and nothing has taken is given up.
  * scn_conv_nin_forward_image: scn_conv_nin_forward_p (d_rules null: scn_nin_forward_p
  * of a matrix of fs nIn columns) with d_W and its image, or null. */
 #define SCN_IMAGES_MAX 32
@@ -470,6 +475,7 @@ typedef struct scn_image_item {
 } scn_image_item;
 int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N, int nIn, int precision);
 int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items, int nItems);
+int scn_weight_images_later(scn_ctx *ctx, const scn_image_item *items, int nItems);
 int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn, const float *d_W,
                                const void *d_image, const float *d_B, const float *d_prelu, float *d_out, int64_t M, int N,
                                float p, int act, int precision);

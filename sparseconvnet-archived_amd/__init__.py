@@ -180,6 +180,7 @@ def lib():
         "scn_conv_input_gradient": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, i64, C.c_int]),
         "scn_weight_image_bytes": (i64, [vp, i64, C.c_int, C.c_int, C.c_int, C.c_int]),
         "scn_weight_images_many": (C.c_int, [vp, P(ImageItem), C.c_int]),
+        "scn_weight_images_later": (C.c_int, [vp, P(ImageItem), C.c_int]),
         "scn_conv_nin_forward_image": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, C.c_int, f32, C.c_int, C.c_int]),
         "scn_background_sums": (C.c_int, [vp, vp, i64, C.c_int, vp, C.c_int, C.c_int]),
         "scn_positions_pitch": (i64, [i64]),
@@ -431,12 +432,12 @@ class Context:
         _check(lib().scn_conv_input_gradient(self.h, d_delta.ptr, d_inverse.ptr, fs, N, d_Wt.ptr, d_image.ptr if d_image is not None else None, d_din.ptr,
                                              inputRows, nIn))
 
-    def weight_images_many(self, items):
+    def weight_images_many(self, items, later=False):
         """items: (d_W, d_image, K, N, fs, precision) tuples"""
         arr = (ImageItem * max(1, len(items)))()
         for k, (w, image, K, n, fs, precision) in enumerate(items):
             arr[k] = ImageItem(w.ptr, image.ptr, K, n, fs, precision)
-        _check(lib().scn_weight_images_many(self.h, arr, len(items)))
+        _check((lib().scn_weight_images_later if later else lib().scn_weight_images_many)(self.h, arr, len(items)))
 
     def conv_nin_forward_image(self, d_in, d_rules, fs, nIn, d_W, d_image, d_B, d_prelu, d_out, M, N, p, act, precision):
         _check(lib().scn_conv_nin_forward_image(self.h, d_in.ptr, d_rules.ptr if d_rules is not None else None, fs, nIn, d_W.ptr, d_image.ptr if d_image is not None else None, d_B.ptr,

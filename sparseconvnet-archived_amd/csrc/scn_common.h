@@ -47,6 +47,14 @@ struct ProfSpan {
 #define SCN_IMAGE_BYTES (16u << 20)
 #define SCN_MAX_PENDING 62 // plans per settle; 16 + 4 * 62 = 264 pinned words
 #define SCN_PINNED_WORDS (16 + 4 * SCN_MAX_PENDING)
+// images of weights to be made (weight_image, scn_image_dev.h)
+struct ImageList {
+  const float *W[SCN_IMAGES_MAX];
+  unsigned char *image[SCN_IMAGES_MAX];
+  unsigned firstBlock[SCN_IMAGES_MAX + 1];
+  int K[SCN_IMAGES_MAX], N[SCN_IMAGES_MAX], fs[SCN_IMAGES_MAX], planes[SCN_IMAGES_MAX];
+  int count;
+};
 struct scn_ctx {
   int device;
   hipStream_t stream;
@@ -77,6 +85,7 @@ struct scn_ctx {
   std::vector<RowsChosen> rowsChosen;
   bool rowsHeld;
   struct ChainState *chain; // recorded rule-book plans (scn_chain.hip)
+  ImageList imagesLater; // scn_weight_images_later's, until a launch takes them along
   // profiling
   bool prof;
   int profTag;

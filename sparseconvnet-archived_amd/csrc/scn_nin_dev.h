@@ -79,6 +79,8 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
 // rules, position by position)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                    long long M, int K, int N, const GatherSource *gs = nullptr);
+// what scn_weight_images_later left, made now
+int scn_images_now(scn_ctx *ctx);
 int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems);
 // out = A Wt^T; false: the caller's other way, or (transpose) scn_planes_forward
 // on the transpose

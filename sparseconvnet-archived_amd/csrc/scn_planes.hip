@@ -16,35 +16,12 @@
 // v_mfma_f32_32x32x16_bf16 does 32768 flops in 32 cycles, v_mfma_f32_32x32x2_f32
 // 4096 in 64, so six of the former are 2.7 times as fast.
 //   PL 3: SCN_FP32; PL 2: SCN_BF16X3 (hi hi, hi lo, lo hi); PL 1: SCN_BF16.
-#include "scn_nin_dev.h"
+#include "scn_image_dev.h"
 #include <math.h>
 #include <utility>
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-// The PL planes of two floats, a word each.
-template <int PL> __device__ __forceinline__ void split2(float a, float b, unsigned (&w)[PL]) {
-#pragma unroll
-  for (int l = 0; l < PL; ++l) {
-    w[l] = pack_bf16x2(a, b);
-    if (l + 1 < PL) {
-      a -= __uint_as_float(w[l] << 16);
-      b -= __uint_as_float(w[l] & 0xffff0000u);
-    }
-  }
-}
-// The PL planes of eight floats, each as an MFMA operand.
-template <int PL>
-__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&p)[PL]) {
-  unsigned w[4][PL];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    split2<PL>(x[2 * i], x[2 * i + 1], w[i]);
-#pragma unroll
-  for (int l = 0; l < PL; ++l)
-    p[l] = __builtin_bit_cast(bf16x8, uint4{w[0][l], w[1][l], w[2][l], w[3][l]});
-}
 
 bool scn_planes_shape(int K) { return K % 32 == 0 && K >= 64; }
 
@@ -1264,54 +1241,7 @@ __global__ void __launch_bounds__(256)
                                 (kg & 1) * 512 + cc * 16) = p[l];
 }
 
-// The image of W that k_nin_lines reads: a chunk of 1 KB for every tile of 32
-// columns, block of 32 k, plane and step of 16 k, in that order.  Those of several
-// layers in one launch (each by itself takes 3 us, whatever it holds).
-//   fs 0: W is [K x N]; -1: [N x K]; more: the filters of the layer whose input's
-//   gradient this is, [fs N x K / fs], its rule positions in the same order.
-struct ImageList {
-  const float *W[SCN_IMAGES_MAX];
-  unsigned char *image[SCN_IMAGES_MAX];
-  unsigned firstBlock[SCN_IMAGES_MAX + 1];
-  int K[SCN_IMAGES_MAX], N[SCN_IMAGES_MAX], fs[SCN_IMAGES_MAX], planes[SCN_IMAGES_MAX];
-  int count;
-};
-template <int PL>
-__device__ __forceinline__ void weight_image(const float *__restrict__ W, unsigned char *__restrict__ image, int K, int N,
-                                             int fs, long long item) {
-  const int T = K / 32, columns = (N + 31) / 32 * 32;
-  if (item >= (long long)T * 4 * columns)
-    return;
-  const int column = (int)(item % columns), kg = (int)(item / columns); // (eight k, column)
-  const int n = column < N ? column : N - 1, k = 8 * kg;
-  float v[8];
-  if (fs == 0) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      v[i] = W[(long long)(k + i) * N + n];
-  } else {
-    const int width = fs < 0 ? K : K / fs, f = k / width; // (a multiple of 8)
-    const float *const src = W + ((long long)f * N + n) * width + (k - f * width);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      v[i] = src[i];
-  }
-  bf16x8 p[PL];
-  split8<PL>(v, p);
-#pragma unroll
-  for (int l = 0; l < PL; ++l)
-    *reinterpret_cast<bf16x8 *>(image + ((((long long)(column / 32) * T + kg / 4) * PL + l) * 2 + kg / 2 % 2) * 1024 +
-                                (kg & 1) * 512 + (column & 31) * 16) = p[l];
-}
-__global__ void __launch_bounds__(256) k_weight_images(ImageList l) {
-  const int lane = threadIdx.x & 63;
-  const int x = __popcll(__ballot(lane < l.count && blockIdx.x >= l.firstBlock[lane < SCN_IMAGES_MAX ? lane : 0])) - 1;
-  const long long item = (long long)(blockIdx.x - l.firstBlock[x]) * 256 + threadIdx.x;
-  if (l.planes[x] == 3)
-    weight_image<3>(l.W[x], l.image[x], l.K[x], l.N[x], l.fs[x], item);
-  else
-    weight_image<1>(l.W[x], l.image[x], l.K[x], l.N[x], l.fs[x], item);
-}
+__global__ void __launch_bounds__(256) k_weight_images(ImageList l) { weight_images_block(l, blockIdx.x); }
 static int64_t image_bytes(int planes, int K, int N) { return (int64_t)scn_ceil_div(N, 32) * 32 * K * 2 * planes; }
 // What k_nin_lines takes: three planes or one, blocks within one filter position, 64
 // rows of the output within the gigabyte that its stores reach (columns that there are
@@ -1731,12 +1661,11 @@ extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N,
     return 0;
   return image_bytes(planes, K, N);
 }
-extern "C" int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items, int nItems) {
+static int image_list(scn_ctx *ctx, const scn_image_item *items, int nItems, ImageList &l) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_weight_images_many: null context");
   SCN_REQUIRE(nItems >= 0 && nItems <= SCN_IMAGES_MAX && (items || nItems == 0), SCN_ERR_ARG,
               "scn_weight_images_many: %d items (at most %d)", nItems, SCN_IMAGES_MAX);
   static_assert(SCN_IMAGES_MAX <= 64, "a lane an item");
-  ImageList l;
   l.count = 0, l.firstBlock[0] = 0;
   long long blocks = 0;
   for (int k = 0; k < nItems; ++k) {
@@ -1750,8 +1679,35 @@ extern "C" int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items,
     SCN_REQUIRE(blocks <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_weight_images_many: %lld workgroups", blocks);
     add_image(l, it.d_W, (unsigned char *)it.d_image, planes, it.K, it.N, it.fs);
   }
+  return SCN_OK;
+}
+extern "C" int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items, int nItems) {
+  ImageList l;
+  SCN_TRY(image_list(ctx, items, nItems, l));
   ProfScope prof(ctx, SCN_K_NIN);
   SCN_TRY(weight_images(ctx, l));
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+// (what an earlier call left and nobody has asked for is given up: its images may be
+// gone)
+extern "C" int scn_weight_images_later(scn_ctx *ctx, const scn_image_item *items, int nItems) {
+  if (ctx)
+    ctx->imagesLater.count = 0;
+  ImageList l;
+  SCN_TRY(image_list(ctx, items, nItems, l));
+  ctx->imagesLater = l;
+  return SCN_OK;
+}
+int scn_images_now(scn_ctx *ctx) {
+  ImageList &l = ctx->imagesLater;
+  if (l.count == 0)
+    return SCN_OK;
+  const int n = l.count;
+  l.count = 0;
+  ImageList now = l;
+  now.count = n;
+  SCN_TRY(weight_images(ctx, now));
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
 }

@@ -544,8 +544,11 @@ void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStr
     at += room(x.bytes);
   }
   scn_prof_tag(ms.ctx, -1); // (no layer's)
-  for (size_t i = 0; i < items.size(); i += SCN_IMAGES_MAX)
-    SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, (int)std::min<size_t>(SCN_IMAGES_MAX, items.size() - i)));
+  // (the last of them beside the first layer, where that takes them along)
+  size_t i = 0;
+  for (; i + SCN_IMAGES_MAX < items.size(); i += SCN_IMAGES_MAX)
+    SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, SCN_IMAGES_MAX));
+  SCN_CHECKED(scn_weight_images_later(ms.ctx, items.data() + i, (int)(items.size() - i)));
 }
 // The two halves of processBatch.  forwardBatch only queues work on the net's
 // stream (every layer, then the copy of the probabilities to the host);

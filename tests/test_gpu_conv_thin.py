@@ -24,3 +24,40 @@ def test_thin_convolution(scn, ctx, rows, fs, nIn, N):
     got, want = one.download(), two.download()
     assert np.all(got[rows:] == 7)
     assert np.array_equal(got, want)
+
+
+# one group of rows and two; columns in one slice and in two, of which one makes the images; images of one workgroup and of
+# many, of three planes and one; and images that no first layer takes along, made before the layer that is given one
+@pytest.mark.parametrize("M,N", [(900, 32), (70001, 160), (600, 300), (0, 32)])
+@pytest.mark.parametrize("shapes", [[(64, 32)], [(256, 96), (640, 320), (64, 4)]])
+def test_images_beside_a_first_layer(scn, ctx, M, N, shapes):
+    rng = np.random.default_rng(M + N)
+    items, want = [], []
+    for k, (K, n) in enumerate(shapes):
+        precision = scn.BF16 if k == 1 else scn.FP32_PLANES
+        W = ctx.array(rng.standard_normal((K, n), dtype=np.float32))
+        words = K * ((n + 31) // 32 * 32) * (3 if precision == scn.FP32_PLANES else 1) // 2
+        now, later = (ctx.array(np.full(words, 7, np.int32)) for _ in range(2))
+        ctx.weight_images_many([(W, now, K, n, 0, precision)])
+        items.append((W, later, K, n, 0, precision))
+        want.append(now)
+    x = rng.standard_normal((500, 3), dtype=np.float32)
+    rules = rng.integers(-1, 500, (max(M, 1), 4)).astype(np.int32)
+    W, B = rng.standard_normal((12, N), dtype=np.float32), rng.standard_normal(N, dtype=np.float32)
+    args = ctx.array(x), ctx.array(rules), 4, 3, ctx.array(W), ctx.array(B), None
+    one, two = (ctx.array(np.full((M + 8, N), 7, np.float32)) for _ in range(2))
+    print("images beside", M, N, shapes, flush=True)
+    ctx.conv_nin_forward(*args, one, M, N)
+    ctx.weight_images_many(items, later=True)
+    ctx.conv_nin_forward(*args, two, M, N)
+    assert np.array_equal(one.download(), two.download())
+    K, n = shapes[0]
+    if M == 0:  # (nothing has been launched: the layer that reads its image has it made)
+        A, out = ctx.array(rng.standard_normal((300, K), dtype=np.float32)), [ctx.empty((300, n), np.float32) for _ in range(2)]
+        bias = ctx.array(np.zeros(n, np.float32))
+        for o, im in zip(out, (want[0], items[0][1])):
+            scn._check(scn.lib().scn_conv_nin_forward_image(ctx.h, A.ptr, None, 1, K, items[0][0].ptr, im.ptr, bias.ptr, None, o.ptr,
+                                                            300, n, 1.0, scn.NOSIGMOID, scn.FP32_PLANES))
+        assert np.array_equal(out[0].download(), out[1].download())
+    for now, (_, later, *_) in zip(want, items):
+        assert np.array_equal(now.download(), later.download())
