@@ -366,6 +366,9 @@ int scn_softmax_rows(scn_ctx *ctx, const float *d_in, float *d_out, int64_t M,
 int scn_softmax_grad(scn_ctx *ctx, const float *d_probs,
                      const int32_t *d_labels, float *d_delta, int64_t batch,
                      int N);
+/* ... and the probabilities to `copy`, device or pinned host memory */
+int scn_softmax_grad_copy(scn_ctx *ctx, const float *d_probs, const int32_t *d_labels, float *d_delta, int64_t batch, int N,
+                          float *copy);
 /* What NetworkInNetwork(PReLU)Layer::backwards does to the output gradient
  * before the two matrix products: applySigmoidBackProp in place
  * (NetworkInNetworkLayer.cu:222, SigmoidLayer.cu:23-177 and :224-262; the
@@ -522,6 +525,9 @@ typedef struct scn_filter_item {
   int32_t fs, nIn, N;
 } scn_filter_item;
 int scn_transpose_filters_many(scn_ctx *ctx, const scn_filter_item *items, int nItems);
+/* scn_fill32_many with zeros and scn_transpose_filters_many in one launch */
+int scn_gradients_begin(scn_ctx *ctx, void *const *d_clear, const size_t *nWords, int nClear,
+                        const scn_filter_item *items, int nItems);
 int scn_conv_input_gradient(scn_ctx *ctx, const float *d_delta, const int32_t *d_inverse, int fs, int N,
                             const float *d_Wt, const void *d_image, float *d_din, int64_t inputRows, int nIn);
 int scn_conv_AtB(scn_ctx *ctx, const float *d_in, const int32_t *d_positions, int fs, int nIn,

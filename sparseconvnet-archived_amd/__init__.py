@@ -172,6 +172,8 @@ def lib():
         "scn_AtB_many": (C.c_int, [vp, P(AtbItem), C.c_int]),
         "scn_sgemm_AtB_sums": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, C.c_int, C.c_int]),
         "scn_maxpool_backward_through": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, C.c_int]),
+        "scn_gradients_begin": (C.c_int, [vp, P(vp), P(sz), C.c_int, P(FilterItem), C.c_int]),
+        "scn_softmax_grad_copy": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, vp]),
         "scn_pool_inverse_slots": (C.c_int, [C.c_int, C.c_int, C.c_int]),
         "scn_pool_inverse_many": (C.c_int, [vp, P(PoolInverseItem), C.c_int]),
         "scn_maxpool_gradient": (C.c_int, [vp, vp, i64, vp, i64, C.c_int, vp, vp, C.c_int, vp, C.c_int, vp, C.c_int, vp,

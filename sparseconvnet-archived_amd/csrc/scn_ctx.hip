@@ -261,44 +261,17 @@ extern "C" int scn_d2d(scn_ctx *c, void *d_dst, const void *d_src,
   return scn_copy(c, d_dst, d_src, bytes);
 }
 
-// Four words a store between the ends that are not on 16 bytes: the fills of the
-// backward kernels of a middle layer (77 MB and less) 9.2 -> 7.0 us on average.
-__device__ __forceinline__ void fill32(uint32_t *dst, uint32_t w, size_t n, size_t i, size_t step) {
-  const size_t off = (16 - ((uintptr_t)dst & 15) & 15) / 4;
-  const size_t head = off < n ? off : n, quads = (n - head) / 4, tail = head + 4 * quads;
-  uint4 *const body = reinterpret_cast<uint4 *>(dst + head);
-  for (size_t q = i; q < quads; q += step)
-    body[q] = make_uint4(w, w, w, w);
-  if (i < head)
-    dst[i] = w;
-  if (i < n - tail)
-    dst[tail + i] = w;
-}
 __global__ __launch_bounds__(256) void k_fill32(uint32_t *dst, uint32_t w, size_t n) {
   fill32(dst, w, n, (size_t)blockIdx.x * 256 + threadIdx.x, (size_t)gridDim.x * 256);
 }
 
-// Several buffers in one launch (a launch of its own is 2 us and the gap before
-// it): a workgroup finds its buffer from the running workgroup counts.
-struct FillList {
-  uint32_t *dst[SCN_FILL_MAX];
-  size_t n[SCN_FILL_MAX];
-  unsigned firstBlock[SCN_FILL_MAX + 1];
-  int count;
-};
-__global__ __launch_bounds__(256) void k_fill32_many(FillList l, uint32_t w) {
-  int t = 0;
-  while (t + 1 < l.count && blockIdx.x >= l.firstBlock[t + 1])
-    ++t;
-  const unsigned blocks = l.firstBlock[t + 1] - l.firstBlock[t];
-  fill32(l.dst[t], w, l.n[t], (size_t)(blockIdx.x - l.firstBlock[t]) * 256 + threadIdx.x, (size_t)blocks * 256);
-}
+__global__ __launch_bounds__(256) void k_fill32_many(FillList l, uint32_t w) { fill32_list_block(l, w, blockIdx.x); }
 
-extern "C" int scn_fill32_many(scn_ctx *c, void *const *d_dst,
-                               const size_t *nWords, int n, uint32_t word) {
+// (the list, and how many workgroups go through it)
+int scn_fill_list(scn_ctx *c, void *const *d_dst, const size_t *nWords, int n, FillList *list, unsigned *blocksOf) {
   SCN_REQUIRE(c && n >= 0 && n <= SCN_FILL_MAX && ((d_dst && nWords) || n == 0), SCN_ERR_ARG,
               "scn_fill32_many: %d buffers (at most %d)", n, SCN_FILL_MAX);
-  FillList l;
+  FillList &l = *list;
   l.count = 0;
   unsigned total = 0;
   for (int k = 0; k < n; ++k) {
@@ -311,9 +284,17 @@ extern "C" int scn_fill32_many(scn_ctx *c, void *const *d_dst,
     l.firstBlock[l.count++] = total;
     total += (unsigned)(blocks < 65536 ? blocks : 65536);
   }
-  if (l.count == 0)
-    return SCN_OK;
   l.firstBlock[l.count] = total;
+  *blocksOf = total;
+  return SCN_OK;
+}
+extern "C" int scn_fill32_many(scn_ctx *c, void *const *d_dst,
+                               const size_t *nWords, int n, uint32_t word) {
+  FillList l;
+  unsigned total = 0;
+  SCN_TRY(scn_fill_list(c, d_dst, nWords, n, &l, &total));
+  if (total == 0)
+    return SCN_OK;
   hipLaunchKernelGGL(k_fill32_many, dim3(total), dim3(256), 0, c->stream, l, word);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;

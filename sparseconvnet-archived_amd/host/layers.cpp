@@ -1235,21 +1235,28 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
     // (SoftmaxClassifier.cu:22-31)
     input.sub->dfeatures.resize64((size_t)input.nSpatialSites *
                                   input.nFeatures);
-    SCN_CHECKED(scn_softmax_grad(memStream.ctx, input.sub->features.dPtr(),
-                                 batch.labels.dPtr(),
-                                 input.sub->dfeatures.dPtr(), batch.batchSize,
-                                 input.nFeatures));
   }
   BatchResultStage &r = *batch.result;
   const size_t n = (size_t)batch.batchSize * input.nFeatures;
   result_room(r, n, memStream);
+  const bool small = n <= ((size_t)1 << 18), along = batch.type == TRAINBATCH && small && !r.copied;
+  if (along) // (the gradient's kernel reads them anyway)
+    SCN_CHECKED(scn_softmax_grad_copy(memStream.ctx, input.sub->features.dPtr(), batch.labels.dPtr(),
+                                      input.sub->dfeatures.dPtr(), batch.batchSize, input.nFeatures, r.pinned));
+  else if (batch.type == TRAINBATCH)
+    SCN_CHECKED(scn_softmax_grad(memStream.ctx, input.sub->features.dPtr(),
+                                 batch.labels.dPtr(),
+                                 input.sub->dfeatures.dPtr(), batch.batchSize,
+                                 input.nFeatures));
   if (!r.arrived)
     SCN_CHECKED(scn_event_create(memStream.ctx, &r.arrived));
   // a kernel copies what a batch usually has: queueing it takes the host a
   // fifth of the time of an asynchronous memcpy
   if (r.copied)
     r.copied = false;
-  else if (n <= ((size_t)1 << 18))
+  else if (along)
+    ;
+  else if (small)
     SCN_CHECKED(scn_copy(memStream.ctx, r.pinned, input.sub->features.dPtr(),
                          n * sizeof(float)));
   else

@@ -476,13 +476,14 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
       n = 0;
     }
   }
-  SCN_CHECKED(scn_fill32_many(memStream.ctx, grads, sizes, n, 0u));
   std::vector<scn_filter_item> filters;
   for (size_t i = 0; i < layers.size(); i++)
     layers[i]->transposedFilters(batch.interfaces[i], filters);
-  for (size_t i = 0; i < filters.size(); i += SCN_FILTERS_MAX)
-    SCN_CHECKED(scn_transpose_filters_many(memStream.ctx, filters.data() + i,
-                                           (int)std::min<size_t>(SCN_FILTERS_MAX, filters.size() - i)));
+  for (size_t i = 0; i == 0 || i < filters.size(); i += SCN_FILTERS_MAX) {
+    SCN_CHECKED(scn_gradients_begin(memStream.ctx, grads, sizes, n, filters.data() + i,
+                                    (int)std::min<size_t>(SCN_FILTERS_MAX, filters.size() - i)));
+    n = 0;
+  }
   batch.updates.clear();
   batch.products.clear();
   batch.collectUpdates = true;

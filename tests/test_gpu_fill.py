@@ -1,5 +1,7 @@
 """Memory that is written whole without being cleared first: fills at any alignment, the masks and scan states of rule
 books whose objects were used for other sites before."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -61,3 +63,37 @@ def test_rule_books_on_used_objects(scn, ctx, d, field, samples, size, stride):
         full = (mask.reshape(samples, -1).sum(1) == out ** d).sum()
         assert results[0][0] == mask.sum() + samples - full or results[0][0] == mask.sum() + samples
         assert all(np.array_equal(a, b) for a, b in zip(*results))
+
+
+# buffers and filters in one launch, either without the other; buffers that end off 16 bytes, none, one past a workgroup's share
+@pytest.mark.parametrize("sizes", [[], [1], [1025, 0, 70000, 3]])
+@pytest.mark.parametrize("filters", [[], [(4, 32, 64)], [(1, 3, 33), (8, 96, 32), (4, 31, 5)]])
+def test_a_backward_pass_begins(scn, ctx, sizes, filters):
+    rng = np.random.default_rng(len(sizes) + 8 * len(filters))
+    bufs = [ctx.array(np.full(n + 4, 7, np.int32)) for n in sizes]
+    Ws = [rng.standard_normal((fs, nIn, N), dtype=np.float32) for fs, nIn, N in filters]
+    outs = [ctx.array(np.full(W.size, 7, np.float32)) for W in Ws]
+    held = [ctx.array(W) for W in Ws]
+    ptrs = (C.c_void_p * max(1, len(sizes)))(*[b.ptr for b in bufs])
+    words = (C.c_size_t * max(1, len(sizes)))(*sizes)
+    items = (scn.FilterItem * max(1, len(filters)))(*[scn.FilterItem(w.ptr, o.ptr, *f) for w, o, f in zip(held, outs, filters)])
+    print("backward begins", sizes, filters, flush=True)
+    scn._check(scn.lib().scn_gradients_begin(ctx.h, ptrs, words, len(sizes), items, len(filters)))
+    for b, n in zip(bufs, sizes):
+        got = b.download()
+        assert np.all(got[:n] == 0) and np.all(got[n:] == 7)
+    for W, o in zip(Ws, outs):
+        assert np.array_equal(o.download().reshape(W.shape[0], W.shape[2], W.shape[1]), W.transpose(0, 2, 1))
+
+
+@pytest.mark.parametrize("batch,N", [(1, 3), (100, 100), (257, 40)])
+def test_classifier_gradient_with_a_copy(scn, ctx, batch, N):
+    rng = np.random.default_rng(batch)
+    p, labels = rng.random((batch, N), dtype=np.float32), rng.integers(0, N, batch).astype(np.int32)
+    delta, copy = (ctx.array(np.full((batch, N), 7, np.float32)) for _ in range(2))
+    held = ctx.array(p), ctx.array(labels)
+    print("gradient and copy", batch, N, flush=True)
+    scn._check(scn.lib().scn_softmax_grad_copy(ctx.h, held[0].ptr, held[1].ptr, delta.ptr, batch, N, copy.ptr))
+    want = p.copy()
+    want[np.arange(batch), labels] -= 1
+    assert np.array_equal(delta.download(), want) and np.array_equal(copy.download(), p)
