@@ -1694,6 +1694,8 @@ extern "C" int scn_weight_images_many(scn_ctx *ctx, const scn_image_item *items,
 extern "C" int scn_weight_images_later(scn_ctx *ctx, const scn_image_item *items, int nItems) {
   if (ctx)
     ctx->imagesLater.count = 0;
+  if (ctx && ctx->prof) // (a launch of its own, which is no layer's, where layers are timed)
+    return nItems == 0 ? SCN_OK : scn_weight_images_many(ctx, items, nItems);
   ImageList l;
   SCN_TRY(image_list(ctx, items, nItems, l));
   ctx->imagesLater = l;

@@ -498,6 +498,7 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   batch.collectUpdates = false;
   for (size_t i = 1; i < batch.interfaces.size(); i++)
     batch.interfaces[i].sub->turnedImage = nullptr;
+  SCN_CHECKED(scn_weight_images_later(memStream.ctx, nullptr, 0));
   scn_prof_tag(memStream.ctx, -1); // (no layer's)
   for (size_t i = 0; i < batch.products.size(); i += SCN_ATB_MAX)
     SCN_CHECKED(scn_AtB_many(memStream.ctx, batch.products.data() + i,
@@ -594,6 +595,9 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
     SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
   for (size_t i = 1; i < batch.interfaces.size(); i++) // (what no layer has taken)
     batch.interfaces[i].sub->weightImage = nullptr;
+  // what no launch has made (a batch of no rows) does not outlast the pass
+  if (batch.type != TRAINBATCH)
+    SCN_CHECKED(scn_weight_images_later(ms.ctx, nullptr, 0));
   SoftmaxClassifierLaunch(batch.interfaces.back(), batch, ms);
 }
 void SparseConvNetCUDA::finishBatch(SpatiallySparseBatch &batch,
