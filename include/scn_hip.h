@@ -482,6 +482,10 @@ int scn_weight_images_later(scn_ctx *ctx, const scn_image_item *items, int nItem
 int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn, const float *d_W,
                                const void *d_image, const float *d_B, const float *d_prelu, float *d_out, int64_t M, int N,
                                float p, int act, int precision);
+/* scn_gather_rows to d_matrix and scn_nin_forward of it, for a few channels in one launch */
+int scn_conv_nin_forward_matrix(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn,
+                                float *d_matrix, const float *d_W, const float *d_B, const float *d_prelu,
+                                float *d_out, int64_t M, int N, float p, int act, int precision);
 /* The backward pass of a convolution without its gathered matrix (no
  * counterpart in the reference, which keeps that matrix and its gradient).
  * scn_rules_inverse_many turns the rules of up to SCN_INVERSE_MAX layers round:

@@ -183,6 +183,7 @@ def lib():
         "scn_weight_image_bytes": (i64, [vp, i64, C.c_int, C.c_int, C.c_int, C.c_int]),
         "scn_weight_images_many": (C.c_int, [vp, P(ImageItem), C.c_int]),
         "scn_weight_images_later": (C.c_int, [vp, P(ImageItem), C.c_int]),
+        "scn_conv_nin_forward_matrix": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, C.c_int, f32, C.c_int, C.c_int]),
         "scn_conv_nin_forward_image": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, C.c_int, f32, C.c_int, C.c_int]),
         "scn_background_sums": (C.c_int, [vp, vp, i64, C.c_int, vp, C.c_int, C.c_int]),
         "scn_positions_pitch": (i64, [i64]),

@@ -514,10 +514,11 @@ __global__ void __launch_bounds__(256)
 // at 66500 x 12 x 160 and 83597 x 12 x 32 two are ahead (16.8, 8.3 with one).
 #define CT_COLS 256
 #define CT_PITCH (TK_MAX_K + 4) // floats: eight rows' reads of four k lie on all banks
-template <int CT_GROUPS>
+template <int CT_GROUPS, bool MATRIX>
 __device__ __forceinline__ void conv_thin_block(const float *__restrict__ A, const float *__restrict__ W,
-                                                float *__restrict__ out, long long M, int K, int N, const Epilogue &ep,
-                                                const GatherSource &gs, const long long *dRows, unsigned block) {
+                                                float *__restrict__ out, float *__restrict__ matrix, long long M,
+                                                int K, int N, const Epilogue &ep, const GatherSource &gs,
+                                                const long long *dRows, unsigned block) {
   M = live_rows(M, dRows);
   const unsigned tiles = (unsigned)((M + 32 * CT_GROUPS - 1) / (32 * CT_GROUPS));
   if (block >= tiles)
@@ -555,6 +556,8 @@ __device__ __forceinline__ void conv_thin_block(const float *__restrict__ A, con
       if (rule[g][j] >= 0)
         v = A[(long long)rule[g][j] * gs.nIn + (k - gather_rule_of(gs, k) * gs.nIn)];
       sA[(32 * g + r) * CT_PITCH + k] = v;
+      if (MATRIX && n0 == 0 && k < K && mFirst + 32 * g < M)
+        matrix[(mFirst + 32 * g) * K + k] = v;
     }
   __syncthreads();
   const float *const arow = sA + r * CT_PITCH;
@@ -598,30 +601,30 @@ __device__ __forceinline__ void conv_thin_block(const float *__restrict__ A, con
   }
 }
 
-template <int CT_GROUPS>
+template <int CT_GROUPS, bool MATRIX>
 __global__ void __launch_bounds__(256)
     k_conv_thin(const float *__restrict__ A, const float *__restrict__ W,
-                float *__restrict__ out, long long M, int K, int N, Epilogue ep,
+                float *__restrict__ out, float *__restrict__ matrix, long long M, int K, int N, Epilogue ep,
                 GatherSource gs, const long long *dRows) {
-  conv_thin_block<CT_GROUPS>(A, W, out, M, K, N, ep, gs, dRows, blockIdx.x);
+  conv_thin_block<CT_GROUPS, MATRIX>(A, W, out, matrix, M, K, N, ep, gs, dRows, blockIdx.x);
 }
 // A net's first layer and, by workgroups before its own, the images of the weights of
 // the layers behind it, which by themselves are a launch of 4.4 to 10 us: 61 images in
 // the wide net 367 -> 358 us, 128 in bf16 354 -> 340, 100 drawings 193 -> 191.
-template <int CT_GROUPS>
+template <int CT_GROUPS, bool MATRIX>
 __global__ void __launch_bounds__(256)
     k_conv_thin_images(ImageList images, unsigned imageBlocks, const float *__restrict__ A, const float *__restrict__ W,
-                       float *__restrict__ out, long long M, int K, int N, Epilogue ep,
+                       float *__restrict__ out, float *__restrict__ matrix, long long M, int K, int N, Epilogue ep,
                        GatherSource gs, const long long *dRows) {
   if (blockIdx.x >= imageBlocks)
-    conv_thin_block<CT_GROUPS>(A, W, out, M, K, N, ep, gs, dRows, blockIdx.x - imageBlocks);
+    conv_thin_block<CT_GROUPS, MATRIX>(A, W, out, matrix, M, K, N, ep, gs, dRows, blockIdx.x - imageBlocks);
   else if (blockIdx.y == 0 && blockIdx.x < images.firstBlock[images.count])
     weight_images_block(images, blockIdx.x);
 }
 
-template <int G>
-static void launch_conv_thin(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
-                             const Epilogue &ep, const GatherSource &gs, const long long *dRows) {
+template <int G, bool MATRIX>
+static void launch_conv_thin(scn_ctx *ctx, const float *A, const float *W, float *out, float *matrix, long long M, int K,
+                             int N, const Epilogue &ep, const GatherSource &gs, const long long *dRows) {
   const size_t lds = (size_t)(G * 32 * CT_PITCH + K * (N < CT_COLS ? N : CT_COLS)) * sizeof(float);
   dim3 grid(scn_ceil_div(M, 32 * G), scn_ceil_div(N, CT_COLS));
   if (ctx->imagesLater.count) {
@@ -629,11 +632,11 @@ static void launch_conv_thin(scn_ctx *ctx, const float *A, const float *W, float
     ctx->imagesLater.count = 0;
     const unsigned blocks = (images.firstBlock[images.count] + 7) / 8 * 8; // (the layer's own keep their XCDs)
     grid.x += blocks;
-    hipLaunchKernelGGL(k_conv_thin_images<G>, grid, dim3(256), lds, ctx->stream, images, blocks, A, W, out, M, K, N, ep, gs,
-                       dRows);
+    hipLaunchKernelGGL((k_conv_thin_images<G, MATRIX>), grid, dim3(256), lds, ctx->stream, images, blocks, A, W, out, matrix, M, K,
+                       N, ep, gs, dRows);
     return;
   }
-  hipLaunchKernelGGL(k_conv_thin<G>, grid, dim3(256), lds, ctx->stream, A, W, out, M, K, N, ep, gs, dRows);
+  hipLaunchKernelGGL((k_conv_thin<G, MATRIX>), grid, dim3(256), lds, ctx->stream, A, W, out, matrix, M, K, N, ep, gs, dRows);
 }
 
 // ---- MFMA path: fp32 operands, v_mfma_f32_32x32x2_f32 ----------------------
@@ -1848,12 +1851,13 @@ static void launch_mfma(scn_ctx *ctx, const float *A, const float *W,
 // size.
 #define PLANES_MIN_FLOPS 4e10
 // rows16: a bf16 copy of the matrix the rules point into, or null; image: the
-// weights for the planes (scn_weight_images_many), or null
+// weights for the planes (scn_weight_images_many), or null; matrix: where
+// k_conv_thin, which it asks for, is to leave the rows, or null
 static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
                        const float *d_B, const float *d_prelu, float *d_out,
                        int64_t M, int K, int N, float p, int act, int precision,
                        const GatherSource *gs, const void *rows16 = nullptr,
-                       const void *image = nullptr) {
+                       const void *image = nullptr, float *matrix = nullptr) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_nin_forward: null context");
   SCN_REQUIRE(M >= 0 && K >= 1 && N >= 1, SCN_ERR_ARG,
               "scn_nin_forward: M %lld K %d N %d", (long long)M, K, N);
@@ -1885,7 +1889,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   const long long *const dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   const bool rounded = precision == SCN_BF16 || precision == SCN_BF16X3; // operands
   const bool shape = vec && scn_planes_shape(K);
-  const bool few = K <= FR_MAX_K && !(shape && N % 16 == 0);
+  const bool few = !matrix && K <= FR_MAX_K && !(shape && N % 16 == 0);
   bool fewRows = few && scn_rows_hint(ctx, M) <= FR_MAX_M;
   auto takes_planes = [&]() {
     return shape && ((rounded && act != SCN_SOFTMAX) || precision == SCN_FP32_PLANES ||
@@ -1902,7 +1906,9 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
     fewRows = few && M <= FR_MAX_M;
     planes = takes_planes();
   }
-  if (few && !(planes && rounded))
+  if (matrix)
+    scn_rows_chosen(ctx, FR_MAX_M, 1ll << 62);
+  else if (few && !(planes && rounded))
     scn_rows_chosen(ctx, fewRows ? -1 : FR_MAX_M, fewRows ? FR_MAX_M : 1ll << 62);
   // bf16 operands only where the contraction is big enough to matter; the
   // classifier head and the thin first layers stay fp32
@@ -1942,10 +1948,10 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
     }
   } else if (vec && gs && gs->nIn % 4 != 0) {
     // channels in other than fours: K <= TK_MAX_K (scn_conv_nin_supported)
-    if (scn_rows_hint(ctx, M) <= 6ll * 32 * ctx->numCU)
-      launch_conv_thin<1>(ctx, d_A, d_W, d_out, (long long)M, K, N, ep, *gs, dRows);
-    else
-      launch_conv_thin<2>(ctx, d_A, d_W, d_out, (long long)M, K, N, ep, *gs, dRows);
+    const bool one = scn_rows_hint(ctx, M) <= 6ll * 32 * ctx->numCU;
+    auto *const launch = matrix ? (one ? launch_conv_thin<1, true> : launch_conv_thin<2, true>)
+                                : (one ? launch_conv_thin<1, false> : launch_conv_thin<2, false>);
+    launch(ctx, d_A, d_W, d_out, matrix, (long long)M, K, N, ep, *gs, dRows);
   } else if (vec && !gs && K <= TK_MAX_K) {
     hipLaunchKernelGGL(k_nin_thin, dim3(scn_ceil_div(M, 32), scn_ceil_div(N, 32)),
                        dim3(256), 0, ctx->stream, d_A, d_W, d_out, (long long)M,
@@ -2127,6 +2133,32 @@ extern "C" int scn_conv_nin_forward_p(scn_ctx *ctx, const float *d_in,
                                       int64_t M, int N, float p, int act,
                                       int precision) {
   return conv_nin_forward(ctx, d_in, d_rules, fs, nIn, d_W, nullptr, d_B, d_prelu, d_out, M, N, p, act, precision);
+}
+// The matrix of a convolution of few channels (scn_gather_rows) and the contraction of
+// its rows in one launch: k_conv_thin holds the rows anyway.  The first layer of
+// 33 voxel fields, 8 x 1 channels, and its matrix: 9.7 us with the images beside it, 18.9
+// in three launches (6.2 the rows, 8.6 k_nin_thin, 4.1 the images); the batch 198 -> 189.
+// No fewer rows than k_nin_fewrows is for, which is ahead there.
+extern "C" int scn_conv_nin_forward_matrix(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn,
+                                           float *d_matrix, const float *d_W, const float *d_B, const float *d_prelu,
+                                           float *d_out, int64_t M, int N, float p, int act, int precision) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_nin_forward_matrix: null context");
+  SCN_REQUIRE(fs >= 1 && nIn >= 1 && (int64_t)fs * nIn <= 0x7fffffff, SCN_ERR_ARG,
+              "scn_conv_nin_forward_matrix: fs %d nIn %d", fs, nIn);
+  SCN_REQUIRE((d_matrix && d_rules) || M == 0, SCN_ERR_ARG, "scn_conv_nin_forward_matrix: null buffer");
+  const int K = fs * nIn;
+  if (conv_thin_shape(fs, nIn, N) && scn_rows_hint(ctx, M) > FR_MAX_M &&
+      (((uintptr_t)d_in | (uintptr_t)d_W | (uintptr_t)d_out) & 15) == 0) {
+    GatherSource gs = GatherSource();
+    gs.rules = d_rules;
+    gs.fs = fs;
+    gs.nIn = nIn;
+    gs.magic = (unsigned)((1ull << 32) / (unsigned)nIn + 1);
+    gs.zeros = ctx->d_zeros;
+    return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, K, N, p, act, precision, &gs, nullptr, nullptr, d_matrix);
+  }
+  SCN_TRY(scn_gather_rows(ctx, d_in, d_matrix, d_rules, M * fs, nIn));
+  return nin_forward(ctx, d_matrix, d_W, d_B, d_prelu, d_out, M, K, N, p, act, precision, nullptr);
 }
 extern "C" int scn_conv_nin_forward_image(scn_ctx *ctx, const float *d_in,
                                           const int32_t *d_rules, int fs, int nIn,

@@ -106,6 +106,7 @@ public:
   ~SparseConvNetCUDA();
   void forwardBatch(SpatiallySparseBatch &batch, int lane = 0);
   void makeWeightImages(SpatiallySparseBatch &batch, cudaMemStream &ms);
+  bool matrixWithNext(SpatiallySparseBatch &batch, size_t i) const;
   void backwardBatch(SpatiallySparseBatch &batch, float learningRate,
                      float momentum);
   // training batches are drawn in shuffled order (BatchProducer.cu:23-26);

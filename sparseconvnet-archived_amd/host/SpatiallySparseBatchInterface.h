@@ -77,6 +77,9 @@ public:
   // layer (fused kernel): the interface whose features the rules index.  The
   // feature matrix of THIS interface is then not materialised.
   SpatiallySparseBatchInterface *deferredGatherFrom;
+  // ... and that layer leaves the matrix here as well (a pass over the net says
+  // so: SparseConvNetCUDA::forwardBatch)
+  bool matrixWithNext = false;
   SpatiallySparseBatchInterface(SpatiallySparseBatchSubInterface *s);
   SpatiallySparseBatchInterface(SpatiallySparseBatchInterface &&o);
   ~SpatiallySparseBatchInterface();

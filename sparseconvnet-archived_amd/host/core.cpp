@@ -371,6 +371,7 @@ void SpatiallySparseBatchInterface::reset() {
   background.resize(0);
   positions.resize(0);
   deferredGatherFrom = nullptr;
+  matrixWithNext = false;
   // deviceGrids keeps its tables for the next batch
 }
 void SpatiallySparseBatchInterface::keepGrids(size_t most) {

@@ -174,7 +174,7 @@ bool ConvolutionalTriangularLayer::defersGather(SpatiallySparseBatch &batch,
 void ConvolutionalLayer::forwards(SpatiallySparseBatch &batch,
                                   SpatiallySparseBatchInterface &input,
                                   SpatiallySparseBatchInterface &output) {
-  if (defersGather(batch, output)) {
+  if (defersGather(batch, output) || output.matrixWithNext) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -237,7 +237,7 @@ void ConvolutionalTriangularLayer::preprocess(
 void ConvolutionalTriangularLayer::forwards(
     SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
     SpatiallySparseBatchInterface &output) {
-  if (defersGather(batch, output)) {
+  if (defersGather(batch, output) || output.matrixWithNext) {
     output.deferredGatherFrom = &input; // the following NiN layer gathers
     return;
   }
@@ -364,6 +364,17 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
     return false;
   const int nIn = src->nFeatures;
   const int fs = input.nFeatures / nIn;
+  if (input.matrixWithNext) {
+    input.matrixWithNext = false;
+    input.deferredGatherFrom = nullptr;
+    const size_t width = (size_t)fs * nIn;
+    input.sub->features.resize64((size_t)input.nSpatialSites * width, kBoundRows * width);
+    SCN_CHECKED(scn_conv_nin_forward_matrix(
+        ms.ctx, src->sub->features.dPtr(), input.rules.dPtr(), fs, nIn, input.sub->features.dPtr(), W.dPtr(), B.dPtr(),
+        prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(), output.nSpatialSites, nFeaturesOut, p, act,
+        abi_precision(precision)));
+    return true;
+  }
   if (!scn_conv_nin_supported_p(fs, nIn, nFeaturesOut, precision)) {
     gather_now(ms, *src, input);
     return false;

@@ -552,6 +552,24 @@ void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStr
     SCN_CHECKED(scn_weight_images_many(ms.ctx, items.data() + i, SCN_IMAGES_MAX));
   SCN_CHECKED(scn_weight_images_later(ms.ctx, items.data() + i, (int)(items.size() - i)));
 }
+// A convolution whose matrix stays, of channels in other than fours (a net's first
+// layer): the layer behind it makes the matrix and reads it in one launch.  Not where
+// there is something to do between the two, or channels that a batch leaves out.
+bool SparseConvNetCUDA::matrixWithNext(SpatiallySparseBatch &batch, size_t i) const {
+  SpatiallySparseBatchInterface &input = batch.interfaces[i], &output = batch.interfaces[i + 1];
+  const int nIn = input.nFeatures;
+  if (nIn % 4 == 0 || batch.type == TRAINBATCH || batch.type == RESCALEBATCH || i + 1 >= layers.size() ||
+      layers[i]->defersGather(batch, output) || (int)input.featuresPresent.size() != nIn ||
+      (int)output.featuresPresent.size() != output.nFeatures ||
+      !(dynamic_cast<ConvolutionalLayer *>(layers[i]) || dynamic_cast<ConvolutionalTriangularLayer *>(layers[i])))
+    return false;
+  int nOut = 0;
+  if (auto *n = dynamic_cast<NetworkInNetworkLayer *>(layers[i + 1]))
+    nOut = n->nFeaturesOut;
+  else if (auto *n = dynamic_cast<NetworkInNetworkPReLULayer *>(layers[i + 1]))
+    nOut = n->nFeaturesOut;
+  return nOut > 0 && scn_conv_nin_supported(output.nFeatures / nIn, nIn, nOut);
+}
 // The two halves of processBatch.  forwardBatch only queues work on the net's
 // stream (every layer, then the copy of the probabilities to the host);
 // finishBatch waits for that copy and does the host-side statistics.  The
@@ -581,6 +599,7 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
                                   batch.interfaces[i], batch.interfaces[i + 1],
                                   batch.interfaces[i + 2], ms, (int)i + 1))
       break;
+    batch.interfaces[i + 1].matrixWithNext = matrixWithNext(batch, i);
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);
     if (batch.type == RESCALEBATCH) {
       std::cout << i << ":"
