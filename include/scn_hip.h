@@ -467,7 +467,8 @@ int scn_sgemm_AtB_sums(scn_ctx *ctx, const float *d_A, const float *d_D, float *
  * them along (a convolution over channels in other than fours, a net's first layer),
  * or before the first call that is given an image; until then the images are not
  * there, d_W and their room must stay, and no other stream may read them.  What an
- * earlier call of it left and nothing has taken is given up.
+ * earlier call of it left and nothing has taken is given up (while spans are recorded,
+ * scn_prof_enable, the images are made at once).
  * scn_conv_nin_forward_image: scn_conv_nin_forward_p (d_rules null: scn_nin_forward_p
  * of a matrix of fs nIn columns) with d_W and its image, or null. */
 #define SCN_IMAGES_MAX 32

@@ -695,7 +695,7 @@ __device__ __forceinline__ void mask_dilate_body(const GridView &in, const Geom 
 }
 // The output's mask, and beside it what needs no more than a few workgroups: the
 // per-sample pass of k_plan_samples (KIND 0), the same over an owners' mask (1) or
-// behind a short scan (2, k_plan_scan_samples), and the rows by rank of the input.
+// behind a short scan (2), and the rows by rank of the input.
 // By themselves these are 5.5 and 5 to 8 us in which most of the chip idles (40
 // samples of 126^3 lattice sites, 460 000 and 1.38 million of them active).  Eight
 // blocks for the samples, of which one works, so that the others keep their XCDs.
