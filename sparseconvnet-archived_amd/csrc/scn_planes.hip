@@ -1702,6 +1702,7 @@ extern "C" int scn_weight_images_later(scn_ctx *ctx, const scn_image_item *items
   return SCN_OK;
 }
 int scn_images_now(scn_ctx *ctx) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_nin_forward: null context");
   ImageList &l = ctx->imagesLater;
   if (l.count == 0)
     return SCN_OK;

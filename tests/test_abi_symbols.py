@@ -27,6 +27,14 @@ def test_version_and_error_string_without_gpu():
     assert isinstance(scn.lib().scn_last_error(), bytes)
 
 
+def test_a_contraction_without_a_context_is_refused():
+    scn = load_scn()
+    for image in (None, 16):  # (with an image of its weights, too)
+        rc = scn.lib().scn_conv_nin_forward_image(None, None, None, 4, 32, None, image, None, None, None, 0, 32, 1.0, scn.RELU,
+                                                  scn.FP32_PLANES)
+        assert rc == 1 and b"null context" in scn.lib().scn_last_error(), image
+
+
 def test_host_library_exports_the_c_facade():
     scn = load_scn()
     from sparseconvnet_archived_amd import hostapi
