@@ -916,10 +916,13 @@ void MaxPoolingLayer::backwards(SpatiallySparseBatch &batch,
                                 SpatiallySparseBatchInterface &output,
                                 float learningRate, float momentum) {
   (void)learningRate, (void)momentum;
-  // (interfaces: .. convolution's output, its input's gradient, this one's output ..)
-  const size_t i = &input - batch.interfaces.data();
-  SpatiallySparseBatchInterface *middle = i > 0 ? &batch.interfaces[i - 1] : nullptr;
-  pool_backwards(memStream, input, output, &batch, middle && middle->deferredGatherFrom ? middle : nullptr);
+  // (interfaces: .. convolution's output, its input's gradient, this one's output ..
+  // A caller's own, which none of the batch's are, have nothing before them)
+  SpatiallySparseBatchInterface *middle = nullptr;
+  for (size_t i = 1; output.poolInverse && i < batch.interfaces.size(); ++i)
+    if (&batch.interfaces[i] == &input && batch.interfaces[i - 1].deferredGatherFrom)
+      middle = &batch.interfaces[i - 1];
+  pool_backwards(memStream, input, output, &batch, middle);
 }
 void MaxPoolingLayer::forwards(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &input,
