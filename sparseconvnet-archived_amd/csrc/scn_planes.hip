@@ -17,6 +17,7 @@
 // 4096 in 64, so six of the former are 2.7 times as fast.
 //   PL 3: SCN_FP32; PL 2: SCN_BF16X3 (hi hi, hi lo, lo hi); PL 1: SCN_BF16.
 #include "scn_image_dev.h"
+#include "scn_planes_choice.h"
 #include <math.h>
 #include <utility>
 
@@ -1242,7 +1243,6 @@ __global__ void __launch_bounds__(256)
 }
 
 __global__ void __launch_bounds__(256) k_weight_images(ImageList l) { weight_images_block(l, blockIdx.x); }
-static int64_t image_bytes(int planes, int K, int N) { return (int64_t)scn_ceil_div(N, 32) * 32 * K * 2 * planes; }
 // What k_nin_lines takes: three planes or one, blocks within one filter position, 64
 // rows of the output within the gigabyte that its stores reach (columns that there are
 // none of lie from 2 GB on, and have to stay there).
@@ -1318,11 +1318,6 @@ static void add_image(ImageList &l, const float *W, unsigned char *image, int pl
   l.W[i] = W, l.image[i] = image, l.K[i] = K, l.N[i] = N, l.fs[i] = fs, l.planes[i] = planes;
   l.firstBlock[i + 1] = l.firstBlock[i] + (unsigned)scn_ceil_div((int64_t)K / 8 * ((N + 31) / 32 * 32), 256);
 }
-// how many workgroups an XCD has of a LONG launch (0: none): a multiple of the slices of columns
-static int lines_long(const scn_ctx *ctx, int T, int splits, int d, bool gather) {
-  const int cus = ctx->numCU / 8;
-  return !gather && T >= d - 1 && splits <= cus ? cus / splits * splits : 0;
-}
 template <int PL, int MT, int NT, int RW, int CW, int D, bool A16 = false>
 static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
                         const Epilogue &ep, const GatherSource *gs, bool wT, const RowRange &rows,
@@ -1341,19 +1336,13 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
   const dim3 grid((unsigned)(scn_ceil_div(M, ROWS) * (long long)nSplits));
   // An XCD takes neighbouring tiles: rows with all their columns, so that they come
   // to its L2 once, or, where the image is the larger part, columns with all rows.
-  const bool byColumns = image_bytes(PL, K, N) > (long long)scn_rows_hint(ctx, M) * (gs ? gs->nIn : K) * 4;
-  // LONG: plain rows, where a compute unit that has room for one workgroup has more than
-  // one tile.  (Gathered rows: 15948 x 1280 x 480 115 us for 110, 15003 x 1920 x 640 232
-  // for 220, with the rules of the next tiles under way; two workgroups to a compute unit
-  // see to that themselves: 139000 x 128 x 64 36 for 29.)
-  if constexpr (PL == 3 && !A16 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160) {
-    const int per = lines_long(ctx, K / 32, nSplits, D, gs != nullptr);
-    if (per && !byColumns && (int64_t)scn_ceil_div(scn_rows_hint(ctx, M), ROWS) * nSplits > ctx->numCU) {
+  const bool byColumns = image_larger(PL, scn_rows_hint(ctx, M), K, N, gs ? gs->nIn : K);
+  if constexpr (PL == 3 && !A16 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160)
+    if (const int per = gs ? 0 : lines_long(ctx->numCU, scn_rows_hint(ctx, M), K, N, ROWS, COLUMNS, D)) {
       hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false, false, true>), dim3(8 * per), dim3(64 * RW * CW), lds,
                          ctx->stream, A, image, out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
       return SCN_OK;
     }
-  }
   if (gs)
     hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, true, A16>), grid, dim3(64 * RW * CW), lds, ctx->stream, A, image,
                        out, M, K, N, ep, *gs, nSplits, byColumns, rows, PlainW{W, wT});
@@ -1464,46 +1453,6 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
   }
   return best;
 }
-// k_nin_lines' tiles.  A workgroup alone on its compute unit takes f + T t1
-// microseconds for T blocks of 32 k, with `resident` of them there (LDS) a block
-// takes all of them tn.  Fitted to 26 shapes (1037 to 1.36 M rows, 128 to 2592 k, 64
-// to 800 columns; 10 % rms), of which it takes 25 to the fastest of these tiles or
-// one within 5 %.  Taller or wider tiles, one wavefront in place of two a SIMD, and
-// deeper rings gained nothing.
-struct LinesTile {
-  int mt, nt, rw, cw, d, resident;
-  float f, t1, tn, next; // next: what a further tile of the same workgroup's begins and ends with (LONG)
-};
-static const LinesTile linesTiles[2][6] = {
-    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f}}, // one plane
-    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 3.3f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 3.4f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 4.5f},
-     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 2.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 1.2f}}};
-static float lines_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool gather, int *tile) {
-  const int T = K / 32;
-  float least = 1e30f;
-  for (int i = 0; i < (planes == 3 ? 6 : 3); ++i) {
-    const LinesTile &x = linesTiles[planes == 3][i];
-    const float n = (float)scn_ceil_div(M, 32 * x.mt * x.rw) * scn_ceil_div(N, 32 * x.nt * x.cw) / ctx->numCU;
-    float cost;
-    if (n <= x.resident) {
-      const float shared = x.resident > 1 ? (fmaxf(ceilf(n), 1.f) - 1.f) / (x.resident - 1) : 0.f;
-      cost = x.f + T * (x.t1 + shared * (x.tn - x.t1));
-    } else if (const int per = x.next > 0.f ? lines_long(ctx, T, scn_ceil_div(N, 32 * x.nt * x.cw), x.d, gather) : 0) {
-      const float long_ = n * ctx->numCU / (8 * per), rounds = long_ <= 3.f ? ceilf(long_) : long_ + .5f;
-      cost = 1.f + rounds * (x.next + T * x.t1);
-    } else {
-      const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
-      cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));
-    }
-    // (rows that few workgroups share, and the clock: 130000 x 512 x 64 63 us in the
-    // second tile, 58 in k_nin_planes)
-    if (planes == 3 && gather && n > (x.mt > 1 ? 1.f : 4.f))
-      cost *= 1.12f;
-    if (cost < least)
-      least = cost, *tile = i;
-  }
-  return least + 4.f;
-}
 // The same of bf16 rows, whose tile goes by the columns, and with the image where it
 // is not made yet.  Fitted to 49 shapes (3500 to 120000 rows, 256 to 1152 k, 64 to
 // 320 columns).  Making the image is what small layers would lose by: us in
@@ -1610,7 +1559,7 @@ static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, c
       !(image || (room && image_bytes(planes, K, N) <= (int64_t)SCN_IMAGE_BYTES)))
     return;
   int tile = 0;
-  const float cost = lines_choose(ctx, planes, M, K, N, gs != nullptr, &tile) + (image ? 0.f : 4.f);
+  const float cost = lines_choose(ctx->numCU, planes, M, K, N, gs != nullptr, &tile) + (image ? 0.f : 4.f);
   if (gs && cost >= choice.cost + 2.f) // (2: what the other's leave out of a launch)
     return;
   choice.lines = tile;
@@ -1657,7 +1606,7 @@ extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N,
     return 0;
   int tile;
   const PlanesChoice choice = planes_choose(ctx, planes, hint > split ? hint : split + 1, K, N, false);
-  if (nIn != K && lines_choose(ctx, planes, hint, K, N, true, &tile) >= choice.cost + 2.f)
+  if (nIn != K && lines_choose(ctx->numCU, planes, hint, K, N, true, &tile) >= choice.cost + 2.f)
     return 0;
   return image_bytes(planes, K, N);
 }

@@ -1,0 +1,70 @@
+// Which of k_nin_lines' tiles a contraction takes (scn_planes.hip), by measured costs: no
+// HIP in it.
+#pragma once
+#include <math.h>
+#include <stdint.h>
+
+static inline int64_t tiles_of(int64_t n, int64_t each) { return (n + each - 1) / each; }
+
+// the bytes of W laid out as planes; whether they are more than those of the rows
+static inline int64_t image_bytes(int planes, int K, int N) { return tiles_of(N, 32) * 32 * K * 2 * planes; }
+static inline bool image_larger(int planes, int64_t rows, int K, int N, int channels) {
+  return image_bytes(planes, K, N) > rows * channels * 4;
+}
+
+// k_nin_lines' tiles.  A workgroup alone on its compute unit takes f + T t1
+// microseconds for T blocks of 32 k, with `resident` of them there (LDS) a block
+// takes all of them tn.  Fitted to 26 shapes (1037 to 1.36 M rows, 128 to 2592 k, 64
+// to 800 columns; 10 % rms), of which it takes 25 to the fastest of these tiles or
+// one within 5 %.  Taller or wider tiles, one wavefront in place of two a SIMD, and
+// deeper rings gained nothing.
+struct LinesTile {
+  int mt, nt, rw, cw, d, resident;
+  float f, t1, tn, next; // next: what a further tile of the same workgroup's begins and ends with (LONG)
+};
+static const LinesTile linesTiles[2][6] = {
+    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f}}, // one plane
+    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 3.3f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 3.4f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 4.5f},
+     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 2.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 1.2f}}};
+// How many workgroups an XCD has of a LONG launch, a multiple of the slices of columns
+// (0: a launch of a workgroup a tile): plain rows of no less than their weights, in three
+// planes, where a compute unit that has room for one workgroup has more than one tile.
+// (Gathered rows: 15948 x 1280 x 480 115 us for 110, 15003 x 1920 x 640 232 for 220,
+// with the rules of the next tiles under way; two workgroups to a compute unit see to
+// that themselves: 139000 x 128 x 64 36 for 29.)  The launch and the choice of its tile
+// both ask here: with LONG's costs for tiles that are not launched so, 2600 x 1024 x
+// 1920 took 78 us and not 68, 2500 x 256 x 2048 28 and not 25.
+static inline int lines_long(int numCU, int64_t M, int K, int N, int rows, int columns, int d) {
+  const int cus = numCU / 8;
+  const int64_t splits = tiles_of(N, columns);
+  return K / 32 >= d - 1 && splits <= cus && !image_larger(3, M, K, N, K) && tiles_of(M, rows) * splits > numCU
+             ? (int)(cus / splits * splits)
+             : 0;
+}
+static inline float lines_cost(int numCU, const LinesTile &x, int planes, int64_t M, int K, int N, bool gather) {
+  const int T = K / 32, rows = 32 * x.mt * x.rw, columns = 32 * x.nt * x.cw;
+  const float n = (float)tiles_of(M, rows) * tiles_of(N, columns) / numCU;
+  float cost;
+  if (n <= x.resident) {
+    const float shared = x.resident > 1 ? (fmaxf(ceilf(n), 1.f) - 1.f) / (x.resident - 1) : 0.f;
+    cost = x.f + T * (x.t1 + shared * (x.tn - x.t1));
+  } else if (const int per = x.next > 0.f && !gather ? lines_long(numCU, M, K, N, rows, columns, x.d) : 0) {
+    const float long_ = n * numCU / (8 * per), rounds = long_ <= 3.f ? ceilf(long_) : long_ + .5f;
+    cost = 1.f + rounds * (x.next + T * x.t1);
+  } else {
+    const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
+    cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));
+  }
+  // (rows that few workgroups share, and the clock: 130000 x 512 x 64 63 us in the
+  // second tile, 58 in k_nin_planes)
+  return planes == 3 && gather && n > (x.mt > 1 ? 1.f : 4.f) ? 1.12f * cost : cost;
+}
+static inline float lines_choose(int numCU, int planes, int64_t M, int K, int N, bool gather, int *tile) {
+  float least = 1e30f;
+  for (int i = 0; i < (planes == 3 ? 6 : 3); ++i) {
+    const float cost = lines_cost(numCU, linesTiles[planes == 3][i], planes, M, K, N, gather);
+    if (cost < least)
+      least = cost, *tile = i;
+  }
+  return least + 4.f;
+}
