@@ -813,10 +813,15 @@ template <int N> __device__ __forceinline__ void lines_landed() {
 // LONG (plain rows): a workgroup goes through several tiles of the same columns, and
 // asks for the next one's rows before it is done with one, D - 1 blocks ahead across the
 // tiles.  Each tile by itself began with a trip to memory and ended in its stores, 4 of
-// the 10 us that one of 128 x 128 x 128 took.  The results go past the caches, which the
-// rows are wanted in: 139000 x 128 x 384 127 us -> 115, so 95; 139000 x 128 x 128 55 -> 37,
-// 400000 x 96 x 128 116 -> 73, 139000 x 256 x 192 109 -> 92, 50000 x 320 x 1280 265 -> 244.
-template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16, bool LONG = false>
+// the 10 us that one of 128 x 128 x 128 took: 139000 x 128 x 128 55 us -> 37, 400000 x 96 x
+// 128 116 -> 73, 139000 x 256 x 192 109 -> 92, 50000 x 320 x 1280 265 -> 244.
+//   2: the results go past the caches, which the rows are wanted in (139000 x 128 x 384
+// 127 -> 115, and so 95): a gradient, which the scatter behind it reads once.
+//   1: they stay, for the pooling that reads a layer's output at once, in its windows'
+// order: contraction and pooling, one tile to a workgroup, past the caches, here: 57000 x
+// 256 x 96 36.5, 38.7, 36.5; 203000 x 64 x 64 48.9, 48.1, 43.1; 60000 x 320 x 160 70.1, 75.1,
+// 66.6; 35000 x 512 x 160 62.4, 64.8, 61.0.
+template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16, int LONG = 0>
 __global__ void __launch_bounds__(64 * RW * CW, 2)
     k_nin_lines(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
                 int K, int N, Epilogue ep, GatherSource gs, int nSplits, bool byColumns, RowRange rows, PlainW plain) {
@@ -1160,7 +1165,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
       for (int v = 0; v < 16; ++v)
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[0][i][j][v], col[j])), to, at[j], 0, LONG ? 2 : 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[0][i][j][v], col[j])), to, at[j], 0, LONG == 2 ? 2 : 0);
           at[j] += v % 4 == 3 ? 5 * pitch : pitch;
         }
   }
@@ -1339,8 +1344,10 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
   const bool byColumns = image_larger(PL, scn_rows_hint(ctx, M), K, N, gs ? gs->nIn : K);
   if constexpr (PL == 3 && !A16 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160)
     if (const int per = gs ? 0 : lines_long(ctx->numCU, scn_rows_hint(ctx, M), K, N, ROWS, COLUMNS, D)) {
-      hipLaunchKernelGGL((k_nin_lines<PL, MT, NT, RW, CW, D, false, false, true>), dim3(8 * per), dim3(64 * RW * CW), lds,
-                         ctx->stream, A, image, out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
+      // (W turned: a gradient)
+      hipLaunchKernelGGL((wT ? k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 2> : k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 1>),
+                         dim3(8 * per), dim3(64 * RW * CW), lds, ctx->stream, A, image, out, M, K, N, ep, GatherSource(), nSplits,
+                         byColumns, rows, PlainW{W, wT});
       return SCN_OK;
     }
   if (gs)

@@ -160,7 +160,8 @@ def test_weight_gradients_by_lines(scn, ctx, M, fs, nIn, N):
 # of its last block by, and more; slices of columns that do not divide an XCD's workgroups (640, 1280: 5 and 10); the last tile
 # of one row, of all but one; rows that are not finite in the first, a middle and the last tile, which are taken again there
 @pytest.mark.parametrize("M,K,N", [(128 * 300 + 1, 64, 384), (128 * 523 - 1, 128, 128), (256 * 300 + 77, 64, 64), (33001, 128, 256),
-                                   (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192)])
+                                   (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192), (16500, 512, 256),
+                                   (70003, 160, 36)])
 def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
     rng = np.random.default_rng(M + K + N)
     A, W = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
@@ -177,3 +178,32 @@ def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
     for r in range(0, M, 20000):
         a = A[r:r + 20000].astype(np.float64)
         assert np.all(np.abs(got[r:r + 20000] - a @ W.T.astype(np.float64)) <= 2e-6 * (np.abs(a) @ np.abs(W.T).astype(np.float64)))
+
+
+# the same forward, with bias and activation, in every tile that is launched so (test_planes_choice.py: these reach all), the bits
+# of the kernels that convert the weights on the way; five and six blocks of k in the ring of six
+SEVERAL = [(38401, 64, 384), (40000, 96, 640), (50001, 256, 192), (33001, 64, 160), (16500, 512, 256), (33001, 128, 256),
+           (8000, 96, 640), (70003, 160, 36), (70003, 192, 64)]
+
+
+@pytest.mark.parametrize("M,K,N", SEVERAL)
+@pytest.mark.parametrize("act", ["LEAKYRELU", "PRELU"])
+def test_several_tiles_to_a_workgroup_forward(scn, ctx, M, K, N, act):
+    rng = np.random.default_rng(M + K + N)
+    A, W = rng.standard_normal((M, K), dtype=np.float32), (rng.standard_normal((K, N)) * np.sqrt(2.0 / K)).astype(np.float32)
+    A[[0, M // 2, M - 1], 3] = [np.inf, np.nan, -np.inf]  # (taken again, in the first, a middle and the last tile)
+    d_A, d_W, d_B = ctx.array(A), ctx.array(W), ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+    slopes = ctx.array(rng.uniform(0.1, 0.4, N).astype(np.float32)) if act == "PRELU" else None
+    image = ctx.empty(((N + 31) // 32 * 32 * K * 6 // 4,), np.float32)
+    ctx.weight_images_many([(d_W, image, K, N, 0, scn.FP32_PLANES)])
+    one, two = (ctx.array(np.full((M + 256, N), 7, np.float32)) for _ in range(2))
+    print("several tiles forward", M, K, N, act, flush=True)
+    ctx.conv_nin_forward_image(d_A, None, 1, K, d_W, image, d_B, slopes, one, M, N, 1.0, getattr(scn, act), scn.FP32_PLANES)
+    ctx.sync()
+    with Graph(ctx) as g:
+        ctx.nin_forward(d_A, d_W, d_B, slopes, two, M, K, N, 1.0, getattr(scn, act), scn.FP32_PLANES)
+    g.replay(ctx)
+    ctx.sync()
+    got, want = one.download(), two.download()
+    g.close()
+    assert np.all(got[M:] == 7) and np.array_equal(got, want, equal_nan=True)

@@ -48,3 +48,10 @@ def test_a_tile_costs_what_its_launch_does(choice, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(2500, 256, 2048), (2600, 1024, 1920)])
 def test_rows_of_less_than_their_weights(choice, M, K, N):
     assert choice.lines_tile(256, 3, M, K, N, 0) == 2
+
+
+def test_shapes_of_several_tiles_to_a_workgroup(choice):
+    """those of the tests on the card are launched so, in all the tiles that can be"""
+    from test_gpu_lines import SEVERAL
+    tiles = [choice.lines_tile(256, 3, M, K, N, 0) for M, K, N in SEVERAL]
+    assert all(choice.lines_tile_long(256, t, *s) > 0 for t, s in zip(tiles, SEVERAL)) and set(tiles) == set(TILES)
