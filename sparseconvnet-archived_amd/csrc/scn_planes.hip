@@ -2279,10 +2279,7 @@ struct AtbList {
   int count, length, part; // of the line; of a workgroup
 };
 constexpr int ATB_MANY = atb_waves(2, 1, true); // wavefronts
-// What a step and a tile's beginning and end take, in sixteenths of a microsecond
-// (measured by the clock in the kernel, layers of 2500 to 84000 rows: by lines 1.42
-// to 1.68 us a step, a first layer's 1.3, and 4.7)
-constexpr int ATB_LINES_COST = 25, ATB_FIRST_COST = 21, ATB_TILE_COST = 75;
+static_assert(ATB_MANY * ATB_STEP == ATB_MANY_ROWS, "a step of a range");
 __device__ __host__ __forceinline__ int atb_step_cost(const int *rules, int nIn) {
   return rules && nIn % 4 ? ATB_FIRST_COST : ATB_LINES_COST;
 }
@@ -2340,32 +2337,32 @@ int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
   AtbList l;
   l.count = 0;
   l.zeros = ctx->d_zeros;
+  AtbShape shape[SCN_ATB_MAX];
+  bool joined[SCN_ATB_MAX];
+  for (int k = 0; k < nItems; ++k)
+    shape[k] = {items[k].M, items[k].fs * items[k].nIn, items[k].N, atb_many_tile(items[k]),
+                atb_step_cost(items[k].d_positions, items[k].nIn)};
+  atb_join(ctx->numCU, shape, nItems, joined);
   long long tiles[SCN_ATB_MAX], steps[SCN_ATB_MAX], work = 0;
   int cost[SCN_ATB_MAX];
   for (int k = 0; k < nItems; ++k) {
     const scn_atb_item &it = items[k];
-    if (it.M == 0)
-      continue;
-    const int m = atb_many_tile(it), K = it.fs * it.nIn;
-    const long long n = m ? (long long)scn_ceil_div(K, 32 * m) * scn_ceil_div(it.N, 32) : 0;
-    const long long s = scn_ceil_div(it.M, ATB_MANY * ATB_STEP);
-    const int each = atb_step_cost(it.d_positions, it.nIn);
-    // one that keeps the chip busy by itself (some 60 us) gains nothing, and two by
-    // two tiles may be better for it
-    if (!m || n > 4096 || n * (s * each + ATB_TILE_COST) > 64ll * 16 * ctx->numCU) {
+    const int K = shape[k].K;
+    if (it.M > 0 && !joined[k]) {
       GatherSource gs = GatherSource();
       gs.rules = it.d_positions;
       gs.fs = it.fs;
       gs.nIn = it.nIn;
       gs.zeros = ctx->d_zeros;
       SCN_TRY(scn_atb_planes(ctx, it.d_in, it.d_D, it.d_dW, it.d_db, it.M, K, it.N, it.d_positions ? &gs : nullptr));
-      continue;
     }
+    if (!joined[k])
+      continue;
     const int c = l.count++;
     l.A[c] = it.d_in, l.D[c] = it.d_D, l.dW[c] = it.d_dW, l.db[c] = it.d_db, l.rules[c] = it.d_positions;
     l.M[c] = (int)it.M, l.K[c] = K, l.N[c] = it.N, l.fs[c] = it.fs;
-    tiles[c] = n, steps[c] = s, cost[c] = each;
-    work += n * s * each;
+    tiles[c] = shape[k].tiles(), steps[c] = shape[k].steps(), cost[c] = shape[k].each;
+    work += tiles[c] * steps[c] * cost[c];
   }
   if (l.count == 0)
     return SCN_OK;

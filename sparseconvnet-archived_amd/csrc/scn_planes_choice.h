@@ -1,5 +1,5 @@
-// Which of k_nin_lines' tiles a contraction takes (scn_planes.hip), by measured costs: no
-// HIP in it.
+// Which of k_nin_lines' tiles a contraction takes, and which weight gradients go into one
+// launch (scn_planes.hip), by measured costs: no HIP in it.
 #pragma once
 #include <math.h>
 #include <stdint.h>
@@ -67,4 +67,40 @@ static inline float lines_choose(int numCU, int planes, int64_t M, int K, int N,
       least = cost, *tile = i;
   }
   return least + 4.f;
+}
+
+// ---- weight gradients of several layers (k_atb_many)
+// What a step and a tile's beginning and end take, in sixteenths of a microsecond
+// (measured by the clock in the kernel, layers of 2500 to 84000 rows: by lines 1.42
+// to 1.68 us a step, a first layer's 1.3, and 4.7)
+constexpr int ATB_LINES_COST = 25, ATB_FIRST_COST = 21, ATB_TILE_COST = 75;
+constexpr int ATB_MANY_ROWS = 192; // of a step
+struct AtbShape {
+  int64_t M;
+  int K, N;
+  int tile; // 32 rows of dW each, 0: not one for k_atb_many
+  int each; // a step's cost
+  int64_t tiles() const { return tile ? tiles_of(K, 32 * tile) * tiles_of(N, 32) : 0; }
+  int64_t steps() const { return tiles_of(M, ATB_MANY_ROWS); }
+};
+// One that keeps the chip busy by itself (some 60 us) gains nothing among others, and
+// two by two tiles may be better for it.  One that is left alone goes by itself, too, in
+// the tile that is best for it: us, alone in k_atb_many and by itself, 1000 x 512 x 160
+// 11.7, 7.4; 11400 x 384 x 128 23.5, 15.7; 28000 x 256 x 96 25.5, 18.6; 57250 x 128 x 64
+// 22.2, 15.5.  Several, in launches of their own and in one: the layers of a batch of
+// drawings, first and second 23.9, 20.9, second and third 29.3, 24.8, fourth and fifth
+// 23.1, 25.1; second to fourth 42.5, 37.4, fourth to sixth 28.6, 25.3; all seven 73.9, 46.8.
+static inline int atb_join(int numCU, const AtbShape *shape, int n, bool *joined) {
+  int count = 0, last = 0;
+  for (int k = 0; k < n; ++k) {
+    const AtbShape &s = shape[k];
+    joined[k] = s.M > 0 && s.tile > 0 && s.tiles() <= 4096 &&
+                s.tiles() * (s.steps() * s.each + ATB_TILE_COST) <= (int64_t)64 * 16 * numCU;
+    if (joined[k])
+      ++count, last = k;
+  }
+  if (count != 1)
+    return count;
+  joined[last] = false;
+  return 0;
 }

@@ -1,4 +1,4 @@
-// The choice of k_nin_lines' tiles on the CPU (test_planes_choice.py).
+// The choices of scn_planes.hip on the CPU (test_planes_choice.py).
 #include "scn_planes_choice.h"
 
 extern "C" int lines_tile(int numCU, int planes, int64_t M, int K, int N, int gather) {
@@ -13,4 +13,15 @@ extern "C" float lines_tile_cost(int numCU, int planes, int tile, int64_t M, int
 extern "C" int lines_tile_long(int numCU, int tile, int64_t M, int K, int N) {
   const LinesTile &x = linesTiles[1][tile];
   return x.next > 0.f ? lines_long(numCU, M, K, N, 32 * x.mt * x.rw, 32 * x.nt * x.cw, x.d) : 0;
+}
+// which of n weight gradients go into one launch; returns how many
+extern "C" int joined(int numCU, int n, const int64_t *M, const int *K, const int *N, const int *tile, const int *each, int *out) {
+  AtbShape shape[64];
+  bool in[64];
+  for (int k = 0; k < n; ++k)
+    shape[k] = {M[k], K[k], N[k], tile[k], each[k]};
+  const int count = atb_join(numCU, shape, n, in);
+  for (int k = 0; k < n; ++k)
+    out[k] = in[k];
+  return count;
 }

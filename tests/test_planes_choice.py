@@ -1,4 +1,4 @@
-"""The choice of a contraction's tile on the CPU: costed as it is launched."""
+"""The choice of a contraction's tile, costed as it is launched, and of the weight gradients that share a launch, on the CPU."""
 import ctypes as C
 import math
 import os
@@ -55,3 +55,18 @@ def test_shapes_of_several_tiles_to_a_workgroup(choice):
     from test_gpu_lines import SEVERAL
     tiles = [choice.lines_tile(256, 3, M, K, N, 0) for M, K, N in SEVERAL]
     assert all(choice.lines_tile_long(256, t, *s) > 0 for t, s in zip(tiles, SEVERAL)) and set(tiles) == set(TILES)
+
+
+SMALL, FIRST, LARGE, EMPTY, OTHER = ((11400, 384, 128, 2, 25), (83597, 12, 32, 1, 21), (139000, 384, 128, 2, 25), (0, 384, 128, 2, 25),
+                                     (5000, 30, 7, 0, 25))
+
+
+# (one alone: 23.5 us in the launch for several, 15.7 by itself)
+@pytest.mark.parametrize("items,want", [([], []), ([SMALL], [0]), ([FIRST], [0]), ([SMALL, FIRST], [1, 1]), ([LARGE, SMALL], [0, 0]),
+                                        ([SMALL, EMPTY, OTHER], [0, 0, 0]), ([SMALL, LARGE, FIRST, EMPTY], [1, 0, 1, 0]),
+                                        ([SMALL] * 24, [1] * 24)])
+def test_weight_gradients_of_one_launch(choice, items, want):
+    columns = [(C.c_int64 if i == 0 else C.c_int) * max(1, len(items)) for i in range(5)]
+    out = (C.c_int * max(1, len(items)))()
+    assert choice.joined(256, len(items), *(t(*(x[i] for x in items)) for i, t in enumerate(columns)), out) == sum(want)
+    assert list(out)[:len(items)] == want
