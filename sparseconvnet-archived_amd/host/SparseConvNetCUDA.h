@@ -2,6 +2,7 @@
 // per-batch forward driver, weight files (SparseConvNetCUDA.h:25-114).  The
 // class keeps the reference's name; the device code underneath is HIP.
 #pragma once
+#include <atomic>
 #include <fstream>
 #include <iostream>
 #include <memory>
@@ -115,6 +116,8 @@ public:
   // rule books of consecutive layers are built together, one workgroup per
   // sample, where the library can (scn_ctx_chain_rules); off: layer by layer
   bool chainRuleBooks = true;
+  // poolings of training batches whose gradient is read through rules turned round
+  std::atomic<int64_t> poolingsTurned{0};
   void finishBatch(SpatiallySparseBatch &batch, std::ofstream &f,
                    std::ofstream &g);
   void processBatch(SpatiallySparseBatch &batch, float learningRate,

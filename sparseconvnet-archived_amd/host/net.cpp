@@ -1084,12 +1084,24 @@ static void leaveOutConvolutions(SparseConvNetCUDA &cnn, scn_ctx *ctx, Spatially
     SCN_CHECKED(scn_rules_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
 }
 // ... and its poolings' rules turned round, where their windows overlap little: a
-// gradient that is read by rows and written once.  (A sample's windows are walked by
-// a workgroup for its background row: some 2 us for every 512 of them.)
+// gradient that is read by rows and written once.  A sample's windows are walked by one
+// workgroup for its background row, 256 of them in 2 us, so that the longest sample
+// decides, not the average: us, turned round and scattered (clearing, adding), of 63800 x
+// 32 in 100 samples with one of 2000 25.8, 36.5, of 3000 33.8, 36.4, of 4850 47, 37, of
+// 39200 (of 100087) 320, 53; of 63800 x 96 with one of 4800 70, 88, of 8000 95, 92; of 14700
+// x 32 with one of 9550 79, 14; of 4 x 2970 x 32 25, 12; of 101700 x 32 voxels, one of
+// 13600, 115, 71.  With sums over the background of the convolution before, which the
+// scatter leaves to scn_background_sums: of the first of these with one of 8000 85, 91, of
+// 21800 215, 149; the voxels 153, 138; 4 x 2970 x 32 31, 20.
+static int64_t longestTurned(SpatiallySparseBatchInterface &in, SpatiallySparseBatchInterface &out) {
+  const int64_t all = out.nSpatialSites * (int64_t)out.featuresPresent.size();
+  return in.gradientSums ? 1000 + 24 * all / 10000 : 600 + 17 * all / 10000;
+}
 static void turnPoolings(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBatch &b) {
   std::vector<scn_pool_inverse_item> items;
   std::vector<SpatiallySparseBatchInterface *> outs;
   auto room = [](size_t n) { return (n + 3) & ~(size_t)3; };
+  const size_t sampleRoom = room(2 * (size_t)b.batchSize + 1);
   size_t total = 0;
   for (size_t i = 0; i < cnn.layers.size(); ++i) {
     MaxPoolingLayer *const pool = dynamic_cast<MaxPoolingLayer *>(cnn.layers[i]);
@@ -1099,26 +1111,47 @@ static void turnPoolings(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBa
     const int slots = scn_pool_inverse_slots(pool->dimension, pool->poolSize, pool->poolStride);
     const int64_t nf = (int64_t)out.featuresPresent.size();
     if (slots == 0 || nf % 4 != 0 || nf == 0 || in.nSpatialSites * std::max<int64_t>(nf, slots) > 0x7fffffffll ||
-        out.nSpatialSites * nf > 0x7fffffffll || out.nSpatialSites > 2048ll * b.batchSize)
+        out.nSpatialSites * nf > 0x7fffffffll ||
+        out.nSpatialSites > longestTurned(in, out) * b.batchSize) // (one is as long as the average)
       continue;
     out.poolSlots = slots;
     items.push_back({in.deviceGrids, out.deviceGrids, out.rules.dPtr(), nullptr, nullptr, out.nSpatialSites,
                      in.nSpatialSites, pool->poolSize, pool->poolStride});
     outs.push_back(&out);
-    total += room((size_t)in.nSpatialSites * slots) + room(2 * (size_t)b.batchSize + 1);
+    total += room((size_t)in.nSpatialSites * slots) + sampleRoom;
   }
+  if (items.empty())
+    return;
   b.poolInverses.resize64(total);
-  int *at = b.poolInverses.dPtr();
+  int *const samples = b.poolInverses.dPtr(), *at = samples + items.size() * sampleRoom;
   for (size_t k = 0; k < items.size(); ++k) {
+    items[k].d_samples = samples + k * sampleRoom;
     items[k].d_inverse = at;
     at += room((size_t)items[k].inputRows * outs[k]->poolSlots);
-    items[k].d_samples = at;
-    at += room(2 * (size_t)b.batchSize + 1);
     outs[k]->poolInverse = items[k].d_inverse;
     outs[k]->poolSamples = items[k].d_samples;
   }
   for (size_t i = 0; i < items.size(); i += SCN_INVERSE_MAX)
     SCN_CHECKED(scn_pool_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
+  const size_t bytes = items.size() * sampleRoom * sizeof(int32_t);
+  b.poolSamples.reserve(bytes);
+  SCN_CHECKED(scn_copy(ctx, b.poolSamples.p, samples, bytes));
+}
+// (when the stream is through: the poolings with a sample too long are scattered)
+static void keepTurnedPoolings(SparseConvNetCUDA &cnn, SpatiallySparseBatch &b) {
+  for (size_t i = 1; i < b.interfaces.size(); ++i) {
+    SpatiallySparseBatchInterface &out = b.interfaces[i];
+    if (!out.poolInverse)
+      continue;
+    const int32_t *const first = b.poolSamples.as<int32_t>() + (out.poolSamples - b.poolInverses.dPtr());
+    int64_t longest = 0;
+    for (int s = 0; s < b.batchSize; ++s)
+      longest = std::max<int64_t>(longest, first[s + 1] - first[s]);
+    if (longest > longestTurned(b.interfaces[i - 1], out))
+      out.poolInverse = out.poolSamples = nullptr;
+    else
+      ++cnn.poolingsTurned;
+  }
 }
 // GPU half: the input grids go to HBM, then every layer builds its rule book,
 // all on the slot's stream
@@ -1165,6 +1198,7 @@ void BatchProducer::preprocessBatchOnDevice(int cc) {
     turnPoolings(cnn, ctx, b);
   }
   SCN_CHECKED(scn_sync(ctx));
+  keepTurnedPoolings(cnn, b);
 }
 void BatchProducer::batchProducerThread(int nThread) {
   RNG rng;

@@ -726,6 +726,7 @@ void scnh_collect_probabilities(scnh_net *net, float *h_all, int64_t capacity) {
   net->allProbs = h_all;
   net->allProbsCapacity = h_all ? capacity : 0;
 }
+int64_t scnh_turned_poolings(scnh_net *net) { return net->cnn->poolingsTurned; }
 void scnh_chain_counts(scnh_net *net, int64_t *chains, int64_t *plans) {
   SparseConvNetCUDA *cnn = net->cnn;
   int64_t c = 0, p = 0;

@@ -236,6 +236,9 @@ void scnh_collect_probabilities(scnh_net *net, float *h_all, int64_t capacity);
 /* recorded-plan runs so far on all streams of the net that build rule books
  * (sums of scn_ctx_chain_count) */
 void scnh_chain_counts(scnh_net *net, int64_t *chains, int64_t *plans);
+/* poolings of training batches so far whose gradient was read through their rules
+ * turned round */
+int64_t scnh_turned_poolings(scnh_net *net);
 /* the library context of the net (scn_ctx *), for timing and raw buffers */
 void *scnh_context(scnh_net *net);
 /* multiply-accumulates of the NiN layers since the last call */

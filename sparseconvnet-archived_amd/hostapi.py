@@ -103,6 +103,7 @@ def lib():
         "scnh_stream_ready_at_start": (i32, [vp]),
         "scnh_collect_probabilities": (None, [vp, vp, i64]),
         "scnh_chain_counts": (None, [vp, P(i64), P(i64)]),
+        "scnh_turned_poolings": (i64, [vp]),
         "scnh_context": (vp, [vp]),
         "scnh_take_multiply_add_count": (C.c_double, []),
     }
@@ -462,6 +463,10 @@ class Net:
         a, b = C.c_int64(), C.c_int64()
         lib().scnh_chain_counts(self.h, C.byref(a), C.byref(b))
         return a.value, b.value
+
+    def turned_poolings(self):
+        """poolings of training batches so far whose gradient was read through their rules turned round"""
+        return lib().scnh_turned_poolings(self.h)
 
     def context_handle(self):
         return lib().scnh_context(self.h)

@@ -97,3 +97,33 @@ def test_pool_gradient_refusals(scn, ctx):
         a.update(kw)
         with pytest.raises(scn.ScnError):
             ctx.maxpool_gradient(**a)
+
+
+# drawings alike: all five poolings by rows.  One that fills its field among seven of few points, whose 2400 windows of the first
+# pooling a workgroup would walk (the average is some 300): that one is scattered
+@pytest.mark.parametrize("sides,turned", [([26] * 8, 5), ([5, 5, 5, 96, 5, 5, 5, 5], 4)])
+def test_the_longest_sample_decides(scn, sides, turned):
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    from test_gpu_training import pair, rel_l2
+    cfg = synthetic.config(2, batch=8)
+    rng = np.random.default_rng(sum(sides))
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TRAINBATCH)
+    for side in sides:
+        at = np.stack(np.meshgrid(np.arange(side), np.arange(side), indexing="ij"), -1).reshape(-1, 2) + (96 - side) // 2
+        ds.add_points(2, cfg.lattice, at.astype(np.int32), rng.uniform(-1, 1, (side * side, 3)).astype(np.float32),
+                      int(rng.integers(0, 100)))
+    left = []
+    for epoch in (True, False):  # (a batch by itself scatters everything)
+        net, _ = pair(cfg, hostapi, 53)
+        net.set_training(0.01, 0.9, shuffle=False)
+        if epoch:
+            net.processDatasetTrain(ds, 8, 0.01, 0.9)
+        else:
+            net.begin(ds, 8)
+            assert net.next_batch()
+        assert net.turned_poolings() == (turned if epoch else 0)
+        left.append([a for i, l in enumerate(net.layers()) if l["kind"].startswith("nin")
+                     for a in net.get_weights(i, momentum=True) if a is not None])
+        net.close()
+    for a, b in zip(*left):  # (the same forward pass, bit for bit: fp32 sums in other orders)
+        assert rel_l2(a, b) <= 1e-5
