@@ -1696,7 +1696,7 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // eight consecutive rows of one column: dword loads (pairs of columns for two
 // tiles) that 32 lanes make of 32 neighbouring columns, whole lines, and no
 // turning in LDS.  A workgroup owns 32 MT x 32 NT of dW and a range of rows; its
-// eight wavefronts take sixteen rows each in turn and their sums meet in LDS.
+// wavefronts, eight or twelve, take sixteen rows each in turn and their sums meet in LDS.
 // The workgroups of one tile add to dW with float atomics, some 200 of which
 // retire in a nanosecond: few workgroups (one a compute unit), each with as many
 // rows as that leaves it (29827 x 256 x 96 in 23 us, where the fp32 MFMA with a
@@ -1704,19 +1704,16 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
 // GATHER: the rows of A through rules, which lie position by position, so that
 // a lane's eight are two loads (eight of them through row by row rules: 17.8 us
 // where this is 15.6 and a gathered matrix 14.5, and 8.2 to gather it).
-#define ATB_STEP 16
 // LINES: the rows come into LDS by whole lines, a ring of steps for each wavefront,
 // which waits for nobody: a kilobyte to a request, where the loads above take 256 or
 // 512 bytes and every request occupies the path for 16 cycles or more, twice what the
 // splitting takes.  A backward layer with dW of 139000 x 384 x 128 384 -> 370 us;
 // dW of 28000 x 256 x 96 and its like 16.5 -> 15.6, of which some 5 are the start and
 // the atomics; 35461 x 256 x 96 20, 198759 x 1728 x 64 328 (A from HBM at 4.2 TB/s).
-// A step's planes are made among the MFMAs of the step before, and where registers
-// and LDS have room there are three wavefronts to a SIMD: the two together 55 -> 50 us
-// for six layers of a batch of drawings in one launch.
+// In tiles of two a step's planes are made among the MFMAs of the step before, by three
+// wavefronts to a SIMD: the two together 55 -> 50 us for six layers of a batch of drawings
+// in one launch.
 constexpr int atb_ring(int MT, int NT) { return MT * NT >= 2 ? 2 : 3; }
-// wavefronts of a workgroup: three a SIMD where registers and LDS have room
-constexpr int atb_waves(int MT, int NT, bool LINES) { return LINES && MT * NT < 4 ? 12 : 8; }
 // (one tile of dW, of the rows from m0 to m1: m0 a multiple of ATB_STEP; GM wavefronts)
 template <int MT, int NT, bool GATHER, bool LINES, int GM>
 __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const float *__restrict__ D, float *__restrict__ dW,
@@ -1936,7 +1933,7 @@ __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const floa
       // Rules are asked for a step before their rows, in front of the rows asked for
       // then: what has landed when all but the last step's rows have holds a step's
       // rows and the next request's rules.
-      if constexpr (MT * NT < 4) {
+      if constexpr (atb_ahead(MT, NT)) {
         // A step's planes are made while the MFMAs of the one before run, dealt out
         // among them.  So a slot is free when its planes have been made, and RING steps
         // are under way.
@@ -1998,12 +1995,27 @@ __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const floa
           step(odd, even, t);
         }
       } else {
-        Rules x = {};
-        fetch(x, 0, 0);
+        static_assert(!GATHER || RING == 3, "the first two steps' rules come together");
+        Rules x;
+        {
+          Rules second;
+          int *const spare = reinterpret_cast<int *>(ring + (RING - 1) * SLOT); // (nothing is asked for there yet)
+          ask(0, spare);
+          ask(1, spare + AU * 64);
+          ask(RING - 1, sRule);
+          w_landed<0>();
+          look(x, spare);
+          look(second, spare + AU * 64);
+          fetch(x, 0, 0);
+          if (RING == 3)
+            fetch(second, 1, 1);
+        }
         int slot = 0, into = RING - 1;
 #pragma unroll 1
         for (int t = 0; t < steps; ++t) {
-          w_landed<0>(); // (and this wavefront's reads of the slot that is asked for again)
+          w_landed<RING == 3 ? FETCH : 0>(); // (and this wavefront's reads of the slot that is asked for again)
+          look(x, sRule);
+          ask(t + RING, sRule);
           fetch(x, t + RING - 1, into);
           Step s;
           take(s, slot);
@@ -2017,7 +2029,7 @@ __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const floa
   } else {
     const long long whole = m1 - ATB_STEP; // last start of a step without a guard
     Step s0, s1;
-    long long m = m0 + ATB_STEP * wave; // a step in eight is this wavefront's
+    long long m = m0 + ATB_STEP * wave; // a step in GM is this wavefront's
     auto fetch = [&](Step &s, long long at) {
       if (at <= whole)
         load(s, at, false);
@@ -2168,7 +2180,7 @@ constexpr size_t atb_lds(int MT, int NT, bool GATHER, bool LINES, int GM) {
 
 template <int MT, int NT, bool GATHER, bool LINES>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
-                      long long M, int K, int N, long long splits, const GatherSource &gs) {
+                      long long M, int K, int N, long long rows, const GatherSource &gs) {
   constexpr int GM = atb_waves(MT, NT, LINES);
   constexpr size_t lds = atb_lds(MT, NT, GATHER, LINES, GM);
   static OncePerDevice configured;
@@ -2181,75 +2193,42 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, f
   SCN_REQUIRE(rc == SCN_OK, SCN_ERR_HIP, "hipFuncSetAttribute failed");
   const int nTiles = scn_ceil_div(N, 32 * NT);
   const long long tiles = (long long)scn_ceil_div(K, 32 * MT) * nTiles;
-  long long rows = (M + splits - 1) / splits;
-  rows = (rows + GM * ATB_STEP - 1) / (GM * ATB_STEP) * (GM * ATB_STEP);
   hipLaunchKernelGGL((k_atb_planes<MT, NT, GATHER, LINES>), dim3((unsigned)tiles, (unsigned)((M + rows - 1) / rows)),
                      dim3(64 * GM), lds, ctx->stream, A, D, dW, db, M, K, N, nTiles, rows, gs, ctx->d_zeros);
   return SCN_OK;
 }
 template <int MT, int NT>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db, long long M, int K, int N,
-                      long long splits, const GatherSource *gs, bool lines) {
+                      long long rows, const GatherSource *gs, bool lines) {
   if constexpr (MT == 2 && NT == 2) // (not gathered: see below)
-    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, splits, GatherSource())
-                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
+    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, rows, GatherSource())
+                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, rows, GatherSource());
   else if (gs)
-    return lines ? launch_atb<MT, NT, true, true>(ctx, A, D, dW, db, M, K, N, splits, *gs)
-                 : launch_atb<MT, NT, true, false>(ctx, A, D, dW, db, M, K, N, splits, *gs);
+    return lines ? launch_atb<MT, NT, true, true>(ctx, A, D, dW, db, M, K, N, rows, *gs)
+                 : launch_atb<MT, NT, true, false>(ctx, A, D, dW, db, M, K, N, rows, *gs);
   else
-    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, splits, GatherSource())
-                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, splits, GatherSource());
+    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, rows, GatherSource())
+                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, rows, GatherSource());
 }
 
-// The tile and the number of row ranges that cost least: rounds of one workgroup
-// a compute unit, each `ti` microseconds for every 128 rows and `f` to start, to sum
-// and to store, and the atomics.  (Fitted where the rows were loaded into registers;
-// by lines it is 0.9 of `ti` for all of them, so that the choice is the same.)
-// Pairs of columns are loaded as one: K (N) even for two row (column) tiles.
-// Two by two tiles, us against two by one: 126507 x 1728 x 64 208, 255; 53325 x 640 x
-// 320 138, 177; 17223 x 1280 x 480 148, 174; 153345 x 384 x 128 106, 130; with the sums
-// of D the same.
-// (The search is 0.1 to 2 us of the host's time, a launch some 5.)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,
                    long long M, int K, int N, const GatherSource *gs) {
-  static const struct {
-    int mt, nt;
-    double ti, f;
-  } tile[] = {{1, 1, .8, 4.}, {2, 1, 1.13, 4.}, {1, 2, 1.13, 4.}, {2, 2, 1.95, 6.}};
-  int best = 0;
-  long long splits = 1;
-  double least = 1e300;
   // (requests of four columns, in one filter position each)
   const bool lines = K % 4 == 0 && N % 4 == 0 && (!gs || gs->nIn % 4 == 0) && (((uintptr_t)A | (uintptr_t)D) & 15) == 0;
-  // (two by two tiles of gathered rows, and with sums but not by lines: 264 bytes a lane spilled)
-  for (int i = 0; i < (gs || (db && !lines) ? 3 : 4); ++i) {
-    if ((tile[i].mt == 2 && ((gs ? gs->nIn : K) % 2 || ((uintptr_t)A & 7))) || (tile[i].nt == 2 && (N % 2 || ((uintptr_t)D & 7))))
-      continue;
-    const long long tiles = (long long)scn_ceil_div(K, 32 * tile[i].mt) * scn_ceil_div(N, 32 * tile[i].nt);
-    if (tiles > 0x7fffffffll)
-      continue;
-    const long long most = scn_ceil_div(M, 8 * ATB_STEP);
-    for (long long s = 1; s <= most && s <= 4096; s += s < 64 ? 1 : s / 32) {
-      const long long rounds = (tiles * s + ctx->numCU - 1) / ctx->numCU;
-      const long long steps = (M + s * 8 * ATB_STEP - 1) / (s * 8 * ATB_STEP);
-      const double cost = rounds * (steps * tile[i].ti + tile[i].f) +
-                          (double)tiles * s * tile[i].mt * tile[i].nt * 1024 / 2e5;
-      if (cost < least)
-        least = cost, best = i, splits = s;
-      if (rounds > 8)
-        break;
-    }
-  }
-  SCN_REQUIRE(least < 1e300, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
-  switch (best) {
+  // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.  (Two by two
+  // tiles of gathered rows, and with sums but not by lines: 264 bytes a lane spilled)
+  const bool pairsA = (gs ? gs->nIn : K) % 2 == 0 && ((uintptr_t)A & 7) == 0, pairsD = N % 2 == 0 && ((uintptr_t)D & 7) == 0;
+  const AtbChoice c = atb_choose(ctx->numCU, M, K, N, lines, pairsA, pairsD, !gs && (!db || lines));
+  SCN_REQUIRE(c.tile >= 0, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
+  switch (c.tile) { // (as in atbTiles)
   case 1:
-    return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
+    return launch_atb<2, 1>(ctx, A, D, dW, db, M, K, N, c.rows, gs, lines);
   case 2:
-    return launch_atb<1, 2>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
+    return launch_atb<1, 2>(ctx, A, D, dW, db, M, K, N, c.rows, gs, lines);
   case 3:
-    return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
+    return launch_atb<2, 2>(ctx, A, D, dW, db, M, K, N, c.rows, gs, lines);
   }
-  return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, splits, gs, lines);
+  return launch_atb<1, 1>(ctx, A, D, dW, db, M, K, N, c.rows, gs, lines);
 }
 
 // ---- the weight gradients of all layers of a net in one launch.  Each by itself is

@@ -69,6 +69,55 @@ static inline float lines_choose(int numCU, int planes, int64_t M, int K, int N,
   return least + 4.f;
 }
 
+// ---- a weight gradient (scn_atb_planes)
+constexpr int ATB_STEP = 16; // rows that a wavefront takes at a time
+// By lines, tiles of two have a step's planes made among the MFMAs of the step before, and
+// three wavefronts to a SIMD.  What a 1 x 1 tile is for is over in a few steps, which
+// begin and end sooner in eight wavefronts without: 400 x 384 x 128 5.4 -> 4.0 us, 1000 x
+// 512 x 160 6.4 -> 5.4, 2500 x 384 x 64 6.2 -> 4.9, 8000 x 256 x 64 7.5 -> 6.3.
+constexpr bool atb_ahead(int MT, int NT) { return MT * NT == 2; }
+constexpr int atb_waves(int MT, int NT, bool LINES) { return LINES && atb_ahead(MT, NT) ? 12 : 8; }
+// The tile and the ranges of rows that cost least: rounds of one workgroup a compute
+// unit, each `ti` microseconds for every step of its wavefronts and `f` to start, to sum
+// and to store, and the atomics.  By lines fitted to 25 shapes (1000 to 198759 rows, 16 to
+// 1728 x 32 to 480, gathered and plain) in every tile and three to seven numbers of
+// ranges, 11 % rms: what it takes is 1.2 % off the fastest of these on average
+// (2.4 with the costs of eight wavefronts and ranges of 128 rows, rounded up to 192 by the
+// launch: 3000 x 864 x 64 10.2 -> 7.7, 45000 x 128 x 64 13.5 -> 12.0).  Where rows are loaded
+// into registers, eight wavefronts, their own costs.  Two by two tiles, us against two by one, plain rows: 126507 x 1728 x 64 175, 246;
+// 53325 x 640 x 320 135, 176; 17223 x 1280 x 480 145, 187; 139000 x 384 x 128 91, 117.
+// (The search is 0.1 to 2 us of the host's time, a launch some 5.)
+struct AtbTile {
+  int mt, nt;
+  double ti[2], f[2]; // registers, lines
+};
+static const AtbTile atbTiles[4] = {
+    {1, 1, {.8, .67}, {4., 2.2}}, {2, 1, {1.13, 1.4}, {4., 3.7}}, {1, 2, {1.13, 1.42}, {4., 4.2}}, {2, 2, {1.95, 1.36}, {6., 3.7}}};
+struct AtbChoice {
+  int tile;     // -1: none
+  int64_t rows; // of a range, whole steps of a workgroup
+  double cost;
+};
+static inline AtbChoice atb_choose(int numCU, int64_t M, int K, int N, bool lines, bool pairsA, bool pairsD, bool twoByTwo) {
+  AtbChoice best = {-1, 0, 1e300};
+  for (int i = 0; i < (twoByTwo ? 4 : 3); ++i) {
+    const AtbTile &t = atbTiles[i];
+    const int64_t tiles = tiles_of(K, 32 * t.mt) * tiles_of(N, 32 * t.nt), each = atb_waves(t.mt, t.nt, lines) * ATB_STEP;
+    if ((t.mt == 2 && !pairsA) || (t.nt == 2 && !pairsD) || tiles > 0x7fffffffll)
+      continue;
+    const int64_t most = tiles_of(M, each);
+    for (int64_t s = 1; s <= most && s <= 4096; s += s < 64 ? 1 : s / 32) {
+      const int64_t steps = tiles_of(M, s * each), ranges = tiles_of(M, steps * each), rounds = tiles_of(tiles * ranges, numCU);
+      const double cost = rounds * (steps * t.ti[lines] + t.f[lines]) + (double)tiles * ranges * t.mt * t.nt * 1024 / 2e5;
+      if (cost < best.cost)
+        best = {i, steps * each, cost};
+      if (rounds > 8)
+        break;
+    }
+  }
+  return best;
+}
+
 // ---- weight gradients of several layers (k_atb_many)
 // What a step and a tile's beginning and end take, in sixteenths of a microsecond
 // (measured by the clock in the kernel, layers of 2500 to 84000 rows: by lines 1.42

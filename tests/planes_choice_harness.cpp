@@ -25,3 +25,9 @@ extern "C" int joined(int numCU, int n, const int64_t *M, const int *K, const in
     out[k] = in[k];
   return count;
 }
+// a weight gradient's tile; out: the rows of a range, its cost
+extern "C" int atb(int numCU, int64_t M, int K, int N, int lines, int pairsA, int pairsD, int twoByTwo, int64_t *rows, double *cost) {
+  const AtbChoice c = atb_choose(numCU, M, K, N, lines != 0, pairsA != 0, pairsD != 0, twoByTwo != 0);
+  *rows = c.rows, *cost = c.cost;
+  return c.tile;
+}

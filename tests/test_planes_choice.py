@@ -1,4 +1,4 @@
-"""The choice of a contraction's tile, costed as it is launched, and of the weight gradients that share a launch, on the CPU."""
+"""The choice of a contraction's tile, costed as it is launched, and of the weight gradients' tiles and of those that share a launch, on the CPU."""
 import ctypes as C
 import math
 import os
@@ -70,3 +70,33 @@ def test_weight_gradients_of_one_launch(choice, items, want):
     out = (C.c_int * max(1, len(items)))()
     assert choice.joined(256, len(items), *(t(*(x[i] for x in items)) for i, t in enumerate(columns)), out) == sum(want)
     assert list(out)[:len(items)] == want
+
+
+# (wavefronts of sixteen rows, microseconds a step of them all and of a range, rows loaded into registers and by lines)
+ATB = [(1, 1, (8, 8), (.8, .67), (4., 2.2)), (2, 1, (8, 12), (1.13, 1.4), (4., 3.7)), (1, 2, (8, 12), (1.13, 1.42), (4., 4.2)),
+       (2, 2, (8, 8), (1.95, 1.36), (6., 3.7))]
+
+
+@pytest.mark.parametrize("M", [1, 127, 129, 193, 1000, 3000, 45000, 139000])
+@pytest.mark.parametrize("K,N", [(32, 32), (12, 32), (384, 128), (864, 64), (1280, 480)])
+@pytest.mark.parametrize("lines,pairsA,pairsD,twoByTwo", [(1, 1, 1, 1), (1, 1, 1, 0), (0, 0, 1, 0), (0, 0, 0, 1)])
+def test_a_weight_gradient_costs_what_its_launch_does(choice, M, K, N, lines, pairsA, pairsD, twoByTwo):
+    """ranges are whole steps of the workgroup that takes them, as many as are costed, and none of the other tiles with any
+    number of ranges up to 64 costs less"""
+    rows, cost = C.c_int64(), C.c_double()
+    choice.atb.argtypes = [C.c_int, C.c_int64] + 6 * [C.c_int] + [C.POINTER(C.c_int64), C.POINTER(C.c_double)]
+    tile = choice.atb(256, M, K, N, lines, pairsA, pairsD, twoByTwo, rows, cost)
+
+    def costs(t, rows):
+        mt, nt, waves, ti, f = ATB[t]
+        tiles, ranges = -(-K // (32 * mt)) * -(-N // (32 * nt)), -(-M // rows)
+        return (-(-tiles * ranges // 256) * (rows // (16 * waves[lines]) * ti[lines] + f[lines]) + tiles * ranges * mt * nt * 1024 / 2e5)
+
+    allowed = [t for t, (mt, nt, *_) in enumerate(ATB) if (t < 3 or twoByTwo) and (mt == 1 or pairsA) and (nt == 1 or pairsD)]
+    assert tile in allowed and rows.value > 0 and rows.value % (16 * ATB[tile][2][lines]) == 0
+    assert cost.value == pytest.approx(costs(tile, rows.value))
+    for t in allowed:
+        each = 16 * ATB[t][2][lines]
+        for s in range(1, min(64, -(-M // each)) + 1):
+            if -(-K // (32 * ATB[t][0])) * -(-N // (32 * ATB[t][1])) * s <= 8 * 256:
+                assert cost.value <= costs(t, -(-M // (s * each)) * each) * (1 + 1e-9)
