@@ -18,26 +18,35 @@ static inline bool image_larger(int planes, int64_t rows, int K, int N, int chan
 // to 800 columns; 10 % rms), of which it takes 25 to the fastest of these tiles or
 // one within 5 %.  Taller or wider tiles, one wavefront in place of two a SIMD, and
 // deeper rings gained nothing.
+// LONG: a workgroup's tiles take `begin`, and each `next` and `tl` a block.  Fitted to 37
+// shapes of plain rows in every tile (9000 to 400000 rows, 64 to 2560 k, 32 to 1280
+// columns; 3 to 11 % rms, all a tenth less than measured, as the others' are of plain
+// rows): what it takes is 1.5 % off the fastest on average.  (With t1 for tl and a smaller
+// `next` 4.7 %: 70000 x 160 x 36 23.4 us and not 19, 70000 x 512 x 64 59 and not 46.)  The
+// ring of six is never the fastest so: 64 x 64 tiles of which two share a compute unit are.
 struct LinesTile {
   int mt, nt, rw, cw, d, resident;
-  float f, t1, tn, next; // next: what a further tile of the same workgroup's begins and ends with (LONG)
+  float f, t1, tn, begin, next, tl; // tl 0: never LONG
 };
 static const LinesTile linesTiles[2][6] = {
-    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f}}, // one plane
-    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 3.3f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 3.4f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 4.5f},
-     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 2.f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 1.2f}}};
+    {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f, 0.f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f, 0.f, 0.f}}, // one plane
+    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 2.5f, 2.1f, 1.12f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 1.6f, 3.f, 1.3f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 3.8f, 2.45f, .88f},
+     {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 3.1f, 1.45f, .71f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 0.f, 0.f, 0.f}}};
 // How many workgroups an XCD has of a LONG launch, a multiple of the slices of columns
 // (0: a launch of a workgroup a tile): plain rows of no less than their weights, in three
-// planes, where a compute unit that has room for one workgroup has more than one tile.
-// (Gathered rows: 15948 x 1280 x 480 115 us for 110, 15003 x 1920 x 640 232 for 220,
-// with the rules of the next tiles under way; two workgroups to a compute unit see to
-// that themselves: 139000 x 128 x 64 36 for 29.)  The launch and the choice of its tile
-// both ask here: with LONG's costs for tiles that are not launched so, 2600 x 1024 x
-// 1920 took 78 us and not 68, 2500 x 256 x 2048 28 and not 25.
+// planes, of no more than 512 k, where a compute unit that has room for one workgroup has
+// more than one tile.  (Longer contractions have little of their time between the tiles:
+// in the tiles that are best for them, a workgroup a tile and LONG, 5000 x 2560 x 800 144,
+// 148, 26000 x 1280 x 480 168, 202; 16500 x 512 x 256 37.4, 38.1, its gradient 40, 37.
+// Gathered rows: 15948 x 1280 x 480 115 us for 110, 15003 x 1920 x 640 232 for 220, with the
+// rules of the next tiles under way; two workgroups to a compute unit see to that
+// themselves: 139000 x 128 x 64 36 for 29.)  The launch and the choice of its tile both ask
+// here: with LONG's costs for tiles that are not launched so, 2600 x 1024 x 1920 took 78 us
+// and not 68, 2500 x 256 x 2048 28 and not 25.
 static inline int lines_long(int numCU, int64_t M, int K, int N, int rows, int columns, int d) {
-  const int cus = numCU / 8;
+  const int cus = numCU / 8, T = K / 32;
   const int64_t splits = tiles_of(N, columns);
-  return K / 32 >= d - 1 && splits <= cus && !image_larger(3, M, K, N, K) && tiles_of(M, rows) * splits > numCU
+  return T >= d - 1 && T <= 16 && splits <= cus && !image_larger(3, M, K, N, K) && tiles_of(M, rows) * splits > numCU
              ? (int)(cus / splits * splits)
              : 0;
 }
@@ -48,9 +57,8 @@ static inline float lines_cost(int numCU, const LinesTile &x, int planes, int64_
   if (n <= x.resident) {
     const float shared = x.resident > 1 ? (fmaxf(ceilf(n), 1.f) - 1.f) / (x.resident - 1) : 0.f;
     cost = x.f + T * (x.t1 + shared * (x.tn - x.t1));
-  } else if (const int per = x.next > 0.f && !gather ? lines_long(numCU, M, K, N, rows, columns, x.d) : 0) {
-    const float long_ = n * numCU / (8 * per), rounds = long_ <= 3.f ? ceilf(long_) : long_ + .5f;
-    cost = 1.f + rounds * (x.next + T * x.t1);
+  } else if (const int per = x.tl > 0.f && !gather ? lines_long(numCU, M, K, N, rows, columns, x.d) : 0) {
+    cost = x.begin + tiles_of(tiles_of(M, rows) * tiles_of(N, columns), 8 * per) * (x.next + T * x.tl);
   } else {
     const float rounds = n / x.resident <= 3.f ? ceilf(n / x.resident) : n / x.resident + .5f;
     cost = rounds * (x.f + T * (x.resident > 1 ? x.tn : x.t1));

@@ -12,7 +12,7 @@ extern "C" float lines_tile_cost(int numCU, int planes, int tile, int64_t M, int
 // how the tile is launched (launch_lines): workgroups an XCD of a LONG launch, 0: a workgroup a tile
 extern "C" int lines_tile_long(int numCU, int tile, int64_t M, int K, int N) {
   const LinesTile &x = linesTiles[1][tile];
-  return x.next > 0.f ? lines_long(numCU, M, K, N, 32 * x.mt * x.rw, 32 * x.nt * x.cw, x.d) : 0;
+  return x.tl > 0.f ? lines_long(numCU, M, K, N, 32 * x.mt * x.rw, 32 * x.nt * x.cw, x.d) : 0;
 }
 // which of n weight gradients go into one launch; returns how many
 extern "C" int joined(int numCU, int n, const int64_t *M, const int *K, const int *N, const int *tile, const int *each, int *out) {

@@ -161,7 +161,7 @@ def test_weight_gradients_by_lines(scn, ctx, M, fs, nIn, N):
 # of one row, of all but one; rows that are not finite in the first, a middle and the last tile, which are taken again there
 @pytest.mark.parametrize("M,K,N", [(128 * 300 + 1, 64, 384), (128 * 523 - 1, 128, 128), (256 * 300 + 77, 64, 64), (33001, 128, 256),
                                    (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192), (16500, 512, 256),
-                                   (70003, 160, 36)])
+                                   (35001, 384, 112), (50001, 96, 160)])
 def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
     rng = np.random.default_rng(M + K + N)
     A, W = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
@@ -181,9 +181,9 @@ def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
 
 
 # the same forward, with bias and activation, in every tile that is launched so (test_planes_choice.py: these reach all), the bits
-# of the kernels that convert the weights on the way; five and six blocks of k in the ring of six
-SEVERAL = [(38401, 64, 384), (40000, 96, 640), (50001, 256, 192), (33001, 64, 160), (16500, 512, 256), (33001, 128, 256),
-           (8000, 96, 640), (70003, 160, 36), (70003, 192, 64)]
+# of the kernels that convert the weights on the way; two, three and more blocks of k
+SEVERAL = [(38401, 64, 384), (40000, 96, 640), (33001, 64, 160), (200003, 96, 64), (50001, 256, 192), (16500, 512, 256),
+           (35001, 384, 112), (33001, 512, 128)]
 
 
 @pytest.mark.parametrize("M,K,N", SEVERAL)

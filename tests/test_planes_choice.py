@@ -8,10 +8,10 @@ import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "sparseconvnet-archived_amd", "csrc")
-# rows, columns, begin, a block of 32 k (alone on its compute unit), a further tile of the same workgroup: of the tiles that
-# fill a compute unit's LDS, three planes
-TILES = {0: (128, 128, 4.1, 1.04, 3.3), 1: (256, 64, 4.3, 1.25, 3.4), 2: (128, 96, 4.5, .87, 4.5), 3: (64, 128, 3.4, .68, 2.),
-         5: (64, 64, 2., .5, 1.2)}
+# of the tiles of which a workgroup may take several, three planes: rows, columns, fewest blocks of 32 k that are several tiles to a
+# workgroup; microseconds of a tile alone and of its block, and of several: of them all, of each and of its block
+TILES = {0: (128, 128, 2, 4.1, 1.04, 2.5, 2.1, 1.12), 1: (256, 64, 2, 4.3, 1.25, 1.6, 3., 1.3), 2: (128, 96, 3, 4.5, .87, 3.8, 2.45, .88),
+         3: (64, 128, 3, 3.4, .68, 3.1, 1.45, .71)}
 
 
 @pytest.fixture(scope="module")
@@ -30,17 +30,18 @@ def choice(tmp_path_factory):
 # plain rows of less than their weights (the image 6 N K bytes, the rows 4 M K) are launched a workgroup a tile, others several
 # tiles to a workgroup; one row more or fewer at the line between the two
 @pytest.mark.parametrize("M,K,N", [(3000, 512, 3008), (2500, 256, 2048), (2600, 1024, 1920), (2880, 128, 1920), (2879, 128, 1920),
-                                   (139000, 384, 128), (40000, 96, 640), (9001, 64, 804), (5000, 64, 4096), (70000, 32, 96)])
+                                   (139000, 384, 128), (40000, 96, 640), (9001, 64, 804), (5000, 64, 4096), (70000, 32, 96),
+                                   (70000, 512, 64), (70000, 544, 64)])
 def test_a_tile_costs_what_its_launch_does(choice, M, K, N):
-    for t, (rows, columns, f, t1, further) in TILES.items():
-        wgs, per = -(-M // rows) * -(-N // columns), choice.lines_tile_long(256, t, M, K, N)
+    for t, (rows, columns, least, f, t1, begin, each, block) in TILES.items():
+        wgs, per, T = -(-M // rows) * -(-N // columns), choice.lines_tile_long(256, t, M, K, N), K // 32
         if wgs <= 256:
             assert per == 0
             continue
-        assert (per > 0) == (-(-N // 32) * 32 * 6 <= 4 * M and K // 32 >= {2: 3, 3: 3, 5: 5}.get(t, 2) and -(-N // columns) <= 32)
-        n = wgs / (8 * per if per else 256)
-        rounds = math.ceil(n - 1e-6) if n <= 3 else n + .5
-        want = 1 + rounds * (further + K // 32 * t1) if per else rounds * (f + K // 32 * t1)
+        assert (per > 0) == (-(-N // 32) * 32 * 6 <= 4 * M and least <= T <= 16 and -(-N // columns) <= 32)
+        n = wgs / 256
+        want = (begin + -(-wgs // (8 * per)) * (each + T * block) if per else
+                (math.ceil(n) if n <= 3 else n + .5) * (f + T * t1))
         assert choice.lines_tile_cost(256, 3, t, M, K, N, 0) == pytest.approx(want, rel=1e-5), t
 
 
@@ -48,6 +49,13 @@ def test_a_tile_costs_what_its_launch_does(choice, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(2500, 256, 2048), (2600, 1024, 1920)])
 def test_rows_of_less_than_their_weights(choice, M, K, N):
     assert choice.lines_tile(256, 3, M, K, N, 0) == 2
+
+
+# measured in every tile: the 64 x 64 of which two share a compute unit 19.0 and 46.4 us, several tiles of the others to a
+# workgroup no less than 20.4 and 52.5
+@pytest.mark.parametrize("M,K,N", [(70000, 160, 36), (70000, 512, 64)])
+def test_rows_of_few_columns(choice, M, K, N):
+    assert choice.lines_tile(256, 3, M, K, N, 0) == 4
 
 
 def test_shapes_of_several_tiles_to_a_workgroup(choice):
