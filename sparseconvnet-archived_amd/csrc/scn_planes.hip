@@ -816,11 +816,7 @@ template <int N> __device__ __forceinline__ void lines_landed() {
 // the 10 us that one of 128 x 128 x 128 took: 139000 x 128 x 128 55 us -> 37, 400000 x 96 x
 // 128 116 -> 73, 139000 x 256 x 192 109 -> 92, 50000 x 320 x 1280 265 -> 244.
 //   2: the results go past the caches, which the rows are wanted in (139000 x 128 x 384
-// 127 -> 115, and so 95): a gradient, which the scatter behind it reads once.
-//   1: they stay, for the pooling that reads a layer's output at once, in its windows'
-// order: contraction and pooling, one tile to a workgroup, past the caches, here: 57000 x
-// 256 x 96 36.5, 38.7, 36.5; 203000 x 64 x 64 48.9, 48.1, 43.1; 60000 x 320 x 160 70.1, 75.1,
-// 66.6; 35000 x 512 x 160 62.4, 64.8, 61.0.
+// 127 -> 115, and so 95); 1: through them (lines_past_caches).
 template <int PL, int MT, int NT, int RW, int CW, int D, bool GATHER, bool A16, int LONG = 0>
 __global__ void __launch_bounds__(64 * RW * CW, 2)
     k_nin_lines(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
@@ -1345,7 +1341,7 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
   if constexpr (PL == 3 && !A16 && D <= 4 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160) // (as linesTiles' tl)
     if (const int per = gs ? 0 : lines_long(ctx->numCU, scn_rows_hint(ctx, M), K, N, ROWS, COLUMNS, D)) {
       // (W turned: a gradient)
-      hipLaunchKernelGGL((wT ? k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 2> : k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 1>),
+      hipLaunchKernelGGL((lines_past_caches(scn_rows_hint(ctx, M), K, N, wT) ? k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 2> : k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 1>),
                          dim3(8 * per), dim3(64 * RW * CW), lds, ctx->stream, A, image, out, M, K, N, ep, GatherSource(), nSplits,
                          byColumns, rows, PlainW{W, wT});
       return SCN_OK;

@@ -50,6 +50,16 @@ static inline int lines_long(int numCU, int64_t M, int K, int N, int rows, int c
              ? (int)(cus / splits * splits)
              : 0;
 }
+// Whether LONG's results are to go past the caches: those of a gradient, which is read
+// once, and what would not be found there anyway, rows and results of more than the 256 MB
+// of the Infinity Cache.  A layer's output is read at once and by windows: contraction and
+// pooling, a workgroup a tile, past the caches, through them, 139000 x 384 x 128 138, 140,
+// 131; 139000 x 256 x 192 161, 165, 152; 100000 x 96 x 192 68, 76, 65; 60000 x 320 x 160 70,
+// 75, 67; 57000 x 256 x 96 36.5, 38.7, 36.5; 250000 x 128 x 192 229, 212, 220; 600000 x 64 x 64
+// 166, 145, 158.
+static inline bool lines_past_caches(int64_t M, int K, int N, bool gradient) {
+  return gradient || M * ((int64_t)K + N) * 4 > (int64_t)256 << 20;
+}
 static inline float lines_cost(int numCU, const LinesTile &x, int planes, int64_t M, int K, int N, bool gather) {
   const int T = K / 32, rows = 32 * x.mt * x.rw, columns = 32 * x.nt * x.cw;
   const float n = (float)tiles_of(M, rows) * tiles_of(N, columns) / numCU;

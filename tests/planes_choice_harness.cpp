@@ -31,3 +31,4 @@ extern "C" int atb(int numCU, int64_t M, int K, int N, int lines, int pairsA, in
   *rows = c.rows, *cost = c.cost;
   return c.tile;
 }
+extern "C" int past_caches(int64_t M, int K, int N, int gradient) { return lines_past_caches(M, K, N, gradient != 0); }

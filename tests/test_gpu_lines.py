@@ -181,9 +181,10 @@ def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
 
 
 # the same forward, with bias and activation, in every tile that is launched so (test_planes_choice.py: these reach all), the bits
-# of the kernels that convert the weights on the way; two, three and more blocks of k
+# of the kernels that convert the weights on the way; two, three and more blocks of k, the last of them rows and results that
+# are more than the caches
 SEVERAL = [(38401, 64, 384), (40000, 96, 640), (33001, 64, 160), (200003, 96, 64), (50001, 256, 192), (16500, 512, 256),
-           (35001, 384, 112), (33001, 512, 128)]
+           (35001, 384, 112), (33001, 512, 128), (720001, 64, 32)]
 
 
 @pytest.mark.parametrize("M,K,N", SEVERAL)

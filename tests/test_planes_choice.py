@@ -65,6 +65,14 @@ def test_shapes_of_several_tiles_to_a_workgroup(choice):
     assert all(choice.lines_tile_long(256, t, *s) > 0 for t, s in zip(tiles, SEVERAL)) and set(tiles) == set(TILES)
 
 
+# measured with the pooling behind it: 100000 x 96 x 192 76 us past the caches and 65 through them, 600000 x 64 x 64 145 and 158
+@pytest.mark.parametrize("M,K,N,gradient,want", [(100000, 96, 192, 0, 0), (100000, 96, 192, 1, 1), (600000, 64, 64, 0, 1),
+                                                 (1 << 19, 64, 64, 0, 0), ((1 << 19) + 1, 64, 64, 0, 1)])
+def test_results_past_the_caches(choice, M, K, N, gradient, want):
+    choice.past_caches.argtypes = [C.c_int64, C.c_int, C.c_int, C.c_int]
+    assert choice.past_caches(M, K, N, gradient) == want
+
+
 SMALL, FIRST, LARGE, EMPTY, OTHER = ((11400, 384, 128, 2, 25), (83597, 12, 32, 1, 21), (139000, 384, 128, 2, 25), (0, 384, 128, 2, 25),
                                      (5000, 30, 7, 0, 25))
 
