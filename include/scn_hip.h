@@ -572,6 +572,9 @@ typedef struct scn_pool_inverse_item {
 } scn_pool_inverse_item;
 int scn_pool_inverse_slots(int dimension, int size, int stride);
 int scn_pool_inverse_many(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems);
+/* ... and where every sample's windows begin, and the last one's end (the first batch + 1
+ * of d_samples), to `copy`, one item behind the other: device or pinned host memory */
+int scn_pool_inverse_many_copy(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems, int32_t *copy);
 int scn_maxpool_gradient(scn_ctx *ctx, float *d_din, int64_t inputRows, const float *d_dout, int64_t rows, int C,
                          const int32_t *d_choice, const float *d_out, int act, const int32_t *d_inverse, int slots,
                          const int32_t *d_samples, int batch, const int32_t *d_background, int fs);

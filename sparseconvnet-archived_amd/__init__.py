@@ -176,6 +176,7 @@ def lib():
         "scn_softmax_grad_copy": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, vp]),
         "scn_pool_inverse_slots": (C.c_int, [C.c_int, C.c_int, C.c_int]),
         "scn_pool_inverse_many": (C.c_int, [vp, P(PoolInverseItem), C.c_int]),
+        "scn_pool_inverse_many_copy": (C.c_int, [vp, P(PoolInverseItem), C.c_int, vp]),
         "scn_maxpool_gradient": (C.c_int, [vp, vp, i64, vp, i64, C.c_int, vp, vp, C.c_int, vp, C.c_int, vp, C.c_int, vp,
                                            C.c_int]),
         "scn_rules_inverse_many": (C.c_int, [vp, P(InverseItem), C.c_int]),
@@ -409,12 +410,15 @@ class Context:
     def maxpool_backward_through(self, d_din, d_dout, count, C, d_choice, d_out, act):
         _check(lib().scn_maxpool_backward_through(self.h, d_din.ptr, d_dout.ptr, count, C, d_choice.ptr, d_out.ptr, act))
 
-    def pool_inverse_many(self, items):
+    def pool_inverse_many(self, items, copy=None):
         """[(input grids, output grids, d_rules, d_inverse, d_samples, rows, inputRows, size, stride)]"""
         arr = (PoolInverseItem * max(1, len(items)))()
         for k, (g, h, rules, inverse, samples, rows, inputRows, size, stride) in enumerate(items):
             arr[k] = PoolInverseItem(g.h, h.h, rules.ptr, inverse.ptr, samples.ptr, rows, inputRows, size, stride)
-        _check(lib().scn_pool_inverse_many(self.h, arr, len(items)))
+        if copy is None:
+            _check(lib().scn_pool_inverse_many(self.h, arr, len(items)))
+        else:
+            _check(lib().scn_pool_inverse_many_copy(self.h, arr, len(items), copy.ptr))
 
     def maxpool_gradient(self, d_din, inputRows, d_dout, rows, C_, d_choice, d_out, act, d_inverse, slots, d_samples, batch,
                          d_background=None, fs=0):

@@ -1387,7 +1387,7 @@ extern "C" int scn_pool_inverse_slots(int dimension, int size, int stride) {
 }
 struct PoolInverseList {
   const int *rules[SCN_INVERSE_MAX], *bg[SCN_INVERSE_MAX], *outBg[SCN_INVERSE_MAX];
-  int *inverse[SCN_INVERSE_MAX], *samples[SCN_INVERSE_MAX];
+  int *inverse[SCN_INVERSE_MAX], *samples[SCN_INVERSE_MAX], *copy[SCN_INVERSE_MAX]; // copy: null, or the host's memory
   long long volume[SCN_INVERSE_MAX];
   int rows[SCN_INVERSE_MAX], inRows[SCN_INVERSE_MAX], batch[SCN_INVERSE_MAX];
   int dimension[SCN_INVERSE_MAX], size[SCN_INVERSE_MAX], stride[SCN_INVERSE_MAX], slots[SCN_INVERSE_MAX];
@@ -1397,6 +1397,7 @@ struct PoolInverseList {
 // a workgroup an item: where the samples' windows begin, and the background rows' marks
 __global__ __launch_bounds__(256) void k_pool_samples(PoolInverseList l) {
   const int t = blockIdx.x, batch = l.batch[t], slots = l.slots[t];
+  int *const copy = l.copy[t];
   // A sample's rows are its sites and then, if it is not full, a background row: its
   // last row follows from that row of the last sample up to it that has one, and the
   // full ones since.  (The last such sample by a running maximum; each looking back by
@@ -1404,8 +1405,11 @@ __global__ __launch_bounds__(256) void k_pool_samples(PoolInverseList l) {
   __shared__ int sLast[256];
   const int lane = threadIdx.x;
   int carry = -1;
-  if (lane == 0)
+  if (lane == 0) {
     l.samples[t][0] = 0;
+    if (copy)
+      copy[0] = 0;
+  }
   for (int base = 0; base < batch; base += 256) { // uniform
     const int s = base + lane, row = s < batch ? l.outBg[t][s] : -1;
     int last = row >= 0 ? s : carry;
@@ -1422,7 +1426,10 @@ __global__ __launch_bounds__(256) void k_pool_samples(PoolInverseList l) {
     __syncthreads();
     if (s < batch) {
       const long long e = last >= 0 ? l.outBg[t][last] + 1 + (s - last) * l.volume[t] : (s + 1) * l.volume[t];
-      l.samples[t][s + 1] = (int)(e < l.rows[t] ? e : l.rows[t]);
+      const int to = (int)(e < l.rows[t] ? e : l.rows[t]);
+      l.samples[t][s + 1] = to;
+      if (copy)
+        copy[s + 1] = to;
     }
   }
   for (int s = threadIdx.x; s < batch; s += 256) {
@@ -1461,6 +1468,9 @@ __global__ __launch_bounds__(256) void k_pool_inverse(PoolInverseList l) {
   }
 }
 extern "C" int scn_pool_inverse_many(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems) {
+  return scn_pool_inverse_many_copy(ctx, items, nItems, nullptr);
+}
+extern "C" int scn_pool_inverse_many_copy(scn_ctx *ctx, const scn_pool_inverse_item *items, int nItems, int32_t *copy) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_pool_inverse_many: null context");
   SCN_REQUIRE(nItems >= 0 && nItems <= SCN_INVERSE_MAX && (items || nItems == 0), SCN_ERR_ARG,
               "scn_pool_inverse_many: %d items (at most %d)", nItems, SCN_INVERSE_MAX);
@@ -1491,6 +1501,9 @@ extern "C" int scn_pool_inverse_many(scn_ctx *ctx, const scn_pool_inverse_item *
     l.volume[c] = it.output->vol;
     l.inverse[c] = it.d_inverse;
     l.samples[c] = it.d_samples;
+    l.copy[c] = copy;
+    if (copy)
+      copy += it.input->batch + 1;
     l.rows[c] = (int)it.rows;
     l.inRows[c] = (int)it.inputRows;
     l.batch[c] = it.input->batch;

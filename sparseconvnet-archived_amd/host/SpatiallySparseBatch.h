@@ -90,10 +90,10 @@ public:
   PinnedStage hostFeatures;
   size_t hostFeatureCount;
   std::unique_ptr<BatchResultStage> result;
-  // an unseen training batch: its poolings' rules turned round, one behind the other
-  // (first where the samples' windows begin, of all of them, which the host reads, too)
+  // an unseen training batch: its poolings' rules turned round, one behind the other, and
+  // where their samples' windows begin, for the host
   vectorCUDA<int> poolInverses;
-  PinnedStage poolSamples;
+  PinnedStage poolStarts;
   // SparseConvNetCUDA::backwardBatch: the layers' momentum steps, put off to the
   // end of the backward pass and queued together (elsewhere every layer queues its
   // own), and the products that they wait for

@@ -1101,7 +1101,6 @@ static void turnPoolings(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBa
   std::vector<scn_pool_inverse_item> items;
   std::vector<SpatiallySparseBatchInterface *> outs;
   auto room = [](size_t n) { return (n + 3) & ~(size_t)3; };
-  const size_t sampleRoom = room(2 * (size_t)b.batchSize + 1);
   size_t total = 0;
   for (size_t i = 0; i < cnn.layers.size(); ++i) {
     MaxPoolingLayer *const pool = dynamic_cast<MaxPoolingLayer *>(cnn.layers[i]);
@@ -1118,35 +1117,37 @@ static void turnPoolings(SparseConvNetCUDA &cnn, scn_ctx *ctx, SpatiallySparseBa
     items.push_back({in.deviceGrids, out.deviceGrids, out.rules.dPtr(), nullptr, nullptr, out.nSpatialSites,
                      in.nSpatialSites, pool->poolSize, pool->poolStride});
     outs.push_back(&out);
-    total += room((size_t)in.nSpatialSites * slots) + sampleRoom;
+    total += room((size_t)in.nSpatialSites * slots) + room(2 * (size_t)b.batchSize + 1);
   }
   if (items.empty())
     return;
   b.poolInverses.resize64(total);
-  int *const samples = b.poolInverses.dPtr(), *at = samples + items.size() * sampleRoom;
+  int *at = b.poolInverses.dPtr();
   for (size_t k = 0; k < items.size(); ++k) {
-    items[k].d_samples = samples + k * sampleRoom;
     items[k].d_inverse = at;
     at += room((size_t)items[k].inputRows * outs[k]->poolSlots);
+    items[k].d_samples = at;
+    at += room(2 * (size_t)b.batchSize + 1);
     outs[k]->poolInverse = items[k].d_inverse;
     outs[k]->poolSamples = items[k].d_samples;
   }
+  const size_t starts = (size_t)b.batchSize + 1;
+  b.poolStarts.reserve(items.size() * starts * sizeof(int32_t));
   for (size_t i = 0; i < items.size(); i += SCN_INVERSE_MAX)
-    SCN_CHECKED(scn_pool_inverse_many(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i)));
-  const size_t bytes = items.size() * sampleRoom * sizeof(int32_t);
-  b.poolSamples.reserve(bytes);
-  SCN_CHECKED(scn_copy(ctx, b.poolSamples.p, samples, bytes));
+    SCN_CHECKED(scn_pool_inverse_many_copy(ctx, items.data() + i, (int)std::min<size_t>(SCN_INVERSE_MAX, items.size() - i),
+                                           b.poolStarts.as<int32_t>() + i * starts));
 }
 // (when the stream is through: the poolings with a sample too long are scattered)
 static void keepTurnedPoolings(SparseConvNetCUDA &cnn, SpatiallySparseBatch &b) {
+  const int32_t *first = b.poolStarts.as<int32_t>();
   for (size_t i = 1; i < b.interfaces.size(); ++i) {
     SpatiallySparseBatchInterface &out = b.interfaces[i];
     if (!out.poolInverse)
       continue;
-    const int32_t *const first = b.poolSamples.as<int32_t>() + (out.poolSamples - b.poolInverses.dPtr());
     int64_t longest = 0;
     for (int s = 0; s < b.batchSize; ++s)
       longest = std::max<int64_t>(longest, first[s + 1] - first[s]);
+    first += b.batchSize + 1;
     if (longest > longestTurned(b.interfaces[i - 1], out))
       out.poolInverse = out.poolSamples = nullptr;
     else

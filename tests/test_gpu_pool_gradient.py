@@ -127,3 +127,26 @@ def test_the_longest_sample_decides(scn, sides, turned):
         net.close()
     for a, b in zip(*left):  # (the same forward pass, bit for bit: fp32 sums in other orders)
         assert rel_l2(a, b) <= 1e-5
+
+
+def test_where_the_samples_begin_is_copied(scn, ctx):
+    """two poolings' one behind the other; to pinned host memory as epochs have it, and nothing behind them"""
+    items, keep, n = [], [], 7
+    for field, size, stride in ((10, 3, 2), (13, 2, 2)):
+        g, _, _, _, _, _ = layer(scn, ctx, 2, field, 2, n, 0.2, field)
+        h, p = scn.Grids(ctx), scn.Grids(ctx)
+        inRows = g.plan_square(h, field, field - 1, 2, 1)
+        rows = h.plan_square(p, field - 1, (field - 1 - size) // stride + 1, size, stride)
+        rules = ctx.empty((rows, size * size), np.int32)
+        h.fill(p, rules, rows * size * size)
+        slots = scn.lib().scn_pool_inverse_slots(2, size, stride)
+        keep.append((g, h, p))
+        items.append((h, p, rules, ctx.empty((inRows, slots), np.int32), ctx.empty(2 * n + 1, np.int32), rows, inRows, size, stride))
+    copy = ctx.host_alloc(4 * 32)
+    to = copy.buffer()
+    host = np.frombuffer(to, np.int32)
+    host[:] = 7
+    ctx.pool_inverse_many(items, copy)
+    ctx.sync()
+    want = np.concatenate([i[4].download()[:n + 1] for i in items])
+    assert np.array_equal(host[:2 * (n + 1)], want) and np.all(host[2 * (n + 1):32] == 7)
