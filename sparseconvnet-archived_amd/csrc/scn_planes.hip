@@ -1338,7 +1338,7 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
   // An XCD takes neighbouring tiles: rows with all their columns, so that they come
   // to its L2 once, or, where the image is the larger part, columns with all rows.
   const bool byColumns = image_larger(PL, scn_rows_hint(ctx, M), K, N, gs ? gs->nIn : K);
-  if constexpr (PL == 3 && !A16 && D <= 4 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160) // (as linesTiles' tl)
+  if constexpr (PL == 3 && !A16 && D <= 4 && NT < 3 && 2 * D * (ROWS / 8 + NT * CW * PL * 2) > 160) // (as linesTiles' tl)
     if (const int per = gs ? 0 : lines_long(ctx->numCU, scn_rows_hint(ctx, M), K, N, ROWS, COLUMNS, D)) {
       // (W turned: a gradient)
       hipLaunchKernelGGL((lines_past_caches(scn_rows_hint(ctx, M), K, N, wT) ? k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 2> : k_nin_lines<PL, MT, NT, RW, CW, D, false, false, 1>),

@@ -23,14 +23,16 @@ static inline bool image_larger(int planes, int64_t rows, int K, int N, int chan
 // columns; 3 to 11 % rms, all a tenth less than measured, as the others' are of plain
 // rows): what it takes is 1.5 % off the fastest on average.  (With t1 for tl and a smaller
 // `next` 4.7 %: 70000 x 160 x 36 23.4 us and not 19, 70000 x 512 x 64 59 and not 46.)  The
-// ring of six is never the fastest so: 64 x 64 tiles of which two share a compute unit are.
+// ring of six is never the fastest so: 64 x 64 tiles of which two share a compute unit
+// are.  Three tiles of columns to a wavefront keep too much from one tile to the next: 35
+// registers spilled, whose memory is allocated when they are first launched.
 struct LinesTile {
   int mt, nt, rw, cw, d, resident;
   float f, t1, tn, begin, next, tl; // tl 0: never LONG
 };
 static const LinesTile linesTiles[2][6] = {
     {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f, 0.f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f, 0.f, 0.f}}, // one plane
-    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 2.5f, 2.1f, 1.12f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 1.6f, 3.f, 1.3f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 3.8f, 2.45f, .88f},
+    {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 2.5f, 2.1f, 1.12f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 1.6f, 3.f, 1.3f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 0.f, 0.f, 0.f},
      {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 3.1f, 1.45f, .71f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 0.f, 0.f, 0.f}}};
 // How many workgroups an XCD has of a LONG launch, a multiple of the slices of columns
 // (0: a launch of a workgroup a tile): plain rows of no less than their weights, in three

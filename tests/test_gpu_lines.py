@@ -160,8 +160,8 @@ def test_weight_gradients_by_lines(scn, ctx, M, fs, nIn, N):
 # of its last block by, and more; slices of columns that do not divide an XCD's workgroups (640, 1280: 5 and 10); the last tile
 # of one row, of all but one; rows that are not finite in the first, a middle and the last tile, which are taken again there
 @pytest.mark.parametrize("M,K,N", [(128 * 300 + 1, 64, 384), (128 * 523 - 1, 128, 128), (256 * 300 + 77, 64, 64), (33001, 128, 256),
-                                   (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192), (16500, 512, 256),
-                                   (35001, 384, 112), (50001, 96, 160)])
+                                   (70003, 128, 96), (40000, 96, 640), (20011, 320, 1280), (50001, 256, 192), (35001, 384, 112),
+                                   (50001, 96, 160)])
 def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
     rng = np.random.default_rng(M + K + N)
     A, W = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
@@ -183,7 +183,7 @@ def test_several_tiles_to_a_workgroup(scn, ctx, M, K, N):
 # the same forward, with bias and activation, in every tile that is launched so (test_planes_choice.py: these reach all), the bits
 # of the kernels that convert the weights on the way; two, three and more blocks of k, the last of them rows and results that
 # are more than the caches
-SEVERAL = [(38401, 64, 384), (40000, 96, 640), (33001, 64, 160), (200003, 96, 64), (50001, 256, 192), (16500, 512, 256),
+SEVERAL = [(38401, 64, 384), (40000, 96, 640), (33001, 64, 160), (200003, 96, 64), (33001, 128, 256), (33001, 512, 256),
            (35001, 384, 112), (33001, 512, 128), (720001, 64, 32)]
 
 

@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "sparseconvnet-archived_amd", "csrc")
 # of the tiles of which a workgroup may take several, three planes: rows, columns, fewest blocks of 32 k that are several tiles to a
 # workgroup; microseconds of a tile alone and of its block, and of several: of them all, of each and of its block
-TILES = {0: (128, 128, 2, 4.1, 1.04, 2.5, 2.1, 1.12), 1: (256, 64, 2, 4.3, 1.25, 1.6, 3., 1.3), 2: (128, 96, 3, 4.5, .87, 3.8, 2.45, .88),
+TILES = {0: (128, 128, 2, 4.1, 1.04, 2.5, 2.1, 1.12), 1: (256, 64, 2, 4.3, 1.25, 1.6, 3., 1.3),
          3: (64, 128, 3, 3.4, .68, 3.1, 1.45, .71)}
 
 
