@@ -418,6 +418,35 @@ def test_infinite_operands_of_the_weight_gradient(scn, ctx, M, fs, nIn, N):
     assert np.all(np.abs(got[sure] - sums[sure]) <= 2e-6 * np.abs(D).sum(0)[sure])
 
 
+# the same of several layers in one launch: rows by lines, a first layer's without, plain rows, some of more than one range,
+# so that a workgroup takes what is not finite again between tiles that are
+def test_infinite_operands_among_many_layers(scn, ctx):
+    rng = np.random.default_rng(6)
+    items, checks = [], []
+    for M, fs, nIn, N in ((391, 3, 36, 44), (20011, 4, 32, 64), (9001, 4, 3, 32), (5003, 1, 160, 96), (700, 1, 64, 100)):
+        n = 300 if fs > 1 else M
+        x, D = rng.standard_normal((n, nIn)).astype(np.float32), (0.1 / M * rng.standard_normal((M, N))).astype(np.float32)
+        x[3, 2], x[77, 2], x[5, 1], x[8, 0], D[M // 2, 11], D[M // 3, 2] = np.inf, -np.inf, np.nan, 3.4e38, np.inf, np.nan
+        rules = rng.integers(-1, n, (M, fs)).astype(np.int32) if fs > 1 else np.arange(M, dtype=np.int32)[:, None]
+        pitch = scn.lib().scn_positions_pitch(M)
+        positions = ctx.array(np.ascontiguousarray(np.pad(rules.T, ((0, 0), (0, pitch - M)), constant_values=-1))) if fs > 1 else None
+        dense = np.where(rules[:, :, None] >= 0, x[np.maximum(rules, 0)], 0).reshape(M, fs * nIn).astype(np.float64)
+        items.append((ctx.array(x), positions, fs, nIn, ctx.array(D), ctx.array(np.zeros((fs * nIn, N), np.float32)),
+                      ctx.array(np.zeros(N, np.float32)), M, N))
+        checks.append((dense, D.astype(np.float64)))
+    print("infinite operands among many", [i[2:4] + i[7:] for i in items], flush=True)
+    ctx.AtB_many(items)
+    for (dense, D), item in zip(checks, items):
+        with np.errstate(invalid="ignore"):
+            want = np.einsum("mk,mn->kn", dense, D)
+            size, sums = np.einsum("mk,mn->kn", np.abs(dense), np.abs(D)), D.sum(0)
+        for got, want, size in ((item[5].download(), want, size), (item[6].download(), sums, np.abs(D).sum(0))):
+            sure = np.isfinite(want)
+            assert not sure.all() and sure.any()
+            assert np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True)
+            assert np.all(np.abs(got[sure] - want[sure]) <= 2e-6 * size[sure])
+
+
 def test_an_epoch_with_an_infinite_weight(scn):
     """of a channel that is never above zero, so that the net's outputs are finite: an epoch of one batch leaves what the
     batch by itself, which gathers, leaves"""

@@ -150,3 +150,58 @@ def test_where_the_samples_begin_is_copied(scn, ctx):
     ctx.sync()
     want = np.concatenate([i[4].download()[:n + 1] for i in items])
     assert np.array_equal(host[:2 * (n + 1)], want) and np.all(host[2 * (n + 1):32] == 7)
+
+
+@pytest.mark.parametrize("d,field,size,stride,C", [(2, 30, 3, 2, 32), (3, 9, 2, 2, 20)])
+@pytest.mark.parametrize("act", ["RELU", "LEAKYRELU", "TANH", None])
+def test_pool_gradient_of_what_is_not_finite(scn, ctx, d, field, size, stride, C, act):
+    """infinities, NaN and the type's largest in the gradient and in what is pooled: each goes to the row that was chosen and
+    to the sums of its positions, and to nothing else"""
+    rng = np.random.default_rng(field + C)
+    batch = 4
+    g, n, _, fs, _, _ = layer(scn, ctx, d, field, 2, batch, 0.15, 3)
+    h, p = scn.Grids(ctx), scn.Grids(ctx)
+    mid = field - 1
+    inRows = g.plan_square(h, field, mid, 2, 1)
+    d_conv = ctx.empty((inRows, fs), np.int32)
+    g.fill(h, d_conv, inRows * fs)
+    rows, width = h.plan_square(p, mid, (mid - size) // stride + 1, size, stride), size ** d
+    d_rules = ctx.empty((rows, width), np.int32)
+    h.fill(p, d_rules, rows * width)
+    slots = scn.lib().scn_pool_inverse_slots(d, size, stride)
+    x, D = rng.standard_normal((inRows, C), dtype=np.float32), rng.standard_normal((rows, C), dtype=np.float32)
+    odd = [np.inf, -np.inf, np.nan, 1e37 if act == "TANH" else 3.4e38]  # (times 1 + o, and then 1 - o)
+    D.reshape(-1)[rng.choice(D.size, 12, replace=False)] = odd * 3
+    x.reshape(-1)[rng.choice(x.size, 8, replace=False)] = odd[:2] * 4
+    y, choice = ctx.empty((rows, C), np.float32), ctx.empty((rows, C), np.int32)
+    ctx.maxpool(ctx.array(x), y, d_rules, rows, width, C, choice)
+    inverse, samples = ctx.empty((inRows, slots), np.int32), ctx.empty(2 * batch + 1, np.int32)
+    ctx.pool_inverse_many([(h, p, d_rules, inverse, samples, rows, inRows, size, stride)])
+    background, convInverse = ctx.empty(inRows + 2 * batch, np.int32), ctx.empty((n, fs), np.int32)
+    ctx.rules_inverse_many([(g, d_conv, convInverse, background, None, inRows, n, fs)])
+    din = ctx.array(np.full((inRows + batch * fs, C), 7, np.float32))
+    print("pool gradient not finite", d, field, size, C, act, flush=True)
+    ctx.maxpool_gradient(din, inRows, ctx.array(D), rows, C, choice, y if act else None, getattr(scn, act) if act else scn.NOSIGMOID,
+                         inverse, slots, samples, batch, background, fs)
+    got, ch, v, o = din.download(), choice.download().astype(np.int64), D.astype(np.float64), y.download().astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        if act == "RELU":
+            v = np.where(o > 0, v, 0)
+        elif act == "LEAKYRELU":
+            v = np.where(o > 0, v, v * 0.01)
+        elif act == "TANH":
+            v = v * ((1 + o) * (1 - o))
+        want, size_of = np.zeros((inRows + batch * fs, C)), np.zeros((inRows + batch * fs, C))
+        first, mask = samples.download()[:batch + 1], background.download()[:inRows]
+        for w, c in zip(*np.nonzero(ch >= 0)):
+            r = ch[w, c] // C
+            s = np.searchsorted(first, w, side="right") - 1
+            for to in [r] + [inRows + s * fs + f for f in range(fs) if mask[r] >> f & 1]:
+                want[to, c] += v[w, c]
+                size_of[to, c] += abs(v[w, c])
+    sure = np.isfinite(want) & (size_of < 3e38)
+    assert sure.mean() > 0.9 and not sure.all()
+    assert np.all(np.abs(got[sure] - want[sure]) <= 4e-6 * size_of[sure] + 1e-30)
+    sure |= size_of > 3e38  # (a sum near the type's largest may round either way)
+    sure[~np.isfinite(want)] = False
+    assert np.array_equal(np.isnan(got[~sure]), np.isnan(want[~sure])) and np.array_equal(got[~sure], want[~sure].astype(np.float32), equal_nan=True)

@@ -271,3 +271,59 @@ def test_a_bound_beyond_32_bit_choices_is_no_batch_beyond_them(scn):
     net.close()
     assert 1.75e9 < rows * 8192 < 2 ** 31 < 1.25 * rows * 8192
     assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+def test_a_first_layer_and_its_matrix_ahead_of_their_rows(scn, ctx):
+    """scn_conv_nin_forward_matrix with rows known on the device: matrix and layer of the rows that there are, whichever way
+    the guess of them sent it (few rows: two launches; more: one)"""
+    rng = np.random.default_rng(15)
+    for nIn, N, fs, densities in ((3, 32, 4, (0.3, 0.3, 0.1, 0.02)), (3, 32, 4, (0.004, 0.004, 0.003))):
+        src, out = scn.Grids(ctx), scn.Grids(ctx)
+        d_W, d_B = (ctx.array(rng.standard_normal(s, dtype=np.float32)) for s in ((fs * nIn, N), (N,)))
+        for i, density in enumerate(densities):
+            samples, nSites = brute.random_samples(rng, 6, 2, 41, density)
+            inp = rng.standard_normal((nSites, nIn)).astype(np.float32)
+            d_in = ctx.array(inp)
+            rules, bound = _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+            matrix, got = ctx.array(np.full((bound, fs * nIn), 7, np.float32)), ctx.array(np.full((bound, N), 7, np.float32))
+            print("matrix ahead", density, bound, flush=True)
+            assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+            scn._check(scn.lib().scn_conv_nin_forward_matrix(ctx.h, d_in.ptr, rules.ptr, fs, nIn, matrix.ptr, d_W.ptr, d_B.ptr, None,
+                                                             got.ptr, bound, N, 1.0, scn.RELU, scn.FP32_PLANES))
+            scn.lib().scn_ctx_rows_from(ctx.h, None)
+            assert scn.settle(ctx)
+            held = C.c_int()
+            assert scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK
+            n = out.info()["nSpatialSites"]
+            r = rules.download().reshape(-1, fs)[:n]
+            dense = np.where(r[:, :, None] >= 0, inp[np.maximum(r, 0)], 0).reshape(n, fs * nIn)
+            assert np.array_equal(matrix.download()[:n], dense)
+            known = ctx.array(np.full((n, N), 7, np.float32))
+            ctx.nin_forward(ctx.array(dense), d_W, d_B, None, known, n, fs * nIn, N, 1.0, scn.RELU, scn.FP32_PLANES)
+            if held.value:
+                assert np.array_equal(got.download()[:n], known.download()), (density, n, bound)
+            else:
+                assert np.allclose(got.download()[:n], known.download(), rtol=1e-5, atol=1e-5)
+
+
+def test_several_tiles_to_a_workgroup_ahead_of_their_rows(scn, ctx):
+    """plain rows known on the device, more and fewer than the batch before had (k_nin_lines' LONG)"""
+    rng = np.random.default_rng(16)
+    K, N = 128, 128
+    src, out = scn.Grids(ctx), scn.Grids(ctx)
+    d_W, d_B = (ctx.array(rng.standard_normal(s, dtype=np.float32)) for s in ((K, N), (N,)))
+    for i, density in enumerate((0.5, 0.5, 0.3, 0.6)):
+        samples, nSites = brute.random_samples(rng, 30, 2, 41, density)
+        _, bound = _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+        A = ctx.array(rng.standard_normal((bound, K), dtype=np.float32))
+        got = ctx.array(np.full((bound, N), 7, np.float32))
+        print("several tiles ahead", density, bound, flush=True)
+        assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+        ctx.nin_forward(A, d_W, d_B, None, got, bound, K, N, 1.0, scn.RELU, scn.FP32_PLANES)
+        scn.lib().scn_ctx_rows_from(ctx.h, None)
+        assert scn.settle(ctx)
+        n = out.info()["nSpatialSites"]
+        known = ctx.array(np.full((n, N), 7, np.float32))
+        ctx.nin_forward(A, d_W, d_B, None, known, n, K, N, 1.0, scn.RELU, scn.FP32_PLANES)
+        assert np.array_equal(got.download()[:n], known.download()), (density, n, bound)
+        assert np.all(got.download()[n:] == 7)
