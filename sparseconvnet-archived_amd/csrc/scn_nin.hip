@@ -610,7 +610,8 @@ __global__ void __launch_bounds__(256)
 }
 // A net's first layer and, by workgroups before its own, the images of the weights of
 // the layers behind it, which by themselves are a launch of 4.4 to 10 us: 61 images in
-// the wide net 367 -> 358 us, 128 in bf16 354 -> 340, 100 drawings 193 -> 191.
+// the wide net 367 -> 358 us, 128 in bf16 354 -> 340, 100 drawings no more than their runs
+// differ by.
 template <int CT_GROUPS, bool MATRIX>
 __global__ void __launch_bounds__(256)
     k_conv_thin_images(ImageList images, unsigned imageBlocks, const float *__restrict__ A, const float *__restrict__ W,
