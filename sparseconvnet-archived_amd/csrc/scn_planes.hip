@@ -1213,6 +1213,253 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   }
 }
 
+// Long contractions of bf16 rows through rules, one plane, with the chip full.  A wavefront
+// owns 64 rows x 32 NT columns: six LDS reads to eight MFMAs (NT 4), where a tile of rows
+// to four of columns reads five to four, all that LDS gives while the pipe is busy, and
+// fetched its rows 32 to an instruction, all that the address unit does.  Rows come into
+// LDS by requests of 16 rows' 64 bytes, into a ring of the wavefront's own, so that a
+// block's place is asked for again as soon as it has been read, without a barrier: they
+// have one and a half blocks' time.  W comes from k_nin_lines' image, a ring for the
+// workgroup, one barrier a block.  A wavefront's rules come four positions at a time,
+// while the four before are used.  A step's operands are read under the step before; sums
+// in k_nin_planes' order: the same bits.
+// LDS: the rows' rings, W's, the rules (two sets of four positions).
+//
+// Microseconds with the rounding of the rows and the image, k_nin_planes -> here: 595610 x
+// 2592 x 128 423 -> 384, x 1728 x 64 225 -> 185; 389361 x 3456 x 96 336 -> 257; 116482 x
+// 1728 x 96 73 -> 56; 176025 x 864 x 192 102 -> 87 (k_nin_lines).  Of the first 16 % is
+// power: with zeros for data 367 -> 322.  The pipe is busy in 54 % of the cycles at 1.88 GHz
+// (46 before); without its requests the loop takes 290 of 358, and half of the rows' do not
+// change it by more than 6 %.  Eight wavefronts to a workgroup, half of W's requests: 387.
+constexpr int ROWS16_WAVES = 4;
+template <int NT>
+__global__ void __launch_bounds__(64 * ROWS16_WAVES, 2)
+    k_nin_rows16(const unsigned char *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out,
+                 long long M, int K, int N, Epilogue ep, GatherSource gs, int nSplits, RowRange rows) {
+  constexpr int WAVES = ROWS16_WAVES, MT = 2, D = 3, ROWS = 32 * MT * WAVES;
+  constexpr int A_BLOCK = 32 * MT * 64, W_BLOCK = NT * 2048; // of a wavefront, of the workgroup
+  constexpr int A_PER = A_BLOCK / 1024, W_PER = (2 * NT + WAVES - 1) / WAVES;
+  extern __shared__ __attribute__((aligned(16))) unsigned char sW[];
+  M = rows.live(M);
+  const unsigned tiles = (unsigned)((M + ROWS - 1) / ROWS) * nSplits;
+  if (blockIdx.x >= tiles)
+    return;
+  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, q = lane >> 5;
+  const int split = tileOf % nSplits;
+  const long long row0 = (long long)(tileOf / nSplits) * ROWS + wave * 32 * MT;
+  const int n0 = split * 32 * NT;
+  const int T = K / 32, perPosition = gs.nIn / 32;
+  unsigned char *const sA = sW + wave * D * A_BLOCK, *const sB = sW + WAVES * D * A_BLOCK;
+  int *const sRules = reinterpret_cast<int *>(sB + D * W_BLOCK) + wave * 2 * 128 * MT;
+  auto lds_at = [](const void *p) {
+    return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
+  };
+  const unsigned ldsA = __builtin_amdgcn_readfirstlane(lds_at(sA)), ldsB = __builtin_amdgcn_readfirstlane(lds_at(sB)),
+                 ldsRules = __builtin_amdgcn_readfirstlane(lds_at(sRules));
+
+  // ---- requests
+  const unsigned char *wSrc[W_PER];
+  const int lastTile = (N + 31) / 32 - 1;
+#pragma unroll
+  for (int u = 0; u < W_PER; ++u) {
+    int x = wave + WAVES * u;
+    x = x < 2 * NT ? x : 2 * NT - 1; // (past the end: the last one again)
+    int tile = split * NT + x / 2;
+    tile = tile < lastTile ? tile : lastTile;
+    wSrc[u] = image + ((long long)tile * T * 2 + x % 2) * 1024 + 16 * lane;
+  }
+  auto fetch_w = [&](int t, int slot, int u) {
+    const int x = wave + WAVES * u;
+    dma_kilobyte(ldsB + slot * W_BLOCK + (x < 2 * NT ? x : 2 * NT - 1) * 1024, wSrc[u] + (long long)t * 2048);
+  };
+  // sixteen rows' rules of four positions, a word a lane (rows and positions past the end:
+  // the last ones)
+  auto fetch_rules = [&](int group, int u) {
+    long long m = row0 + 16 * u + lane / 4;
+    m = m < M ? m : M - 1;
+    const int f = 4 * group + lane % 4;
+    dma_words(ldsRules + ((group & 1) * 2 * MT + u) * 256, gs.rules + m * gs.fs + (f < gs.fs ? f : gs.fs - 1));
+  };
+  // (two rows lie on 32 banks and four on all: a row's four pieces are rotated by pairs of
+  // rows, and again every eight)
+  const int piece = 16 * ((lane & 3) ^ (lane >> 3 & 3) ^ (lane >> 5));
+  const unsigned char *rowPtr[A_PER];
+  int f = 0, ch = 0; // the block to ask for
+  int rule[A_PER];
+  auto look_up = [&]() { // (rules that have landed; before the first block of a position)
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u)
+      rule[u] = sRules[((f >> 2 & 1) * 2 * MT + u) * 64 + (lane & ~3) + (f & 3)];
+  };
+  auto aim = [&]() {
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u)
+      asm volatile("" : "+v"(rule[u])); // (all of them waited for at once)
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u) {
+      const unsigned long long from = (unsigned long long)(uintptr_t)A + (unsigned long long)(unsigned)rule[u] * (unsigned)(gs.nIn * 2);
+      rowPtr[u] = reinterpret_cast<const unsigned char *>(rule[u] >= 0 ? from : (unsigned long long)(uintptr_t)gs.zeros) + piece;
+    }
+    // (a quarter of the next four, ahead of the rows: landed when all but those have)
+    if (4 * (f / 4 + 1) < gs.fs)
+      fetch_rules(f / 4 + 1, f & 3);
+  };
+  auto fetch_a = [&](int slot, int u) {
+    dma_kilobyte(ldsA + slot * A_BLOCK + u * 1024, rowPtr[u] + ch * 64);
+  };
+  auto advance = [&]() {
+    if (++ch == perPosition)
+      ch = 0, ++f;
+  };
+
+  // ---- operands
+  const unsigned char *const aLane = sA + c * 64;
+  const int swizzle = (c >> 1 & 3) ^ (c >> 3 & 1);
+  const unsigned char *const wLane = sB + lane * 16;
+  bf16x8 a[2][MT], b[2][NT]; // of a step
+  auto read = [&](int slot, int s, int x) { // the x'th operand of a step
+    if (x < MT)
+      a[s][x] = *reinterpret_cast<const bf16x8 *>(aLane + slot * A_BLOCK + x * 2048 + (((2 * s + q) ^ swizzle) * 16));
+    else if (x < MT + NT)
+      b[s][x - MT] = *reinterpret_cast<const bf16x8 *>(wLane + slot * W_BLOCK + ((x - MT) * 2 + s) * 1024);
+  };
+
+  // ---- prologue
+  ColEpilogue col[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + 32 * j + c;
+    col[j] = load_col(ep, n < N ? n : N - 1);
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) // (asked for now: nothing the compiler waits for is left for the loop)
+    asm volatile("" : "+v"(col[j].pb), "+v"(col[j].slope));
+#pragma unroll
+  for (int u = 0; u < 2 * MT; ++u)
+    fetch_rules(0, u);
+#pragma unroll
+  for (int t = 0; t < D - 1; ++t) // (T is at least two)
+#pragma unroll
+    for (int u = 0; u < W_PER; ++u)
+      fetch_w(t, t, u);
+  lines_landed<(D - 1) * W_PER>();
+#pragma unroll 1
+  for (int t = 0; t < D && t < T; ++t) {
+    if (ch == 0) {
+      look_up();
+      aim();
+    }
+#pragma unroll
+    for (int u = 0; u < A_PER; ++u)
+      fetch_a(t, u);
+    advance();
+  }
+  lines_landed<0>();
+  barrier_lds();
+
+  floatx16 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[i][j][v] = 0.f;
+  int cur = 0, next = 1, last = 2; // slots of blocks t, t + 1 and t - 1 (or t + 2)
+#pragma unroll
+  for (int x = 0; x < MT + NT; ++x)
+    read(0, 0, x);
+
+  constexpr int G = MT * NT, SPREAD = G / 4; // MFMAs of a step; the next step's operands are read behind the first of them
+  auto step = [&](int s, int slot, auto &&between) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int i = g / NT, j = g % NT;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][i], b[s][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      read(slot, s ^ 1, g);
+      if (g == G - 1)
+#pragma unroll
+        for (int x = G; x < MT + NT; ++x)
+          read(slot, s ^ 1, x);
+      between(g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // A block's requests, among the MFMAs: in its second step the W of block t + 2 and the
+  // first half of block t + 3's rows, in the next block's first step the other half.
+  auto block = [&](int t, auto steady) { // steady: with blocks to ask for
+    const bool rest = steady || t + D - 1 < T; // uniform: the last block's other half
+    const int before = last;
+    step(0, cur, [&](int g) {
+#pragma unroll
+      for (int u = A_PER / 2; u < A_PER; ++u)
+        if (g == (u - A_PER / 2) * SPREAD && rest && t > 0)
+          fetch_a(before, u);
+      if (g == SPREAD * A_PER / 2 && rest && t > 0)
+        advance();
+    });
+    // Of what this wavefront has asked for, all but the rows of block t + 2 has landed,
+    // and behind the barrier the others' parts of block t + 1's W too; nobody reads
+    // block t - 1's any more, whose place block t + 2's takes.
+    if (steady)
+      lines_landed<A_PER>();
+    else
+      lines_landed<0>();
+    asm volatile("s_barrier" ::: "memory");
+    const bool more = steady || t + D < T, turn = more && ch == 0; // uniform
+    if (turn)
+      look_up();
+    step(1, next, [&](int g) {
+#pragma unroll
+      for (int u = 0; u < W_PER; ++u)
+        if (g == u * SPREAD && (steady || t + 2 < T))
+          fetch_w(t + 2, last, u);
+      // (this block's rows are in registers since this step's first MFMAs: its place is
+      // asked for again)
+      if (g == G / 2 - 1 && turn)
+        aim();
+#pragma unroll
+      for (int u = 0; u < A_PER / 2; ++u)
+        if (g == G / 2 + u * SPREAD && more)
+          fetch_a(cur, u);
+    });
+    const int was = cur;
+    cur = next, next = last, last = was;
+  };
+  int t = 0;
+#pragma unroll 1
+  for (; t + D < T; ++t)
+    block(t, std::true_type());
+#pragma unroll 1
+  for (; t < T; ++t)
+    block(t, std::false_type());
+
+  // ---- epilogue: register v of a tile is row 8 (v / 4) + 4 q + v % 4
+  // (what lies past the last row, or in no column, is past the buffer's end: not stored)
+  const long long left = ((M - row0) * N - n0) * 4;
+  const __amdgpu_buffer_rsrc_t to =
+      __builtin_amdgcn_make_buffer_rsrc(out + row0 * N + n0, 0, (int)(left < 0 ? 0 : left < 0x40000000 ? left : 0x40000000),
+                                        0x00020000);
+  const unsigned pitch = 4u * (unsigned)N;
+  unsigned at[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    at[j] = n0 + 32 * j + c < N ? (unsigned)(4 * q) * pitch + 128u * j + 4u * c : 0x80000000u;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(finish(acc[i][j][v], col[j])), to, at[j], 0, 0);
+        at[j] += v % 4 == 3 ? 5 * pitch : pitch;
+      }
+}
+
 // The image of W that k_nin_planes reads: for every slice of 32 NT
 // columns and every block of 32 k what w_store leaves in LDS, in that order.
 template <int PL, int NT>
@@ -1354,6 +1601,23 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
                        out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
   return SCN_OK;
 }
+// (nIn in 32s; an image made by the call where there is none)
+template <int NT>
+static int launch_rows16(scn_ctx *ctx, const void *A, const float *W, float *out, long long M, int K, int N,
+                         const Epilogue &ep, const GatherSource &gs, const RowRange &rows, const unsigned char *image) {
+  if (!image) {
+    ImageList l;
+    l.count = 0, l.firstBlock[0] = 0;
+    add_image(l, W, ctx->d_image, 1, K, N, 0);
+    SCN_TRY(weight_images(ctx, l));
+    image = ctx->d_image;
+  }
+  const int nSplits = scn_ceil_div(N, 32 * NT);
+  const size_t lds = ROWS16_WAVES * (3 * 4096 + 2048) + 3 * NT * 2048; // (NT 4: two workgroups to a compute unit, just)
+  hipLaunchKernelGGL((k_nin_rows16<NT>), dim3((unsigned)(scn_ceil_div(M, 64 * ROWS16_WAVES) * (long long)nSplits)),
+                     dim3(64 * ROWS16_WAVES), lds, ctx->stream, (const unsigned char *)A, image, out, M, K, N, ep, gs, nSplits, rows);
+  return SCN_OK;
+}
 template <int PL>
 static int launch_splitk(scn_ctx *ctx, const float *A, const float *W,
                          float *out, long long M, int K, int N,
@@ -1429,6 +1693,7 @@ struct PlanesChoice {
   bool image;
   float cost; // microseconds, about
   int lines = -1; // k_nin_lines, a tile of its own: index into linesTiles
+  int rows16 = 0; // k_nin_rows16, of so many tiles of columns
   const unsigned char *weights = nullptr; // the image it reads, null: to be made
 };
 // needImage: of the tiles, only from the image (scn_planes_abt: whether there is one)
@@ -1497,6 +1762,15 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
   } else if (choice.tile < 0) {
     return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
   }
+  if constexpr (PL == 1)
+    switch (choice.rows16) {
+    case 2:
+      return launch_rows16<2>(ctx, A, W, out, M, K, N, ep, *gs, rows, choice.weights);
+    case 3:
+      return launch_rows16<3>(ctx, A, W, out, M, K, N, ep, *gs, rows, choice.weights);
+    case 4:
+      return launch_rows16<4>(ctx, A, W, out, M, K, N, ep, *gs, rows, choice.weights);
+    }
 #define SCN_LINES_CASE(I, MT, NT, RW, CW, D)                                                                             \
   case I:                                                                                                               \
     return launch_lines<PL, MT, NT, RW, CW, D>(ctx, A, W, out, M, K, N, ep, gs, wT, rows, choice.weights);
@@ -1583,11 +1857,14 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
   // positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444 us against 474.
   // k_nin_planes' cost is 2 too high where it converts W on the way, of layers that
   // small.)
-  if (a16 && choice.tile >= 0 && K <= 1280 && N > 32 && lines_shape(1, K, N, gs->nIn) &&
-      (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES)) &&
-      lines_rows16(ctx, rows, K, N, image != nullptr) < choice.cost - (choice.image ? 0.f : 2.f)) {
-    choice.lines = N <= 64 ? 4 : 3;
-    choice.weights = (const unsigned char *)image;
+  if (a16 && choice.tile >= 0 && N > 32 && lines_shape(1, K, N, gs->nIn) &&
+      (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES))) {
+    choice.rows16 = rows16_tiles(ctx->numCU, rows, K, N);
+    if (choice.rows16 == 0 && K <= 1280 &&
+        lines_rows16(ctx, rows, K, N, image != nullptr) < choice.cost - (choice.image ? 0.f : 2.f))
+      choice.lines = N <= 64 ? 4 : 3;
+    if (choice.rows16 || choice.lines >= 0)
+      choice.weights = (const unsigned char *)image;
   }
   if (choice.tile >= 0 && !a16)
     lines_instead(ctx, planes, rows, K, N, gs, image, room, choice);

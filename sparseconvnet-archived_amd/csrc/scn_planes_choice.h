@@ -89,6 +89,25 @@ static inline float lines_choose(int numCU, int planes, int64_t M, int K, int N,
   return least + 4.f;
 }
 
+// k_nin_rows16: how many tiles of columns a wavefront of it takes, 0: not one for it (bf16
+// rows through rules; more than 32 columns).  Slices cost what their columns do and the
+// fetching of the rows.  Measured against what else there is (k_nin_planes, k_nin_lines) on 69 shapes of
+// 800 to 674000 rows, 256 to 3456 k and 64 to 320 columns, by workgroups to a compute unit: two
+// tiles of columns 0.73 to 1.3 of them 1.09, 2.2 to 2.3 0.93 to 0.98 (2592 k 0.95), from 3.6
+// on 0.70 to 0.96; three 0.45 1.09, 0.86 to 1.1 0.91 to 0.94, from 1.6 on 0.71 to 0.95; four 0.15 to 0.3
+// 1.1 to 1.3, 0.33 to 0.76 from 2016 k on 0.91 to 0.99, 1.1 to 1.4 0.84 to 1.03, then 0.77 to
+// 0.94.  Shorter ones, of 256 to 864 k, have more of their time in a workgroup's start and stores:
+// up to 3 workgroups 0.99 to 1.5, from 4 on 0.79 to 1.01.
+static inline int rows16_tiles(int numCU, int64_t M, int K, int N) {
+  int tiles = 0;
+  int64_t least = INT64_MAX;
+  for (int nt = 4; nt >= 2; --nt)
+    if (const int64_t cost = tiles_of(N, 32 * nt) * (nt + 1); cost < least)
+      least = cost, tiles = nt;
+  const float n = (float)tiles_of(M, 256) * tiles_of(N, 32 * tiles) / numCU;
+  return n >= (K < 896 ? 4.f : tiles == 2 ? 2.f : tiles == 4 && K >= 2000 ? .4f : .8f) ? tiles : 0;
+}
+
 // ---- a weight gradient (scn_atb_planes)
 constexpr int ATB_STEP = 16; // rows that a wavefront takes at a time
 // By lines, tiles of two have a step's planes made among the MFMAs of the step before, and
