@@ -1916,7 +1916,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   if (planes && rounded && act != SCN_SOFTMAX) {
     const bool a16 = precision == SCN_BF16 && rows16 && gs && gs->nIn % 8 == 0 && ((uintptr_t)rows16 & 15) == 0;
     SCN_TRY(scn_planes_forward(ctx, precision == SCN_BF16 ? 1 : 2, a16 ? (const float *)rows16 : d_A, d_W, d_out, M,
-                               K, N, ep, gs, a16, image));
+                               K, N, ep, gs, a16, image, d_A));
   } else if (tiledBf16) {
     SCN_REQUIRE(!gs, SCN_ERR_ARG,
                 "fused convolution: shape outside the bf16 kernel's range");

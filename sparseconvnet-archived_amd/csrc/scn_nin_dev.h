@@ -70,11 +70,12 @@ int scn_conv_named(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int 
 bool scn_planes_shape(int K);
 // ... takes the split contraction: few rows
 bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N);
-// (image: W as scn_weight_images_many leaves it, or null)
+// (image: W as scn_weight_images_many leaves it, or null; a16: A holds bf16 rows, those
+// of A32 rounded)
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
                        const Epilogue &ep, const GatherSource *gs, bool a16,
-                       const void *image = nullptr);
+                       const void *image = nullptr, const float *A32 = nullptr);
 // dW += A^T D, db (may be null) += the column sums of D (gs: the rows of A through
 // rules, position by position)
 int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db,

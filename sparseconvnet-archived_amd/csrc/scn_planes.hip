@@ -1213,6 +1213,268 @@ __global__ void __launch_bounds__(64 * RW * CW, 2)
   }
 }
 
+// The split contraction where there are more rows: 64 rows x 64 columns a workgroup, whose
+// eight wavefronts take the blocks of 32 k in turn, as k_nin_planes_splitk's do, with the same
+// sums in the same order: the same bits.  A wavefront owns all of the tile, so that no two
+// want the same piece of A or W: rows come into a ring of its own in LDS by whole lines (each
+// sixteen bytes through the rule of its own position), W straight into registers, from
+// k_nin_lines' image or as it stands, and there is no barrier between the first block and
+// the last.  The eight partial tiles meet in the rings' place.
+// What bounds it: a block is 20 KB for 48 MFMAs, and a wavefront waits once a step for what
+// it asked for a step before: eight blocks take 2.5 us where the MFMAs are 1.4.  The tiles of
+// k_nin_lines move half of that and leave compute units idle at so few rows: split_rows has
+// both sides' times.  1037 x 2560 x 800 49 -> 32 us (W as it stands: 37), 16000 x 1728 x 64 36
+// -> 24, channels in other than 32s 1037 x 1600 x 800 54 -> 26; 61 images 354 -> 337.
+enum { S64_IMAGE, S64_PLAIN, S64_TURNED }; // W: its image, [K x N], [N x K]
+template <int PL, bool GATHER, int WM>
+__global__ void __launch_bounds__(512, 2)
+    k_nin_split64(const float *__restrict__ A, const unsigned char *__restrict__ image, float *__restrict__ out, long long M,
+                  int K, int N, Epilogue ep, GatherSource gs, int nSplits, bool byColumns, RowRange rows, PlainW plain) {
+  constexpr int SLOT = 8192, RING = 2 * SLOT;
+  extern __shared__ __attribute__((aligned(16))) unsigned char sW[]; // [8][RING], then the rules
+  M = rows.live(M);
+  const unsigned rowTiles = (unsigned)((M + 63) / 64), tiles = rowTiles * nSplits;
+  if (blockIdx.x >= tiles)
+    return;
+  const unsigned tileOf = xcd_eighth(blockIdx.x, tiles);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, q = lane >> 5;
+  const int split = byColumns ? tileOf / rowTiles : tileOf % nSplits;
+  const long long row0 = (long long)(byColumns ? tileOf % rowTiles : tileOf / nSplits) * 64;
+  const int n0 = split * 64;
+  const int T = K / 32;
+  int *const sRules = reinterpret_cast<int *>(sW + 8 * RING);
+  unsigned char *const ring = sW + wave * RING;
+  const unsigned ldsRing =
+      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)ring);
+  const unsigned char *const Ab = reinterpret_cast<const unsigned char *>(A);
+
+  // ---- W: a step's chunks of the image, or its eight k of a lane's two columns
+  const int lastTile = (N + 31) / 32 - 1;
+  const unsigned char *wSrc[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int tile = 2 * split + j < lastTile ? 2 * split + j : lastTile;
+    wSrc[j] = image + (long long)tile * T * (2 * PL * 1024) + 16 * lane;
+  }
+  constexpr int WS = WM == S64_IMAGE ? 2 : 1;
+  bf16x8 w[WS][2][PL]; // of a step
+  float wRaw[2][WM == S64_IMAGE ? 1 : 8]; // of the next one
+  auto load_w = [&](int t, int s) {
+    t = t < T ? t : T - 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (WM == S64_IMAGE) {
+#pragma unroll
+        for (int l = 0; l < PL; ++l)
+          w[s % WS][j][l] = *reinterpret_cast<const bf16x8 *>(wSrc[j] + ((long long)t * (2 * PL) + 2 * l + s) * 1024);
+      } else {
+        const int n = n0 + 32 * j + c < N ? n0 + 32 * j + c : N - 1, k = 32 * t + 16 * s + 8 * q;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          wRaw[j][i % (WM == S64_IMAGE ? 1 : 8)] = plain.W[WM == S64_TURNED ? (long long)n * K + k + i : (long long)(k + i) * N + n];
+      }
+    }
+  };
+  auto take_w = [&](int t, int s) { // the step whose W was asked for last, and the next one's asked for
+    if constexpr (WM == S64_IMAGE) {
+      load_w(t, s);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        split8<PL>(reinterpret_cast<const float(&)[8]>(wRaw[j]), w[0][j]);
+      load_w(t, s);
+    }
+  };
+  // ---- rows: eight of them, a line each, to a request; a line's pieces are rotated by the row
+  const int piece = (lane & 7) ^ (lane >> 3);
+  int f = 0;         // GATHER: the position of this lane's piece, and where in a row of it
+  unsigned in = 0;
+  auto aim = [&](int t) {
+    t = t < T ? t : T - 1;
+    const unsigned k = 32 * t + 4 * piece;
+    f = GATHER ? (int)__umulhi(k, gs.magic) : 0;
+    in = 4 * (k - (GATHER ? f * gs.nIn : 0));
+  };
+  auto fetch = [&](int slot, int u) { // of the block aimed at
+    int r = 8 * u + (lane >> 3);
+    asm volatile("" : "+v"(r)); // (no address is kept from block to block)
+    unsigned long long from;
+    if (GATHER) {
+      const int rule = sRules[r * gs.fs + f];
+      from = rule >= 0 ? (unsigned long long)(uintptr_t)Ab + (unsigned long long)(unsigned)rule * (unsigned)(gs.nIn * 4)
+                       : (unsigned long long)(uintptr_t)gs.zeros;
+    } else {
+      const long long m = row0 + r < M ? row0 + r : M - 1; // rows past the end: read a valid row, store nothing
+      from = (unsigned long long)(uintptr_t)Ab + (unsigned long long)m * (unsigned)K * 4;
+    }
+    dma_kilobyte(ldsRing + slot * SLOT + u * 1024, reinterpret_cast<const unsigned char *>(from + in));
+  };
+
+  // ---- operands
+  floatx4 raw[2];
+  unsigned ap[2][PL][4]; // words of an MFMA operand: two k each
+  auto read_a = [&](int slot, int u) { // unit u of a block: (step, row tile)
+    const unsigned char *const p = ring + slot * SLOT + (u % 2) * 4096 + c * 128;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      raw[h] = *reinterpret_cast<const floatx4 *>(p + (((4 * (u / 2) + 2 * q + h) ^ (c & 7)) * 16));
+  };
+  auto a_split = [&](int dst, int p) { // a quarter of it
+    const floatx4 x = raw[p / 2];
+    unsigned v[PL];
+    split2<PL>(x[2 * (p % 2)], x[2 * (p % 2) + 1], v);
+#pragma unroll
+    for (int l = 0; l < PL; ++l) {
+      asm volatile("" : "+v"(v[l])); // (here, and not where it is used)
+      ap[dst][l][p] = v[l];
+    }
+  };
+  auto operand = [&](int src, int l) {
+    return __builtin_bit_cast(bf16x8, uint4{ap[src][l][0], ap[src][l][1], ap[src][l][2], ap[src][l][3]});
+  };
+  constexpr int NACC = PL > 1 ? 2 : 1;
+  floatx16 acc[NACC][2][2];
+#pragma unroll
+  for (int h = 0; h < NACC; ++h)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[h][i][j][v] = 0.f;
+
+  // ---- the blocks
+  load_w(wave, 0);
+  if (GATHER) {
+    const long long first = row0 * gs.fs, last = M * gs.fs - 1;
+    for (int i = tid; i < 64 * gs.fs; i += 512) {
+      const long long r = first + i;
+      sRules[i] = gs.rules[r < last ? r : last];
+    }
+    __syncthreads();
+  }
+  if (wave < T) {
+    aim(wave);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      fetch(0, u);
+    lines_landed<0>();
+    read_a(0, 0);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      a_split(0, p);
+    read_a(0, 1);
+    int cur = 0;
+#pragma unroll 1
+    for (int t = wave; t < T; t += 8) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int s = u / 2, i = u % 2, src = u & 1;
+        if (u == 2) // the next block's rows, and this one's other W
+          lines_landed<0>();
+        if (u == 0)
+          take_w(t, 1);
+        if (u == 2)
+          take_w(t + 8, 0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+          for (int x = 0; x < PL; ++x)
+#pragma unroll
+            for (int y = 0; x + y < PL; ++y) {
+              floatx16 &d = acc[x + y == 0 ? 0 : NACC - 1][i][j];
+              d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(src, x), w[s % WS][j][y], d, 0, 0, 0);
+            }
+#pragma unroll
+          for (int p = 2 * j; p < 2 * j + 2; ++p)
+            a_split(src ^ 1, p);
+          if (j == 1) // (split: its registers take the next but one)
+            read_a(u + 2 < 4 ? cur : cur ^ 1, (u + 2) % 4);
+          if (s == 0) { // (the next block's rows: the last one's place)
+            if (u == 0 && j == 0)
+              aim(t + 8);
+            fetch(cur ^ 1, 4 * i + 2 * j);
+            fetch(cur ^ 1, 4 * i + 2 * j + 1);
+          }
+#pragma unroll
+          for (int x = 0; x < PL * (PL + 1) / 2; ++x) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x320, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, PL == 3 ? 8 : 16, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      cur ^= 1;
+    }
+  }
+  lines_landed<0>(); // (nothing is on its way into the rings)
+
+  // ---- the partial tiles
+  float *const sPart = reinterpret_cast<float *>(sW); // [8][64][64]: wavefront, register, lane
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        sPart[(wave * 64 + (2 * i + j) * 16 + v) * 64 + lane] =
+            NACC == 2 ? acc[0][i][j][v] + acc[NACC - 1][i][j][v] : acc[0][i][j][v];
+  ColEpilogue col[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = n0 + 32 * j + c;
+    col[j] = load_col(ep, n < N ? n : N - 1);
+  }
+  __syncthreads();
+  // register v of tile (i, j), lane (c, q), is row 32 i + 8 (v / 4) + 4 q + v % 4; this
+  // wavefront's are v = wave and wave + 8 of every tile
+  unsigned again[4];
+  float sum[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    again[e] = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int v = 8 * h + wave;
+      float x = sPart[(e * 16 + v) * 64 + lane];
+#pragma unroll
+      for (int k = 1; k < 8; ++k)
+        x += sPart[(k * 64 + e * 16 + v) * 64 + lane];
+      sum[2 * e + h] = x;
+      if (doubtful<PL>(x))
+        again[e] |= 1u << v;
+    }
+  }
+  if constexpr (PL == 3) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (__any(again[e] != 0)) {
+        const int r = 32 * (e / 2) + c;
+        const long long m = row0 + r < M ? row0 + r : M - 1;
+        const int n = n0 + 32 * (e % 2) + c < N ? n0 + 32 * (e % 2) + c : N - 1;
+        const floatx16 exact = tile_f32<GATHER>(A, gs, sRules + (GATHER ? (int)(m - row0) * gs.fs : 0), plain, m, n, K, N, again[e]);
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          if (again[e] >> v & 1)
+            sum[2 * e + v / 8] = exact[v];
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int v = 8 * h + wave;
+      const long long r = row0 + 32 * (e / 2) + 8 * (v / 4) + 4 * q + v % 4;
+      const int n = n0 + 32 * (e % 2) + c;
+      if (r < M && n < N)
+        out[r * N + n] = finish(sum[2 * e + h], col[e % 2]);
+    }
+}
+
 // Long contractions of bf16 rows through rules, one plane, with the chip full.  A wavefront
 // owns 64 rows x 32 NT columns: six LDS reads to eight MFMAs (NT 4), where a tile of rows
 // to four of columns reads five to four, all that LDS gives while the pipe is busy, and
@@ -1601,6 +1863,22 @@ static int launch_lines(scn_ctx *ctx, const float *A, const float *W, float *out
                        out, M, K, N, ep, GatherSource(), nSplits, byColumns, rows, PlainW{W, wT});
   return SCN_OK;
 }
+template <int PL, int WM>
+static int launch_split64(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int K, int N,
+                          const Epilogue &ep, const GatherSource *gs, const RowRange &rows, const unsigned char *image) {
+  const int nSplits = scn_ceil_div(N, 64);
+  const size_t lds = 128 * 1024 + (gs ? (size_t)64 * gs->fs * 4 : 0);
+  const dim3 grid((unsigned)(scn_ceil_div(M, 64) * (long long)nSplits));
+  const bool byColumns = image_larger(PL, scn_rows_hint(ctx, M), K, N, gs ? gs->nIn : K);
+  const PlainW plain = {W, WM == S64_TURNED};
+  if (!gs)
+    hipLaunchKernelGGL((k_nin_split64<PL, false, WM>), grid, dim3(512), lds, ctx->stream, A, image, out, M, K, N, ep,
+                       GatherSource(), nSplits, byColumns, rows, plain);
+  else if constexpr (WM != S64_TURNED)
+    hipLaunchKernelGGL((k_nin_split64<PL, true, WM>), grid, dim3(512), lds, ctx->stream, A, image, out, M, K, N, ep, *gs,
+                       nSplits, byColumns, rows, plain);
+  return SCN_OK;
+}
 // (nIn in 32s; an image made by the call where there is none)
 template <int NT>
 static int launch_rows16(scn_ctx *ctx, const void *A, const float *W, float *out, long long M, int K, int N,
@@ -1680,12 +1958,25 @@ static const PlanesCost planesCost[3][4][2] = {
 // planes, 512 k 2.4 11.2, 12.2, and 3.1 14.5, 12.8; 768 k 2.5 15.0, 17.0, and 3.2
 // 19.4, 17.6; 256 k 1.8 6.2, 7.7, and 2.4 8.5, 8.0; 2560 k 2.2 41.7, 45.9, and 3.1
 // 51.7, 46.5; one plane, 512 k 1.6 6.9, 7.2, and 2.0 9.3, 7.4; 256 k 1.8 5.4, 5.4.
-static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
+static long long few_rows(scn_ctx *ctx, int planes, int K, int N) {
   if (N > 1 << 26) // (a lane's place in nine rows of W has 32 bits)
     return 0;
   const float perCU = planes == 1 ? 2.f : fminf(1.f + K / 230.f, planes == 2 ? 3.1f : 2.6f);
   const long long rows = (long long)(perCU * ctx->numCU / scn_ceil_div(N, 32));
   return 32 * (rows < 1 ? 1 : rows);
+}
+// Beyond those k_nin_split64 takes it while its workgroups are no more than the compute
+// units: what one takes is its wavefronts' blocks, 2.5 us each in three planes and 1.1 in one,
+// and 5 to 7, and a second round as long again (2257 x 1920 x 640, 360 of them, 45.5 us
+// where tiles take 46, and 21.7 where they take 17.7). us, rows through rules, images made
+// before, the tiles and here: three planes, 1037 x 2560 x 800 49.5, 31.8; 2257 x 1920 x 448 37.4,
+// 26.1; 8000 x 1024 x 128 22.1, 16.4; 3000 x 768 x 320 17.3, 13.2; 5000 x 512 x 192 13.0,
+// 10.9; one plane 22.0, 15.2; 17.1, 12.1; 11.7, 9.3; 9.5, 8.3; 7.9, 7.4; W as it stands,
+// with nothing made before, 12383 x 448 x 64 14.4, 13.5, but 3909 x 256 x 160 9.7, 11.8:
+// below 448 k there is no more than a block or two to a wavefront.
+static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
+  const long long few = few_rows(ctx, planes, K, N), more = 64ll * (ctx->numCU / scn_ceil_div(N, 64));
+  return planes != 2 && K >= 448 && few > 0 && more > few ? more : few;
 }
 
 struct PlanesChoice {
@@ -1695,6 +1986,7 @@ struct PlanesChoice {
   int lines = -1; // k_nin_lines, a tile of its own: index into linesTiles
   int rows16 = 0; // k_nin_rows16, of so many tiles of columns
   const unsigned char *weights = nullptr; // the image it reads, null: to be made
+  const unsigned char *given = nullptr;   // the image there is, for the split contraction
 };
 // needImage: of the tiles, only from the image (scn_planes_abt: whether there is one)
 static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16,
@@ -1733,11 +2025,31 @@ static float lines_rows16(scn_ctx *ctx, long long M, int K, int N, bool image) {
          (image ? 0.f : 3.f + (float)K * N / 150000.f);
 }
 bool scn_planes_splitk(scn_ctx *ctx, int planes, long long M, int K, int N) {
-  return M <= split_rows(ctx, planes, K, N);
+  return M <= few_rows(ctx, planes, K, N);
+}
+
+// The split contraction, in the kernel for so many rows.  (bf16 rows: k_nin_split64 rounds
+// the fp32 ones, the same bits.)
+template <int PL>
+static int launch_split(scn_ctx *ctx, const float *A, const float *A32, const float *W, float *out, long long M, int K, int N,
+                        const Epilogue &ep, const GatherSource *gs, bool a16, bool wT, const RowRange &rows,
+                        const unsigned char *image) {
+  const long long few = few_rows(ctx, PL, K, N);
+  if constexpr (PL != 2)
+    if (split_rows(ctx, PL, K, N) > few && scn_rows_hint(ctx, M) > few) {
+      const float *const from = a16 ? A32 : A;
+      if (image)
+        return launch_split64<PL, S64_IMAGE>(ctx, from, W, out, M, K, N, ep, gs, rows, image);
+      if constexpr (PL == 3)
+        if (wT)
+          return launch_split64<PL, S64_TURNED>(ctx, from, W, out, M, K, N, ep, gs, rows, nullptr);
+      return launch_split64<PL, S64_PLAIN>(ctx, from, W, out, M, K, N, ep, gs, rows, nullptr);
+    }
+  return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
 }
 
 template <int PL>
-static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
+static int planes_forward(scn_ctx *ctx, const float *A, const float *A32, const float *W,
                           float *out, long long M, int K, int N,
                           const Epilogue &ep, const GatherSource *gs, bool a16,
                           const PlanesChoice &choice, bool wT = false) {
@@ -1747,20 +2059,23 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
     // it the guess decides, and is held against the counts when they are known.
     // A kernel launched by itself is launched for every row there may be: where
     // the guess was wrong its rows are rounded otherwise, not left out.
+    // (A launch that finds nothing to do is 4 to 5 us, a pass queued again hundreds: of the
+    // larger matrices that k_nin_split64 takes, whose batches vary less, within a fifteenth.)
     const long long split = split_rows(ctx, PL, K, N), hint = scn_rows_hint(ctx, M);
-    if (M > split && 6 * hint > 5 * split && 5 * hint < 6 * split) {
+    const int near = split > few_rows(ctx, PL, K, N) ? 15 : 5;
+    if (M > split && (near + 1) * hint > near * split && near * hint < (near + 1) * split) {
       RowRange upper = rows;
       rows.upTo = upper.above = split;
-      SCN_TRY(launch_splitk<PL>(ctx, A, W, out, split, K, N, ep, gs, a16, wT, rows));
+      SCN_TRY(launch_split<PL>(ctx, A, A32, W, out, split, K, N, ep, gs, a16, wT, rows, choice.given));
       rows = upper;
     } else if (hint <= split) {
       scn_rows_chosen(ctx, -1, split);
-      return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
+      return launch_split<PL>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, wT, rows, choice.given);
     } else {
       scn_rows_chosen(ctx, split, 1ll << 62);
     }
   } else if (choice.tile < 0) {
-    return launch_splitk<PL>(ctx, A, W, out, M, K, N, ep, gs, a16, wT, rows);
+    return launch_split<PL>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, wT, rows, choice.given);
   }
   if constexpr (PL == 1)
     switch (choice.rows16) {
@@ -1831,13 +2146,15 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *W,
 // k_nin_lines where it is the faster (the same bits): for rows that are not gathered
 // wherever it can run, as k_nin_planes' costs are too low for those.
 static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, const GatherSource *gs, const void *image,
-                          bool room, PlanesChoice &choice) {
+                          bool room, bool unlikely, PlanesChoice &choice) {
   if (!lines_shape(planes, K, N, gs ? gs->nIn : K) ||
       !(image || (room && image_bytes(planes, K, N) <= (int64_t)SCN_IMAGE_BYTES)))
     return;
   int tile = 0;
   const float cost = lines_choose(ctx->numCU, planes, M, K, N, gs != nullptr, &tile) + (image ? 0.f : 4.f);
-  if (gs && cost >= choice.cost + 2.f) // (2: what the other's leave out of a launch)
+  // (2: what the other's leave out of a launch; unlikely: for rows there probably are not, without
+  // a launch for an image where there is one)
+  if (gs && cost >= choice.cost + 2.f && !(unlikely && image))
     return;
   choice.lines = tile;
   choice.weights = (const unsigned char *)image;
@@ -1846,11 +2163,12 @@ static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, c
 int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
                        float *out, long long M, int K, int N,
                        const Epilogue &ep, const GatherSource *gs, bool a16,
-                       const void *image) {
+                       const void *image, const float *A32) {
   // (rows guessed: a tile in any case, they may be more)
   const long long split = split_rows(ctx, planes, K, N), hint = scn_rows_hint(ctx, M);
   const long long rows = M > split && hint <= split ? split + 1 : hint;
   PlanesChoice choice = planes_choose(ctx, planes, rows, K, N, a16);
+  choice.given = (const unsigned char *)image;
   const bool room = planes_image(ctx);
   choice.image = choice.image && room;
   // (bf16 rows: a block takes half a line of each; long contractions, of 27
@@ -1867,10 +2185,10 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
       choice.weights = (const unsigned char *)image;
   }
   if (choice.tile >= 0 && !a16)
-    lines_instead(ctx, planes, rows, K, N, gs, image, room, choice);
-  return planes == 3   ? planes_forward<3>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
-         : planes == 2 ? planes_forward<2>(ctx, A, W, out, M, K, N, ep, gs, a16, choice)
-                       : planes_forward<1>(ctx, A, W, out, M, K, N, ep, gs, a16, choice);
+    lines_instead(ctx, planes, rows, K, N, gs, image, room, hint <= split, choice);
+  return planes == 3   ? planes_forward<3>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice)
+         : planes == 2 ? planes_forward<2>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice)
+                       : planes_forward<1>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice);
 }
 
 // The planes of a call of that precision, 0: none that take an image
@@ -1881,9 +2199,11 @@ extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N,
   const int planes = image_planes(precision);
   if (!ctx || M < 1 || K < 1 || N < 1 || nIn < 1 || planes == 0 || N % 4 != 0 || !lines_shape(planes, K, N, nIn))
     return 0;
-  const long long hint = scn_rows_hint(ctx, M), split = split_rows(ctx, planes, K, N);
-  if (6 * hint <= 5 * split)
+  const long long hint = scn_rows_hint(ctx, M), few = few_rows(ctx, planes, K, N), split = split_rows(ctx, planes, K, N);
+  if (split > few ? hint <= few : 6 * hint <= 5 * split)
     return 0;
+  if (split > few && hint <= split) // (k_nin_split64)
+    return image_bytes(planes, K, N);
   int tile;
   const PlanesChoice choice = planes_choose(ctx, planes, hint > split ? hint : split + 1, K, N, false);
   if (nIn != K && lines_choose(ctx->numCU, planes, hint, K, N, true, &tile) >= choice.cost + 2.f)
@@ -1955,12 +2275,12 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
   PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
   const bool room = planes_image(ctx);
   if (choice.tile >= 0)
-    lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, choice);
+    lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, false, choice);
   if (choice.tile >= 0 && choice.lines < 0) {
     *transpose = choice.image;
     return false;
   }
-  *rc = planes_forward<3>(ctx, A, Wt, out, M, K, N, ep, nullptr, false, choice, true);
+  *rc = planes_forward<3>(ctx, A, A, Wt, out, M, K, N, ep, nullptr, false, choice, true);
   return true;
 }
 
