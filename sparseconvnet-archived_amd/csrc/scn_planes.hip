@@ -1988,9 +1988,10 @@ struct PlanesChoice {
   const unsigned char *weights = nullptr; // the image it reads, null: to be made
   const unsigned char *given = nullptr;   // the image there is, for the split contraction
 };
-// needImage: of the tiles, only from the image (scn_planes_abt: whether there is one)
-static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16,
-                                   bool needImage = false) {
+// images: of the tiles only those from the image (scn_planes_abt: whether there is one), or
+// only the others
+enum { TILES_ALL, TILES_IMAGE, TILES_CONVERT };
+static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, int N, bool a16, int images = TILES_ALL) {
   if (M <= split_rows(ctx, planes, K, N))
     return {-1, false, 0.f};
   const int T = K / 32;
@@ -2002,7 +2003,7 @@ static PlanesChoice planes_choose(scn_ctx *ctx, int planes, long long M, int K, 
     const float wgs = (float)(scn_ceil_div(M, 128 * mt) * nSplits) / ctx->numCU;
     const float n = wgs <= 4.f ? ceilf(wgs) : wgs + .5f;
     const int units = 4 * mt * nt;
-    for (int img = needImage; img < 2; ++img) {
+    for (int img = images == TILES_IMAGE; img < (images == TILES_CONVERT ? 1 : 2); ++img) {
       if (img && (size_t)nSplits * T * planes * 2 * nt * 1024 > SCN_IMAGE_BYTES)
         continue;
       const PlanesCost &c = planesCost[planes > 1 ? 2 : a16][i][img];
@@ -2097,6 +2098,7 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *A32, const 
       SCN_LINES_CASE(3, 1, 2, 2, 2, 4)
       SCN_LINES_CASE(4, 1, 1, 2, 2, 3)
       SCN_LINES_CASE(5, 1, 1, 2, 2, 6)
+      SCN_LINES_CASE(LINES_NARROW, 1, 1, 4, 1, 3)
     }
   } else if constexpr (PL == 1) {
     switch (choice.lines) {
@@ -2146,16 +2148,26 @@ static int planes_forward(scn_ctx *ctx, const float *A, const float *A32, const 
 // k_nin_lines where it is the faster (the same bits): for rows that are not gathered
 // wherever it can run, as k_nin_planes' costs are too low for those.
 static void lines_instead(scn_ctx *ctx, int planes, long long M, int K, int N, const GatherSource *gs, const void *image,
-                          bool room, bool unlikely, PlanesChoice &choice) {
+                          bool room, bool unlikely, bool wT, PlanesChoice &choice) {
   if (!lines_shape(planes, K, N, gs ? gs->nIn : K) ||
       !(image || (room && image_bytes(planes, K, N) <= (int64_t)SCN_IMAGE_BYTES)))
     return;
+  // Plain rows of up to four tiles of 32 x 32 to a compute unit, in three planes: what
+  // the image's launch takes is a third of all. us, from an image made by the call and converted on the
+  // way, 5760 x 256 x 160 13.6, 9.9; 10474 x 256 x 96 13.6, 9.7; 9307 x 128 x 64 9.3, 7.1; 3810 x 544 x 256 16.8, 14.7;
+  // at 4.3 to a unit 11818 x 224 x 96 12.9, 12.7, at 4.8 4872 x 608 x 256 20.1, 25.1.
+  if (!gs && !image && !wT && planes == 3 && tiles_of(M, 32) * tiles_of(N, 32) <= 4ll * ctx->numCU) {
+    choice = planes_choose(ctx, 3, M, K, N, false, TILES_CONVERT);
+    return;
+  }
   int tile = 0;
   const float cost = lines_choose(ctx->numCU, planes, M, K, N, gs != nullptr, &tile) + (image ? 0.f : 4.f);
   // (2: what the other's leave out of a launch; unlikely: for rows there probably are not, without
   // a launch for an image where there is one)
   if (gs && cost >= choice.cost + 2.f && !(unlikely && image))
     return;
+  if (!gs && planes == 3 && N <= 32) // (gathered rows of one tile of columns are k_nin_planes')
+    tile = LINES_NARROW;
   choice.lines = tile;
   choice.weights = (const unsigned char *)image;
 }
@@ -2185,7 +2197,7 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
       choice.weights = (const unsigned char *)image;
   }
   if (choice.tile >= 0 && !a16)
-    lines_instead(ctx, planes, rows, K, N, gs, image, room, hint <= split, choice);
+    lines_instead(ctx, planes, rows, K, N, gs, image, room, hint <= split, false, choice);
   return planes == 3   ? planes_forward<3>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice)
          : planes == 2 ? planes_forward<2>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice)
                        : planes_forward<1>(ctx, A, A32, W, out, M, K, N, ep, gs, a16, choice);
@@ -2272,10 +2284,10 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
   *transpose = false;
   if (!scn_planes_shape(K) || ((uintptr_t)A & 15) || ((uintptr_t)out & 15) || N % 4 != 0)
     return false;
-  PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, true);
+  PlanesChoice choice = planes_choose(ctx, 3, M, K, N, false, TILES_IMAGE);
   const bool room = planes_image(ctx);
   if (choice.tile >= 0)
-    lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, false, choice);
+    lines_instead(ctx, 3, M, K, N, nullptr, nullptr, room, false, true, choice);
   if (choice.tile >= 0 && choice.lines < 0) {
     *transpose = choice.image;
     return false;

@@ -34,6 +34,10 @@ static const LinesTile linesTiles[2][6] = {
     {{1, 2, 4, 2, 3, 2, 1.9f, .53f, .92f, 0.f, 0.f, 0.f}, {1, 2, 2, 2, 4, 2, 3.f, .22f, .38f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 3, 4, 1.9f, .36f, .58f, 0.f, 0.f, 0.f}}, // one plane
     {{1, 2, 4, 2, 3, 1, 4.1f, 1.04f, 0.f, 2.5f, 2.1f, 1.12f}, {2, 1, 4, 2, 3, 1, 4.3f, 1.25f, 0.f, 1.6f, 3.f, 1.3f}, {1, 3, 4, 1, 4, 1, 4.5f, .87f, 0.f, 0.f, 0.f, 0.f},
      {1, 2, 2, 2, 4, 1, 3.4f, .68f, 0.f, 3.1f, 1.45f, .71f}, {1, 1, 2, 2, 3, 2, 2.f, .58f, .85f, 0.f, 0.f, 0.f}, {1, 1, 2, 2, 6, 1, 2.f, .5f, 0.f, 0.f, 0.f, 0.f}}};
+// (One more of three planes, for plain rows of one tile of columns, which the others give 64:
+// 128 x 32, two of which share a compute unit.  With the image us, 64 x 64 and this, 123606 x 768 x 32 97,
+// 87; 174344 x 1728 x 32 277, 237; 43000 x 256 x 32 18.6, 15.4; 300000 x 128 x 32 46, 38.)
+constexpr int LINES_NARROW = 6;
 // How many workgroups an XCD has of a LONG launch, a multiple of the slices of columns
 // (0: a launch of a workgroup a tile): plain rows of no less than their weights, in three
 // planes, of no more than 512 k, where a compute unit that has room for one workgroup has
