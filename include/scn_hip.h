@@ -355,6 +355,13 @@ int scn_terminal_classifier(scn_ctx *ctx, const float *d_in,
                             float *d_pooled, const float *d_W,
                             const float *d_B, float *d_probs, float *copy,
                             int K, int N, float p);
+/* The same for a training batch: with scn_softmax_grad's d_delta [M x N] by d_labels. */
+int scn_terminal_classifier_train(scn_ctx *ctx, const float *d_in,
+                                  const int32_t *d_rules, int64_t M, int S,
+                                  float *d_pooled, const float *d_W,
+                                  const float *d_B, float *d_probs, float *copy,
+                                  int K, int N, float p,
+                                  const int32_t *d_labels, float *d_delta);
 /* dSigmoidSoftmax (SigmoidLayer.cu:160-177). */
 int scn_softmax_rows(scn_ctx *ctx, const float *d_in, float *d_out, int64_t M,
                      int N);
@@ -618,6 +625,17 @@ int scn_maxpool_backward_through(scn_ctx *ctx, float *d_din, const float *d_dout
 int scn_terminal_pool_backward(scn_ctx *ctx, float *d_din, const float *d_dout,
                                const int32_t *d_rules, int64_t count, int C,
                                int S);
+/* A net's end backwards, in one launch: scn_sgemm_ABt of the classifier's d_delta [M
+ * x N] and d_W [K x N] into d_dpooled [M x K], scn_terminal_pool_backward of that into
+ * d_din (which the caller zeroes), and the derivative of the activation `act` that
+ * made the rows pooled, d_features, taken in the rows listed; for SCN_PRELU the
+ * slopes' gradient is added to d_dprelu.  (The bias gradient is d_din's column
+ * sums: scn_sgemm_AtB_sums.)  K up to 1024 and N up to 128, multiples of 4. */
+int scn_terminal_gradient_supported(int K, int N);
+int scn_terminal_gradient(scn_ctx *ctx, const float *d_delta, const float *d_W,
+                          float *d_dpooled, const int32_t *d_rules, int64_t M,
+                          int S, float *d_din, const float *d_features, int act,
+                          const float *d_prelu, float *d_dprelu, int K, int N);
 
 /* ---- per-kernel timing -------------------------------------------------- */
 /* HIP events recorded on the context's stream around every kernel of one

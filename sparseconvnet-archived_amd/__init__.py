@@ -155,6 +155,10 @@ def lib():
         "scn_terminal_pool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
         "scn_terminal_classifier_supported": (C.c_int, [i64, C.c_int, C.c_int]),
         "scn_terminal_classifier": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float]),
+        "scn_terminal_classifier_train": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float,
+                                                    vp, vp]),
+        "scn_terminal_gradient_supported": (C.c_int, [C.c_int, C.c_int]),
+        "scn_terminal_gradient": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, vp, vp, C.c_int, vp, vp, C.c_int, C.c_int]),
         "scn_softmax_rows": (C.c_int, [vp, vp, vp, i64, C.c_int]),
         "scn_softmax_grad": (C.c_int, [vp, vp, vp, vp, i64, C.c_int]),
         "scn_activation_backward": (C.c_int, [vp, vp, vp, i64, C.c_int, C.c_int, vp, vp, vp]),
@@ -369,6 +373,16 @@ class Context:
     def terminal_classifier(self, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, p=1.0):
         _check(lib().scn_terminal_classifier(self.h, d_in.ptr, d_rules.ptr, M, S, d_pooled.ptr, d_W.ptr, d_B.ptr,
                                              d_probs.ptr, copy.ptr if copy is not None else None, K, N, p))
+
+    def terminal_classifier_train(self, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, d_labels, d_delta, p=1.0):
+        _check(lib().scn_terminal_classifier_train(self.h, d_in.ptr, d_rules.ptr, M, S, d_pooled.ptr, d_W.ptr, d_B.ptr,
+                                                   d_probs.ptr, copy.ptr if copy is not None else None, K, N, p, d_labels.ptr,
+                                                   d_delta.ptr))
+
+    def terminal_gradient(self, d_delta, d_W, d_dpooled, d_rules, M, S, d_din, d_features, act, d_prelu, d_dprelu, K, N):
+        _check(lib().scn_terminal_gradient(self.h, d_delta.ptr, d_W.ptr, d_dpooled.ptr, d_rules.ptr, M, S, d_din.ptr,
+                                           d_features.ptr, act, d_prelu.ptr if d_prelu is not None else None,
+                                           d_dprelu.ptr if d_dprelu is not None else None, K, N))
 
     def softmax_rows(self, d_in, d_out, M, N):
         _check(lib().scn_softmax_rows(self.h, d_in.ptr, d_out.ptr, M, N))

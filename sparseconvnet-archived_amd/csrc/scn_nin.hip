@@ -292,6 +292,8 @@ struct TerminalSource {
   const long long *meta;
   float *pooled; // [M x K]
   float *copy;   // [M x N], or null
+  const int *labels; // a training batch's, and the gradient of its cost by the soft-max's input
+  float *delta;      // [M x N], or null
 };
 template <bool TERMINAL>
 __global__ void __launch_bounds__(FR_THREADS)
@@ -413,6 +415,7 @@ __global__ void __launch_bounds__(FR_THREADS)
   const long long m = m0 + wave;
   if (wave >= CL_ROWS || m >= M)
     return;
+  const int label = TERMINAL && ts.delta ? ts.labels[m] : 0;
   float z[2], mx = -10000.0f;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -445,6 +448,8 @@ __global__ void __launch_bounds__(FR_THREADS)
       out[m * N + 64 * j + lane] = y;
       if (TERMINAL && ts.copy)
         ts.copy[m * N + 64 * j + lane] = y;
+      if (TERMINAL && ts.delta)
+        ts.delta[m * N + 64 * j + lane] = y - (64 * j + lane == label ? 1.f : 0.f);
     }
 }
 
@@ -2188,9 +2193,9 @@ extern "C" int scn_terminal_classifier_supported(int64_t M, int K, int N) {
   return M >= 1 && M <= FR_MAX_M && K >= 1 && K <= FR_MAX_K && N >= 1 && N <= 128 && K % 4 == 0 && N % 4 == 0 &&
          !(N % 16 == 0 && scn_planes_shape(K));
 }
-extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
-                                       float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
-                                       float *copy, int K, int N, float p) {
+static int terminal_classifier(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S, float *d_pooled,
+                               const float *d_W, const float *d_B, float *d_probs, float *copy, int K, int N, float p,
+                               const int32_t *d_labels, float *d_delta) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_terminal_classifier: null context");
   SCN_REQUIRE(S >= 1 && scn_terminal_classifier_supported(M, K, N), SCN_ERR_ARG,
               "scn_terminal_classifier: M %lld S %d K %d N %d", (long long)M, S, K, N);
@@ -2203,9 +2208,22 @@ extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const in
   ep.p = p;
   ep.act = SCN_SOFTMAX;
   ProfScope prof(ctx, SCN_K_NET_END);
-  TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy};
+  TerminalSource ts = {d_rules, S, ctx->d_meta, d_pooled, copy, d_labels, d_delta};
   hipLaunchKernelGGL((k_classifier<true>), dim3(scn_ceil_div(M, CL_ROWS)), dim3(FR_THREADS), 0, ctx->stream, d_in, d_W,
                      d_probs, (long long)M, K, N, ep, ctx->d_meta ? ctx->d_meta + META_SITES : nullptr, ts);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
+}
+extern "C" int scn_terminal_classifier(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
+                                       float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
+                                       float *copy, int K, int N, float p) {
+  return terminal_classifier(ctx, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, p, nullptr, nullptr);
+}
+// (a training batch of 100 drawings: pooling, classifier and the gradient 4.6 + 5.0 + 4.2 us -> 7.3)
+extern "C" int scn_terminal_classifier_train(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int64_t M, int S,
+                                             float *d_pooled, const float *d_W, const float *d_B, float *d_probs,
+                                             float *copy, int K, int N, float p, const int32_t *d_labels,
+                                             float *d_delta) {
+  SCN_REQUIRE(d_labels && d_delta, SCN_ERR_ARG, "scn_terminal_classifier_train: null buffer");
+  return terminal_classifier(ctx, d_in, d_rules, M, S, d_pooled, d_W, d_B, d_probs, copy, K, N, p, d_labels, d_delta);
 }

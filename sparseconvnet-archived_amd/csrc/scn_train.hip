@@ -1795,6 +1795,186 @@ extern "C" int scn_terminal_pool_backward(scn_ctx *ctx, float *d_din,
   return SCN_OK;
 }
 
+// The backward pass of a net's end in one launch: the classifier's d input = D W^T,
+// spread by the terminal pooling over its rows, times the derivative of the activation
+// that made them, with the sums of a PReLU's slopes.  Every launch of such a batch is 4
+// us whatever it holds (100 drawings: W transposed 2.7, the product 5.5, spread 3.6,
+// derivative 6.0 us and a gap each -> 7.3).  A workgroup has two samples, as k_classifier;
+// 32 lanes take a row of W, its products with both are summed across them.  Then a lane
+// has four channels of a sample: its rows four at a time.  Code that is run once is
+// fetched by every compute unit, which is most of what is left: with the derivative's
+// cases and eight rows laid out one after the other it took 10 to 14 us.
+#define TG_ROWS 2
+#define TG_THREADS 512
+#define TG_DEPTH 12
+#define TG_MAX_K 1024
+#define TG_MAX_N 128
+struct TerminalGradient {
+  const float *delta, *W; // [M x N], [K x N]
+  float *dpooled;         // [M x K]
+  const int *rules;       // [M x S]
+  float *din;
+  const float *features; // of the rows that are pooled
+  const float *prelu;
+  float *dprelu;
+  long long M;
+  int S, K, N, act;
+};
+// the sum over 32 lanes, in all of them
+__device__ __forceinline__ float sum32(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));  // 1 0 3 2
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));  // 2 3 0 1
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)); // eight turned round
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true)); // sixteen
+  return v + __shfl_xor(v, 16, 64);
+}
+__global__ __launch_bounds__(TG_THREADS) void k_terminal_gradient(TerminalGradient g) {
+  __shared__ __attribute__((aligned(16))) float sD[TG_ROWS][TG_MAX_N], sT[TG_ROWS][TG_MAX_K];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long long m0 = (long long)blockIdx.x * TG_ROWS;
+  const int K = g.K, N = g.N, S = g.S;
+  static_assert(TG_THREADS == TG_ROWS * TG_MAX_K / 4, "a lane four channels");
+  const int row = tid / (TG_MAX_K / 4), k = 4 * (tid % (TG_MAX_K / 4));
+  const long long m = m0 + row;
+  constexpr int RULES = 4; // at a time
+  int rule[RULES];
+  auto load_rules = [&](int p0) {
+#pragma unroll
+    for (int u = 0; u < RULES; ++u)
+      rule[u] = m < g.M && p0 + u < S ? g.rules[m * S + p0 + u] : -1;
+  };
+  load_rules(0);
+  if (tid < TG_ROWS * TG_MAX_N) {
+    const int r = tid / TG_MAX_N, j = tid % TG_MAX_N;
+    sD[r][j] = m0 + r < g.M && j < N ? g.delta[(m0 + r) * N + j] : 0.f;
+  }
+  // rows of W: two a wavefront and load, sixteen a workgroup
+  const int j4 = 4 * (lane & 31), c0 = 2 * wave + (lane >> 5);
+  const float *const w = g.W + (j4 < N ? j4 : 0); // (past the end: times zero)
+  float4 wv[TG_DEPTH];
+  auto load_w = [&](int from) {
+#pragma unroll
+    for (int i = 0; i < TG_DEPTH; ++i) {
+      const int c = from + 16 * i < K ? from + 16 * i : K - 1; // (not stored)
+      wv[i] = *reinterpret_cast<const float4 *>(w + (long long)c * N);
+    }
+  };
+  load_w(c0);
+  __syncthreads();
+  float4 d[TG_ROWS];
+#pragma unroll
+  for (int r = 0; r < TG_ROWS; ++r)
+    d[r] = j4 < N ? *reinterpret_cast<const float4 *>(&sD[r][j4]) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+  for (int from = c0;; from += 16 * TG_DEPTH) {
+    float t[TG_ROWS][TG_DEPTH];
+#pragma unroll
+    for (int i = 0; i < TG_DEPTH; ++i)
+#pragma unroll
+      for (int r = 0; r < TG_ROWS; ++r)
+        t[r][i] = j4 < N ? fmaf(wv[i].x, d[r].x, wv[i].y * d[r].y) + fmaf(wv[i].z, d[r].z, wv[i].w * d[r].w) : 0.f;
+    const bool more = from - c0 + 16 * TG_DEPTH < K; // uniform
+    if (more)
+      load_w(from + 16 * TG_DEPTH);
+#pragma unroll
+    for (int i = 0; i < TG_DEPTH; ++i)
+#pragma unroll
+      for (int r = 0; r < TG_ROWS; ++r) {
+        t[r][i] = sum32(t[r][i]);
+        if ((lane & 31) == 0 && from + 16 * i < K)
+          sT[r][from + 16 * i] = t[r][i];
+      }
+    if (!more)
+      break;
+  }
+  __syncthreads();
+  float slope[4] = {0.f, 0.f, 0.f, 0.f};
+  if (m < g.M && k < K) {
+    const float4 t4 = *reinterpret_cast<const float4 *>(&sT[row][k]);
+    *reinterpret_cast<float4 *>(g.dpooled + m * K + k) = t4;
+    // the rows up to the first negative rule
+    int count = 0;
+    bool more = true;
+#pragma unroll 1
+    for (int p0 = 0; p0 < S && more; p0 += RULES) {
+      if (p0)
+        load_rules(p0);
+#pragma unroll
+      for (int u = 0; u < RULES; ++u) {
+        more = more && rule[u] >= 0;
+        count += more;
+      }
+    }
+    const bool curved = g.act == SCN_TANH || g.act == SCN_SIGMOID;
+    float t[4] = {t4.x / (float)count, t4.y / (float)count, t4.z / (float)count, t4.w / (float)count}, neg[4], alpha[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { // (as act_derivative)
+      alpha[i] = g.act == SCN_PRELU ? g.prelu[k + i] : g.act == SCN_LEAKYRELU ? 0.01f : 0.333f;
+      neg[i] = g.act == SCN_RELU ? 0.f : g.act == SCN_NOSIGMOID || g.act == SCN_SOFTMAX ? t[i] : t[i] * alpha[i];
+    }
+#pragma unroll 1
+    for (int p0 = 0; p0 < count; p0 += RULES) {
+      if (S > RULES)
+        load_rules(p0);
+      float4 y[RULES];
+#pragma unroll
+      for (int u = 0; u < RULES; ++u) // (past the last: that one again)
+        y[u] = *reinterpret_cast<const float4 *>(g.features + (long long)(p0 + u < count ? rule[u] : rule[0]) * K + k);
+#pragma unroll
+      for (int u = 0; u < RULES; ++u) {
+        const float v[4] = {y[u].x, y[u].y, y[u].z, y[u].w};
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          r[i] = v[i] > 0 ? t[i] : neg[i];
+        if (curved) { // uniform
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            r[i] = g.act == SCN_TANH ? t[i] * (1 + v[i]) * (1 - v[i]) : t[i] * v[i] * (1 - v[i]);
+        }
+        if (p0 + u < count) {
+          *reinterpret_cast<float4 *>(g.din + (long long)rule[u] * K + k) = make_float4(r[0], r[1], r[2], r[3]);
+          if (g.act == SCN_PRELU) // uniform
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              slope[i] += v[i] > 0 ? 0.f : t[i] * (v[i] / alpha[i]);
+        }
+      }
+    }
+  }
+  if (g.act != SCN_PRELU) // uniform
+    return;
+  __syncthreads(); // (sT has been read)
+  if (k < K)
+    *reinterpret_cast<float4 *>(&sT[row][k]) = make_float4(slope[0], slope[1], slope[2], slope[3]);
+  __syncthreads();
+  for (int c = tid; c < K; c += TG_THREADS)
+    unsafeAtomicAdd(g.dprelu + c, sT[0][c] + sT[1][c]);
+}
+extern "C" int scn_terminal_gradient_supported(int K, int N) {
+  return K >= 4 && K <= TG_MAX_K && K % 4 == 0 && N >= 4 && N <= TG_MAX_N && N % 4 == 0;
+}
+extern "C" int scn_terminal_gradient(scn_ctx *ctx, const float *d_delta, const float *d_W, float *d_dpooled,
+                                     const int32_t *d_rules, int64_t M, int S, float *d_din, const float *d_features,
+                                     int act, const float *d_prelu, float *d_dprelu, int K, int N) {
+  SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_terminal_gradient: null context");
+  SCN_REQUIRE(M >= 0 && S >= 1 && scn_terminal_gradient_supported(K, N) && act >= SCN_NOSIGMOID && act <= SCN_SIGMOID,
+              SCN_ERR_ARG, "scn_terminal_gradient: M %lld S %d K %d N %d activation %d", (long long)M, S, K, N, act);
+  if (M == 0)
+    return SCN_OK;
+  SCN_REQUIRE(scn_ceil_div(M, TG_ROWS) <= 0x7fffffffll, SCN_ERR_CAPACITY, "scn_terminal_gradient: %lld samples", (long long)M);
+  // (d_din and d_features may be null: no rows, every rule negative)
+  SCN_REQUIRE(d_delta && d_W && d_dpooled && d_rules && (act != SCN_PRELU || (d_prelu && d_dprelu)), SCN_ERR_ARG,
+              "scn_terminal_gradient: null buffer");
+  SCN_REQUIRE((((uintptr_t)d_W | (uintptr_t)d_dpooled | (uintptr_t)d_din | (uintptr_t)d_features) & 15) == 0, SCN_ERR_ARG,
+              "scn_terminal_gradient: matrices start on 16 bytes");
+  ProfScope prof(ctx, SCN_K_BACKWARD);
+  const TerminalGradient g = {d_delta, d_W, d_dpooled, d_rules, d_din, d_features, d_prelu, d_dprelu, M, S, K, N, act};
+  hipLaunchKernelGGL(k_terminal_gradient, dim3((unsigned)scn_ceil_div(M, TG_ROWS)), dim3(TG_THREADS), 0, ctx->stream, g);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 // ------------------------------------------------ dropout during training
 // A training batch keeps a random subset of every layer's features
 // (featuresPresent); the layer then works on the sub-matrix of its weights

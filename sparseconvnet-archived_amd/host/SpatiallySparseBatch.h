@@ -14,6 +14,7 @@ struct BatchResultStage {
   float *pinned;
   size_t capacity; // floats
   bool copied; // the forward pass has left the probabilities in `pinned` already
+  bool graded = false; // ... and a training batch's gradient of the cost by the soft-max's input
   scn_event *arrived;
   bool pending;
   // a training batch: the point of the net's stream behind the backward pass,

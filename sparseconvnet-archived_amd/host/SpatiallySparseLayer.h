@@ -53,6 +53,14 @@ public:
   // The derivative of this layer's activation (and the sums that go with it) over
   // the outputs of a pooling that chooses from this layer's: `pooled` gets what the
   // pooling is to spread.  Nothing, where the layer has to do that itself.
+  // The layer's activation, whose derivative the gradient of the terminal pooling
+  // behind it takes, with a PReLU's slopes and the sums for them, cleared.  False:
+  // not here.
+  virtual bool activationUnder(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                               SpatiallySparseBatchInterface &output, int &act, const float *&slopes, float *&sums) {
+    (void)batch, (void)input, (void)output, (void)act, (void)slopes, (void)sums;
+    return false;
+  }
   virtual void activationAhead(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &output,
@@ -193,6 +201,8 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  bool activationUnder(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                       SpatiallySparseBatchInterface &output, int &act, const float *&slopes, float *&sums);
   void weightImages(SpatiallySparseBatch &batch,
                     SpatiallySparseBatchInterface &input,
                     SpatiallySparseBatchInterface &output,
@@ -245,6 +255,8 @@ public:
                        SpatiallySparseBatchInterface &input,
                        SpatiallySparseBatchInterface &output,
                        SpatiallySparseBatchInterface &pooled);
+  bool activationUnder(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                       SpatiallySparseBatchInterface &output, int &act, const float *&slopes, float *&sums);
   void weightImages(SpatiallySparseBatch &batch,
                     SpatiallySparseBatchInterface &input,
                     SpatiallySparseBatchInterface &output,
@@ -411,6 +423,18 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
                                cudaMemStream &ms, int last);
+// ... and backwards, with the derivative of the layer under the pooling: false: not
+// of that kind, nothing done
+bool backwardTerminalClassifier(SpatiallySparseBatch &batch,
+                                SpatiallySparseLayer *under,
+                                SpatiallySparseLayer *pooling,
+                                SpatiallySparseLayer *classifier,
+                                SpatiallySparseBatchInterface &below,
+                                SpatiallySparseBatchInterface &input,
+                                SpatiallySparseBatchInterface &middle,
+                                SpatiallySparseBatchInterface &output,
+                                cudaMemStream &ms, float learningRate,
+                                float momentum);
 
 // utilities.h
 int ipow(int base, int exp);

@@ -639,6 +639,29 @@ void NetworkInNetworkLayer::activationAhead(
     nin_activation_ahead(memStream, input, output, pooled, (int)fn, nullptr, dw,
                          db, nullptr, gradsClean);
 }
+bool NetworkInNetworkLayer::activationUnder(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                                            SpatiallySparseBatchInterface &output, int &act, const float *&slopes,
+                                            float *&sums) {
+  if (nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    return false;
+  act = (int)fn;
+  slopes = sums = nullptr;
+  output.activationDone = true;
+  return true;
+}
+bool NetworkInNetworkPReLULayer::activationUnder(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
+                                                 SpatiallySparseBatchInterface &output, int &act, const float *&slopes,
+                                                 float *&sums) {
+  if (nin_shrunk(batch, nFeaturesIn, nFeaturesOut, input, output))
+    return false;
+  if (!nin_gradients(dw, db, &dprelu, nFeaturesIn, nFeaturesOut, gradsClean))
+    dprelu.setZero(memStream);
+  act = PRELU;
+  slopes = PReLU.dPtr();
+  sums = dprelu.dPtr();
+  output.activationDone = true;
+  return true;
+}
 void NetworkInNetworkLayer::weightImages(SpatiallySparseBatch &batch, SpatiallySparseBatchInterface &input,
                                          SpatiallySparseBatchInterface &output,
                                          const SpatiallySparseBatchInterface *before,
@@ -1194,9 +1217,14 @@ static void result_room(BatchResultStage &r, size_t n, cudaMemStream &memStream)
   SCN_CHECKED(scn_host_alloc(memStream.ctx, r.capacity * sizeof(float),
                              (void **)&r.pinned));
 }
+// (a batch that did not come from a BatchProducer has its labels on the host still)
+static void keep_labels(SpatiallySparseBatch &batch) {
+  if (batch.type != UNLABELEDBATCH && (int)batch.result->labels.size() != batch.batchSize)
+    batch.result->labels = batch.labels.hVector();
+}
 // A net's end, a terminal pooling and the classifier, in one launch that also
-// leaves the probabilities where the host reads them.  False: not of that kind,
-// nothing done.
+// leaves the probabilities where the host reads them, and a training batch's
+// gradient.  False: not of that kind, nothing done.
 bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseLayer *pooling,
                                SpatiallySparseLayer *classifier,
@@ -1205,8 +1233,10 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &output,
                                cudaMemStream &ms, int last) {
   auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
-  if (batch.type == TRAINBATCH || batch.type == RESCALEBATCH || !n ||
-      n->fn != SOFTMAX ||
+  const bool train = batch.type == TRAINBATCH;
+  if (batch.type == RESCALEBATCH || !n || n->fn != SOFTMAX ||
+      (train && (n->dropout > 0 || (int)middle.featuresPresent.size() != n->nFeaturesIn ||
+                 (int)output.featuresPresent.size() != n->nFeaturesOut)) ||
       !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
       middle.nSpatialSites != batch.batchSize ||
       !scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn,
@@ -1219,14 +1249,63 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   output.sub->features.resize64(M * N, kBoundRows * N);
   result_room(*batch.result, M * N, ms);
   scn_prof_tag(ms.ctx, last);
-  SCN_CHECKED(scn_terminal_classifier(
-      ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
-      (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
-      n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
-      (int)N, 1.0f - n->dropout));
+  if (train) {
+    keep_labels(batch);
+    output.sub->dfeatures.resize64(M * N);
+    SCN_CHECKED(scn_terminal_classifier_train(
+        ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
+        (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
+        n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
+        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr()));
+  } else {
+    SCN_CHECKED(scn_terminal_classifier(
+        ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
+        (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
+        n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
+        (int)N, 1.0f - n->dropout));
+  }
   batch.result->copied = true;
+  batch.result->graded = train;
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)M * K * N);
+  return true;
+}
+
+// The other way: the classifier's gradients, and its input's spread over the rows
+// that were pooled with the derivative of what made them taken, in one launch.
+bool backwardTerminalClassifier(SpatiallySparseBatch &batch,
+                                SpatiallySparseLayer *under,
+                                SpatiallySparseLayer *pooling,
+                                SpatiallySparseLayer *classifier,
+                                SpatiallySparseBatchInterface &below,
+                                SpatiallySparseBatchInterface &input,
+                                SpatiallySparseBatchInterface &middle,
+                                SpatiallySparseBatchInterface &output,
+                                cudaMemStream &ms, float learningRate,
+                                float momentum) {
+  auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
+  if (!n || n->fn != SOFTMAX || n->dropout > 0 || !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
+      middle.nSpatialSites != batch.batchSize || (int)middle.featuresPresent.size() != n->nFeaturesIn ||
+      (int)output.featuresPresent.size() != n->nFeaturesOut || !middle.backpropErrors || !input.backpropErrors ||
+      input.sub->features.size64() != (size_t)input.nSpatialSites * n->nFeaturesIn ||
+      !scn_terminal_gradient_supported(n->nFeaturesIn, n->nFeaturesOut))
+    return false;
+  int act = 0;
+  const float *slopes = nullptr;
+  float *sums = nullptr;
+  if (!under->activationUnder(batch, below, input, act, slopes, sums))
+    return false;
+  const int64_t M = batch.batchSize;
+  const int K = n->nFeaturesIn, N = n->nFeaturesOut;
+  middle.backpropErrors = false; // (the gradient of its input comes with the pooling's)
+  n->backwards(batch, middle, output, learningRate, momentum);
+  middle.backpropErrors = true;
+  addMultiplyAdds((__int128_t)M * K * N);
+  middle.sub->dfeatures.resize64((size_t)M * K);
+  clear_gradient(ms, input, (size_t)K);
+  SCN_CHECKED(scn_terminal_gradient(
+      ms.ctx, output.sub->dfeatures.dPtr(), n->W.dPtr(), middle.sub->dfeatures.dPtr(), middle.rules.dPtr(), M,
+      (int)(middle.rules.size64() / M), input.sub->dfeatures.dPtr(), input.sub->features.dPtr(), act, slopes, sums, K, N));
   return true;
 }
 
@@ -1240,24 +1319,21 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
                              cudaMemStream &memStream) {
   assert(batch.batchSize == input.nSpatialSites);
   assert(input.nFeatures == (int)input.featuresPresent.size());
-  // (a batch that did not come from a BatchProducer has its labels on the host still)
-  if (batch.type != UNLABELEDBATCH &&
-      (int)batch.result->labels.size() != batch.batchSize)
-    batch.result->labels = batch.labels.hVector();
-  if (batch.type == TRAINBATCH) {
+  keep_labels(batch);
+  BatchResultStage &r = *batch.result;
+  if (batch.type == TRAINBATCH && !r.graded) {
     // the backward pass starts here: d cost / d soft-max input
     // (SoftmaxClassifier.cu:22-31)
     input.sub->dfeatures.resize64((size_t)input.nSpatialSites *
                                   input.nFeatures);
   }
-  BatchResultStage &r = *batch.result;
   const size_t n = (size_t)batch.batchSize * input.nFeatures;
   result_room(r, n, memStream);
   const bool small = n <= ((size_t)1 << 18), along = batch.type == TRAINBATCH && small && !r.copied;
   if (along) // (the gradient's kernel reads them anyway)
     SCN_CHECKED(scn_softmax_grad_copy(memStream.ctx, input.sub->features.dPtr(), batch.labels.dPtr(),
                                       input.sub->dfeatures.dPtr(), batch.batchSize, input.nFeatures, r.pinned));
-  else if (batch.type == TRAINBATCH)
+  else if (batch.type == TRAINBATCH && !r.graded)
     SCN_CHECKED(scn_softmax_grad(memStream.ctx, input.sub->features.dPtr(),
                                  batch.labels.dPtr(),
                                  input.sub->dfeatures.dPtr(), batch.batchSize,

@@ -489,6 +489,13 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
   batch.collectUpdates = true;
   for (int i = (int)layers.size() - 1; i >= 0; i--) {
     scn_prof_tag(memStream.ctx, i);
+    if (i >= 2 && i + 1 == (int)layers.size() &&
+        backwardTerminalClassifier(batch, layers[i - 2], layers[i - 1], layers[i], batch.interfaces[i - 2],
+                                   batch.interfaces[i - 1], batch.interfaces[i], batch.interfaces[i + 1], memStream,
+                                   learningRate, momentum)) {
+      --i; // (the pooling, too)
+      continue;
+    }
     if (i > 0 && layers[i]->choosesInputs())
       layers[i - 1]->activationAhead(batch, batch.interfaces[i - 1],
                                      batch.interfaces[i], batch.interfaces[i + 1]);
@@ -588,7 +595,7 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   // a RESCALEBATCH rescales every layer's weights right after its forward
   // pass (SparseConvNetCUDA.cu:230-241)
   float scalingUnderneath = 1;
-  batch.result->copied = false;
+  batch.result->copied = batch.result->graded = false;
   for (size_t i = 0; i < layers.size(); i++) {
     batch.interfaces[i + 1].sub->reset();
     scn_prof_tag(ms.ctx, (int)i);
