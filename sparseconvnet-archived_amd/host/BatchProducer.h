@@ -1,6 +1,6 @@
 // Builds batches for processDataset (BatchProducer.h:8-25).  As in the
 // reference, each worker thread owns one batch slot and runs the whole
-// preprocessing of its batches: distort + codifyInputData on the CPU, then the
+// preprocessing of its batches (of sites given as points, all of them run parts of each): distort + codifyInputData on the CPU, then the
 // upload of the input sites and every layer's preprocess() -- here GPU rule-book
 // kernels -- on the slot's own stream.  nextBatch() hands finished slots to the
 // caller in order, so rule books of the next batches are built while the
@@ -84,6 +84,18 @@ public:
   void preprocessBatchOnDevice(int cc);
 
 private:
+  // Batches whose pictures several threads code, as many parts as there are threads:
+  // the batch whose parts are being handed out, the next of them, and which slots
+  // are with the workers or the caller.
+  bool inParts = false;
+  int nextOpen = 0, nextPart = 0;
+  std::vector<char> slotOpen;
+  void sharedProducerThread(int nThread);
+  int firstOfPart(int size, int part) const;
+  void openBatch(int c, int cc);
+  void preprocessPart(int c, int cc, int part);
+  void normalise(std::vector<float> &features);
+  void stageBatch(int cc, int nParts);
   static SpatiallySparseDataset emptyDataset;
   bool unseen = false;
   std::vector<ResidentBatch> residents; // empty: batches come from the dataset

@@ -62,6 +62,10 @@ public:
     entries_.insert(entries_.end(), kv, kv + n);
     stale_ = stale_ || n > 0;
   }
+  void addToRows(int n) {
+    for (auto &e : entries_)
+      e.second += n;
+  }
   // room for n sites without growing on the way (optional)
   void reserve(size_t n) {
     entries_.reserve(n);

@@ -65,6 +65,15 @@ public:
   batchType type;
   int batchSize;
   std::vector<int> sampleNumbers;
+  // the features of a picture batch as its pictures were coded, in parts by several
+  // threads or in one; kept for the slot's next batch
+  struct Part {
+    std::vector<float> features;
+    std::vector<int> labels;
+    int rows;
+  };
+  std::vector<Part> parts;
+  int partsLeft; // (still being coded)
   std::vector<SpatiallySparseBatchInterface> interfaces;
   vectorCUDA<int> labels;
   std::vector<std::vector<int>> predictions;
@@ -81,10 +90,10 @@ public:
   // a training batch between whose layers nobody looks (processDataset's): what
   // only its layers' kernels would read need not be there
   bool unseen;
-  // device staging of the input sites (sample, key as two ints, row,
-  // backgroundCol), reused from batch to batch
-  vectorCUDA<int> stagingSample, stagingKey, stagingRow, stagingBackground;
-  // the same four arrays on the host, pinned, and how many sites they hold
+  // device staging of the input sites (sample, key as two ints, row),
+  // reused from batch to batch
+  vectorCUDA<int> stagingSample, stagingKey, stagingRow;
+  // the same arrays and backgroundCol on the host, pinned, and how many sites they hold
   PinnedStage hostSample, hostKey, hostRow, hostBackground;
   size_t hostSites;
   // ... and the input features, moved there from the interface's host vector

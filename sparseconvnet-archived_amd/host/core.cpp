@@ -442,7 +442,7 @@ SpatiallySparseBatch::SpatiallySparseBatch(
     : inputSub(inputSub), preprocessStream(nullptr), forwardStream(nullptr),
       labels(false, 0),
       stagingSample(true, 0), stagingKey(true, 0), stagingRow(true, 0),
-      stagingBackground(true, 0), hostSites(0), hostFeatureCount(0),
+      hostSites(0), hostFeatureCount(0),
       result(new BatchResultStage()), poolInverses(true, 0) {
   interfaces.emplace_back(inputSub);
   reset();

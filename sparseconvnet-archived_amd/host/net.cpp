@@ -1,4 +1,5 @@
 // Net runtime, batch production, public facades and canned architectures.
+#include <typeinfo>
 #include <cstring>
 #include <algorithm>
 #include <atomic>
@@ -977,10 +978,17 @@ BatchProducer::BatchProducer(SparseConvNetCUDA &cnn,
 void BatchProducer::start() {
   cnn.ensureInterfaces();
   slotFull.assign(cnn.nBatchProducerThreads, 0);
+  slotOpen.assign(cnn.nBatchProducerThreads, 0);
+  // (pictures that are coded without random numbers, each for itself; a class derived
+  // from theirs may do otherwise)
+  inParts = residents.empty() && cnn.nBatchProducerThreads > 1;
+  for (size_t i = 0; inParts && i < dataset.pictures.size(); ++i)
+    inParts = typeid(*dataset.pictures[i]) == typeid(SparsePointsPicture);
   for (int c = 0; c < cnn.nBatchProducerThreads; c++)
     cnn.batchPool[c].batchSize = 0;
   for (int nThread = 0; nThread < cnn.nBatchProducerThreads; ++nThread)
-    workers.emplace_back(&BatchProducer::batchProducerThread, this, nThread);
+    workers.emplace_back(inParts ? &BatchProducer::sharedProducerThread : &BatchProducer::batchProducerThread, this,
+                         nThread);
 }
 BatchProducer::~BatchProducer() {
   {
@@ -993,7 +1001,7 @@ BatchProducer::~BatchProducer() {
       w.join();
 }
 // CPU half of BatchProducer.cu:40-87: distort, codify, normalise
-void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
+void BatchProducer::openBatch(int c, int cc) {
   SpatiallySparseBatch &b = cnn.batchPool[cc];
   SpatiallySparseBatchInterface &in = b.interfaces[0];
   in.keepGrids(batchSize);
@@ -1005,7 +1013,6 @@ void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
   in.featuresPresent.hVector() = range(dataset.nFeatures);
   const int last = std::min((c + 1) * batchSize, (int)dataset.pictures.size());
   for (int i = c * batchSize; i < last; i++) {
-    Picture *pic = dataset.pictures[permutation[i]]->distort(rng, dataset.type);
     b.sampleNumbers.push_back(permutation[i]);
     b.batchSize++;
     if (in.spareGrids.empty()) {
@@ -1014,49 +1021,96 @@ void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
       in.grids.push_back(std::move(in.spareGrids.back()));
       in.spareGrids.pop_back();
     }
-    b.labels.hVector().push_back(pic->label);
-    pic->codifyInputData(in.grids.back(), in.sub->features.hVector(),
-                         in.nSpatialSites, in.spatialSize);
-    if (pic != dataset.pictures[permutation[i]])
+  }
+}
+void BatchProducer::normalise(std::vector<float> &features) {
+  if (cnn.inputNormalizingConstants.size() > 0)
+    for (size_t i = 0; i < features.size(); ++i)
+      features[i] *= cnn.inputNormalizingConstants[i % dataset.nFeatures];
+}
+void BatchProducer::preprocessBatch(int c, int cc, RNG &rng) {
+  openBatch(c, cc);
+  SpatiallySparseBatch &b = cnn.batchPool[cc];
+  SpatiallySparseBatchInterface &in = b.interfaces[0];
+  b.parts.resize(std::max<size_t>(b.parts.size(), 1));
+  std::vector<float> &features = b.parts[0].features;
+  std::vector<int> &labels = b.parts[0].labels;
+  features.clear();
+  labels.clear();
+  for (int i = 0; i < b.batchSize; i++) {
+    Picture *const own = dataset.pictures[b.sampleNumbers[i]], *pic = own->distort(rng, dataset.type);
+    labels.push_back(pic->label);
+    pic->codifyInputData(in.grids[i], features, in.nSpatialSites, in.spatialSize);
+    if (pic != own)
       delete pic;
   }
-  assert(in.sub->features.size64() ==
-         (size_t)in.nFeatures * (size_t)in.nSpatialSites);
-  if (cnn.inputNormalizingConstants.size() > 0) {
-    std::vector<float> &features = in.sub->features.hVector();
-    for (size_t i = 0; i < features.size(); ++i)
-      features[i] *= cnn.inputNormalizingConstants[i % in.nFeatures];
+  assert(features.size() == (size_t)in.nFeatures * (size_t)in.nSpatialSites);
+  normalise(features);
+  b.parts[0].rows = in.nSpatialSites;
+  stageBatch(cc, 1);
+}
+// The pictures of part `part` of batch c, their rows numbered from 0
+void BatchProducer::preprocessPart(int c, int cc, int part) {
+  SpatiallySparseBatch &b = cnn.batchPool[cc];
+  SpatiallySparseBatchInterface &in = b.interfaces[0];
+  SpatiallySparseBatch::Part &p = b.parts[part];
+  p.features.clear();
+  p.rows = 0;
+  p.labels.clear();
+  for (int i = firstOfPart(b.batchSize, part); i < firstOfPart(b.batchSize, part + 1); ++i) {
+    Picture *const pic = dataset.pictures[permutation[c * batchSize + i]];
+    p.labels.push_back(pic->label);
+    pic->codifyInputData(in.grids[i], p.features, p.rows, in.spatialSize);
   }
-  // The grids as the four arrays scn_grids_build takes, and the features, in
-  // the slot's pinned staging: still on the CPU's time, no stream is held yet,
-  // and the upload is then five queued copies.
-  size_t n = 0;
+  assert(p.features.size() == (size_t)in.nFeatures * (size_t)p.rows);
+  normalise(p.features);
+}
+// The grids as the four arrays scn_grids_build takes, and the features, in
+// the slot's pinned staging: still on the CPU's time, no stream is held yet.
+void BatchProducer::stageBatch(int cc, int nParts) {
+  SpatiallySparseBatch &b = cnn.batchPool[cc];
+  SpatiallySparseBatchInterface &in = b.interfaces[0];
+  size_t n = 0, nFeatures = 0;
   for (auto &g : in.grids)
     n += g.mp.size();
+  for (int part = 0; part < nParts; ++part)
+    nFeatures += b.parts[part].features.size();
   b.hostSample.reserve(n * sizeof(int32_t));
   b.hostKey.reserve(n * sizeof(int64_t));
   b.hostRow.reserve(n * sizeof(int32_t));
   b.hostBackground.reserve((size_t)b.batchSize * sizeof(int32_t));
+  b.hostFeatures.reserve(nFeatures * sizeof(float));
   int32_t *sample = b.hostSample.as<int32_t>(), *row = b.hostRow.as<int32_t>(),
           *bg = b.hostBackground.as<int32_t>();
   int64_t *key = b.hostKey.as<int64_t>();
-  size_t at = 0;
-  for (int item = 0; item < b.batchSize; ++item) {
-    bg[item] = in.grids[item].backgroundCol;
-    for (auto &e : in.grids[item].mp.entries()) {
-      sample[at] = item;
-      key[at] = e.first;
-      row[at] = e.second;
-      ++at;
+  size_t at = 0, to = 0;
+  int base = 0; // the rows of the parts before
+  for (int part = 0; part < nParts; ++part) {
+    const int end = nParts == 1 ? b.batchSize : firstOfPart(b.batchSize, part + 1);
+    for (int item = nParts == 1 ? 0 : firstOfPart(b.batchSize, part); item < end; ++item) {
+      SparseGrid &g = in.grids[item];
+      if (base) {
+        g.backgroundCol += g.backgroundCol < 0 ? 0 : base;
+        g.mp.addToRows(base);
+      }
+      bg[item] = g.backgroundCol;
+      for (auto &e : g.mp.entries()) {
+        sample[at] = item;
+        key[at] = e.first;
+        row[at] = e.second;
+        ++at;
+      }
     }
+    const SpatiallySparseBatch::Part &p = b.parts[part];
+    b.labels.hVector().insert(b.labels.hVector().end(), p.labels.begin(), p.labels.end());
+    if (!p.features.empty())
+      std::memcpy(b.hostFeatures.as<float>() + to, p.features.data(), p.features.size() * sizeof(float));
+    to += p.features.size();
+    base += p.rows;
   }
+  in.nSpatialSites = base;
   b.hostSites = n;
-  std::vector<float> &features = in.sub->features.hVector();
-  b.hostFeatureCount = features.size();
-  b.hostFeatures.reserve(features.size() * sizeof(float));
-  if (!features.empty())
-    std::memcpy(b.hostFeatures.p, features.data(), features.size() * sizeof(float));
-  features.clear();
+  b.hostFeatureCount = nFeatures;
 }
 // Of an unseen training batch the convolutions whose gathered matrix, and that
 // matrix's gradient, the layer behind can do without: no dropout on either side,
@@ -1168,32 +1222,37 @@ void BatchProducer::preprocessBatchOnDevice(int cc) {
   SpatiallySparseBatchInterface &in = b.interfaces[0];
   cudaMemStream &ms = b.preprocessStream ? *b.preprocessStream : cnn.memStream;
   scn_ctx *ctx = ms.ctx;
-  // (flattened into pinned memory by preprocessBatch)
-  const size_t n = b.hostSites;
-  b.stagingSample.resize64(n);
-  b.stagingKey.resize64(2 * n);
-  b.stagingRow.resize64(n);
-  b.stagingBackground.resize64((size_t)b.batchSize);
-  SCN_CHECKED(scn_h2d_async(ctx, b.stagingSample.dPtr(), b.hostSample.p, n * 4));
-  SCN_CHECKED(scn_h2d_async(ctx, b.stagingKey.dPtr(), b.hostKey.p, n * 8));
-  SCN_CHECKED(scn_h2d_async(ctx, b.stagingRow.dPtr(), b.hostRow.p, n * 4));
-  SCN_CHECKED(scn_h2d_async(ctx, b.stagingBackground.dPtr(), b.hostBackground.p,
-                            (size_t)b.batchSize * 4));
+  // (flattened into pinned memory by stageBatch; read from there or copied first as in
+  // preprocessResident: five queued copies of a megabyte kept a thread for 100 to 160 us
+  // beside nine others)
+  const size_t n = b.hostSites, bytes = b.hostFeatureCount * sizeof(float);
+  const bool byCopyEngine = n * 16 + bytes >= kCopyEngineBytes;
+  const int32_t *sample = b.hostSample.as<int32_t>(), *row = b.hostRow.as<int32_t>();
+  const int64_t *key = b.hostKey.as<int64_t>();
+  if (byCopyEngine) {
+    b.stagingSample.resize64(n);
+    b.stagingKey.resize64(2 * n);
+    b.stagingRow.resize64(n);
+    SCN_CHECKED(scn_h2d_async(ctx, b.stagingSample.dPtr(), sample, n * 4));
+    SCN_CHECKED(scn_h2d_async(ctx, b.stagingKey.dPtr(), key, n * 8));
+    SCN_CHECKED(scn_h2d_async(ctx, b.stagingRow.dPtr(), row, n * 4));
+    sample = b.stagingSample.dPtr();
+    key = (const int64_t *)b.stagingKey.dPtr();
+    row = b.stagingRow.dPtr();
+  }
   if (!in.deviceGrids) {
     SCN_CHECKED(scn_grids_create(ctx, &in.deviceGrids));
     in.ownsDeviceGrids = true;
   }
   scn_prof_tag(ctx, -1);
   clearDeviceGrids(ctx, b);
-  SCN_CHECKED(scn_grids_build(ctx, in.deviceGrids, b.batchSize, cnn.dimension,
-                              in.spatialSize, b.stagingSample.dPtr(),
-                              (const int64_t *)b.stagingKey.dPtr(),
-                              b.stagingRow.dPtr(), (int64_t)n,
-                              b.stagingBackground.dPtr(), in.nSpatialSites));
   in.sub->features.copyToGPU(); // (its host vector is empty: nothing moves)
   in.sub->features.resize64(b.hostFeatureCount);
-  SCN_CHECKED(scn_h2d_async(ctx, in.sub->features.dPtr(), b.hostFeatures.p,
-                            b.hostFeatureCount * sizeof(float)));
+  SCN_CHECKED(scn_grids_build_copy(ctx, in.deviceGrids, b.batchSize, cnn.dimension, in.spatialSize, sample, key, row,
+                                   (int64_t)n, b.hostBackground.as<int32_t>(), in.nSpatialSites,
+                                   in.sub->features.dPtr(), b.hostFeatures.p, byCopyEngine ? 0 : bytes));
+  if (byCopyEngine)
+    SCN_CHECKED(scn_h2d_async(ctx, in.sub->features.dPtr(), b.hostFeatures.p, bytes));
   if (b.type == TRAINBATCH) {
     // the classifier's gradient reads the labels on the device: uploaded here,
     // on this slot's stream, so that the net's stream is never waited for
@@ -1238,6 +1297,60 @@ void BatchProducer::batchProducerThread(int nThread) {
     slotChanged.notify_all();
   }
 }
+int BatchProducer::firstOfPart(int size, int part) const {
+  return (int)((int64_t)size * part / cnn.nBatchProducerThreads);
+}
+// The threads take the pictures in the order of the batches, a part of a batch at a
+// time, and the one that ends a batch's last part does its GPU half: the first batch of
+// an epoch, for which the net waits, is coded by all of them in a tenth of the time (400
+// us beside nine others that code the next ones), and is alone in launching its rule
+// books' kernels.
+void BatchProducer::sharedProducerThread(int) {
+  const int nSlots = cnn.nBatchProducerThreads;
+  for (;;) {
+    int c, cc, part;
+    {
+      std::unique_lock<std::mutex> lock(slotMutex);
+      slotChanged.wait(lock, [&] { return stopping || nextOpen >= nBatches || !slotOpen[nextOpen % nSlots] || nextPart; });
+      if (stopping || nextOpen >= nBatches)
+        return;
+      c = nextOpen;
+      cc = c % nSlots;
+      part = nextPart++;
+      SpatiallySparseBatch &b = cnn.batchPool[cc];
+      if (part == 0) {
+        slotOpen[cc] = 1;
+        openBatch(c, cc);
+        b.parts.resize(std::max<size_t>(b.parts.size(), nSlots));
+        b.partsLeft = nSlots;
+      }
+      if (nextPart == nSlots) {
+        ++nextOpen;
+        nextPart = 0;
+        if (nextOpen >= nBatches)
+          slotChanged.notify_all();
+      }
+    }
+    if (part == 0)
+      slotChanged.notify_all(); // (who waited for the slot has parts to take)
+    preprocessPart(c, cc, part);
+    {
+      std::lock_guard<std::mutex> lock(slotMutex);
+      if (--cnn.batchPool[cc].partsLeft > 0)
+        continue;
+    }
+    stageBatch(cc, nSlots);
+    cudaMemStream *stream = cnn.acquireProducerStream(c);
+    cnn.batchPool[cc].preprocessStream = stream;
+    preprocessBatchOnDevice(cc);
+    cnn.releaseProducerStream(stream);
+    {
+      std::lock_guard<std::mutex> lock(slotMutex);
+      slotFull[cc] = 1;
+    }
+    slotChanged.notify_all();
+  }
+}
 int BatchProducer::slotsReady() {
   std::lock_guard<std::mutex> lock(slotMutex);
   int n = 0;
@@ -1259,7 +1372,7 @@ SpatiallySparseBatch *BatchProducer::nextBatch() {
     cnn.batchPool[cc].batchSize = 0;
     {
       std::lock_guard<std::mutex> lock(slotMutex);
-      slotFull[cc] = 0;
+      slotFull[cc] = slotOpen[cc] = 0;
     }
     slotChanged.notify_all();
   }
