@@ -66,8 +66,8 @@ enum {
  * fp32 MFMA's (0.31 to 0.38 of it in root mean square, K 256 to 2592).  The three
  * planes are the operand exactly down to the 2^-133 that a bf16 resolves: an
  * operand below 2^-110 loses its bits below that, 2^-134 at most.  SCN_FP32 runs
- * on the fp32 MFMA except for long contractions (4 GFLOP) and few rows, which it
- * computes as SCN_FP32_PLANES does. */
+ * on the fp32 MFMA except for long contractions and few rows, which it computes
+ * as SCN_FP32_PLANES does. */
 enum { SCN_FP32 = 0, SCN_BF16 = 1, SCN_BF16X3 = 2, SCN_FP32_PLANES = 3 };
 
 typedef struct scn_ctx scn_ctx;

@@ -1845,23 +1845,19 @@ static void launch_mfma(scn_ctx *ctx, const float *A, const float *W,
                        ctx->stream, A, W, out, M, K, N, ep, GatherSource());
 }
 
-// SCN_FP32 goes to the bf16 matrix cores where the contraction is long (4 GFLOP, or 40 for
-// one tile of columns) or its rows are few (the split contraction: 600 x 384 x 128 in 5.0
-// us for 9.5).  In between it keeps to fp32 MFMA, and so to the bits it has always given.
-// us, fp32 MFMA and planes, their image made by the call where they take one: rows through
-// rules 53325 x 640 x 320 220, 127; 35615 x 3456 x 128 331, 241; 28915 x 864 x 128 71, 42;
-// 148881 x 256 x 128 102, 72; 80899 x 256 x 96 (4.0 GFLOP) 47.5, 39.5; 1.36 M x 1728 x 64 and its
-// pooling 2240, 1410; plain 28955 x 512 x 256 72, 48; 10746 x 1728 x 128 64, 40; 46 shapes of 4 to
-// 40 GFLOP 0.55 to 0.92 of it through rules, plain 0.46 to 0.94.  Below, it would gain as
-// much through rules (37629 x 256 x 64 26.5, 18), and plain lose at some sizes (6136 x 192 x
-// 256 11.6, 12.8).  Of 32 columns plain 123606 x 768 83, 87; 23769 x 3456 83, 117; but
-// 174344 x 1728 267, 237 (through rules 0.85).  The sizes decide, and not the rules: a fused
-// layer has the bits of gather and contraction.  The error against 64 bits is a third of
-// the fp32 MFMA's (64 to 3456 k: root mean square 0.34 to 0.42, largest 0.28 to 0.5).
-// SCN_FP32_PLANES, which the host classes ask for, takes the planes at every size.
-static bool long_contraction(int64_t M, int K, int N) {
-  return 2e0 * M * K * N >= (N > 32 || (K >= 800 && M >= 40000) ? 4e9 : 4e10);
-}
+// SCN_FP32 goes to the bf16 matrix cores where the contraction is long (40
+// GFLOP: 1.36 M x 1728 x 64 and its pooling 2.24 -> 1.41 ms) or its rows are few
+// (the split contraction: 600 x 384 x 128 in 5.0 us for 9.5).  In between it
+// keeps to fp32 MFMA, and so to the bits it has always given, though the planes,
+// their image made by the call, have become the faster there but for the shortest
+// contractions of plain rows (us, fp32 MFMA and planes, rows through rules: 35461 x
+// 256 x 96 35, 23; 17223 x 384 x 128 39, 22; 53325 x 640 x 320 220, 127; 11742 x 1920 x
+// 640 269, 144; 126507 x 1728 x 64 233, 142; 118775 x 128 x 32 19.5, 15.8, plain 16.8,
+// 26.5; 46 shapes of 4 to 40 GFLOP 0.55 to 0.92 of it through rules, plain 0.46 to 0.94):
+// a rectifier that other bits put on the other side of its threshold takes its share of the
+// gradients with it, 1e-3 of a layer's for a background row's.  SCN_FP32_PLANES, which
+// the host classes ask for, takes the planes at every size.
+#define PLANES_MIN_FLOPS 4e10
 // rows16: a bf16 copy of the matrix the rules point into, or null; image: the
 // weights for the planes (scn_weight_images_many), or null; matrix: where
 // k_conv_thin, which it asks for, is to leave the rows, or null
@@ -1905,7 +1901,7 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
   bool fewRows = few && scn_rows_hint(ctx, M) <= FR_MAX_M;
   auto takes_planes = [&]() {
     return shape && ((rounded && act != SCN_SOFTMAX) || precision == SCN_FP32_PLANES ||
-                     long_contraction(M, K, N) || scn_planes_splitk(ctx, 3, M, K, N));
+                     2e0 * M * K * N >= PLANES_MIN_FLOPS || scn_planes_splitk(ctx, 3, M, K, N));
   };
   bool planes = takes_planes();
   const bool tiledBf16 = vec && K >= 64 && act != SCN_SOFTMAX && rounded && !planes;
