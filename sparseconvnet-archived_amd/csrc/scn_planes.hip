@@ -2324,7 +2324,7 @@ template <int MT, int NT, bool GATHER, bool LINES, int GM>
 __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const float *__restrict__ D, float *__restrict__ dW,
                                          float *__restrict__ db, long long M, int K, int N, int nTiles,
                                          GatherSource gs, const float *zeros, unsigned tile, long long m0,
-                                         long long m1) {
+                                         long long m1, int nBase = 0) {
   constexpr int PL = 3;
   constexpr int TILE = 32 * MT * 32 * NT; // floats of a wavefront's tile
   extern __shared__ __attribute__((aligned(16))) float sTile[]; // [GM][TILE], [GM][32 NT], a flag
@@ -2335,7 +2335,7 @@ __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const floa
   const int lane = tid & 63, wave = tid >> 6;
   const int c = lane & 31, q = lane >> 5;
   const int k0 = (int)(tile / nTiles) * 32 * MT;
-  const int n0 = (int)(tile % nTiles) * 32 * NT;
+  const int n0 = nBase + (int)(tile % nTiles) * 32 * NT;
   // this lane's columns (past the end: the last ones, not stored)
   int ka = k0 + MT * c, na = n0 + NT * c;
   ka = ka + MT <= K ? ka : K - MT;
@@ -2600,7 +2600,7 @@ __device__ __forceinline__ void atb_tile(const float *__restrict__ A, const floa
           step(odd, even, t);
         }
       } else {
-        static_assert(!GATHER || RING == 3, "the first two steps' rules come together");
+        static_assert(!GATHER || RING <= 3, "the first two steps' rules come together");
         Rules x;
         {
           Rules second;
@@ -2805,9 +2805,10 @@ static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, f
 template <int MT, int NT>
 static int launch_atb(scn_ctx *ctx, const float *A, const float *D, float *dW, float *db, long long M, int K, int N,
                       long long rows, const GatherSource *gs, bool lines) {
-  if constexpr (MT == 2 && NT == 2) // (not gathered: see below)
-    return lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, rows, GatherSource())
-                 : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, rows, GatherSource());
+  if constexpr (MT == 2 && NT == 2) // (gathered by lines only: see below)
+    return gs      ? launch_atb<MT, NT, true, true>(ctx, A, D, dW, db, M, K, N, rows, *gs)
+           : lines ? launch_atb<MT, NT, false, true>(ctx, A, D, dW, db, M, K, N, rows, GatherSource())
+                   : launch_atb<MT, NT, false, false>(ctx, A, D, dW, db, M, K, N, rows, GatherSource());
   else if (gs)
     return lines ? launch_atb<MT, NT, true, true>(ctx, A, D, dW, db, M, K, N, rows, *gs)
                  : launch_atb<MT, NT, true, false>(ctx, A, D, dW, db, M, K, N, rows, *gs);
@@ -2821,9 +2822,17 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
   // (requests of four columns, in one filter position each)
   const bool lines = K % 4 == 0 && N % 4 == 0 && (!gs || gs->nIn % 4 == 0) && (((uintptr_t)A | (uintptr_t)D) & 15) == 0;
   // Pairs of columns are loaded as one: K (N) even for two row (column) tiles.  (Two by two
-  // tiles of gathered rows, and with sums but not by lines: 264 bytes a lane spilled)
+  // tiles not by lines, of gathered rows or with sums: 264 bytes a lane spilled)
   const bool pairsA = (gs ? gs->nIn : K) % 2 == 0 && ((uintptr_t)A & 7) == 0, pairsD = N % 2 == 0 && ((uintptr_t)D & 7) == 0;
-  const AtbChoice c = atb_choose(ctx->numCU, M, K, N, lines, pairsA, pairsD, !gs && (!db || lines));
+  AtbChoice c = atb_choose(ctx->numCU, M, K, N, lines, pairsA, pairsD, !gs && (!db || lines));
+  // (through rules they take a quarter longer than of plain rows: us, two by one and two by
+  // two, 150000 x 1728 x 64 257, 209; 139000 x 384 x 128 118, 96; 12000 x 1152 x 128 38, 33.5;
+  // 30000 x 256 x 128, which costs 20.3 and 19.5 by atb_choose, 22, 25; 60000 x 256 x 64 22, 24.7)
+  if (gs && lines) {
+    const AtbChoice two = atb_choose(ctx->numCU, M, K, N, true, pairsA, pairsD, true);
+    if (1.25 * two.cost < c.cost)
+      c = two;
+  }
   SCN_REQUIRE(c.tile >= 0, SCN_ERR_CAPACITY, "scn_sgemm_AtB: K %d N %d", K, N);
   switch (c.tile) { // (as in atbTiles)
   case 1:
@@ -2847,75 +2856,85 @@ int scn_atb_planes(scn_ctx *ctx, const float *A, const float *D, float *dW, floa
 // a batch of 100 drawings (83597 x 12 x 32 to 100 x 192 x 100): 81 us in launches of
 // their own, 57 with workgroups of one range each, 51 so; without the first layer 65,
 // 50, 48.  12 batches of drawings 6515 -> 6260 us, of voxel models 5430 -> 5285.
-// What is left of it: 0.13 us a wavefront's step on a compute unit, in which vector
-// instructions are issued for half of the time, MFMAs run for a fifth and the
-// address unit works for a third; with any one of the three left out 0.11.
-// Tiles of two by one, by lines, through rules and without; one by one of rows that
-// are no whole requests, a net's first layer.
+// The tiles are two by two where dW has the columns, by eight wavefronts: its rows and
+// D's are then read half as often, and split into planes two thirds as often, as for tiles
+// of two by one by twelve wavefronts, which a step took for as long as all its requests,
+// vector instructions and MFMAs one after the other (0.13 us a wavefront on a compute
+// unit; with any one of them left out 0.11): seven layers of drawings 47 -> 39 us, six of
+// voxel models 39.5 -> 34.  Wider tiles shared by the wavefronts would end in more
+// atomics, of which 256 workgroups of 4096 each are some 5 us.
+// What is left of up to half a tile at the end of dW's columns is two by one; rows that
+// are no whole requests, a net's first layer, one by one.
+constexpr int ATB_ENTRIES = 2 * SCN_ATB_MAX; // (a layer may be two of them)
 struct AtbList {
-  const float *A[SCN_ATB_MAX], *D[SCN_ATB_MAX];
-  float *dW[SCN_ATB_MAX], *db[SCN_ATB_MAX];
-  const int *rules[SCN_ATB_MAX]; // null: plain rows
+  const float *A[ATB_ENTRIES], *D[ATB_ENTRIES];
+  float *dW[ATB_ENTRIES], *db[ATB_ENTRIES];
+  const int *rules[ATB_ENTRIES]; // null: plain rows
   const float *zeros;
-  int M[SCN_ATB_MAX], K[SCN_ATB_MAX], N[SCN_ATB_MAX], fs[SCN_ATB_MAX];
-  int steps[SCN_ATB_MAX]; // of a range, ATB_MANY ATB_STEP rows each
-  int first[SCN_ATB_MAX]; // place in the line
+  int M[ATB_ENTRIES], K[ATB_ENTRIES], N[ATB_ENTRIES], fs[ATB_ENTRIES];
+  int steps[ATB_ENTRIES]; // of a range, ATB_MANY ATB_STEP rows each
+  int first[ATB_ENTRIES]; // place in the line
+  // the first of its columns of dW, tiles of columns, of what kind.  (Words, not bytes: with
+  // an array of bytes beside them the compiler takes its index into the base of the
+  // pointers' scalar loads, whose address loses the last two bits of each of its parts.)
+  int column[ATB_ENTRIES], nTiles[ATB_ENTRIES], kind[ATB_ENTRIES];
   int count, length, part; // of the line; of a workgroup
 };
-constexpr int ATB_MANY = atb_waves(2, 1, true); // wavefronts
+constexpr int ATB_MANY = 8; // wavefronts
 static_assert(ATB_MANY * ATB_STEP == ATB_MANY_ROWS, "a step of a range");
-__device__ __host__ __forceinline__ int atb_step_cost(const int *rules, int nIn) {
-  return rules && nIn % 4 ? ATB_FIRST_COST : ATB_LINES_COST;
-}
+static_assert(sizeof(AtbList) <= 4096, "a kernel's arguments");
 __global__ void __launch_bounds__(64 * ATB_MANY, ATB_MANY / 4) k_atb_many(AtbList l) {
-  static_assert(SCN_ATB_MAX <= 64, "a lane an item");
+  static_assert(ATB_ENTRIES <= 64, "a lane an entry");
   int pos = (int)xcd_eighth(blockIdx.x, gridDim.x) * l.part; // (neighbours to one XCD)
   const int end = pos + l.part < l.length ? pos + l.part : l.length;
 #pragma unroll 1
   while (pos < end) { // uniform
     const int lane = __lane_id(); // (anew)
-    const int t = __popcll(__ballot(lane < l.count && pos >= l.first[lane < SCN_ATB_MAX ? lane : 0])) - 1;
-    const int K = l.K[t], N = l.N[t], steps = l.steps[t], M = l.M[t];
+    const int t = __popcll(__ballot(lane < l.count && pos >= l.first[lane < ATB_ENTRIES ? lane : 0])) - 1;
+    const int K = l.K[t], N = l.N[t], steps = l.steps[t], M = l.M[t], kind = l.kind[t];
     GatherSource gs = GatherSource();
     gs.rules = l.rules[t];
     gs.fs = l.fs[t];
     gs.nIn = K / gs.fs;
     gs.zeros = l.zeros;
-    const int cost = atb_step_cost(gs.rules, gs.nIn), whole = ATB_TILE_COST + steps * cost;
+    const int cost = atbKinds[kind].step, begin = atbKinds[kind].tile, whole = begin + steps * cost;
     // the range of a tile that this is in, tile after tile of one range of rows
     const unsigned unit = (unsigned)(pos - l.first[t]) / whole;
     const int from = pos - l.first[t] - (int)unit * whole;
     const int to = whole - from < end - pos ? whole : from + end - pos;
-    auto step = [&](int place) { return place <= ATB_TILE_COST ? 0 : (place - ATB_TILE_COST + cost - 1) / cost; };
+    auto step = [&](int place) { return place <= begin ? 0 : (place - begin + cost - 1) / cost; };
     pos += to - from;
-    const int nTiles = (N + 31) / 32;
-#define SCN_ATB_TILE(MT, GATHER, LINES)                                                                         \
-  const unsigned tiles = (K + 32 * MT - 1) / (32 * MT) * nTiles;                                                \
-  const long long r0 = (long long)(unit / tiles) * steps;                                                       \
-  const long long m0 = (r0 + step(from)) * (ATB_MANY * ATB_STEP), m1 = (r0 + step(to)) * (ATB_MANY * ATB_STEP); \
-  if (m0 < (m1 < M ? m1 : M)) {                                                                                 \
-    __syncthreads(); /* (the one before is done with LDS) */                                                    \
-    atb_tile<MT, 1, GATHER, LINES, ATB_MANY>(l.A[t], l.D[t], l.dW[t], l.db[t], M, K, N, nTiles, gs, l.zeros,    \
-                                             unit % tiles, m0, m1 < M ? m1 : M);                                \
-  }
-    if (gs.rules && gs.nIn % 4 == 0) {
-      SCN_ATB_TILE(2, true, true);
-    } else if (gs.rules) {
-      SCN_ATB_TILE(1, true, false);
-    } else {
-      SCN_ATB_TILE(2, false, true);
-    }
+    const int nTiles = l.nTiles[t];
+    const unsigned tiles = (unsigned)(K + 32 * atbKinds[kind].mt - 1) / (32 * atbKinds[kind].mt) * nTiles;
+    const long long r0 = (long long)(unit / tiles) * steps;
+    const long long m0 = (r0 + step(from)) * ATB_MANY_ROWS, m1 = (r0 + step(to)) * ATB_MANY_ROWS;
+    if (m0 >= (m1 < M ? m1 : M))
+      continue;
+    __syncthreads(); // (the one before is done with LDS)
+#define SCN_ATB_TILE(MT, NT, GATHER, LINES)                                                                   \
+  atb_tile<MT, NT, GATHER, LINES, ATB_MANY>(l.A[t], l.D[t], l.dW[t], l.db[t], M, K, N, nTiles, gs, l.zeros, \
+                                            unit % tiles, m0, m1 < M ? m1 : M, l.column[t])
+    if (kind == ATB_WIDE && gs.rules)
+      SCN_ATB_TILE(2, 2, true, true);
+    else if (kind == ATB_WIDE)
+      SCN_ATB_TILE(2, 2, false, true);
+    else if (kind == ATB_FIRST)
+      SCN_ATB_TILE(1, 1, true, false);
+    else if (gs.rules)
+      SCN_ATB_TILE(2, 1, true, true);
+    else
+      SCN_ATB_TILE(2, 1, false, true);
 #undef SCN_ATB_TILE
   }
 }
-// the tile that an item takes among many, or 0: not one for it
-static int atb_many_tile(const scn_atb_item &it) {
+// how an item is taken among many: -1: not one for it
+static int atb_many_kind(const scn_atb_item &it) {
   const int K = it.fs * it.nIn;
   if (it.M > (1 << 30) || it.N % 4 || (((uintptr_t)it.d_in | (uintptr_t)it.d_D) & 15))
-    return 0;
-  if (it.d_positions)
-    return it.nIn % 4 == 0 ? 2 : K <= 32 ? 1 : 0;
-  return K % 4 == 0 ? 2 : 0;
+    return -1;
+  if (it.d_positions && it.nIn % 4)
+    return K <= 32 ? ATB_FIRST : -1;
+  return K % 4 ? -1 : it.N > 32 ? ATB_WIDE : ATB_NARROW;
 }
 int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
   AtbList l;
@@ -2923,30 +2942,39 @@ int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
   l.zeros = ctx->d_zeros;
   AtbShape shape[SCN_ATB_MAX];
   bool joined[SCN_ATB_MAX];
-  for (int k = 0; k < nItems; ++k)
-    shape[k] = {items[k].M, items[k].fs * items[k].nIn, items[k].N, atb_many_tile(items[k]),
-                atb_step_cost(items[k].d_positions, items[k].nIn)};
+  int kinds[SCN_ATB_MAX];
+  for (int k = 0; k < nItems; ++k) {
+    kinds[k] = atb_many_kind(items[k]);
+    shape[k] = {items[k].M, items[k].fs * items[k].nIn, items[k].N, kinds[k] < 0 ? 0 : atbKinds[kinds[k]].mt,
+                kinds[k] < 0 ? 0 : atbKinds[kinds[k]].step / atbKinds[kinds[k]].nt};
+  }
   atb_join(ctx->numCU, shape, nItems, joined);
-  long long tiles[SCN_ATB_MAX], steps[SCN_ATB_MAX], work = 0;
-  int cost[SCN_ATB_MAX];
+  long long tiles[ATB_ENTRIES], steps[ATB_ENTRIES], work = 0;
+  auto enter = [&](const scn_atb_item &it, int kind, int column, int columns) {
+    const int c = l.count++, K = it.fs * it.nIn;
+    const AtbKind &x = atbKinds[kind];
+    l.A[c] = it.d_in, l.D[c] = it.d_D, l.dW[c] = it.d_dW, l.db[c] = it.d_db, l.rules[c] = it.d_positions;
+    l.M[c] = (int)it.M, l.K[c] = K, l.N[c] = it.N, l.fs[c] = it.fs, l.kind[c] = kind;
+    l.column[c] = column, l.nTiles[c] = (int)scn_ceil_div(columns, 32 * x.nt);
+    tiles[c] = scn_ceil_div(K, 32 * x.mt) * l.nTiles[c], steps[c] = scn_ceil_div(it.M, ATB_MANY_ROWS);
+    work += tiles[c] * steps[c] * x.step;
+  };
   for (int k = 0; k < nItems; ++k) {
     const scn_atb_item &it = items[k];
-    const int K = shape[k].K;
     if (it.M > 0 && !joined[k]) {
       GatherSource gs = GatherSource();
       gs.rules = it.d_positions;
       gs.fs = it.fs;
       gs.nIn = it.nIn;
       gs.zeros = ctx->d_zeros;
-      SCN_TRY(scn_atb_planes(ctx, it.d_in, it.d_D, it.d_dW, it.d_db, it.M, K, it.N, it.d_positions ? &gs : nullptr));
+      SCN_TRY(scn_atb_planes(ctx, it.d_in, it.d_D, it.d_dW, it.d_db, it.M, shape[k].K, it.N, it.d_positions ? &gs : nullptr));
     }
     if (!joined[k])
       continue;
-    const int c = l.count++;
-    l.A[c] = it.d_in, l.D[c] = it.d_D, l.dW[c] = it.d_dW, l.db[c] = it.d_db, l.rules[c] = it.d_positions;
-    l.M[c] = (int)it.M, l.K[c] = K, l.N[c] = it.N, l.fs[c] = it.fs;
-    tiles[c] = shape[k].tiles(), steps[c] = shape[k].steps(), cost[c] = shape[k].each;
-    work += tiles[c] * steps[c] * cost[c];
+    const int rest = kinds[k] == ATB_WIDE && (it.N - 1) % 64 < 32 ? (it.N - 1) % 64 + 1 : 0; // (columns of half a tile)
+    enter(it, kinds[k], 0, it.N - rest);
+    if (rest)
+      enter(it, ATB_NARROW, it.N - rest, rest);
   }
   if (l.count == 0)
     return SCN_OK;
@@ -2955,16 +2983,19 @@ int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems) {
   const long long part = scn_ceil_div(work, ctx->numCU);
   long long length = 0;
   for (int c = 0; c < l.count; ++c) {
-    long long ranges = (steps[c] * cost[c] + part / 2) / part;
+    const AtbKind &x = atbKinds[l.kind[c]];
+    long long ranges = (steps[c] * x.step + part / 2) / part;
     ranges = ranges < 1 ? 1 : ranges > steps[c] ? steps[c] : ranges;
     l.steps[c] = (int)scn_ceil_div(steps[c], ranges);
     l.first[c] = (int)length;
-    length += tiles[c] * scn_ceil_div(steps[c], l.steps[c]) * (ATB_TILE_COST + (long long)l.steps[c] * cost[c]);
+    length += tiles[c] * scn_ceil_div(steps[c], l.steps[c]) * (x.tile + (long long)l.steps[c] * x.step);
   }
   l.length = (int)length; // (at most SCN_ATB_MAX times what an item may be, and a range more of each)
   l.part = scn_ceil_div(length, ctx->numCU);
-  constexpr size_t lds = atb_lds(2, 1, true, true, ATB_MANY);
-  static_assert(lds >= atb_lds(2, 1, false, true, ATB_MANY) && lds >= atb_lds(1, 1, true, false, ATB_MANY), "one size for all");
+  constexpr size_t lds = atb_lds(2, 2, true, true, ATB_MANY);
+  static_assert(lds <= 160 << 10 && lds >= atb_lds(2, 2, false, true, ATB_MANY) && lds >= atb_lds(2, 1, true, true, ATB_MANY) &&
+                    lds >= atb_lds(2, 1, false, true, ATB_MANY) && lds >= atb_lds(1, 1, true, false, ATB_MANY),
+                "one size for all");
   static OncePerDevice configured;
   const int rc = configured.run(ctx->device, [&]() {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(k_atb_many), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -162,11 +162,17 @@ static inline AtbChoice atb_choose(int numCU, int64_t M, int K, int N, bool line
 }
 
 // ---- weight gradients of several layers (k_atb_many)
-// What a step and a tile's beginning and end take, in sixteenths of a microsecond
-// (measured by the clock in the kernel, layers of 2500 to 84000 rows: by lines 1.42
-// to 1.68 us a step, a first layer's 1.3, and 4.7)
-constexpr int ATB_LINES_COST = 25, ATB_FIRST_COST = 21, ATB_TILE_COST = 75;
-constexpr int ATB_MANY_ROWS = 192; // of a step
+// How a layer is taken: a first layer's few columns, two by one tiles for what is no more
+// than 32 columns of dW wide, two by two.  What a step and a tile's beginning and end
+// take, in sixteenths of a microsecond: these of eleven sets, by which the layers of a
+// batch of drawings took 39 to 44 us and of voxel models 34 to 37.
+enum { ATB_FIRST, ATB_NARROW, ATB_WIDE };
+struct AtbKind {
+  int mt, nt, step, tile;
+};
+constexpr AtbKind atbKinds[3] = {{1, 1, 16, 75}, {2, 1, 17, 75}, {2, 2, 27, 88}};
+constexpr int ATB_TILE_COST = 75; // (for atb_join)
+constexpr int ATB_MANY_ROWS = 128; // of a step
 struct AtbShape {
   int64_t M;
   int K, N;
