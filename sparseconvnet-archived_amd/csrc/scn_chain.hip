@@ -1261,6 +1261,7 @@ static int chain_flush_pyramid(scn_ctx *ctx, ChainState *cs, std::vector<ChainRe
   a.dense = (long long)src->batch * src->vol <= SCN_DENSE_MAX_SITES ? src->dense.p : nullptr;
   a.shift = 64 - src->log2cap;
   a.mask = (1u << src->log2cap) - 1u;
+  scn_grids_hold_mask(ctx, src);
   a.bits = src->bits.p;
   a.bg = src->bg.p;
   // Pass A: a wavefront per (sample, level, slab), each level from the source's
@@ -1331,6 +1332,7 @@ int scn_chain_flush(scn_ctx *ctx) {
   a.dense = (long long)src->batch * src->vol <= SCN_DENSE_MAX_SITES ? src->dense.p : nullptr;
   a.shift = 64 - src->log2cap;
   a.mask = (1u << src->log2cap) - 1u;
+  scn_grids_hold_mask(ctx, src);
   a.bits = src->bits.p;
   a.bg = src->bg.p;
   a.vol0 = src->vol;

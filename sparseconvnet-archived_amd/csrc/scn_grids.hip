@@ -47,15 +47,24 @@ template <int N> __device__ __forceinline__ void or_run(unsigned &lo, unsigned &
 // a site), so runs of up to 16 lanes with sites of one word make one of it
 // (11.5 us).  The workgroups behind the sites' copy `bytes` from src to dst: a
 // batch's features, a launch of 2 us and the gap before it otherwise (the
-// classification of one drawing, 125 us with the two launches: 121).
+// classification of one drawing, 125 us with the two launches: 121).  Those behind
+// empty the mask that the next batch will take (scn_grids_clear_many).
 __global__ void __launch_bounds__(256) k_grid_build(GridView g, const int *sample,
                              const long long *key, const int *row, long long n,
                              long long *ekey, int *erow,
                              unsigned long long *badSites,
-                             const int *bgIn, int *bgOut, unsigned siteBlocks,
-                             const unsigned char *src, unsigned char *dst, size_t bytes) {
+                             const int *bgIn, int *bgOut, unsigned siteBlocks, unsigned copyBlocks,
+                             const unsigned char *src, unsigned char *dst, size_t bytes,
+                             unsigned long long *spare, size_t spareWords) {
+  if (blockIdx.x >= siteBlocks + copyBlocks) {
+    const size_t i = (size_t)(blockIdx.x - siteBlocks - copyBlocks) * 256 + threadIdx.x;
+    const size_t step = (size_t)(gridDim.x - siteBlocks - copyBlocks) * 256;
+    for (size_t k = i; k < spareWords; k += step)
+      spare[k] = 0ull;
+    return;
+  }
   if (blockIdx.x >= siteBlocks) {
-    const size_t i = (size_t)(blockIdx.x - siteBlocks) * 256 + threadIdx.x, step = (size_t)(gridDim.x - siteBlocks) * 256;
+    const size_t i = (size_t)(blockIdx.x - siteBlocks) * 256 + threadIdx.x, step = (size_t)copyBlocks * 256;
     const size_t n16 = (((uintptr_t)src | (uintptr_t)dst) & 15) ? 0 : bytes / 16;
     for (size_t k = i; k < n16; k += step)
       reinterpret_cast<uint4 *>(dst)[k] = reinterpret_cast<const uint4 *>(src)[k];
@@ -1264,7 +1273,18 @@ static bool dense_rows(const scn_grids *g) {
   return (long long)(g->batch > 0 ? g->batch : 1) * g->vol <= SCN_DENSE_MAX_SITES;
 }
 
-GridView view_of(const scn_grids *g) {
+void scn_grids_hold_mask(scn_ctx *ctx, const scn_grids *g) {
+  if (g->maskHeld)
+    return;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess)
+    (void)hipGetLastError(); // (not known: as if it were)
+  else if (capturing == hipStreamCaptureStatusNone)
+    return;
+  g->maskHeld = true;
+}
+GridView view_of(scn_ctx *ctx, const scn_grids *g) {
+  scn_grids_hold_mask(ctx, g);
   GridView v;
   v.table = g->tableValid && !dense_rows(g) ? g->table.p : nullptr;
   v.dense = g->tableValid && dense_rows(g) ? g->dense.p : nullptr;
@@ -1375,7 +1395,10 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
   return SCN_OK;
 }
 
-// One launch empties the tables and masks of up to CLEAR_MANY grids objects.
+// One launch empties the tables and masks of up to CLEAR_MANY grids objects, but for
+// those that have an empty mask to go on with: a launch of 3 us and the gap behind it,
+// at the beginning of every batch (us, one drawing 115 -> 101 to 111, 100 drawings 188 -> 179
+// to 190, 32 voxel models 185 -> 180: runs fall into one of two groups).
 #define CLEAR_MANY 24
 struct ClearList {
   uint4 *slots[CLEAR_MANY];
@@ -1411,6 +1434,17 @@ extern "C" int scn_grids_clear_many(scn_ctx *ctx, scn_grids **grids, int n) {
       if (!g->indexValid || ((!g->table.p || g->cleanSlots >= g->table.cap) &&
                              (!g->bits.p || g->cleanWords >= g->bits.cap)))
         continue;
+      g->emptied = true;
+      scn_grids_hold_mask(ctx, g);
+      if (g->spare && g->spareClean && g->spareCap == g->bits.cap && !g->maskHeld &&
+          (!g->table.p || g->cleanSlots >= g->table.cap)) { // (what was in use: emptied by the build)
+        std::swap(g->bits.p, g->spare);
+        g->spareClean = false;
+        g->cleanWords = g->bits.cap;
+        g->rankValid = g->rankRowValid = g->tableValid = false;
+        g->nActive = 0;
+        continue;
+      }
       l.slots[m] = (uint4 *)g->table.p;
       l.nSlots[m] = g->table.p ? g->table.cap : 0;
       l.bits[m] = g->bits.p;
@@ -1477,7 +1511,7 @@ static int ensure_index(scn_ctx *ctx, scn_grids *g) {
   g->chained = chained;
   if (nActive > 0) {
     hipLaunchKernelGGL(k_grid_index, dim3(scn_ceil_div(nActive, 256)), dim3(256),
-                       0, ctx->stream, view_of(g), g->ekey.p, g->erow.p,
+                       0, ctx->stream, view_of(ctx, g), g->ekey.p, g->erow.p,
                        count_active(g), pending ? g->meta.p : nullptr);
     SCN_HIP_CHECK(hipGetLastError());
   }
@@ -1492,6 +1526,7 @@ static int ensure_prefix(scn_ctx *ctx, scn_grids *g) {
   const bool cleared = g->rankStateFor == g->nWords + 1; // (by the kernel that wrote or cleared the mask)
   g->rankStateFor = 0;
   SCN_TRY(g->scanTmp.reserve(scn_scan_tmp_elems(g->nWords + 1)));
+  scn_grids_hold_mask(ctx, g);
   // one word past the mask so that the rank of the end position is defined
   SCN_TRY(scn_scan_exclusive_popc64(ctx->stream,
                                     (const uint64_t *)g->bits.p, g->prefix.p,
@@ -1516,7 +1551,7 @@ static int ensure_rank(scn_ctx *ctx, scn_grids *g) {
   SCN_TRY(missing_rank_rows(g, &rows));
   if (rows.rankRow) {
     hipLaunchKernelGGL(k_rank_rows, dim3(xcd_grid(scn_ceil_div(g->nActive, 256))), dim3(256), 0, ctx->stream,
-                       view_of(g), rows);
+                       view_of(ctx, g), rows);
     SCN_HIP_CHECK(hipGetLastError());
   }
   g->rankRowValid = true;
@@ -1550,7 +1585,7 @@ int scn_grids_ensure_table(scn_ctx *ctx, scn_grids *g) {
   g->tableValid = true; // (view_of hands the table out from here on)
   if (g->nActive > 0) {
     hipLaunchKernelGGL(k_grid_table, dim3(scn_ceil_div(g->nActive, 256)),
-                       dim3(256), 0, ctx->stream, view_of(g), g->ekey.p,
+                       dim3(256), 0, ctx->stream, view_of(ctx, g), g->ekey.p,
                        g->erow.p, count_active(g),
                        g->pending ? g->meta.p : nullptr);
     SCN_HIP_CHECK(hipGetLastError());
@@ -1736,6 +1771,7 @@ extern "C" int scn_grids_destroy(scn_ctx *ctx, scn_grids *g) {
   g->table.release();
   g->dense.release();
   g->bits.release();
+  (void)hipFree(g->spare);
   g->prefix.release();
   g->rankRow.release();
   g->ekey.release();
@@ -1758,6 +1794,8 @@ extern "C" int scn_grids_destroy(scn_ctx *ctx, scn_grids *g) {
   return SCN_OK;
 }
 
+// masks that are emptied beside the next batch's build and not before it: 1 MB
+#define SPARE_MASK_WORDS ((size_t)1 << 17)
 extern "C" int scn_grids_build(scn_ctx *ctx, scn_grids *g, int batch,
                                int dimension, int spatialSize,
                                const int32_t *d_sample, const int64_t *d_key,
@@ -1795,14 +1833,30 @@ extern "C" int scn_grids_build_copy(scn_ctx *ctx, scn_grids *g, int batch,
   const long long lanes = n > batch ? n : batch;
   const unsigned siteBlocks = (unsigned)scn_ceil_div(lanes, 256);
   const size_t copyBlocks = bytes ? std::min((bytes / 16 + 255) / 256 + 1, (size_t)4096) : 0;
+  const GridView view = view_of(ctx, g);
+  size_t spareWords = 0;
+  if (siteBlocks + copyBlocks > 0 && g->emptied && !g->maskHeld && g->bits.cap <= SPARE_MASK_WORDS) {
+    if (g->spareCap != g->bits.cap) {
+      (void)hipFree(g->spare);
+      g->spareCap = g->bits.cap;
+      g->spareClean = false;
+      if (hipMalloc((void **)&g->spare, g->spareCap * sizeof(*g->spare)) != hipSuccess) { // (done without)
+        (void)hipGetLastError();
+        g->spare = nullptr;
+      }
+    }
+    spareWords = g->spare && !g->spareClean ? g->spareCap : 0;
+  }
+  const size_t spareBlocks = std::min((spareWords + 1023) / 1024, (size_t)256);
   if (siteBlocks + copyBlocks > 0) {
-    hipLaunchKernelGGL(k_grid_build, dim3((unsigned)(siteBlocks + copyBlocks)), dim3(256), 0,
-                       ctx->stream, view_of(g), d_sample,
+    hipLaunchKernelGGL(k_grid_build, dim3((unsigned)(siteBlocks + copyBlocks + spareBlocks)), dim3(256), 0,
+                       ctx->stream, view, d_sample,
                        (const long long *)d_key, d_row, (long long)n, g->ekey.p,
                        g->erow.p, (unsigned long long *)(ctx->d_scalars + 15),
-                       d_background, g->bg.p, siteBlocks, (const unsigned char *)src,
-                       (unsigned char *)dst, bytes);
+                       d_background, g->bg.p, siteBlocks, (unsigned)copyBlocks, (const unsigned char *)src,
+                       (unsigned char *)dst, bytes, g->spare, spareWords);
     SCN_HIP_CHECK(hipGetLastError());
+    g->spareClean = g->spareClean || spareWords;
   }
   return SCN_OK;
 }
@@ -1842,7 +1896,7 @@ extern "C" int scn_grids_download(scn_ctx *ctx, const scn_grids *cg,
     SCN_TRY(g->dlRow.reserve((size_t)n));
     SCN_TRY(g->dlKey.reserve((size_t)n));
     hipLaunchKernelGGL(k_download, dim3(scn_ceil_div(n, 256)), dim3(256), 0,
-                       ctx->stream, view_of(g), g->ekey.p, g->erow.p, n,
+                       ctx->stream, view_of(ctx, g), g->ekey.p, g->erow.p, n,
                        g->dlSample.p, g->dlKey.p, g->dlRow.p);
     SCN_HIP_CHECK(hipGetLastError());
     SCN_TRY(scn_d2h(ctx, h_sample, g->dlSample.p, n * sizeof(int)));
@@ -1862,7 +1916,7 @@ extern "C" int scn_grids_find(scn_ctx *ctx, const scn_grids *g,
     return SCN_OK;
   SCN_TRY(scn_grids_ensure_table(ctx, const_cast<scn_grids *>(g)));
   hipLaunchKernelGGL(k_find, dim3(scn_ceil_div(n, 256)), dim3(256), 0,
-                     ctx->stream, view_of(g), d_sample,
+                     ctx->stream, view_of(ctx, g), d_sample,
                      (const long long *)d_key, (long long)n, d_row);
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
@@ -1931,7 +1985,7 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   RankRows rows;
   SCN_TRY(ensure_index(ctx, in));
   SCN_TRY(missing_rank_rows(in, &rows));
-  GridView vin = view_of(in);
+  GridView vin = view_of(ctx, in);
   // number of candidates of one input: (ceil(size / stride))^d at most
   long long maxCand = 1;
   for (int a = 0; a < D; ++a)
@@ -2055,7 +2109,7 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
     mark_pending(ctx, out, slot);
   SCN_TRY(out->siteKey.reserve((size_t)nSites + 1));
   long long nThreads = nE > in->batch ? nE : in->batch;
-  GridView vout = view_of(out);
+  GridView vout = view_of(ctx, out);
   if (dilated)
     vout.bits = nullptr;
   if (tiled) {
@@ -2325,7 +2379,7 @@ extern "C" int scn_rules_terminal_plan(scn_ctx *ctx, const scn_grids *cin,
   const int slot = deferred ? (int)ctx->pendingGrids.size() : -1;
   const long long ticket = ++ctx->ticket;
   hipLaunchKernelGGL(k_terminal_plan, dim3(1), dim3(SCAN1_THREADS), 0, ctx->stream,
-                     view_of(in), out->sampleStart.p,
+                     view_of(ctx, in), out->sampleStart.p,
                      (long long *)ctx->d_pinned, ticket, out->meta.p,
                      in->pending ? in->meta.p : nullptr, boundWidth, slot);
   SCN_HIP_CHECK(hipGetLastError());
@@ -2341,7 +2395,7 @@ extern "C" int scn_rules_terminal_plan(scn_ctx *ctx, const scn_grids *cin,
     mark_pending(ctx, out, slot);
   if (in->batch > 0) {
     hipLaunchKernelGGL(k_terminal_out, dim3(scn_ceil_div(in->batch, 256)),
-                       dim3(256), 0, ctx->stream, view_of(out), out->ekey.p,
+                       dim3(256), 0, ctx->stream, view_of(ctx, out), out->ekey.p,
                        out->erow.p, out->bg.p);
     SCN_HIP_CHECK(hipGetLastError());
   }
@@ -2378,7 +2432,7 @@ extern "C" int scn_rules_fill(scn_ctx *ctx, const scn_grids *in,
               "the chain runs; plan again to fill another buffer");
   ProfScope ps(ctx, SCN_K_RULES);
   SCN_TRY(ensure_rank(ctx, const_cast<scn_grids *>(in)));
-  GridView vin = view_of(in);
+  GridView vin = view_of(ctx, in);
   if (out->planKind == PLAN_TERMINAL) {
     long long total = (long long)in->batch * out->termS;
     SCN_REQUIRE(capacity >= total, SCN_ERR_CAPACITY,

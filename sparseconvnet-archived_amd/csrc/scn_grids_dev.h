@@ -135,6 +135,14 @@ struct scn_grids {
   }
   // how much of table / bits is known to be empty right now (scn_grids_clear_many)
   size_t cleanSlots = 0, cleanWords = 0;
+  // Grids that are emptied by scn_grids_clear_many and built again batch after batch
+  // have a second mask, which the build of one batch empties and the next one takes
+  // (spareClean: it is empty, once the stream is through): emptying costs no launch.
+  // maskHeld: the first one's address is in a captured graph, and it stays.
+  unsigned long long *spare = nullptr;
+  size_t spareCap = 0;
+  bool spareClean = false, emptied = false;
+  mutable bool maskHeld = false;
   // Deferred counts: while pending, nActive / nSites / termS hold upper bounds
   // and the real values are in meta (device) and on their way to the pinned
   // slot; seen* are the largest values this object has ever held, from which
@@ -733,7 +741,9 @@ __device__ __forceinline__ int split_site(long long p, long long vol, int n,
 }
 
 // ---- host helpers shared by scn_grids.hip and scn_chain.hip
-GridView view_of(const scn_grids *g);
+// (what is launched while the stream is captured keeps the mask's address)
+void scn_grids_hold_mask(scn_ctx *ctx, const scn_grids *g);
+GridView view_of(scn_ctx *ctx, const scn_grids *g);
 long long grow_bound(long long &bound, long long seen, long long slack, long long cap);
 void mark_pending(scn_ctx *ctx, scn_grids *g, int slot);
 // fills the hash table of grids that do not have it yet (scn_grids.hip)
