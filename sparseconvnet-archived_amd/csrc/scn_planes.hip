@@ -1973,14 +1973,12 @@ static long long few_rows(scn_ctx *ctx, int planes, int K, int N) {
 // 26.1; 8000 x 1024 x 128 22.1, 16.4; 3000 x 768 x 320 17.3, 13.2; 5000 x 512 x 192 13.0,
 // 10.9; one plane 22.0, 15.2; 17.1, 12.1; 11.7, 9.3; 9.5, 8.3; 7.9, 7.4; W as it stands,
 // with nothing made before, 12383 x 448 x 64 14.4, 13.5, but 3909 x 256 x 160 9.7, 11.8:
-// below 448 k there is no more than a block or two to a wavefront.  One plane up to seven
-// eighths of the compute units: beyond, the tiles leave few of them idle and it gains less
-// (13.2, 11.0 with 247 of 256) than the launch that finds nothing, 4.6, costs batches near
-// the line.
+// below 448 k there is no more than a block or two to a wavefront.  One plane from 1024 k on:
+// below, it gains a microsecond or two (1152 x 800 x 800 12.8, 11.0), and a batch near the line
+// pays 4.6 for the launch that finds nothing.
 static long long split_rows(scn_ctx *ctx, int planes, int K, int N) {
-  const long long few = few_rows(ctx, planes, K, N);
-  const long long more = 64ll * ((planes == 1 ? ctx->numCU * 7 / 8 : ctx->numCU) / scn_ceil_div(N, 64));
-  return planes != 2 && K >= 448 && few > 0 && more > few ? more : few;
+  const long long few = few_rows(ctx, planes, K, N), more = 64ll * (ctx->numCU / scn_ceil_div(N, 64));
+  return planes != 2 && K >= (planes == 1 ? 1024 : 448) && few > 0 && more > few ? more : few;
 }
 
 struct PlanesChoice {
