@@ -328,6 +328,17 @@ int scn_conv_nin_forward_a16(scn_ctx *ctx, const float *d_in, int64_t nInRows,
                              int nIn, const float *d_W, const float *d_B,
                              const float *d_prelu, float *d_out, int64_t M,
                              int N, float p, int act);
+/* The same for rows that d_in16 holds rounded already, with an image of the weights
+ * (scn_weight_images_many, SCN_BF16) or null; and whether it is the faster of the
+ * two with that image, for a caller that can have the rows rounded on the way
+ * (scn_maxpool_rounded). */
+int scn_conv_nin_forward_rounded(scn_ctx *ctx, const float *d_in,
+                                 const void *d_in16, const int32_t *d_rules,
+                                 int fs, int nIn, const float *d_W,
+                                 const void *d_image, const float *d_B,
+                                 const float *d_prelu, float *d_out, int64_t M,
+                                 int N, float p, int act);
+int scn_rounded_rows_pay(scn_ctx *ctx, int64_t M, int fs, int nIn, int N);
 /* maxPool (MaxPoolingLayer.h:6-7; MaxPoolingLayer.cu:9-72): first maximum
  * wins, negative rules skipped, choice = rule * C + channel. */
 int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
@@ -339,6 +350,11 @@ int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
  * refused with SCN_ERR_CAPACITY instead of being indexed modulo 2^32. */
 int scn_maxpool_checked(scn_ctx *ctx, const float *d_in, int64_t nInRows,
                         float *d_out, const int32_t *d_rules,
+                        int64_t nOutSites, int ps, int C, int32_t *d_choice);
+/* ... and d_out rounded to bf16 in d_out16 (or null), for C a multiple of 4 and
+ * buffers on 16 bytes. */
+int scn_maxpool_rounded(scn_ctx *ctx, const float *d_in, int64_t nInRows,
+                        float *d_out, void *d_out16, const int32_t *d_rules,
                         int64_t nOutSites, int ps, int C, int32_t *d_choice);
 /* terminalPool (TerminalPoolingLayer.cu:22-46): mean over the rows listed
  * before the first negative rule, summed in rule order. */

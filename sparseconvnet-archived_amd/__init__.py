@@ -151,6 +151,9 @@ def lib():
         "scn_conv_nin_forward_a16": (C.c_int, [vp, vp, i64, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, i64, C.c_int, f32,
                                                C.c_int]),
         "scn_maxpool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int, vp]),
+        "scn_conv_nin_forward_rounded": (C.c_int, [vp, vp, vp, vp, C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, C.c_int, f32, C.c_int]),
+        "scn_rounded_rows_pay": (C.c_int, [vp, i64, C.c_int, C.c_int, C.c_int]),
+        "scn_maxpool_rounded": (C.c_int, [vp, vp, i64, vp, vp, vp, i64, C.c_int, C.c_int, vp]),
         "scn_maxpool_checked": (C.c_int, [vp, vp, i64, vp, vp, i64, C.c_int, C.c_int, vp]),
         "scn_terminal_pool": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int]),
         "scn_terminal_classifier_supported": (C.c_int, [i64, C.c_int, C.c_int]),
@@ -363,6 +366,16 @@ class Context:
         _check(lib().scn_conv_nin_forward_a16(self.h, d_in.ptr, nInRows, d_in16.ptr, d_rules.ptr, fs, nIn, d_W.ptr,
                                               d_B.ptr, d_prelu.ptr if d_prelu is not None else None, d_out.ptr, M, N,
                                               p, act))
+
+    def conv_nin_forward_rounded(self, d_in, d_in16, d_rules, fs, nIn, d_W, d_image, d_B, d_prelu, d_out, M, N, p=1.0, act=RELU):
+        """conv_nin_forward_image at BF16 of rows that are rounded already (maxpool_rounded)"""
+        _check(lib().scn_conv_nin_forward_rounded(self.h, d_in.ptr, d_in16.ptr, d_rules.ptr, fs, nIn, d_W.ptr,
+                                                  d_image.ptr if d_image is not None else None, d_B.ptr,
+                                                  d_prelu.ptr if d_prelu is not None else None, d_out.ptr, M, N, p, act))
+
+    def maxpool_rounded(self, d_in, nInRows, d_out, d_out16, d_rules, nOutSites, ps, Cn, d_choice):
+        _check(lib().scn_maxpool_rounded(self.h, d_in.ptr, nInRows, d_out.ptr, d_out16.ptr if d_out16 is not None else None,
+                                         d_rules.ptr, nOutSites, ps, Cn, d_choice.ptr))
 
     def maxpool(self, d_in, d_out, d_rules, nOutSites, ps, Cn, d_choice):
         _check(lib().scn_maxpool(self.h, d_in.ptr, d_out.ptr, d_rules.ptr, nOutSites, ps, Cn, d_choice.ptr))

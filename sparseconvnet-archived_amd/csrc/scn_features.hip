@@ -2,6 +2,7 @@
 // average, softmax.  All of them move bytes: they are sized and indexed for
 // HBM bandwidth (128-bit accesses wherever the channel count allows, rule
 // offsets staged in LDS, 64-bit element offsets).
+#include "scn_nin_dev.h"
 #include "scn_common.h"
 
 #define GATHER_TILE 256 // rules per block iteration
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(256)
     k_maxpool(const float *__restrict__ in, float *__restrict__ out,
               const int *__restrict__ rules, long long bound, int ps,
               int C, int chunks, PoolDivisor div, int *__restrict__ choice,
-              const float *__restrict__ spare, const long long *dRows) {
+              const float *__restrict__ spare, const long long *dRows, uint2 *__restrict__ out16) {
   __shared__ int sRules[PS ? MP_RULES : 1];
   if (PS)
     ps = PS;
@@ -207,15 +208,16 @@ __global__ void __launch_bounds__(256)
         make_float4(best[0], best[1], best[2], best[3]);
     *reinterpret_cast<int4 *>(choice + o) =
         make_int4(arg[0], arg[1], arg[2], arg[3]);
+    if (out16) // uniform
+      out16[o / 4] = make_uint2(pack_bf16x2(best[0], best[1]), pack_bf16x2(best[2], best[3]));
   } else {
     out[o] = best[0];
     choice[o] = arg[0];
   }
 }
 
-extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
-                           const int32_t *d_rules, int64_t nOutSites, int ps,
-                           int C, int32_t *d_choice) {
+static int maxpool(scn_ctx *ctx, const float *d_in, float *d_out, const int32_t *d_rules, int64_t nOutSites, int ps,
+                   int C, int32_t *d_choice, void *d_out16) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_maxpool: null context");
   SCN_REQUIRE(nOutSites >= 0 && ps >= 1 && C >= 1, SCN_ERR_ARG,
               "scn_maxpool: nOutSites %lld ps %d C %d", (long long)nOutSites,
@@ -228,6 +230,8 @@ extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
   ProfScope prof(ctx, SCN_K_MAXPOOL);
   const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   const bool wide = C % 4 == 0 && aligned16(d_in) && aligned16(d_out) && aligned16(d_choice);
+  SCN_REQUIRE(!d_out16 || (wide && ((uintptr_t)d_out16 & 7) == 0), SCN_ERR_ARG,
+              "scn_maxpool_rounded: %d features, or a buffer that does not start on 16 bytes", C);
   const int chunks = wide ? C / 4 : C;
   const long long total = nOutSites * chunks;
   PoolDivisor div = {0u, 0};
@@ -240,7 +244,7 @@ extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
   const bool fits = (256 / chunks + 2ll) * ps <= MP_RULES;
 #define SCN_MP_GO(VEC, PS)                                                                                       \
   hipLaunchKernelGGL((k_maxpool<VEC, PS>), dim3(scn_ceil_div(total, 256)), dim3(256), 0, ctx->stream, d_in, d_out, \
-                     d_rules, (long long)nOutSites, ps, C, chunks, div, d_choice, (const float *)ctx->d_zeros, dRows)
+                     d_rules, (long long)nOutSites, ps, C, chunks, div, d_choice, (const float *)ctx->d_zeros, dRows, (uint2 *)d_out16)
   if (!wide)
     SCN_MP_GO(1, 0);
   else if (fits && ps == 9)
@@ -256,17 +260,26 @@ extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out,
   return SCN_OK;
 }
 
+extern "C" int scn_maxpool(scn_ctx *ctx, const float *d_in, float *d_out, const int32_t *d_rules, int64_t nOutSites,
+                           int ps, int C, int32_t *d_choice) {
+  return maxpool(ctx, d_in, d_out, d_rules, nOutSites, ps, C, d_choice, nullptr);
+}
+
 extern "C" int scn_maxpool_checked(scn_ctx *ctx, const float *d_in,
                                    int64_t nInRows, float *d_out,
                                    const int32_t *d_rules, int64_t nOutSites,
                                    int ps, int C, int32_t *d_choice) {
+  return scn_maxpool_rounded(ctx, d_in, nInRows, d_out, nullptr, d_rules, nOutSites, ps, C, d_choice);
+}
+extern "C" int scn_maxpool_rounded(scn_ctx *ctx, const float *d_in, int64_t nInRows, float *d_out, void *d_out16,
+                                   const int32_t *d_rules, int64_t nOutSites, int ps, int C, int32_t *d_choice) {
   SCN_REQUIRE(nInRows >= 0 && C >= 1, SCN_ERR_ARG,
               "scn_maxpool_checked: nInRows %lld C %d", (long long)nInRows, C);
   SCN_REQUIRE(nInRows * (int64_t)C <= 2147483647ll, SCN_ERR_CAPACITY,
               "scn_maxpool: %lld input rows of %d features are %lld elements; "
               "the 32-bit pooling choices index at most 2^31 - 1",
               (long long)nInRows, C, (long long)(nInRows * (int64_t)C));
-  return scn_maxpool(ctx, d_in, d_out, d_rules, nOutSites, ps, C, d_choice);
+  return maxpool(ctx, d_in, d_out, d_rules, nOutSites, ps, C, d_choice, d_out16);
 }
 
 // dTerminalPool (TerminalPoolingLayer.cu:22-34): sequential fp32 sum in rule

@@ -2185,14 +2185,13 @@ int scn_planes_forward(scn_ctx *ctx, int planes, const float *A, const float *W,
   choice.given = (const unsigned char *)image;
   const bool room = planes_image(ctx);
   choice.image = choice.image && room;
-  // (bf16 rows: a block takes half a line of each; long contractions, of 27
-  // positions, stay ahead in k_nin_planes: 595000 x 2592 x 128 444 us against 474.
-  // k_nin_planes' cost is 2 too high where it converts W on the way, of layers that
-  // small.)
+  // (bf16 rows: a block takes half a line of each.  k_nin_planes' cost is 2 too high where
+  // it converts W on the way, of layers that small.  Long contractions of few rows: 8000 x
+  // 1536 x 256 23.4 -> 17.1 us, 6000 x 1920 x 640 40 -> 27.6, 20000 x 1728 x 128 38 -> 21.)
   if (a16 && choice.tile >= 0 && N > 32 && lines_shape(1, K, N, gs->nIn) &&
       (image || (room && image_bytes(1, K, N) <= (int64_t)SCN_IMAGE_BYTES))) {
     choice.rows16 = rows16_tiles(ctx->numCU, rows, K, N);
-    if (choice.rows16 == 0 && K <= 1280 &&
+    if (choice.rows16 == 0 &&
         lines_rows16(ctx, rows, K, N, image != nullptr) < choice.cost - (choice.image ? 0.f : 2.f))
       choice.lines = N <= 64 ? 4 : 3;
     if (choice.rows16 || choice.lines >= 0)
@@ -2223,6 +2222,19 @@ extern "C" int64_t scn_weight_image_bytes(scn_ctx *ctx, int64_t M, int K, int N,
   if (nIn != K && lines_choose(ctx->numCU, planes, hint, K, N, true, &tile) >= choice.cost + 2.f)
     return 0;
   return image_bytes(planes, K, N);
+}
+// Rows that a pooling has rounded on the way (2 bytes more of the some 24 to 44 that it
+// moves for a feature), us of fp32 rows and of these, with the image: 41600 x 640 x 320 36, 31;
+// 10500 x 1280 x 480 29.5, 24.7; 26000 x 1280 x 480 60, 39; 110000 x 512 x 160 60, 39; 60000 x
+// 256 x 96 12.8, 11.1; 90000 x 512 x 96 of eight positions 30, 19.7.  Below 2e9 products it is a
+// microsecond or none (26000 x 384 x 128 10.3, 9.3; 6000 x 896 x 256 11.3, 11.8), and longer ones
+// need the rows for k_nin_rows16 (10500 x 1920 x 640 46, 33; 8000 42, 32.5; 6000 26, 28; 6000 x
+// 2560 x 800 50, 40; 4500 33, 39; 30000 x 2592 x 128 37, 42).
+extern "C" int scn_rounded_rows_pay(scn_ctx *ctx, int64_t M, int fs, int nIn, int N) {
+  if (!ctx || M < 1 || fs < 1 || nIn < 1 || N < 1 || !lines_shape(1, fs * nIn, N, nIn))
+    return 0;
+  const long long rows = scn_rows_hint(ctx, M), K = (long long)fs * nIn;
+  return (double)rows * K * N >= 2e9 && (K <= 1280 || tiles_of(rows, 256) * tiles_of(N, 128) >= .6 * ctx->numCU);
 }
 static int image_list(scn_ctx *ctx, const scn_image_item *items, int nItems, ImageList &l) {
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_weight_images_many: null context");

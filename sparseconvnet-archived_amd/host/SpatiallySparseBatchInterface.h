@@ -12,10 +12,12 @@ public:
   vectorCUDA<float> dfeatures; // gradient of the cost, training batches only
   vectorCUDA<float> dactivated; // of a pooling's output: that, times the derivative of the layer below
   vectorCUDA<int> poolingChoices;
-  // room for a bf16 copy of `features` (two bytes an element), made by a
-  // following fused convolution with bf16 operands whose window is large
-  // enough for the rows to be read many times over
+  // room for a bf16 copy of `features` (two bytes an element), for a following fused
+  // convolution with bf16 operands: made by it, where its window is large enough for
+  // the rows to be read many times over, or
   vectorCUDA<float> features16;
+  // by the pooling that makes the features: is to be, and has been in this pass
+  bool roundedToo = false, rounded = false;
   // the weights of the layer whose output this is, laid out for its forward pass
   // and, turned round, for the gradient of its input: made for one batch by
   // SparseConvNetCUDA::makeWeightImages, in the stream's room for them, and used up

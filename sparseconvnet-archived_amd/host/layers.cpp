@@ -340,9 +340,10 @@ static void nin_weight_images(SpatiallySparseBatch &batch, cudaMemStream &ms, Sp
                               SpatiallySparseBatchInterface &output, const SpatiallySparseBatchInterface *before,
                               vectorCUDA<float> &W, int K, int N, int precision, std::vector<WeightImage> &items) {
   const int nIn = before ? before->nFeatures : K, fs = K / nIn, p = abi_precision(precision);
-  const int64_t bytes = before && rounds_rows(precision, fs, nIn, output.nSpatialSites)
-                            ? 0
-                            : scn_weight_image_bytes(ms.ctx, output.nSpatialSites, K, N, nIn, p);
+  const bool rounds = before && rounds_rows(precision, fs, nIn, output.nSpatialSites);
+  const int64_t bytes = rounds ? 0 : scn_weight_image_bytes(ms.ctx, output.nSpatialSites, K, N, nIn, p);
+  if (before && p == SCN_BF16 && nIn % 8 == 0)
+    before->sub->roundedToo = rounds || (bytes && scn_rounded_rows_pay(ms.ctx, output.nSpatialSites, fs, nIn, N));
   if (bytes)
     items.push_back({{W.dPtr(), nullptr, K, N, 0, p}, bytes, &output.sub->weightImage});
   if (batch.type != TRAINBATCH || !input.leftOut || !before || !before->backpropErrors)
@@ -378,6 +379,13 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
   if (!scn_conv_nin_supported_p(fs, nIn, nFeaturesOut, precision)) {
     gather_now(ms, *src, input);
     return false;
+  }
+  if (src->sub->rounded && precision == SCN_BF16) {
+    SCN_CHECKED(scn_conv_nin_forward_rounded(
+        ms.ctx, src->sub->features.dPtr(), src->sub->features16.dPtr(), input.rules.dPtr(), fs, nIn, W.dPtr(), image,
+        B.dPtr(), prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(), output.nSpatialSites, nFeaturesOut, p,
+        act));
+    return true;
   }
   if (rounds_rows(precision, fs, nIn, output.nSpatialSites)) {
     const size_t elems = (size_t)src->nSpatialSites * nIn;
@@ -887,9 +895,13 @@ static void pool_forwards(cudaMemStream &ms,
   const size_t nf = output.featuresPresent.size();
   output.sub->poolingChoices.resize64((size_t)output.nSpatialSites * nf, kBoundRows * nf);
   output.sub->features.resize64((size_t)output.nSpatialSites * nf, kBoundRows * nf);
-  SCN_CHECKED(scn_maxpool_checked(ms.ctx, input.sub->features.dPtr(),
+  output.sub->rounded = output.sub->roundedToo && nf % 8 == 0;
+  if (output.sub->rounded)
+    output.sub->features16.resize64((size_t)output.nSpatialSites * nf / 2 + 8, kBoundRows * nf / 2);
+  SCN_CHECKED(scn_maxpool_rounded(ms.ctx, input.sub->features.dPtr(),
                                   input.nSpatialSites,
                                   output.sub->features.dPtr(),
+                                  output.sub->rounded ? output.sub->features16.dPtr() : nullptr,
                                   output.rules.dPtr(), output.nSpatialSites,
                                   width, (int)nf,
                                   output.sub->poolingChoices.dPtr()));

@@ -533,6 +533,7 @@ void SparseConvNetCUDA::makeWeightImages(SpatiallySparseBatch &batch, cudaMemStr
   for (size_t i = 0; i < layers.size(); i++) {
     SpatiallySparseBatchInterface &input = batch.interfaces[i], &output = batch.interfaces[i + 1];
     output.sub->weightImage = output.sub->turnedImage = nullptr;
+    output.sub->roundedToo = output.sub->rounded = false;
     if (batch.type == RESCALEBATCH) // (whose weights change on the way)
       continue;
     if (batch.countsPending)
@@ -620,8 +621,10 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   }
   if (batch.countsPending)
     SCN_CHECKED(scn_ctx_rows_from(ms.ctx, nullptr));
-  for (size_t i = 1; i < batch.interfaces.size(); i++) // (what no layer has taken)
+  for (size_t i = 1; i < batch.interfaces.size(); i++) { // (what no layer has taken)
     batch.interfaces[i].sub->weightImage = nullptr;
+    batch.interfaces[i].sub->roundedToo = batch.interfaces[i].sub->rounded = false;
+  }
   // what no launch has made (a batch of no rows) does not outlast the pass
   if (batch.type != TRAINBATCH)
     SCN_CHECKED(scn_weight_images_later(ms.ctx, nullptr, 0));
