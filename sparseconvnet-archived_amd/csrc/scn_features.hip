@@ -5,28 +5,31 @@
 #include "scn_nin_dev.h"
 #include "scn_common.h"
 
-#define GATHER_TILE 256 // rules per block iteration
+#define GATHER_TILE 256 // rules per block iteration at most
 #define GATHER_THREADS 256
 
 // out[c * nIn + j] = in[rules[c] * nIn + j]   (ConvolutionalLayer.cu:12-31)
 // The output is one contiguous run per tile, so consecutive lanes write
 // consecutive 16-byte chunks; reads are contiguous per rule.  A negative rule
 // (the reference reads out of bounds on one) gathers a row of zeros.
+// `tile`: rules a workgroup takes at a time.  What it waits for is a trip to the rules and
+// one to the rows for every four loads of a lane: fewer rules, down to four loads, where
+// there are not as many workgroups as compute units (us, with 256 and so: 2000 rows of 8 x
+// 128 6.6, 4.9; 60 of 8 x 160 6.5, 4.8; with more workgroups it loses: 30000 of 4 x 64 7.9, 8.5).
 template <typename VecT, int VEC>
 __global__ void __launch_bounds__(GATHER_THREADS)
     k_gather(const float *__restrict__ in, float *__restrict__ out,
              const int *__restrict__ rules, long long count, int nIn,
-             int chunks, const long long *dRows, int perRow) {
+             int chunks, const long long *dRows, int perRow, int tile) {
   if (dRows)
     count = live_rows(count / perRow, dRows) * perRow;
   __shared__ long long roff[GATHER_TILE];
   const int tid = threadIdx.x;
   const int q0 = tid / chunks, ch0 = tid - q0 * chunks;
   const int dq = GATHER_THREADS / chunks, dch = GATHER_THREADS - dq * chunks;
-  for (long long c0 = (long long)blockIdx.x * GATHER_TILE; c0 < count;
-       c0 += (long long)gridDim.x * GATHER_TILE) {
+  for (long long c0 = (long long)blockIdx.x * tile; c0 < count; c0 += (long long)gridDim.x * tile) {
     long long left = count - c0;
-    const int n = left < GATHER_TILE ? (int)left : GATHER_TILE;
+    const int n = left < tile ? (int)left : tile;
     if (tid < n) {
       int rule = rules[c0 + tid];
       roff[tid] = rule < 0 ? -1 : (long long)rule * nIn;
@@ -87,17 +90,22 @@ extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
   // (rows not known on the host yet: count is their bound times the rule width)
   const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   const int perRow = dRows && ctx->rowsBound > 0 ? (int)(count / ctx->rowsBound) : 1;
-  long long tiles = (count + GATHER_TILE - 1) / GATHER_TILE;
-  long long maxBlocks = (long long)ctx->numCU * 16;
+  const bool wide = nIn % 4 == 0 && aligned16(d_in) && aligned16(d_out);
+  const int chunks = wide ? nIn / 4 : nIn;
+  const long long maxBlocks = (long long)ctx->numCU * 16;
+  int tile = GATHER_TILE;
+  while (tile > 16 && tile * chunks > 4 * GATHER_THREADS && (count + tile - 1) / tile < ctx->numCU)
+    tile /= 2;
+  const long long tiles = (count + tile - 1) / tile;
   int blocks = (int)(tiles < maxBlocks ? tiles : maxBlocks);
-  if (nIn % 4 == 0 && aligned16(d_in) && aligned16(d_out)) {
+  if (wide) {
     hipLaunchKernelGGL((k_gather<float4, 4>), dim3(blocks),
                        dim3(GATHER_THREADS), 0, ctx->stream, d_in, d_out,
-                       d_rules, (long long)count, nIn, nIn / 4, dRows, perRow);
+                       d_rules, (long long)count, nIn, chunks, dRows, perRow, tile);
   } else {
     hipLaunchKernelGGL((k_gather<float, 1>), dim3(blocks),
                        dim3(GATHER_THREADS), 0, ctx->stream, d_in, d_out,
-                       d_rules, (long long)count, nIn, nIn, dRows, perRow);
+                       d_rules, (long long)count, nIn, chunks, dRows, perRow, tile);
   }
   SCN_HIP_CHECK(hipGetLastError());
   return SCN_OK;
