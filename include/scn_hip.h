@@ -121,6 +121,10 @@ int scn_d2d(scn_ctx *ctx, void *d_dst, const void *d_src, size_t bytes);
  * host memory (scn_host_alloc) that the device reaches over the bus: an
  * upload or download that costs the host one kernel launch. */
 int scn_copy(scn_ctx *ctx, void *dst, const void *src, size_t bytes);
+/* up to SCN_COPY_MAX of these in one launch, none overlapping another */
+#define SCN_COPY_MAX 8
+int scn_copy_many(scn_ctx *ctx, void *const *dst, const void *const *src,
+                  const size_t *bytes, int n);
 int scn_fill32(scn_ctx *ctx, void *d_dst, uint32_t word, size_t nWords);
 /* up to SCN_FILL_MAX buffers in one launch */
 #define SCN_FILL_MAX 32

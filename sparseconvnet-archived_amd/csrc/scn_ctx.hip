@@ -256,6 +256,45 @@ extern "C" int scn_copy(scn_ctx *c, void *dst, const void *src, size_t bytes) {
   return SCN_OK;
 }
 
+// Several at once, a row of workgroups each
+struct CopyList {
+  const uint8_t *src[SCN_COPY_MAX];
+  uint8_t *dst[SCN_COPY_MAX];
+  size_t bytes[SCN_COPY_MAX];
+};
+__global__ __launch_bounds__(256) void k_copy_many(CopyList l) {
+  const uint8_t *const src = l.src[blockIdx.y];
+  uint8_t *const dst = l.dst[blockIdx.y];
+  const size_t bytes = l.bytes[blockIdx.y], n16 = (((uintptr_t)src | (uintptr_t)dst) & 15) ? 0 : bytes / 16;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  for (size_t k = i; k < n16; k += step)
+    reinterpret_cast<uint4 *>(dst)[k] = reinterpret_cast<const uint4 *>(src)[k];
+  for (size_t k = n16 * 16 + i; k < bytes; k += step)
+    dst[k] = src[k];
+}
+extern "C" int scn_copy_many(scn_ctx *c, void *const *dst, const void *const *src, const size_t *bytes, int n) {
+  SCN_REQUIRE(c, SCN_ERR_ARG, "scn_copy_many: null context");
+  SCN_REQUIRE(n >= 0 && n <= SCN_COPY_MAX && (n == 0 || (dst && src && bytes)), SCN_ERR_ARG,
+              "scn_copy_many: %d copies (at most %d)", n, SCN_COPY_MAX);
+  CopyList l;
+  size_t most = 0;
+  int m = 0;
+  for (int k = 0; k < n; ++k) {
+    if (bytes[k] == 0)
+      continue;
+    SCN_REQUIRE(dst[k] && src[k], SCN_ERR_ARG, "scn_copy_many: null buffer %d", k);
+    l.dst[m] = (uint8_t *)dst[k], l.src[m] = (const uint8_t *)src[k], l.bytes[m++] = bytes[k];
+    most = bytes[k] > most ? bytes[k] : most;
+  }
+  if (m == 0)
+    return SCN_OK;
+  size_t blocks = (most / 16 + 255) / 256;
+  blocks = blocks < 1 ? 1 : (blocks > 4096 ? 4096 : blocks);
+  hipLaunchKernelGGL(k_copy_many, dim3((unsigned)blocks, (unsigned)m), dim3(256), 0, c->stream, l);
+  SCN_HIP_CHECK(hipGetLastError());
+  return SCN_OK;
+}
+
 extern "C" int scn_d2d(scn_ctx *c, void *d_dst, const void *d_src,
                        size_t bytes) {
   return scn_copy(c, d_dst, d_src, bytes);
