@@ -1274,7 +1274,7 @@ static bool dense_rows(const scn_grids *g) {
 }
 
 void scn_grids_hold_mask(scn_ctx *ctx, const scn_grids *g) {
-  if (g->maskHeld)
+  if (g->maskHeld || !g->emptied)
     return;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess)
@@ -1427,14 +1427,16 @@ extern "C" int scn_grids_clear_many(scn_ctx *ctx, scn_grids **grids, int n) {
     size_t most = 0;
     for (int i = first; i < n && i < first + CLEAR_MANY; ++i) {
       scn_grids *g = grids[i];
-      if (!g || (!g->table.p && !g->bits.p))
+      if (!g || (!g->table.p && !g->bits.p)) {
+        if (g)
+          g->emptied = true;
         continue;
+      }
       // nothing to do for grids whose table and mask are not in use (a chain
       // of recorded plans fills the entry list only) or are empty already
       if (!g->indexValid || ((!g->table.p || g->cleanSlots >= g->table.cap) &&
                              (!g->bits.p || g->cleanWords >= g->bits.cap)))
         continue;
-      g->emptied = true;
       scn_grids_hold_mask(ctx, g);
       if (g->spare && g->spareClean && g->spareCap == g->bits.cap && !g->maskHeld &&
           (!g->table.p || g->cleanSlots >= g->table.cap)) { // (what was in use: emptied by the build)
