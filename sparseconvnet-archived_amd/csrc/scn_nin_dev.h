@@ -85,5 +85,6 @@ int scn_images_now(scn_ctx *ctx);
 int scn_atb_planes_many(scn_ctx *ctx, const scn_atb_item *items, int nItems);
 // out = A Wt^T; false: the caller's other way, or (transpose) scn_planes_forward
 // on the transpose
+bool scn_abt_narrow(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int n, int K);
 bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
                     long long M, int K, int N, const Epilogue &ep, int *rc, bool *transpose);

@@ -2310,6 +2310,130 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
   return true;
 }
 
+// out = A W^T for A [M x n], W [K x n] of no more than 32 columns: a gradient by a layer
+// of few outputs.  What bounds it is writing out.  A wavefront has 64 rows of A as planes
+// in its registers and goes through the rows of W, 32 at a time, which are split as they
+// come, the next ones under way; twelve MFMAs make 4 KB of out.
+// Behind it the fp32 kernel for short contractions, which keeps to vector instructions, us:
+// 118144 x 896 of 32 249 -> 105 (4.0 TB/s), 30000 x 864 67 -> 28, 100000 x 128 36 -> 16, 9000 x 64 8.5 -> 7.1,
+// 40000 x 512 of 16 35 -> 21; of 1000 rows 8.8, 10.0 (the line: 2048).  The error against 64 bits
+// is 0.4 of its.  The results go past the caches (through them 114).
+constexpr int NARROW_MT = 2, NARROW_WAVES = 4;
+__global__ void __launch_bounds__(64 * NARROW_WAVES, 2)
+    k_abt_narrow(const float *__restrict__ A, const float *__restrict__ W, float *__restrict__ out, long long M, int n, int K,
+                 int tiles) { // (of columns, to a workgroup)
+  constexpr int PL = 3, MT = NARROW_MT;
+  const int lane = threadIdx.x & 63, c = lane & 31, q = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned at = xcd_eighth(blockIdx.x, gridDim.x);
+  const long long row0 = ((long long)at * NARROW_WAVES + wave) * 32 * MT;
+  if (row0 >= M) // (no barrier below)
+    return;
+  bf16x8 a[MT][2][PL];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const long long r = row0 + 32 * i + c < M ? row0 + 32 * i + c : M - 1; // (not stored)
+      const int k = 16 * s + 8 * q;
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (k < n) {
+        const floatx4 x = *reinterpret_cast<const floatx4 *>(A + r * n + k), y = *reinterpret_cast<const floatx4 *>(A + r * n + k + 4);
+        v[0] = x[0], v[1] = x[1], v[2] = x[2], v[3] = x[3], v[4] = y[0], v[5] = y[1], v[6] = y[2], v[7] = y[3];
+      }
+      split8<PL>(v, a[i][s]);
+    }
+  const int t0 = blockIdx.y * tiles, all = (K + 31) / 32, t1 = t0 + tiles < all ? t0 + tiles : all;
+  const bool whole = row0 + 32 * MT <= M; // uniform
+  const unsigned place = 4 * q * (unsigned)K + c; // this lane's in a tile
+  floatx4 raw[2][2];
+  auto load = [&](int t) {
+    const int row = 32 * t + c < K ? 32 * t + c : K - 1; // (not stored)
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = 16 * s + 8 * q;
+        raw[s][h] = k < n ? *reinterpret_cast<const floatx4 *>(W + (long long)row * n + k + 4 * h) : floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  load(t0);
+#pragma unroll 1
+  for (int t = t0; t < t1; ++t) {
+    bf16x8 b[2][PL];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const float v[8] = {raw[s][0][0], raw[s][0][1], raw[s][0][2], raw[s][0][3], raw[s][1][0], raw[s][1][1], raw[s][1][2], raw[s][1][3]};
+      split8<PL>(v, b[s]);
+    }
+    load(t + 1 < t1 ? t + 1 : t);
+    floatx16 acc[2][MT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[h][i][v] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int x = 0; x < PL; ++x)
+#pragma unroll
+        for (int y = 0; x + y < PL; ++y)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) {
+            floatx16 &d = acc[x + y == 0 ? 0 : 1][i];
+            d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][s][x], b[s][y], d, 0, 0, 0);
+          }
+    float none[4] = {0.f, 0.f, 0.f, 0.f}; // 0 sum: NaN for a sum that is not finite
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[0][i][v] += acc[1][i][v];
+        none[v % 4] = fmaf(acc[0][i][v], 0.f, none[v % 4]);
+      }
+    const int col = 32 * t + c;
+    if (__any((none[0] + none[1]) + (none[2] + none[3]) != 0.f)) { // these rows and columns as fp32 has them
+      for (int x = 0; x < 16 * MT && col < K; ++x) {
+        const long long row = row0 + 2 * x + q;
+        if (row >= M)
+          break;
+        float sum = 0.f;
+        for (int k = 0; k < n; ++k)
+          sum = fmaf(A[row * n + k], W[(long long)col * n + k], sum);
+        out[row * K + col] = sum;
+      }
+      continue;
+    }
+    if (col < K) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int r = 32 * i + 8 * (v / 4) + v % 4; // uniform
+          if (whole || row0 + r + 4 * q < M)
+            __builtin_nontemporal_store(acc[0][i][v], out + (row0 + r) * K + 32 * t + place);
+        }
+    }
+  }
+}
+// Whether it is one for this; then it has been launched
+bool scn_abt_narrow(scn_ctx *ctx, const float *A, const float *W, float *out, long long M, int n, int K) {
+  if (n > 32 || n % 8 || (((uintptr_t)A | (uintptr_t)W) & 15) || M < 2048 || M >= 1ll << 32 || K < 64 || K > 1 << 24)
+    return false;
+  const long long groups = (M + 32 * NARROW_MT * NARROW_WAVES - 1) / (32 * NARROW_MT * NARROW_WAVES);
+  const int all = (K + 31) / 32;
+  // (two workgroups a compute unit, of four tiles of columns at least)
+  int parts = (int)std::max<long long>(1, std::min<long long>((2 * ctx->numCU + groups - 1) / groups, all / 4));
+  const int tiles = (all + parts - 1) / parts;
+  parts = (all + tiles - 1) / tiles;
+  hipLaunchKernelGGL(k_abt_narrow, dim3((unsigned)groups, (unsigned)parts), dim3(64 * NARROW_WAVES), 0, ctx->stream, A, W, out,
+                     M, n, K, tiles);
+  return true;
+}
+
 // ------------------------------------------------------- dW = A^T D in planes
 // The contraction runs over the rows of both matrices, so an MFMA operand is
 // eight consecutive rows of one column: dword loads (pairs of columns for two
