@@ -74,6 +74,24 @@ __global__ void __launch_bounds__(GATHER_THREADS)
   }
 }
 
+// Rows of one word: four rules to a lane and nothing in LDS (21.5 M rules 46 us, 69 beside what
+// a layer does before it, -> 30; 900000 5.5 -> 5.2)
+__global__ void __launch_bounds__(256)
+    k_gather_words(const float *__restrict__ in, float *__restrict__ out, const int *__restrict__ rules, long long count,
+                   const long long *dRows, int perRow) {
+  if (dRows)
+    count = live_rows(count / perRow, dRows) * perRow;
+  const long long at = 4 * ((long long)xcd_eighth(blockIdx.x, gridDim.x) * 256 + threadIdx.x);
+  if (at + 4 <= count) {
+    const int4 r = *reinterpret_cast<const int4 *>(rules + at);
+    *reinterpret_cast<float4 *>(out + at) = make_float4(r.x < 0 ? 0.f : in[r.x], r.y < 0 ? 0.f : in[r.y], r.z < 0 ? 0.f : in[r.z],
+                                                        r.w < 0 ? 0.f : in[r.w]);
+  } else {
+    for (long long i = at; i < count; ++i)
+      out[i] = rules[i] < 0 ? 0.f : in[rules[i]];
+  }
+}
+
 static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
@@ -90,6 +108,12 @@ extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
   // (rows not known on the host yet: count is their bound times the rule width)
   const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   const int perRow = dRows && ctx->rowsBound > 0 ? (int)(count / ctx->rowsBound) : 1;
+  if (nIn == 1 && aligned16(d_rules) && aligned16(d_out) && count < (long long)1 << 40) {
+    hipLaunchKernelGGL(k_gather_words, dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, ctx->stream, d_in, d_out, d_rules,
+                       (long long)count, dRows, perRow);
+    SCN_HIP_CHECK(hipGetLastError());
+    return SCN_OK;
+  }
   const bool wide = nIn % 4 == 0 && aligned16(d_in) && aligned16(d_out);
   const int chunks = wide ? nIn / 4 : nIn;
   const long long maxBlocks = (long long)ctx->numCU * 16;

@@ -503,6 +503,71 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Rows of up to GR_MAX_K columns in other than fours, the matrix of a first layer's window of
+// three: the products of k_nin_generic in its order.  A workgroup's 64 rows are one piece
+// of memory, whole requests of it, and lie in LDS as they are; a lane has four columns
+// of four rows (up to 32 columns: of two).  us, k_nin_generic and this: 797192 x 27 x 64 136, 105;
+// 175934 x 27 x 64 32, 23; 100000 x 18 x 160 46, 32; 60000 x 54 x 32 16.6, 9.4; 40000 x 81 x 128 31, 27;
+// 3000 x 27 x 32 10, 5.6.
+#define GR_MAX_K 128
+template <int QUADS>
+__global__ void __launch_bounds__(256) k_nin_rows(const float *__restrict__ A, const float *__restrict__ W, float *__restrict__ out,
+                                                  long long M, int K, int N, Epilogue ep) {
+  constexpr int ROWS = 64, GROUPS = 256 / QUADS, R = ROWS / GROUPS, COLS = 4 * QUADS;
+  extern __shared__ __attribute__((aligned(16))) float grLds[]; // [ROWS][K], [K][COLS]
+  float *const sW = grLds + ROWS * K;
+  const int tid = threadIdx.x, quad = tid % QUADS, group = tid / QUADS, n0 = blockIdx.y * COLS;
+  const long long m0 = (long long)xcd_eighth(blockIdx.x, gridDim.x) * ROWS;
+  const float *const from = A + m0 * K;
+  const long long left = (M - m0) * K;
+  const int floats = left < ROWS * K ? (int)left : ROWS * K;
+  for (int i = 4 * tid; i < ROWS * K; i += 1024) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i + 4 <= floats) {
+      v = *reinterpret_cast<const float4 *>(from + i);
+    } else {
+      v.x = i < floats ? from[i] : 0.f;
+      v.y = i + 1 < floats ? from[i + 1] : 0.f;
+      v.z = i + 2 < floats ? from[i + 2] : 0.f;
+    }
+    *reinterpret_cast<float4 *>(grLds + i) = v;
+  }
+  for (int i = tid; i < K * QUADS; i += 256) {
+    const int k = i / QUADS, n = n0 + 4 * (i % QUADS);
+    *reinterpret_cast<float4 *>(sW + 4 * i) =
+        n < N ? *reinterpret_cast<const float4 *>(W + (long long)k * N + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __syncthreads();
+  float acc[R][4];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc[i][j] = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < K; ++k) {
+    const float4 w = *reinterpret_cast<const float4 *>(sW + k * COLS + 4 * quad);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const float a = grLds[(group + i * GROUPS) * K + k];
+      acc[i][0] = fmaf(a, w.x, acc[i][0]);
+      acc[i][1] = fmaf(a, w.y, acc[i][1]);
+      acc[i][2] = fmaf(a, w.z, acc[i][2]);
+      acc[i][3] = fmaf(a, w.w, acc[i][3]);
+    }
+  }
+  const int n = n0 + 4 * quad;
+  if (n >= N)
+    return;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const long long m = m0 + group + i * GROUPS;
+    if (m < M)
+      *reinterpret_cast<float4 *>(out + m * N + n) = make_float4(apply_act(acc[i][0], n, ep), apply_act(acc[i][1], n + 1, ep),
+                                                                 apply_act(acc[i][2], n + 2, ep), apply_act(acc[i][3], n + 3, ep));
+  }
+}
+
 // The same with the row of A read through the rules (the receptive field of
 // output site m) -- any number of channels, so a convolution over one to three
 // input channels, the first layer of most nets, needs no matrix either.  A
@@ -1995,6 +2060,12 @@ static int nin_forward(scn_ctx *ctx, const float *d_A, const float *d_W,
         break;
       }
     }
+  } else if (K <= GR_MAX_K && N % 4 == 0 && (((uintptr_t)d_A | (uintptr_t)d_W | (uintptr_t)d_out) & 15) == 0) {
+    const int cols = N <= 32 ? 32 : 64;
+    const dim3 grid((unsigned)((M + 63) / 64), scn_ceil_div(N, cols));
+    const size_t lds = (size_t)K * (64 + cols) * sizeof(float); // (64 KB at most)
+    hipLaunchKernelGGL((N <= 32 ? k_nin_rows<8> : k_nin_rows<16>), grid, dim3(256), lds, ctx->stream, d_A, d_W, d_out,
+                       (long long)M, K, N, ep);
   } else {
     dim3 grid(scn_ceil_div(M, GT_BM), scn_ceil_div(N, GT_BN));
     hipLaunchKernelGGL(k_nin_generic, grid, dim3(256), 0, ctx->stream, d_A,
