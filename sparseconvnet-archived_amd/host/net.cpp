@@ -1309,6 +1309,7 @@ int BatchProducer::firstOfPart(int size, int part) const {
 // us beside nine others that code the next ones), and is alone in launching its rule
 // books' kernels.
 void BatchProducer::sharedProducerThread(int) {
+  RNG rng; // (not drawn from: with SCN_SEED set, the generators made later have the numbers that they had)
   const int nSlots = cnn.nBatchProducerThreads;
   for (;;) {
     int c, cc, part;
