@@ -382,6 +382,18 @@ int scn_terminal_classifier_train(scn_ctx *ctx, const float *d_in,
                                   const float *d_B, float *d_probs, float *copy,
                                   int K, int N, float p,
                                   const int32_t *d_labels, float *d_delta);
+/* ... and scn_gradients_begin for the backward pass that follows, in the same launch:
+ * nothing of what that clears and writes is this call's. */
+struct scn_filter_item;
+int scn_terminal_classifier_begin(scn_ctx *ctx, const float *d_in,
+                                  const int32_t *d_rules, int64_t M, int S,
+                                  float *d_pooled, const float *d_W,
+                                  const float *d_B, float *d_probs, float *copy,
+                                  int K, int N, float p,
+                                  const int32_t *d_labels, float *d_delta,
+                                  void *const *d_clear, const size_t *nWords,
+                                  int nClear, const struct scn_filter_item *items,
+                                  int nItems);
 /* dSigmoidSoftmax (SigmoidLayer.cu:160-177). */
 int scn_softmax_rows(scn_ctx *ctx, const float *d_in, float *d_out, int64_t M,
                      int N);

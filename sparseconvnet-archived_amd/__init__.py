@@ -161,6 +161,8 @@ def lib():
         "scn_terminal_classifier": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float]),
         "scn_terminal_classifier_train": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float,
                                                     vp, vp]),
+        "scn_terminal_classifier_begin": (C.c_int, [vp, vp, vp, i64, C.c_int, vp, vp, vp, vp, vp, C.c_int, C.c_int, C.c_float,
+                                                    vp, vp, P(vp), P(sz), C.c_int, P(FilterItem), C.c_int]),
         "scn_terminal_gradient_supported": (C.c_int, [C.c_int, C.c_int]),
         "scn_terminal_gradient": (C.c_int, [vp, vp, vp, vp, vp, i64, C.c_int, vp, vp, C.c_int, vp, vp, C.c_int, C.c_int]),
         "scn_softmax_rows": (C.c_int, [vp, vp, vp, i64, C.c_int]),

@@ -200,14 +200,63 @@ struct FillList {
   unsigned firstBlock[SCN_FILL_MAX + 1];
   int count;
 };
-__device__ __forceinline__ void fill32_list_block(const FillList &l, uint32_t w, unsigned block) {
+__device__ __forceinline__ void fill32_list_block(const FillList &l, uint32_t w, unsigned block, unsigned tid) {
   int t = 0;
   while (t + 1 < l.count && block >= l.firstBlock[t + 1])
     ++t;
   const unsigned blocks = l.firstBlock[t + 1] - l.firstBlock[t];
-  fill32(l.dst[t], w, l.n[t], (size_t)(block - l.firstBlock[t]) * 256 + threadIdx.x, (size_t)blocks * 256);
+  fill32(l.dst[t], w, l.n[t], (size_t)(block - l.firstBlock[t]) * 256 + tid, (size_t)blocks * 256);
 }
 int scn_fill_list(scn_ctx *c, void *const *d_dst, const size_t *nWords, int n, FillList *list, unsigned *blocksOf);
+
+// What a backward pass begins with: buffers cleared, and Wt[(f N + n) nIn + c] = W[(f nIn
+// + c) N + n], the weights of the convolutions that its inputs' gradients are, all
+// layers', a tile of 32 x 32 to 256 lanes.
+struct FilterList {
+  const float *W[SCN_FILTERS_MAX];
+  float *Wt[SCN_FILTERS_MAX];
+  unsigned firstBlock[SCN_FILTERS_MAX + 1];
+  int nIn[SCN_FILTERS_MAX], N[SCN_FILTERS_MAX];
+  int count;
+};
+struct BeginList {
+  FilterList filters;
+  FillList fill;
+  unsigned fillBlocks, blocks; // of 256 lanes; the fills' come first
+};
+// (called by 256 lanes for each block, and by all of a workgroup together: a block
+// past the last one does nothing)
+__device__ __forceinline__ void begin_list_block(const BeginList &b, unsigned block, unsigned tid, float (&tile)[32][33]) {
+  const FilterList &l = b.filters;
+  const bool filter = block >= b.fillBlocks && block < b.blocks;
+  const int tx = tid & 31, ty = tid >> 5; // 32 x 8
+  int nIn = 0, N = 0, n0 = 0, c0 = 0;
+  float *Wt = nullptr;
+  if (filter) {
+    const unsigned at = block - b.fillBlocks;
+    const int lane = tid & 63;
+    const int t = __popcll(__ballot(lane < l.count && at >= l.firstBlock[lane < SCN_FILTERS_MAX ? lane : 0])) - 1;
+    nIn = l.nIn[t], N = l.N[t];
+    const int across = (N + 31) / 32, down = (nIn + 31) / 32;
+    const unsigned x = at - l.firstBlock[t];
+    const int f = (int)(x / (across * down));
+    n0 = (int)(x % across) * 32, c0 = (int)(x / across % down) * 32;
+    const float *const W = l.W[t] + (long long)f * nIn * N;
+    Wt = l.Wt[t] + (long long)f * nIn * N;
+    for (int i = ty; i < 32; i += 8)
+      if (c0 + i < nIn && n0 + tx < N)
+        tile[i][tx] = W[(long long)(c0 + i) * N + n0 + tx];
+  } else if (block < b.fillBlocks) {
+    fill32_list_block(b.fill, 0u, block, tid);
+  }
+  __syncthreads();
+  if (filter)
+    for (int i = ty; i < 32; i += 8)
+      if (n0 + i < N && c0 + tx < nIn)
+        Wt[(long long)(n0 + i) * nIn + c0 + tx] = tile[tx][i];
+}
+int scn_begin_list(scn_ctx *ctx, void *const *d_clear, const size_t *nWords, int nClear, const scn_filter_item *items,
+                   int nItems, BeginList *list);
 
 // Kernel attributes (the dynamic LDS limit) are set per device: fn runs once for
 // every device a context of this process lives on, and again if it failed.

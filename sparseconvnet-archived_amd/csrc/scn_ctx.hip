@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256) void k_fill32(uint32_t *dst, uint32_t w, size_
   fill32(dst, w, n, (size_t)blockIdx.x * 256 + threadIdx.x, (size_t)gridDim.x * 256);
 }
 
-__global__ __launch_bounds__(256) void k_fill32_many(FillList l, uint32_t w) { fill32_list_block(l, w, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_fill32_many(FillList l, uint32_t w) { fill32_list_block(l, w, blockIdx.x, threadIdx.x); }
 
 // (the list, and how many workgroups go through it)
 int scn_fill_list(scn_ctx *c, void *const *d_dst, const size_t *nWords, int n, FillList *list, unsigned *blocksOf) {

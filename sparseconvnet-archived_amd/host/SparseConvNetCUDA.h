@@ -108,6 +108,7 @@ public:
   void forwardBatch(SpatiallySparseBatch &batch, int lane = 0);
   void makeWeightImages(SpatiallySparseBatch &batch, cudaMemStream &ms);
   bool matrixWithNext(SpatiallySparseBatch &batch, size_t i) const;
+  void startOfBackward(SpatiallySparseBatch &batch, BackwardStart &start);
   void backwardBatch(SpatiallySparseBatch &batch, float learningRate,
                      float momentum);
   // training batches are drawn in shuffled order (BatchProducer.cu:23-26);

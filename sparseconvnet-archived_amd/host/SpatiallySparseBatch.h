@@ -87,6 +87,8 @@ public:
   // the rule books' counts are still on the device: the interfaces hold bounds
   // until SparseConvNetCUDA::settleRuleBooks
   bool countsPending;
+  // the forward pass has done what the backward pass begins with
+  bool backwardStarted = false;
   // a training batch between whose layers nobody looks (processDataset's): what
   // only its layers' kernels would read need not be there
   bool unseen;

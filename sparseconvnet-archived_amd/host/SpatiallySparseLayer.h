@@ -416,13 +416,19 @@ void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
 
 // the last two layers of a test batch's forward pass and that copy in one launch,
 // where they are a terminal pooling and a classifier (layer `last`) that it takes
+// (start: what the batch's backward pass begins with, done beside it)
+struct BackwardStart {
+  std::vector<void *> clear;
+  std::vector<size_t> words;
+  std::vector<scn_filter_item> filters;
+};
 bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseLayer *pooling,
                                SpatiallySparseLayer *classifier,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
-                               cudaMemStream &ms, int last);
+                               cudaMemStream &ms, int last, const BackwardStart *start = nullptr);
 // ... and backwards, with the derivative of the layer under the pooling: false: not
 // of that kind, nothing done
 bool backwardTerminalClassifier(SpatiallySparseBatch &batch,

@@ -1243,7 +1243,7 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
-                               cudaMemStream &ms, int last) {
+                               cudaMemStream &ms, int last, const BackwardStart *start) {
   auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
   const bool train = batch.type == TRAINBATCH;
   if (batch.type == RESCALEBATCH || !n || n->fn != SOFTMAX ||
@@ -1264,11 +1264,14 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   if (train) {
     keep_labels(batch);
     output.sub->dfeatures.resize64(M * N);
-    SCN_CHECKED(scn_terminal_classifier_train(
+    static const BackwardStart nothing;
+    const BackwardStart &b = start ? *start : nothing;
+    SCN_CHECKED(scn_terminal_classifier_begin(
         ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
         (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
         n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
-        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr()));
+        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr(), b.clear.data(), b.words.data(),
+        (int)b.clear.size(), b.filters.data(), (int)b.filters.size()));
   } else {
     SCN_CHECKED(scn_terminal_classifier(
         ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,

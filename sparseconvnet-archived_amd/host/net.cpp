@@ -441,16 +441,10 @@ void SparseConvNetCUDA::processBatch(SpatiallySparseBatch &batch,
     backwardBatch(batch, learningRate, momentum);
   finishBatch(batch, f, g);
 }
-// The training half of processBatch (SparseConvNetCUDA.cu:248-252): the
-// classifier has left d cost / d soft-max input in the top interface; every
-// layer, last to first, hands the gradient down and updates its weights.
-void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
-                                      float learningRate, float momentum) {
-  // the gradients that layers add to, cleared in one launch (a dozen of 4 us
-  // between the others otherwise)
-  void *grads[SCN_FILL_MAX];
-  size_t sizes[SCN_FILL_MAX];
-  int n = 0;
+// What a backward pass begins with, in one launch: the gradients that layers add to are
+// cleared (a dozen launches of 4 us between the others otherwise) and the filters
+// turned round.
+void SparseConvNetCUDA::startOfBackward(SpatiallySparseBatch &batch, BackwardStart &start) {
   for (size_t i = 0; i < layers.size(); i++) {
     SpatiallySparseBatchInterface &input = batch.interfaces[i];
     const size_t nf = input.featuresPresent.size();
@@ -470,21 +464,33 @@ void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
     input.sub->dfeatures.resize64(own + sums);
     if (writes)
       continue;
-    sizes[n] = input.gradientCleared ? own + sums : sums;
-    grads[n++] = input.sub->dfeatures.dPtr() + (input.gradientCleared ? 0 : own);
-    if (n == SCN_FILL_MAX) {
-      SCN_CHECKED(scn_fill32_many(memStream.ctx, grads, sizes, n, 0u));
+    start.words.push_back(input.gradientCleared ? own + sums : sums);
+    start.clear.push_back(input.sub->dfeatures.dPtr() + (input.gradientCleared ? 0 : own));
+  }
+  for (size_t i = 0; i < layers.size(); i++)
+    layers[i]->transposedFilters(batch.interfaces[i], start.filters);
+}
+// The training half of processBatch (SparseConvNetCUDA.cu:248-252): the
+// classifier has left d cost / d soft-max input in the top interface; every
+// layer, last to first, hands the gradient down and updates its weights.
+void SparseConvNetCUDA::backwardBatch(SpatiallySparseBatch &batch,
+                                      float learningRate, float momentum) {
+  // (done already where the forward pass ended in a launch that takes it along)
+  if (!batch.backwardStarted) {
+    BackwardStart start;
+    startOfBackward(batch, start);
+    size_t n = start.clear.size();
+    for (; n > SCN_FILL_MAX; n -= SCN_FILL_MAX)
+      SCN_CHECKED(scn_fill32_many(memStream.ctx, start.clear.data() + n - SCN_FILL_MAX,
+                                  start.words.data() + n - SCN_FILL_MAX, SCN_FILL_MAX, 0u));
+    for (size_t i = 0; i == 0 || i < start.filters.size(); i += SCN_FILTERS_MAX) {
+      SCN_CHECKED(scn_gradients_begin(memStream.ctx, start.clear.data(), start.words.data(), (int)n,
+                                      start.filters.data() + i,
+                                      (int)std::min<size_t>(SCN_FILTERS_MAX, start.filters.size() - i)));
       n = 0;
     }
   }
-  std::vector<scn_filter_item> filters;
-  for (size_t i = 0; i < layers.size(); i++)
-    layers[i]->transposedFilters(batch.interfaces[i], filters);
-  for (size_t i = 0; i == 0 || i < filters.size(); i += SCN_FILTERS_MAX) {
-    SCN_CHECKED(scn_gradients_begin(memStream.ctx, grads, sizes, n, filters.data() + i,
-                                    (int)std::min<size_t>(SCN_FILTERS_MAX, filters.size() - i)));
-    n = 0;
-  }
+  batch.backwardStarted = false;
   batch.updates.clear();
   batch.products.clear();
   batch.collectUpdates = true;
@@ -598,16 +604,24 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
   // pass (SparseConvNetCUDA.cu:230-241)
   float scalingUnderneath = 1;
   batch.result->copied = batch.result->graded = false;
+  batch.backwardStarted = false;
   for (size_t i = 0; i < layers.size(); i++) {
     batch.interfaces[i + 1].sub->reset();
     scn_prof_tag(ms.ctx, (int)i);
     if (batch.countsPending)
       SCN_CHECKED(scn_ctx_rows_from(ms.ctx, batch.interfaces[i + 1].deviceGrids));
-    if (i + 2 == layers.size() &&
-        forwardTerminalClassifier(batch, layers[i], layers[i + 1],
-                                  batch.interfaces[i], batch.interfaces[i + 1],
-                                  batch.interfaces[i + 2], ms, (int)i + 1))
-      break;
+    if (i + 2 == layers.size()) {
+      BackwardStart start;
+      if (batch.type == TRAINBATCH && !batch.countsPending)
+        startOfBackward(batch, start);
+      const bool fits = start.clear.size() <= SCN_FILL_MAX && start.filters.size() <= SCN_FILTERS_MAX;
+      if (forwardTerminalClassifier(batch, layers[i], layers[i + 1],
+                                    batch.interfaces[i], batch.interfaces[i + 1],
+                                    batch.interfaces[i + 2], ms, (int)i + 1, fits ? &start : nullptr)) {
+        batch.backwardStarted = batch.type == TRAINBATCH && !batch.countsPending && fits;
+        break;
+      }
+    }
     batch.interfaces[i + 1].matrixWithNext = matrixWithNext(batch, i);
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);
     if (batch.type == RESCALEBATCH) {

@@ -1,5 +1,7 @@
 """A net's end in a training batch: the classifier with its cost's gradient in one launch (the bits of the three calls), and
 backwards the classifier's input gradient, spread over the pooled rows with the activation's derivative, in another."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -73,6 +75,38 @@ def test_terminal_gradient(scn, ctx, M, K, N, S, act):
         assert np.all(np.abs(dprelu.download() - start - terms.sum(0)) <= 2.0 ** -21 * (np.abs(terms).sum(0) + np.abs(start)))
     else:
         assert np.array_equal(dprelu.download(), start)
+
+
+# what the backward pass begins with beside the classifier: odd numbers of 256-lane blocks, buffers off 16 bytes, none, filters alone
+@pytest.mark.parametrize("M,K,N,S", [(1, 4, 4, 1), (33, 128, 40, 8), (100, 192, 100, 4)])
+@pytest.mark.parametrize("sizes,filters", [([], [(1, 3, 33)]), ([1025, 0, 3], []), ([70000], [(4, 31, 5), (8, 96, 32), (4, 32, 64)])])
+def test_classifier_with_the_beginning(scn, ctx, M, K, N, S, sizes, filters):
+    rng = np.random.default_rng(M + K)
+    rules, rows, count = pooled_rows(rng, M, S)
+    rules[count == 0, 0] = 0
+    d_x, d_rules = ctx.array(rng.standard_normal((rows, K), dtype=np.float32)), ctx.array(rules)
+    d_W, d_B = ctx.array((rng.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32)), ctx.array(rng.standard_normal(N, dtype=np.float32))
+    d_labels = ctx.array(rng.integers(0, N, M).astype(np.int32))
+    outs = [[ctx.array(np.full((M + 3, w), 7, np.float32)) for w in (K, N, N, N)] for _ in range(2)]
+    bufs = [ctx.array(np.full(n + 4, 7, np.int32)) for n in sizes]
+    Ws = [rng.standard_normal(f, dtype=np.float32) for f in filters]
+    turned, held = [ctx.array(np.full(W.size + 4, 7, np.float32)) for W in Ws], [ctx.array(W) for W in Ws]
+    ptrs = (C.c_void_p * max(1, len(sizes)))(*[b.ptr for b in bufs])
+    words = (C.c_size_t * max(1, len(sizes)))(*sizes)
+    items = (scn.FilterItem * max(1, len(filters)))(*[scn.FilterItem(w.ptr, o.ptr, *f) for w, o, f in zip(held, turned, filters)])
+    print("classifier and beginning", M, K, N, S, sizes, filters, flush=True)
+    pooled, probs, copy, delta = outs[0]
+    scn._check(scn.lib().scn_terminal_classifier_begin(ctx.h, d_x.ptr, d_rules.ptr, M, S, pooled.ptr, d_W.ptr, d_B.ptr, probs.ptr, copy.ptr,
+                                                       K, N, 1.0, d_labels.ptr, delta.ptr, ptrs, words, len(sizes), items, len(filters)))
+    pooled, probs, copy, delta = outs[1]
+    ctx.terminal_classifier_train(d_x, d_rules, M, S, pooled, d_W, d_B, probs, copy, K, N, d_labels, delta)
+    for a, b in zip(*outs):
+        assert np.array_equal(a.download(), b.download())
+    for b, n in zip(bufs, sizes):
+        assert np.all(b.download()[:n] == 0) and np.all(b.download()[n:] == 7)
+    for W, o in zip(Ws, turned):
+        got = o.download()
+        assert np.array_equal(got[:-4].reshape(W.shape[0], W.shape[2], W.shape[1]), W.transpose(0, 2, 1)) and np.all(got[-4:] == 7)
 
 
 def test_what_is_not_supported_is_refused(scn, ctx):
