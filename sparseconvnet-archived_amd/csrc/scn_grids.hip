@@ -1325,8 +1325,35 @@ static int grids_check(int batch, int d, int n) {
               SCN_ERR_CAPACITY, "grids: %d samples of side %d", batch, n);
   return SCN_OK;
 }
+// masks that are emptied beside the next batch's build and not before it: 1 MB
+#define SPARE_MASK_WORDS ((size_t)1 << 17)
+// Room for a mask of n words, and for a second one of that size behind it where `spare`
+// says so and it is not too large: one allocation, as before there was a second (a new
+// net's first pass over 24 batches makes 1864; with one for each second mask 1874, and ten
+// frees).
+static int reserve_mask(scn_grids *g, size_t n, bool spare) {
+  if (n <= g->bits.cap)
+    return SCN_OK;
+  const size_t want = (n + n / 4 + 64 + 31) & ~(size_t)31; // (both on 256 bytes)
+  spare = spare && want <= SPARE_MASK_WORDS;
+  unsigned long long *q = nullptr;
+  if (spare && hipMalloc((void **)&q, 2 * want * sizeof(*q)) != hipSuccess) { // (done without)
+    (void)hipGetLastError();
+    spare = false;
+  }
+  if (!spare)
+    SCN_HIP_CHECK(hipMalloc((void **)&q, want * sizeof(*q)));
+  if (g->maskMemory)
+    (void)hipFree(g->maskMemory);
+  g->maskMemory = g->bits.p = q;
+  g->bits.cap = want;
+  g->spare = spare ? q + want : nullptr;
+  g->spareClean = false;
+  return SCN_OK;
+}
+// (spare: masks of a batch's sites that are emptied and made again)
 static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
-                         long long nActive, bool withTable = false, bool wholeMask = false) {
+                         long long nActive, bool withTable = false, bool wholeMask = false, bool spare = false) {
   SCN_TRY(grids_check(batch, d, n));
   const long long vol = ipow_ll(n, d);
   g->rankStateFor = 0;
@@ -1357,7 +1384,7 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
     SCN_TRY(g->dense.reserve((size_t)((long long)batch * vol) + 1));
   else if (withTable)
     SCN_TRY(g->table.reserve(cap));
-  SCN_TRY(g->bits.reserve(g->nWords + 8)); // the scan reads whole 32-byte groups
+  SCN_TRY(reserve_mask(g, g->nWords + 8, spare)); // the scan reads whole 32-byte groups
   if (g->table.p != hadTable)
     g->cleanSlots = 0; // fresh memory
   if (g->bits.p != hadBits)
@@ -1438,7 +1465,7 @@ extern "C" int scn_grids_clear_many(scn_ctx *ctx, scn_grids **grids, int n) {
                              (!g->bits.p || g->cleanWords >= g->bits.cap)))
         continue;
       scn_grids_hold_mask(ctx, g);
-      if (g->spare && g->spareClean && g->spareCap == g->bits.cap && !g->maskHeld &&
+      if (g->spare && g->spareClean && !g->maskHeld &&
           (!g->table.p || g->cleanSlots >= g->table.cap)) { // (what was in use: emptied by the build)
         std::swap(g->bits.p, g->spare);
         g->spareClean = false;
@@ -1772,8 +1799,8 @@ extern "C" int scn_grids_destroy(scn_ctx *ctx, scn_grids *g) {
   g->meta.release();
   g->table.release();
   g->dense.release();
-  g->bits.release();
-  (void)hipFree(g->spare);
+  if (g->maskMemory)
+    (void)hipFree(g->maskMemory);
   g->prefix.release();
   g->rankRow.release();
   g->ekey.release();
@@ -1796,8 +1823,6 @@ extern "C" int scn_grids_destroy(scn_ctx *ctx, scn_grids *g) {
   return SCN_OK;
 }
 
-// masks that are emptied beside the next batch's build and not before it: 1 MB
-#define SPARE_MASK_WORDS ((size_t)1 << 17)
 extern "C" int scn_grids_build(scn_ctx *ctx, scn_grids *g, int batch,
                                int dimension, int spatialSize,
                                const int32_t *d_sample, const int64_t *d_key,
@@ -1829,26 +1854,15 @@ extern "C" int scn_grids_build_copy(scn_ctx *ctx, scn_grids *g, int batch,
   for (int a = 0; a < dimension && a < 3; ++a)
     sites *= spatialSize > 0 ? spatialSize : 1;
   SCN_TRY(grids_prepare(ctx, g, batch, dimension, spatialSize, n,
-                        sites <= SCN_DENSE_MAX_SITES));
+                        sites <= SCN_DENSE_MAX_SITES, false, g->emptied));
   g->nSites = nSpatialSites;
   // (backgroundCol is copied by the same launch: lane e < batch takes entry e)
   const long long lanes = n > batch ? n : batch;
   const unsigned siteBlocks = (unsigned)scn_ceil_div(lanes, 256);
   const size_t copyBlocks = bytes ? std::min((bytes / 16 + 255) / 256 + 1, (size_t)4096) : 0;
   const GridView view = view_of(ctx, g);
-  size_t spareWords = 0;
-  if (siteBlocks + copyBlocks > 0 && g->emptied && !g->maskHeld && g->bits.cap <= SPARE_MASK_WORDS) {
-    if (g->spareCap != g->bits.cap) {
-      (void)hipFree(g->spare);
-      g->spareCap = g->bits.cap;
-      g->spareClean = false;
-      if (hipMalloc((void **)&g->spare, g->spareCap * sizeof(*g->spare)) != hipSuccess) { // (done without)
-        (void)hipGetLastError();
-        g->spare = nullptr;
-      }
-    }
-    spareWords = g->spare && !g->spareClean ? g->spareCap : 0;
-  }
+  const size_t spareWords =
+      siteBlocks + copyBlocks > 0 && g->spare && !g->spareClean && !g->maskHeld ? g->bits.cap : 0;
   const size_t spareBlocks = std::min((spareWords + 1023) / 1024, (size_t)256);
   if (siteBlocks + copyBlocks > 0) {
     hipLaunchKernelGGL(k_grid_build, dim3((unsigned)(siteBlocks + copyBlocks + spareBlocks)), dim3(256), 0,
@@ -2057,7 +2071,7 @@ static int plan_regions_d(scn_ctx *ctx, scn_grids *in, scn_grids *out,
   if (dilated) {
     // (needs no count: runs while the host waits for them.  It also clears the
     // state of the scan that gives the mask its ranks)
-    SCN_TRY(out->bits.reserve(outWords + 8)); // the scan reads whole 32-byte groups
+    SCN_TRY(reserve_mask(out, outWords + 8, false)); // the scan reads whole 32-byte groups
     const long long words = (long long)outWords + 2; // all that grids_prepare would clear
     const Dilate to = {out->bits.p, words, volOutAll, scn_scan_state(outWords + 1, out->scanTmp.p),
                        xcd_grid(scn_ceil_div(words, 256))}; // (whole rounds of the 8 XCDs)

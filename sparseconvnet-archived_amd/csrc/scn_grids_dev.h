@@ -136,12 +136,11 @@ struct scn_grids {
   // how much of table / bits is known to be empty right now (scn_grids_clear_many)
   size_t cleanSlots = 0, cleanWords = 0;
   // Grids that are emptied by scn_grids_clear_many and built again batch after batch, from
-  // the first one on (`emptied`), have a second mask, which the build of one batch
-  // empties and the next one takes (spareClean: it is empty, once the stream is
-  // through): emptying costs no launch.  maskHeld: the first one's address is in a
+  // the first one on (`emptied`), have a second mask of the same size, which the build of
+  // one batch empties and the next one takes (spareClean: it is empty, once the stream
+  // is through): emptying costs no launch.  maskHeld: the first one's address is in a
   // captured graph, and it stays.  (Others are not asked about: 0.3 us a call.)
-  unsigned long long *spare = nullptr;
-  size_t spareCap = 0;
+  unsigned long long *maskMemory = nullptr, *spare = nullptr;
   bool spareClean = false, emptied = false;
   mutable bool maskHeld = false;
   // Deferred counts: while pending, nActive / nSites / termS hold upper bounds
@@ -157,7 +156,10 @@ struct scn_grids {
   DevBuf<long long> meta; // META_* words
   DevBuf<Slot> table;
   DevBuf<int> dense;
-  DevBuf<unsigned long long> bits;
+  struct {
+    unsigned long long *p = nullptr;
+    size_t cap = 0; // words
+  } bits; // in maskMemory
   DevBuf<unsigned> prefix;
   DevBuf<int> rankRow;
   DevBuf<long long> ekey;
