@@ -16,8 +16,12 @@ public:
   // convolution with bf16 operands: made by it, where its window is large enough for
   // the rows to be read many times over, or
   vectorCUDA<float> features16;
-  // by the pooling that makes the features: is to be, and has been in this pass
+  // by the pooling that makes the features: is to be, and has been in this pass, in the
+  // room behind them, from that element on (allocations of its own were two of a new
+  // wide net's first pass)
   bool roundedToo = false, rounded = false;
+  size_t roundedAt = 0;
+  float *roundedRows() { return features.dPtr() + roundedAt; }
   // the weights of the layer whose output this is, laid out for its forward pass
   // and, turned round, for the gradient of its input: made for one batch by
   // SparseConvNetCUDA::makeWeightImages, in the stream's room for them, and used up

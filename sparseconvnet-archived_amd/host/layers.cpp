@@ -382,7 +382,7 @@ static bool nin_fused(cudaMemStream &ms, SpatiallySparseBatchInterface &input,
   }
   if (src->sub->rounded && precision == SCN_BF16) {
     SCN_CHECKED(scn_conv_nin_forward_rounded(
-        ms.ctx, src->sub->features.dPtr(), src->sub->features16.dPtr(), input.rules.dPtr(), fs, nIn, W.dPtr(), image,
+        ms.ctx, src->sub->features.dPtr(), src->sub->roundedRows(), input.rules.dPtr(), fs, nIn, W.dPtr(), image,
         B.dPtr(), prelu ? prelu->dPtr() : nullptr, output.sub->features.dPtr(), output.nSpatialSites, nFeaturesOut, p,
         act));
     return true;
@@ -894,14 +894,15 @@ static void pool_forwards(cudaMemStream &ms,
                           SpatiallySparseBatchInterface &output, int width) {
   const size_t nf = output.featuresPresent.size();
   output.sub->poolingChoices.resize64((size_t)output.nSpatialSites * nf, kBoundRows * nf);
-  output.sub->features.resize64((size_t)output.nSpatialSites * nf, kBoundRows * nf);
-  output.sub->rounded = output.sub->roundedToo && nf % 8 == 0;
-  if (output.sub->rounded)
-    output.sub->features16.resize64((size_t)output.nSpatialSites * nf / 2 + 8, kBoundRows * nf / 2);
+  output.sub->rounded = output.sub->roundedToo && nf % 8 == 0; // (so that they start on 16 bytes)
+  output.sub->roundedAt = (size_t)output.nSpatialSites * nf;
+  if (output.sub->rounded) // (room for both)
+    output.sub->features.resize64(output.sub->roundedAt + output.sub->roundedAt / 2 + 8, kBoundRows * (nf + nf / 2));
+  output.sub->features.resize64(output.sub->roundedAt, kBoundRows * nf);
   SCN_CHECKED(scn_maxpool_rounded(ms.ctx, input.sub->features.dPtr(),
                                   input.nSpatialSites,
                                   output.sub->features.dPtr(),
-                                  output.sub->rounded ? output.sub->features16.dPtr() : nullptr,
+                                  output.sub->rounded ? output.sub->roundedRows() : nullptr,
                                   output.rules.dPtr(), output.nSpatialSites,
                                   width, (int)nf,
                                   output.sub->poolingChoices.dPtr()));
