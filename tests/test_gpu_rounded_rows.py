@@ -1,9 +1,13 @@
 """Rows that a pooling leaves rounded to bf16 beside its output: the contraction's bits are those of fp32 rows, which it
 rounds itself, in every kernel that takes them."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+import brute
 from test_gpu_capture import Graph
+from test_gpu_run_ahead import _one_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +73,89 @@ def test_a_net_of_bf16_operands(scn):
         small = cases._prepare_net(dict(case, batch=2), 4)
         runs.append(np.concatenate([out[0], cases._run_net(small).copy()]))
     assert np.isfinite(runs[0]).all() and np.array_equal(runs[0], runs[1])
+
+
+# (a contraction split over few rows, tiles, k_nin_rows16)
+@pytest.mark.parametrize("nIn,N,densities", [(64, 96, (0.02, 0.02, 0.01)), (256, 320, (0.4, 0.4, 0.2, 0.42)),
+                                             (512, 128, (0.5, 0.5, 0.35, 0.6))])
+def test_rounded_rows_ahead_of_their_counts(scn, ctx, nIn, N, densities):
+    """rows known on the device only: a pooling that rounds, and contractions of rounded rows, as with known counts"""
+    rng = np.random.default_rng(nIn)
+    fs, src, out = 4, scn.Grids(ctx), scn.Grids(ctx)
+    d_W = ctx.array((rng.standard_normal((fs * nIn, N)) * np.sqrt(0.5 / nIn)).astype(np.float32))
+    d_B = ctx.array(rng.uniform(-0.5, 0.5, N).astype(np.float32))
+    rounds = []
+    for i, density in enumerate(densities):
+        samples, nSites = brute.random_samples(rng, 30, 2, 41, density)
+        x = rng.standard_normal((nSites, nIn), dtype=np.float32)
+        d_x, d_x16, room = ctx.array(x), ctx.array(rounded(x).view(np.int32)), ctx.empty((nSites, nIn // 2), np.float32)
+        rules, bound = _one_plan(scn, ctx, src, out, samples, nSites, i > 0)
+        outs = [ctx.array(np.full((bound, N), 7, np.float32)) for _ in range(2)]
+        pooled = [ctx.array(np.full((bound, c), 7, t)) for c, t in ((nIn, np.float32), (nIn // 2, np.int32), (nIn, np.int32))]
+        print("rounded rows ahead", nIn, N, density, bound, flush=True)
+        assert scn.lib().scn_ctx_rows_from(ctx.h, out.h) == scn.OK
+        ctx.maxpool_rounded(d_x, nSites, *pooled[:2], rules, bound, fs, nIn, pooled[2])
+        ctx.conv_nin_forward_rounded(d_x, d_x16, rules, fs, nIn, d_W, None, d_B, None, outs[0], bound, N)
+        ctx.conv_nin_forward_a16(d_x, nSites, room, rules, fs, nIn, d_W, d_B, None, outs[1], bound, N)
+        scn.lib().scn_ctx_rows_from(ctx.h, None)
+        assert scn.settle(ctx)
+        held = C.c_int()
+        assert scn.lib().scn_ctx_rows_held(ctx.h, C.byref(held)) == scn.OK
+        n = out.info()["nSpatialSites"]
+        known = [ctx.array(np.full((n, c), 7, t)) for c, t in ((nIn, np.float32), (nIn // 2, np.int32), (nIn, np.int32), (N, np.float32))]
+        ctx.maxpool_rounded(d_x, nSites, *known[:2], rules, n, fs, nIn, known[2])
+        ctx.conv_nin_forward(d_x, rules, fs, nIn, d_W, d_B, None, known[3], n, N, 1.0, scn.RELU, scn.BF16)
+        for a, b in zip(pooled, known):
+            a = a.download()
+            assert np.array_equal(a[:n], b.download()) and np.all(a[n:] == 7)
+        want = known[3].download()
+        for a in outs:
+            a = a.download()
+            assert np.all(a[n:] == 7)
+            if held.value:
+                assert np.array_equal(a[:n], want), (i, n, bound)
+            else:  # two orders of summation of the same K products
+                scale = np.abs(x).max() * np.abs(d_W.download()).sum(0).max() + 0.5
+                assert np.abs(a[:n] - want).max() <= 2 * fs * nIn * 2.0 ** -24 * scale
+        rounds.append(held.value)
+    assert rounds[:2] == [1, 1]
+
+
+def test_an_epoch_of_bf16_operands(scn):
+    """The poolings of a training batch round, too: an epoch of one batch, whose convolutions are left out and read rounded
+    rows, costs what the batch by itself, which gathers, costs, and leaves its gradients."""
+    from sparseconvnet_archived_amd import hostapi, synthetic
+    batch = 70
+    cfg = synthetic.config(4, batch=batch)
+    ds = hostapi.Dataset(cfg.name, cfg.nInputFeatures, cfg.nClasses, hostapi.TRAINBATCH)
+    for pts, f, label in synthetic.make_samples(cfg, 44):
+        ds.add_points(cfg.dimension, cfg.lattice, pts, f, label)
+    costs, left, pay = [], [], 0
+    for epoch in (True, False):
+        net = hostapi.Net(cfg.dimension, cfg.nInputFeatures, cfg.nClasses, threads=1)
+        cfg.build(net)
+        net.setPrecision(scn.BF16)
+        for i, (W, B, pr) in synthetic.he_normal_weights(net.layers(), 45).items():
+            net.set_weights(i, W, B, pr)
+        net.set_training(0.01, 0.9, shuffle=False)
+        if epoch:
+            costs.append(net.processDatasetTrain(ds, batch, 0.01, 0.9))
+        else:
+            net.begin(ds, batch)
+            assert net.next_batch()
+            costs.append(net.batch_outputs()["nll"] / batch)
+            for i, l in enumerate(net.layers()):
+                if l["kind"].startswith("nin") and i > 1 and l["nIn"] % 4 == 0:
+                    rows = net.interface(i + 1, want_features=False)["nSpatialSites"]
+                    pay += scn.lib().scn_rounded_rows_pay(C.c_void_p(net.context_handle()), rows, 4, l["nIn"] // 4, l["nOut"])
+            net.end()
+        left.append([net.get_weights(i, True) for i, l in enumerate(net.layers()) if l["kind"].startswith("nin")])
+        net.close()
+    assert pay >= 2  # (layers whose rows come rounded)
+    print("costs", costs, "gradients", [[float(np.linalg.norm(u - v) / np.linalg.norm(v)) for u, v in zip(a, b) if v is not None]
+                                        for a, b in zip(*left)], flush=True)
+    assert abs(costs[0] - costs[1]) <= 1e-6 * abs(costs[1])
+    # (the same bits forward; sums of up to 10^5 products in another order backward, through six layers: sqrt(1e5) 2^-24 each)
+    for a, b in zip(*left):
+        for u, v in zip(a, b):
+            assert v is None or np.linalg.norm(u - v) <= 6 * 2e-5 * np.linalg.norm(v)
