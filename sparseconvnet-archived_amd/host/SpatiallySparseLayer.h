@@ -414,16 +414,19 @@ void SoftmaxClassifierLaunch(SpatiallySparseBatchInterface &input,
 void SoftmaxClassifierCollect(SpatiallySparseBatchInterface &input,
                               SpatiallySparseBatch &batch, int nTop);
 
-// the last two layers of a test batch's forward pass and that copy in one launch,
-// where they are a terminal pooling and a classifier (layer `last`) that it takes
-// (start: what the batch's backward pass begins with, done beside it)
+// the last two layers of a forward pass and that copy in one launch, where
+// isTerminalClassifier says that they are a terminal pooling and a classifier (layer
+// `last`) that it takes (start: what a training batch's backward pass begins with, done
+// beside it, or null)
 struct BackwardStart {
   std::vector<void *> clear;
   std::vector<size_t> words;
   std::vector<scn_filter_item> filters;
 };
-bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
-                               SpatiallySparseLayer *pooling,
+bool isTerminalClassifier(const SpatiallySparseBatch &batch, SpatiallySparseLayer *pooling,
+                          SpatiallySparseLayer *classifier, SpatiallySparseBatchInterface &middle,
+                          SpatiallySparseBatchInterface &output);
+void forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseLayer *classifier,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,

@@ -1237,24 +1237,27 @@ static void keep_labels(SpatiallySparseBatch &batch) {
 }
 // A net's end, a terminal pooling and the classifier, in one launch that also
 // leaves the probabilities where the host reads them, and a training batch's
-// gradient.  False: not of that kind, nothing done.
-bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
-                               SpatiallySparseLayer *pooling,
+// gradient: whether it is of that kind,
+bool isTerminalClassifier(const SpatiallySparseBatch &batch, SpatiallySparseLayer *pooling,
+                          SpatiallySparseLayer *classifier, SpatiallySparseBatchInterface &middle,
+                          SpatiallySparseBatchInterface &output) {
+  auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
+  return batch.type != RESCALEBATCH && n && n->fn == SOFTMAX &&
+         (batch.type != TRAINBATCH ||
+          (n->dropout <= 0 && (int)middle.featuresPresent.size() == n->nFeaturesIn &&
+           (int)output.featuresPresent.size() == n->nFeaturesOut)) &&
+         dynamic_cast<TerminalPoolingLayer *>(pooling) && middle.nSpatialSites == batch.batchSize &&
+         scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn, n->nFeaturesOut);
+}
+// and, of one that is, the launch
+void forwardTerminalClassifier(SpatiallySparseBatch &batch,
                                SpatiallySparseLayer *classifier,
                                SpatiallySparseBatchInterface &input,
                                SpatiallySparseBatchInterface &middle,
                                SpatiallySparseBatchInterface &output,
                                cudaMemStream &ms, int last, const BackwardStart *start) {
-  auto *n = dynamic_cast<NetworkInNetworkLayer *>(classifier);
+  auto *n = static_cast<NetworkInNetworkLayer *>(classifier);
   const bool train = batch.type == TRAINBATCH;
-  if (batch.type == RESCALEBATCH || !n || n->fn != SOFTMAX ||
-      (train && (n->dropout > 0 || (int)middle.featuresPresent.size() != n->nFeaturesIn ||
-                 (int)output.featuresPresent.size() != n->nFeaturesOut)) ||
-      !dynamic_cast<TerminalPoolingLayer *>(pooling) ||
-      middle.nSpatialSites != batch.batchSize ||
-      !scn_terminal_classifier_supported(batch.batchSize, n->nFeaturesIn,
-                                         n->nFeaturesOut))
-    return false;
   const size_t K = n->nFeaturesIn, N = n->nFeaturesOut, M = batch.batchSize;
   output.sub->reset();
   middle.sub->poolingChoices.resize64(M * K, kBoundRows * K);
@@ -1265,14 +1268,20 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   if (train) {
     keep_labels(batch);
     output.sub->dfeatures.resize64(M * N);
-    static const BackwardStart nothing;
-    const BackwardStart &b = start ? *start : nothing;
+  }
+  if (train && start) {
     SCN_CHECKED(scn_terminal_classifier_begin(
         ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
         (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
         n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
-        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr(), b.clear.data(), b.words.data(),
-        (int)b.clear.size(), b.filters.data(), (int)b.filters.size()));
+        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr(), start->clear.data(), start->words.data(),
+        (int)start->clear.size(), start->filters.data(), (int)start->filters.size()));
+  } else if (train) {
+    SCN_CHECKED(scn_terminal_classifier_train(
+        ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
+        (int)(middle.rules.size64() / M), middle.sub->features.dPtr(), n->W.dPtr(),
+        n->B.dPtr(), output.sub->features.dPtr(), batch.result->pinned, (int)K,
+        (int)N, 1.0f, batch.labels.dPtr(), output.sub->dfeatures.dPtr()));
   } else {
     SCN_CHECKED(scn_terminal_classifier(
         ms.ctx, input.sub->features.dPtr(), middle.rules.dPtr(), M,
@@ -1284,7 +1293,6 @@ bool forwardTerminalClassifier(SpatiallySparseBatch &batch,
   batch.result->graded = train;
   if (!batch.countsPending) // (else counted when they are settled)
     addMultiplyAdds((__int128_t)M * K * N);
-  return true;
 }
 
 // The other way: the classifier's gradients, and its input's spread over the rows

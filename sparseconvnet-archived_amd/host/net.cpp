@@ -610,17 +610,18 @@ void SparseConvNetCUDA::forwardBatch(SpatiallySparseBatch &batch, int lane) {
     scn_prof_tag(ms.ctx, (int)i);
     if (batch.countsPending)
       SCN_CHECKED(scn_ctx_rows_from(ms.ctx, batch.interfaces[i + 1].deviceGrids));
-    if (i + 2 == layers.size()) {
+    if (i + 2 == layers.size() && isTerminalClassifier(batch, layers[i], layers[i + 1], batch.interfaces[i + 1],
+                                                       batch.interfaces[i + 2])) {
+      // (of those two layers the backward pass begins with nothing that their forward
+      // calls would set; counts that are pending may be other ones by then)
       BackwardStart start;
-      if (batch.type == TRAINBATCH && !batch.countsPending)
+      const bool begins = batch.type == TRAINBATCH && !batch.countsPending;
+      if (begins)
         startOfBackward(batch, start);
-      const bool fits = start.clear.size() <= SCN_FILL_MAX && start.filters.size() <= SCN_FILTERS_MAX;
-      if (forwardTerminalClassifier(batch, layers[i], layers[i + 1],
-                                    batch.interfaces[i], batch.interfaces[i + 1],
-                                    batch.interfaces[i + 2], ms, (int)i + 1, fits ? &start : nullptr)) {
-        batch.backwardStarted = batch.type == TRAINBATCH && !batch.countsPending && fits;
-        break;
-      }
+      batch.backwardStarted = begins && start.clear.size() <= SCN_FILL_MAX && start.filters.size() <= SCN_FILTERS_MAX;
+      forwardTerminalClassifier(batch, layers[i + 1], batch.interfaces[i], batch.interfaces[i + 1],
+                                batch.interfaces[i + 2], ms, (int)i + 1, batch.backwardStarted ? &start : nullptr);
+      break;
     }
     batch.interfaces[i + 1].matrixWithNext = matrixWithNext(batch, i);
     layers[i]->forwards(batch, batch.interfaces[i], batch.interfaces[i + 1]);

@@ -99,6 +99,22 @@ def test_train_fused_setting_gathers_while_training(scn):
     train_and_compare(scn, cfg, synthetic.make_samples(cfg, 303), 1, fused=True)
 
 
+# (more classes than the launch for a net's end takes, in fours and not; no terminal pooling in front of the classifier)
+@pytest.mark.parametrize("classes,terminal", [(132, True), (7, True), (12, False)])
+def test_train_with_ends_of_other_kinds(scn, classes, terminal):
+    from sparseconvnet_archived_amd import synthetic
+    stack = [("addLeNetLayerMP", 32, 2, 1, 3, 2, synthetic.RELU), ("addLeNetLayerMP", 64, 2, 1, 2, 2, synthetic.PRELU)]
+    stack += [("addTerminalPoolingLayer", 2)] * terminal + [("addSoftmaxLayer",)]
+    cfg = synthetic.Config("ends", 2, 3, classes, 8, 5, stack)
+    cfg.number = 2
+    rng = np.random.default_rng(classes)
+    samples = []
+    for _ in range(8):
+        pts = np.array([(a, b) for a in range(5) for b in range(5) if rng.random() < 0.5], np.int32).reshape(-1, 2)
+        samples.append((pts, rng.uniform(-1, 1, (len(pts), 3)).astype(np.float32), int(rng.integers(0, classes))))
+    train_and_compare(scn, cfg, samples, 2)
+
+
 def test_train_triangular_leaky_tanh(scn):
     from sparseconvnet_archived_amd import synthetic
     stack = [("addLeNetLayerMP", 32, 2, 1, 2, 2, synthetic.VLEAKYRELU), ("addLeNetLayerMP", 64, 2, 1, 2, 2, synthetic.TANH),
