@@ -85,9 +85,10 @@ public:
 
 private:
   // Batches whose pictures several threads code, as many parts as there are threads:
-  // the batch whose parts are being handed out, the next of them, and which slots
-  // are with the workers or the caller.
-  bool inParts = false;
+  // the batch whose parts are being handed out, the next of them, whether a thread is
+  // getting that batch ready for them, and which slots are with the workers or the
+  // caller.
+  bool inParts = false, opening = false;
   int nextOpen = 0, nextPart = 0;
   std::vector<char> slotOpen;
   void sharedProducerThread(int nThread);

@@ -1330,19 +1330,25 @@ void BatchProducer::sharedProducerThread(int) {
     int c, cc, part;
     {
       std::unique_lock<std::mutex> lock(slotMutex);
-      slotChanged.wait(lock, [&] { return stopping || nextOpen >= nBatches || !slotOpen[nextOpen % nSlots] || nextPart; });
+      slotChanged.wait(lock, [&] {
+        return stopping || nextOpen >= nBatches || nextPart || (!opening && !slotOpen[nextOpen % nSlots]);
+      });
       if (stopping || nextOpen >= nBatches)
         return;
       c = nextOpen;
       cc = c % nSlots;
-      part = nextPart++;
-      SpatiallySparseBatch &b = cnn.batchPool[cc];
-      if (part == 0) {
+      if (nextPart == 0) { // (this thread's batch until it has parts to take)
         slotOpen[cc] = 1;
+        opening = true;
+        lock.unlock();
+        SpatiallySparseBatch &b = cnn.batchPool[cc];
         openBatch(c, cc);
         b.parts.resize(std::max<size_t>(b.parts.size(), nSlots));
         b.partsLeft = nSlots;
+        lock.lock();
+        opening = false;
       }
+      part = nextPart++;
       if (nextPart == nSlots) {
         ++nextOpen;
         nextPart = 0;
