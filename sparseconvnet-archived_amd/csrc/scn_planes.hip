@@ -2306,6 +2306,7 @@ bool scn_planes_abt(scn_ctx *ctx, const float *A, const float *Wt, float *out,
     *transpose = choice.image;
     return false;
   }
+  ProfScope prof(ctx, SCN_K_BACKWARD);
   *rc = planes_forward<3>(ctx, A, A, Wt, out, M, K, N, ep, nullptr, false, choice, true);
   return true;
 }
@@ -2429,6 +2430,7 @@ bool scn_abt_narrow(scn_ctx *ctx, const float *A, const float *W, float *out, lo
   int parts = (int)std::max<long long>(1, std::min<long long>((2 * ctx->numCU + groups - 1) / groups, all / 4));
   const int tiles = (all + parts - 1) / parts;
   parts = (all + tiles - 1) / tiles;
+  ProfScope prof(ctx, SCN_K_BACKWARD);
   hipLaunchKernelGGL(k_abt_narrow, dim3((unsigned)groups, (unsigned)parts), dim3(64 * NARROW_WAVES), 0, ctx->stream, A, W, out,
                      M, n, K, tiles);
   return true;

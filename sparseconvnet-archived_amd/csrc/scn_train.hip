@@ -709,16 +709,12 @@ extern "C" int scn_sgemm_ABt(scn_ctx *ctx, const float *d_D, const float *d_W,
   ep.bias = ctx->d_zeros;
   ep.p = 1.f;
   ep.act = SCN_NOSIGMOID;
-  {
-    ProfScope prof(ctx, SCN_K_BACKWARD);
-    if (scn_abt_narrow(ctx, d_D, d_W, d_dA, (long long)M, N, K)) {
-      SCN_HIP_CHECK(hipGetLastError());
-      return SCN_OK;
-    }
+  if (scn_abt_narrow(ctx, d_D, d_W, d_dA, (long long)M, N, K)) {
+    SCN_HIP_CHECK(hipGetLastError());
+    return SCN_OK;
   }
   if (K <= SCN_ZERO_FLOATS) { // the planes read W [K x N] as it stands
     int rc = SCN_OK;
-    ProfScope prof(ctx, SCN_K_BACKWARD);
     if (scn_planes_abt(ctx, d_D, d_W, d_dA, (long long)M, N, K, ep, &rc, &transpose)) {
       SCN_TRY(rc);
       SCN_HIP_CHECK(hipGetLastError());

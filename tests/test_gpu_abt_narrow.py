@@ -48,3 +48,19 @@ def test_what_is_not_finite_is_what_fp32_makes_of_it(scn, ctx):
     sure = np.isfinite(want) & ~most
     assert np.array_equal(got[~np.isfinite(want)], want[~np.isfinite(want)].astype(np.float32), equal_nan=True)
     assert np.all(np.abs(got[sure] - want[sure]) <= n * 2.0 ** -24 * scale[sure])
+
+
+# (rows of few columns; by planes, in tiles and split; on the transpose)
+@pytest.mark.parametrize("M,N,K,launches", [(3000, 32, 128, 1), (20000, 256, 128, 1), (500, 256, 128, 1), (90, 30, 20, 2), (3000, 20, 128, 2)])
+def test_a_profile_has_no_spans_without_a_launch(scn, M, N, K, launches):
+    rng = np.random.default_rng(M)
+    c = scn.Context()
+    D, W = c.array(rng.standard_normal((M, N), dtype=np.float32)), c.array(rng.standard_normal((K, N), dtype=np.float32))
+    dA, ws = c.empty((M, K), np.float32), c.empty(scn.lib().scn_sgemm_ABt_workspace(N, K), np.float32)
+    c.sgemm_ABt(D, W, dA, M, N, K, ws)
+    c.prof_enable(True)
+    c.sgemm_ABt(D, W, dA, M, N, K, ws)
+    spans = c.prof_spans()
+    c.prof_enable(False)
+    print(spans, flush=True)
+    assert len(spans) == launches
