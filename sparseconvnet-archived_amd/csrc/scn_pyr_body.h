@@ -141,10 +141,11 @@ template <int D, typename E> PYR_BODY void pyr_masks_body(E &e, const PyrArgs &a
   });
 }
 
-// Level x's mask of sample b, its slab a.slabOf[y], by one wavefront
+// The mask of sample b at the level of pair y of a.slab, one slab of it, by one wavefront
 template <int D, int RW, typename E>
 PYR_BODY void pyr_levels_body(E &e, const PyrArgs &a, unsigned char *lds, int b, int y) {
-  const int x = a.slabLevel[y], slab = a.slabOf[y];
+  const PyrPair of = pyr_pair(a.slab, y);
+  const int x = of.a, slab = of.b;
   const PyrLevel &L = a.lv[x];
   const int nOut = L.nOut, n0 = a.lv[0].nOut;
   const long long vol0 = a.lv[0].volOut;
@@ -304,10 +305,11 @@ template <int D, typename E> PYR_BODY void pyr_rules_body(E &e, const PyrArgs &a
   // chunk now, what lies before it once the chunks' sums are there
   unsigned *const sums = reinterpret_cast<unsigned *>(lds + PYR_HDR_BYTES + 8ll * a.pyrStride);
   e.waves(a.nChunks, [&](int i) {
-    const int x = a.chunkLevel[i];
+    const PyrPair of = pyr_pair(a.chunk, i);
+    const int x = of.a;
     if (x < xFirst || x > xLast)
       return;
-    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * a.chunkOf[i];
+    const int words = h->words[x], at = h->maskOff[x], w0 = PYR_CHUNK * of.b;
     typename E::template Wave<PyrFour> pc;
     e.wave([&](int lane) {
       PYR_UNROLL
@@ -330,7 +332,8 @@ template <int D, typename E> PYR_BODY void pyr_rules_body(E &e, const PyrArgs &a
   });
   e.sync();
   e.waves(a.nChunks, [&](int i) {
-    const int x = a.chunkLevel[i], c = a.chunkOf[i];
+    const PyrPair of = pyr_pair(a.chunk, i);
+    const int x = of.a, c = of.b;
     if (c == 0 || x < xFirst || x > xLast)
       return;
     const unsigned before = e.sum([&](int lane) {

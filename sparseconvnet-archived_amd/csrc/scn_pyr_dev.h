@@ -73,13 +73,17 @@ struct PyrLevel {
 
 // What a workgroup of pass B does of a sample: layers la .. lb, or (F > 1, la ==
 // lb) the f-th of F slabs of one layer's output field along its first axis.
-struct PyrPart {
+struct alignas(4) PyrPart { // (a word: see PyrArgs)
   unsigned char la, lb, f, F;
 };
 #define PYR_MAX_PARTS 24
 #define PYR_MAX_SLABS 48
 #define PYR_MAX_CHUNKS 88
 
+// The arguments of a launch.  Its lists are of whole words: with a list of bytes beside
+// pointers the compiler can take the bytes' index into the base of the scalar loads of
+// those (as it did for k_atb_many's), whose address loses the last two bits of each of
+// its parts.
 struct PyrArgs {
   int nLevels; // recorded layers: levels 1 .. nLevels
   int nMasks;  // levels with a mask: 0 .. nMasks - 1 (the terminal layer has none)
@@ -94,14 +98,14 @@ struct PyrArgs {
   pyr_u64 *pyramid; // [batch][maskWords]
   int slabs;        // wavefronts of pass A a level may be shared out among
   int nSlabs;       // levels and slabs there are
-  unsigned char slabLevel[PYR_MAX_SLABS], slabOf[PYR_MAX_SLABS];
+  unsigned slab[PYR_MAX_SLABS / 2]; // pyr_pair: the level, which of its slabs
   int *counts;      // [nMasks][batch][slabs]: sites
   long long *scalars;
   const long long *badSites;
   int ldsBytesB; // dynamic LDS pass B is launched with
   // rank prefixes are made a chunk of a level's mask words at a time
   int nChunks;
-  unsigned char chunkLevel[PYR_MAX_CHUNKS], chunkOf[PYR_MAX_CHUNKS];
+  unsigned chunk[PYR_MAX_CHUNKS / 2]; // pyr_pair: the level, which of its chunks
   int nParts;
   PyrPart parts[PYR_MAX_PARTS];
   PyrLevel lv[PYR_MAX_LEVELS + 1];
@@ -120,6 +124,18 @@ PYR_FN unsigned pyr_div(unsigned x, unsigned d, unsigned magic) {
   return d == 1 ? x : pyr_mulhi(x, magic);
 }
 PYR_FN unsigned pyr_magic(long long d) { return (unsigned)((1ull << 32) / (pyr_u64)(d > 0 ? d : 1) + 1); }
+// two numbers below 256 each, two such pairs to a word, put in order
+PYR_FN void pyr_put(unsigned *list, int i, int a, int b) {
+  const unsigned v = (unsigned)a | (unsigned)b << 8;
+  list[i / 2] = i & 1 ? list[i / 2] | v << 16 : v;
+}
+struct PyrPair {
+  int a, b;
+};
+PYR_FN PyrPair pyr_pair(const unsigned *list, int i) {
+  const unsigned v = list[i >> 1] >> (i & 1) * 16;
+  return {(int)(v & 255), (int)(v >> 8 & 255)};
+}
 PYR_FN pyr_u64 pyr_even_bits(pyr_u64 x) {
   x &= 0x5555555555555555ull;
   x = (x | (x >> 1)) & 0x3333333333333333ull;
@@ -516,10 +532,8 @@ PYR_FN long long pyr_plan_slabs(PyrArgs &a, int RW) {
       const PyrLevel &L = a.lv[x];
       const int slabs = pyr_slabs(a.d, n0, L, most);
       for (int z = 0; z < slabs; ++z, ++a.nSlabs) {
-        if (a.nSlabs < PYR_MAX_SLABS) {
-          a.slabLevel[a.nSlabs] = (unsigned char)x;
-          a.slabOf[a.nSlabs] = (unsigned char)z;
-        }
+        if (a.nSlabs < PYR_MAX_SLABS)
+          pyr_put(a.slab, a.nSlabs, x, z);
         const long long words = pyr_slab_words(a.d, RW, n0, L, pyr_slab(a.d, L, L.magicN, z, slabs));
         need = x > 0 && words > need ? words : need;
       }
@@ -633,8 +647,7 @@ PYR_FN bool pyr_set_chunks(PyrArgs &a) {
     for (int c = 0; PYR_CHUNK * c < a.lv[x].words + 2; ++c, ++a.nChunks) {
       if (a.nChunks == PYR_MAX_CHUNKS)
         return false;
-      a.chunkLevel[a.nChunks] = (unsigned char)x;
-      a.chunkOf[a.nChunks] = (unsigned char)c;
+      pyr_put(a.chunk, a.nChunks, x, c);
     }
   return true;
 }
