@@ -108,7 +108,9 @@ extern "C" int scn_gather_rows(scn_ctx *ctx, const float *d_in, float *d_out,
   // (rows not known on the host yet: count is their bound times the rule width)
   const long long *dRows = ctx->d_meta ? ctx->d_meta + META_SITES : nullptr;
   const int perRow = dRows && ctx->rowsBound > 0 ? (int)(count / ctx->rowsBound) : 1;
-  if (nIn == 1 && aligned16(d_rules) && aligned16(d_out) && count < (long long)1 << 40) {
+  // (a launch has fewer than 2^32 lanes, and four rules to a lane: far more rules are the
+  // other kernel's, whose workgroups go round)
+  if (nIn == 1 && aligned16(d_rules) && aligned16(d_out) && count < (long long)1 << 32) {
     hipLaunchKernelGGL(k_gather_words, dim3((unsigned)((count + 1023) / 1024)), dim3(256), 0, ctx->stream, d_in, d_out, d_rules,
                        (long long)count, dRows, perRow);
     SCN_HIP_CHECK(hipGetLastError());
