@@ -13,8 +13,9 @@
 // consecutive 16-byte chunks; reads are contiguous per rule.  A negative rule
 // (the reference reads out of bounds on one) gathers a row of zeros.
 // `tile`: rules a workgroup takes at a time.  What it waits for is a trip to the rules and
-// one to the rows for every four loads of a lane: fewer rules, down to four loads, where
-// there are not as many workgroups as compute units (us, with 256 and so: 2000 rows of 8 x
+// one to the rows for every four loads of a lane: fewer rules, halved while a lane has more
+// than four loads (so down to between two and four), where there are not as many
+// workgroups as compute units (us, with 256 and so: 2000 rows of 8 x
 // 128 6.6, 4.9; 60 of 8 x 160 6.5, 4.8; with more workgroups it loses: 30000 of 4 x 64 7.9, 8.5).
 template <typename VecT, int VEC>
 __global__ void __launch_bounds__(GATHER_THREADS)

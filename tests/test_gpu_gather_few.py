@@ -1,4 +1,4 @@
-"""scn_gather_rows of few rules: workgroups of fewer rules, to four loads a lane, and the bytes are the same."""
+"""scn_gather_rows of few rules: workgroups of fewer rules, down to between two and four loads a lane, and the bytes are the same."""
 import numpy as np
 import pytest
 
