@@ -2193,8 +2193,8 @@ extern "C" int scn_conv_nin_forward_rounded(scn_ctx *ctx, const float *d_in, con
   SCN_REQUIRE(ctx, SCN_ERR_ARG, "scn_conv_nin_forward_rounded: null context");
   SCN_REQUIRE(nIn % 8 == 0 && scn_conv_nin_supported_p(fs, nIn, N, SCN_BF16), SCN_ERR_ARG,
               "scn_conv_nin_forward_rounded: fs %d nIn %d N %d is outside the bf16 fused kernel's range", fs, nIn, N);
-  // (d_in and d_in16 may be null: no rows, every rule negative)
-  SCN_REQUIRE((d_rules && d_W && d_B && d_out && (act != SCN_PRELU || d_prelu)) || M == 0, SCN_ERR_ARG,
+  // (d_in16 may be null: d_in is rounded on the way)
+  SCN_REQUIRE((d_in && d_rules && d_W && d_B && d_out && (act != SCN_PRELU || d_prelu)) || M == 0, SCN_ERR_ARG,
               "scn_conv_nin_forward_rounded: null buffer");
   SCN_REQUIRE((((uintptr_t)d_in | (uintptr_t)d_W | (uintptr_t)d_in16 | (uintptr_t)d_image) & 15) == 0, SCN_ERR_ARG,
               "scn_conv_nin_forward_rounded: buffers must be 16-byte aligned");
@@ -2208,8 +2208,7 @@ extern "C" int scn_conv_nin_forward_rounded(scn_ctx *ctx, const float *d_in, con
   gs.nIn = nIn;
   gs.magic = (unsigned)((1ull << 32) / (unsigned)nIn + 1);
   gs.zeros = ctx->d_zeros;
-  return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p, act, SCN_BF16, &gs, d_in ? d_in16 : nullptr,
-                     d_image);
+  return nin_forward(ctx, d_in, d_W, d_B, d_prelu, d_out, M, fs * nIn, N, p, act, SCN_BF16, &gs, d_in16, d_image);
 }
 static int conv_nin_forward(scn_ctx *ctx, const float *d_in, const int32_t *d_rules, int fs, int nIn,
                             const float *d_W, const void *d_image, const float *d_B, const float *d_prelu,
