@@ -1423,9 +1423,12 @@ static int grids_prepare(scn_ctx *ctx, scn_grids *g, int batch, int d, int n,
 }
 
 // One launch empties the tables and masks of up to CLEAR_MANY grids objects, but for
-// those that have an empty mask to go on with: a launch of 3 us and the gap behind it,
-// at the beginning of every batch (us, one drawing 115 -> 101 to 111, 100 drawings 188 -> 179
-// to 190, 32 voxel models 185 -> 180: runs fall into one of two groups).
+// those that have an empty mask to go on with: a launch at the beginning of every batch
+// less.  us, medians of passes without a second mask and with one, eight processes of
+// each in turn, of which four to six are in the faster of the two groups that they fall
+// into: one drawing 103 to 104, 100 to 103; 100 drawings 180 to 184, 177 to 179; 33 voxel models
+// 170 to 171, 167 to 169.  The groups are 9 to 20 apart, which is more; epochs take the
+// same time, their masks were emptied beside other batches.
 #define CLEAR_MANY 24
 struct ClearList {
   uint4 *slots[CLEAR_MANY];

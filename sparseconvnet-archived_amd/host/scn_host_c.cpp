@@ -165,8 +165,9 @@ static void put(vectorCUDA<float> &v, const float *src) {
 }
 // A layer's vectors, written to pinned memory by one kernel and waited for once (a
 // blocking copy of each to ordinary memory takes 18 us, whatever its size: 0.6 ms
-// of reading a net of seven such layers back; with a launch for each vector a layer of two
-// took 20.5 to 35 us, with three 28, now 17 to 31 and 22)
+// of reading a net of seven such layers back).  With a launch for each vector and in one,
+// medians of 300 calls to an idle net, the same in each of four processes: layers of two
+// 22.5 us, 19.6, one of three 26.3, 21.6; the fourteen calls for a net's state 336, 293.
 static void get(scnh_net *net, std::initializer_list<std::pair<vectorCUDA<float> *, float *>> vectors) {
   std::lock_guard<std::mutex> lock(net->readBackMutex);
   scn_ctx *ctx = net->cnn->memStream.ctx;
